@@ -56,6 +56,10 @@ extern "C" {
                               range's slice over the whole of K, keeps the result in LDS and expands it into its
                               range; needs no workspace */
 
+#define MLORA_FORM_PAIR 9  /* a shrink launch over (tile, slice, K part) and an expand launch over (tile, column range) that
+                              meet in the workspace; 16-token tiles for few tokens per slot, else 64-token tiles; weights and
+                              x rows go straight to LDS; 16- and 32-bit elements */
+
 /* error codes (negative) */
 #define MLORA_E_INVALID (-1)     /* malformed argument (NULL pointer, negative size, bad dtype) */
 #define MLORA_E_UNSUPPORTED (-2) /* well-formed but outside what the selected form handles */

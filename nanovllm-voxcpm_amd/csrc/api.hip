@@ -79,7 +79,7 @@ namespace {
 
 // Diagnostic knobs, read from the environment once per process.
 struct ApiKnobs {
-  int generation = -1, small_batch_tokens, force_form, no_split, split_min_rk, split_max_tokens, auto_fused, slot_max_slots, no_wide;
+  int generation = -1, small_batch_tokens, force_form, no_split, split_min_rk, split_max_tokens, auto_fused, slot_max_slots, no_wide, no_pair;
   void read() {
     generation = knob_generation();
     small_batch_tokens = env_int("MLORA_SMALL_BATCH_TOKENS", 0);
@@ -92,6 +92,7 @@ struct ApiKnobs {
     // does not pay for the wait on the slowest role of each unit.  AUTO keeps the two launches.
     auto_fused = env_int("MLORA_AUTO_FUSED", 0);
     no_wide = env_int("MLORA_NO_WIDE", 0);
+    no_pair = env_int("MLORA_NO_PAIR", 0);
     // The split form pays when A[slot], which every workgroup of a tile would otherwise fetch whole,
     // is large: rank x K >= 131072 elements (256 KB).  Measured on the decode batch (256 tokens, 32
     // adapters), one workgroup per (tile, column range) against the split form, us per call: rank 16,
@@ -167,6 +168,42 @@ static bool slot_major_pays(const MloraAddArgs* a) {
   return a->num_tokens >= 4 * a->num_slots;
 }
 
+// Where the shrink and the expand as two launches over 16-token tiles (pair.hip) beat the form that
+// `form` names.  A second launch costs about 3 us; what it saves is the repeated intake of A[slot] by
+// every column range of a tile, which grows with rank x K and with the number of ranges.  Measured, us per
+// call, that form / the pair (replayed graphs; 201 tokens over 48 slots of mixed rank 8..64, K = 2048:
+// qkv 27.6 / 17.0, o 23.6 / 11.8, gate_up 43.5 / 31.9, down 38.7 / 17.5):
+//  - split form (rank x K >= 131072, few tokens): 4 of 4 shapes at 1..512 tokens, rank 16..64 (one token:
+//    rank 64, K = 2048: 10.9 / 7.1; rank 16, K = 8192: 7.3 / 7.1; 64 tokens, rank 32, K = 8192: 15.3 / 10.7);
+//  - one workgroup per (tile, column range): from rank x K = 131072 on (1234 tokens, rank 32, K = 4096: 19.1 /
+//    13.9; it loses below: rank 16, K = 4096, 2000 tokens 11.5 / 12.5, and ties at rank 32, K = 2048), and for
+//    buffers of a rank between the instances', whose code is the general one away from K = 1024 (64 tokens, rank 48, K = 2048:
+//    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9) and which have no form over 64-token tiles (6000
+//    tokens, rank 48: 40.5 / 32.7, 24.3 / 22.6, 115 / 74, 50 / 35; at 1500 tokens and rank 24 qkv and o are
+//    still the faster ones in one launch: 12.7 / 13.3, 8.1 / 11.2);
+//  - 64-token tiles: tokens x rank up to 1.4e5, beyond which the small tiles fetch A and B too often (rank
+//    64, K = 4096: 18.9 / 13.4 at 1000 tokens, 22.2 / 22.4 at 3001),
+//    where A is as large; wide outputs stay with them (rank 64, K = 2048 -> 16384: 32.2 / 33.2 at 1000).
+static bool pair_pays(const MloraAddArgs* a, int form) {
+  const long long rk = static_cast<long long>(a->r) * a->k;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  const bool few = static_cast<long long>(a->num_tokens) * a->r <= 140000;
+  switch (form) {
+    case MLORA_FORM_SPLIT: return true;
+    case MLORA_FORM_MFMA: {
+      if (!exact_rank(a->r)) {
+        const double width = static_cast<double>(a->num_slices) * a->k + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
+        return a->k != 1024 || a->num_tokens * width > (a->r > 32 ? 1.0e7 : 2.0e7);
+      }
+      return rk >= 131072;
+    }
+    case MLORA_FORM_SGMV:
+    case MLORA_FORM_WIDE: return few && rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k);
+    default: return false;
+  }
+}
+
 namespace {
 
 int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace);
@@ -185,7 +222,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
   if (a->dtype != MLORA_DTYPE_F32 && a->dtype != MLORA_DTYPE_F16 && a->dtype != MLORA_DTYPE_BF16) {
     set_error("mlora_add_lora: unknown dtype %d", a->dtype); return MLORA_E_INVALID;
   }
-  if (a->form < MLORA_FORM_AUTO || a->form > MLORA_FORM_WIDE) { set_error("mlora_add_lora: unknown form %d", a->form); return MLORA_E_INVALID; }
+  if (a->form < MLORA_FORM_AUTO || a->form > MLORA_FORM_PAIR) { set_error("mlora_add_lora: unknown form %d", a->form); return MLORA_E_INVALID; }
   if (a->num_slices > MLORA_MAX_SLICES) { set_error("mlora_add_lora: %d slices exceed %d", a->num_slices, MLORA_MAX_SLICES); return MLORA_E_TOO_LARGE; }
   if (a->r > MLORA_MAX_RANK) { set_error("mlora_add_lora: rank %d exceeds %d", a->r, MLORA_MAX_RANK); return MLORA_E_TOO_LARGE; }
   if (a->num_slots > MLORA_MAX_SLOTS) { set_error("mlora_add_lora: %d slots exceed %d", a->num_slots, MLORA_MAX_SLOTS); return MLORA_E_TOO_LARGE; }
@@ -211,7 +248,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
   const bool vec = vector_ok(a);
   if (form == MLORA_FORM_AUTO) {
     const int forced = knobs().force_form;
-    if (forced >= MLORA_FORM_TOKEN && forced <= MLORA_FORM_WIDE && (forced == MLORA_FORM_TOKEN || vec)) form = forced;
+    if (forced >= MLORA_FORM_TOKEN && forced <= MLORA_FORM_PAIR && (forced == MLORA_FORM_TOKEN || vec)) form = forced;
   }
   if (form == MLORA_FORM_AUTO) {
     // Small batches (decode) are one launch over 16-token tiles; large ones split into 64-token
@@ -238,6 +275,8 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
       knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a))
     form = MLORA_FORM_SLOT;
+  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form))
+    form = MLORA_FORM_PAIR;
   // long-segment batches in one launch, on request
   if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_SGMV && knobs().auto_fused && fused_supported(a))
     form = MLORA_FORM_FUSED;
@@ -257,6 +296,13 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
         return MLORA_E_UNSUPPORTED;
       }
       return launch_wide(a);
+    case MLORA_FORM_PAIR:
+      if (!pair_supported(a)) {
+        set_error("mlora_add_lora: the pair form needs a plan, a workspace, rows of x of a multiple of 128 bytes, B rows of 16 to 128 (fp32: 256) bytes "
+                  "in steps the kernels have, 16-byte aligned rows and no empty slice");
+        return MLORA_E_UNSUPPORTED;
+      }
+      return launch_pair(a);
     case MLORA_FORM_SGMV:
     case MLORA_FORM_FUSED:
     case MLORA_FORM_SPLIT:

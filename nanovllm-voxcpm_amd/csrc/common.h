@@ -91,6 +91,19 @@ template <> struct Mma<_Float16> {
   }
 };
 
+// fp32 operands on the same 16-byte pieces: four 16x16x4 products, product j taking element j of
+// every lane's piece (both operands order the contraction the same way, so any order will do).
+template <> struct Mma<float> {
+  static __device__ __forceinline__ f32x4 run(const Pack8& a, const Pack8& b, f32x4 c) {
+    f32x4 x, y;
+    __builtin_memcpy(&x, &a, 16);
+    __builtin_memcpy(&y, &b, 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], y[j], c, 0, 0, 0);
+    return c;
+  }
+};
+
 // 16x16x16 variant (four operand elements per lane): for rank 16 the contraction of the
 // expand is exactly sixteen long, so no lane fetches B elements it would multiply by zero.
 typedef short s16x4 __attribute__((ext_vector_type(4)));

@@ -14,6 +14,7 @@ extern "C" int mlora_trace_set(void* buf) {
   fused_trace_set(buf);
   sgmv_trace_set(buf);
   wide_trace_set(buf);
+  pair_trace_set(buf);
   return 0;
 #else
   (void)buf;

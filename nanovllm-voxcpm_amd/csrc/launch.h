@@ -62,6 +62,11 @@ bool wide_supported(const MloraAddArgs* a);
 bool wide_pays(const MloraAddArgs* a);
 int launch_wide(const MloraAddArgs* a);
 
+// pair.hip: a shrink launch and an expand launch over the 16- or the 64-token tiles, operands through
+// LDS by direct loads; 16- and 32-bit elements.
+bool pair_supported(const MloraAddArgs* a);
+int launch_pair(const MloraAddArgs* a);
+
 // in-kernel timeline of trace builds (no-ops otherwise)
 void decode_trace_set(void* buf);
 void slot_trace_set(void* buf);
@@ -69,5 +74,6 @@ void split_trace_set(void* buf);
 void fused_trace_set(void* buf);
 void sgmv_trace_set(void* buf);
 void wide_trace_set(void* buf);
+void pair_trace_set(void* buf);
 
 }  // namespace mlora

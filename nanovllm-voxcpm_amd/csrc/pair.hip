@@ -1,0 +1,585 @@
+// The apply in two launches, shrink then expand, with every weight and x row passing through LDS by
+// direct loads.  Computes what the reference computes with a shrink launch, a temporary
+// [slices, T, r] tensor and one or two expand launches (nanovllm_voxcpm/lora.py:291-381,
+// lora_ops/triton_ops/lora_shrink_op.py:16-173, lora_expand_op.py:11-91).
+//
+// What it is for.  The one-launch forms over small tiles let every column range of a tile fetch the
+// tile's x rows and all of A[slot] again; with a large A[slot] (rank x K) that repeated intake is
+// most of a call.  Here a workgroup of the first launch takes one (tile, slice, K part), so every
+// A line is fetched once per tile, and leaves its block of partial sums in the
+// workspace; a workgroup of the second takes one (tile, column range), adds the parts up and expands.
+//
+// How operands travel.  The matrix cores want sixteen different rows in sixteen consecutive lanes,
+// and a 128-bit load laid out like that costs the compute unit's address unit four times what a load
+// along one row costs.  Direct-to-LDS loads (16 bytes per lane, lane i to byte 16 i behind a base)
+// walk along rows at the full rate, need no registers for what is on its way, and put the chunks where
+// the operand reads want them: chunk p of a row goes to place p ^ (row & 7) of the row's eight, so
+// that the sixteen rows of an operand read fall on different banks.  The loads are inline assembly,
+// which the compiler does not count among the loads in flight: every wait for them is written here,
+// and counts the younger requests of this file's own.
+#include "common.h"
+#include "launch.h"
+#include "sgmv_body.h"
+
+namespace mlora {
+
+namespace {
+
+constexpr int kPairWaves = 4;
+constexpr int kPairThreads = kPairWaves * kWave;
+constexpr int kChunk = 128;     // bytes of a row that a step of the shrink takes
+constexpr int kMaxParts = 8;    // most K parts of a launch
+constexpr int kPartsAhead = 4;  // of which the expand requests this many together
+
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(p)));
+}
+__device__ __forceinline__ const char* uniform(const char* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// One 1 KB direct load: lane i's 16 bytes at base + voff go to LDS byte lds + 16 i.
+__device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds) {
+#ifdef MLORA_TRACE
+  base = uniform(static_cast<const char*>(base));  // (the branches around the stamps cost the compiler its proof of that)
+#endif
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+}
+
+// ---- shrink -------------------------------------------------------------------------------------
+// A wavefront's own share of a (tile, slice, K part): chunks [c0, c1) of 128 bytes of every row, through
+// a private ring of NST stages in LDS, so that no barrier stands between request and product.
+// The share is two eighths of the part, [c0, cm) and [cm, c1), whose sums stay apart (first, acc): the
+// eight sums of a part are then added in order, which are the sums the split form (split.hip) takes
+// over its eight wavefronts and in its order, so that at the same K parts both leave the same bits.
+// NA8: groups of eight ranks.  acc[rb]: lane holds ranks 16 rb + 4 (lane / 16) .. + 3 of token lane % 16.
+template <int NA8> struct ShrinkShape {
+  static constexpr int RB = (NA8 + 1) / 2;
+  static constexpr int ND = NA8 + 2;                 // direct loads per stage
+  static constexpr int NST = ND <= 6 ? 4 : 2;        // stages of a wavefront's ring: 48-96 KB per workgroup on their way
+  static constexpr int BYTES = NST * ND * 1024;      // of LDS per wavefront
+};
+
+template <typename T, int NA8>
+__device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
+                                              int c0, int cm, int c1, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
+  typedef ShrinkShape<NA8> S;
+  constexpr int RB = S::RB, ND = S::ND, NST = S::NST;
+  const int lane = threadIdx.x & (kWave - 1), lr = lane & 15, lg = lane >> 4;
+  const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;
+  uint32_t aoff[NA8];
+#pragma unroll
+  for (int g = 0; g < NA8; ++g) {
+    const int row = g * 8 + (lane >> 3);
+    aoff[g] = static_cast<uint32_t>(row < rbuf ? row : rbuf - 1) * arow + swz;
+  }
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) first[rb] = acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_address(ring));
+  auto issue = [&](int c, int stage) {
+    const char* a = abase + static_cast<int64_t>(c) * kChunk;
+    const char* x = xbase + static_cast<int64_t>(c) * kChunk;
+    const uint32_t to = lds + stage * (ND * 1024);
+#pragma unroll
+    for (int g = 0; g < NA8; ++g) dma16(a, aoff[g], to + g * 1024);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16(x, xoff[i] + swz, to + (NA8 + i) * 1024);
+  };
+  const int n = c1 - c0;
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < n) issue(c0 + s, s);
+  MLORA_STAMP(2);  // shrink: first stages requested
+  int stage = 0, into = NST - 1;
+  for (int c = 0; c < n; ++c) {
+    if (c + NST - 1 < n) {
+      wait_lds();  // the operand reads of the step before, from the stage that is filled next, are through
+      issue(c0 + c + NST - 1, into);
+    }
+    const int younger = n - 1 - c < NST - 1 ? n - 1 - c : NST - 1;  // stages requested behind this one
+    if constexpr (NST == 4) {
+      if (younger >= 3) wait_loads<3 * ND>();
+      else if (younger == 2) wait_loads<2 * ND>();
+      else if (younger == 1) wait_loads<ND>();
+      else wait_loads<0>();
+    } else {
+      if (younger >= 1) wait_loads<ND>();
+      else wait_loads<0>();
+    }
+    if (c0 + c == cm) {  // the first of the wavefront's two shares is complete
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        first[rb] = acc[rb];
+        acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    const char* st = ring + stage * (ND * 1024) + lr * 128 + ((lg ^ (lr & 7)) * 16);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const char* at = st + (ks == 0 ? 0 : (lg ^ (lr & 7)) & 4 ? -64 : 64);  // chunk lg, then chunk lg + 4, of the swizzled row
+      Pack8 xa;
+      xa.raw = *reinterpret_cast<const i32x4*>(at + NA8 * 1024);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        Pack8 aw;
+        aw.raw = *reinterpret_cast<const i32x4*>(at + rb * 2048);
+        acc[rb] = Mma<T>::run(aw, xa, acc[rb]);
+      }
+    }
+    stage = stage + 1 == NST ? 0 : stage + 1;
+    into = into + 1 == NST ? 0 : into + 1;
+  }
+  MLORA_STAMP(3);  // shrink: multiplied
+  mfma_settle(acc);  // (the last product and the reads of the sums lie on two sides of the loop's exit)
+}
+
+// dst: this tile's block of partial sums, sixteen rows of rp floats.
+template <typename T, int NA8>
+__device__ __forceinline__ void shrink_tile(char* lds, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2], int c0,
+                                            int cm, int c1, float* __restrict__ dst, int rp, int m) {
+  typedef ShrinkShape<NA8> S;
+  constexpr int RB = S::RB;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  char* ring = lds + wave * S::BYTES;
+  f32x4 first[RB], acc[RB];
+  shrink_chunks<T, NA8>(ring, abase, arow, rbuf, xbase, xoff, c0, cm, c1, first, acc);
+  // sum over the eighths of the part, the first one first, through the rings' memory
+  static_assert(2 * RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    *reinterpret_cast<f32x4*>(ring + (rb * kWave + lane) * 16) = first[rb];
+    *reinterpret_cast<f32x4*>(ring + ((RB + rb) * kWave + lane) * 16) = acc[rb];
+  }
+  __syncthreads();
+  MLORA_STAMP(4);  // shrink: every wavefront's sums in LDS
+  if (wave < RB) {
+    f32x4 s = *reinterpret_cast<const f32x4*>(lds + tid * 16);
+#pragma unroll
+    for (int w = 1; w < 2 * kPairWaves; ++w) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(lds + (w >> 1) * S::BYTES + (w & 1) * (RB * 1024) + tid * 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] += v[i];
+    }
+    const int tok = lane & 15;
+    if (tok < m) *reinterpret_cast<f32x4*>(dst + tok * rp + wave * 16 + 4 * (lane >> 4)) = s;
+  }
+}
+
+// A tile's record, with the plan header's verdict on it.
+struct PairTile {
+  int slot, m, ok, plan_ok;
+};
+__device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __restrict__ plan, int tile, int T_, int num_slots) {
+  const i32x4 h0 = *reinterpret_cast<const i32x4*>(plan), h1 = *reinterpret_cast<const i32x4*>(plan + 4), h2 = *reinterpret_cast<const i32x4*>(plan + 8);
+  PairTile t;
+  t.slot = r0[0];
+  t.m = r0[1];
+  t.plan_ok = int(h0[MLORA_PLAN_MAGIC] == MLORA_PLAN_MAGIC_VALUE) & int(h0[MLORA_PLAN_NUM_TOKENS] == T_) & int(h0[MLORA_PLAN_MAX_SLOTS] == num_slots);
+  t.ok = t.plan_ok & int(tile < h1[MLORA_PLAN_TILES_SHORT - 4] + h2[MLORA_PLAN_TILES_LONG_SMALL - 8]) & int(t.m > 0) & int(t.slot >= 0) &
+         int(t.slot < num_slots);
+  return t;
+}
+
+// grid (8, slices * K parts, tiles / 8): blockIdx.x is the XCD, so that the workgroups of a tile share an L2.
+template <typename T>
+__global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
+                                                                   int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, int rbuf,
+                                                                   int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // ---- one trip: tile record, plan header, the tile's token rows, the slots' ranks ------------------
+  MLORA_STAMP(0);  // shrink: first instruction
+  const int tile = blockIdx.z * 8 + blockIdx.x;
+  const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
+  const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
+  int row[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) row[i] = rec[MLORA_SMALL_TILE_ROWS + i * 8 + (lane >> 3)];
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!t.ok) {
+    count_rejected_plan(plan, t.plan_ok);
+    return;
+  }
+  MLORA_STAMP(1);  // shrink: record here
+  const int slot = __builtin_amdgcn_readfirstlane(t.slot), m = __builtin_amdgcn_readfirstlane(t.m);
+  const int eff = rank_pick(ranks, eff_rank, num_slots, slot, rbuf);
+  if (eff == 0) return;
+  const int slice = blockIdx.y >> parts_log2, part = blockIdx.y - (slice << parts_log2);
+  const int p0 = (part * kchunks) >> parts_log2, p1 = ((part + 1) * kchunks) >> parts_log2;
+  const int c0 = p0 + wave * (p1 - p0) / kPairWaves, c1 = p0 + (wave + 1) * (p1 - p0) / kPairWaves;
+  const int cm = p0 + (2 * wave + 1) * (p1 - p0) / (2 * kPairWaves);
+  const uint32_t arow = static_cast<uint32_t>(kchunks) * kChunk;
+  const char* abase = uniform(static_cast<const char*>(sl.a[slice]) + static_cast<int64_t>(slot) * rbuf * arow);
+  const char* xbase = static_cast<const char*>(xv);
+  uint32_t xoff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) xoff[i] = static_cast<uint32_t>(row[i]) * xrow;
+  const int rp = (rbuf + 15) & ~15;
+  float* dst = hws + (static_cast<int64_t>(part * num_slices + slice) * (gridDim.z * 8) + tile) * (MLORA_TILE_SMALL * rp);
+  const int groups = (eff + 7) >> 3;
+  if (groups <= 1) shrink_tile<T, 1>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+  else if (groups == 2) shrink_tile<T, 2>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+  else if (groups <= 4) shrink_tile<T, 4>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+  else if (groups <= 6) shrink_tile<T, 6>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+  else shrink_tile<T, 8>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+#ifdef MLORA_TRACE
+  MLORA_STAMP(5);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  MLORA_STAMP(6);  // shrink: sums acknowledged
+#endif
+}
+
+// An adapter of few ranks may have a deeper ring than one that fills the buffers: the most of all.
+int shrink_lds(int rbuf) {
+  const int groups = (rbuf + 7) / 8;
+  int most = ShrinkShape<1>::BYTES;
+  auto with = [&](int b) { most = b > most ? b : most; };
+  if (groups > 1) with(ShrinkShape<2>::BYTES);
+  if (groups > 2) with(ShrinkShape<4>::BYTES);
+  if (groups > 4) with(ShrinkShape<6>::BYTES);
+  if (groups > 6) with(ShrinkShape<8>::BYTES);
+  return most * kPairWaves;
+}
+
+// ---- expand -------------------------------------------------------------------------------------
+// A wavefront takes SP spans of 64 columns.  C: 16-byte pieces of a B row (rank x element size / 16).
+template <typename T> struct PieceOf { static constexpr int E = 16 / sizeof(T); };
+
+// Zero the elements of a piece that hold ranks at or above `eff`; `first` is the rank of its element 0.
+template <typename T> __device__ __forceinline__ void mask_piece(Pack8& p, int first, int eff) {
+  if constexpr (sizeof(T) == 2) {
+    mask_ranks(p, first, eff);
+  } else {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) p.u[d] = first + d < eff ? p.u[d] : 0u;
+  }
+}
+
+template <typename T, int C, int SP>
+__device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__ hsrc, int64_t part_stride, int kparts, const f32x4 (&hv)[kPartsAhead], const char* bbase,
+                                            T* __restrict__ ybase, const int64_t ys, const i32x4 rows, int n0, int n1, int m, int eff,
+                                            float scaling) {
+  constexpr int E = PieceOf<T>::E;          // elements per piece
+  constexpr int R = C * E;                  // rank of the buffers
+  constexpr int KSTEPS = (C + 3) / 4;       // operand steps of the contraction (four pieces each)
+  constexpr int RP = (R + 15) & ~15;
+  constexpr bool SPLIT = sizeof(T) == 2;    // 16-bit operands: the intermediate as leading part and remainder
+  constexpr int HROW = KSTEPS * 64 + 16;    // bytes of an LDS row of the intermediate (one part)
+  constexpr int SH = C * 4 >= 64 ? 6 : C * 4 >= 32 ? 5 : C * 4 >= 16 ? 4 : 3;  // the swizzle of the B pieces: lanes' rows lie 4 C pieces apart
+  constexpr int NB = SP * C;                // direct loads of a wavefront's B rows
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lr = lane & 15, lg = lane >> 4;
+  char* s_h = lds;                                                   // [2][16] rows
+  char* s_b = lds + 2 * 16 * HROW + wave * (SP * 64 * C * 16);  // this wavefront's B rows
+
+  // the first K parts of the intermediate, B rows, y
+  const int tok = tid / 16, q4 = tid & 15;  // sixteen threads per token, four ranks (RP = 64: all of them busy) each
+  const int c0 = n0 + wave * (SP * 64);
+  const bool mine = c0 < n1;
+  if (mine) {
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds_address(s_b));
+    const char* src = bbase + static_cast<int64_t>(c0) * (C * 16);
+    const uint32_t last = static_cast<uint32_t>(n1 - c0) * C - 1;  // last piece of the range
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const uint32_t u = i * 64 + lane;
+      uint32_t s = u ^ ((u >> SH) & 7);
+      const uint32_t kc = s % C;
+      s = s < last ? s : last;
+      if (kc * E < static_cast<uint32_t>(eff)) dma16(src, s * 16, to + i * 1024);  // (piece 0 of a row is always fetched: some lane takes part)
+    }
+  }
+  typedef typename std::conditional<sizeof(T) == 2, uint2, uint4>::type Y4;
+  Y4 yq[SP][4];
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    int c = c0 + s * 64 + 4 * lr;
+    c = c < n1 ? c : n1 - 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) yq[s][i] = *reinterpret_cast<const Y4*>(ybase + static_cast<int64_t>(rows[i]) * ys + c);
+  }
+  MLORA_STAMP(10);  // expand: B rows and y requested
+  // the intermediate: parts summed in order, scaled, split, to LDS in operand rows (its first
+  // kPartsAhead parts were requested with the record)
+  f32x4 sum = hv[0];
+#pragma unroll
+  for (int kp = 1; kp < kPartsAhead; ++kp) {
+    if (kp < kparts) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] += hv[kp][j];
+    }
+  }
+  const float* p = hsrc + tok * RP + (q4 * 4 < RP ? q4 * 4 : 0);
+  for (int kp = kPartsAhead; kp < kparts; kp += kPartsAhead) {
+    f32x4 v[kPartsAhead];
+#pragma unroll
+    for (int k = 0; k < kPartsAhead; ++k) v[k] = *reinterpret_cast<const f32x4*>(p + (kp + k < kparts ? kp + k : 0) * part_stride);
+#pragma unroll
+    for (int k = 0; k < kPartsAhead; ++k) {
+      if (kp + k < kparts) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += v[k][j];
+      }
+    }
+  }
+  if (q4 * 4 < KSTEPS * 4 * E) {
+    T hi[4], lo[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float v = (tok < m && q4 * 4 + j < eff) ? sum[j] * scaling : 0.f;
+      hi[j] = from_f32<T>(v);
+      lo[j] = from_f32<T>(v - to_f32(hi[j]));
+    }
+    __builtin_memcpy(__builtin_assume_aligned(s_h + tok * HROW + q4 * 4 * sizeof(T), 8), hi, sizeof(hi));
+    if constexpr (SPLIT) __builtin_memcpy(__builtin_assume_aligned(s_h + (16 + tok) * HROW + q4 * 4 * sizeof(T), 8), lo, sizeof(lo));
+  }
+  __syncthreads();
+  MLORA_STAMP(11);  // expand: intermediate in LDS
+  if (!mine) return;
+  Pack8 hop[KSTEPS], hlo[SPLIT ? KSTEPS : 1];
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    hop[ks].raw = *reinterpret_cast<const i32x4*>(s_h + lr * HROW + (ks * 4 + lg) * 16);
+    if constexpr (SPLIT) hlo[ks].raw = *reinterpret_cast<const i32x4*>(s_h + (16 + lr) * HROW + (ks * 4 + lg) * 16);
+  }
+  wait_loads<0>();
+  MLORA_STAMP(12);  // expand: B rows and y here
+  const bool mask = eff < KSTEPS * 4 * E;
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    const int c = c0 + s * 64 + 4 * lr;
+    f32x4 out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      out[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        int kc = ks * 4 + lg;
+        if (C % 4) kc = kc < C ? kc : C - 1;
+        const uint32_t u = (s * 64 + 4 * lr + j) * C + kc;
+        Pack8 bo;
+        bo.raw = *reinterpret_cast<const i32x4*>(s_b + (u ^ ((u >> SH) & 7)) * 16);
+        if (mask) mask_piece<T>(bo, (ks * 4 + lg) * E, eff);
+        if constexpr (SPLIT) out[j] = Mma<T>::run(hlo[ks], bo, out[j]);
+        out[j] = Mma<T>::run(hop[ks], bo, out[j]);
+      }
+    }
+    if (c < n1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (4 * lg + i < m) {
+          union { Y4 raw; T e[4]; } v;
+          v.raw = yq[s][i];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v.e[j] = from_f32<T>(to_f32(v.e[j]) + out[j][i]);
+          *reinterpret_cast<Y4*>(ybase + static_cast<int64_t>(rows[i]) * ys + c) = v.raw;
+        }
+      }
+    }
+  }
+}
+
+#ifdef MLORA_TRACE
+#define MLORA_STAMP_END(i) do { MLORA_STAMP(i); asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); MLORA_STAMP(i + 1); } while (0)
+#else
+#define MLORA_STAMP_END(i) do { } while (0)
+#endif
+// grid (8, column ranges, tiles / 8)
+template <typename T, int C, int SP>
+__global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws, void* __restrict__ yv_,
+                                                                   int64_t ys, int small_off, int T_, int num_slots, int kparts, int num_slices,
+                                                                   float scaling, const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  constexpr int R = C * PieceOf<T>::E, RP = (R + 15) & ~15;
+  const int lane = threadIdx.x & (kWave - 1), lg = lane >> 4;
+  MLORA_STAMP(8);  // expand: first instruction
+  const ExpandSplit sp = splits.split[blockIdx.y];
+  const int tile = blockIdx.z * 8 + blockIdx.x;
+  const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
+  const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
+  const i32x4 rows = *reinterpret_cast<const i32x4*>(rec + MLORA_SMALL_TILE_ROWS + 4 * lg);  // tokens 4 * lg .. + 3
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
+  // the intermediate's partial sums lie where the tile's place says: requested with the record
+  const int64_t stride = static_cast<int64_t>(num_slices) * (gridDim.z * 8) * (MLORA_TILE_SMALL * RP);  // from K part to K part
+  const float* hsrc = hws + (static_cast<int64_t>(sp.slice) * (gridDim.z * 8) + tile) * (MLORA_TILE_SMALL * RP);
+  f32x4 hv[kPartsAhead];
+  {
+    const int tok = threadIdx.x / 16, q4 = threadIdx.x & 15;
+#pragma unroll
+    for (int kp = 0; kp < kPartsAhead; ++kp)
+      hv[kp] = *reinterpret_cast<const f32x4*>(hsrc + (kp < kparts ? kp : 0) * stride + tok * RP + (q4 * 4 < RP ? q4 * 4 : 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (!t.ok) return;
+  MLORA_STAMP(9);  // expand: record here
+  const int slot = __builtin_amdgcn_readfirstlane(t.slot), m = __builtin_amdgcn_readfirstlane(t.m);
+  const int eff = rank_pick(ranks, eff_rank, num_slots, slot, R);
+  if (eff == 0) return;
+  const char* bbase = uniform(static_cast<const char*>(sp.b) + static_cast<int64_t>(slot) * sp.n * (C * 16));
+  expand_tile<T, C, SP>(lds, hsrc, stride, kparts, hv, bbase, static_cast<T*>(yv_) + sp.y_col, ys, rows, sp.n0, sp.n1, m, eff, scaling);
+  MLORA_STAMP_END(13);  // expand: stores issued, acknowledged
+}
+
+int expand_lds(int c, int sp) {
+  const int ksteps = (c + 3) / 4, hrow = ksteps * 64 + 16;
+  return 2 * 16 * hrow + kPairWaves * sp * 64 * c * 16;
+}
+
+// Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
+struct PairKnobs {
+  int generation = -1, kparts, sp, wgs;
+  void read() {
+    generation = knob_generation();
+    kparts = env_int("MLORA_PAIR_KPARTS", 0);
+    sp = env_int("MLORA_PAIR_SP", 0);
+    wgs = env_int("MLORA_PAIR_WGS", 192);
+  }
+};
+const PairKnobs& pair_knobs() {
+  static PairKnobs k;
+  if (k.generation != knob_generation()) k.read();
+  return k;
+}
+
+int element_bytes(int dtype) { return dtype == MLORA_DTYPE_F32 ? 4 : 2; }
+// One K part's partial sums: sixteen rows of the padded rank per place of the tile list and slice.
+size_t part_bytes(const MloraAddArgs* a, const PlanLayout& lay) {
+  return static_cast<size_t>(lay.cap_small) * MLORA_TILE_SMALL * a->num_slices * ((a->r + 15) & ~15) * sizeof(float);
+}
+
+struct PairLaunch {
+  const MloraAddArgs* a;
+  PlanLayout lay;
+  int parts_log2, sp;
+};
+
+template <typename F> bool allow_lds(F* kernel) {
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  return true;
+}
+
+template <typename T> void launch_pair_shrink(const PairLaunch& l) {
+  const MloraAddArgs* a = l.a;
+  ShrinkSlices sl;
+  for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = i < a->num_slices ? a->slices[i].a : nullptr;
+  static const bool once = allow_lds(pair_shrink_kernel<T>);
+  (void)once;
+  hipLaunchKernelGGL((pair_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
+                     dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
+                     a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
+                     l.parts_log2, a->num_slices, a->effective_rank, sl);
+}
+
+template <typename T, int C, int SP> void launch_pair_expand_one(const PairLaunch& l, const ExpandSplits& splits, int total) {
+  const MloraAddArgs* a = l.a;
+  static const bool once = allow_lds(pair_expand_kernel<T, C, SP>);
+  (void)once;
+  hipLaunchKernelGGL((pair_expand_kernel<T, C, SP>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
+                     expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
+                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, splits);
+}
+
+template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const ExpandSplits& splits, int total) {
+  if (l.sp == 1) launch_pair_expand_one<T, C, 1>(l, splits, total);
+  else launch_pair_expand_one<T, C, 2>(l, splits, total);
+  return true;
+}
+
+template <typename T> bool launch_pair_type(const PairLaunch& l, const ExpandSplits& splits, int total) {
+  launch_pair_shrink<T>(l);
+  switch (l.a->r * static_cast<int>(sizeof(T)) / 16) {
+    case 2: return launch_pair_expand<T, 2>(l, splits, total);
+    case 4: return launch_pair_expand<T, 4>(l, splits, total);
+    case 8: return launch_pair_expand<T, 8>(l, splits, total);
+  }
+  if constexpr (sizeof(T) == 2) {
+    switch (l.a->r / 8) {
+      case 1: return launch_pair_expand<T, 1>(l, splits, total);
+      case 3: return launch_pair_expand<T, 3>(l, splits, total);
+      case 5: return launch_pair_expand<T, 5>(l, splits, total);
+      case 6: return launch_pair_expand<T, 6>(l, splits, total);
+      case 7: return launch_pair_expand<T, 7>(l, splits, total);
+    }
+    return false;
+  } else {
+    return l.a->r == 64 ? launch_pair_expand<T, 16>(l, splits, total) : false;
+  }
+}
+
+}  // namespace
+
+void pair_trace_set(void* buf) {
+#ifdef MLORA_TRACE
+  (void)hipMemcpyToSymbol(HIP_SYMBOL(trace_buf), &buf, sizeof(buf));
+#else
+  (void)buf;
+#endif
+}
+
+bool pair_supported(const MloraAddArgs* a) {
+  const int64_t e = element_bytes(a->dtype);
+  if (a->k <= 0 || (a->k * e) % kChunk || !a->plan) return false;
+  if (e == 2 ? !padded_rank(a->r) : !exact_rank(a->r)) return false;
+  // 32-bit offsets of the x rows, A rows and B pieces; 16-byte loads of x and B, four columns of y at a time
+  if (a->num_tokens * (a->x_stride * e) >= (1ll << 32) || a->r * (a->k * e) >= (1ll << 32)) return false;
+  if ((a->x_stride * e) % 16 || a->y_stride % 4 || !a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255)) return false;
+  if ((reinterpret_cast<uintptr_t>(a->x) & 15) || (reinterpret_cast<uintptr_t>(a->y) & (4 * e - 1))) return false;
+  for (int i = 0; i < a->num_slices; ++i) {
+    const MloraSlice& s = a->slices[i];
+    if (s.n <= 0 || s.n % 4 || s.y_col % 4 || (reinterpret_cast<uintptr_t>(s.a) & 15) || (reinterpret_cast<uintptr_t>(s.b) & 15)) return false;
+    if (s.n * (a->r * e) >= (1ll << 32)) return false;
+  }
+  int total = 0;
+  for (int i = 0; i < a->num_slices; ++i) total += (a->slices[i].n + 511) / 512;
+  return total <= kMaxSplits && partials_room(a) >= part_bytes(a, plan_layout(a->num_tokens, a->num_slots));
+}
+
+int launch_pair(const MloraAddArgs* a) {
+  PairLaunch l;
+  l.a = a;
+  l.lay = plan_layout(a->num_tokens, a->num_slots);
+  const int segs = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+  const int by_tokens = (a->num_tokens + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL;
+  const int tiles = segs > by_tokens ? segs : by_tokens;  // about the number of tiles in use
+  const int kchunks = static_cast<int>(static_cast<int64_t>(a->k) * element_bytes(a->dtype) / kChunk);
+  const size_t room = partials_room(a) / part_bytes(a, l.lay);
+  // K parts: workgroups for most compute units, no more (every column range of the second launch
+  // takes in every part's sums), and a chunk per wavefront at least
+  int want = pair_knobs().kparts;
+  l.parts_log2 = 0;
+  while ((2u << l.parts_log2) <= room && (2 << l.parts_log2) <= kMaxParts && (2 << l.parts_log2) * kPairWaves <= kchunks &&
+         (want > 0 ? (2 << l.parts_log2) <= want : (tiles * a->num_slices << l.parts_log2) < pair_knobs().wgs))
+    ++l.parts_log2;
+  l.sp = pair_knobs().sp > 0 ? pair_knobs().sp : 1;
+  ExpandSplits splits;
+  int nt, total;
+  for (;; l.sp = 2) {
+    nt = l.sp * 64 * kPairWaves;
+    total = 0;
+    for (int i = 0; i < a->num_slices; ++i) total += (a->slices[i].n + nt - 1) / nt;
+    if (total <= kMaxSplits || l.sp == 2) break;
+  }
+  int s = 0;
+  for (int i = 0; i < a->num_slices; ++i)
+    for (int n0 = 0; n0 < a->slices[i].n; n0 += nt) {
+      ExpandSplit& d = splits.split[s++];
+      d.b = a->slices[i].b; d.n = a->slices[i].n; d.y_col = a->slices[i].y_col; d.slice = i; d.pad = 0;
+      d.n0 = n0; d.n1 = n0 + nt < a->slices[i].n ? n0 + nt : a->slices[i].n;
+    }
+  if (l.lay.cap_small == 0) return 0;
+  bool ok;
+  if (a->dtype == MLORA_DTYPE_BF16) ok = launch_pair_type<__bf16>(l, splits, total);
+  else if (a->dtype == MLORA_DTYPE_F16) ok = launch_pair_type<_Float16>(l, splits, total);
+  else ok = launch_pair_type<float>(l, splits, total);
+  if (!ok) { set_error("mlora_add_lora(pair): unsupported rank %d", a->r); return MLORA_E_UNSUPPORTED; }
+  return check_launch("mlora_add_lora(shrink and expand launches)");
+}
+
+}  // namespace mlora

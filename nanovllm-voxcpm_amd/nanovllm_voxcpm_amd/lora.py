@@ -227,7 +227,8 @@ class HipLoRABackend:
         return plan
 
     def _new_scratch(self, device: torch.device, nbytes: int, stream: int | None) -> torch.Tensor:
-        buf = torch.empty(max(nbytes, 4 << 20), dtype=torch.uint8, device=device)
+        # (some room beyond what every form needs: batches of few tokens cut K into more parts with it)
+        buf = torch.empty(nbytes + (8 << 20), dtype=torch.uint8, device=device)
         _hip.workspace_init(buf, stream)  # one kernel, once per buffer: head cleared, signature written
         return buf
 
