@@ -257,7 +257,11 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
     const bool small_tiles = mfma_supported(a) && decode_supported(a);
     const bool two_launches = mfma_supported(a) && sgmv_supported(a) && sgmv_workspace_ok(a);
     const bool one_launch = mfma_supported(a) && wide_supported(a) && wide_pays(a) && !knobs().no_wide;
-    if (!vec) form = MLORA_FORM_TOKEN;
+    // (fp32 rows and anything else the 128-bit kernels for 16-bit elements do not take: one workgroup per token,
+    // which fetches A and B per token and walks K in chained steps, except where the pair of launches has the
+    // element type: config 1's batch, 64 tokens over 4 slots, rank 16, fp32, qkv / o / gate_up / down 25 / 25 / 27 /
+    // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches)
+    if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
     else if (one_launch && !(small_tiles && small_batch(a, true))) form = MLORA_FORM_WIDE;
     else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false))) form = MLORA_FORM_SGMV;
     else if (small_tiles) form = MLORA_FORM_SPLIT;

@@ -96,6 +96,16 @@ class _UnavailableBackend:
 
 
 _VECTOR_RANKS = (8, 16, 24, 32, 40, 48, 56, 64)  # rows of B start on 16-byte boundaries and an instance of the kernels covers them
+_VECTOR_RANKS_F32 = (8, 16, 32, 64)
+
+
+def _vector_shape(dtype: torch.dtype, rank: int, k: int) -> bool:
+    """Element type, rank and K for which the library has a form that walks a plan."""
+    if dtype == torch.float32:
+        return rank in _VECTOR_RANKS_F32 and k % 32 == 0  # the two-launch form over 16-token tiles
+    return dtype in (torch.float16, torch.bfloat16) and rank in _VECTOR_RANKS and k % 8 == 0
+
+
 _PLAN_ATTR = "_mlora_segment_plans"
 _CONTEXT_PLANS_ATTR = "_mlora_context_plans"  # plan table of the LoRAContext a metadata object was made from
 
@@ -291,11 +301,9 @@ class HipLoRABackend:
     def _vectorisable(x: torch.Tensor, y: torch.Tensor, a_list, b_list, cols) -> bool:
         """Host mirror of the library's test for the 128-bit kernels (a plan is only built when
         it can be used)."""
-        if x.dtype not in (torch.float16, torch.bfloat16):
+        if not _vector_shape(x.dtype, a_list[0].size(-2), x.size(1)):
             return False
-        if a_list[0].size(-2) not in _VECTOR_RANKS:
-            return False
-        if x.size(1) % 8 or x.stride(0) % 8 or y.stride(0) % 8 or x.data_ptr() % 16 or y.data_ptr() % 16:
+        if x.stride(0) % 8 or y.stride(0) % 8 or x.data_ptr() % 16 or y.data_ptr() % 16:
             return False
         for a, b, col in zip(a_list, b_list, cols):
             if b.size(1) % 8 or col % 8 or a.data_ptr() % 16 or b.data_ptr() % 16:
@@ -338,7 +346,7 @@ class HipLoRABackend:
         args = site.args = _hip.MloraAddArgs()
         args.k, args.r, args.num_slots, args.num_slices, args.dtype = k, rank, slots, len(a_list), _hip.dtype_code(dt)
         args.form = _hip.FORMS[self.form]
-        col, ok = 0, dt in (torch.float16, torch.bfloat16) and rank in _VECTOR_RANKS and k % 8 == 0
+        col, ok = 0, _vector_shape(dt, rank, k)
         for i, (a, b, w) in enumerate(zip(a_list, b_list, widths)):
             sl = args.slices[i]
             sl.a, sl.b, sl.n, sl.y_col = a.data_ptr(), b.data_ptr(), w, col
