@@ -290,6 +290,9 @@ typedef struct MloraMetaArgs {
 } MloraMetaArgs;
 
 int mlora_meta_build(const MloraMetaArgs* args);
+/* Several independent batches (the domains of a step) in one launch, all on the stream of the first. */
+#define MLORA_META_BATCH 4
+int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count);
 
 /* Fused slot install:  A[slot, :, :] = 0; A[slot, 0:rank, :] = a_src[0:rank, :];
  * B[slot, :, :] = 0; B[slot, :, 0:rank] = b_src[:, 0:rank] * scaling  in one launch.

@@ -29,14 +29,25 @@ struct MetaParams {
   int32_t* scalars;
 };
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    int n = __shfl_up(v, o, kWave);
-    if (lane >= o) v += n;
-  }
+// Inclusive scan over the wavefront with DPP moves (within rows of sixteen, then row to row): six steps
+// of a few cycles where shuffles through the LDS unit take over a hundred each.
+template <typename F> __device__ __forceinline__ int wave_incl(int v, F&& op) {
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
   return v;
 }
+__device__ __forceinline__ int wave_incl_scan(int v) { return wave_incl(v, [](int a, int b) { return a + b; }); }
+__device__ __forceinline__ int wave_max_of_nonnegative(int v) {
+  return __builtin_amdgcn_readlane(wave_incl(v, [](int a, int b) { return a > b ? a : b; }), kWave - 1);
+}
+
+// A barrier for what passes through LDS: it does not wait for the global stores on their way, as
+// __syncthreads does (a store's acknowledgement is most of a microsecond away).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Largest b in [0, n) with arr[b] <= q, for a non-decreasing arr[0..n].
 __device__ __forceinline__ int find_bucket(const int* arr, int n, int q) {
@@ -48,8 +59,17 @@ __device__ __forceinline__ int find_bucket(const int* arr, int n, int q) {
   return lo;
 }
 
-__global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
+// Several batches share a launch: each has a workgroup of its own.
+struct MetaTable { MetaParams p[MLORA_META_BATCH]; };
+
+// What bounds it: the latency of one workgroup's chain - slot ids from memory, histogram, scans, stores -
+// and the 1.6 us of being a launch at all.  A decode step runs it for the batch's context, for the graph
+// buffers of every domain and for the plan, so at one to 512 tokens it is the microseconds of the chain
+// that count: the slot ids are requested once and first of all, scans go through DPP moves, and no
+// barrier waits for stores unless something is stored to twice.
+__global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
   extern __shared__ int lds[];
+  const MetaParams p = table.p[blockIdx.x];
   const int NB = p.L + 1;  // bucket b holds slot b - 1; bucket 0 is "no LoRA"
   int* hist = lds;                     // [waves][NB]: per-wave counts, later running write cursors
   int* total = hist + kMetaWaves * NB; // [NB]
@@ -65,10 +85,6 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int T = p.T, L = p.L;
 
-  for (int i = tid; i < kMetaWaves * NB; i += kMetaThreads) hist[i] = 0;
-  if (tid == 0) { s_bad = 0; s_max = 0; }
-  __syncthreads();
-
   // Each wave owns one contiguous span of tokens, so wave order equals token order.
   int span = (T + kMetaWaves - 1) / kMetaWaves;
   span = (span + kWave - 1) & ~(kWave - 1);
@@ -78,14 +94,21 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
   // A wavefront walks its span in steps of 64 tokens with the slot ids of the next four steps
   // requested ahead: a step is a few hundred cycles of work and a request to memory takes several
   // times that, so with one step in flight the walk runs at the pace of the memory's latency.
+  // Both walks start from the same first four steps, held in registers.
   constexpr int kAhead = 4;
+  int held[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) {
+    const int t = beg + j * kWave + lane;
+    held[j] = t < end ? p.tts[t] : -1;
+  }
+  for (int i = tid; i < kMetaWaves * NB; i += kMetaThreads) hist[i] = 0;
+  if (tid == 0) { s_bad = 0; s_max = 0; }
+  lds_barrier();
   auto walk = [&](auto&& step) {
     int q[kAhead];
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const int t = beg + j * kWave + lane;
-      q[j] = t < end ? p.tts[t] : -1;
-    }
+    for (int j = 0; j < kAhead; ++j) q[j] = held[j];
     for (int base = beg; base < end; base += kAhead * kWave) {
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) {
@@ -107,19 +130,21 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
   if (p.padded_tts) {
     for (int i = tid; i < p.padded_len; i += kMetaThreads) p.padded_tts[i] = i < T ? p.tts[i] : -1;
   }
-  __syncthreads();
+  lds_barrier();
 
   // Per bucket: turn the per-wave counts into exclusive prefixes over waves.
   for (int b = tid; b < NB; b += kMetaThreads) {
-    int run = 0;
+    int c[kMetaWaves], run = 0;
+#pragma unroll
+    for (int w = 0; w < kMetaWaves; ++w) c[w] = hist[w * NB + b];
+#pragma unroll
     for (int w = 0; w < kMetaWaves; ++w) {
-      int c = hist[w * NB + b];
       hist[w * NB + b] = run;
-      run += c;
+      run += c[w];
     }
     total[b] = run;
   }
-  __syncthreads();
+  lds_barrier();
 
   // Wave 0: exclusive scans over the buckets.
   const int b0 = p.no_lora_bucket ? 0 : 1;  // first bucket of the compact arrays
@@ -137,8 +162,8 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
       int v3 = is_short ? 0 : nsmall;
       int v4 = is_short ? 0 : (c + MLORA_TILE_BIG - 1) / MLORA_TILE_BIG;
       int v5 = nsmall > 1 ? nsmall - 1 : 0;
-      int i0 = wave_incl_scan(v0, lane), i1 = wave_incl_scan(v1, lane), i2 = wave_incl_scan(v2, lane);
-      int i3 = wave_incl_scan(v3, lane), i4 = wave_incl_scan(v4, lane), i5 = wave_incl_scan(v5, lane);
+      int i0 = wave_incl_scan(v0), i1 = wave_incl_scan(v1), i2 = wave_incl_scan(v2);
+      int i3 = wave_incl_scan(v3), i4 = wave_incl_scan(v4), i5 = wave_incl_scan(v5);
       if (b < NB) {
         off[b] = run0 + i0 - v0;
         cidx[b] = run1 + i1 - v1;
@@ -147,16 +172,14 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
         ts_big[b] = run4 + i4 - v4;
         ts_over[b] = run5 + i5 - v5;
       }
-      run0 += __shfl(i0, kWave - 1, kWave);
-      run1 += __shfl(i1, kWave - 1, kWave);
-      run2 += __shfl(i2, kWave - 1, kWave);
-      run3 += __shfl(i3, kWave - 1, kWave);
-      run4 += __shfl(i4, kWave - 1, kWave);
-      run5 += __shfl(i5, kWave - 1, kWave);
+      run0 += __builtin_amdgcn_readlane(i0, kWave - 1);
+      run1 += __builtin_amdgcn_readlane(i1, kWave - 1);
+      run2 += __builtin_amdgcn_readlane(i2, kWave - 1);
+      run3 += __builtin_amdgcn_readlane(i3, kWave - 1);
+      run4 += __builtin_amdgcn_readlane(i4, kWave - 1);
+      run5 += __builtin_amdgcn_readlane(i5, kWave - 1);
       nlong += __popcll(__ballot(b < NB && !is_short));
-      int m = c;
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) { int n = __shfl_xor(m, o, kWave); m = n > m ? n : m; }
+      const int m = wave_max_of_nonnegative(c);
       mx = m > mx ? m : mx;
     }
     if (lane == 0) {
@@ -165,7 +188,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
       s_nlong = nlong;
     }
   }
-  __syncthreads();
+  lds_barrier();
 
   const int n_lora = off[NB];
   // With the "no LoRA" bucket requested and no LoRA token at all, the reference's builder returns
@@ -227,8 +250,10 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
     if (p.compact_offsets) p.compact_offsets[i + 1] = 0;
   }
 
-  // Tile lists of the plan.  A small-tile record starts with its header and zeroed row entries;
-  // the scatter below fills all sixteen (the tile's tokens, repeated cyclically past its count).
+  // Tile lists of the plan.  A small tile's header is written here; the scatter below fills all sixteen
+  // row entries (the tile's tokens, repeated cyclically past its count), so only the records of slots
+  // without tokens have theirs zeroed: no word of a small-tile record is stored to twice.
+  constexpr int kRecordTail = (MLORA_SMALL_TILE_ROWS + MLORA_TILE_SMALL) / 4;  // 128-bit words of header and rows
   i32x4* small = p.plan ? reinterpret_cast<i32x4*>(p.plan + lay.small_off) : nullptr;
   // place of big tile q (in slot order) in the list: runs of `run` consecutive tiles go to the
   // blocks (XCDs) in turn
@@ -237,7 +262,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
   if (p.plan) {
     i32x4* big = reinterpret_cast<i32x4*>(p.plan + lay.big_off);
     for (int q = tid; q < lay.cap_big; q += kMetaThreads) big[q] = i32x4{-1, 0, 0, 0};
-    __syncthreads();  // (a place is cleared by one thread and may be filled by another)
+    if (n_big > 0) __syncthreads();  // (a place is cleared by one thread and may be filled by another)
     for (int q = tid; q < n_short + n_long; q += kMetaThreads) {
       const bool is_short = q < n_short;
       const int* ts = is_short ? ts_short : ts_long;
@@ -248,7 +273,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
       i32x4* rec = small + q * (MLORA_SMALL_TILE_WORDS / 4);
       rec[0] = i32x4{b - 1, left < MLORA_TILE_SMALL ? left : MLORA_TILE_SMALL, off[b] + j * MLORA_TILE_SMALL, 0};
 #pragma unroll
-      for (int w = 1; w < MLORA_SMALL_TILE_WORDS / 4; ++w) rec[w] = i32x4{0, 0, 0, 0};
+      for (int w = kRecordTail; w < MLORA_SMALL_TILE_WORDS / 4; ++w) rec[w] = i32x4{0, 0, 0, 0};
     }
     for (int q = tid; q < n_big; q += kMetaThreads) {
       int b = find_bucket(ts_big, NB, q);
@@ -278,11 +303,15 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaParams p) {
       }
       i32x4* rec = byslot + q * (MLORA_SMALL_TILE_WORDS / 4);
       rec[0] = head;
+      if (head[1] == 0) {
 #pragma unroll
-      for (int w = 1; w < MLORA_SMALL_TILE_WORDS / 4; ++w) rec[w] = i32x4{0, 0, 0, 0};
+        for (int w = 1; w < kRecordTail; ++w) rec[w] = i32x4{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int w = kRecordTail; w < MLORA_SMALL_TILE_WORDS / 4; ++w) rec[w] = i32x4{0, 0, 0, 0};
     }
+    if (n_big > 0) __syncthreads();  // (the row lists of the big tiles were cleared, the scatter fills them)
   }
-  __syncthreads();
 
   // Stable scatter: every wave walks its span again in token order.  The rank of a token
   // among the equal keys of its 64-token step is counted lane against lane; the running cursor
@@ -352,8 +381,9 @@ extern "C" size_t mlora_plan_workspace_bytes(int32_t num_tokens, int32_t max_slo
   return static_cast<size_t>(plan_layout(num_tokens, max_slots).total_words) * sizeof(int32_t);
 }
 
-extern "C" int mlora_meta_build(const MloraMetaArgs* a) {
-  if (!a) { set_error("mlora_meta_build: NULL args"); return MLORA_E_INVALID; }
+namespace {
+
+int check_meta(const MloraMetaArgs* a) {
   if (a->num_tokens < 0 || a->max_slots < 0 || a->compact_capacity < 0 || a->padded_len < 0) {
     set_error("mlora_meta_build: negative size"); return MLORA_E_INVALID;
   }
@@ -366,8 +396,7 @@ extern "C" int mlora_meta_build(const MloraMetaArgs* a) {
     set_error("mlora_meta_build: padded_len=%d is shorter than num_tokens=%d", a->padded_len, a->num_tokens);
     return MLORA_E_INVALID;
   }
-  const bool wants_compact = a->compact_ids || a->compact_counts || a->compact_offsets;
-  if (wants_compact) {
+  if (a->compact_ids || a->compact_counts || a->compact_offsets) {
     const int t = a->num_tokens, l = a->max_slots + (a->no_lora_bucket ? 1 : 0);
     const int need = t < l ? t : l;
     if (a->compact_capacity < need) {
@@ -375,16 +404,42 @@ extern "C" int mlora_meta_build(const MloraMetaArgs* a) {
       return MLORA_E_INVALID;
     }
   }
-  MetaParams p;
-  p.tts = a->token_to_slot; p.T = a->num_tokens; p.L = a->max_slots; p.no_lora_bucket = a->no_lora_bucket ? 1 : 0;
-  p.plan = a->plan; p.sorted_idx = a->sorted_idx;
-  p.compact_ids = a->compact_ids; p.compact_counts = a->compact_counts; p.compact_offsets = a->compact_offsets;
-  p.compact_capacity = wants_compact ? a->compact_capacity : 0;
-  p.dense_counts = a->dense_counts; p.dense_offsets = a->dense_offsets;
-  p.padded_tts = a->padded_token_to_slot; p.padded_len = a->padded_len;
-  p.scalars = a->scalars;
-  const int NB = p.L + 1;
-  const size_t lds = sizeof(int) * (static_cast<size_t>(kMetaWaves + 1) * NB + 6 * (NB + 1));
-  hipLaunchKernelGGL(meta_kernel, dim3(1), dim3(kMetaThreads), lds, static_cast<hipStream_t>(a->stream), p);
-  return check_launch("mlora_meta_build");
+  return 0;
+}
+
+}  // namespace
+
+extern "C" int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count) {
+  if (count < 0 || (count > 0 && !list)) { set_error("mlora_meta_build: NULL args"); return MLORA_E_INVALID; }
+  for (int i = 0; i < count; ++i) {
+    if (int rc = check_meta(list + i)) return rc;
+  }
+  for (int first = 0; first < count; first += MLORA_META_BATCH) {
+    const int n = count - first < MLORA_META_BATCH ? count - first : MLORA_META_BATCH;
+    MetaTable table;
+    size_t lds = 0;
+    for (int i = 0; i < n; ++i) {
+      const MloraMetaArgs* a = list + first + i;
+      MetaParams& p = table.p[i];
+      p.tts = a->token_to_slot; p.T = a->num_tokens; p.L = a->max_slots; p.no_lora_bucket = a->no_lora_bucket ? 1 : 0;
+      p.plan = a->plan; p.sorted_idx = a->sorted_idx;
+      p.compact_ids = a->compact_ids; p.compact_counts = a->compact_counts; p.compact_offsets = a->compact_offsets;
+      p.compact_capacity = a->compact_ids || a->compact_counts || a->compact_offsets ? a->compact_capacity : 0;
+      p.dense_counts = a->dense_counts; p.dense_offsets = a->dense_offsets;
+      p.padded_tts = a->padded_token_to_slot; p.padded_len = a->padded_len;
+      p.scalars = a->scalars;
+      const int NB = p.L + 1;
+      const size_t need = sizeof(int) * (static_cast<size_t>(kMetaWaves + 1) * NB + 6 * (NB + 1));
+      lds = need > lds ? need : lds;
+    }
+    for (int i = n; i < MLORA_META_BATCH; ++i) table.p[i] = table.p[0];  // (not in the grid)
+    hipLaunchKernelGGL(meta_kernel, dim3(n), dim3(kMetaThreads), lds, static_cast<hipStream_t>(list[0].stream), table);
+    if (int rc = check_launch("mlora_meta_build")) return rc;
+  }
+  return 0;
+}
+
+extern "C" int mlora_meta_build(const MloraMetaArgs* a) {
+  if (!a) { set_error("mlora_meta_build: NULL args"); return MLORA_E_INVALID; }
+  return mlora_meta_build_many(a, 1);
 }

@@ -60,6 +60,7 @@ EXPORTS = (
     "mlora_expand",
     "mlora_plan_workspace_bytes",
     "mlora_meta_build",
+    "mlora_meta_build_many",
     "mlora_install_slot",
     "mlora_stream_capture_id",
     "mlora_abi_version",
@@ -222,6 +223,8 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(args)]
         fn.restype = C.c_int
+    lib.mlora_meta_build_many.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32]
+    lib.mlora_meta_build_many.restype = C.c_int
     lib.mlora_plan_workspace_bytes.argtypes = [C.c_int32, C.c_int32]
     lib.mlora_plan_workspace_bytes.restype = C.c_size_t
     lib.mlora_add_workspace_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32]
@@ -284,24 +287,41 @@ def load_error() -> str | None:
     return None
 
 
+_FASTCALL: object = ()  # () until the import was tried
+
+
 def load_fastcall():
-    """The module with the C++ host path of the usual add_lora call (csrc/fastcall.cpp, built beside
-    the library by ``make fastcall``), or None where it is not built or does not load: the Python
-    path then does every call.  It launches nothing itself: it calls the library's entry points."""
-    try:
-        from nanovllm_voxcpm_amd import _mlora_fastcall
-    except ImportError:
-        return None
-    return _mlora_fastcall
+    """The module with the C++ host paths (csrc/fastcall.cpp, built beside the library by ``make
+    fastcall``), or None where it is not built or does not load: the Python paths then do every
+    call.  It launches nothing itself: it calls the library's entry points."""
+    global _FASTCALL
+    if _FASTCALL == ():
+        try:
+            from nanovllm_voxcpm_amd import _mlora_fastcall
+        except ImportError:
+            _mlora_fastcall = None
+        _FASTCALL = _mlora_fastcall
+    return _FASTCALL
 
 
 def entry_point_addresses() -> tuple[int, int] | None:
     """Addresses of mlora_add_lora and mlora_add_workspace_bytes in the loaded library, None without it."""
     try:
-        lib = load()
+        load()
     except RuntimeError:
         return None
-    return C.cast(lib.mlora_add_lora, C.c_void_p).value, C.cast(lib.mlora_add_workspace_bytes, C.c_void_p).value
+    return entry_point("mlora_add_lora"), entry_point("mlora_add_workspace_bytes")
+
+
+_ADDRESSES: dict[str, int] = {}
+
+
+def entry_point(name: str) -> int:
+    """Address of a function of the loaded library."""
+    address = _ADDRESSES.get(name)
+    if address is None:
+        address = _ADDRESSES[name] = C.cast(getattr(load(), name), C.c_void_p).value
+    return address
 
 
 def _check(rc: int, what: str) -> None:
@@ -562,10 +582,6 @@ def expand(
         _check(lib.mlora_expand(C.byref(args)), "mlora_expand")
 
 
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return t.data_ptr() if t is not None else None
-
-
 def meta_build(
     token_to_slot: torch.Tensor,
     max_slots: int,
@@ -583,29 +599,43 @@ def meta_build(
     scalars: torch.Tensor | None = None,
 ) -> None:
     """One launch of the on-device counting sort; every output tensor is optional."""
+    meta_build_many([dict(token_to_slot=token_to_slot, max_slots=max_slots, no_lora_bucket=no_lora_bucket, plan=plan, sorted_idx=sorted_idx,
+                          compact_ids=compact_ids, compact_counts=compact_counts, compact_offsets=compact_offsets,
+                          compact_capacity=compact_capacity, dense_counts=dense_counts, dense_offsets=dense_offsets,
+                          padded_token_to_slot=padded_token_to_slot, scalars=scalars)])
+
+
+_META_OUTPUTS = ("plan", "sorted_idx", "compact_ids", "compact_counts", "compact_offsets", "dense_counts", "dense_offsets",
+                 "padded_token_to_slot", "scalars")
+
+
+def meta_build_many(batches: list[dict]) -> None:
+    """The counting sorts of several batches (keyword arguments of ``meta_build`` each, all on one
+    device) in one launch."""
     lib = load()
-    _require_cuda(token_to_slot, "token_to_slot")
-    if token_to_slot.dtype != torch.int32 or not token_to_slot.is_contiguous():
-        raise ValueError("token_to_slot must be a contiguous int32 tensor")
-    args = MloraMetaArgs()
-    args.stream = _stream(token_to_slot.device)
-    args.token_to_slot = token_to_slot.data_ptr()
-    args.num_tokens = token_to_slot.numel()
-    args.max_slots = max_slots
-    args.no_lora_bucket = 1 if no_lora_bucket else 0
-    args.plan = _ptr(plan)
-    args.sorted_idx = _ptr(sorted_idx)
-    args.compact_ids = _ptr(compact_ids)
-    args.compact_counts = _ptr(compact_counts)
-    args.compact_offsets = _ptr(compact_offsets)
-    args.compact_capacity = compact_capacity
-    args.dense_counts = _ptr(dense_counts)
-    args.dense_offsets = _ptr(dense_offsets)
-    args.padded_token_to_slot = _ptr(padded_token_to_slot)
-    args.padded_len = padded_token_to_slot.numel() if padded_token_to_slot is not None else 0
-    args.scalars = _ptr(scalars)
-    with _on(token_to_slot.device):
-        _check(lib.mlora_meta_build(C.byref(args)), "mlora_meta_build")
+    block = (MloraMetaArgs * len(batches))()
+    device = batches[0]["token_to_slot"].device
+    for args, batch in zip(block, batches):
+        slots = batch["token_to_slot"]
+        _require_cuda(slots, "token_to_slot")
+        if slots.dtype != torch.int32 or not slots.is_contiguous():
+            raise ValueError("token_to_slot must be a contiguous int32 tensor")
+        if slots.device != device:
+            raise ValueError("batches of one launch must live on one device")
+        args.token_to_slot = slots.data_ptr()
+        args.num_tokens = slots.numel()
+        args.max_slots = batch["max_slots"]
+        args.no_lora_bucket = 1 if batch.get("no_lora_bucket") else 0
+        for name in _META_OUTPUTS:
+            t = batch.get(name)
+            if t is not None:
+                setattr(args, name, t.data_ptr())
+        args.compact_capacity = batch.get("compact_capacity", 0)
+        padded = batch.get("padded_token_to_slot")
+        args.padded_len = padded.numel() if padded is not None else 0
+    block[0].stream = _stream(device)
+    with _on(device):
+        _check(lib.mlora_meta_build_many(block, len(batches)), "mlora_meta_build")
 
 
 def install_slot(

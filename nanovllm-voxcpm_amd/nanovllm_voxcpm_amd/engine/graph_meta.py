@@ -38,41 +38,56 @@ def make_graph_domain_buffers(
     }
 
 
-def copy_lora_domain_to_graph_vars(domain_vars: dict[str, torch.Tensor], context: LoRAContext) -> None:
-    """Refresh one domain's buffers in place for the batch described by ``context``."""
+def _refresh_of(domain_vars: dict[str, torch.Tensor], context: LoRAContext) -> dict:
+    """Arguments of the metadata launch that refreshes one domain's buffers for ``context``."""
     tts_buf = domain_vars["token_to_slot"]
     if not tts_buf.is_cuda:
         raise RuntimeError("graph LoRA buffers must live on the GPU; the HIP LoRA path has no host fallback")
-    buckets = domain_vars["num_tokens_per_slot"].numel()
     if context.no_lora_flag or context.token_to_slot is None:
-        source = torch.empty(0, dtype=torch.int32, device=tts_buf.device)
+        source = tts_buf[:0]
     else:
         source = as_slot_vector(context.token_to_slot)
         if source.numel() > tts_buf.numel():
             raise ValueError(f"{source.numel()} rows exceed the {tts_buf.numel()} rows captured for this graph")
-    _hip.meta_build(
-        source,
-        buckets - 1,
+    return dict(
+        token_to_slot=source,
+        max_slots=domain_vars["num_tokens_per_slot"].numel() - 1,
         sorted_idx=domain_vars["token_indices_sorted_by_slot"],
         dense_counts=domain_vars["num_tokens_per_slot"],
         dense_offsets=domain_vars["slot_start_offsets"],
         padded_token_to_slot=tts_buf,
     )
-    # Installed contexts that view these buffers were just rewritten in place (by a kernel, which
-    # no tensor version counter sees): what they derived from the old contents is dropped.
+
+
+def _drop_derived(buffers: set[int]) -> None:
+    """Installed contexts that view these slot vectors (addresses) were just rewritten in place (by a
+    kernel, which no tensor version counter sees): what they derived from the old contents is dropped."""
     for domain in LORA_DOMAINS:
         installed = get_lora_context(domain)
         view = installed.token_to_slot
-        if view is not None and view.is_cuda and view.numel() and view.data_ptr() == tts_buf.data_ptr():
+        if view is not None and view.is_cuda and view.numel() and view.data_ptr() in buffers:
             invalidate_lora_context(installed)
 
 
+def copy_lora_domain_to_graph_vars(domain_vars: dict[str, torch.Tensor], context: LoRAContext) -> None:
+    """Refresh one domain's buffers in place for the batch described by ``context``."""
+    _hip.meta_build(**_refresh_of(domain_vars, context))
+    _drop_derived({domain_vars["token_to_slot"].data_ptr()})
+
+
 def set_graph_lora_contexts(graph_vars: dict, contexts: dict[str, LoRAContext]) -> None:
-    """Refresh every domain and install contexts that view the fixed buffers."""
+    """Refresh every domain (one launch for all of them) and install contexts that view the fixed buffers."""
+    every = graph_vars["lora_domains"]
+    batches = [_refresh_of(every[domain], contexts[domain]) for domain in LORA_DOMAINS]
+    buffers = {every[domain]["token_to_slot"].data_ptr() for domain in LORA_DOMAINS}
+    if any(batch["token_to_slot"].data_ptr() in buffers for batch in batches):  # a context that views a buffer of the set
+        for batch in batches:
+            _hip.meta_build(**batch)
+    else:
+        _hip.meta_build_many(batches)
+    _drop_derived(buffers)
     for domain in LORA_DOMAINS:
-        context = contexts[domain]
-        domain_vars = graph_vars["lora_domains"][domain]
-        copy_lora_domain_to_graph_vars(domain_vars, context)
+        context, domain_vars = contexts[domain], every[domain]
         rows = 0 if context.token_to_slot is None else context.token_to_slot.size(0)
         set_lora_context(
             LoRAContext(

@@ -10,9 +10,13 @@ re-exported here under the reference's import path.
 
 from __future__ import annotations
 
+from array import array
+
+import numpy as np
 import torch
 
 from nanovllm_voxcpm_amd import _hip
+from nanovllm_voxcpm_amd.lora import attach_plan
 from nanovllm_voxcpm_amd.utils.context import LoRAContext
 
 
@@ -23,7 +27,7 @@ class LoRABatchPlan:
     four segment arrays may be left out and are then derived from ``token_to_slot`` on demand
     (the device path never reads them: the GPU sorts the tokens itself)."""
 
-    __slots__ = ("adapter_to_slot", "token_to_slot", "_sorted", "_active", "_counts", "_offsets")
+    __slots__ = ("adapter_to_slot", "_tokens", "_runs", "_sorted", "_active", "_counts", "_offsets")
 
     def __init__(
         self,
@@ -35,11 +39,34 @@ class LoRABatchPlan:
         slot_start_offsets: list[int] | None = None,
     ) -> None:
         self.adapter_to_slot = adapter_to_slot
-        self.token_to_slot = token_to_slot
+        self._tokens: list[int] | None = token_to_slot
+        self._runs: tuple[list[int], list[int]] | None = None
         self._sorted = token_indices_sorted_by_slot
         self._active = active_slot_ids
         self._counts = num_tokens_per_slot
         self._offsets = slot_start_offsets
+
+    @classmethod
+    def from_runs(cls, adapter_to_slot: dict[int, int], slots: list[int], counts: list[int]) -> "LoRABatchPlan":
+        """The plan of a batch known per sequence (slot id and token count): the per-token list, which
+        the device path does not need, is only written out when somebody asks for it."""
+        plan = cls(adapter_to_slot, None)  # type: ignore[arg-type]
+        plan._runs = (slots, counts)
+        return plan
+
+    @property
+    def token_to_slot(self) -> list[int]:
+        if self._tokens is None:
+            self._tokens = expand_token_to_slot(*self._runs)
+        return self._tokens
+
+    @token_to_slot.setter
+    def token_to_slot(self, tokens: list[int]) -> None:
+        self._tokens, self._runs = tokens, None
+
+    def runs(self) -> tuple[list[int], list[int]]:
+        """(slot ids, token counts) whose expansion is ``token_to_slot``."""
+        return self._runs if self._runs is not None else (self._tokens, [1] * len(self._tokens))
 
     def __repr__(self) -> str:
         return f"LoRABatchPlan(adapter_to_slot={self.adapter_to_slot!r}, token_to_slot={self.token_to_slot!r})"
@@ -51,12 +78,15 @@ class LoRABatchPlan:
 
     @property
     def num_lora_tokens(self) -> int:
-        return sum(1 for s in self.token_to_slot if s >= 0)
+        slots, counts = self.runs()
+        return sum([c for s, c in zip(slots, counts) if s >= 0])
 
     @property
     def active_slot_ids(self) -> list[int]:
         if self._active is None:
-            self._active = sorted({s for s in self.token_to_slot if s >= 0})
+            slots, counts = self.runs()
+            used = set(slots) if 0 not in counts else {s for s, c in zip(slots, counts) if c > 0}
+            self._active = sorted([s for s in used if s >= 0])
         return self._active
 
     @property
@@ -99,8 +129,11 @@ def expand_token_to_slot(adapter_slots: list[int], token_counts: list[int]) -> l
     return out
 
 
-def _upload_int32(values: list[int], device: torch.device | str) -> torch.Tensor:
-    host = torch.tensor(values, dtype=torch.int32, device="cpu", pin_memory=True)
+def _upload_runs(slots: list[int], counts: list[int], n: int, device: torch.device | str) -> torch.Tensor:
+    """The per-token slot ids on the device: expanded into a pinned buffer, one asynchronous copy."""
+    host = torch.empty(n, dtype=torch.int32, device="cpu", pin_memory=True)
+    ids = np.frombuffer(array("i", slots), dtype=np.int32)
+    host.numpy()[:] = ids if counts.count(1) == len(counts) else np.repeat(ids, counts)
     return host.to(device, non_blocking=True)
 
 
@@ -111,36 +144,37 @@ def build_lora_context_from_batch_plan(
     device: torch.device | str = "cuda",
 ) -> LoRAContext:
     """One H2D copy of the slot ids, one metadata launch, no device->host traffic: the array
-    lengths and the two host flags come from the host list the plan already holds."""
-    slots = plan.token_to_slot
-    tts = _upload_int32(slots, device) if slots else torch.empty(0, dtype=torch.int32, device=device)
+    lengths and the two host flags come from the host list the plan already holds.  A second
+    workgroup of the launch builds the segment plan of eager calls, which costs no time of its own."""
+    slots, counts = plan.runs()
+    n = sum(counts)
+    tts = _upload_runs(slots, counts, n, device) if n else torch.empty(0, dtype=torch.int32, device=device)
     active = plan.active_slot_ids
     if not active:
         return LoRAContext(token_to_slot=tts, no_lora_flag=True, num_active_loras=0)
-    n, n_lora, n_active = len(slots), plan.num_lora_tokens, len(active)
+    n_lora, n_active = plan.num_lora_tokens, len(active)
     if max_slots is None:
         max_slots = active[-1] + 1
     elif active[-1] >= max_slots:
         raise ValueError(f"slot id {active[-1]} is outside the {max_slots} resident slots")
     cap = min(n, max_slots)
     i32 = dict(dtype=torch.int32, device=tts.device)
-    # one allocation, four views
-    packed = torch.empty(n + 2 * cap + cap + 1, **i32)
-    sorted_idx, ids, counts, offsets = packed.split([n, cap, cap, cap + 1])
-    _hip.meta_build(
-        tts,
-        max_slots,
-        sorted_idx=sorted_idx,
-        compact_ids=ids,
-        compact_counts=counts,
-        compact_offsets=offsets,
-        compact_capacity=cap,
-    )
+    # one allocation, four views and the segment plan (its start on a 256-byte boundary)
+    head = (n + 2 * cap + cap + 1 + 63) & ~63
+    packed = torch.empty(head + _hip.plan_workspace_words(n, max_slots), **i32)
+    sorted_idx, ids, per_slot, offsets = packed[: n + 2 * cap + cap + 1].split([n, cap, cap, cap + 1])
+    workspace = packed[head:]
+    _hip.meta_build_many([
+        dict(token_to_slot=tts, max_slots=max_slots, sorted_idx=sorted_idx, compact_ids=ids, compact_counts=per_slot,
+             compact_offsets=offsets, compact_capacity=cap),
+        dict(token_to_slot=tts, max_slots=max_slots, plan=workspace),
+    ])
+    attach_plan(tts, workspace, max_slots)
     return LoRAContext(
         token_to_slot=tts,
         token_indices_sorted_by_slot=sorted_idx[:n_lora],
         active_slot_ids=ids[:n_active],
-        num_tokens_per_slot=counts[:n_active],
+        num_tokens_per_slot=per_slot[:n_active],
         slot_start_offsets=offsets[: n_active + 1],
         no_lora_flag=False,
         num_active_loras=n_active,

@@ -271,7 +271,7 @@ class LoRARuntime(_LoRAStateBase):
     ):
         """Admit the adapters of a batch and return its ``LoRABatchPlan`` (one adapter id, or
         None, and one token count per sequence)."""
-        from nanovllm_voxcpm_amd.engine.lora_manager import build_lora_batch_plan_from_token_to_slot, expand_token_to_slot
+        from nanovllm_voxcpm_amd.engine.lora_manager import LoRABatchPlan, build_lora_batch_plan_from_token_to_slot
 
         if len(adapter_ids) != len(token_counts):
             raise ValueError("adapter_ids and token_counts must have the same length")
@@ -279,14 +279,16 @@ class LoRARuntime(_LoRAStateBase):
             return build_lora_batch_plan_from_token_to_slot({}, [-1] * sum(token_counts))
         self._refresh_slot_states()
         adapter_to_slot: dict[int, int] = {}
-        for adapter_id in dict.fromkeys(a for a in adapter_ids if a is not None):  # first-use order
+        for adapter_id in dict.fromkeys(adapter_ids):  # first-use order
+            if adapter_id is None:
+                continue
             entry = self.get_entry(adapter_id)
             slot = self._slots[self._admit(entry, load_lora)]
             adapter_to_slot[adapter_id] = slot.slot_id
             entry.last_used_ts = slot.last_used_ts = self._tick()
             slot.resident_state = _residency(entry)
-        per_sequence = [adapter_to_slot.get(a, -1) if a is not None else -1 for a in adapter_ids]
-        return build_lora_batch_plan_from_token_to_slot(adapter_to_slot, expand_token_to_slot(per_sequence, token_counts))
+        slot_of = {None: -1, **adapter_to_slot}
+        return LoRABatchPlan.from_runs(adapter_to_slot, [slot_of[a] for a in adapter_ids], list(token_counts))
 
     def _admit(self, entry: LoRARuntimeEntry, load_lora: Callable[[int, LoRAModelPayload], None]) -> int:
         """Slot of ``entry``, loading it into an empty slot or over the least recently used idle

@@ -107,6 +107,15 @@ def _vector_shape(dtype: torch.dtype, rank: int, k: int) -> bool:
 
 
 _PLAN_ATTR = "_mlora_segment_plans"
+_SLOTS_PLAN_ATTR = "_mlora_plan"  # on a slot vector: the plan that was built together with it
+
+
+def attach_plan(slots: torch.Tensor, workspace: torch.Tensor, max_slots: int) -> None:
+    """Leave a segment plan with the slot vector it was built from (eagerly, on the current stream); it
+    serves eager calls until the vector is rewritten.  Inference tensors, whose rewrites nobody
+    counts, get none."""
+    if not slots.is_inference() and not _hip.stream_capture_id(slots.device):
+        setattr(slots, _SLOTS_PLAN_ATTR, (workspace, max_slots, slots._version))
 _CONTEXT_PLANS_ATTR = "_mlora_context_plans"  # plan table of the LoRAContext a metadata object was made from
 
 
@@ -233,7 +242,12 @@ class HipLoRABackend:
         if plan is None:
             if len(cache) >= 4:
                 cache.clear()
-            plan = cache[key] = build_segment_plan(tts, max_slots)
+            made = getattr(own, _SLOTS_PLAN_ATTR, None)
+            if made is not None and not capture and made[1:] == (max_slots, version) and own.numel() == tts.numel():
+                plan = SegmentPlan(workspace=made[0], token_to_slot=tts, num_tokens=tts.numel(), max_slots=max_slots)
+            else:
+                plan = build_segment_plan(tts, max_slots)
+            cache[key] = plan
         return plan
 
     def _new_scratch(self, device: torch.device, nbytes: int, stream: int | None) -> torch.Tensor:
