@@ -313,6 +313,16 @@ typedef struct MloraInstallArgs {
 } MloraInstallArgs;
 
 int mlora_install_slot(const MloraInstallArgs* args);
+/* Several targets (an adapter's, say) in as few launches as their table fits; all on one stream, no two
+ * of them the same slot of the same buffers.  Everything is checked before anything is launched.
+ * `states` (one per target, or NULL): vectors of the layer that are entered with the weights. */
+typedef struct MloraInstallState {
+  int32_t* rank;          /* [slots] or NULL: entry `slot` := rank */
+  void* scaling[2];       /* [slots] of `dtype` or NULL, both: entry `slot` := scaling */
+  int32_t dtype;
+} MloraInstallState;
+
+int mlora_install_slots(const MloraInstallArgs* list, const MloraInstallState* states, int32_t count);
 
 /* Identifier of the graph capture in progress on `stream`, 0 when the stream is not
  * capturing.  No counterpart in the reference: lets a host-side cache tell work recorded

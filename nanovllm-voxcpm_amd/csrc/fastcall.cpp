@@ -21,6 +21,7 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -351,7 +352,258 @@ PyObject* py_counters(PyObject*, PyObject* cap) {
   return Py_BuildValue("(LL)", s->handled, s->passed_on);
 }
 
+// ---- the low-level ops -------------------------------------------------------------------------------
+// shrink(address of mlora_shrink, inputs, lora_a weights, output, slot vector, scaling) and
+// expand(address of mlora_expand, inputs, lora_b weights, output, slot vector, offset, add): the usual call
+// of lora_ops.lora_shrink / lora_expand, checked and enqueued; NOT_HANDLED for anything that
+// needs a view, a copy, a conversion or an exception.
+
+// The weights of a call: contiguous [slots, rows, cols] tensors of one element type on `dev`.
+bool op_weights(PyObject* list, int dev, c10::ScalarType dtype, Py_ssize_t* n, const at::Tensor* (&w)[MLORA_MAX_SLICES]) {
+  if (!(PyList_Check(list) || PyTuple_Check(list))) return false;
+  *n = PySequence_Fast_GET_SIZE(list);
+  if (*n < 1 || *n > MLORA_MAX_SLICES) return false;
+  for (Py_ssize_t i = 0; i < *n; ++i) {
+    PyObject* o = PySequence_Fast_GET_ITEM(list, i);
+    if (!THPVariable_Check(o)) return false;
+    w[i] = &THPVariable_Unpack(o);
+    if (w[i]->dim() != 3 || !w[i]->is_contiguous() || w[i]->scalar_type() != dtype || !on_device(*w[i], dev)) return false;
+  }
+  return true;
+}
+
+int code_of(c10::ScalarType t) {
+  return t == c10::ScalarType::Float ? MLORA_DTYPE_F32 : t == c10::ScalarType::Half ? MLORA_DTYPE_F16 : t == c10::ScalarType::BFloat16 ? MLORA_DTYPE_BF16 : -1;
+}
+
+bool op_slots(const at::Tensor& slots, int64_t rows, int dev) {
+  return slots.scalar_type() == c10::ScalarType::Int && slots.dim() == 1 && slots.is_contiguous() && slots.numel() >= rows && on_device(slots, dev);
+}
+
+long op_shrink(PyObject* const* args) {
+  if (!THPVariable_Check(args[1]) || !THPVariable_Check(args[3]) || !THPVariable_Check(args[4])) return kNotHandled;
+  const at::Tensor &x = THPVariable_Unpack(args[1]), &out = THPVariable_Unpack(args[3]), &slots = THPVariable_Unpack(args[4]);
+  if (x.dim() != 2 || !x.is_cuda() || x.stride(1) != 1 || x.size(0) < 1 || x.size(0) > INT32_MAX) return kNotHandled;
+  const int dev = x.device().index();
+  const at::Tensor* w[MLORA_MAX_SLICES];
+  Py_ssize_t n;
+  if (!op_weights(args[2], dev, x.scalar_type(), &n, w) || !op_slots(slots, x.size(0), dev)) return kNotHandled;
+  for (Py_ssize_t i = 1; i < n; ++i)
+    if (w[i]->sizes() != w[0]->sizes()) return kNotHandled;
+  const int dtype = code_of(x.scalar_type()), out_dtype = code_of(out.scalar_type());
+  if (dtype < 0 || out_dtype < 0 || w[0]->size(2) != x.size(1) || out.dim() != 3 || !out.is_contiguous() || !on_device(out, dev) || out.size(0) != n ||
+      out.size(1) != x.size(0) || out.size(2) != w[0]->size(1) || c10::hip::current_device() != dev)
+    return kNotHandled;
+  MloraShrinkArgs a = {};
+  a.scaling = static_cast<float>(PyFloat_AsDouble(args[5]));
+  if (PyErr_Occurred()) return kNotHandled;
+  a.stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
+  a.x = x.data_ptr(); a.out = out.data_ptr(); a.x_stride = x.stride(0);
+  a.token_to_slot = static_cast<const int32_t*>(slots.data_ptr());
+  a.num_tokens = static_cast<int32_t>(x.size(0)); a.k = static_cast<int32_t>(x.size(1));
+  a.r = static_cast<int32_t>(w[0]->size(1)); a.num_slots = static_cast<int32_t>(w[0]->size(0)); a.num_slices = static_cast<int32_t>(n);
+  a.dtype = dtype; a.out_dtype = out_dtype;
+  for (Py_ssize_t i = 0; i < n; ++i) a.a[i] = w[i]->data_ptr();
+  const auto fn = reinterpret_cast<int (*)(const MloraShrinkArgs*)>(PyLong_AsSize_t(args[0]));
+  return PyErr_Occurred() ? kNotHandled : fn(&a);
+}
+
+long op_expand(PyObject* const* args) {
+  if (!THPVariable_Check(args[1]) || !THPVariable_Check(args[3]) || !THPVariable_Check(args[4])) return kNotHandled;
+  const at::Tensor &h = THPVariable_Unpack(args[1]), &y = THPVariable_Unpack(args[3]), &slots = THPVariable_Unpack(args[4]);
+  if (h.dim() != 3 || !h.is_cuda() || !h.is_contiguous() || h.size(1) < 1 || h.size(1) > INT32_MAX) return kNotHandled;
+  const int dev = h.device().index();
+  const at::Tensor* w[MLORA_MAX_SLICES];
+  Py_ssize_t n;
+  if (!op_weights(args[2], dev, y.scalar_type(), &n, w) || n != h.size(0) || !op_slots(slots, h.size(1), dev)) return kNotHandled;
+  const int dtype = code_of(y.scalar_type()), h_dtype = code_of(h.scalar_type());
+  if (dtype < 0 || h_dtype < 0 || y.dim() != 2 || y.stride(1) != 1 || y.size(0) < h.size(1) || !on_device(y, dev) || c10::hip::current_device() != dev)
+    return kNotHandled;
+  MloraExpandArgs a = {};
+  a.offset_start = static_cast<int32_t>(PyLong_AsLong(args[5]));
+  a.add_inputs = PyObject_IsTrue(args[6]) == 1;
+  if (PyErr_Occurred() || a.offset_start < 0) return kNotHandled;
+  int64_t width = a.offset_start;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    if (w[i]->size(2) != h.size(2) || w[i]->size(0) != w[0]->size(0)) return kNotHandled;
+    a.b[i] = w[i]->data_ptr();
+    a.n[i] = static_cast<int32_t>(w[i]->size(1));
+    width += w[i]->size(1);
+  }
+  if (width > y.size(1)) return kNotHandled;
+  a.stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
+  a.h = h.data_ptr(); a.y = y.data_ptr(); a.y_stride = y.stride(0);
+  a.token_to_slot = static_cast<const int32_t*>(slots.data_ptr());
+  a.num_tokens = static_cast<int32_t>(h.size(1)); a.r = static_cast<int32_t>(h.size(2));
+  a.num_slots = static_cast<int32_t>(w[0]->size(0)); a.num_slices = static_cast<int32_t>(n);
+  a.dtype = dtype; a.h_dtype = h_dtype;
+  const auto fn = reinterpret_cast<int (*)(const MloraExpandArgs*)>(PyLong_AsSize_t(args[0]));
+  return PyErr_Occurred() ? kNotHandled : fn(&a);
+}
+
+template <typename F> PyObject* run_op(F f, PyObject* const* args, Py_ssize_t nargs, Py_ssize_t want) {
+  if (nargs != want) {
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments", want);
+    return nullptr;
+  }
+  long rc;
+  try {
+    rc = f(args);
+  } catch (...) {
+    rc = kNotHandled;
+  }
+  if (PyErr_Occurred()) PyErr_Clear();
+  return PyLong_FromLong(rc);
+}
+PyObject* py_shrink(PyObject*, PyObject* const* args, Py_ssize_t nargs) { return run_op(op_shrink, args, nargs, 6); }
+PyObject* py_expand(PyObject*, PyObject* const* args, Py_ssize_t nargs) { return run_op(op_expand, args, nargs, 7); }
+
+// ---- slot installs -----------------------------------------------------------------------------------
+// An adapter's targets, collected module by module and handed to mlora_install_slots together.
+struct InstallBatch {
+  std::vector<MloraInstallArgs> args;
+  std::vector<MloraInstallState> states;
+  int device = -1;
+};
+const char* kInstallCapsule = "mlora.fastcall.installs";
+void destroy_installs(PyObject* capsule) { delete static_cast<InstallBatch*>(PyCapsule_GetPointer(capsule, kInstallCapsule)); }
+
+PyObject* py_install_batch(PyObject*, PyObject*) { return PyCapsule_New(new InstallBatch(), kInstallCapsule, destroy_installs); }
+
+// Address of a payload tensor on `dev`: its own, or that of its copy where it lies in the packed host buffer.
+const void* source_on(const at::Tensor& t, int dev, const at::Tensor* packed, const at::Tensor* staged) {
+  if (t.is_cuda()) return t.device().index() == dev ? t.data_ptr() : nullptr;
+  if (!packed || !staged || !t.is_cpu() || t.scalar_type() != packed->scalar_type() || !t.is_contiguous()) return nullptr;
+  const char* at = static_cast<const char*>(t.data_ptr());
+  const char* base = static_cast<const char*>(packed->data_ptr());
+  if (at < base || at + t.numel() * t.element_size() > base + packed->numel() * packed->element_size()) return nullptr;
+  return static_cast<const char*>(staged->data_ptr()) + (at - base);
+}
+
+// install_add(batch, A buffer, tuple of B buffers, lora_a, lora_b, slot, rank, scaling, packed, its device copy,
+// rank vector, scaling vector, second scaling vector) -> bool: everything set_slot_lora and the payload check of the
+// layer look at is in order and the module's targets are in the batch; False: nothing was added and the
+// layer's own methods say what is wrong, or do it.
+bool install_add(InstallBatch* batch, PyObject* const* args) {
+  if (!THPVariable_Check(args[1]) || !PyTuple_Check(args[2]) || !THPVariable_Check(args[3])) return false;
+  const at::Tensor &A = THPVariable_Unpack(args[1]), &a_src = THPVariable_Unpack(args[3]);
+  if (!A.is_cuda() || !A.is_contiguous()) return false;
+  const bool multi = A.dim() == 4;
+  if (!multi && A.dim() != 3) return false;
+  const Py_ssize_t n = PyTuple_GET_SIZE(args[2]);
+  const int64_t slots = A.size(-3), r = A.size(-2), k = A.size(-1);
+  if (n < 1 || (multi ? A.size(0) != n : n != 1)) return false;
+  if (multi ? !PyList_Check(args[4]) || PyList_GET_SIZE(args[4]) != n : !THPVariable_Check(args[4])) return false;
+  const long long slot = PyLong_AsLongLong(args[5]), rank = PyLong_AsLongLong(args[6]);
+  const double scaling = PyFloat_AsDouble(args[7]);
+  if (PyErr_Occurred() || slot < 0 || slot >= slots || rank < 1 || rank > r || !std::isfinite(scaling)) return false;
+  const at::Tensor* packed = THPVariable_Check(args[8]) ? &THPVariable_Unpack(args[8]) : nullptr;
+  const at::Tensor* staged = THPVariable_Check(args[9]) ? &THPVariable_Unpack(args[9]) : nullptr;
+  const int dev = A.device().index();
+  if (dev != c10::hip::current_device() || (batch->device >= 0 && batch->device != dev)) return false;
+  if (staged && (!on_device(*staged, dev) || staged->numel() != packed->numel() || staged->scalar_type() != packed->scalar_type())) return false;
+  if (a_src.dim() != (multi ? 3 : 2) || (multi && a_src.size(0) != n) || a_src.size(-2) < rank || a_src.size(-1) != k || a_src.stride(-1) != 1) return false;
+  const int dtype = code_of(A.scalar_type()), src_dtype = code_of(a_src.scalar_type());
+  if (dtype < 0 || src_dtype < 0) return false;
+  const void* a_base = source_on(a_src, dev, packed, staged);
+  if (!a_base) return false;
+  MloraInstallState state = {};
+  for (int i = 10; i < 13; ++i) {
+    if (!THPVariable_Check(args[i])) return false;
+    const at::Tensor& t = THPVariable_Unpack(args[i]);
+    if (!on_device(t, dev) || t.dim() != 1 || t.size(0) != slots || !t.is_contiguous()) return false;
+    if (i == 10) {
+      if (t.scalar_type() != c10::ScalarType::Int) return false;
+      state.rank = static_cast<int32_t*>(t.data_ptr());
+    } else {
+      const int code = code_of(t.scalar_type());
+      if (code < 0 || (i == 12 && code != state.dtype)) return false;
+      state.dtype = code;
+      state.scaling[i - 11] = t.data_ptr();
+    }
+  }
+  const size_t before = batch->args.size();
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* bo = PyTuple_GET_ITEM(args[2], i);
+    PyObject* so = multi ? PyList_GET_ITEM(args[4], i) : args[4];
+    bool ok = THPVariable_Check(bo) && THPVariable_Check(so);
+    if (ok) {
+      const at::Tensor &B = THPVariable_Unpack(bo), &b_src = THPVariable_Unpack(so);
+      const void* b_base = source_on(b_src, dev, packed, staged);
+      ok = b_base && B.dim() == 3 && B.is_contiguous() && on_device(B, dev) && B.scalar_type() == A.scalar_type() && B.size(0) == slots &&
+           B.size(2) == r && b_src.dim() == 2 && b_src.scalar_type() == a_src.scalar_type() && b_src.size(0) == B.size(1) &&
+           b_src.size(1) >= rank && b_src.stride(1) == 1;
+      if (ok) {
+        MloraInstallArgs m = {};
+        m.a_dst = static_cast<char*>(A.data_ptr()) + i * slots * r * k * static_cast<int64_t>(A.element_size());
+        m.b_dst = B.data_ptr();
+        m.a_src = static_cast<const char*>(a_base) + (multi ? i * a_src.stride(0) * static_cast<int64_t>(a_src.element_size()) : 0);
+        m.b_src = b_base;
+        m.a_src_stride = a_src.stride(-2); m.b_src_stride = b_src.stride(0);
+        m.slot = static_cast<int32_t>(slot); m.k = static_cast<int32_t>(k); m.n = static_cast<int32_t>(B.size(1)); m.r = static_cast<int32_t>(r);
+        m.rank = static_cast<int32_t>(rank); m.dtype = dtype; m.src_dtype = src_dtype; m.scaling = static_cast<float>(scaling);
+        m.num_slots = static_cast<int32_t>(slots);
+        ok = m.a_src_stride >= k && m.b_src_stride >= rank;
+        if (ok) {
+          batch->args.push_back(m);
+          batch->states.push_back(i == 0 ? state : MloraInstallState{});
+        }
+      }
+    }
+    if (!ok) {
+      batch->args.resize(before);
+      batch->states.resize(before);
+      return false;
+    }
+  }
+  batch->device = dev;
+  return true;
+}
+
+PyObject* py_install_add(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 13) {
+    PyErr_SetString(PyExc_TypeError, "install_add() takes thirteen arguments");
+    return nullptr;
+  }
+  auto* batch = static_cast<InstallBatch*>(PyCapsule_GetPointer(args[0], kInstallCapsule));
+  if (!batch) return nullptr;
+  bool ok;
+  try {
+    ok = install_add(batch, args);
+  } catch (...) {
+    ok = false;
+  }
+  if (PyErr_Occurred()) PyErr_Clear();
+  return PyBool_FromLong(ok);
+}
+
+// install_flush(batch, address of mlora_install_slots) -> 0 or a library error code; the batch is empty then
+PyObject* py_install_flush(PyObject*, PyObject* args) {
+  PyObject* cap;
+  unsigned long long fn = 0;
+  if (!PyArg_ParseTuple(args, "OK", &cap, &fn)) return nullptr;
+  auto* batch = static_cast<InstallBatch*>(PyCapsule_GetPointer(cap, kInstallCapsule));
+  if (!batch) return nullptr;
+  long rc = 0;
+  if (!batch->args.empty()) {
+    void* stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(batch->device)).stream();
+    for (auto& m : batch->args) m.stream = stream;
+    rc = reinterpret_cast<int (*)(const MloraInstallArgs*, const MloraInstallState*, int32_t)>(static_cast<uintptr_t>(fn))(
+        batch->args.data(), batch->states.data(), static_cast<int32_t>(batch->args.size()));
+  }
+  batch->args.clear();
+  batch->states.clear();
+  return PyLong_FromLong(rc);
+}
+
+template <typename F> PyCFunction method(F* f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
+
 PyMethodDef kMethods[] = {
+    {"shrink", method(py_shrink), METH_FASTCALL, "shrink(address of mlora_shrink, inputs, weights, output, slots, scaling) -> 0, a library error code, or NOT_HANDLED"},
+    {"expand", method(py_expand), METH_FASTCALL, "expand(address of mlora_expand, inputs, weights, output, slots, offset, add) -> 0, a library error code, or NOT_HANDLED"},
+    {"install_batch", py_install_batch, METH_NOARGS, "install_batch() -> an empty batch of slot installs"},
+    {"install_add", method(py_install_add), METH_FASTCALL, "install_add(batch, A, Bs, lora_a, lora_b, slot, rank, scaling, packed, staged, ranks, scalings, base scalings) -> bool"},
+    {"install_flush", py_install_flush, METH_VARARGS, "install_flush(batch, address of mlora_install_slots) -> 0 or a library error code"},
     {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora, address of mlora_add_workspace_bytes) -> state"},
     {"register_site", py_register_site, METH_VARARGS, "register_site(state, a_list, b_list, widths, block address, block owner, vectorisable) -> bool"},
     {"clear_sites", py_clear_sites, METH_O, "clear_sites(state)"},
@@ -359,7 +611,7 @@ PyMethodDef kMethods[] = {
     {"forget_step", py_forget_step, METH_O, "forget_step(state)"},
     {"set_scratch", py_set_scratch, METH_VARARGS, "set_scratch(state, device index, stream, address, bytes)"},
     {"counters", py_counters, METH_O, "counters(state) -> (calls enqueued here, calls left to the Python path)"},
-    {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_call)), METH_FASTCALL,
+    {"call", method(py_call), METH_FASTCALL,
      "call(state, y_slices, x, lora_a_slices, lora_b_slices, indices, metadata, scaling, y_packed, effective_rank) -> 0, a library error code, or NOT_HANDLED"},
     {nullptr, nullptr, 0, nullptr},
 };

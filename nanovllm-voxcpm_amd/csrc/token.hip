@@ -200,33 +200,107 @@ __global__ __launch_bounds__(kTokThreads) void token_expand_vec_kernel(TokenExpa
   }
 }
 
+// ---- slot install -------------------------------------------------------------------------------
+// One slot of A and B of one target: rows / columns below `rank` are copied (B scaled, rounded first
+// to the source type as a tensor-times-scalar product would be), the rest are zeroed.
 struct InstallParams {
-  void* a_dst; void* b_dst;
+  void* a_dst; void* b_dst;  // the slot's own rows
   const void* a_src; const void* b_src;
-  int64_t a_ss, b_ss;
-  int slot, K, N, r, rank;
+  int a_ss, b_ss;
+  int K, N, r, rank;
   float scaling;
+  int slot;
+  short state_dtype, vec;
+  int32_t* rank_out; void* scale_out; void* base_out;  // per-slot state of the layer, or null
 };
+// An adapter has a target for every projection of every layer, and a launch per target costs the host
+// several microseconds where the copy itself takes well below one: the targets of an admission
+// share a launch, whose table travels by value (40 entries are 3.8 KB of the 4 KB a launch may carry).
+constexpr int kInstallBatch = 40;
+struct InstallTable { InstallParams p[kInstallBatch]; };
+static_assert(sizeof(InstallTable) <= 4096, "the table is a kernel argument");
 
-// One slot of A and B rewritten in a single pass: rows / columns below `rank` are copied
-// (B scaled, rounded first to the source type as a tensor-times-scalar product would be),
-// the rest are zeroed.
+template <typename T> __device__ __forceinline__ void load8(const T* src, float (&f)[8]) {
+  if constexpr (sizeof(T) == 2) {
+    Pack8 v;
+    v.raw = load128(src);
+    unpack8<T>(v, f);
+  } else {
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { f[e] = lo[e]; f[4 + e] = hi[e]; }
+  }
+}
+template <typename T> __device__ __forceinline__ void store8(T* dst, const float (&f)[8]) {
+  T v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = from_f32<T>(f[e]);
+  __builtin_memcpy(__builtin_assume_aligned(dst, 16), v, sizeof(v));
+}
+
+// grid (workgroups of the largest target, targets)
 template <typename D, typename S>
-__global__ __launch_bounds__(256) void install_kernel(InstallParams p) {
+__global__ __launch_bounds__(256) void install_kernel(InstallTable table) {
+  const InstallParams& p = table.p[blockIdx.y];
   const int64_t na = static_cast<int64_t>(p.r) * p.K, nb = static_cast<int64_t>(p.N) * p.r;
-  D* A = static_cast<D*>(p.a_dst) + static_cast<int64_t>(p.slot) * na;
-  D* B = static_cast<D*>(p.b_dst) + static_cast<int64_t>(p.slot) * nb;
+  D* A = static_cast<D*>(p.a_dst);
+  D* B = static_cast<D*>(p.b_dst);
   const S* as = static_cast<const S*>(p.a_src);
   const S* bs = static_cast<const S*>(p.b_src);
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < na + nb; i += stride) {
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int rank = p.rank;
+  const float scaling = p.scaling;
+  // the product rounded to the source type as torch's kernel rounds it: once from the exact product for
+  // fp16 (its multiply is a mixed-precision one), by way of fp32 for bf16
+  auto scaled = [&](float v) {
+    if constexpr (std::is_same<S, _Float16>::value) return static_cast<float>(static_cast<_Float16>(static_cast<double>(v) * static_cast<double>(scaling)));
+    else return to_f32(from_f32<S>(v * scaling));
+  };
+  if (first == 0) {
+    if (p.rank_out) p.rank_out[p.slot] = rank;
+    auto put = [&](void* to) {
+      if (!to) return;
+      if (p.state_dtype == MLORA_DTYPE_F32) static_cast<float*>(to)[p.slot] = scaling;
+      else if (p.state_dtype == MLORA_DTYPE_F16) static_cast<_Float16*>(to)[p.slot] = from_f32<_Float16>(scaling);
+      else static_cast<__bf16*>(to)[p.slot] = from_f32<__bf16>(scaling);
+    };
+    put(p.scale_out);
+    put(p.base_out);
+  }
+  if (p.vec) {  // rows in pieces of eight elements
+    const int ka = p.K / 8, kb = p.r / 8;
+    const int pa = p.r * ka, pb = p.N * kb;
+    for (int64_t i = first; i < pa + pb; i += stride) {
+      float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (i < pa) {
+        const int j = static_cast<int>(i) / ka, k = static_cast<int>(i) % ka * 8;
+        if (j < rank) load8<S>(as + static_cast<int64_t>(j) * p.a_ss + k, f);
+        store8<D>(A + i * 8, f);
+      } else {
+        const int e = static_cast<int>(i - pa), n = e / kb, j = e % kb * 8;
+        const S* src = bs + static_cast<int64_t>(n) * p.b_ss + j;
+        if (j + 8 <= rank) {
+          load8<S>(src, f);
+        } else {  // (a row of the source may end at the adapter's rank)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) f[q] = j + q < rank ? to_f32(src[q]) : 0.f;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) f[q] = scaled(f[q]);
+        store8<D>(B + static_cast<int64_t>(e) * 8, f);
+      }
+    }
+    return;
+  }
+  for (int64_t i = first; i < na + nb; i += stride) {
     if (i < na) {
       const int j = static_cast<int>(i / p.K), k = static_cast<int>(i % p.K);
-      A[i] = j < p.rank ? from_f32<D>(to_f32(as[j * p.a_ss + k])) : from_f32<D>(0.f);
+      A[i] = j < rank ? from_f32<D>(to_f32(as[static_cast<int64_t>(j) * p.a_ss + k])) : from_f32<D>(0.f);
     } else {
       const int64_t e = i - na;
       const int n = static_cast<int>(e / p.r), j = static_cast<int>(e % p.r);
-      B[e] = j < p.rank ? from_f32<D>(to_f32(from_f32<S>(to_f32(bs[n * p.b_ss + j]) * p.scaling))) : from_f32<D>(0.f);
+      B[e] = j < rank ? from_f32<D>(scaled(to_f32(bs[static_cast<int64_t>(n) * p.b_ss + j]))) : from_f32<D>(0.f);
     }
   }
 }
@@ -303,12 +377,34 @@ void launch_expand_h(const TokenExpandParams& p, dim3 grid, int h_dtype, hipStre
 }
 
 template <typename D>
-void launch_install_src(const InstallParams& p, dim3 grid, int src_dtype, hipStream_t st) {
+void launch_install_src(const InstallTable& t, dim3 grid, int src_dtype, hipStream_t st) {
   switch (src_dtype) {
-    case MLORA_DTYPE_F32: hipLaunchKernelGGL((install_kernel<D, float>), grid, dim3(256), 0, st, p); break;
-    case MLORA_DTYPE_F16: hipLaunchKernelGGL((install_kernel<D, _Float16>), grid, dim3(256), 0, st, p); break;
-    default: hipLaunchKernelGGL((install_kernel<D, __bf16>), grid, dim3(256), 0, st, p); break;
+    case MLORA_DTYPE_F32: hipLaunchKernelGGL((install_kernel<D, float>), grid, dim3(256), 0, st, t); break;
+    case MLORA_DTYPE_F16: hipLaunchKernelGGL((install_kernel<D, _Float16>), grid, dim3(256), 0, st, t); break;
+    default: hipLaunchKernelGGL((install_kernel<D, __bf16>), grid, dim3(256), 0, st, t); break;
   }
+}
+
+int element_size(int dtype) { return dtype == MLORA_DTYPE_F32 ? 4 : 2; }
+
+int check_install(const MloraInstallArgs* a) {
+  if (a->slot < 0 || a->k < 0 || a->n < 0 || a->r < 0 || a->rank < 0 || a->rank > a->r) {
+    set_error("mlora_install_slot: bad sizes (slot=%d k=%d n=%d r=%d rank=%d)", a->slot, a->k, a->n, a->r, a->rank);
+    return MLORA_E_INVALID;
+  }
+  if (a->slot >= a->num_slots) {
+    set_error("mlora_install_slot: slot %d is outside the %d slots of the buffers", a->slot, a->num_slots);
+    return MLORA_E_INVALID;
+  }
+  if (a->rank > 0 && (a->a_src_stride < a->k || a->b_src_stride < a->rank)) {
+    set_error("mlora_install_slot: source row strides (%lld, %lld) are shorter than the rows they carry (%d, %d)",
+              static_cast<long long>(a->a_src_stride), static_cast<long long>(a->b_src_stride), a->k, a->rank);
+    return MLORA_E_INVALID;
+  }
+  if (a->a_src_stride > INT32_MAX || a->b_src_stride > INT32_MAX) { set_error("mlora_install_slot: source row stride exceeds 2^31 - 1"); return MLORA_E_TOO_LARGE; }
+  if (!valid_dtype(a->dtype) || !valid_dtype(a->src_dtype)) { set_error("mlora_install_slot: unknown dtype"); return MLORA_E_INVALID; }
+  if (!a->a_dst || !a->b_dst || (a->rank > 0 && (!a->a_src || !a->b_src))) { set_error("mlora_install_slot: NULL pointer"); return MLORA_E_INVALID; }
+  return 0;
 }
 
 }  // namespace
@@ -374,37 +470,54 @@ extern "C" int mlora_expand(const MloraExpandArgs* a) {
   return check_launch("mlora_expand");
 }
 
-extern "C" int mlora_install_slot(const MloraInstallArgs* a) {
-  if (!a) { set_error("mlora_install_slot: NULL args"); return MLORA_E_INVALID; }
-  if (a->slot < 0 || a->k < 0 || a->n < 0 || a->r < 0 || a->rank < 0 || a->rank > a->r) {
-    set_error("mlora_install_slot: bad sizes (slot=%d k=%d n=%d r=%d rank=%d)", a->slot, a->k, a->n, a->r, a->rank);
-    return MLORA_E_INVALID;
+extern "C" int mlora_install_slots(const MloraInstallArgs* list, const MloraInstallState* states, int32_t count) {
+  if (count < 0 || (count > 0 && !list)) { set_error("mlora_install_slot: NULL args"); return MLORA_E_INVALID; }
+  for (int i = 0; i < count; ++i) {
+    if (int rc = check_install(list + i)) return rc;
+    if (states && !valid_dtype(states[i].dtype)) { set_error("mlora_install_slots: unknown dtype"); return MLORA_E_INVALID; }
+    if (list[i].stream != list[0].stream) { set_error("mlora_install_slots: the entries name different streams"); return MLORA_E_INVALID; }
   }
-  if (a->slot >= a->num_slots) {
-    set_error("mlora_install_slot: slot %d is outside the %d slots of the buffers", a->slot, a->num_slots);
-    return MLORA_E_INVALID;
+  for (int i = 0; i < count;) {
+    // consecutive entries of the same element types share a launch
+    InstallTable t = {};
+    int n = 0;
+    int64_t most = 0;
+    const int dtype = list[i].dtype, src_dtype = list[i].src_dtype;
+    for (; i < count && n < kInstallBatch && list[i].dtype == dtype && list[i].src_dtype == src_dtype; ++i) {
+      const MloraInstallArgs& a = list[i];
+      const int64_t na = static_cast<int64_t>(a.r) * a.k, nb = static_cast<int64_t>(a.n) * a.r;
+      InstallParams& p = t.p[n++];
+      const int e = element_size(dtype), se = element_size(src_dtype);
+      p.a_dst = static_cast<char*>(a.a_dst) + a.slot * na * e;
+      p.b_dst = static_cast<char*>(a.b_dst) + a.slot * nb * e;
+      p.a_src = a.a_src; p.b_src = a.b_src; p.a_ss = static_cast<int>(a.a_src_stride); p.b_ss = static_cast<int>(a.b_src_stride);
+      p.K = a.k; p.N = a.n; p.r = a.r; p.rank = a.rank; p.scaling = a.scaling; p.slot = a.slot;
+      if (states) {
+        p.rank_out = states[i].rank; p.scale_out = states[i].scaling[0]; p.base_out = states[i].scaling[1]; p.state_dtype = static_cast<short>(states[i].dtype);
+      }
+      // 128-bit pieces where every row of both sides starts on a 16-byte boundary
+      p.vec = a.k % 8 == 0 && a.r % 8 == 0 && a.a_src_stride * se % 16 == 0 && a.b_src_stride * se % 16 == 0 && aligned16(a.a_src) &&
+              aligned16(a.b_src) && aligned16(p.a_dst) && aligned16(p.b_dst) && na + nb < (1ll << 31);
+      const int64_t units = p.vec ? (na + nb) / 8 : na + nb;
+      most = units > most ? units : most;
+    }
+    if (most == 0) {
+      bool state = false;
+      for (int k = 0; k < n; ++k) state |= t.p[k].rank_out || t.p[k].scale_out || t.p[k].base_out;
+      if (!state) continue;
+    }
+    int64_t blocks = (most + 255) / 256;
+    blocks = blocks < 1 ? 1 : blocks > 2048 ? 2048 : blocks;
+    const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(n));
+    hipStream_t st = static_cast<hipStream_t>(list[0].stream);
+    switch (dtype) {
+      case MLORA_DTYPE_F32: launch_install_src<float>(t, grid, src_dtype, st); break;
+      case MLORA_DTYPE_F16: launch_install_src<_Float16>(t, grid, src_dtype, st); break;
+      default: launch_install_src<__bf16>(t, grid, src_dtype, st); break;
+    }
+    if (int rc = check_launch("mlora_install_slots")) return rc;
   }
-  if (a->rank > 0 && (a->a_src_stride < a->k || a->b_src_stride < a->rank)) {
-    set_error("mlora_install_slot: source row strides (%lld, %lld) are shorter than the rows they carry (%d, %d)",
-              static_cast<long long>(a->a_src_stride), static_cast<long long>(a->b_src_stride), a->k, a->rank);
-    return MLORA_E_INVALID;
-  }
-  if (!valid_dtype(a->dtype) || !valid_dtype(a->src_dtype)) { set_error("mlora_install_slot: unknown dtype"); return MLORA_E_INVALID; }
-  if (!a->a_dst || !a->b_dst || (a->rank > 0 && (!a->a_src || !a->b_src))) { set_error("mlora_install_slot: NULL pointer"); return MLORA_E_INVALID; }
-  const int64_t total = static_cast<int64_t>(a->r) * a->k + static_cast<int64_t>(a->n) * a->r;
-  if (total == 0) return 0;
-  InstallParams p;
-  p.a_dst = a->a_dst; p.b_dst = a->b_dst; p.a_src = a->a_src; p.b_src = a->b_src;
-  p.a_ss = a->a_src_stride; p.b_ss = a->b_src_stride;
-  p.slot = a->slot; p.K = a->k; p.N = a->n; p.r = a->r; p.rank = a->rank; p.scaling = a->scaling;
-  int64_t blocks = (total + 255) / 256;
-  if (blocks > 2048) blocks = 2048;
-  dim3 grid(static_cast<unsigned>(blocks));
-  hipStream_t st = static_cast<hipStream_t>(a->stream);
-  switch (a->dtype) {
-    case MLORA_DTYPE_F32: launch_install_src<float>(p, grid, a->src_dtype, st); break;
-    case MLORA_DTYPE_F16: launch_install_src<_Float16>(p, grid, a->src_dtype, st); break;
-    default: launch_install_src<__bf16>(p, grid, a->src_dtype, st); break;
-  }
-  return check_launch("mlora_install_slot");
+  return 0;
 }
+
+extern "C" int mlora_install_slot(const MloraInstallArgs* a) { return mlora_install_slots(a, nullptr, 1); }

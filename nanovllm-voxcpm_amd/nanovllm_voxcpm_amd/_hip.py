@@ -62,6 +62,7 @@ EXPORTS = (
     "mlora_meta_build",
     "mlora_meta_build_many",
     "mlora_install_slot",
+    "mlora_install_slots",
     "mlora_stream_capture_id",
     "mlora_abi_version",
     "mlora_last_error",
@@ -184,6 +185,10 @@ class MloraInstallArgs(C.Structure):
     ]
 
 
+class MloraInstallState(C.Structure):
+    _fields_ = [("rank", C.c_void_p), ("scaling", C.c_void_p * 2), ("dtype", C.c_int32)]
+
+
 _LIB: C.CDLL | None = None
 _LOAD_ERROR: str | None = None
 
@@ -225,6 +230,8 @@ def load() -> C.CDLL:
         fn.restype = C.c_int
     lib.mlora_meta_build_many.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32]
     lib.mlora_meta_build_many.restype = C.c_int
+    lib.mlora_install_slots.argtypes = [C.POINTER(MloraInstallArgs), C.POINTER(MloraInstallState), C.c_int32]
+    lib.mlora_install_slots.restype = C.c_int
     lib.mlora_plan_workspace_bytes.argtypes = [C.c_int32, C.c_int32]
     lib.mlora_plan_workspace_bytes.restype = C.c_size_t
     lib.mlora_add_workspace_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32]

@@ -294,6 +294,23 @@ class _LoRALayerBase(nn.Module):
             self._install(slot_id, 0, lora_a, lora_b, effective_rank, scaling)
         self._record_slot(slot_id, effective_rank, scaling)
 
+    def queue_slot_lora(self, fast, batch, slot_id: int, lora_a, lora_b, effective_rank: int, scaling: float, packed, staged) -> bool:
+        """Add this adapter's targets to a batch of installs (of the C++ host path ``fast``) that one launch
+        carries out; ``staged`` is the device copy of the host buffer ``packed`` the payload lies in.
+        False, with nothing added: ``validate_slot_lora_payload`` and ``set_slot_lora`` have to see it."""
+        if not self.supports_lora:
+            return False
+        a, b = self._parameters.get("lora_A"), tuple([self._parameters.get(name) for name in self._b_names()])
+        vectors = self._buffers
+        return fast.install_add(batch, a, b, lora_a, lora_b, slot_id, effective_rank, scaling, packed, staged,
+                                vectors["effective_lora_rank"], vectors["lora_scaling"], vectors["lora_base_scaling"])
+
+    def note_queued_slot(self, slot_id: int, effective_rank: int, scaling: float) -> None:
+        """The host mirrors of a slot whose install has been launched (the device vectors are part of it)."""
+        self._effective_lora_rank_values[slot_id] = effective_rank
+        self._lora_scaling_values[slot_id] = scaling
+        self._lora_base_scaling_values[slot_id] = scaling
+
     def _zero_slot(self, slot_id: int, position: int) -> None:
         a = self._a_of(position)
         (a.data if isinstance(a, nn.Parameter) else a.detach())[slot_id].zero_()
@@ -372,6 +389,9 @@ class _MultiTargetMixin:
 
     def _b_of(self, position: int) -> nn.Parameter:
         return getattr(self, f"lora_B_{self.lora_targets[position]}")
+
+    def _b_names(self) -> list[str]:
+        return [f"lora_B_{target}" for target in self.lora_targets]
 
     def _make_lora_b_weight_loader(self, target):
         def loader(param: nn.Parameter, loaded_weight: torch.Tensor):
@@ -519,6 +539,9 @@ class _SingleTargetMixin:
 
     def _b_of(self, position: int) -> nn.Parameter:
         return self.lora_B
+
+    def _b_names(self) -> list[str]:
+        return ["lora_B"]
 
 
 class LoRARowParallelLinear(_SingleTargetMixin, _LoRALayerBase):

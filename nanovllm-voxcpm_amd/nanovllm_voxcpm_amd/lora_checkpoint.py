@@ -13,7 +13,7 @@ payload per rank is returned: packed (column-parallel) modules shard every B alo
 
 ``install_lora_payload`` is the slot-loading step of the reference's model runner
 (engine/model_runner.py:389-420): clear what the slot's previous occupant populated, then one
-``set_slot_lora`` (here: one fused install launch) per module of the payload.
+``set_slot_lora`` per module of the payload (here: one install launch for up to forty targets).
 """
 
 from __future__ import annotations
@@ -24,7 +24,9 @@ from pathlib import Path
 import torch
 from safetensors import safe_open
 
+from nanovllm_voxcpm_amd import _hip
 from nanovllm_voxcpm_amd.engine.lora_runtime import LoRAModelPayload, LoRAModulePayload
+from nanovllm_voxcpm_amd.layers.lora import _LORA_MODULE_TYPES
 
 WEIGHTS_FILE = "lora_weights.safetensors"
 CONFIG_FILE = "lora_config.json"
@@ -207,40 +209,78 @@ def install_lora_payload(model: torch.nn.Module, slot_id: int, payload: LoRAMode
     ``loaded`` (slot id -> module names, kept by the caller across calls) limits the clearing
     of the previous occupant to the modules it actually populated; without it every
     LoRA-capable module not named in the payload is cleared."""
-    every = dict(model.named_modules())  # one walk over the model per admission
-    modules = {name: m for name, m in every.items() if hasattr(m, "set_slot_lora")}
+    modules: dict = {}
     for name in payload.modules:
-        if name not in every:
+        module = _find(model, name)
+        if module is None:
             raise ValueError(f"Unknown LoRA target module '{name}'")
-        if name not in modules:
+        if not hasattr(module, "set_slot_lora"):
             raise ValueError(f"Module '{name}' does not support LoRA slots")
-    # every module's payload is checked against the module before anything is written: a payload
-    # for another hidden size, rank budget or TP shard must not leave a half-installed slot
+        modules[name] = module
+    packed, staged = getattr(payload, "packed", None), {}  # device -> copy of the payload's packed host buffer
+    # Every module's payload is checked against the module before anything is written: a payload
+    # for another hidden size, rank budget or TP shard must not leave a half-installed slot.  What the
+    # C++ host path has checked waits in its batch, whose targets share a launch; the rest is
+    # checked by the layers themselves and installed one by one.
+    fast = _hip.load_fastcall()
+    batch = fast.install_batch() if fast is not None else None
+    queued, single = [], []
     for name, m in payload.modules.items():
-        modules[name].validate_slot_lora_payload(m.lora_a, m.lora_b, m.effective_rank, m.scaling)
-        if not 0 <= slot_id < modules[name].max_loras:
-            raise IndexError(f"slot_id={slot_id} is outside the {modules[name].max_loras} slots of '{name}'")
-    previous = loaded.get(slot_id) if loaded is not None and slot_id in loaded else list(modules)
-    for name in previous:
-        if name not in payload.modules and name in modules:
-            modules[name].clear_slot_lora(slot_id)
-    staged: dict = {}  # device -> copy of the payload's packed host buffer
-
-    for name, m in payload.modules.items():
-        device = next(modules[name].parameters()).device
+        module = modules[name]
+        shared = any(module is other for other, _ in queued)  # (a module of two names: one install after the other)
+        if batch is not None and not shared and type(module) in _LORA_MODULE_TYPES and module.supports_lora:
+            device = module.lora_A.device
+            if device.type == "cuda" and module.queue_slot_lora(fast, batch, slot_id, m.lora_a, m.lora_b, m.effective_rank, m.scaling, packed,
+                                                                _staged(packed, staged, device)):
+                queued.append((module, m))
+                continue
+        module.validate_slot_lora_payload(m.lora_a, m.lora_b, m.effective_rank, m.scaling)
+        if not 0 <= slot_id < module.max_loras:
+            raise IndexError(f"slot_id={slot_id} is outside the {module.max_loras} slots of '{name}'")
+        single.append((module, m))
+    if loaded is not None and slot_id in loaded:
+        others = [(name, _find(model, name)) for name in loaded[slot_id] if name not in payload.modules]
+    else:
+        others = [(name, module) for name, module in model.named_modules() if name not in payload.modules]
+    for _, module in others:
+        if module is not None and hasattr(module, "set_slot_lora"):
+            module.clear_slot_lora(slot_id)
+    if queued:
+        _hip._check(fast.install_flush(batch, _hip.entry_point("mlora_install_slots")), "mlora_install_slots")
+        for module, m in queued:
+            module.note_queued_slot(slot_id, m.effective_rank, m.scaling)
+    for module, m in single:
+        device = next(module.parameters()).device
 
         def put(t: torch.Tensor) -> torch.Tensor:
-            packed = getattr(payload, "packed", None)
             if packed is not None and device.type == "cuda" and t.is_contiguous():
                 first = (t.data_ptr() - packed.data_ptr()) // packed.element_size()
                 if t.dtype == packed.dtype and 0 <= first and first + t.numel() <= packed.numel():
-                    if device not in staged:
-                        staged[device] = packed.to(device=device, non_blocking=True)
-                    return staged[device][first : first + t.numel()].view(t.shape)
+                    return _staged(packed, staged, device)[first : first + t.numel()].view(t.shape)
             return t.to(device=device, non_blocking=True)
 
-        modules[name].set_slot_lora(slot_id=slot_id, lora_a=put(m.lora_a),
-                                    lora_b=[put(t) for t in m.lora_b] if isinstance(m.lora_b, list) else put(m.lora_b),
-                                    effective_rank=m.effective_rank, scaling=m.scaling)
+        module.set_slot_lora(slot_id=slot_id, lora_a=put(m.lora_a),
+                             lora_b=[put(t) for t in m.lora_b] if isinstance(m.lora_b, list) else put(m.lora_b),
+                             effective_rank=m.effective_rank, scaling=m.scaling)
     if loaded is not None:
         loaded[slot_id] = list(payload.modules)
+
+
+def _find(model: torch.nn.Module, name: str) -> torch.nn.Module | None:
+    """The module of that dotted name (a walk over the whole model per admission would cost more than the
+    look-ups), None when there is none."""
+    module: torch.nn.Module | None = model
+    if name:
+        for part in name.split("."):
+            module = module._modules.get(part)
+            if module is None:
+                return None
+    return module
+
+
+def _staged(packed: torch.Tensor | None, staged: dict, device: torch.device) -> torch.Tensor | None:
+    if packed is None:
+        return None
+    if device not in staged:
+        staged[device] = packed.to(device=device, non_blocking=True)
+    return staged[device]
