@@ -34,7 +34,9 @@ def _as_3d(weight: torch.Tensor, what: str) -> torch.Tensor:
     return weight
 
 
-@torch.inference_mode()
+_FAST = _hip.load_fastcall()
+
+
 def lora_shrink(
     inputs: torch.Tensor,
     lora_a_weights: list[torch.Tensor],
@@ -56,6 +58,15 @@ def lora_shrink(
     """
     if no_lora_flag:
         return
+    if _FAST is not None:  # the usual call, checked and enqueued in C++
+        rc = _FAST.shrink(_hip.entry_point("mlora_shrink"), inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling)
+        if rc <= 0:
+            return _hip._check(rc, "mlora_shrink")
+    _shrink(inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling)
+
+
+@torch.inference_mode()
+def _shrink(inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling) -> None:
     weights = [_as_3d(w, "lora_a weight") for w in lora_a_weights]
     shapes = {tuple(w.shape) for w in weights}
     if len(shapes) != 1:
@@ -68,7 +79,6 @@ def lora_shrink(
     _hip.shrink(x, weights, output_tensor, as_slot_vector(token_lora_mapping), float(scaling))
 
 
-@torch.inference_mode()
 def lora_expand(
     inputs: torch.Tensor,
     lora_b_weights: list[torch.Tensor],
@@ -90,6 +100,15 @@ def lora_expand(
     """
     if no_lora_flag:
         return
+    if _FAST is not None:
+        rc = _FAST.expand(_hip.entry_point("mlora_expand"), inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs)
+        if rc <= 0:
+            return _hip._check(rc, "mlora_expand")
+    _expand(inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs)
+
+
+@torch.inference_mode()
+def _expand(inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs) -> None:
     weights = [_as_3d(w, "lora_b weight") for w in lora_b_weights]
     if inputs.ndim != 3 or inputs.size(0) != len(weights):
         raise ValueError("inputs must be [num_slices, num_tokens, rank]")
