@@ -126,6 +126,9 @@ typedef struct MloraAddArgs {
 } MloraAddArgs;
 
 int mlora_add_lora(const MloraAddArgs* args);
+/* The same with the number of slots that have tokens in this batch, where the host knows it (0: it does not);
+ * only MLORA_FORM_AUTO's choice depends on it. */
+int mlora_add_lora_active(const MloraAddArgs* args, int32_t active_slots);
 
 /* The same fused apply for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the

@@ -157,10 +157,20 @@ static bool small_batch(const MloraAddArgs* a, bool one_launch) {
 // All of this was measured on decode batches; on batches of many tiles per slot (a prefill of
 // 2098 tokens over 8 slot ids, o: 15.4 us per call against 10.1 tile-major) the grid over the slots
 // is the slower one: it is taken up to 32 tokens per slot id.
-static bool slot_major_pays(const MloraAddArgs* a) {
+// With K shared out the requests for unused slots end it too (down, us per call, slot-major / the best
+// other form): rank 16: 6.2 / 6.3 at 32 slot ids, 6.3 / 6.0 at 40, 8.0 / 6.2 at 64; rank 32: 8.7 / 9.6 at
+// 48, 10.8 / 10.6 at 64; rank 64: 12.0 / 12.6 at 48, 14.8 / 13.9 at 64.
+// `active` (when the caller knows it, else 0) is the number of slots with tokens.  Prompts are few long
+// segments: most of the grid is then workgroups without a tile, and the tiles behind a slot's first one learn
+// their slot from a record after all (rank 32, 37 tokens of one slot of 8: gate_up 7.4 / 4.9; 100 tokens
+// of 4 slots: gate_up 7.7 / 5.0; rank 64, 200 tokens of 3 slots of 32: qkv 9.0 / 6.5, gate_up 12.9 / 10.0,
+// down 10.2 / 9.1; rank 16, 250 tokens of 4 slots of 8: 4.05 / 4.11, 3.86 / 3.97, 5.67 / 5.58).
+static bool slot_major_pays(const MloraAddArgs* a, int active) {
   if (a->num_slots > knobs().slot_max_slots) return false;
   if (a->num_tokens > 32 * a->num_slots) return false;
-  if (slot_k_parts(a) > 1) return true;
+  const bool sparse = active > 0 && 2 * active <= a->num_slots;
+  if (slot_k_parts(a) > 1) return a->num_slots <= (a->r <= 16 ? 32 : 48) && !(sparse && a->r * a->num_slots >= 2048);
+  if (sparse || (active > 0 && a->num_tokens > MLORA_TILE_SMALL * active)) return false;
   double cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double per_slot = 2.0 * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
@@ -206,15 +216,16 @@ static bool pair_pays(const MloraAddArgs* a, int form) {
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace);
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active);
 
 }  // namespace
 
-extern "C" int mlora_add_lora(const MloraAddArgs* a) { return add_lora_impl(a, false); }
+extern "C" int mlora_add_lora(const MloraAddArgs* a) { return add_lora_impl(a, false, 0); }
+extern "C" int mlora_add_lora_active(const MloraAddArgs* a, int32_t active_slots) { return add_lora_impl(a, false, active_slots); }
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
   if (!a) { set_error("mlora_add_lora: NULL args"); return MLORA_E_INVALID; }
   if (a->num_tokens < 0 || a->k < 0 || a->r < 0 || a->num_slots < 0 || a->num_slices < 0) {
     set_error("mlora_add_lora: negative size"); return MLORA_E_INVALID;
@@ -277,7 +288,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace) {
   // the workgroups of a tile itself (down, decode batch, us per call, slot-major / split form:
   // rank 32: 8.1 / 10.6, rank 64: 10.7 / 17.0).
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
-      knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a))
+      knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, active))
     form = MLORA_FORM_SLOT;
   if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form))
     form = MLORA_FORM_PAIR;
@@ -413,7 +424,7 @@ extern "C" int mlora_add_lora_static(const MloraAddArgs* a) {
   b.workspace_bytes = MLORA_STATIC_SCRATCH_BYTES;
   // The array starts out zeroed (it is part of the loaded image) and only this library's kernels
   // ever write it, so its head is always either in the initial state or as a launch left it.
-  return add_lora_impl(&b, /*trusted_workspace=*/true);
+  return add_lora_impl(&b, /*trusted_workspace=*/true, 0);
 }
 
 extern "C" size_t mlora_add_workspace_bytes(int32_t num_tokens, int32_t num_slices, int32_t r, int32_t dtype) {

@@ -7,7 +7,7 @@
 // same reads and checks on the tensors' C++ objects.  It decides nothing by itself: it handles a
 // call only when everything the Python path would look up for it is what the Python path looked up
 // last time (the argument block of these weight buffers, the plan of this step's slot vector, the
-// scratch buffer of this stream), fills the per-step fields of the block and calls mlora_add_lora.
+// scratch buffer of this stream), fills the per-step fields of the block and calls mlora_add_lora_active.
 // Everything else - a first call, another step, a capture in progress, anything that has to raise
 // - is answered with "not handled", and the Python path runs as if this module did not exist, then
 // tells it what it found (register_site, set_step, set_scratch).
@@ -44,7 +44,7 @@ struct Site {
 };
 
 struct State {
-  int (*add_lora)(const MloraAddArgs*) = nullptr;
+  int (*add_lora)(const MloraAddArgs*, int32_t) = nullptr;  // mlora_add_lora_active
   size_t (*workspace_bytes)(int32_t, int32_t, int32_t, int32_t) = nullptr;
   std::unordered_map<std::string, Site> sites;
   // what the last call of the Python path looked up for its step
@@ -109,7 +109,7 @@ PyObject* py_create(PyObject*, PyObject* args) {
   unsigned long long add = 0, ws = 0;
   if (!PyArg_ParseTuple(args, "KK", &add, &ws)) return nullptr;
   State* s = new State();
-  s->add_lora = reinterpret_cast<int (*)(const MloraAddArgs*)>(static_cast<uintptr_t>(add));
+  s->add_lora = reinterpret_cast<int (*)(const MloraAddArgs*, int32_t)>(static_cast<uintptr_t>(add));
   s->workspace_bytes = reinterpret_cast<size_t (*)(int32_t, int32_t, int32_t, int32_t)>(static_cast<uintptr_t>(ws));
   return PyCapsule_New(s, kCapsule, destroy);
 }
@@ -212,32 +212,9 @@ PyObject* py_set_scratch(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-// The call itself.  Returns 0 (enqueued), a negative code of the library (the caller raises with
-// the library's message), or kNotHandled.
-long call(State* s, PyObject* y_slices, PyObject* x_obj, PyObject* a_list, PyObject* b_list, PyObject* indices, PyObject* metadata,
-          double scaling, PyObject* y_packed, PyObject* eff_obj) {
-  if (metadata == Py_None || !THPVariable_Check(x_obj)) return kNotHandled;
-  if (!(PyList_Check(y_slices) || PyTuple_Check(y_slices)) || !(PyList_Check(a_list) || PyTuple_Check(a_list)) ||
-      !(PyList_Check(b_list) || PyTuple_Check(b_list)))
-    return kNotHandled;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(y_slices);
-  if (n < 1 || n > MLORA_MAX_SLICES || PySequence_Fast_GET_SIZE(a_list) != n || PySequence_Fast_GET_SIZE(b_list) != n) return kNotHandled;
-  PyObject* target_obj = y_packed != Py_None ? y_packed : (n == 1 ? PySequence_Fast_GET_ITEM(y_slices, 0) : nullptr);
-  if (!target_obj || !THPVariable_Check(target_obj)) return kNotHandled;
-
-  std::string key;
-  const at::Tensor* a0 = nullptr;
-  if (!weights_key(a_list, b_list, n, &key, &a0)) return kNotHandled;
-  const auto it = s->sites.find(key);
-  if (it == s->sites.end()) return kNotHandled;
-  const Site& site = it->second;
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject* o = PySequence_Fast_GET_ITEM(y_slices, i);
-    if (!THPVariable_Check(o)) return kNotHandled;
-    const at::Tensor& y = THPVariable_Unpack(o);
-    if (y.dim() < 1 || y.size(-1) != site.widths[static_cast<size_t>(i)]) return kNotHandled;
-  }
-
+// The call itself, at the site of its weight buffers.  Returns 0 (enqueued), a negative code of the library
+// (the caller raises with the library's message), or kNotHandled.
+long call_at(State* s, const Site& site, PyObject* x_obj, PyObject* target_obj, PyObject* indices, PyObject* metadata, double scaling, PyObject* eff_obj) {
   const at::Tensor& x = THPVariable_Unpack(x_obj);
   const at::Tensor& target = THPVariable_Unpack(target_obj);
   if (x.dim() != 2 || x.stride(1) != 1 || target.dim() != 2 || target.stride(1) != 1) return kNotHandled;
@@ -245,12 +222,19 @@ long call(State* s, PyObject* y_slices, PyObject* x_obj, PyObject* a_list, PyObj
   if (rows <= 0 || rows > INT32_MAX) return kNotHandled;
 
   // the flag and the slot vector of the step's metadata (attribute reads: the object is the engine's)
-  PyObject* flag = PyObject_GetAttrString(metadata, "no_lora_flag");
+  static PyObject* const kNoLora = PyUnicode_InternFromString("no_lora_flag");
+  static PyObject* const kSlots = PyUnicode_InternFromString("token_to_slot");
+  PyObject* flag = PyObject_GetAttr(metadata, kNoLora);
   if (!flag) { PyErr_Clear(); return kNotHandled; }
   const int no_lora = PyObject_IsTrue(flag);
   Py_DECREF(flag);
   if (no_lora != 0) { PyErr_Clear(); return kNotHandled; }
-  const Ref tts{PyObject_GetAttrString(metadata, "token_to_slot")};
+  static PyObject* const kActive = PyUnicode_InternFromString("num_active_loras");
+  const Ref active{PyObject_GetAttr(metadata, kActive)};
+  long active_slots = active.p ? PyLong_AsLong(active.p) : 0;
+  if (PyErr_Occurred()) PyErr_Clear();
+  if (active_slots < 0 || active_slots > INT32_MAX) active_slots = 0;  // (not known)
+  const Ref tts{PyObject_GetAttr(metadata, kSlots)};
   if (!tts.p) { PyErr_Clear(); return kNotHandled; }
   PyObject* source_obj = tts.p != Py_None ? tts.p : indices;
   if (!THPVariable_Check(source_obj)) return kNotHandled;
@@ -282,12 +266,8 @@ long call(State* s, PyObject* y_slices, PyObject* x_obj, PyObject* a_list, PyObj
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) { (void)hipGetLastError(); return kNotHandled; }
     if (capturing != hipStreamCaptureStatusNone) return kNotHandled;
-    uint32_t version = 0;
-    try {
-      version = source._version();
-    } catch (...) {  // inference tensors carry no version counter: nothing is remembered for them
-      return kNotHandled;
-    }
+    if (source.is_inference()) return kNotHandled;  // no version counter: nothing is remembered for them
+    const uint32_t version = source._version();
     if (s->metadata != metadata || s->source != source_obj || s->version != version || s->stream != stream || s->num_slots != site.num_slots ||
         s->rows != rows || !s->plan)
       return kNotHandled;
@@ -321,7 +301,73 @@ long call(State* s, PyObject* y_slices, PyObject* x_obj, PyObject* a_list, PyObj
   a->workspace = ws;
   a->workspace_bytes = ws_bytes;
   a->effective_rank = static_cast<const int32_t*>(eff_ptr);
-  return s->add_lora(a);
+  return s->add_lora(a, static_cast<int32_t>(active_slots));
+}
+
+// A call with lists of slices.
+long call(State* s, PyObject* y_slices, PyObject* x_obj, PyObject* a_list, PyObject* b_list, PyObject* indices, PyObject* metadata,
+          double scaling, PyObject* y_packed, PyObject* eff_obj) {
+  if (metadata == Py_None || !THPVariable_Check(x_obj)) return kNotHandled;
+  if (!(PyList_Check(y_slices) || PyTuple_Check(y_slices)) || !(PyList_Check(a_list) || PyTuple_Check(a_list)) ||
+      !(PyList_Check(b_list) || PyTuple_Check(b_list)))
+    return kNotHandled;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(y_slices);
+  if (n < 1 || n > MLORA_MAX_SLICES || PySequence_Fast_GET_SIZE(a_list) != n || PySequence_Fast_GET_SIZE(b_list) != n) return kNotHandled;
+  PyObject* target_obj = y_packed != Py_None ? y_packed : (n == 1 ? PySequence_Fast_GET_ITEM(y_slices, 0) : nullptr);
+  if (!target_obj || !THPVariable_Check(target_obj)) return kNotHandled;
+
+  std::string key;
+  const at::Tensor* a0 = nullptr;
+  if (!weights_key(a_list, b_list, n, &key, &a0)) return kNotHandled;
+  const auto it = s->sites.find(key);
+  if (it == s->sites.end()) return kNotHandled;
+  const Site& site = it->second;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* o = PySequence_Fast_GET_ITEM(y_slices, i);
+    if (!THPVariable_Check(o)) return kNotHandled;
+    const at::Tensor& y = THPVariable_Unpack(o);
+    if (y.dim() < 1 || y.size(-1) != site.widths[static_cast<size_t>(i)]) return kNotHandled;
+  }
+  return call_at(s, site, x_obj, target_obj, indices, metadata, scaling, eff_obj);
+}
+
+// A call with the buffers of a LoRA linear as the layer holds them: one A buffer [targets, slots, r, K] (or
+// [slots, r, K]), its B buffers, and an output whose columns are the targets' blocks in order.  It saves the
+// layer the views that the lists are made of.
+long call_stacked(State* s, PyObject* target_obj, PyObject* x_obj, PyObject* a_obj, PyObject* b_tuple, PyObject* indices, PyObject* metadata,
+                  double scaling, PyObject* eff_obj) {
+  if (metadata == Py_None || !THPVariable_Check(x_obj) || !THPVariable_Check(target_obj) || !THPVariable_Check(a_obj) || !PyTuple_Check(b_tuple))
+    return kNotHandled;
+  const Py_ssize_t n = PyTuple_GET_SIZE(b_tuple);
+  const at::Tensor& a = THPVariable_Unpack(a_obj);
+  if (n < 1 || n > MLORA_MAX_SLICES || !a.is_contiguous() || (a.dim() == 4 ? a.size(0) != n : a.dim() != 3 || n != 1)) return kNotHandled;
+  int64_t buf[2 * MLORA_MAX_SLICES * 4 + 1];
+  int at = 0;
+  const int64_t one = a.size(-3) * a.size(-2) * a.size(-1) * static_cast<int64_t>(a.element_size());
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    buf[at++] = reinterpret_cast<int64_t>(a.data_ptr()) + i * one;
+    buf[at++] = a.size(-3);
+    buf[at++] = a.size(-2);
+    buf[at++] = a.size(-1);
+  }
+  int64_t width = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* o = PyTuple_GET_ITEM(b_tuple, i);
+    if (!THPVariable_Check(o)) return kNotHandled;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (t.dim() != 3 || !t.is_contiguous()) return kNotHandled;
+    buf[at++] = reinterpret_cast<int64_t>(t.data_ptr());
+    buf[at++] = t.size(0);
+    buf[at++] = t.size(1);
+    buf[at++] = t.size(2);
+    width += t.size(1);
+  }
+  buf[at++] = static_cast<int64_t>(a.scalar_type());
+  const auto it = s->sites.find(std::string(reinterpret_cast<const char*>(buf), static_cast<size_t>(at) * sizeof(int64_t)));
+  if (it == s->sites.end()) return kNotHandled;
+  const at::Tensor& target = THPVariable_Unpack(target_obj);
+  if (target.dim() != 2 || target.size(1) != width) return kNotHandled;
+  return call_at(s, it->second, x_obj, target_obj, indices, metadata, scaling, eff_obj);
 }
 
 // call(state, y_slices, x, lora_a_slices, lora_b_slices, indices, metadata, scaling, y_packed, effective_rank)
@@ -338,6 +384,27 @@ PyObject* py_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   try {
     rc = call(s, args[1], args[2], args[3], args[4], args[5], args[6], scaling, args[8], args[9]);
   } catch (...) {  // whatever a tensor accessor objects to: the Python path says it in its own words
+    rc = kNotHandled;
+  }
+  if (PyErr_Occurred()) PyErr_Clear();
+  if (rc == kNotHandled) ++s->passed_on;
+  else ++s->handled;
+  return PyLong_FromLong(rc);
+}
+
+// call_stacked(state, target, x, A, Bs, indices, metadata, scaling, effective_rank)
+PyObject* py_call_stacked(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 9) {
+    PyErr_SetString(PyExc_TypeError, "call_stacked() takes nine arguments");
+    return nullptr;
+  }
+  State* s = state_of(args[0]);
+  if (!s) return nullptr;
+  long rc;
+  try {
+    const double scaling = PyFloat_AsDouble(args[7]);
+    rc = PyErr_Occurred() ? kNotHandled : call_stacked(s, args[1], args[2], args[3], args[4], args[5], args[6], scaling, args[8]);
+  } catch (...) {
     rc = kNotHandled;
   }
   if (PyErr_Occurred()) PyErr_Clear();
@@ -599,12 +666,14 @@ PyObject* py_install_flush(PyObject*, PyObject* args) {
 template <typename F> PyCFunction method(F* f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
 
 PyMethodDef kMethods[] = {
+    {"call_stacked", method(py_call_stacked), METH_FASTCALL,
+     "call_stacked(state, target, x, A, Bs, indices, metadata, scaling, effective_rank) -> 0, a library error code, or NOT_HANDLED"},
     {"shrink", method(py_shrink), METH_FASTCALL, "shrink(address of mlora_shrink, inputs, weights, output, slots, scaling) -> 0, a library error code, or NOT_HANDLED"},
     {"expand", method(py_expand), METH_FASTCALL, "expand(address of mlora_expand, inputs, weights, output, slots, offset, add) -> 0, a library error code, or NOT_HANDLED"},
     {"install_batch", py_install_batch, METH_NOARGS, "install_batch() -> an empty batch of slot installs"},
     {"install_add", method(py_install_add), METH_FASTCALL, "install_add(batch, A, Bs, lora_a, lora_b, slot, rank, scaling, packed, staged, ranks, scalings, base scalings) -> bool"},
     {"install_flush", py_install_flush, METH_VARARGS, "install_flush(batch, address of mlora_install_slots) -> 0 or a library error code"},
-    {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora, address of mlora_add_workspace_bytes) -> state"},
+    {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora_active, address of mlora_add_workspace_bytes) -> state"},
     {"register_site", py_register_site, METH_VARARGS, "register_site(state, a_list, b_list, widths, block address, block owner, vectorisable) -> bool"},
     {"clear_sites", py_clear_sites, METH_O, "clear_sites(state)"},
     {"set_step", py_set_step, METH_VARARGS, "set_step(state, metadata, source, version, stream, num_slots, rows, plan address)"},

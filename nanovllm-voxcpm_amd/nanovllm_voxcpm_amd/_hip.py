@@ -53,6 +53,7 @@ _DTYPES = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: D
 
 EXPORTS = (
     "mlora_add_lora",
+    "mlora_add_lora_active",
     "mlora_add_lora_static",
     "mlora_add_workspace_bytes",
     "mlora_workspace_init",
@@ -228,6 +229,8 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(args)]
         fn.restype = C.c_int
+    lib.mlora_add_lora_active.argtypes = [C.POINTER(MloraAddArgs), C.c_int32]
+    lib.mlora_add_lora_active.restype = C.c_int
     lib.mlora_meta_build_many.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32]
     lib.mlora_meta_build_many.restype = C.c_int
     lib.mlora_install_slots.argtypes = [C.POINTER(MloraInstallArgs), C.POINTER(MloraInstallState), C.c_int32]
@@ -312,12 +315,12 @@ def load_fastcall():
 
 
 def entry_point_addresses() -> tuple[int, int] | None:
-    """Addresses of mlora_add_lora and mlora_add_workspace_bytes in the loaded library, None without it."""
+    """Addresses of mlora_add_lora_active and mlora_add_workspace_bytes in the loaded library, None without it."""
     try:
         load()
     except RuntimeError:
         return None
-    return entry_point("mlora_add_lora"), entry_point("mlora_add_workspace_bytes")
+    return entry_point("mlora_add_lora_active"), entry_point("mlora_add_workspace_bytes")
 
 
 _ADDRESSES: dict[str, int] = {}
@@ -434,13 +437,15 @@ def add_lora(
     stream: int | None = None,
     static_scratch: bool = False,
     effective_rank: torch.Tensor | None = None,
+    active_slots: int = 0,
 ) -> None:
     """y[:, col_i : col_i + n_i] += scaling * (x . A_i[slot]^T) . B_i[slot]^T for every slice.
     ``stream``: handle of the stream to launch on, torch's current one when omitted.
     ``static_scratch``: call the entry point that allocates nothing and keeps its scratch in the
     library's own device image (``workspace`` is ignored then).
     ``effective_rank``: int32 [slots] on the device, rank of the adapter resident in each slot of
-    these buffers; rows / columns at or above it are then neither read nor multiplied."""
+    these buffers; rows / columns at or above it are then neither read nor multiplied.
+    ``active_slots``: how many slots have tokens in this batch, where known."""
     lib = load()
     if len(a_slices) > MAX_SLICES:
         raise ValueError(f"at most {MAX_SLICES} slices per call, got {len(a_slices)}")
@@ -504,12 +509,12 @@ def add_lora(
         if static_scratch:
             _check(lib.mlora_add_lora_static(C.byref(args)), "mlora_add_lora_static")
         else:
-            _check(lib.mlora_add_lora(C.byref(args)), "mlora_add_lora")
+            _check(lib.mlora_add_lora_active(C.byref(args), active_slots), "mlora_add_lora")
 
 
-def call_add_lora(args: MloraAddArgs) -> None:
+def call_add_lora(args: MloraAddArgs, active_slots: int) -> None:
     """Enqueue the fused apply described by an argument block the caller filled and checked."""
-    rc = load().mlora_add_lora(C.byref(args))
+    rc = load().mlora_add_lora_active(C.byref(args), active_slots)
     if rc != 0:
         _check(rc, "mlora_add_lora")
 

@@ -185,17 +185,22 @@ class _LoRALayerBase(nn.Module):
         if token_to_slot is None:
             return base_out
         out_flat = base_out if base_out.ndim == 2 else base_out.reshape(-1, base_out.size(-1))
+        metadata, backend = self._runtime_metadata(), get_backend()
+        effective_rank = self.effective_lora_rank if self._wants_rank_masking() and getattr(backend, "takes_effective_rank", False) else None
+        in_order = block_of_target == list(range(len(block_sizes)))
+        stacked = getattr(backend, "add_lora_stacked", None)
+        if in_order and stacked is not None and stacked(out_flat, x_flat, self.lora_A, self._b_buffers(), token_to_slot, metadata, effective_rank):
+            return out_flat if x.ndim == 2 else out_flat.reshape(*x.shape[:-1], out_flat.size(-1))
         a_slices = [self._a_of(p) for p in range(len(block_of_target))]
         b_slices = [self._b_of(p) for p in range(len(block_of_target))]
-        call = dict(indices=token_to_slot, metadata=self._runtime_metadata(), scaling=1.0)
-        backend = get_backend()
-        if self._wants_rank_masking() and getattr(backend, "takes_effective_rank", False):
-            call["effective_rank"] = self.effective_lora_rank
+        call = dict(indices=token_to_slot, metadata=metadata, scaling=1.0)
+        if effective_rank is not None:
+            call["effective_rank"] = effective_rank
         if len(block_sizes) == 1:
             out_flat = backend.add_lora([out_flat], x_flat, a_slices, b_slices, **call)[0]
         else:
             blocks = list(out_flat.split(block_sizes, dim=-1))
-            if block_of_target == list(range(len(block_sizes))):
+            if in_order:
                 # every block has a target, in order: accumulate straight into the packed output
                 backend.add_lora(blocks, x_flat, a_slices, b_slices, y_packed=out_flat, **call)
             else:
@@ -300,9 +305,8 @@ class _LoRALayerBase(nn.Module):
         False, with nothing added: ``validate_slot_lora_payload`` and ``set_slot_lora`` have to see it."""
         if not self.supports_lora:
             return False
-        a, b = self._parameters.get("lora_A"), tuple([self._parameters.get(name) for name in self._b_names()])
         vectors = self._buffers
-        return fast.install_add(batch, a, b, lora_a, lora_b, slot_id, effective_rank, scaling, packed, staged,
+        return fast.install_add(batch, self.lora_A, self._b_buffers(), lora_a, lora_b, slot_id, effective_rank, scaling, packed, staged,
                                 vectors["effective_lora_rank"], vectors["lora_scaling"], vectors["lora_base_scaling"])
 
     def note_queued_slot(self, slot_id: int, effective_rank: int, scaling: float) -> None:
@@ -390,8 +394,9 @@ class _MultiTargetMixin:
     def _b_of(self, position: int) -> nn.Parameter:
         return getattr(self, f"lora_B_{self.lora_targets[position]}")
 
-    def _b_names(self) -> list[str]:
-        return [f"lora_B_{target}" for target in self.lora_targets]
+    def _b_buffers(self) -> tuple:
+        held = self._parameters
+        return tuple([held[f"lora_B_{target}"] for target in self.lora_targets])
 
     def _make_lora_b_weight_loader(self, target):
         def loader(param: nn.Parameter, loaded_weight: torch.Tensor):
@@ -540,8 +545,8 @@ class _SingleTargetMixin:
     def _b_of(self, position: int) -> nn.Parameter:
         return self.lora_B
 
-    def _b_names(self) -> list[str]:
-        return ["lora_B"]
+    def _b_buffers(self) -> tuple:
+        return (self._parameters["lora_B"],)
 
 
 class LoRARowParallelLinear(_SingleTargetMixin, _LoRALayerBase):

@@ -447,7 +447,7 @@ class HipLoRABackend:
         _STEP_HEAD.pack_into(site.view, 0, stream or 0, x_ptr, y_ptr, xs, ys, source.data_ptr(), plan_ptr, rows)
         _STEP_SCALE.pack_into(site.view, _OFF_SCALING, scaling)
         _STEP_TAIL.pack_into(site.view, _OFF_WORKSPACE, ws_ptr, ws_bytes, eff_ptr)
-        _hip.call_add_lora(args)
+        _hip.call_add_lora(args, getattr(metadata, "num_active_loras", 0))
         return True
 
     # -- the fused apply -------------------------------------------------------------------
@@ -562,10 +562,22 @@ class HipLoRABackend:
                     plan = self._plan_for(metadata, tts, a_list[0].size(0), capture).workspace
                     scratch = self._scratch_for(x2, len(chunk), a_list[0].size(-2), stream, capture)
                 _hip.add_lora(target, x2, a_list, b_list, c_list, tts, plan, float(scaling), form, scratch, stream,
-                              effective_rank=effective_rank)
+                              effective_rank=effective_rank, active_slots=getattr(metadata, "num_active_loras", 0))
         if staged is not None:
             staged.copy_(target)
         return outputs
+
+    def add_lora_stacked(self, target, x, lora_a, lora_bs, indices, metadata, effective_rank=None) -> bool:
+        """``add_lora`` for the buffers of a LoRA linear as it holds them (A of all targets in one tensor,
+        a tuple of B's) into an output made of the targets' blocks in order; False, with nothing
+        done, unless the C++ host path handles the call."""
+        fast = getattr(self._sites, "fast", None)
+        if fast is None:
+            return False
+        rc = self._fastcall.call_stacked(fast, target, x, lora_a, lora_bs, indices, metadata, 1.0, effective_rank)
+        if rc < 0:
+            _hip._check(rc, "mlora_add_lora")
+        return rc == 0
 
     # -- single-adapter helpers of the protocol -----------------------------------------------
     def shrink(self, x: torch.Tensor, lora_a: torch.Tensor) -> torch.Tensor:
