@@ -79,7 +79,8 @@ class LoRABatchPlan:
     @property
     def num_lora_tokens(self) -> int:
         slots, counts = self.runs()
-        return sum([c for s, c in zip(slots, counts) if s >= 0])
+        without = sum([c for s, c in zip(slots, counts) if s < 0]) if min(slots, default=0) < 0 else 0
+        return sum(counts) - without
 
     @property
     def active_slot_ids(self) -> list[int]:
@@ -133,7 +134,7 @@ def _upload_runs(slots: list[int], counts: list[int], n: int, device: torch.devi
     """The per-token slot ids on the device: expanded into a pinned buffer, one asynchronous copy."""
     host = torch.empty(n, dtype=torch.int32, device="cpu", pin_memory=True)
     ids = np.frombuffer(array("i", slots), dtype=np.int32)
-    host.numpy()[:] = ids if counts.count(1) == len(counts) else np.repeat(ids, counts)
+    host.numpy()[:] = ids if counts.count(1) == len(counts) else np.repeat(ids, np.frombuffer(array("q", counts), dtype=np.int64))
     return host.to(device, non_blocking=True)
 
 

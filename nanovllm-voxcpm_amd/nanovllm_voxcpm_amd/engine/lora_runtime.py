@@ -216,14 +216,15 @@ class _LoRAStateBase:
 
     # -- slots ----------------------------------------------------------------------------------
     def _refresh_slot_states(self) -> None:
+        entries, active, idle = self._entries, LoRAResidentState.ACTIVE, LoRAResidentState.IDLE
         for slot in self._slots:
             if slot.adapter_id is None:
                 continue
-            entry = self._entries.get(slot.adapter_id)
+            entry = entries.get(slot.adapter_id)
             if entry is None:
                 self._release(slot)
             else:
-                slot.resident_state = _residency(entry)
+                slot.resident_state = active if entry.gpu_running_ref_count > 0 else idle
 
     def _reclaimable(self, keep: Iterable[int]) -> list[LoRASlot]:
         """Occupied slots that may be given to another adapter: idle and not in ``keep``."""
@@ -279,14 +280,19 @@ class LoRARuntime(_LoRAStateBase):
             return build_lora_batch_plan_from_token_to_slot({}, [-1] * sum(token_counts))
         self._refresh_slot_states()
         adapter_to_slot: dict[int, int] = {}
+        # (runs for every adapter of every step: what is looked up and called per adapter is kept down)
+        entries, slots, active, idle = self._entries, self._slots, LoRAResidentState.ACTIVE, LoRAResidentState.IDLE
         for adapter_id in dict.fromkeys(adapter_ids):  # first-use order
             if adapter_id is None:
                 continue
-            entry = self.get_entry(adapter_id)
-            slot = self._slots[self._admit(entry, load_lora)]
-            adapter_to_slot[adapter_id] = slot.slot_id
-            entry.last_used_ts = slot.last_used_ts = self._tick()
-            slot.resident_state = _residency(entry)
+            entry = entries[adapter_id]
+            slot_id = entry.slot_id
+            if slot_id is None:
+                slot_id = self._admit(entry, load_lora)
+            slot = slots[slot_id]
+            adapter_to_slot[adapter_id] = slot_id
+            self._clock = entry.last_used_ts = slot.last_used_ts = self._clock + 1
+            slot.resident_state = active if entry.gpu_running_ref_count > 0 else idle
         slot_of = {None: -1, **adapter_to_slot}
         return LoRABatchPlan.from_runs(adapter_to_slot, [slot_of[a] for a in adapter_ids], list(token_counts))
 
