@@ -19,6 +19,7 @@
 // and counts the younger requests of this file's own.
 #include "common.h"
 #include "launch.h"
+#include "dma.h"
 #include "sgmv_body.h"
 
 namespace mlora {
@@ -30,25 +31,6 @@ constexpr int kPairThreads = kPairWaves * kWave;
 constexpr int kChunk = 128;     // bytes of a row that a step of the shrink takes
 constexpr int kMaxParts = 8;    // most K parts of a launch
 constexpr int kPartsAhead = 4;  // of which the expand requests this many together
-
-template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(p)));
-}
-__device__ __forceinline__ const char* uniform(const char* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-
-// One 1 KB direct load: lane i's 16 bytes at base + voff go to LDS byte lds + 16 i.
-__device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds) {
-#ifdef MLORA_TRACE
-  base = uniform(static_cast<const char*>(base));  // (the branches around the stamps cost the compiler its proof of that)
-#endif
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
 
 // ---- shrink -------------------------------------------------------------------------------------
 // A wavefront's own share of a (tile, slice, K part): chunks [c0, c1) of 128 bytes of every row, through

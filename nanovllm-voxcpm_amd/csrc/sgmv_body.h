@@ -789,7 +789,7 @@ size_t partials_room(const MloraAddArgs* a) {
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
 struct SgmvKnobs {
-  int generation = -1, kr, ksplit, all_slices, xdb, group, wgs, nt, cpl;
+  int generation = -1, kr, ksplit, all_slices, xdb, group, wgs, nt, cpl, slab;
   void read() {
     generation = knob_generation();
     kr = env_int("MLORA_SGMV_KR", 0);
@@ -800,6 +800,7 @@ struct SgmvKnobs {
     wgs = env_int("MLORA_SGMV_WGS", 2048);
     nt = env_int("MLORA_SGMV_NT", 0);
     cpl = env_int("MLORA_SGMV_CPL", 8);
+    slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay
   }
 };
 const SgmvKnobs& sgmv_knobs() {
@@ -844,6 +845,7 @@ struct SgmvShape {
   int big_cap;    // tiles below this index are 64-token tiles
   int kr, xw;     // shrink: A slab width, x batch width
   int ksplit, krange, all_slices;
+  bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
   int group;      // expand: consecutive 64-token tiles per workgroup
   int cpl;        // expand: columns per lane
   int nsplit;     // expand: column ranges
@@ -915,6 +917,35 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
   if (xw == 512 && s.krange > xw && sgmv_knobs().xdb) { xw = 256; kr = 256; }
   s.kr = kr;
   s.xw = xw;
+  // Which shrink.  Measured, us per call, this file's kernel / slab.hip's: rank 64, 9392 tokens (K = 1024): qkv
+  // 39.0 / 33.0, gate_up 85.4 / 84.7, o 25.0 / 24.6, down (K = 4096) 43.9 / 46.8; rank 64, 8192 mixed
+  // tokens: 41.8 / 39.6, 99.0 / 98.3, 24.7 / 23.5, 44.5 / 45.9; rank 64, 4000 tokens, K = 2048: qkv 35.0 / 28.4;
+  // rank 32, 5000 tokens: 19.3 / 18.5, 50.3 / 49.6, 13.6 / 13.5, 21.0 / 18.5; rank 32, 2000 tokens: 14.7 / 12.1,
+  // 21.3 / 19.3, 12.0 / 11.0, 14.3 / 13.4.  At rank 64 a workgroup of it holds half a compute unit's LDS,
+  // and what is left of the last round of long parts costs about what the operands' path saves.
+  // (Whoever asks for the two-launch form by name gets the shrink whose sums the one-launch form repeats bit by bit:
+  // slab.hip adds K up in another order.)
+  s.slab = !one_launch && slab_supported(a) &&
+           (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
+  if (s.slab) {
+    // Workgroups for half of the compute units, for most of them where a part would be long, a stage of K per
+    // wavefront at least.  Measured, us per call with one / two / four parts: rank 32, 5000 tokens, down (K =
+    // 4096): 23.4 / 18.5 / 19.2; rank 32, 2000 tokens: o 12.7 / 11.6 / 11.1, qkv 13.2 / 12.1 / 12.4; rank 64, 9392
+    // tokens, qkv 33.0 / 35.9 / 42.4.
+    s.all_slices = 0;
+    ksplit = sgmv_knobs().ksplit;
+    if (ksplit <= 0) {
+      ksplit = 1;
+      auto more = [&]() {
+        const long long wgs = static_cast<long long>(est_tiles) * a->num_slices * ksplit;
+        return wgs < 128 || (wgs < 192 && a->k / ksplit > 2048);
+      };
+      while (ksplit < kMaxKSplit && a->k / 64 >= ksplit * 2 * 4 && more()) ksplit *= 2;
+    }
+    if (ksplit > max_parts) ksplit = max_parts;
+    if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
+    s.ksplit = ksplit;
+  }
 
   // expand: consecutive tiles per workgroup (they share their B rows when they share their
   // slot), then column ranges so that the grid has about 2048 workgroups
