@@ -206,9 +206,16 @@ static bool pair_pays(const MloraAddArgs* a, int form) {
         const double width = static_cast<double>(a->num_slices) * a->k + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
         return a->k != 1024 || a->num_tokens * width > (a->r > 32 ? 1.0e7 : 2.0e7);
       }
+      // three slices and tiles for a second round of workgroups, whose every range repeats its slice's shrink
+      // (K = 1024, 600 / 1200 / 2500 tokens: rank 64 qkv 6.9 / 9.1, 15.5 / 11.1; rank 32 5.0 / 8.2, 10.5 / 9.5, 11.8 / 13.5)
+      if (a->num_slices > 2 && a->r >= 32 && a->num_tokens > 1000 && a->num_tokens < 2000) return true;
       return rk >= 131072;
     }
     case MLORA_FORM_SGMV:
+      // (up to rank 32 the 64-token tiles have the direct loads as well and win from 2200 tokens on: rank 32, 2000 /
+      // 2500 tokens, K = 4096 12.3 / 13.0, 15.8 / 14.9, K = 8192 - , 23.1 / 20.5; rank 16, 3001 tokens, K = 8192 20.5 / 19.0)
+      if (a->r <= 32 && a->num_tokens > 2200) return false;
+      return few && rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k);
     case MLORA_FORM_WIDE: return few && rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k);
     default: return false;
   }

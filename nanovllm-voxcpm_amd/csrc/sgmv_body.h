@@ -15,6 +15,7 @@ MLORA_TRACE_DECL
 
 constexpr int kMaxSplits = 64;
 constexpr int kExpandWaves = 4;
+constexpr int kSlabStages = 4;  // 128-byte pieces of K in a part of slab.hip's at least
 constexpr int kMaxKSplit = 4;  // most K parts the shrink ever uses (the workspace has room for them)
 
 struct ShrinkSlices {
@@ -928,19 +929,18 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
   s.slab = !one_launch && slab_supported(a) &&
            (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
   if (s.slab) {
-    // Workgroups for half of the compute units, for most of them where a part would be long, a stage of K per
-    // wavefront at least.  Measured, us per call with one / two / four parts: rank 32, 5000 tokens, down (K =
-    // 4096): 23.4 / 18.5 / 19.2; rank 32, 2000 tokens: o 12.7 / 11.6 / 11.1, qkv 13.2 / 12.1 / 12.4; rank 64, 9392
-    // tokens, qkv 33.0 / 35.9 / 42.4.
+    // About 205 workgroups (parts need not be a power of two), a stage of K per wavefront at least.  Measured, us
+    // per call with one / two / three / four parts, rank 32: down (K = 4096) of 2000 tokens 20.8 / 15.7 / 14.0 / 13.4,
+    // of 4000 22.3 / 17.5 / 16.6 / 18.1, of 5000 23.4 / 18.5 / 20.8 / 19.2, of 6500 29.6 / 22.4 / 25.0 / 23.1; K = 8192,
+    // 4000 tokens 48.8 / 37.5 / 32.0 / 36.1; o of 2000 tokens 12.7 / 11.6 / 11.3 / 11.1; gate_up of 6500 56.5 / 57.0 / 58.3.
     s.all_slices = 0;
     ksplit = sgmv_knobs().ksplit;
     if (ksplit <= 0) {
-      ksplit = 1;
-      auto more = [&]() {
-        const long long wgs = static_cast<long long>(est_tiles) * a->num_slices * ksplit;
-        return wgs < 128 || (wgs < 192 && a->k / ksplit > 2048);
-      };
-      while (ksplit < kMaxKSplit && a->k / 64 >= ksplit * 2 * 4 && more()) ksplit *= 2;
+      const int units = est_tiles * a->num_slices;
+      ksplit = (205 + 2 * units / 5) / units;
+      if (ksplit < 1) ksplit = 1;
+      if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
+      while (ksplit > 1 && a->k / 64 < ksplit * kSlabStages) --ksplit;
     }
     if (ksplit > max_parts) ksplit = max_parts;
     if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
