@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from nanovllm_voxcpm_amd import _hip
 from nanovllm_voxcpm_amd.lora import LoRAMetadata, get_backend
-from nanovllm_voxcpm_amd.utils.context import LM_LORA_DOMAIN, get_lora_context
+from nanovllm_voxcpm_amd.utils.context import LM_LORA_DOMAIN, get_lora_context, installed_lora_context
 
 ShardId = str | int
 
@@ -81,6 +81,7 @@ class _LoRALayerBase(nn.Module):
         self._effective_lora_rank_values = [0] * max_loras
         self._rank_summary_of: list | None = None  # the mirror the summary below was made from
         self._rank_summary = (False, False)
+        self._targets_in_order = True  # every output block has a target, in order
 
     # ---- subclass contract ------------------------------------------------------------------
     def _target_keys(self) -> list:
@@ -174,6 +175,26 @@ class _LoRALayerBase(nn.Module):
         return meta  # type: ignore[return-value]
 
     # ---- the LoRA half of forward -------------------------------------------------------------
+    def _add_lora_quickly(self, x: torch.Tensor, out: torch.Tensor) -> bool:
+        """The usual forward of a step whose first linear has been through ``_add_lora``: nothing about it is
+        new, and the C++ host path takes the layer's buffers as they are.  False, with nothing done,
+        for everything else (and whatever has to raise), which ``_add_lora`` then sees to."""
+        context = installed_lora_context(self.lora_domain)
+        if context is None or context.no_lora_flag or not self.supports_lora or not self._targets_in_order or x.dim() != 2:
+            return False
+        metadata, slots, active = context._cached_metadata, context.token_to_slot, context.active_slot_ids
+        if metadata is None or slots is None or metadata.token_to_slot is not slots or metadata.no_lora_flag or slots.size(0) != x.size(0):
+            return False
+        if active is not None and not active.is_cuda:
+            return False
+        some_resident, some_below = self._residency()
+        backend = get_backend()
+        stacked = getattr(backend, "add_lora_stacked", None)
+        if not some_resident or stacked is None:
+            return False
+        ranks = self._buffers["effective_lora_rank"] if some_below and self.max_lora_rank > 16 and backend.takes_effective_rank else None
+        return stacked(out, x, self._parameters["lora_A"], self._b_buffers(), slots, metadata, ranks)
+
     def _add_lora(self, x: torch.Tensor, base_out: torch.Tensor, block_sizes: list[int], block_of_target: list[int]):
         """Add every target's update to its column block of ``base_out``.
 
@@ -188,9 +209,6 @@ class _LoRALayerBase(nn.Module):
         metadata, backend = self._runtime_metadata(), get_backend()
         effective_rank = self.effective_lora_rank if self._wants_rank_masking() and getattr(backend, "takes_effective_rank", False) else None
         in_order = block_of_target == list(range(len(block_sizes)))
-        stacked = getattr(backend, "add_lora_stacked", None)
-        if in_order and stacked is not None and stacked(out_flat, x_flat, self.lora_A, self._b_buffers(), token_to_slot, metadata, effective_rank):
-            return out_flat if x.ndim == 2 else out_flat.reshape(*x.shape[:-1], out_flat.size(-1))
         a_slices = [self._a_of(p) for p in range(len(block_of_target))]
         b_slices = [self._b_of(p) for p in range(len(block_of_target))]
         call = dict(indices=token_to_slot, metadata=metadata, scaling=1.0)
@@ -396,7 +414,7 @@ class _MultiTargetMixin:
 
     def _b_buffers(self) -> tuple:
         held = self._parameters
-        return tuple([held[f"lora_B_{target}"] for target in self.lora_targets])
+        return tuple([held[name] for name in self._b_names])
 
     def _make_lora_b_weight_loader(self, target):
         def loader(param: nn.Parameter, loaded_weight: torch.Tensor):
@@ -408,6 +426,7 @@ class _MultiTargetMixin:
         return loader
 
     def _alloc_lora(self, in_dim: int, out_dim_of: dict) -> None:
+        self._b_names = [f"lora_B_{target}" for target in self.lora_targets]
         self.target_to_index = {target: idx for idx, target in enumerate(self.lora_targets)}
         if not self.supports_lora:
             return
@@ -465,6 +484,7 @@ class LoRAQKVParallelLinear(_MultiTargetMixin, _LoRALayerBase):
         else:
             self.register_parameter("bias", None)
         self.lora_targets = targets
+        self._targets_in_order = targets == ["q", "k", "v"]
         self._alloc_lora(hidden_size, {"q": self.q_size, "k": self.kv_size, "v": self.kv_size})
 
     def _base_weight_loader(self, param: nn.Parameter, loaded_weight: torch.Tensor, loaded_shard_id: ShardId | None = None):
@@ -478,6 +498,8 @@ class LoRAQKVParallelLinear(_MultiTargetMixin, _LoRALayerBase):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         qkv = F.linear(x, self.weight, self.bias)
+        if self._add_lora_quickly(x, qkv):
+            return qkv
         blocks = [self._BLOCK[t] for t in self.lora_targets]
         return self._add_lora(x, qkv, [self.q_size, self.kv_size, self.kv_size], blocks)
 
@@ -516,6 +538,7 @@ class LoRAMergedColumnParallelLinear(_MultiTargetMixin, _LoRALayerBase):
         else:
             self.register_parameter("bias", None)
         self.lora_targets = targets
+        self._targets_in_order = targets == list(range(len(output_sizes)))
         self._alloc_lora(input_size, dict(enumerate(self.shard_output_sizes)))
 
     def _base_weight_loader(self, param: nn.Parameter, loaded_weight: torch.Tensor, loaded_shard_id: ShardId | None = None):
@@ -529,6 +552,8 @@ class LoRAMergedColumnParallelLinear(_MultiTargetMixin, _LoRALayerBase):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         out = F.linear(x, self.weight, self.bias)
+        if self._add_lora_quickly(x, out):
+            return out
         return self._add_lora(x, out, list(self.shard_output_sizes), list(self.lora_targets))
 
     def validate_slot_lora_payload(self, lora_a, lora_b, effective_rank: int, scaling: float) -> None:
@@ -593,7 +618,8 @@ class LoRARowParallelLinear(_SingleTargetMixin, _LoRALayerBase):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = F.linear(x, self.weight, self.bias if self.tp_rank == 0 else None)
-        y = self._add_lora(x, y, [self.output_size], [0])
+        if not self._add_lora_quickly(x, y):
+            y = self._add_lora(x, y, [self.output_size], [0])
         if self.tp_size > 1 and dist.is_available() and dist.is_initialized():
             dist.all_reduce(y)
         return y
@@ -629,6 +655,8 @@ class LoRALinear(_SingleTargetMixin, _LoRALayerBase):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = F.linear(x, self.weight, self.bias)
+        if self._add_lora_quickly(x, y):
+            return y
         return self._add_lora(x, y, [self.out_features], [0])
 
     def validate_slot_lora_payload(self, lora_a, lora_b, effective_rank: int, scaling: float) -> None:

@@ -47,6 +47,11 @@ def get_lora_context(domain: str = LM_LORA_DOMAIN) -> LoRAContext:
     return ctx if ctx is not None else LoRAContext()
 
 
+def installed_lora_context(domain: str) -> LoRAContext | None:
+    """The domain's context, None when none is installed."""
+    return _DOMAINS.get(domain)
+
+
 def set_lora_context(lora_context: LoRAContext, *, domain: str = LM_LORA_DOMAIN) -> None:
     invalidate_lora_context(lora_context)
     _DOMAINS[domain] = lora_context
