@@ -296,6 +296,12 @@ int mlora_meta_build(const MloraMetaArgs* args);
 /* Several independent batches (the domains of a step) in one launch, all on the stream of the first. */
 #define MLORA_META_BATCH 4
 int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count);
+/* The same for one batch known on the host as runs of tokens (slot id and token count each), which travel with
+ * the launch: token_to_slot of the entries is not read, padded_token_to_slot puts the vector on the device.
+ * At most MLORA_META_RUNS runs, or MLORA_META_SINGLES when every run is one token. */
+#define MLORA_META_RUNS 336
+#define MLORA_META_SINGLES 1024
+int mlora_meta_build_runs(const MloraMetaArgs* list, int32_t count, const int32_t* run_slots, const int32_t* run_counts, int32_t runs);
 
 /* Fused slot install:  A[slot, :, :] = 0; A[slot, 0:rank, :] = a_src[0:rank, :];
  * B[slot, :, :] = 0; B[slot, :, 0:rank] = b_src[:, 0:rank] * scaling  in one launch.

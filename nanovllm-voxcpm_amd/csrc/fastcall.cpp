@@ -52,7 +52,7 @@ struct State {
   const PyObject* source = nullptr;
   uint32_t version = 0;
   void* stream = nullptr;
-  int num_slots = 0;
+  int num_slots = 0, active_slots = 0;
   int64_t rows = -1;
   const void* plan = nullptr;
   // the eager scratch buffer of a stream
@@ -170,21 +170,21 @@ PyObject* py_clear_sites(PyObject*, PyObject* cap) {
   Py_RETURN_NONE;
 }
 
-// set_step(state, metadata, source, version, stream, num_slots, rows, plan address): what a call
+// set_step(state, metadata, source, version, stream, num_slots, rows, plan address, active slots): what a call
 // outside any capture looked up; the caller keeps metadata, source and the plan alive for as long
 // as this stands.  forget_step(state) withdraws it.
 PyObject* py_set_step(PyObject*, PyObject* args) {
   PyObject *cap, *metadata, *source;
   unsigned long version = 0;
   unsigned long long stream = 0, plan = 0;
-  int num_slots = 0;
+  int num_slots = 0, active_slots = 0;
   long long rows = 0;
-  if (!PyArg_ParseTuple(args, "OOOkKiLK", &cap, &metadata, &source, &version, &stream, &num_slots, &rows, &plan)) return nullptr;
+  if (!PyArg_ParseTuple(args, "OOOkKiLKi", &cap, &metadata, &source, &version, &stream, &num_slots, &rows, &plan, &active_slots)) return nullptr;
   State* s = state_of(cap);
   if (!s) return nullptr;
   s->metadata = metadata; s->source = source; s->version = static_cast<uint32_t>(version);
   s->stream = reinterpret_cast<void*>(static_cast<uintptr_t>(stream));
-  s->num_slots = num_slots; s->rows = rows;
+  s->num_slots = num_slots; s->rows = rows; s->active_slots = active_slots < 0 ? 0 : active_slots;
   s->plan = reinterpret_cast<const void*>(static_cast<uintptr_t>(plan));
   Py_RETURN_NONE;
 }
@@ -229,11 +229,6 @@ long call_at(State* s, const Site& site, PyObject* x_obj, PyObject* target_obj, 
   const int no_lora = PyObject_IsTrue(flag);
   Py_DECREF(flag);
   if (no_lora != 0) { PyErr_Clear(); return kNotHandled; }
-  static PyObject* const kActive = PyUnicode_InternFromString("num_active_loras");
-  const Ref active{PyObject_GetAttr(metadata, kActive)};
-  long active_slots = active.p ? PyLong_AsLong(active.p) : 0;
-  if (PyErr_Occurred()) PyErr_Clear();
-  if (active_slots < 0 || active_slots > INT32_MAX) active_slots = 0;  // (not known)
   const Ref tts{PyObject_GetAttr(metadata, kSlots)};
   if (!tts.p) { PyErr_Clear(); return kNotHandled; }
   PyObject* source_obj = tts.p != Py_None ? tts.p : indices;
@@ -301,7 +296,7 @@ long call_at(State* s, const Site& site, PyObject* x_obj, PyObject* target_obj, 
   a->workspace = ws;
   a->workspace_bytes = ws_bytes;
   a->effective_rank = static_cast<const int32_t*>(eff_ptr);
-  return s->add_lora(a, static_cast<int32_t>(active_slots));
+  return s->add_lora(a, plan ? s->active_slots : 0);
 }
 
 // A call with lists of slices.
@@ -525,6 +520,81 @@ template <typename F> PyObject* run_op(F f, PyObject* const* args, Py_ssize_t na
 PyObject* py_shrink(PyObject*, PyObject* const* args, Py_ssize_t nargs) { return run_op(op_shrink, args, nargs, 6); }
 PyObject* py_expand(PyObject*, PyObject* const* args, Py_ssize_t nargs) { return run_op(op_expand, args, nargs, 7); }
 
+// ---- batch contexts --------------------------------------------------------------------------------------
+// The runs of a batch (slot ids and token counts as Python lists) as arrays.
+bool read_runs(PyObject* slots, PyObject* counts, std::vector<int32_t>* s, std::vector<int32_t>* c) {
+  if (!PyList_Check(slots) || !PyList_Check(counts) || PyList_GET_SIZE(slots) != PyList_GET_SIZE(counts)) return false;
+  const Py_ssize_t n = PyList_GET_SIZE(slots);
+  if (n > MLORA_META_SINGLES) return false;
+  s->resize(static_cast<size_t>(n));
+  c->resize(static_cast<size_t>(n));
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const long a = PyLong_AsLong(PyList_GET_ITEM(slots, i)), b = PyLong_AsLong(PyList_GET_ITEM(counts, i));
+    if ((a == -1 || b == -1) && PyErr_Occurred()) return false;
+    if (b < 0 || b > INT32_MAX || a < INT32_MIN || a > INT32_MAX) return false;
+    (*s)[static_cast<size_t>(i)] = static_cast<int32_t>(a);
+    (*c)[static_cast<size_t>(i)] = static_cast<int32_t>(b);
+  }
+  return true;
+}
+
+// run_totals(slots, counts) -> (tokens, tokens with a slot, slots with tokens, largest slot with tokens), or None for
+// what the Python path has to see to
+PyObject* py_run_totals(PyObject*, PyObject* args) {
+  PyObject *slots, *counts;
+  if (!PyArg_ParseTuple(args, "OO", &slots, &counts)) return nullptr;
+  std::vector<int32_t> s, c;
+  if (!read_runs(slots, counts, &s, &c)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  long long tokens = 0, with_slot = 0;
+  int active = 0, largest = -1;
+  bool seen[MLORA_MAX_SLOTS] = {}, singles = true;
+  for (size_t i = 0; i < s.size(); ++i) {
+    tokens += c[i];
+    singles &= c[i] == 1;
+    if (s[i] < 0 || c[i] == 0) continue;
+    if (s[i] >= MLORA_MAX_SLOTS) Py_RETURN_NONE;
+    with_slot += c[i];
+    if (!seen[s[i]]) { seen[s[i]] = true; ++active; }
+    if (s[i] > largest) largest = s[i];
+  }
+  if (tokens > INT32_MAX || (!singles && s.size() > MLORA_META_RUNS)) Py_RETURN_NONE;
+  return Py_BuildValue("LLii", tokens, with_slot, active, largest);
+}
+
+// build_context(address of mlora_meta_build_runs, slots, counts, device index, max_slots, capacity, addresses of slot vector, sorted
+// indices, ids, counts, offsets and plan) -> 0 or a library error code: slot vector, index arrays and plan in one launch on
+// the current stream
+PyObject* py_build_context(PyObject*, PyObject* args) {
+  PyObject *slots, *counts;
+  unsigned long long fn, tts, sorted, ids, per_slot, offsets, plan;
+  int device, max_slots, capacity;
+  if (!PyArg_ParseTuple(args, "KOOiiiKKKKKK", &fn, &slots, &counts, &device, &max_slots, &capacity, &tts, &sorted, &ids, &per_slot, &offsets, &plan))
+    return nullptr;
+  std::vector<int32_t> s, c;
+  if (!read_runs(slots, counts, &s, &c)) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "runs of a batch: two lists of equal length");
+    return nullptr;
+  }
+  int64_t tokens = 0;
+  for (const int32_t n : c) tokens += n;
+  MloraMetaArgs a[2] = {};
+  auto at = [](unsigned long long address) { return reinterpret_cast<int32_t*>(static_cast<uintptr_t>(address)); };
+  a[0].stream = a[1].stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+  a[0].num_tokens = a[1].num_tokens = static_cast<int32_t>(tokens);
+  a[0].max_slots = a[1].max_slots = max_slots;
+  a[0].padded_token_to_slot = at(tts);
+  a[0].padded_len = static_cast<int32_t>(tokens);
+  a[0].sorted_idx = at(sorted);
+  a[0].compact_ids = at(ids); a[0].compact_counts = at(per_slot); a[0].compact_offsets = at(offsets);
+  a[0].compact_capacity = capacity;
+  a[1].plan = at(plan);
+  return PyLong_FromLong(reinterpret_cast<int (*)(const MloraMetaArgs*, int32_t, const int32_t*, const int32_t*, int32_t)>(static_cast<uintptr_t>(fn))(
+      a, 2, s.data(), c.data(), static_cast<int32_t>(s.size())));
+}
+
 // ---- slot installs -----------------------------------------------------------------------------------
 // An adapter's targets, collected module by module and handed to mlora_install_slots together.
 struct InstallBatch {
@@ -670,13 +740,15 @@ PyMethodDef kMethods[] = {
      "call_stacked(state, target, x, A, Bs, indices, metadata, scaling, effective_rank) -> 0, a library error code, or NOT_HANDLED"},
     {"shrink", method(py_shrink), METH_FASTCALL, "shrink(address of mlora_shrink, inputs, weights, output, slots, scaling) -> 0, a library error code, or NOT_HANDLED"},
     {"expand", method(py_expand), METH_FASTCALL, "expand(address of mlora_expand, inputs, weights, output, slots, offset, add) -> 0, a library error code, or NOT_HANDLED"},
+    {"run_totals", py_run_totals, METH_VARARGS, "run_totals(slots, counts) -> (tokens, with a slot, active slots, largest slot) or None"},
+    {"build_context", py_build_context, METH_VARARGS, "build_context(address of mlora_meta_build_runs, slots, counts, device, max_slots, capacity, six addresses) -> rc"},
     {"install_batch", py_install_batch, METH_NOARGS, "install_batch() -> an empty batch of slot installs"},
     {"install_add", method(py_install_add), METH_FASTCALL, "install_add(batch, A, Bs, lora_a, lora_b, slot, rank, scaling, packed, staged, ranks, scalings, base scalings) -> bool"},
     {"install_flush", py_install_flush, METH_VARARGS, "install_flush(batch, address of mlora_install_slots) -> 0 or a library error code"},
     {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora_active, address of mlora_add_workspace_bytes) -> state"},
     {"register_site", py_register_site, METH_VARARGS, "register_site(state, a_list, b_list, widths, block address, block owner, vectorisable) -> bool"},
     {"clear_sites", py_clear_sites, METH_O, "clear_sites(state)"},
-    {"set_step", py_set_step, METH_VARARGS, "set_step(state, metadata, source, version, stream, num_slots, rows, plan address)"},
+    {"set_step", py_set_step, METH_VARARGS, "set_step(state, metadata, source, version, stream, num_slots, rows, plan address, active slots)"},
     {"forget_step", py_forget_step, METH_O, "forget_step(state)"},
     {"set_scratch", py_set_scratch, METH_VARARGS, "set_scratch(state, device index, stream, address, bytes)"},
     {"counters", py_counters, METH_O, "counters(state) -> (calls enqueued here, calls left to the Python path)"},

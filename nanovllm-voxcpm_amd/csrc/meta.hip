@@ -62,14 +62,24 @@ __device__ __forceinline__ int find_bucket(const int* arr, int n, int q) {
 // Several batches share a launch: each has a workgroup of its own.
 struct MetaTable { MetaParams p[MLORA_META_BATCH]; };
 
+// The batch's slot ids by value: one per token, or runs of tokens (the slot of each and where it ends).  They
+// come with the launch, so that no pinned buffer has to be filled and no copy has to run before it.
+struct RunTable {
+  int runs, singles;  // singles: every run is one token
+  union {
+    int16_t slot_of_token[MLORA_META_SINGLES];
+    struct { int32_t end[MLORA_META_RUNS]; int16_t slot[MLORA_META_RUNS]; } run;
+  };
+};
+static_assert(sizeof(RunTable) + sizeof(MetaTable) <= 4096, "both are kernel arguments");
+
 // What bounds it: the latency of one workgroup's chain - slot ids from memory, histogram, scans, stores -
 // and the 1.6 us of being a launch at all.  A decode step runs it for the batch's context, for the graph
 // buffers of every domain and for the plan, so at one to 512 tokens it is the microseconds of the chain
 // that count: the slot ids are requested once and first of all, scans go through DPP moves, and no
 // barrier waits for stores unless something is stored to twice.
-__global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
-  extern __shared__ int lds[];
-  const MetaParams p = table.p[blockIdx.x];
+template <typename F>
+__device__ __forceinline__ void meta_batch(const MetaParams& p, int* lds, F&& slot_of) {
   const int NB = p.L + 1;  // bucket b holds slot b - 1; bucket 0 is "no LoRA"
   int* hist = lds;                     // [waves][NB]: per-wave counts, later running write cursors
   int* total = hist + kMetaWaves * NB; // [NB]
@@ -100,7 +110,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) {
     const int t = beg + j * kWave + lane;
-    held[j] = t < end ? p.tts[t] : -1;
+    held[j] = t < end ? slot_of(t) : -1;
   }
   for (int i = tid; i < kMetaWaves * NB; i += kMetaThreads) hist[i] = 0;
   if (tid == 0) { s_bad = 0; s_max = 0; }
@@ -115,7 +125,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
         const int t = base + j * kWave + lane;
         const int s = q[j];
         const int tn = t + kAhead * kWave;
-        q[j] = tn < end ? p.tts[tn] : -1;
+        q[j] = tn < end ? slot_of(tn) : -1;
         if (base + j * kWave < end) step(t, s);
       }
     }
@@ -128,7 +138,7 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
     }
   });
   if (p.padded_tts) {
-    for (int i = tid; i < p.padded_len; i += kMetaThreads) p.padded_tts[i] = i < T ? p.tts[i] : -1;
+    for (int i = tid; i < p.padded_len; i += kMetaThreads) p.padded_tts[i] = i < T ? slot_of(i) : -1;
   }
   lds_barrier();
 
@@ -370,6 +380,35 @@ __global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
   });
 }
 
+__global__ __launch_bounds__(kMetaThreads) void meta_kernel(MetaTable table) {
+  extern __shared__ int lds[];
+  const MetaParams p = table.p[blockIdx.x];
+  meta_batch(p, lds, [&](int t) { return p.tts[t]; });
+}
+
+__global__ __launch_bounds__(kMetaThreads) void meta_runs_kernel(MetaTable table, RunTable given) {
+  extern __shared__ int lds[];
+  __shared__ int s_end[MLORA_META_RUNS], s_slot[MLORA_META_RUNS];
+  const MetaParams p = table.p[blockIdx.x];
+  if (given.singles) {
+    meta_batch(p, lds, [&](int t) { return static_cast<int>(given.slot_of_token[t]); });
+    return;
+  }
+  for (int r = threadIdx.x; r < given.runs; r += kMetaThreads) {
+    s_end[r] = given.run.end[r];
+    s_slot[r] = given.run.slot[r];
+  }
+  lds_barrier();
+  meta_batch(p, lds, [&](int t) {
+    int lo = 0, hi = given.runs - 1;  // the first run that ends behind t
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (s_end[mid] > t) hi = mid; else lo = mid + 1;
+    }
+    return s_slot[lo];
+  });
+}
+
 }  // namespace
 
 }  // namespace mlora
@@ -383,14 +422,14 @@ extern "C" size_t mlora_plan_workspace_bytes(int32_t num_tokens, int32_t max_slo
 
 namespace {
 
-int check_meta(const MloraMetaArgs* a) {
+int check_meta(const MloraMetaArgs* a, bool by_value) {
   if (a->num_tokens < 0 || a->max_slots < 0 || a->compact_capacity < 0 || a->padded_len < 0) {
     set_error("mlora_meta_build: negative size"); return MLORA_E_INVALID;
   }
   if (a->max_slots > MLORA_MAX_SLOTS) {
     set_error("mlora_meta_build: max_slots=%d exceeds %d", a->max_slots, MLORA_MAX_SLOTS); return MLORA_E_TOO_LARGE;
   }
-  if (a->num_tokens > 0 && !a->token_to_slot) { set_error("mlora_meta_build: NULL token_to_slot"); return MLORA_E_INVALID; }
+  if (a->num_tokens > 0 && !a->token_to_slot && !by_value) { set_error("mlora_meta_build: NULL token_to_slot"); return MLORA_E_INVALID; }
   if (reinterpret_cast<uintptr_t>(a->plan) & 15) { set_error("mlora_meta_build: plan must be 16-byte aligned"); return MLORA_E_INVALID; }
   if (a->padded_token_to_slot && a->padded_len < a->num_tokens) {
     set_error("mlora_meta_build: padded_len=%d is shorter than num_tokens=%d", a->padded_len, a->num_tokens);
@@ -409,10 +448,12 @@ int check_meta(const MloraMetaArgs* a) {
 
 }  // namespace
 
-extern "C" int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count) {
+namespace {
+
+int build_many(const MloraMetaArgs* list, int32_t count, const RunTable* given) {
   if (count < 0 || (count > 0 && !list)) { set_error("mlora_meta_build: NULL args"); return MLORA_E_INVALID; }
   for (int i = 0; i < count; ++i) {
-    if (int rc = check_meta(list + i)) return rc;
+    if (int rc = check_meta(list + i, given != nullptr)) return rc;
   }
   for (int first = 0; first < count; first += MLORA_META_BATCH) {
     const int n = count - first < MLORA_META_BATCH ? count - first : MLORA_META_BATCH;
@@ -433,10 +474,50 @@ extern "C" int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count) {
       lds = need > lds ? need : lds;
     }
     for (int i = n; i < MLORA_META_BATCH; ++i) table.p[i] = table.p[0];  // (not in the grid)
-    hipLaunchKernelGGL(meta_kernel, dim3(n), dim3(kMetaThreads), lds, static_cast<hipStream_t>(list[0].stream), table);
+    hipStream_t st = static_cast<hipStream_t>(list[0].stream);
+    if (given) hipLaunchKernelGGL(meta_runs_kernel, dim3(n), dim3(kMetaThreads), lds, st, table, *given);
+    else hipLaunchKernelGGL(meta_kernel, dim3(n), dim3(kMetaThreads), lds, st, table);
     if (int rc = check_launch("mlora_meta_build")) return rc;
   }
   return 0;
+}
+
+}  // namespace
+
+extern "C" int mlora_meta_build_many(const MloraMetaArgs* list, int32_t count) { return build_many(list, count, nullptr); }
+
+extern "C" int mlora_meta_build_runs(const MloraMetaArgs* list, int32_t count, const int32_t* run_slots, const int32_t* run_counts, int32_t runs) {
+  if (count < 0 || runs < 0 || (count > 0 && !list) || (runs > 0 && (!run_slots || !run_counts))) {
+    set_error("mlora_meta_build_runs: NULL args"); return MLORA_E_INVALID;
+  }
+  RunTable t;
+  t.runs = runs;
+  t.singles = 1;
+  int64_t total = 0;
+  for (int i = 0; i < runs; ++i) {
+    if (run_counts[i] < 0) { set_error("mlora_meta_build_runs: run %d has a negative count", i); return MLORA_E_INVALID; }
+    t.singles &= run_counts[i] == 1;
+    total += run_counts[i];
+  }
+  for (int i = 0; i < count; ++i) {
+    if (list[i].num_tokens != total) {
+      set_error("mlora_meta_build_runs: the runs hold %lld tokens, batch %d has %d", static_cast<long long>(total), i, list[i].num_tokens);
+      return MLORA_E_INVALID;
+    }
+  }
+  if (runs > (t.singles ? MLORA_META_SINGLES : MLORA_META_RUNS)) { set_error("mlora_meta_build_runs: %d runs", runs); return MLORA_E_TOO_LARGE; }
+  int end = 0;
+  for (int i = 0; i < runs; ++i) {
+    const int slot = run_slots[i] < -1 ? -1 : run_slots[i] > 0x7fff ? 0x7fff : run_slots[i];  // (no slot; beyond every slot)
+    end += run_counts[i];
+    if (t.singles) {
+      t.slot_of_token[i] = static_cast<int16_t>(slot);
+    } else {
+      t.run.end[i] = end;
+      t.run.slot[i] = static_cast<int16_t>(slot);
+    }
+  }
+  return build_many(list, count, &t);
 }
 
 extern "C" int mlora_meta_build(const MloraMetaArgs* a) {

@@ -26,6 +26,8 @@ FORM_AUTO, FORM_TOKEN, FORM_BGMV, FORM_SGMV, FORM_MFMA, FORM_SPLIT, FORM_FUSED, 
 FORMS = {"auto": FORM_AUTO, "token": FORM_TOKEN, "bgmv": FORM_BGMV, "sgmv": FORM_SGMV, "mfma": FORM_MFMA, "split": FORM_SPLIT,
          "fused": FORM_FUSED, "slot": FORM_SLOT, "wide": FORM_WIDE, "pair": FORM_PAIR}
 
+META_RUNS, META_SINGLES = 336, 1024  # most runs of a batch whose slot ids travel with the metadata launch
+
 PLAN_HEADER_WORDS = 16
 (
     PLAN_MAGIC,
@@ -62,6 +64,7 @@ EXPORTS = (
     "mlora_plan_workspace_bytes",
     "mlora_meta_build",
     "mlora_meta_build_many",
+    "mlora_meta_build_runs",
     "mlora_install_slot",
     "mlora_install_slots",
     "mlora_stream_capture_id",
@@ -233,6 +236,8 @@ def load() -> C.CDLL:
     lib.mlora_add_lora_active.restype = C.c_int
     lib.mlora_meta_build_many.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32]
     lib.mlora_meta_build_many.restype = C.c_int
+    lib.mlora_meta_build_runs.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32, C.c_void_p, C.c_void_p, C.c_int32]
+    lib.mlora_meta_build_runs.restype = C.c_int
     lib.mlora_install_slots.argtypes = [C.POINTER(MloraInstallArgs), C.POINTER(MloraInstallState), C.c_int32]
     lib.mlora_install_slots.restype = C.c_int
     lib.mlora_plan_workspace_bytes.argtypes = [C.c_int32, C.c_int32]

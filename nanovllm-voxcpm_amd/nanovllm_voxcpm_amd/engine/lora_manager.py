@@ -138,16 +138,52 @@ def _upload_runs(slots: list[int], counts: list[int], n: int, device: torch.devi
     return host.to(device, non_blocking=True)
 
 
+def _context_in_one_launch(slots: list[int], counts: list[int], max_slots: int | None, device: torch.device | str) -> LoRAContext | None:
+    """The context of a batch whose runs fit the arguments of the metadata launch; None (nothing done) for others."""
+    fast = _hip.load_fastcall()
+    if fast is None or not torch.cuda.is_initialized():
+        return None
+    totals = fast.run_totals(slots, counts)
+    if totals is None:
+        return None
+    n, n_lora, n_active, largest = totals
+    if max_slots is None:
+        max_slots = largest + 1
+    if n_active == 0 or largest >= max_slots:
+        return None
+    cap = min(n, max_slots)
+    # slot vector | sorted indices | ids | counts | offsets | plan (its start on a 256-byte boundary)
+    head = (2 * n + 3 * cap + 1 + 63) & ~63
+    words = _hip.plan_workspace_words(n, max_slots)
+    packed = torch.empty(head + words, dtype=torch.int32, device=device)
+    index = packed.device.index
+    if index is None or index != _hip.current_device_index():
+        return None
+    tts, sorted_idx, _, ids, _, per_slot, _, offsets, _, workspace = packed.split_with_sizes(
+        [n, n_lora, n - n_lora, n_active, cap - n_active, n_active, cap - n_active, n_active + 1, head - 2 * n - 2 * cap - n_active - 1, words])
+    at = packed.data_ptr()
+    rc = fast.build_context(_hip.entry_point("mlora_meta_build_runs"), slots, counts, index, max_slots, cap, at, at + 4 * n, at + 8 * n,
+                            at + 8 * n + 4 * cap, at + 8 * n + 8 * cap, at + 4 * head)
+    _hip._check(rc, "mlora_meta_build_runs")
+    attach_plan(tts, workspace, max_slots)
+    return LoRAContext(token_to_slot=tts, token_indices_sorted_by_slot=sorted_idx, active_slot_ids=ids, num_tokens_per_slot=per_slot,
+                       slot_start_offsets=offsets, no_lora_flag=False, num_active_loras=n_active)
+
+
 def build_lora_context_from_batch_plan(
     plan: LoRABatchPlan,
     *,
     max_slots: int | None = None,
     device: torch.device | str = "cuda",
 ) -> LoRAContext:
-    """One H2D copy of the slot ids, one metadata launch, no device->host traffic: the array
-    lengths and the two host flags come from the host list the plan already holds.  A second
-    workgroup of the launch builds the segment plan of eager calls, which costs no time of its own."""
+    """One metadata launch, no device->host traffic: the array lengths and the two host flags come
+    from the host list the plan already holds.  A second workgroup of the launch builds the segment
+    plan of eager calls, which costs no time of its own.  The slot ids travel with the launch, those of batches
+    of very many sequences through one H2D copy ahead of it."""
     slots, counts = plan.runs()
+    context = _context_in_one_launch(slots, counts, max_slots, device)
+    if context is not None:
+        return context
     n = sum(counts)
     tts = _upload_runs(slots, counts, n, device) if n else torch.empty(0, dtype=torch.int32, device=device)
     active = plan.active_slot_ids

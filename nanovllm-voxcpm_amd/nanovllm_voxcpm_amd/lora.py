@@ -435,7 +435,8 @@ class HipLoRABackend:
                     if capture or version is None:
                         self._fastcall.forget_step(fast)
                     else:  # (the tuple above keeps metadata, slot vector and plan alive for as long as this stands)
-                        self._fastcall.set_step(fast, metadata, source, version, stream or 0, site.num_slots, rows, plan_ptr)
+                        self._fastcall.set_step(fast, metadata, source, version, stream or 0, site.num_slots, rows, plan_ptr,
+                                                getattr(metadata, "num_active_loras", 0))
             scratch = self._scratch_for(x, site.num_slices, site.rank, stream, capture)
             ws_ptr, ws_bytes = scratch.data_ptr(), scratch.numel()
             if not capture:
