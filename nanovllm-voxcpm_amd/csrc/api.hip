@@ -169,6 +169,10 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   if (a->num_slots > knobs().slot_max_slots) return false;
   if (a->num_tokens > 32 * a->num_slots) return false;
   const bool sparse = active > 0 && 2 * active <= a->num_slots;
+  // Eight parts (K = 8192) are twice the workgroups of a tile, and past one per compute unit they wait for
+  // each other in two rounds (slot-major / the pair: rank 32: 5.4 / 7.2 at 8 slot ids, 11.5 / 10.9 at 32; rank 16: 5.7 /
+  // 7.1 at 16, 9.3 / 9.7 at 32, 9.9 / 8.5 at 40; rank 64: 9.0 / 9.6 at 8, 18.4 / 16.4 at 32).
+  if (slot_k_parts(a) > 4) return a->num_slots <= 32 && a->num_slots * compute_rank(a->r) <= 640;
   if (slot_k_parts(a) > 1) return a->num_slots <= (a->r <= 16 ? 32 : 48) && !(sparse && a->r * a->num_slots >= 2048);
   if (sparse || (active > 0 && a->num_tokens > MLORA_TILE_SMALL * active)) return false;
   double cols = 0;
@@ -335,7 +339,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "
-                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or with one slice of at most 4096 columns and an "
+                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or (4096 and 8192) with one slice of at most 4096 columns and an "
                     "initialised workspace");
           return MLORA_E_UNSUPPORTED;
         }

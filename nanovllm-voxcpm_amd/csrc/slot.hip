@@ -25,7 +25,7 @@
 // (z beyond the slot layers), which learn their slot from their record like the tile-major
 // kernel: a batch with every token on one adapter spreads over as many workgroups as before.
 //
-// Long K (KP > 1).  What a compute unit can take in per unit of time is what bounds a decode
+// Long K (KP > 1; KP = 8 at K = 8192).  What a compute unit can take in per unit of time is what bounds a decode
 // launch (about 35 bytes per cycle, whether the lines come from HBM or from the L2), and with one
 // workgroup per column range every range pulls ALL of x's tile and of A[slot]: at K = 4096 that is
 // 256 KB per workgroup against 16 KB of B and y.  With KP > 1 the KP workgroups of a tile each take
@@ -717,19 +717,21 @@ void launch_spans(const Launch& l) {
 
 template <typename T, int R, int KSPW, int KP>
 void launch_one(const Launch& l) {
+  const bool one_span = KP == 8 || l.widest <= kNW * 64;
+  constexpr int kTwo = KP == 8 ? 1 : 2;  // (ranges of two spans are not cut into eight parts)
   if constexpr (R >= 32) {
     if (l.a->r != R) {  // buffers of a rank between the instances': the masked code with the buffers' rank as stride
-      if (l.widest <= kNW * 64) launch_spans<T, R, KSPW, KP, true, true, 1>(l);
-      else launch_spans<T, R, KSPW, KP, true, true, 2>(l);
+      if (one_span) launch_spans<T, R, KSPW, KP, true, true, 1>(l);
+      else launch_spans<T, R, KSPW, KP, true, true, kTwo>(l);
       return;
     }
   }
   if (l.a->effective_rank) {
-    if (l.widest <= kNW * 64) launch_spans<T, R, KSPW, KP, true, false, 1>(l);
-    else launch_spans<T, R, KSPW, KP, true, false, 2>(l);
+    if (one_span) launch_spans<T, R, KSPW, KP, true, false, 1>(l);
+    else launch_spans<T, R, KSPW, KP, true, false, kTwo>(l);
   } else {
-    if (l.widest <= kNW * 64) launch_spans<T, R, KSPW, KP, false, false, 1>(l);
-    else launch_spans<T, R, KSPW, KP, false, false, 2>(l);
+    if (one_span) launch_spans<T, R, KSPW, KP, false, false, 1>(l);
+    else launch_spans<T, R, KSPW, KP, false, false, kTwo>(l);
   }
 }
 
@@ -750,6 +752,13 @@ bool launch_rank(const Launch& l, int rank, int kspw, int kp) {
       case 16: launch_one<T, 16, 4, 4>(l); return true;
       case 32: launch_one<T, 32, 4, 4>(l); return true;
       case 64: launch_one<T, 64, 4, 4>(l); return true;
+    }
+  } else if (kspw == 4 && kp == 8) {
+    switch (r) {
+      case 8: launch_one<T, 8, 4, 8>(l); return true;
+      case 16: launch_one<T, 16, 4, 8>(l); return true;
+      case 32: launch_one<T, 32, 4, 8>(l); return true;
+      case 64: launch_one<T, 64, 4, 8>(l); return true;
     }
   } else if (kspw == 16 && kp == 1) {
     switch (r) {
@@ -798,18 +807,22 @@ SlotKnobs& slot_knobs() {
   return k;
 }
 
-// K parts of a launch: four for K = 4096 when the tile's workgroups can hand each other partial
-// sums (one slice of at most 4096 columns, a workspace whose exchange area holds every tile's parts),
-// else one.
+// K parts of a launch: of 1024 columns each for K = 4096 and 8192 when the tile's workgroups can hand each
+// other partial sums (one slice of at most 1024 columns per part, a workspace whose exchange area holds every
+// tile's parts), else one.  Eight parts at K = 8192 against the shrink and expand launches (pair.hip): one token,
+// rank 32, 8 slot ids 7.2 -> 5.4 us per call, 16 tokens, rank 16, 16 ids 7.1 -> 5.7.
 int k_parts(const MloraAddArgs* a) {
-  if (a->k != 4096 || a->num_slices != 1 || slot_knobs().kparts != 4) return 1;
-  if (a->slices[0].n > 4 * 1024 || a->slices[0].n < 4 * 64) return 1;
-  if (a->r > 32 && a->slices[0].n > 4 * 512) return 1;  // (two spans per wavefront at rank 64 do not fit the registers beside the parts)
+  if ((a->k != 4096 && a->k != 8192) || a->num_slices != 1 || slot_knobs().kparts == 1) return 1;
+  const int kp = a->k / 1024;
+  if (a->slices[0].n > kp * 1024 || a->slices[0].n < kp * 64) return 1;
+  if ((kp - 1) * (((a->slices[0].n + kp - 1) / kp + 63) & ~63) >= a->slices[0].n) return 1;  // (a part without columns would leave the tile)
+  if (kp == 8 && a->slices[0].n > kp * 512) return 1;   // (instances of one span per wavefront only)
+  if (a->r > 32 && a->slices[0].n > kp * 512) return 1;  // (two spans per wavefront at rank 64 do not fit the registers beside the parts)
   if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return 1;
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
-  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * 4 * ((compute_rank(a->r) + 15) / 16) * 256;
+  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * kp * ((compute_rank(a->r) + 15) / 16) * 256;
   if (words * 8 > kWsXchgBytes) return 1;
-  return 4;
+  return kp;
 }
 
 }  // namespace
@@ -840,6 +853,7 @@ bool slot_supported(const MloraAddArgs* a) {
   }
   if (kspw == 4) return true;
   if (kspw == 16) return a->r <= 16 || k_parts(a) == 4;
+  if (kspw == 32) return k_parts(a) == 8;
   return false;
 }
 
