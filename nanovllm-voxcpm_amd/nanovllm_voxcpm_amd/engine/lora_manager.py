@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora import attach_plan
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import attach_plan
 from nanovllm_voxcpm_amd.utils.context import LoRAContext
 
 

@@ -23,7 +23,7 @@ from typing import Protocol
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, build_segment_plan
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, attached_plan, build_segment_plan
 
 
 @dataclass(frozen=True)
@@ -107,15 +107,6 @@ def _vector_shape(dtype: torch.dtype, rank: int, k: int) -> bool:
 
 
 _PLAN_ATTR = "_mlora_segment_plans"
-_SLOTS_PLAN_ATTR = "_mlora_plan"  # on a slot vector: the plan that was built together with it
-
-
-def attach_plan(slots: torch.Tensor, workspace: torch.Tensor, max_slots: int) -> None:
-    """Leave a segment plan with the slot vector it was built from (eagerly, on the current stream); it
-    serves eager calls until the vector is rewritten.  Inference tensors, whose rewrites nobody
-    counts, get none."""
-    if not slots.is_inference() and not _hip.stream_capture_id(slots.device):
-        setattr(slots, _SLOTS_PLAN_ATTR, (workspace, max_slots, slots._version))
 _CONTEXT_PLANS_ATTR = "_mlora_context_plans"  # plan table of the LoRAContext a metadata object was made from
 
 
@@ -197,7 +188,7 @@ class HipLoRABackend:
         """One metadata launch per batch: every LoRA layer of a step shares the metadata
         object, so the plan is kept on it.
 
-        Two holders, neither of which can go stale silently:
+        Two holders:
 
         * a metadata object made from a ``LoRAContext`` carries the context's own plan table
           (``_mlora_context_plans``).  The plan is then a derived array of the context, like the
@@ -206,8 +197,13 @@ class HipLoRABackend:
           one, and whoever refreshes the context's buffers in a way the version does not see
           (``graph_meta.copy_lora_domain_to_graph_vars``, inference tensors) drops it;
         * any other metadata object gets a table keyed by the slot vector's address, length and
-          in-place version.  Inference tensors have no version counter, so an in-place rewrite
-          could not be noticed: for them nothing is kept and every call builds its plan.
+          in-place version (a rewrite that the counter does not see takes a new metadata object).
+          Inference tensors have no version counter, so an in-place rewrite could not be
+          noticed: for them nothing is kept and every call builds its plan.
+
+        A slot vector that a batch context was built with carries the plan of the same launch
+        (``segment_meta.attach_plan``) until its version changes or its context is installed or
+        invalidated; a table that has no plan yet starts with that one.
 
         Either way a plan is reused only inside the stream capture it was built in: a plan built
         eagerly during warm-up must not satisfy a later graph capture, or the captured graph
@@ -242,11 +238,8 @@ class HipLoRABackend:
         if plan is None:
             if len(cache) >= 4:
                 cache.clear()
-            made = getattr(own, _SLOTS_PLAN_ATTR, None)
-            if made is not None and not capture and made[1:] == (max_slots, version) and own.numel() == tts.numel():
-                plan = SegmentPlan(workspace=made[0], token_to_slot=tts, num_tokens=tts.numel(), max_slots=max_slots)
-            else:
-                plan = build_segment_plan(tts, max_slots)
+            made = attached_plan(own, max_slots) if not capture and own.numel() == tts.numel() else None
+            plan = build_segment_plan(tts, max_slots) if made is None else SegmentPlan(made, tts, tts.numel(), max_slots)
             cache[key] = plan
         return plan
 

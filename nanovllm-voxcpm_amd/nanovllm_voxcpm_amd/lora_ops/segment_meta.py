@@ -56,6 +56,29 @@ def build_segment_plan(token_to_slot: torch.Tensor, max_slots: int) -> SegmentPl
     return SegmentPlan(workspace=workspace, token_to_slot=tts, num_tokens=tts.numel(), max_slots=max_slots)
 
 
+_ATTACHED_PLAN = "_mlora_plan"  # on a slot vector: the plan that was built together with it
+
+
+def attach_plan(slots: torch.Tensor, workspace: torch.Tensor, max_slots: int) -> None:
+    """Leave a segment plan with the slot vector it was built from (eagerly, on the current stream); it
+    serves eager calls until the vector is rewritten: ``attached_plan`` sees what the vector's version
+    counter counts, any other rewrite is announced by invalidating the context that holds the
+    vector, which drops the plan.  Inference tensors, whose rewrites nobody counts, get none."""
+    if not slots.is_inference() and not _hip.stream_capture_id(slots.device):
+        setattr(slots, _ATTACHED_PLAN, (workspace, max_slots, slots._version))
+
+
+def attached_plan(slots: torch.Tensor, max_slots: int) -> torch.Tensor | None:
+    """Workspace of the plan left with this very vector, None when there is none or it no longer fits."""
+    made = getattr(slots, _ATTACHED_PLAN, None)
+    return made[0] if made is not None and made[1] == max_slots and made[2] == slots._version else None
+
+
+def drop_attached_plan(slots: torch.Tensor) -> None:
+    if getattr(slots, _ATTACHED_PLAN, None) is not None:
+        delattr(slots, _ATTACHED_PLAN)
+
+
 @dataclass
 class LoRAKernelMeta:
     """Preallocated index buffers in the layout of the reference's grouped kernels.

@@ -13,7 +13,7 @@ from dataclasses import dataclass, field
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector, drop_attached_plan
 
 LM_LORA_DOMAIN = "lm_domain"
 PROJ_LORA_DOMAIN = "proj_domain"
@@ -61,6 +61,8 @@ def invalidate_lora_context(lora_context: LoRAContext) -> None:
     """Forget everything derived from the context's tensors (call after rewriting them in place)."""
     lora_context._cached_metadata = None
     lora_context._segment_plans.clear()
+    if lora_context.token_to_slot is not None:
+        drop_attached_plan(lora_context.token_to_slot)
 
 
 def reset_lora_context(domain: str | None = None) -> None:
