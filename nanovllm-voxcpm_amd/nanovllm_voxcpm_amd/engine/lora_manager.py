@@ -56,25 +56,29 @@ class LoRABatchPlan:
 
     @property
     def token_to_slot(self) -> list[int]:
-        if self._tokens is None:
-            self._tokens = expand_token_to_slot(*self._runs)
+        if self._tokens is None:  # from here on the list, which the caller may edit, is what counts
+            self._tokens, self._runs = expand_token_to_slot(*self._runs), None
         return self._tokens
 
     @token_to_slot.setter
     def token_to_slot(self, tokens: list[int]) -> None:
         self._tokens, self._runs = tokens, None
 
+    def _listed(self) -> list[int]:
+        """The per-token slot ids for reading: not handed out, so the runs stay in force."""
+        return self._tokens if self._tokens is not None else expand_token_to_slot(*self._runs)
+
     def runs(self) -> tuple[list[int], list[int]]:
         """(slot ids, token counts) whose expansion is ``token_to_slot``."""
         return self._runs if self._runs is not None else (self._tokens, [1] * len(self._tokens))
 
     def __repr__(self) -> str:
-        return f"LoRABatchPlan(adapter_to_slot={self.adapter_to_slot!r}, token_to_slot={self.token_to_slot!r})"
+        return f"LoRABatchPlan(adapter_to_slot={self.adapter_to_slot!r}, token_to_slot={self._listed()!r})"
 
     def __eq__(self, other) -> bool:
         if not isinstance(other, LoRABatchPlan):
             return NotImplemented
-        return self.adapter_to_slot == other.adapter_to_slot and list(self.token_to_slot) == list(other.token_to_slot)
+        return self.adapter_to_slot == other.adapter_to_slot and list(self._listed()) == list(other._listed())
 
     @property
     def num_lora_tokens(self) -> int:
@@ -85,15 +89,19 @@ class LoRABatchPlan:
     @property
     def active_slot_ids(self) -> list[int]:
         if self._active is None:
-            slots, counts = self.runs()
-            used = set(slots) if 0 not in counts else {s for s, c in zip(slots, counts) if c > 0}
-            self._active = sorted([s for s in used if s >= 0])
+            self._active = self._used_slots()
         return self._active
+
+    def _used_slots(self) -> list[int]:
+        slots, counts = self.runs()
+        used = set(slots) if 0 not in counts else {s for s, c in zip(slots, counts) if c > 0}
+        return sorted([s for s in used if s >= 0])
 
     @property
     def num_tokens_per_slot(self) -> list[int]:
         if self._counts is None:
-            self._counts = [sum(1 for s in self.token_to_slot if s == slot) for slot in self.active_slot_ids]
+            tokens = self._listed()
+            self._counts = [sum(1 for s in tokens if s == slot) for slot in self.active_slot_ids]
         return self._counts
 
     @property
@@ -108,7 +116,7 @@ class LoRABatchPlan:
     @property
     def token_indices_sorted_by_slot(self) -> list[int]:
         if self._sorted is None:
-            keyed = [(s, t) for t, s in enumerate(self.token_to_slot) if s >= 0]
+            keyed = [(s, t) for t, s in enumerate(self._listed()) if s >= 0]
             self._sorted = [t for _, t in sorted(keyed)]
         return self._sorted
 
@@ -186,7 +194,7 @@ def build_lora_context_from_batch_plan(
         return context
     n = sum(counts)
     tts = _upload_runs(slots, counts, n, device) if n else torch.empty(0, dtype=torch.int32, device=device)
-    active = plan.active_slot_ids
+    active = plan._used_slots()
     if not active:
         return LoRAContext(token_to_slot=tts, no_lora_flag=True, num_active_loras=0)
     n_lora, n_active = plan.num_lora_tokens, len(active)

@@ -51,6 +51,49 @@ def test_batch_plan_loads_slot_and_expands_tokens():
     assert plan.adapter_to_slot == {a: 0}
 
 
+def _from_runtime(slots, counts):
+    from nanovllm_voxcpm_amd.engine.lora_manager import LoRARuntime
+
+    rt = LoRARuntime(max_loras=4)
+    for i in range(4):
+        rt.register_lora(f"adapter {i}", _payload())
+        rt.on_sequence_enqueued(i)
+    rt.build_batch_plan([0, 1, 2, 3], [1, 1, 1, 1], lambda *_: None)  # adapter i in slot i
+    return rt.build_batch_plan([None if s < 0 else s for s in slots], counts, lambda *_: None)
+
+
+def _from_constructor(slots, counts):
+    from nanovllm_voxcpm_amd.engine.lora_manager import LoRABatchPlan, expand_token_to_slot
+
+    return LoRABatchPlan({s: s for s in slots if s >= 0}, expand_token_to_slot(slots, counts))
+
+
+@pytest.mark.parametrize("make", [_from_runtime, _from_constructor])
+def test_edits_of_a_plans_token_list_count(make):
+    """However the plan was made, what the device path reads (runs, counts, active slots) follows the list."""
+    from nanovllm_voxcpm_amd.engine.lora_manager import expand_token_to_slot
+
+    untouched = make([2, -1, 3], [3, 1, 2])
+    assert repr(untouched).endswith("token_to_slot=[2, 2, 2, -1, 3, 3])") and untouched.token_indices_sorted_by_slot == [0, 1, 2, 4, 5]
+    assert untouched == make([2, -1, 3], [3, 1, 2]) and (untouched.num_lora_tokens, untouched.active_slot_ids) == (5, [2, 3])
+
+    plan = make([2, -1, 3], [3, 1, 2])
+    plan.token_to_slot[0] = -1
+    plan.token_to_slot.append(0)
+    want = [-1, 2, 2, -1, 3, 3, 0]
+    assert plan.token_to_slot == want and expand_token_to_slot(*plan.runs()) == want
+    assert plan.num_lora_tokens == 5 and plan.active_slot_ids == [0, 2, 3]
+    assert plan.num_tokens_per_slot == [1, 2, 2] and plan.token_indices_sorted_by_slot == [6, 1, 2, 4, 5]
+
+    plan = make([2, -1, 3], [3, 1, 2])
+    assert plan.active_slot_ids == [2, 3]
+    plan.token_to_slot[4:] = [1, 1]
+    assert plan._used_slots() == [1, 2]  # what the context is built with; the list handed out before stands as it was
+
+    plan.token_to_slot = [1]
+    assert plan.num_lora_tokens == 1 and expand_token_to_slot(*plan.runs()) == [1]
+
+
 def test_capacity_and_lru_eviction():
     from nanovllm_voxcpm_amd.engine.lora_manager import LoRARuntime
 
