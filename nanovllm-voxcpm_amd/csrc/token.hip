@@ -342,7 +342,7 @@ __global__ __launch_bounds__(256) void install_kernel(InstallTable table) {
           for (int q = 0; q < 8; ++q) f[q] = j + q < rank ? to_f32(src[q]) : 0.f;
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) f[q] = scaled(f[q]);
+        for (int q = 0; q < 8; ++q) f[q] = j + q < rank ? scaled(f[q]) : 0.f;  // (zero also under a negative or non-finite scaling)
         store8<D>(B + static_cast<int64_t>(e) * 8, f);
       }
     }
