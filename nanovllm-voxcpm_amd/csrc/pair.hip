@@ -20,6 +20,7 @@
 #include "common.h"
 #include "launch.h"
 #include "dma.h"
+#include "lds.h"
 #include "sgmv_body.h"
 
 namespace mlora {
@@ -442,17 +443,11 @@ struct PairLaunch {
   int parts_log2, sp;
 };
 
-template <typename F> bool allow_lds(F* kernel) {
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  return true;
-}
-
 template <typename T> void launch_pair_shrink(const PairLaunch& l) {
   const MloraAddArgs* a = l.a;
   ShrinkSlices sl;
   for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = i < a->num_slices ? a->slices[i].a : nullptr;
-  static const bool once = allow_lds(pair_shrink_kernel<T>);
-  (void)once;
+  allow_lds<pair_shrink_kernel<T>>(shrink_lds(a->r));
   hipLaunchKernelGGL((pair_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
                      dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
                      a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
@@ -461,8 +456,7 @@ template <typename T> void launch_pair_shrink(const PairLaunch& l) {
 
 template <typename T, int C, int SP> void launch_pair_expand_one(const PairLaunch& l, const ExpandSplits& splits, int total) {
   const MloraAddArgs* a = l.a;
-  static const bool once = allow_lds(pair_expand_kernel<T, C, SP>);
-  (void)once;
+  allow_lds<pair_expand_kernel<T, C, SP>>(expand_lds(C, SP));
   hipLaunchKernelGGL((pair_expand_kernel<T, C, SP>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
                      expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
                      a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, splits);

@@ -16,6 +16,7 @@
 #include "common.h"
 #include "dma.h"
 #include "launch.h"
+#include "lds.h"
 #include "sgmv_body.h"
 
 namespace mlora {
@@ -191,11 +192,7 @@ int slab_lds(int r) {
 }
 
 template <typename T> void launch_slab_type(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const ShrinkSlices& sl) {
-  static const bool once = [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(slab_shrink_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    return true;
-  }();
-  (void)once;
+  allow_lds<slab_shrink_kernel<T>>(slab_lds(a->r));
   hipLaunchKernelGGL((slab_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices * parts), static_cast<unsigned>(tiles8)), dim3(kSlabThreads),
                      slab_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), lay.big_off, lay.small_off, big_cap,
                      lay.bigrows_off, a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kPiece),

@@ -91,6 +91,47 @@ def test_ctypes_structs_match_the_c_layout(tmp_path):
     assert re.search(r"#define MLORA_STATIC_SCRATCH_BYTES \(16u << 20\)", text) and _hip.STATIC_SCRATCH_BYTES == 16 << 20
 
 
+def test_large_lds_is_allowed_for_every_device_a_kernel_runs_on(tmp_path):
+    """csrc/lds.h against a runtime that only keeps count: per kernel and device, not per process, again
+    after a failure, and only where more than 64 KB are asked for."""
+    src = tmp_path / "probe.cpp"
+    src.write_text("""
+#include "lds.h"
+#include <stdio.h>
+static int device = 0, calls = 0;
+static hipError_t answer = hipSuccess;
+extern "C" hipError_t hipGetDevice(int* d) { *d = device; return hipSuccess; }
+extern "C" hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { ++calls; return answer; }
+static void one() {}
+template <int> static void many() {}
+int main() {
+  mlora::allow_lds<one>(64 * 1024);
+  printf("%d ", calls);
+  for (int round = 0; round < 2; ++round)
+    for (device = 0; device < 3; ++device) mlora::allow_lds<one>(96 * 1024);
+  printf("%d ", calls);
+  device = 1;
+  mlora::allow_lds<many<1>>(96 * 1024);
+  mlora::allow_lds<many<2>>(96 * 1024);
+  mlora::allow_lds<many<2>>(96 * 1024);
+  printf("%d ", calls);
+  answer = hipErrorInvalidValue;
+  device = 5;
+  mlora::allow_lds<one>(96 * 1024);
+  answer = hipSuccess;
+  mlora::allow_lds<one>(96 * 1024);
+  mlora::allow_lds<one>(96 * 1024);
+  printf("%d", calls);
+}
+""")
+    exe = tmp_path / "probe"
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT / 'nanovllm-voxcpm_amd' / 'csrc'}",
+                    str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout == "0 3 5 7"
+    for name in ("pair.hip", "slab.hip"):  # nothing sets the attribute by another way
+        assert "hipFuncSetAttribute" not in (ROOT / "nanovllm-voxcpm_amd" / "csrc" / name).read_text()
+
+
 def test_arguments_are_rejected_before_any_launch():
     from nanovllm_voxcpm_amd import _hip
 
