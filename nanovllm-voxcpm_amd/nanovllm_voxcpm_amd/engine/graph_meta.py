@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector, mark_capacity
 from nanovllm_voxcpm_amd.utils.context import LORA_DOMAINS, LoRAContext, get_lora_context, invalidate_lora_context, set_lora_context
 
 
@@ -93,7 +93,7 @@ def set_graph_lora_contexts(graph_vars: dict, contexts: dict[str, LoRAContext]) 
             LoRAContext(
                 token_to_slot=domain_vars["token_to_slot"][:rows],
                 token_indices_sorted_by_slot=domain_vars["token_indices_sorted_by_slot"][:rows],
-                active_slot_ids=domain_vars["active_slot_ids"],
+                active_slot_ids=mark_capacity(domain_vars["active_slot_ids"]),
                 num_tokens_per_slot=domain_vars["num_tokens_per_slot"],
                 slot_start_offsets=domain_vars["slot_start_offsets"],
                 no_lora_flag=context.no_lora_flag,

@@ -23,7 +23,7 @@ from typing import Protocol
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, attached_plan, build_segment_plan
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, attached_plan, build_segment_plan, known_active_slots
 
 
 @dataclass(frozen=True)
@@ -404,7 +404,7 @@ class HipLoRABackend:
         if dev.index is not None and dev.index != _hip.current_device_index():
             return False  # another GPU of this process: the general path makes it current
         stream = _hip.current_stream_handle(dev)
-        plan_ptr = ws_ptr = ws_bytes = 0
+        plan_ptr = ws_ptr = ws_bytes = capture = 0
         if site.weights_vectorisable and args.form != _hip.FORM_TOKEN and not (xs % 8 or ys % 8 or x_ptr % 16 or y_ptr % 16):
             capture = _hip.current_stream_capture_id(dev, stream)
             # every LoRA linear of a step calls with the same metadata object, slot vector, stream
@@ -429,7 +429,7 @@ class HipLoRABackend:
                         self._fastcall.forget_step(fast)
                     else:  # (the tuple above keeps metadata, slot vector and plan alive for as long as this stands)
                         self._fastcall.set_step(fast, metadata, source, version, stream or 0, site.num_slots, rows, plan_ptr,
-                                                getattr(metadata, "num_active_loras", 0))
+                                                known_active_slots(metadata, site.num_slots, capture))
             scratch = self._scratch_for(x, site.num_slices, site.rank, stream, capture)
             ws_ptr, ws_bytes = scratch.data_ptr(), scratch.numel()
             if not capture:
@@ -441,7 +441,7 @@ class HipLoRABackend:
         _STEP_HEAD.pack_into(site.view, 0, stream or 0, x_ptr, y_ptr, xs, ys, source.data_ptr(), plan_ptr, rows)
         _STEP_SCALE.pack_into(site.view, _OFF_SCALING, scaling)
         _STEP_TAIL.pack_into(site.view, _OFF_WORKSPACE, ws_ptr, ws_bytes, eff_ptr)
-        _hip.call_add_lora(args, getattr(metadata, "num_active_loras", 0))
+        _hip.call_add_lora(args, known_active_slots(metadata, site.num_slots, capture))
         return True
 
     # -- the fused apply -------------------------------------------------------------------
@@ -556,7 +556,7 @@ class HipLoRABackend:
                     plan = self._plan_for(metadata, tts, a_list[0].size(0), capture).workspace
                     scratch = self._scratch_for(x2, len(chunk), a_list[0].size(-2), stream, capture)
                 _hip.add_lora(target, x2, a_list, b_list, c_list, tts, plan, float(scaling), form, scratch, stream,
-                              effective_rank=effective_rank, active_slots=getattr(metadata, "num_active_loras", 0))
+                              effective_rank=effective_rank, active_slots=known_active_slots(metadata, a_list[0].size(0), capture))
         if staged is not None:
             staged.copy_(target)
         return outputs

@@ -79,6 +79,25 @@ def drop_attached_plan(slots: torch.Tensor) -> None:
         delattr(slots, _ATTACHED_PLAN)
 
 
+_CAPACITY = "_mlora_capacity"  # on the slot ids of a context whose lengths are capacities
+
+
+def mark_capacity(active_slot_ids: torch.Tensor) -> torch.Tensor:
+    """Note on a context's slot ids that their number, and the context's ``num_active_loras``, is what the buffers
+    hold and not how many slots the batch uses."""
+    setattr(active_slot_ids, _CAPACITY, True)
+    return active_slot_ids
+
+
+def known_active_slots(metadata, num_slots: int, capture: int | None) -> int:
+    """How many slots have tokens, 0 where nobody knows: behind capacities, and in a captured call, which
+    will be replayed for other batches than the one it was captured with."""
+    if capture or getattr(getattr(metadata, "active_slot_ids", None), _CAPACITY, False):
+        return 0
+    active = getattr(metadata, "num_active_loras", 0)
+    return active if 0 < active <= num_slots else 0
+
+
 @dataclass
 class LoRAKernelMeta:
     """Preallocated index buffers in the layout of the reference's grouped kernels.

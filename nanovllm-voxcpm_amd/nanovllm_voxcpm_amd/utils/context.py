@@ -13,7 +13,7 @@ from dataclasses import dataclass, field
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector, drop_attached_plan
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import as_slot_vector, drop_attached_plan, mark_capacity
 
 LM_LORA_DOMAIN = "lm_domain"
 PROJ_LORA_DOMAIN = "proj_domain"
@@ -121,7 +121,7 @@ def build_lora_context_from_token_to_slot(
         return LoRAContext(
             token_to_slot=tts,
             token_indices_sorted_by_slot=sorted_idx,
-            active_slot_ids=ids,
+            active_slot_ids=mark_capacity(ids),
             num_tokens_per_slot=counts,
             slot_start_offsets=offsets,
             no_lora_flag=False,
