@@ -303,13 +303,19 @@ def load_error() -> str | None:
 
 
 _FASTCALL: object = ()  # () until the import was tried
+_KEEP_TO_PYTHON: bool | None = None  # what MLORA_NO_FASTCALL said when it was last read
 
 
 def load_fastcall():
     """The module with the C++ host paths (csrc/fastcall.cpp, built beside the library by ``make
-    fastcall``), or None where it is not built or does not load: the Python paths then do every
-    call.  It launches nothing itself: it calls the library's entry points."""
-    global _FASTCALL
+    fastcall``), or None where it is not built or does not load, or MLORA_NO_FASTCALL=1 keeps it out
+    (read once, and again after ``reload_knobs``): the Python paths then do every call.  Every host
+    path asks here on each call.  The module launches nothing itself: it calls the library's entry points."""
+    global _FASTCALL, _KEEP_TO_PYTHON
+    if _KEEP_TO_PYTHON is None:
+        _KEEP_TO_PYTHON = os.environ.get("MLORA_NO_FASTCALL", "0") not in ("", "0")
+    if _KEEP_TO_PYTHON:
+        return None
     if _FASTCALL == ():
         try:
             from nanovllm_voxcpm_amd import _mlora_fastcall
@@ -709,7 +715,10 @@ def stream_capture_id(device: torch.device, stream: int | None = None) -> int:
 
 
 def reload_knobs() -> None:
-    """Make the library read its MLORA_* environment variables again (it keeps them otherwise)."""
+    """Make the library, and the choice of host path, read their MLORA_* environment variables again (they
+    keep them otherwise)."""
+    global _KEEP_TO_PYTHON
+    _KEEP_TO_PYTHON = None
     load().mlora_reload_knobs()
 
 

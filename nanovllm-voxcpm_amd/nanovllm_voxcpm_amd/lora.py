@@ -145,7 +145,8 @@ class HipLoRABackend:
         self._spares: dict = {}          # device -> initialised buffer kept for the next graph capture
         self._graph_scratch: dict = {}   # device -> buffers captured graphs refer to (the last one is in use)
         self._sites = threading.local()  # per thread: weight buffers -> _CallSite
-        # the C++ host path of the usual call (optional: built beside the library; MLORA_NO_FASTCALL=1 keeps to Python)
+        # the C++ host path of the usual call (optional: built beside the library; MLORA_NO_FASTCALL=1, as it
+        # stands now, keeps this backend to Python)
         self._fastcall = None if os.environ.get("MLORA_NO_FASTCALL", "0") not in ("", "0") else _hip.load_fastcall()
 
     def _fast_state(self):

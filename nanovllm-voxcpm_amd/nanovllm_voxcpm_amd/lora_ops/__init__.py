@@ -34,9 +34,6 @@ def _as_3d(weight: torch.Tensor, what: str) -> torch.Tensor:
     return weight
 
 
-_FAST = _hip.load_fastcall()
-
-
 def lora_shrink(
     inputs: torch.Tensor,
     lora_a_weights: list[torch.Tensor],
@@ -58,8 +55,9 @@ def lora_shrink(
     """
     if no_lora_flag:
         return
-    if _FAST is not None:  # the usual call, checked and enqueued in C++
-        rc = _FAST.shrink(_hip.entry_point("mlora_shrink"), inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling)
+    fast = _hip.load_fastcall()
+    if fast is not None:  # the usual call, checked and enqueued in C++
+        rc = fast.shrink(_hip.entry_point("mlora_shrink"), inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling)
         if rc <= 0:
             return _hip._check(rc, "mlora_shrink")
     _shrink(inputs, lora_a_weights, output_tensor, token_lora_mapping, scaling)
@@ -100,8 +98,9 @@ def lora_expand(
     """
     if no_lora_flag:
         return
-    if _FAST is not None:
-        rc = _FAST.expand(_hip.entry_point("mlora_expand"), inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs)
+    fast = _hip.load_fastcall()
+    if fast is not None:
+        rc = fast.expand(_hip.entry_point("mlora_expand"), inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs)
         if rc <= 0:
             return _hip._check(rc, "mlora_expand")
     _expand(inputs, lora_b_weights, output_tensor, token_lora_mapping, offset_start, add_inputs)
