@@ -18,12 +18,14 @@ __device__ __forceinline__ const char* uniform(const char* p) {
   return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// One 1 KB direct load: lane i's 16 bytes at base + voff go to LDS byte lds + 16 i.
+// One 1 KB direct load: lane i's 16 bytes at base + voff go to LDS byte lds + 16 i.  The load takes the LDS address from
+// m0, which the compiler itself puts there for the asm (an asm that wrote it could not say so: m0 is a reserved
+// register and has no place among the clobbers); between that write and the load lies one wait state.
 __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds) {
 #ifdef MLORA_TRACE
   base = uniform(static_cast<const char*>(base));  // (the branches around the stamps cost the compiler its proof of that)
 #endif
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(base) : "memory");
 }
 
 }  // namespace
