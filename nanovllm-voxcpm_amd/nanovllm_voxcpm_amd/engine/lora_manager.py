@@ -138,12 +138,12 @@ def expand_token_to_slot(adapter_slots: list[int], token_counts: list[int]) -> l
     return out
 
 
-def _upload_runs(slots: list[int], counts: list[int], n: int, device: torch.device | str) -> torch.Tensor:
-    """The per-token slot ids on the device: expanded into a pinned buffer, one asynchronous copy."""
+def _pinned_slots(slots: list[int], counts: list[int], n: int) -> torch.Tensor:
+    """The per-token slot ids expanded into a pinned buffer."""
     host = torch.empty(n, dtype=torch.int32, device="cpu", pin_memory=True)
     ids = np.frombuffer(array("i", slots), dtype=np.int32)
     host.numpy()[:] = ids if counts.count(1) == len(counts) else np.repeat(ids, np.frombuffer(array("q", counts), dtype=np.int64))
-    return host.to(device, non_blocking=True)
+    return host
 
 
 def _context_in_one_launch(slots: list[int], counts: list[int], max_slots: int | None, device: torch.device | str) -> LoRAContext | None:
@@ -193,9 +193,9 @@ def build_lora_context_from_batch_plan(
     if context is not None:
         return context
     n = sum(counts)
-    tts = _upload_runs(slots, counts, n, device) if n else torch.empty(0, dtype=torch.int32, device=device)
     active = plan._used_slots()
     if not active:
+        tts = _pinned_slots(slots, counts, n).to(device, non_blocking=True) if n else torch.empty(0, dtype=torch.int32, device=device)
         return LoRAContext(token_to_slot=tts, no_lora_flag=True, num_active_loras=0)
     n_lora, n_active = plan.num_lora_tokens, len(active)
     if max_slots is None:
@@ -203,11 +203,11 @@ def build_lora_context_from_batch_plan(
     elif active[-1] >= max_slots:
         raise ValueError(f"slot id {active[-1]} is outside the {max_slots} resident slots")
     cap = min(n, max_slots)
-    i32 = dict(dtype=torch.int32, device=tts.device)
-    # one allocation, four views and the segment plan (its start on a 256-byte boundary)
-    head = (n + 2 * cap + cap + 1 + 63) & ~63
-    packed = torch.empty(head + _hip.plan_workspace_words(n, max_slots), **i32)
-    sorted_idx, ids, per_slot, offsets = packed[: n + 2 * cap + cap + 1].split([n, cap, cap, cap + 1])
+    # one allocation: slot vector, index arrays, segment plan (its start on a 256-byte boundary)
+    head = (2 * n + 2 * cap + cap + 1 + 63) & ~63
+    packed = torch.empty(head + _hip.plan_workspace_words(n, max_slots), dtype=torch.int32, device=device)
+    tts, sorted_idx, ids, per_slot, offsets = packed[: 2 * n + 2 * cap + cap + 1].split([n, n, cap, cap, cap + 1])
+    tts.copy_(_pinned_slots(slots, counts, n), non_blocking=True)
     workspace = packed[head:]
     _hip.meta_build_many([
         dict(token_to_slot=tts, max_slots=max_slots, sorted_idx=sorted_idx, compact_ids=ids, compact_counts=per_slot,

@@ -23,6 +23,15 @@ LORA_DOMAINS = (LM_LORA_DOMAIN, PROJ_LORA_DOMAIN, DIT_LORA_DOMAIN)
 
 @dataclass
 class LoRAContext:
+    """What the LoRA linears of a domain know of the batch.
+
+    Streams: the arrays of a context from ``build_lora_context_from_batch_plan`` and the segment plan made
+    with them are one allocation of the stream that was current there.  Work on another stream waits for
+    that stream before its first use, and ``token_to_slot.record_stream(other)`` (any of the arrays
+    does: they share the block) holds the memory for it until everything the context was used for
+    there has run; the plan is read by every call of the step, so that is the whole of the step.
+    """
+
     token_to_slot: torch.Tensor | None = None
     token_indices_sorted_by_slot: torch.Tensor | None = None
     active_slot_ids: torch.Tensor | None = None

@@ -46,3 +46,18 @@ def test_context_of_runs_bit_exact(name):
     head = 16 + (len(tokens) + 3 & ~3)
     assert workspace[:16].tolist() == want[:16].tolist() and workspace[16 : 16 + len(sorted_idx)].tolist() == list(sorted_idx)
     assert workspace[head : head + max_slots + 1].tolist() == want[head : head + max_slots + 1].tolist()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["singles", "singles_over", "runs", "runs_over"])
+def test_a_context_and_its_plan_are_one_allocation(name):
+    """What is recorded for the slot vector on another stream holds for everything the kernels read there."""
+    from nanovllm_voxcpm_amd.engine.lora_manager import LoRABatchPlan, build_lora_context_from_batch_plan
+
+    max_slots, runs = CASES[name]
+    torch.zeros(1, device="cuda")
+    context = build_lora_context_from_batch_plan(LoRABatchPlan.from_runs({}, [s for s, _ in runs], [c for _, c in runs]), max_slots=max_slots,
+                                                 device="cuda:0")
+    arrays = [context.token_to_slot, context.token_indices_sorted_by_slot, context.active_slot_ids, context.num_tokens_per_slot,
+              context.slot_start_offsets, context.token_to_slot._mlora_plan[0]]
+    assert len({t.untyped_storage().data_ptr() for t in arrays}) == 1
