@@ -145,6 +145,13 @@ static bool small_batch(const MloraAddArgs* a, bool one_launch) {
   return a->num_tokens * width <= limit;
 }
 
+// About how many 16-token tiles a batch has: its segments end anywhere inside their last tile.
+static int small_tiles_about(const MloraAddArgs* a, int active) {
+  const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+  const int tiles = static_cast<int>((a->num_tokens + 7ll * segs) / MLORA_TILE_SMALL);
+  return tiles > segs ? tiles : segs;
+}
+
 // Where the slot-major grid pays.  Its workgroups request the weights of EVERY slot id, with or
 // without tokens, so what it costs grows with the slot ids nobody uses: measured on decode batches of
 // 4..256 tokens over 32 slot ids (us per call, slot-major / tile-major): gate_up, whose slots weigh
@@ -169,11 +176,21 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   if (a->num_slots > knobs().slot_max_slots) return false;
   if (a->num_tokens > 32 * a->num_slots) return false;
   const bool sparse = active > 0 && 2 * active <= a->num_slots;
-  // Eight parts (K = 8192) are twice the workgroups of a tile, and past one per compute unit they wait for
-  // each other in two rounds (slot-major / the pair: rank 32: 5.4 / 7.2 at 8 slot ids, 11.5 / 10.9 at 32; rank 16: 5.7 /
-  // 7.1 at 16, 9.3 / 9.7 at 32, 9.9 / 8.5 at 40; rank 64: 9.0 / 9.6 at 8, 18.4 / 16.4 at 32).
-  if (slot_k_parts(a) > 4) return a->num_slots <= 32 && a->num_slots * compute_rank(a->r) <= 640;
-  if (slot_k_parts(a) > 1) return a->num_slots <= (a->r <= 16 ? 32 : 48) && !(sparse && a->r * a->num_slots >= 2048);
+  const int parts = slot_k_parts(a);
+  // Buffers of a rank between 32 and 64 run rank 64's code masked, whose K parts lose to the pair at almost every
+  // size (rank 48, one token per slot id, slot-major / pair: K = 8192 11.5 / 7.8 at 8 slot ids, 19.8 / 11.9 at 32; K = 4096
+  // 7.4 / 7.5 and 9.8 / 9.7, four tokens per slot id 8.7 / 7.9 and 10.5 / 10.2).
+  if (parts > 1 && a->r > 32 && !exact_rank(a->r)) return false;
+  // Eight parts (K = 8192) are twice the workgroups of a tile, slots without tokens have theirs too, and once they no
+  // longer fit the chip together they wait for each other.  K parts x tiles (or slot ids, where more), slot-major /
+  // pair, K = 8192 -> 2048, 2 to 64 slot ids: rank 16 up to 192: 4.6 / 6.1 to 7.2 / 7.6, at 256: 8.2 / 7.5; rank 8 at
+  // 184: 7.0 / 7.4, at 224 and 256: 9.9 / 7.8 and 9.3 / 6.9; rank 32 at 192: 7.5 / 7.8 and 8.7 / 8.5, at 224 and 256: 12.6 /
+  // 11.0 and 11.7 / 9.8; rank 24 like 32; rank 64 at 96 to 136: 8.9 / 9.4 to 10.8 / 11.3, at 128: 10.2 / 9.9, at 160: 11.2 / 10.8.
+  if (parts > 4) {
+    const int tiles = small_tiles_about(a, active);
+    return parts * (tiles > a->num_slots ? tiles : a->num_slots) <= (a->r > 32 ? 144 : 200);
+  }
+  if (parts > 1) return a->num_slots <= (a->r <= 16 ? 32 : 48) && !(sparse && a->r * a->num_slots >= 2048);
   if (sparse || (active > 0 && a->num_tokens > MLORA_TILE_SMALL * active)) return false;
   double cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
@@ -195,14 +212,20 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
 //    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9) and which have no form over 64-token tiles (6000
 //    tokens, rank 48: 40.5 / 32.7, 24.3 / 22.6, 115 / 74, 50 / 35; at 1500 tokens and rank 24 qkv and o are
 //    still the faster ones in one launch: 12.7 / 13.3, 8.1 / 11.2);
-//  - 64-token tiles: tokens x rank up to 1.4e5, beyond which the small tiles fetch A and B too often (rank
-//    64, K = 4096: 18.9 / 13.4 at 1000 tokens, 22.2 / 22.4 at 3001),
-//    where A is as large; wide outputs stay with them (rank 64, K = 2048 -> 16384: 32.2 / 33.2 at 1000).
-static bool pair_pays(const MloraAddArgs* a, int form) {
+//  - 64-token tiles, where A is as large and the outputs are not wide (rank 64, K = 2048 -> 16384: 32.2 / 33.2 at 1000
+//    tokens): while two K parts of every (tile, slice) find a compute unit, tiles x slices <= 128.  The shrink is
+//    one workgroup per compute unit, and a second round of them costs what the first one does.  64-token tiles /
+//    pair, at 1900 and 2200 tokens of 4 slots (123 and 141 tiles): rank 64, K = 4096 16.8 / 13.1, 17.1 / 19.0, K = 2048
+//    14.9 / 12.8, 15.2 / 17.7, K = 8192 23.4 / 20.0, 24.4 / 29.9; rank 32, K = 4096 12.8 / 11.2, 13.2 / 15.2; rank 16, K =
+//    8192 15.7 / 13.8, 16.5 / 17.2.  At 1300 and 1600 tokens of 100 slots (125 and 144 tiles): rank 64, K = 4096 23.4 / 22.3,
+//    23.7 / 28.5; rank 32, K = 4096 16.0 / 15.3, 16.7 / 18.8.  Two slices, rank 32, K = 4096, 900 and 1300 tokens of 4
+//    slots (58 and 83 tiles): 12.6 / 11.6, 13.0 / 15.5; three, rank 64, K = 2048, 500 and 700 (33 and 46): 14.6 / 12.5,
+//    14.7 / 16.7.  (Below the line batches of 16 to 32 slots and more than about 40 tokens in each lose up to a quarter: rank
+//    64, K = 4096, 32 slots: 14.6 / 16.2 at 700 tokens, 19.2 / 20.1 at 1600.)
+static bool pair_pays(const MloraAddArgs* a, int form, int active) {
   const long long rk = static_cast<long long>(a->r) * a->k;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  const bool few = static_cast<long long>(a->num_tokens) * a->r <= 140000;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;
     case MLORA_FORM_MFMA: {
@@ -210,19 +233,27 @@ static bool pair_pays(const MloraAddArgs* a, int form) {
         const double width = static_cast<double>(a->num_slices) * a->k + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
         return a->k != 1024 || a->num_tokens * width > (a->r > 32 ? 1.0e7 : 2.0e7);
       }
-      // three slices and tiles for a second round of workgroups, whose every range repeats its slice's shrink
-      // (K = 1024, 600 / 1200 / 2500 tokens: rank 64 qkv 6.9 / 9.1, 15.5 / 11.1; rank 32 5.0 / 8.2, 10.5 / 9.5, 11.8 / 13.5)
-      if (a->num_slices > 2 && a->r >= 32 && a->num_tokens > 1000 && a->num_tokens < 2000) return true;
       return rk >= 131072;
     }
     case MLORA_FORM_SGMV:
-      // (up to rank 32 the 64-token tiles have the direct loads as well and win from 2200 tokens on: rank 32, 2000 /
-      // 2500 tokens, K = 4096 12.3 / 13.0, 15.8 / 14.9, K = 8192 - , 23.1 / 20.5; rank 16, 3001 tokens, K = 8192 20.5 / 19.0)
-      if (a->r <= 32 && a->num_tokens > 2200) return false;
-      return few && rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k);
-    case MLORA_FORM_WIDE: return few && rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k);
+    case MLORA_FORM_WIDE:
+      return rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active)) * a->num_slices <= 128;
     default: return false;
   }
+}
+
+// Where three slices over 16-token tiles (one workgroup per tile and column range) give way to one launch over 64-token
+// tiles although the batch is small: once the tiles' workgroups, tile t on XCD t % 8, no longer fit the 32 compute
+// units of an XCD, they run in two rounds, each of which shrinks its tile anew.  16-token / 64-token tiles, us per call, q|k|v
+// at workgroups per XCD: K = 1024, rank 64: 11.7 / 13.7 at 32, 16.6 / 13.8 at 36, 17.5 / 12.8 at 44, 17.7 / 13.6 at 48; rank
+// 32: 7.5 / 9.3 at 32, 10.4 / 10.9 at 36, 10.9 / 9.1 at 44; K = 768, rank 64: 10.7 / 12.6 at 32, 17.3 / 12.5 at 36; rank 32: 7.0 /
+// 8.7 and 10.9 / 9.9; K = 512, rank 64: 7.7 / 9.7 and 11.8 / 10.8.  With a smaller A the rounds are too short to matter (K = 512,
+// rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
+// of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
+static bool wide_instead(const MloraAddArgs* a, int active) {
+  if (a->num_slices < 3 || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a)) return false;
+  int columns;
+  return (small_tiles_about(a, active) + 7) / 8 * decode_ranges(a, &columns) > 32;
 }
 
 namespace {
@@ -301,8 +332,11 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
       knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, active))
     form = MLORA_FORM_SLOT;
-  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form))
+  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, active))
     form = MLORA_FORM_PAIR;
+  if (form == MLORA_FORM_MFMA && a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_wide && knobs().small_batch_tokens <= 0 &&
+      wide_instead(a, active))
+    form = MLORA_FORM_WIDE;
   // long-segment batches in one launch, on request
   if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_SGMV && knobs().auto_fused && fused_supported(a))
     form = MLORA_FORM_FUSED;

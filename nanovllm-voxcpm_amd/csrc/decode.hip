@@ -587,8 +587,44 @@ struct DecodeKnobs {
     nt = env_int("MLORA_DECODE_NT", 0);
   }
 };
+const DecodeKnobs& decode_knobs() {
+  static DecodeKnobs k;
+  if (k.generation != knob_generation()) k.read();
+  return k;
+}
 
 }  // namespace
+
+// Columns per range of a launch, and the number of ranges (0: no columns).  Every range repeats the
+// shrink of its tile, but a compute unit takes in only 30-60 bytes per cycle even from the L2, so a
+// launch is fastest when its bytes are spread over 150-250 workgroups: ranges shrink down to 128
+// columns for narrow projections and stay at 1024 (two 64-column spans per wavefront, all loads still
+// in registers) for wide ones.  Measured per launch at 32 tiles: o 6.2 us at 1024 columns, 5.1 at 512,
+// 4.7 at 256; gate_up 8.2 / 8.9 / 11.1.
+int decode_ranges(const MloraAddArgs* a, int* columns) {
+  int nt = decode_knobs().nt;
+  if (nt <= 0) {
+    long long cols = 0;
+    for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+    const int segs = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+    const int by_tokens = (a->num_tokens + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL;
+    const long long tiles = segs > by_tokens ? segs : by_tokens;  // about the number of tiles in use
+    nt = static_cast<int>(cols * tiles / 160);
+    if (nt > 1024) nt = 1024;
+    if (nt < 128) nt = 128;
+  }
+  if (nt < 64) nt = 64;
+  nt = (nt + 63) & ~63;
+  int total;
+  for (;;) {
+    total = 0;
+    for (int i = 0; i < a->num_slices; ++i) total += (a->slices[i].n + nt - 1) / nt;
+    if (total <= kMaxSplits) break;
+    nt *= 2;
+  }
+  *columns = nt;
+  return total;
+}
 
 // Nothing in the kernel limits the size of x or y.
 bool decode_supported(const MloraAddArgs*) { return true; }
@@ -602,8 +638,6 @@ void decode_trace_set(void* buf) {
 }
 
 int launch_decode(const MloraAddArgs* a, bool include_long) {
-  static DecodeKnobs knobs;
-  if (knobs.generation != knob_generation()) knobs.read();
   DecodeSplits splits;
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   int cap = lay.cap_small;
@@ -616,34 +650,10 @@ int launch_decode(const MloraAddArgs* a, bool include_long) {
 
   Launch l;
   l.a = a; l.small_off = lay.small_off; l.include_long = include_long ? 1 : 0; l.splits = &splits;
-  l.staged = knobs.staged;
+  l.staged = decode_knobs().staged;
 
-  // Column range per workgroup.  Every range repeats the shrink of its tile, but a compute unit
-  // takes in only 30-60 bytes per cycle even from the L2, so a launch is fastest when its
-  // bytes are spread over 150-250 workgroups: ranges shrink down to 128 columns for narrow
-  // projections and stay at 1024 (two 64-column spans per wavefront, all loads still in
-  // registers) for wide ones.  Measured per launch at 32 tiles: o 6.2 us at 1024 columns,
-  // 5.1 at 512, 4.7 at 256; gate_up 8.2 / 8.9 / 11.1.
-  int nt = knobs.nt;
-  if (nt <= 0) {
-    long long cols = 0;
-    for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-    const int segs = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-    const int by_tokens = (a->num_tokens + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL;
-    const long long tiles = segs > by_tokens ? segs : by_tokens;  // about the number of tiles in use
-    nt = static_cast<int>(cols * tiles / 160);
-    if (nt > 1024) nt = 1024;
-    if (nt < 128) nt = 128;
-  }
-  if (nt < 64) nt = 64;
-  nt = (nt + 63) & ~63;
-  int total = 0;
-  for (;;) {
-    total = 0;
-    for (int i = 0; i < a->num_slices; ++i) total += (a->slices[i].n + nt - 1) / nt;
-    if (total <= kMaxSplits) break;
-    nt *= 2;
-  }
+  int nt;
+  const int total = decode_ranges(a, &nt);
   if (total == 0) return 0;
   int s = 0;
   l.widest = 0;

@@ -31,11 +31,12 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 // (tile, column range).
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
 int launch_decode(const MloraAddArgs* a, bool include_long);
+int decode_ranges(const MloraAddArgs* a, int* columns);  // column ranges of that launch, and columns per range
 
 // slot.hip: the same small tiles, the grid laid over the slots: weights are requested from the
 // workgroup index alone, before the slot's record has arrived.
 bool slot_supported(const MloraAddArgs* a);
-int slot_k_parts(const MloraAddArgs* a);  // 4 when the workgroups of a tile would share K out, else 1
+int slot_k_parts(const MloraAddArgs* a);  // 4 or 8 when the workgroups of a tile would share K out, else 1
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace);
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.
