@@ -146,6 +146,14 @@ def _pinned_slots(slots: list[int], counts: list[int], n: int) -> torch.Tensor:
     return host
 
 
+def _with_plan(tts: torch.Tensor, workspace: torch.Tensor, max_slots: int, **fields) -> LoRAContext:
+    """A context over arrays made here, its slot vector with the segment plan of the same launch."""
+    attach_plan(tts, workspace, max_slots)
+    context = LoRAContext(token_to_slot=tts, **fields)
+    context._unseen = True
+    return context
+
+
 def _context_in_one_launch(slots: list[int], counts: list[int], max_slots: int | None, device: torch.device | str) -> LoRAContext | None:
     """The context of a batch whose runs fit the arguments of the metadata launch; None (nothing done) for others."""
     fast = _hip.load_fastcall()
@@ -173,9 +181,8 @@ def _context_in_one_launch(slots: list[int], counts: list[int], max_slots: int |
     rc = fast.build_context(_hip.entry_point("mlora_meta_build_runs"), slots, counts, index, max_slots, cap, at, at + 4 * n, at + 8 * n,
                             at + 8 * n + 4 * cap, at + 8 * n + 8 * cap, at + 4 * head)
     _hip._check(rc, "mlora_meta_build_runs")
-    attach_plan(tts, workspace, max_slots)
-    return LoRAContext(token_to_slot=tts, token_indices_sorted_by_slot=sorted_idx, active_slot_ids=ids, num_tokens_per_slot=per_slot,
-                       slot_start_offsets=offsets, no_lora_flag=False, num_active_loras=n_active)
+    return _with_plan(tts, workspace, max_slots, token_indices_sorted_by_slot=sorted_idx, active_slot_ids=ids, num_tokens_per_slot=per_slot,
+                      slot_start_offsets=offsets, no_lora_flag=False, num_active_loras=n_active)
 
 
 def build_lora_context_from_batch_plan(
@@ -214,9 +221,10 @@ def build_lora_context_from_batch_plan(
              compact_offsets=offsets, compact_capacity=cap),
         dict(token_to_slot=tts, max_slots=max_slots, plan=workspace),
     ])
-    attach_plan(tts, workspace, max_slots)
-    return LoRAContext(
-        token_to_slot=tts,
+    return _with_plan(
+        tts,
+        workspace,
+        max_slots,
         token_indices_sorted_by_slot=sorted_idx[:n_lora],
         active_slot_ids=ids[:n_active],
         num_tokens_per_slot=per_slot[:n_active],

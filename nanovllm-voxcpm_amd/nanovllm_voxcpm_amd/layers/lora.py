@@ -182,7 +182,7 @@ class _LoRALayerBase(nn.Module):
         context = installed_lora_context(self.lora_domain)
         if context is None or context.no_lora_flag or not self.supports_lora or not self._targets_in_order or x.dim() != 2:
             return False
-        metadata, slots, active = context._cached_metadata, context.token_to_slot, context.active_slot_ids
+        metadata, slots, active = context._cached_metadata, context._slots, context.active_slot_ids
         if metadata is None or slots is None or metadata.token_to_slot is not slots or metadata.no_lora_flag or slots.size(0) != x.size(0):
             return False
         if active is not None and not active.is_cuda:

@@ -46,7 +46,26 @@ class LoRAContext:
     # like the sorted indices above): valid until the context is installed again or its buffers
     # are refreshed in place, both of which empty the table
     _segment_plans: dict = field(default_factory=dict, repr=False, compare=False)
+    # the slot vector was made by the builder and nobody has been given it yet: it cannot have been
+    # rewritten, and the plan that it brings along survives the first installation
+    _unseen: bool = field(default=False, repr=False, compare=False)
 
+    def __getstate__(self) -> dict:  # (a copy shares the vector)
+        self._unseen = False
+        return self.__dict__
+
+
+def _give_slots(self: LoRAContext) -> torch.Tensor | None:
+    self._unseen = False
+    return self._slots
+
+
+def _take_slots(self: LoRAContext, token_to_slot: torch.Tensor | None) -> None:
+    self._slots = token_to_slot  # what the LoRA linears read, which give the vector to nobody but the backend
+    self._unseen = False
+
+
+LoRAContext.token_to_slot = property(_give_slots, _take_slots)  # type: ignore[assignment]
 
 _DOMAINS: dict[str, LoRAContext] = {}
 
@@ -62,7 +81,10 @@ def installed_lora_context(domain: str) -> LoRAContext | None:
 
 
 def set_lora_context(lora_context: LoRAContext, *, domain: str = LM_LORA_DOMAIN) -> None:
-    invalidate_lora_context(lora_context)
+    if lora_context._unseen:
+        lora_context._unseen = False
+    else:
+        invalidate_lora_context(lora_context)
     _DOMAINS[domain] = lora_context
 
 
@@ -70,8 +92,9 @@ def invalidate_lora_context(lora_context: LoRAContext) -> None:
     """Forget everything derived from the context's tensors (call after rewriting them in place)."""
     lora_context._cached_metadata = None
     lora_context._segment_plans.clear()
-    if lora_context.token_to_slot is not None:
-        drop_attached_plan(lora_context.token_to_slot)
+    lora_context._unseen = False
+    if lora_context._slots is not None:
+        drop_attached_plan(lora_context._slots)
 
 
 def reset_lora_context(domain: str | None = None) -> None:

@@ -2,6 +2,9 @@
 built from and no rewritten one: rewrites that the version counter sees, and rewrites that it does not see and that
 are announced by invalidating or installing the context."""
 
+import copy
+import dataclasses
+
 import pytest
 import torch
 
@@ -61,6 +64,24 @@ def test_attached_plan_goes_with_a_rewrite(built, announce):
         announce(context)
     assert HipLoRABackend._plan_for(_metadata(context), tts, SLOTS, 0).workspace is not workspace
     assert len(built) == 1
+
+
+def _built(workspace: torch.Tensor) -> LoRAContext:
+    from nanovllm_voxcpm_amd.engine.lora_manager import _with_plan
+
+    return _with_plan(torch.tensor([0, 1, 2, 3, 0], dtype=torch.int32), workspace, SLOTS, no_lora_flag=False, num_active_loras=4)
+
+
+@pytest.mark.parametrize("first", [None, lambda c: c.token_to_slot, copy.copy, copy.deepcopy, dataclasses.replace, repr, invalidate_lora_context,
+                                   set_lora_context])
+def test_the_plan_survives_an_installation_only_while_nobody_could_have_rewritten_the_vector(built, first):
+    workspace = torch.zeros(16, dtype=torch.int32)
+    context = _built(workspace)
+    if first is not None:
+        first(context)
+    set_lora_context(context)
+    plan = HipLoRABackend._plan_for(_metadata(context), context._slots, SLOTS, 0)
+    assert (plan.workspace is workspace) == (first is None) and len(built) == (first is not None)
 
 
 @pytest.mark.gpu
