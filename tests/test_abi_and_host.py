@@ -62,6 +62,7 @@ def test_ctypes_structs_match_the_c_layout(tmp_path):
         "MloraExpandArgs": _hip.MloraExpandArgs,
         "MloraMetaArgs": _hip.MloraMetaArgs,
         "MloraInstallArgs": _hip.MloraInstallArgs,
+        "MloraInstallState": _hip.MloraInstallState,
     }
     lines = ['#include <stdio.h>', '#include <stddef.h>', '#include "mlora.h"', "int main(void) {"]
     for name, st in structs.items():

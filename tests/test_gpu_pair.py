@@ -3,11 +3,13 @@ token, full and barely started tiles, K of one 128-byte chunk and of many parts,
 inside a span, every rank's B row length, adapters below the buffers' rank with NaN beyond it, fp32."""
 
 import random
+import types
 
 import pytest
 import torch
 
 from oracle import lora_apply as oracle
+from test_gpu_parity import _check, _exact
 
 B16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 
@@ -70,5 +72,8 @@ def test_pair_form_against_fp64(case):
         runs.append(out.cpu())
     assert torch.equal(runs[0], runs[1])
     assert torch.equal(runs[0][indices < 0], y[indices < 0])
-    tol = dict(rtol=1e-5, atol=2e-5) if dtype == F32 else dict(rtol=1e-2, atol=2e-3)
-    assert torch.allclose(runs[0].float(), want.float(), **tol)
+    if dtype == F32:
+        assert torch.allclose(runs[0], want, rtol=1e-5, atol=2e-5)
+    else:  # to one rounding of the exact sum and of the intermediate
+        exact, mag = _exact(types.SimpleNamespace(a=shown_a, b=shown_b, widths=widths), x, y, indices, 0.75)
+        _check(runs[0], y, exact, mag, indices, f"pair {CASES[case]}")

@@ -2,10 +2,12 @@
 wrong: one token, full and further tiles of a slot, parts of 64 to 512 output columns, a last part that is short,
 every rank, adapters below the buffers' rank; the same bits whether partners' words are accepted or not."""
 
+import types
+
 import pytest
 import torch
 
-from oracle import lora_apply as oracle
+from test_gpu_parity import _check, _exact
 
 B16, F16 = torch.bfloat16, torch.float16
 CASES = [  # tokens, slots, rank, columns, element type, adapters of lower rank
@@ -36,7 +38,6 @@ def test_eight_parts_of_k_against_fp64(case, monkeypatch):
     ranks = [(5, rank, 8, rank // 2)[s % 4] if mixed else rank for s in range(slots)]
     for s, r in enumerate(ranks):
         a[s, r:], b[s, :, r:] = 0, 0
-    (want,) = oracle.fused_add_lora([y], x, [a], [b], indices=indices, scaling=0.75, accumulate=torch.float64)
     eff = torch.tensor(ranks, dtype=torch.int32, device="cuda") if mixed else None
     plan = build_segment_plan(indices.cuda(), slots)
     scratch = torch.empty(_hip.add_workspace_bytes(tokens, 1, rank, dtype), dtype=torch.uint8, device="cuda")
@@ -56,4 +57,5 @@ def test_eight_parts_of_k_against_fp64(case, monkeypatch):
         _hip.reload_knobs()
     assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])
     assert torch.equal(runs[0][indices < 0], y[indices < 0])
-    assert torch.allclose(runs[0].float(), want.float(), rtol=1e-2, atol=2e-3)
+    exact, mag = _exact(types.SimpleNamespace(a=[a], b=[b], widths=[n]), x, y, indices, 0.75)
+    _check(runs[0], y, exact, mag, indices, f"eight parts {CASES[case]}")
