@@ -56,9 +56,9 @@ extern "C" {
                               range's slice over the whole of K, keeps the result in LDS and expands it into its
                               range; needs no workspace */
 
-#define MLORA_FORM_PAIR 9  /* a shrink launch over (tile, slice, K part) and an expand launch over (tile, column range) that
-                              meet in the workspace; 16-token tiles for few tokens per slot, else 64-token tiles; weights and
-                              x rows go straight to LDS; 16- and 32-bit elements */
+#define MLORA_FORM_PAIR 9  /* small tiles, a shrink launch over (tile, slice, K part) and an expand launch over (tile, column
+                              range) that meet in the workspace; weights and x rows go straight to LDS; 16- and 32-bit
+                              elements */
 
 /* error codes (negative) */
 #define MLORA_E_INVALID (-1)     /* malformed argument (NULL pointer, negative size, bad dtype) */
@@ -108,8 +108,8 @@ typedef struct MloraAddArgs {
   float scaling;
   MloraSlice slices[MLORA_MAX_SLICES];
   void* workspace;        /* device scratch for the rank-r intermediate: between the producer and the
-                             consumer workgroups of MLORA_FORM_SPLIT and between the two launches of
-                             MLORA_FORM_SGMV; 256-byte aligned and at least MLORA_WORKSPACE_HEAD_BYTES
+                             consumer workgroups of MLORA_FORM_SPLIT, the workgroups of a tile of MLORA_FORM_SLOT
+                             and the two launches of MLORA_FORM_SGMV and MLORA_FORM_PAIR; 256-byte aligned and at least MLORA_WORKSPACE_HEAD_BYTES
                              long, or NULL (AUTO then keeps to MLORA_FORM_MFMA).  Counterpart of the
                              [S, T, r] buffer the reference allocates between its two kernels
                              (reference: nanovllm_voxcpm/lora.py:299-381).  Pass it to
@@ -145,7 +145,9 @@ int mlora_add_lora_static(const MloraAddArgs* args);
 
 /* Bytes of MloraAddArgs.workspace that let mlora_add_lora use every form it has for this shape
  * (a smaller workspace of at least MLORA_WORKSPACE_HEAD_BYTES is legal: the two-launch form then
- * splits K less, or AUTO does not choose it). */
+ * splits K less, or AUTO does not choose it).  MLORA_FORM_PAIR, whose partial sums lie by tile, may need more for
+ * a batch of few tokens per slot: behind the head 64 x slices x (r rounded up to 16) bytes for each of up to
+ * num_tokens / 16 + min(num_slots, num_tokens) tiles; without them AUTO takes the single-launch forms. */
 size_t mlora_add_workspace_bytes(int32_t num_tokens, int32_t num_slices, int32_t r, int32_t dtype);
 
 /* A workspace starts with a head of MLORA_WORKSPACE_HEAD_BYTES bytes: a signature word, the

@@ -227,7 +227,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active) {
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   switch (form) {
-    case MLORA_FORM_SPLIT: return true;
+    case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
     case MLORA_FORM_MFMA: {
       if (!exact_rank(a->r)) {
         const double width = static_cast<double>(a->num_slices) * a->k + cols * (cols > 4096 ? cols / 4096.0 : 1.0);

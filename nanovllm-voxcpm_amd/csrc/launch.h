@@ -68,8 +68,8 @@ bool wide_supported(const MloraAddArgs* a);
 bool wide_pays(const MloraAddArgs* a);
 int launch_wide(const MloraAddArgs* a);
 
-// pair.hip: a shrink launch and an expand launch over the 16- or the 64-token tiles, operands through
-// LDS by direct loads; 16- and 32-bit elements.
+// pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
+// direct loads; 16- and 32-bit elements.
 bool pair_supported(const MloraAddArgs* a);
 int launch_pair(const MloraAddArgs* a);
 

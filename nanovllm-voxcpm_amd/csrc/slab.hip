@@ -2,9 +2,10 @@
 // K part), fp32 partial sums to the workspace.  Computes what the reference computes with its segment-grouped
 // shrink kernel (nanovllm_voxcpm/lora_ops/triton_ops/lora_shrink_op.py:16-101).
 //
-// What bounds it is the bytes a compute unit takes in and how few instructions ask for them.  A 128-bit load in the matrix
-// cores' operand layout (sixteen rows in sixteen consecutive lanes) keeps the address unit busy four
-// times as long as one along a row, and operands that wait in registers limit what can be on its way.
+// What bounds it is the bytes a compute unit takes in and how few instructions ask for them.  128-bit loads in the matrix
+// cores' operand layout (sixteen rows in sixteen consecutive lanes) bring 9.4 TB/s out of the L2 into 256 compute units,
+// loads along rows straight to LDS 33.0 (from HBM both bring 6.0), and operands that wait in registers limit
+// what can be on its way.
 // Here both operands go to LDS by direct loads of whole row pieces (128 bytes of eight rows per load), into a
 // ring of two to four stages that each wavefront has to itself: the two wavefronts of a workgroup
 // cut K between them, each multiplies all tokens and ranks of the tile over its share, so nothing but

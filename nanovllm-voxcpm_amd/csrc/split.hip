@@ -31,6 +31,10 @@
 // so results never depend on timing and every workgroup exits whatever the others do.  The same
 // path serves a workspace that was never initialised (no signature): nobody publishes, nobody
 // waits.
+//
+// Who runs it: callers that ask for it, and under AUTO those whose workspace has no room for the shrink and
+// expand launches (pair.hip), which are faster at every shape measured (api.hip) and whose partial sums need
+// 16 x tile records x slices x rank x 4 bytes behind the head; the Python backend's scratch always has it.
 #include "common.h"
 #include "launch.h"
 

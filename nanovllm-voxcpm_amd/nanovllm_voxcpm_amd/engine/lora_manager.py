@@ -2,8 +2,8 @@
 
 Counterpart of the index builders of the reference's ``nanovllm_voxcpm/engine/lora_manager.py``
 (:67-180).  The reference sorts the tokens by slot in Python for every step and domain
-(:77-91) and uploads five packed arrays (:118-176); here only the slot-id vector crosses PCIe
-(one pinned copy) and one launch of the on-device counting sort produces the rest.  The
+(:77-91) and uploads five packed arrays (:118-176); here the slot ids travel with the launch of the
+on-device counting sort (those of very many sequences through one pinned copy), which produces the rest.  The
 adapter lifecycle / LRU residency half of that file lives in ``lora_runtime.py`` and is
 re-exported here under the reference's import path.
 """

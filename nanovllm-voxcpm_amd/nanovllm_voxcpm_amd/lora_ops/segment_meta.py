@@ -1,7 +1,7 @@
 """Segment metadata built on the GPU from the per-token slot-id vector.
 
 `SegmentPlan` is the workspace the fused apply kernels walk (tokens grouped by slot, tiles
-of at most 8 / 64 tokens).  `LoRAKernelMeta` keeps the reference's buffer-holding dataclass
+of at most 16 / 64 tokens).  `LoRAKernelMeta` keeps the reference's buffer-holding dataclass
 and field names (reference: nanovllm_voxcpm/lora_ops/triton_ops/lora_kernel_metadata.py:9-79)
 but fills every buffer with one launch of the on-device counting sort instead of
 sort / unique / cumsum plus a host read-back per call.
