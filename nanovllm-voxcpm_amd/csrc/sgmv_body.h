@@ -933,11 +933,18 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
     // per call with one / two / three / four parts, rank 32: down (K = 4096) of 2000 tokens 20.8 / 15.7 / 14.0 / 13.4,
     // of 4000 22.3 / 17.5 / 16.6 / 18.1, of 5000 23.4 / 18.5 / 20.8 / 19.2, of 6500 29.6 / 22.4 / 25.0 / 23.1; K = 8192,
     // 4000 tokens 48.8 / 37.5 / 32.0 / 36.1; o of 2000 tokens 12.7 / 11.6 / 11.3 / 11.1; gate_up of 6500 56.5 / 57.0 / 58.3.
+    // Long K is cut further: a workgroup's two wavefronts walk 2048 columns in about the time the rest of a tile takes, and
+    // uncut parts lose to the other shrink (sgmv.hip's / one / two / three / four parts, rank 16: K = 4096, 8200 tokens of 6
+    // slots 31.4 / 34.0 / 31.4 / 29.1 / 29.8, of 9392 33.8 / 37.9 / 35.8 / 33.1 / 34.0, of 9392 of 32 slots 34.3 / 38.5 / 36.6 /
+    // 37.4 / 35.0, of 12000 38.1 / 44.7 / 40.1 / 41.6 / 39.2; K = 8192, 5500 tokens 41.5 / 51.5 / 42.9 / 43.0 / 39.4, 7000 45.6 /
+    // 55.4 / 49.7 / 47.2 / 45.2, 9392 61.4 / 67.5 / 70.2 / 58.8 / 60.5; rank 32 alike): four parts where one would be
+    // taken from K = 4096 on, and from K = 8192 on throughout.
     s.all_slices = 0;
     ksplit = sgmv_knobs().ksplit;
     if (ksplit <= 0) {
       const int units = est_tiles * a->num_slices;
       ksplit = (205 + 2 * units / 5) / units;
+      if (a->k >= 8192 || (a->k >= 4096 && ksplit <= 1)) ksplit = kMaxKSplit;
       if (ksplit < 1) ksplit = 1;
       if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
       while (ksplit > 1 && a->k / 64 < ksplit * kSlabStages) --ksplit;

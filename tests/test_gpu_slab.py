@@ -22,6 +22,8 @@ CASES = [
     ([130, 20, 64, 31, 5], 64, 2048, [512], 4, F16, True, True),
     ([257, 16], 32, 4096, [1032], 2, B16, True, False),
     ([500, 40, 9], 16, 8192, [72, 200], 3, F16, False, True),
+    ([300, 40], 32, 8192, [72], 0, B16, True, False),  # four parts from K = 8192 on
+    ([4000, 4200], 16, 4096, [8], 0, F16, False, False),  # four parts of K = 4096 where tiles alone fill the chip
 ]
 
 
