@@ -1,0 +1,580 @@
+// The low-level shrink and expand over tiles of up to sixteen tokens of a slot, both products on the matrix cores.  Reference
+// semantics as in token.hip: lora_shrink (zero-filled output, scaling in the shrink: lora_ops/triton_ops/lora_shrink_op.py:257-341),
+// lora_expand (offset_start, add_inputs, product rounded to B's type first: lora_expand_op.py:94-170).
+//
+// The ops are given a slot id per token and nothing a kernel could trust to be sorted, so the one-workgroup-per-token
+// kernels (token.hip) let every token fetch A[slot] and B[slot] again and add 64 lanes up per rank.  Here a workgroup serves a
+// tile of a slot: it requests the slot vector and, from its own index or its token's id, the slot's weights, finds
+// its tokens among the ids as they arrive, and fetches each weight once for all of them.
+//
+// What bounds it: two trips to memory (ids, then the rows they name) and a compute unit's intake of weights in the second one;
+// hence ranks in blocks of eight or sixteen and tokens in tiles of four to sixteen, as many workgroups as the chip takes.
+#include "common.h"
+#include "launch.h"
+
+namespace mlora {
+
+namespace {
+
+// What the grid is laid over.  By slot: places are (tile of a slot, slot), then the tiles that no slot is expected to have (a
+// popular adapter's), which find out from a histogram whose they are.  By token: a place is a token; the first token of every
+// tile stands for it, the others leave.
+constexpr int kBySlot = 0, kByToken = 1;
+
+struct Places {
+  const int32_t* tts;
+  int T, num_slots;
+  int width;        // tokens of a tile: 4, 8 or 16 (tiles beyond the expected ones: 16)
+  int slots8;       // by slot: slot ids (and, in the shrink, one for the tokens without a slot) rounded up to eight
+  int tiles;        // by slot: tiles of a slot that have a place of their own
+};
+
+__device__ __forceinline__ int known_slot(const Places& p, int id) { return id >= 0 && id < p.num_slots ? id : p.num_slots; }
+
+// Lists in s_rows the tokens of `slot` from token `from` on: of those the ones at [first, first + width), in ascending order.  Returns
+// their number, or 0 when the tokens of the slot before `from` do not fill whole tiles.  s_wave: two words per wavefront.
+template <int THREADS>
+__device__ __forceinline__ int list_tile(const Places& p, int first_id, int slot, int from, int first, int width, int* __restrict__ s_rows,
+                                         int* __restrict__ s_wave) {
+  constexpr int W = THREADS / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  int late = 0, early = 0, id = first_id, half = 0;
+  for (int base = 0; base < p.T; base += THREADS) {
+    const int t = base + tid;
+    if (base > 0) id = p.tts[t < p.T ? t : p.T - 1];
+    const bool match = t < p.T && known_slot(p, id) == slot;
+    const uint64_t set = __builtin_amdgcn_ballot_w64(match && t >= from), before = __builtin_amdgcn_ballot_w64(match && t < from);
+    if (lane == 0) s_wave[half * W + wave] = __popcll(set) | (__popcll(before) << 16);
+    __syncthreads();
+    const int c = s_wave[half * W + (lane < W ? lane : 0)];
+    int pos = late;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int n = __builtin_amdgcn_readlane(c, w);
+      if (w < wave) pos += n & 0xffff;
+      late += n & 0xffff;
+      early += n >> 16;
+    }
+    pos += __popcll(set & ((1ull << lane) - 1ull)) - first;
+    if (match && t >= from && pos >= 0 && pos < width) s_rows[pos] = t;
+    half ^= 1;
+  }
+  __syncthreads();
+  const int n = late - first;
+  return early % width != 0 || n <= 0 ? 0 : n < width ? n : width;
+}
+
+// By slot, behind the expected tiles: the slot and first token position of the q-th tile beyond them, or slot -1.
+template <int THREADS>
+__device__ __forceinline__ void find_tile(const Places& p, int first_id, int q, int* __restrict__ s_hist, int* __restrict__ s_found) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  for (int s = tid; s < p.num_slots; s += THREADS) s_hist[s] = 0;
+  if (tid == 0) s_found[0] = -1;
+  __syncthreads();
+  for (int base = 0; base < p.T; base += THREADS) {
+    const int t = base + tid, s = t < p.T ? known_slot(p, base == 0 ? first_id : p.tts[t]) : p.num_slots;
+    // (the first token's slot in one addition: one adapter's tokens, each with an addition of its own to the same word, are a queue
+    // of 512 at the LDS unit)
+    const uint64_t any = __builtin_amdgcn_ballot_w64(s < p.num_slots);
+    if (any != 0) {
+      const int one = __builtin_amdgcn_readlane(s, __builtin_ctzll(any));
+      const uint64_t same = __builtin_amdgcn_ballot_w64(s == one);
+      if (lane == 0) atomicAdd(&s_hist[one], __popcll(same));
+      if (s < p.num_slots && s != one) atomicAdd(&s_hist[s], 1);
+    }
+  }
+  __syncthreads();
+  if (tid < kWave) {
+    const int covered = p.tiles * p.width;
+    int run = 0;
+    for (int base = 0; base < p.num_slots; base += kWave) {
+      const int s = base + lane, c = s < p.num_slots ? s_hist[s] - covered : 0;
+      const int mine = c > 0 ? (c + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL : 0;
+      int sum = mine;
+#pragma unroll
+      for (int d = 1; d < kWave; d *= 2) {
+        const int up = __shfl_up(sum, d, kWave);
+        if (lane >= d) sum += up;
+      }
+      const int at = q - (run + sum - mine);
+      if (at >= 0 && at < mine) {
+        s_found[0] = s;
+        s_found[1] = covered + at * MLORA_TILE_SMALL;
+      }
+      run += __builtin_amdgcn_readlane(sum, kWave - 1);
+    }
+  }
+  __syncthreads();
+}
+
+// ---- shrink -------------------------------------------------------------------------------------
+constexpr int kShrinkWaves = 8;  // a wavefront takes an eighth of K, in rounds of 128 columns
+constexpr int kShrinkThreads = kShrinkWaves * kWave;
+constexpr int kRound = 128 * kShrinkWaves;
+
+struct GroupShrinkParams {
+  void* out;
+  int64_t xs;
+  int out_dtype;
+  float scaling;
+  const void* a[MLORA_MAX_SLICES];
+};
+
+__device__ __forceinline__ void store_as(void* out, int64_t at, float v, int dtype) {
+  if (dtype == MLORA_DTYPE_F32) static_cast<float*>(out)[at] = v;
+  else if (dtype == MLORA_DTYPE_F16) static_cast<_Float16*>(out)[at] = from_f32<_Float16>(v);
+  else static_cast<__bf16*>(out)[at] = from_f32<__bf16>(v);
+}
+
+// out[slice, t, :] = scaling * x[t] . A[s]^T, zero for rows without a slot; grid (8, slices * blocks, places / 8), blockIdx.x the XCD
+// (a slot's workgroups share one).  RW: ranks of a workgroup (8 or 16); CH: rounds whose operands are on their way together.
+template <typename T, int RW, int CH, int GRID>
+__global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width_, int slots8,
+                                                                      int tiles, int blocks, int K, int r, const void* __restrict__ x,
+                                                                      GroupShrinkParams p) {
+  const Places pl{tts, T_, num_slots, width_, slots8, tiles};
+  constexpr int kStageRow = 17;  // 16 chunks of 16 bytes + one of padding: operand reads hit every bank once
+  constexpr int AI = RW / 4;     // loads of a round's A rows, four rows each
+  __shared__ __attribute__((aligned(16))) i32x4 s_stage[kShrinkWaves * 2 * 16 * kStageRow];
+  __shared__ __attribute__((aligned(16))) float s_red[kShrinkWaves * 64 * 4];
+  __shared__ int s_rows[MLORA_TILE_SMALL], s_wave[2 * kShrinkWaves], s_found[2];
+  static_assert(sizeof(s_stage) >= MLORA_MAX_SLOTS * sizeof(int), "the histogram takes the staging area");
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int place = blockIdx.z * 8 + blockIdx.x;
+  const int first_id = tts[tid < T_ ? tid : T_ - 1];
+  const int place_id = GRID == kByToken ? tts[place < T_ ? place : T_ - 1] : 0;
+  const int slice = blockIdx.y / blocks, r0 = (blockIdx.y - slice * blocks) * RW;
+  const int rounds = K / kRound;
+  const int64_t out0 = static_cast<int64_t>(slice) * T_ * r;
+  int slot, from = 0, first = 0, width = width_;
+  if constexpr (GRID == kByToken) {
+    if (place >= T_) return;
+    slot = known_slot(pl, __builtin_amdgcn_readfirstlane(place_id));
+    from = place;
+    if (slot == num_slots) {
+      if (tid < RW && r0 + tid < r) store_as(p.out, out0 + static_cast<int64_t>(place) * r + r0 + tid, 0.f, p.out_dtype);
+      return;
+    }
+  } else {
+    const int tile = place / slots8;
+    slot = place - tile * slots8;
+    first = tile * width;
+    if (tile >= tiles) {
+      find_tile<kShrinkThreads>(pl, first_id, place - tiles * slots8, reinterpret_cast<int*>(s_stage), s_found);
+      slot = __builtin_amdgcn_readfirstlane(s_found[0]);
+      if (slot < 0) return;
+      first = __builtin_amdgcn_readfirstlane(s_found[1]);
+      width = MLORA_TILE_SMALL;
+    } else if (slot >= num_slots) {
+      if (slot == num_slots && tile == 0) {  // the tokens without a slot
+        for (int e = tid; e < T_ * RW; e += kShrinkThreads) {
+          const int t = e / RW, rank = r0 + e % RW;
+          if (rank < r && known_slot(pl, tts[t]) == num_slots) store_as(p.out, out0 + static_cast<int64_t>(t) * r + rank, 0.f, p.out_dtype);
+        }
+      }
+      return;
+    }
+  }
+  i32x4 ast[AI * CH];
+  const T* A = static_cast<const T*>(p.a[slice]) + static_cast<int64_t>(slot) * r * K + wave * (rounds * 128) + lr * 8;
+  auto request_a = [&](const int from_round) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int k = (from_round + c < rounds ? from_round + c : rounds - 1) * 128;
+#pragma unroll
+      for (int i = 0; i < AI; ++i) {
+        const int row = r0 + 4 * i + lg;
+        ast[AI * c + i] = load128(A + static_cast<int64_t>(row < r ? row : r - 1) * K + k);
+      }
+    }
+  };
+  request_a(0);
+  __builtin_amdgcn_sched_barrier(0);
+  const int left = list_tile<kShrinkThreads>(pl, first_id, slot, from, first, width, s_rows, s_wave);
+  if (left == 0) {
+    // (named as used here too, or the compiler sinks the requests behind the listing of the tokens)
+#pragma unroll
+    for (int j = 0; j < AI * CH; ++j) asm volatile("" ::"v"(ast[j]));
+    return;
+  }
+  i32x4* stage = s_stage + wave * 2 * 16 * kStageRow;
+  const T* xrow[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int at = 4 * i + lg < left ? 4 * i + lg : left - 1;
+    xrow[i] = static_cast<const T*>(x) + static_cast<int64_t>(s_rows[at]) * p.xs + wave * (rounds * 128) + lr * 8;
+  }
+  f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+  for (int now = 0; now < rounds; now += CH) {
+    i32x4 xst[4 * CH];
+    if (now > 0) request_a(now);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i == 0 || 4 * i < left) {  // (rows of absent tokens are products nobody stores: any value will do)
+#pragma unroll
+        for (int c = 0; c < CH; ++c) xst[4 * c + i] = load128(xrow[i] + (now + c < rounds ? now + c : rounds - 1) * 128);
+      } else {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) xst[4 * c + i] = i32x4{0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (now + c >= rounds) break;
+      Pack8 xa[4], aw[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) stage[(4 * i + lg) * kStageRow + lr] = xst[4 * c + i];
+#pragma unroll
+      for (int i = 0; i < AI; ++i) stage[(16 + 4 * i + lg) * kStageRow + lr] = ast[AI * c + i];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        xa[i].raw = stage[lr * kStageRow + 4 * i + lg];
+        aw[i].raw = stage[(16 + (lr & (RW - 1))) * kStageRow + 4 * i + lg];
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[0] = Mma<T>::run(xa[i], aw[i], acc[0]);
+    }
+  }
+  mfma_settle(acc);  // (the rounds end behind a branch)
+  // sum of the wavefronts' shares: a lane holds H[token 4 * lg + i][rank r0 + lr]
+  *reinterpret_cast<f32x4*>(&s_red[(wave * 64 + lane) * 4]) = acc[0];
+  __syncthreads();
+  const int tok = tid / RW, rank = tid % RW;
+  if (tok < left && r0 + rank < r) {
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kShrinkWaves; ++w) sum += s_red[(w * 64 + (tok >> 2) * 16 + rank) * 4 + (tok & 3)];
+    store_as(p.out, out0 + static_cast<int64_t>(s_rows[tok]) * r + r0 + rank, sum * p.scaling, p.out_dtype);
+  }
+}
+
+// ---- expand -------------------------------------------------------------------------------------
+constexpr int kExpandWaves = 4;
+constexpr int kExpandThreads = kExpandWaves * kWave;
+
+struct GroupExpandParams {
+  const void* h; void* y;
+  int64_t ys;
+  int add_inputs, num_slices;
+  int first[MLORA_MAX_SLICES];  // first column range of a slice
+  const void* b[MLORA_MAX_SLICES];
+  int n[MLORA_MAX_SLICES];
+  int col[MLORA_MAX_SLICES];
+};
+
+// Eight ranks of the intermediate at the weight's precision, as the reference's kernel casts it.
+template <typename T, typename H> __device__ __forceinline__ Pack8 load_h(const H* p) {
+  Pack8 v;
+  if constexpr (std::is_same<H, T>::value) {
+    v.raw = load128(p);
+  } else {
+    float f[8];
+    if constexpr (sizeof(H) == 4) {
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { f[e] = lo[e]; f[4 + e] = hi[e]; }
+    } else {
+      Pack8 q;
+      q.raw = load128(p);
+      unpack8<H>(q, f);
+    }
+    pack8<T>(f, v);
+  }
+  return v;
+}
+
+// y[t, col_i + n] (+)= round_T(h[i, t] . B_i[s]^T); grid (8, column ranges, places / 8).  A wavefront takes SP spans of 64 columns.
+template <typename T, typename H, int KSTEPS, int SP, int GRID>
+__global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width_, int slots8,
+                                                                      int tiles, int r, GroupExpandParams p) {
+  const Places pl{tts, T_, num_slots, width_, slots8, tiles};
+  __shared__ int s_hist[GRID == kBySlot ? MLORA_MAX_SLOTS : 1], s_rows[MLORA_TILE_SMALL], s_wave[2 * kExpandWaves], s_found[2];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int place = blockIdx.z * 8 + blockIdx.x;
+  const int first_id = tts[tid < T_ ? tid : T_ - 1];
+  const int place_id = GRID == kByToken ? tts[place < T_ ? place : T_ - 1] : 0;
+  int slice = 0;
+  while (slice + 1 < p.num_slices && static_cast<int>(blockIdx.y) >= p.first[slice + 1]) ++slice;
+  const int n = p.n[slice], c0 = ((static_cast<int>(blockIdx.y) - p.first[slice]) * kExpandWaves + wave) * (SP * 64);
+  int slot, from = 0, first = 0, width = width_;
+  if constexpr (GRID == kByToken) {
+    if (place >= T_) return;
+    slot = known_slot(pl, __builtin_amdgcn_readfirstlane(place_id));
+    from = place;
+  } else {
+    const int tile = place / slots8;
+    slot = place - tile * slots8;
+    first = tile * width;
+    if (tile >= tiles) {
+      find_tile<kExpandThreads>(pl, first_id, place - tiles * slots8, s_hist, s_found);
+      slot = __builtin_amdgcn_readfirstlane(s_found[0]);
+      if (slot < 0) return;
+      first = __builtin_amdgcn_readfirstlane(s_found[1]);
+      width = MLORA_TILE_SMALL;
+    }
+  }
+  if (slot >= num_slots) return;
+  // (requested whether a span exists or not, clamped into the slice)
+  Pack8 bop[SP][4][KSTEPS];
+  const T* B = static_cast<const T*>(p.b[slice]) + static_cast<int64_t>(slot) * n * r;
+#pragma unroll
+  for (int s = 0; s < SP; ++s)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int col = c0 + s * 64 + 4 * lr + j;
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        const int piece = lg + 4 * ks;
+        bop[s][j][ks].raw = load128(B + static_cast<int64_t>(col < n ? col : n - 1) * r + (piece * 8 < r ? piece * 8 : 0));
+      }
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  const int left = list_tile<kExpandThreads>(pl, first_id, slot, from, first, width, s_rows, s_wave);
+  if (left == 0 || c0 >= n) {
+    // (named as used here too, or the compiler sinks the requests behind the listing of the tokens)
+#pragma unroll
+    for (int s = 0; s < SP; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" ::"v"(bop[s][j][ks].raw));
+    return;
+  }
+  const H* hin = static_cast<const H*>(p.h) + static_cast<int64_t>(slice) * T_ * r;
+  T* const y = static_cast<T*>(p.y) + p.col[slice];
+  // token j of a tile is row 4 * (j % 4) + j / 4 of the product: a lane then holds tokens lg, 4 + lg, 8 + lg, 12 + lg, and a
+  // tile of four tokens is one request for y and one store
+  Pack8 hop[KSTEPS];
+  {
+    const int tok = 4 * (lr & 3) + (lr >> 2);
+    const H* row = hin + static_cast<int64_t>(s_rows[tok < left ? tok : left - 1]) * r;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const int piece = lg + 4 * ks;
+      hop[ks] = load_h<T, H>(row + (piece * 8 < r ? piece * 8 : 0));
+    }
+  }
+  int row[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) row[i] = s_rows[4 * i + lg < left ? 4 * i + lg : left - 1];
+  uint2 yq[SP][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (p.add_inputs && 4 * i < left) {
+#pragma unroll
+      for (int s = 0; s < SP; ++s) {
+        const int c = c0 + s * 64 + 4 * lr;
+        yq[s][i] = *reinterpret_cast<const uint2*>(y + static_cast<int64_t>(row[i]) * p.ys + (c < n ? c : n - 4));
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SP; ++s) yq[s][i] = uint2{0, 0};
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    f32x4 out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      out[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        Pack8 hv = hop[ks], bv = bop[s][j][ks];
+        if ((lg + 4 * ks) * 8 >= r) hv.raw = bv.raw = i32x4{0, 0, 0, 0};  // (pieces beyond the rank)
+        out[j] = Mma<T>::run(hv, bv, out[j]);
+      }
+    }
+    const int c = c0 + s * 64 + 4 * lr;
+    if (c < n) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (4 * i + lg < left) {
+          union { uint2 raw; T e[4]; } v;
+          v.raw = yq[s][i];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const T d = from_f32<T>(out[j][i]);
+            v.e[j] = p.add_inputs ? from_f32<T>(to_f32(v.e[j]) + to_f32(d)) : d;
+          }
+          *reinterpret_cast<uint2*>(y + static_cast<int64_t>(row[i]) * p.ys + c) = v.raw;
+        }
+      }
+    }
+  }
+}
+
+bool aligned(const void* p, int to) { return reinterpret_cast<uintptr_t>(p) % to == 0; }
+
+// Diagnostic knob, read from the environment once and again after mlora_reload_knobs().
+struct GroupKnobs {
+  int generation = -1, use;
+  void read() {
+    generation = knob_generation();
+    use = env_int("MLORA_GROUP", 1);  // 0: never, 2: also where one workgroup per token is the faster one
+  }
+};
+const GroupKnobs& group_knobs() {
+  static GroupKnobs k;
+  if (k.generation != knob_generation()) k.read();
+  return k;
+}
+
+constexpr int kMostTokens = 4096;  // of a call (every workgroup reads the slot vector)
+
+int groups_about(int tokens, int slots) { return tokens < slots ? tokens : slots; }  // slots with tokens, at most
+
+// Fills in how a launch of `parts` workgroups per tile is laid out; returns its places.  extra: places for the tokens without a slot.
+int lay_out(Places& p, int* over, long long parts, int extra) {
+  const int groups = groups_about(p.T, p.num_slots);
+  // tiles of four tokens while that many workgroups find room on the chip, else eight, else sixteen
+  p.width = 4;
+  while (p.width < 16 && parts * groups * (1 + p.T / (groups * p.width)) > 256) p.width *= 2;
+  // over the tokens where slots without any would be most of the places
+  *over = p.T <= p.num_slots ? kByToken : kBySlot;
+  p.slots8 = p.tiles = 0;
+  if (*over == kByToken) return p.T;
+  p.slots8 = (p.num_slots + extra + 7) & ~7;
+  p.tiles = 1 + p.T / (p.num_slots * p.width);
+  const int covered = p.tiles * p.width;
+  return p.slots8 * p.tiles + (p.T > covered ? (p.T - covered + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL : 0);
+}
+
+struct ShrinkLaunch {
+  const MloraShrinkArgs* a;
+  Places at;
+  int over, blocks;
+  dim3 grid;
+  GroupShrinkParams p;
+};
+template <typename T, int RW, int CH> void shrink_grid(const ShrinkLaunch& l) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, l.grid, dim3(kShrinkThreads), 0, static_cast<hipStream_t>(l.a->stream), l.at.tts, l.at.T, l.at.num_slots, l.at.width,
+                       l.at.slots8, l.at.tiles, l.blocks, l.a->k, l.a->r, l.a->x, l.p);
+  };
+  if (l.over == kBySlot) launch(group_shrink_kernel<T, RW, CH, kBySlot>);
+  else launch(group_shrink_kernel<T, RW, CH, kByToken>);
+}
+template <typename T, int RW> void shrink_rounds(const ShrinkLaunch& l) {
+  const int rounds = l.a->k / kRound;
+  if (rounds == 1) shrink_grid<T, RW, 1>(l);
+  else if (rounds == 2) shrink_grid<T, RW, 2>(l);
+  else shrink_grid<T, RW, 4>(l);
+}
+template <typename T> void shrink_type(const ShrinkLaunch& l, int rw) {
+  if (rw == 8) shrink_rounds<T, 8>(l);
+  else shrink_rounds<T, 16>(l);
+}
+
+struct ExpandLaunch {
+  const MloraExpandArgs* a;
+  Places at;
+  int over, spans;
+  dim3 grid;
+  GroupExpandParams p;
+};
+template <typename T, typename H, int KSTEPS, int SP> void expand_grid(const ExpandLaunch& l) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, l.grid, dim3(kExpandThreads), 0, static_cast<hipStream_t>(l.a->stream), l.at.tts, l.at.T, l.at.num_slots, l.at.width,
+                       l.at.slots8, l.at.tiles, l.a->r, l.p);
+  };
+  if (l.over == kBySlot) launch(group_expand_kernel<T, H, KSTEPS, SP, kBySlot>);
+  else launch(group_expand_kernel<T, H, KSTEPS, SP, kByToken>);
+}
+template <typename T, typename H> void expand_ranks(const ExpandLaunch& l) {
+  if (l.a->r <= 32) l.spans == 1 ? expand_grid<T, H, 1, 1>(l) : expand_grid<T, H, 1, 2>(l);
+  else l.spans == 1 ? expand_grid<T, H, 2, 1>(l) : expand_grid<T, H, 2, 2>(l);
+}
+template <typename T> void expand_type(const ExpandLaunch& l) {
+  if (l.a->h_dtype == MLORA_DTYPE_F32) expand_ranks<T, float>(l);
+  else if (l.a->h_dtype == MLORA_DTYPE_F16) expand_ranks<T, _Float16>(l);
+  else expand_ranks<T, __bf16>(l);
+}
+
+}  // namespace
+
+// Where tiles of a slot beat one workgroup per token.  What a token's workgroup costs grows with the A rows it takes in, so from rank 32
+// on the tiles are the faster ones at every size; below, the listing of the tokens (0.5 us) has to be earned.  Replayed graphs, us per call,
+// per token / tiles: rank 32 and 64, K = 1024, one token: 4.3 / 3.7 and 6.7 / 3.7, 130 tokens over 64 slots, three slices: 7.0 / 5.9 and
+// 11.7 / 9.2, K = 8192, 37 tokens: 15.3 / 7.9 (rank 32) and 41 / 12.5.  Rank 16 by tokens x slices x rank x K in millions: 0.6:
+// 3.4 / 3.8, 4.2: 4.2 / 4.4, 6.4: 4.8 / 4.8, 8.4: 4.75 / 4.75, 12.6 (256 tokens over 32 slots, three slices): 5.4 / 4.4, 25: 7.7 / 4.7; with
+// long K earlier: K = 4096, 2.4: 6.1 / 5.4, K = 8192, 1.2: 8.1 / 7.5; rank 8 alike (0.3 at K = 4096: 4.3 / 5.3).  Beyond 512 tokens every workgroup reads the slot
+// vector in several steps (1000 tokens over 4 slots, rank 64, three slices: 19 / 26).
+bool group_shrink_supported(const MloraShrinkArgs* a) {
+  if (group_knobs().use == 0 || a->dtype == MLORA_DTYPE_F32 || a->num_slots < 1 || a->num_slots > MLORA_MAX_SLOTS || a->num_tokens > kMostTokens) return false;
+  if (a->r < 1 || a->r > 64 || a->k < kRound || a->k % kRound || a->x_stride % 8 || !aligned(a->x, 16)) return false;
+  for (int i = 0; i < a->num_slices; ++i)
+    if (!aligned(a->a[i], 16)) return false;
+  if (group_knobs().use == 2) return true;
+  if (a->r <= 16) {
+    const double cells = static_cast<double>(a->num_tokens) * a->num_slices * a->r * a->k;
+    if (cells < (a->k >= 4096 ? 1.2e6 : 7.0e6) || a->num_tokens > 64 * a->num_slots) return false;
+  }
+  return a->num_tokens <= 512;
+}
+
+int launch_group_shrink(const MloraShrinkArgs* a) {
+  ShrinkLaunch l = {};
+  l.a = a;
+  l.at.tts = a->token_to_slot; l.at.T = a->num_tokens; l.at.num_slots = a->num_slots;
+  l.p.out = a->out; l.p.xs = a->x_stride; l.p.out_dtype = a->out_dtype; l.p.scaling = a->scaling;
+  for (int i = 0; i < a->num_slices; ++i) l.p.a[i] = a->a[i];
+  // ranks in blocks of eight where blocks of sixteen would leave half of the compute units without a workgroup
+  const int rw = a->r <= 8 || static_cast<long long>(groups_about(l.at.T, l.at.num_slots)) * a->num_slices * ((a->r + 15) / 16) < 128 ? 8 : 16;
+  l.blocks = (a->r + rw - 1) / rw;
+  const int places = lay_out(l.at, &l.over, static_cast<long long>(a->num_slices) * l.blocks, 1);
+  l.grid = dim3(8, static_cast<unsigned>(a->num_slices * l.blocks), static_cast<unsigned>((places + 7) / 8));
+  if (a->dtype == MLORA_DTYPE_BF16) shrink_type<__bf16>(l, rw);
+  else shrink_type<_Float16>(l, rw);
+  return check_launch("mlora_shrink");
+}
+
+// Measured as above, per token / tiles: rank 16, 1024 columns: one token 3.1 / 2.9, 256 over 32 slots 4.4 / 3.3, 512 over 64 5.6 / 4.4;
+// 8192 columns: 256 over 32 10.8 / 6.4; rank 64: one token 6.0 / 3.2, 130 over 64, 8192 columns 120 / 16, 512 over 64 349 / 20.
+// Not where a grid over the tokens would be mostly workgroups that leave again while B rows are short (rank 16, 8192 columns, 37 tokens of 64
+// slots: 5.4 / 6.1; 16384: 7.3 / 8.7), nor at rank 8 except for many tokens of many slots (512 over 64: 12.6 / 8.3, over 4 slots
+// 9.1 / 9.7), nor, up to rank 16, beyond 64 tokens per slot id or 1024 in all (512 over 4, 1024 columns: 4.0 / 4.6; 1000 over 32 6.2 / 7.0,
+// 8192 columns 29 / 16; 4096 over 32 14.2 / 17.3).  All tokens on one slot of many: 512 tokens, 24 slots, rank 16 3.9 / 5.4, rank 64 17.7 / 6.9.
+bool group_expand_supported(const MloraExpandArgs* a) {
+  if (group_knobs().use == 0 || a->dtype == MLORA_DTYPE_F32 || a->num_slots < 1 || a->num_slots > MLORA_MAX_SLOTS || a->num_tokens > kMostTokens) return false;
+  if (a->r < 8 || a->r > 64 || a->r % 8 || a->y_stride % 4 || a->offset_start % 4 || !aligned(a->y, 8) || !aligned(a->h, 16)) return false;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) {
+    if (a->n[i] % 4 || !aligned(a->b[i], 16)) return false;
+    cols += a->n[i];
+  }
+  if (cols > 1 << 23) return false;  // (column ranges of the grid)
+  if (group_knobs().use == 2) return true;
+  if (a->r <= 8 && !(a->num_tokens >= 256 && a->num_slots >= 16)) return false;
+  if (a->r > 16) return true;
+  if (a->num_tokens <= a->num_slots && cols >= 8192) return false;
+  return a->num_tokens <= 1024 && a->num_tokens <= 64 * a->num_slots;
+}
+
+int launch_group_expand(const MloraExpandArgs* a) {
+  ExpandLaunch l = {};
+  l.a = a;
+  l.at.tts = a->token_to_slot; l.at.T = a->num_tokens; l.at.num_slots = a->num_slots;
+  l.p.h = a->h; l.p.y = a->y; l.p.ys = a->y_stride; l.p.add_inputs = a->add_inputs ? 1 : 0; l.p.num_slices = a->num_slices;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->n[i];
+  l.spans = cols * groups_about(l.at.T, l.at.num_slots) >= 131072 ? 2 : 1;
+  const int nt = l.spans * 64 * kExpandWaves;
+  int col = a->offset_start, total = 0;
+  for (int i = 0; i < a->num_slices; ++i) {
+    l.p.first[i] = total;
+    l.p.b[i] = a->b[i]; l.p.n[i] = a->n[i]; l.p.col[i] = col;
+    col += a->n[i];
+    total += (a->n[i] + nt - 1) / nt;
+  }
+  const int places = lay_out(l.at, &l.over, total, 0);
+  l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>((places + 7) / 8));
+  if (a->dtype == MLORA_DTYPE_BF16) expand_type<__bf16>(l);
+  else expand_type<_Float16>(l);
+  return check_launch("mlora_expand");
+}
+
+}  // namespace mlora

@@ -73,6 +73,12 @@ int launch_wide(const MloraAddArgs* a);
 bool pair_supported(const MloraAddArgs* a);
 int launch_pair(const MloraAddArgs* a);
 
+// group.hip: the low-level shrink and expand over tiles of a slot; `supported` says where they are the faster ones too.
+bool group_shrink_supported(const MloraShrinkArgs* a);
+int launch_group_shrink(const MloraShrinkArgs* a);
+bool group_expand_supported(const MloraExpandArgs* a);
+int launch_group_expand(const MloraExpandArgs* a);
+
 // in-kernel timeline of trace builds (no-ops otherwise)
 void decode_trace_set(void* buf);
 void slot_trace_set(void* buf);

@@ -6,6 +6,7 @@
 // add_inputs, product rounded to B's type first: lora_expand_op.py:94-170), set_slot_lora
 // (slot zeroed, rank-limited copy, alpha / r folded into B: nanovllm_voxcpm/layers/lora.py:395-417).
 #include "common.h"
+#include "launch.h"
 
 namespace mlora {
 
@@ -103,23 +104,25 @@ __global__ __launch_bounds__(kTokThreads) void token_shrink_kernel(TokenShrinkPa
 // wavefront at rank 16 were four such trips; x is asked for with the slot id and the rows of a step
 // together: 256 tokens, rank 16, three slices or one, 6.0 -> 5.0 us.
 constexpr int kRowsTogether = 4;
+// (x, the slot vector and the sizes are leading arguments, which arrive in scalar registers: the first trip waits for no argument fetch)
 template <typename T, typename O>
-__global__ __launch_bounds__(kTokThreads) void token_shrink_vec_kernel(TokenShrinkParams p) {
+__global__ __launch_bounds__(kTokThreads) void token_shrink_vec_kernel(const void* __restrict__ rows, const int32_t* __restrict__ tts, int64_t xs, int K,
+                                                                       TokenShrinkParams p) {
   const int t = blockIdx.x, i = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   O* out = static_cast<O*>(p.out) + (static_cast<int64_t>(i) * p.T + t) * p.r;
-  const T* x = static_cast<const T*>(p.x) + static_cast<int64_t>(t) * p.xs;
-  const int chunks = p.K / 8;
+  const T* x = static_cast<const T*>(rows) + static_cast<int64_t>(t) * xs;
+  const int chunks = K / 8;
   constexpr int kHeld = 2;  // of a lane's x pieces: all of them up to K = 1024
   Pack8 xv[kHeld];
 #pragma unroll
   for (int q = 0; q < kHeld; ++q) xv[q].raw = load128(x + (lane + q * kWave < chunks ? lane + q * kWave : 0) * 8);
-  const int s = p.tts[t];
+  const int s = tts[t];
   if (s < 0 || s >= p.num_slots) {
     for (int j = tid; j < p.r; j += kTokThreads) out[j] = from_f32<O>(0.f);
     return;
   }
-  const T* A = static_cast<const T*>(p.a[i]) + static_cast<int64_t>(s) * p.r * p.K;
+  const T* A = static_cast<const T*>(p.a[i]) + static_cast<int64_t>(s) * p.r * K;
   for (int j0 = wave; j0 < p.r; j0 += kTokWaves * kRowsTogether) {
     float acc[kRowsTogether];
     int64_t row[kRowsTogether];
@@ -127,7 +130,7 @@ __global__ __launch_bounds__(kTokThreads) void token_shrink_vec_kernel(TokenShri
     for (int u = 0; u < kRowsTogether; ++u) {
       acc[u] = 0.f;
       const int j = j0 + u * kTokWaves;
-      row[u] = static_cast<int64_t>(j < p.r ? j : j0) * p.K;
+      row[u] = static_cast<int64_t>(j < p.r ? j : j0) * K;
     }
     auto step = [&](int c, const Pack8& xc) {
       Pack8 av[kRowsTogether];
@@ -198,21 +201,22 @@ __global__ __launch_bounds__(kTokThreads) void token_expand_kernel(TokenExpandPa
 // (256 tokens, rank 16: 5.8 -> 4.6 us).
 constexpr int kColumns = 4;
 template <typename T, typename H>
-__global__ __launch_bounds__(kTokThreads) void token_expand_vec_kernel(TokenExpandParams p) {
+__global__ __launch_bounds__(kTokThreads) void token_expand_vec_kernel(const void* __restrict__ hv, const int32_t* __restrict__ tts, int T_, int r,
+                                                                       TokenExpandParams p) {
   __shared__ float h[MLORA_MAX_RANK];
   const int t = blockIdx.x, i = blockIdx.z;
   const int tid = threadIdx.x;
-  const H* hin = static_cast<const H*>(p.h) + (static_cast<int64_t>(i) * p.T + t) * p.r;
+  const H* hin = static_cast<const H*>(hv) + (static_cast<int64_t>(i) * T_ + t) * r;
   // (the intermediate's place does not depend on the slot: asked for together with the slot id)
-  for (int j = tid; j < p.r; j += kTokThreads) h[j] = to_f32(from_f32<T>(to_f32(hin[j])));
-  const int s = p.tts[t];
+  for (int j = tid; j < r; j += kTokThreads) h[j] = to_f32(from_f32<T>(to_f32(hin[j])));
+  const int s = tts[t];
   if (s < 0 || s >= p.num_slots) return;
   const int N = p.n[i];
   const int chunk = (N + p.nsplit - 1) / p.nsplit;
   const int n0 = blockIdx.y * chunk;
   const int n1 = n0 + chunk < N ? n0 + chunk : N;
   if (n0 >= n1) return;
-  const T* B = static_cast<const T*>(p.b[i]) + static_cast<int64_t>(s) * N * p.r;
+  const T* B = static_cast<const T*>(p.b[i]) + static_cast<int64_t>(s) * N * r;
   T* y = static_cast<T*>(p.y) + static_cast<int64_t>(t) * p.ys + p.col[i];
   bool waited = false;
   for (int base = n0; base < n1; base += kTokThreads * kColumns) {
@@ -223,7 +227,7 @@ __global__ __launch_bounds__(kTokThreads) void token_expand_vec_kernel(TokenExpa
     for (int u = 0; u < kColumns; ++u) {
       const int n = base + u * kTokThreads + tid;
       at[u] = n < n1 ? n : n1 - 1;
-      first[u].raw = load128(B + at[u] * p.r);
+      first[u].raw = load128(B + at[u] * r);
       yv[u] = p.add_inputs ? y[at[u]] : T(0);
     }
     if (!waited) __syncthreads();
@@ -231,11 +235,11 @@ __global__ __launch_bounds__(kTokThreads) void token_expand_vec_kernel(TokenExpa
     float acc[kColumns];
 #pragma unroll
     for (int u = 0; u < kColumns; ++u) acc[u] = 0.f;
-    for (int j = 0; j < p.r; j += 8) {
+    for (int j = 0; j < r; j += 8) {
       Pack8 next[kColumns];
-      if (j + 8 < p.r) {
+      if (j + 8 < r) {
 #pragma unroll
-        for (int u = 0; u < kColumns; ++u) next[u].raw = load128(B + at[u] * p.r + j + 8);
+        for (int u = 0; u < kColumns; ++u) next[u].raw = load128(B + at[u] * r + j + 8);
       }
 #pragma unroll
       for (int u = 0; u < kColumns; ++u) {
@@ -405,18 +409,18 @@ void launch_shrink_out(const TokenShrinkParams& p, dim3 grid, int out_dtype, hip
 template <typename T>
 void launch_shrink_vec_out(const TokenShrinkParams& p, dim3 grid, int out_dtype, hipStream_t st) {
   switch (out_dtype) {
-    case MLORA_DTYPE_F32: hipLaunchKernelGGL((token_shrink_vec_kernel<T, float>), grid, dim3(kTokThreads), 0, st, p); break;
-    case MLORA_DTYPE_F16: hipLaunchKernelGGL((token_shrink_vec_kernel<T, _Float16>), grid, dim3(kTokThreads), 0, st, p); break;
-    default: hipLaunchKernelGGL((token_shrink_vec_kernel<T, __bf16>), grid, dim3(kTokThreads), 0, st, p); break;
+    case MLORA_DTYPE_F32: hipLaunchKernelGGL((token_shrink_vec_kernel<T, float>), grid, dim3(kTokThreads), 0, st, p.x, p.tts, p.xs, p.K, p); break;
+    case MLORA_DTYPE_F16: hipLaunchKernelGGL((token_shrink_vec_kernel<T, _Float16>), grid, dim3(kTokThreads), 0, st, p.x, p.tts, p.xs, p.K, p); break;
+    default: hipLaunchKernelGGL((token_shrink_vec_kernel<T, __bf16>), grid, dim3(kTokThreads), 0, st, p.x, p.tts, p.xs, p.K, p); break;
   }
 }
 
 template <typename T>
 void launch_expand_vec_h(const TokenExpandParams& p, dim3 grid, int h_dtype, hipStream_t st) {
   switch (h_dtype) {
-    case MLORA_DTYPE_F32: hipLaunchKernelGGL((token_expand_vec_kernel<T, float>), grid, dim3(kTokThreads), 0, st, p); break;
-    case MLORA_DTYPE_F16: hipLaunchKernelGGL((token_expand_vec_kernel<T, _Float16>), grid, dim3(kTokThreads), 0, st, p); break;
-    default: hipLaunchKernelGGL((token_expand_vec_kernel<T, __bf16>), grid, dim3(kTokThreads), 0, st, p); break;
+    case MLORA_DTYPE_F32: hipLaunchKernelGGL((token_expand_vec_kernel<T, float>), grid, dim3(kTokThreads), 0, st, p.h, p.tts, p.T, p.r, p); break;
+    case MLORA_DTYPE_F16: hipLaunchKernelGGL((token_expand_vec_kernel<T, _Float16>), grid, dim3(kTokThreads), 0, st, p.h, p.tts, p.T, p.r, p); break;
+    default: hipLaunchKernelGGL((token_expand_vec_kernel<T, __bf16>), grid, dim3(kTokThreads), 0, st, p.h, p.tts, p.T, p.r, p); break;
   }
 }
 
@@ -480,6 +484,7 @@ extern "C" int mlora_shrink(const MloraShrinkArgs* a) {
     if (!a->a[i]) { set_error("mlora_shrink: NULL A pointer for slice %d", i); return MLORA_E_INVALID; }
     p.a[i] = a->a[i];
   }
+  if (group_shrink_supported(a)) return launch_group_shrink(a);
   dim3 grid(a->num_tokens, a->num_slices);
   hipStream_t st = static_cast<hipStream_t>(a->stream);
   bool vec = a->dtype != MLORA_DTYPE_F32 && a->k % 8 == 0 && a->x_stride % 8 == 0 && aligned16(a->x);
@@ -512,6 +517,7 @@ extern "C" int mlora_expand(const MloraExpandArgs* a) {
     n_max = a->n[i] > n_max ? a->n[i] : n_max;
   }
   if (n_max == 0) return 0;
+  if (group_expand_supported(a)) return launch_group_expand(a);
   p.nsplit = column_splits(n_max);
   dim3 grid(a->num_tokens, p.nsplit, a->num_slices);
   hipStream_t st = static_cast<hipStream_t>(a->stream);
