@@ -8,9 +8,10 @@
 // call only when everything the Python path would look up for it is what the Python path looked up
 // last time (the argument block of these weight buffers, the plan of this step's slot vector, the
 // scratch buffer of this stream), fills the per-step fields of the block and calls mlora_add_lora_active.
-// Everything else - a first call, another step, a capture in progress, anything that has to raise
-// - is answered with "not handled", and the Python path runs as if this module did not exist, then
-// tells it what it found (register_site, set_step, set_scratch).
+// One lookup it makes itself: the first call of a step whose slot vector carries a plan (take_step below).
+// Everything else - a first call of these buffers, a step without a plan, a capture in progress, anything
+// that has to raise - is answered with "not handled", and the Python path runs as if this module did not
+// exist, then tells it what it found (register_site, set_step, set_scratch).
 //
 // One state object per backend and thread; every function runs under the interpreter lock.
 #include <Python.h>
@@ -26,6 +27,7 @@
 #include <cstring>
 #include <string>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "mlora.h"
@@ -55,6 +57,7 @@ struct State {
   int num_slots = 0, active_slots = 0;
   int64_t rows = -1;
   const void* plan = nullptr;
+  PyObject* held[3] = {};  // metadata, slot vector and plan of a step that was taken here (set_step's are its caller's to hold)
   // the eager scratch buffer of a stream
   void* sc_stream = nullptr;
   int sc_device = -1;
@@ -65,6 +68,7 @@ struct State {
   long long handled = 0, passed_on = 0;  // calls enqueued here / left to the Python path
 
   ~State() {
+    for (PyObject* o : held) Py_XDECREF(o);
     for (auto& kv : sites) Py_XDECREF(kv.second.keep);
   }
 };
@@ -101,6 +105,13 @@ bool weights_key(PyObject* a_list, PyObject* b_list, Py_ssize_t n, std::string* 
 struct Ref {  // an owned reference, given back at the end of the scope
   PyObject* p;
   ~Ref() { Py_XDECREF(p); }
+};
+
+// Gives back, at the end of the scope, the objects of a step that stands no longer: the state is consistent by then.
+struct Released {
+  PyObject* p[3] = {};
+  explicit Released(State* s) { std::swap(p, s->held); }
+  ~Released() { for (PyObject* o : p) Py_XDECREF(o); }
 };
 
 bool on_device(const at::Tensor& t, int device) { return t.is_cuda() && t.device().index() == device; }
@@ -182,6 +193,7 @@ PyObject* py_set_step(PyObject*, PyObject* args) {
   if (!PyArg_ParseTuple(args, "OOOkKiLKi", &cap, &metadata, &source, &version, &stream, &num_slots, &rows, &plan, &active_slots)) return nullptr;
   State* s = state_of(cap);
   if (!s) return nullptr;
+  const Released before(s);
   s->metadata = metadata; s->source = source; s->version = static_cast<uint32_t>(version);
   s->stream = reinterpret_cast<void*>(static_cast<uintptr_t>(stream));
   s->num_slots = num_slots; s->rows = rows; s->active_slots = active_slots < 0 ? 0 : active_slots;
@@ -192,6 +204,7 @@ PyObject* py_set_step(PyObject*, PyObject* args) {
 PyObject* py_forget_step(PyObject*, PyObject* cap) {
   State* s = state_of(cap);
   if (!s) return nullptr;
+  const Released before(s);
   s->metadata = nullptr; s->source = nullptr; s->rows = -1; s->plan = nullptr;
   Py_RETURN_NONE;
 }
@@ -210,6 +223,45 @@ PyObject* py_set_scratch(PyObject*, PyObject* args) {
   s->sc_ptr = reinterpret_cast<void*>(static_cast<uintptr_t>(ptr));
   s->sc_bytes = bytes;
   Py_RETURN_NONE;
+}
+
+// What a Python object has been given under this name (its own attributes alone); nullptr without.  Borrowed.
+PyObject* given(PyObject* o, PyObject* name) {
+  PyObject** dict = _PyObject_GetDictPtr(o);
+  return dict && *dict ? PyDict_GetItem(*dict, name) : nullptr;
+}
+
+// The first call of a step: what the Python path looks up for it (HipLoRABackend._plan_for, known_active_slots), where
+// the metadata's own slot vector of exactly these rows carries the plan of the launch that made it
+// (segment_meta.attach_plan) and has not been rewritten since.  The state holds the three objects from then
+// on.  Eager calls only.  In Python this lookup cost 15 us of every step (passes back to back on one host: sixteen calls in
+// fp32 134 us, 119 with this; sixteen linears of 1234 tokens 500, 479).
+bool take_step(State* s, const Site& site, PyObject* metadata, PyObject* source_obj, const at::Tensor& source, uint32_t version, void* stream, int64_t rows) {
+  static PyObject* const kPlan = PyUnicode_InternFromString("_mlora_plan");
+  static PyObject* const kCapacity = PyUnicode_InternFromString("_mlora_capacity");
+  static PyObject* const kActiveIds = PyUnicode_InternFromString("active_slot_ids");
+  static PyObject* const kActive = PyUnicode_InternFromString("num_active_loras");
+  if (source.numel() != rows) return false;
+  PyObject* made = given(source_obj, kPlan);  // (workspace, max_slots, version)
+  if (!made || !PyTuple_Check(made) || PyTuple_GET_SIZE(made) != 3 || !THPVariable_Check(PyTuple_GET_ITEM(made, 0))) return false;
+  const at::Tensor& plan = THPVariable_Unpack(PyTuple_GET_ITEM(made, 0));
+  const long slots = PyLong_AsLong(PyTuple_GET_ITEM(made, 1));
+  const unsigned long at = PyLong_AsUnsignedLong(PyTuple_GET_ITEM(made, 2));
+  if (PyErr_Occurred() || slots != site.num_slots || at != version || !on_device(plan, site.device)) return false;
+  const Ref plan_held{(Py_INCREF(made), made)};  // (the attribute reads below can run Python code)
+  long active = 0;
+  const Ref ids{PyObject_GetAttr(metadata, kActiveIds)}, number{PyObject_GetAttr(metadata, kActive)};
+  PyErr_Clear();
+  PyObject* capacity = ids.p ? given(ids.p, kCapacity) : nullptr;
+  if (number.p && !(capacity && PyObject_IsTrue(capacity) == 1)) active = PyLong_AsLong(number.p);
+  if (PyErr_Occurred()) return false;
+  const Released before(s);
+  s->held[0] = metadata; s->held[1] = source_obj; s->held[2] = made;
+  for (PyObject* o : s->held) Py_INCREF(o);
+  s->metadata = metadata; s->source = source_obj; s->version = version; s->stream = stream;
+  s->num_slots = site.num_slots; s->rows = rows; s->plan = plan.data_ptr();
+  s->active_slots = active > 0 && active <= site.num_slots ? static_cast<int>(active) : 0;
+  return true;
 }
 
 // The call itself, at the site of its weight buffers.  Returns 0 (enqueued), a negative code of the library
@@ -263,9 +315,9 @@ long call_at(State* s, const Site& site, PyObject* x_obj, PyObject* target_obj, 
     if (capturing != hipStreamCaptureStatusNone) return kNotHandled;
     if (source.is_inference()) return kNotHandled;  // no version counter: nothing is remembered for them
     const uint32_t version = source._version();
-    if (s->metadata != metadata || s->source != source_obj || s->version != version || s->stream != stream || s->num_slots != site.num_slots ||
-        s->rows != rows || !s->plan)
-      return kNotHandled;
+    const bool known = s->metadata == metadata && s->source == source_obj && s->version == version && s->stream == stream &&
+                       s->num_slots == site.num_slots && s->rows == rows && s->plan;
+    if (!known && (tts.p == Py_None || !take_step(s, site, metadata, source_obj, source, version, stream, rows))) return kNotHandled;
     plan = s->plan;
     const uint64_t shape = (static_cast<uint64_t>(rows) << 24) | (static_cast<uint64_t>(site.num_slices) << 16) |
                            (static_cast<uint64_t>(site.rank) << 4) | static_cast<uint64_t>(site.dtype_code);

@@ -176,13 +176,13 @@ class _LoRALayerBase(nn.Module):
 
     # ---- the LoRA half of forward -------------------------------------------------------------
     def _add_lora_quickly(self, x: torch.Tensor, out: torch.Tensor) -> bool:
-        """The usual forward of a step whose first linear has been through ``_add_lora``: nothing about it is
-        new, and the C++ host path takes the layer's buffers as they are.  False, with nothing done,
-        for everything else (and whatever has to raise), which ``_add_lora`` then sees to."""
+        """The usual forward, about whose buffers nothing is new: the C++ host path takes them as the layer
+        holds them.  False, with nothing done, for everything else (and whatever has to raise), which
+        ``_add_lora`` then sees to."""
         context = installed_lora_context(self.lora_domain)
         if context is None or context.no_lora_flag or not self.supports_lora or not self._targets_in_order or x.dim() != 2:
             return False
-        metadata, slots, active = context._cached_metadata, context._slots, context.active_slot_ids
+        metadata, slots, active = context._cached_metadata or self._runtime_metadata(), context._slots, context.active_slot_ids
         if metadata is None or slots is None or metadata.token_to_slot is not slots or metadata.no_lora_flag or slots.size(0) != x.size(0):
             return False
         if active is not None and not active.is_cuda:
