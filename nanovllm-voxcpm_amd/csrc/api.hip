@@ -146,7 +146,7 @@ static bool small_batch(const MloraAddArgs* a, bool one_launch) {
 }
 
 // About how many 16-token tiles a batch has: its segments end anywhere inside their last tile.
-static int small_tiles_about(const MloraAddArgs* a, int active) {
+int mlora::small_tiles_about(const MloraAddArgs* a, int active) {
   const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
   const int tiles = static_cast<int>((a->num_tokens + 7ll * segs) / MLORA_TILE_SMALL);
   return tiles > segs ? tiles : segs;
@@ -158,15 +158,11 @@ static int small_tiles_about(const MloraAddArgs* a, int active) {
 // 327 KB each, 5.9 / 3.9 at 4 tokens, 5.6 / 5.2 at 64, 6.1 / 6.0 at 128, 6.7 / 6.8 at 256; o (64 KB per
 // slot) 3.5 / 3.4 at 4 tokens, 3.7 / 3.8 at 64, 3.8 / 4.1 at 256; over 8 slot ids it is the faster
 // grid at every batch size and every projection; with 128 slot ids of which 32 are in use it
-// takes 967 us per decode step against 629.  With K shared out between a tile's workgroups (down) it
-// is the faster one throughout (5.2 / 5.6 at 4 tokens, 6.4 / 6.8 at 256).  So: always with K parts;
-// else while all slots together weigh at most 3 MB, or when the batch has four tokens per slot id.
+// takes 967 us per decode step against 629.  With K shared out between a tile's workgroups the lines are others
+// (below).  So, without: while all slots together weigh at most 3 MB, or when the batch has four tokens per slot id.
 // All of this was measured on decode batches; on batches of many tiles per slot (a prefill of
 // 2098 tokens over 8 slot ids, o: 15.4 us per call against 10.1 tile-major) the grid over the slots
 // is the slower one: it is taken up to 32 tokens per slot id.
-// With K shared out the requests for unused slots end it too (down, us per call, slot-major / the best
-// other form): rank 16: 6.2 / 6.3 at 32 slot ids, 6.3 / 6.0 at 40, 8.0 / 6.2 at 64; rank 32: 8.7 / 9.6 at
-// 48, 10.8 / 10.6 at 64; rank 64: 12.0 / 12.6 at 48, 14.8 / 13.9 at 64.
 // `active` (when the caller knows it, else 0) is the number of slots with tokens.  Prompts are few long
 // segments: most of the grid is then workgroups without a tile, and the tiles behind a slot's first one learn
 // their slot from a record after all (rank 32, 37 tokens of one slot of 8: gate_up 7.4 / 4.9; 100 tokens
@@ -181,16 +177,27 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   // size (rank 48, one token per slot id, slot-major / pair: K = 8192 11.5 / 7.8 at 8 slot ids, 19.8 / 11.9 at 32; K = 4096
   // 7.4 / 7.5 and 9.8 / 9.7, four tokens per slot id 8.7 / 7.9 and 10.5 / 10.2).
   if (parts > 1 && a->r > 32 && !exact_rank(a->r)) return false;
-  // Eight parts (K = 8192) are twice the workgroups of a tile, slots without tokens have theirs too, and once they no
-  // longer fit the chip together they wait for each other.  K parts x tiles (or slot ids, where more), slot-major /
-  // pair, K = 8192 -> 2048, 2 to 64 slot ids: rank 16 up to 192: 4.6 / 6.1 to 7.2 / 7.6, at 256: 8.2 / 7.5; rank 8 at
-  // 184: 7.0 / 7.4, at 224 and 256: 9.9 / 7.8 and 9.3 / 6.9; rank 32 at 192: 7.5 / 7.8 and 8.7 / 8.5, at 224 and 256: 12.6 /
-  // 11.0 and 11.7 / 9.8; rank 24 like 32; rank 64 at 96 to 136: 8.9 / 9.4 to 10.8 / 11.3, at 128: 10.2 / 9.9, at 160: 11.2 / 10.8.
-  if (parts > 4) {
-    const int tiles = small_tiles_about(a, active);
-    return parts * (tiles > a->num_slots ? tiles : a->num_slots) <= (a->r > 32 ? 144 : 200);
+  if (parts > 1) {
+    // K shared out: the lines lie where the requests for slots without tokens, and at K = 8192 more workgroups than fit
+    // the chip together, cost what the second launch does.  us per call, slot-major / the best other form, at
+    // one and four tokens per slot id unless said:
+    const int tiles = small_tiles_about(a, active), slots = a->num_slots, rank = compute_rank(a->r);
+    const bool few = sparse || 2 * a->num_tokens <= slots;
+    // K = 2048: rank 64 8 slot ids 6.3 / 6.8, 32 8.0 / 10.4 and 8.6 / 11.4, 64 11.1 / 13.5; 8 tokens of 64 8.8 / 7.6.  Rank 32 16 ids
+    // 5.2 / 5.3, 48 6.2 / 7.0, 64 7.4 / 8.3; 8 tokens of 32 5.2 / 5.1, 37 of one slot of 8 5.3 / 5.2.  Rank 16 40 ids 4.6 / 4.5, 48 4.7 /
+    // 4.8, 64 5.3 / 5.4, 512 tokens of 32 (46 tiles) 5.2 / 5.2, 1000 (76) 6.2 / 7.6; rank 8 alike.
+    if (a->k == 2048) return rank <= 16 ? !few && tiles >= 48 : !(few && (rank == 32 || rank * slots >= 2048));
+    // K = 4096: 64 slot ids 5.1 / 5.7 at rank 8, 5.7 / 6.1, 8.7 / 10.3, 13.6 / 14.4 at rank 64; 8 tokens of 64 4.8 / 5.3, 5.3 / 5.4, 7.2 /
+    // 6.8, 11.7 / 7.9; 64 tokens of 4 slots of 32 4.6 / 4.7, 4.6 / 4.8, 5.6 / 5.7, 9.2 / 8.0.
+    if (a->k == 4096) return !(few && rank * slots >= 2048);
+    // K = 8192: rank 8 48 ids 8.7 / 9.3 and 9.4 / 15.0, 64 10.5 / 10.2 and 11.4 / 15.5, 64 tokens of 8 slots of 64 10.3 / 15.0.  Rank 16 64
+    // ids 9.2 / 9.9 and 10.1 / 11.1, 64 tokens of 4 slots of 32 6.0 / 6.9, 250 of 8 8.4 / 7.7.  Rank 32 40 ids 12.7 / 13.2, 48 13.4 / 12.1,
+    // 512 tokens of 32 (46 tiles) 11.3 / 13.1, 1000 (76) 17.5 / 16.9, 8 of 32 7.6 / 7.4.  Rank 64 32 ids 13.7 / 15.0, 40 20.2 / 20.0, 512
+    // tokens of 32 16.5 / 17.8, 2 of 16 9.3 / 9.2 (rank 32 6.0 / 7.2), 37 of one slot of 8 8.0 / 8.3.
+    if (few) return slots <= 8 || rank <= 8 || (rank <= 32 && slots <= 16) || (rank <= 16 && slots <= 32 && tiles <= 16);
+    if (rank <= 8) return slots <= 48 || a->num_tokens >= 2 * slots;
+    return rank <= 16 || (tiles <= 48 && slots <= (rank <= 32 ? 40 : 32));
   }
-  if (parts > 1) return a->num_slots <= (a->r <= 16 ? 32 : 48) && !(sparse && a->r * a->num_slots >= 2048);
   if (sparse || (active > 0 && a->num_tokens > MLORA_TILE_SMALL * active)) return false;
   double cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
@@ -373,7 +380,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "
-                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or (4096 and 8192) with one slice of at most 4096 columns and an "
+                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or (2048, 4096 and 8192) with one slice of at most 4096 columns and an "
                     "initialised workspace");
           return MLORA_E_UNSUPPORTED;
         }

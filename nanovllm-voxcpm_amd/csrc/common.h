@@ -258,33 +258,70 @@ __device__ __forceinline__ void count_rejected_plan(const int32_t* plan, bool he
 }
 
 // ---- workspace head (see MLORA_WORKSPACE_HEAD_BYTES in mlora.h) -------------------------------
-// uint32 words:  [0] signature | [1] waits that ran out (diagnostic) | ... ; at byte kWsTileOff the
-// {generation, arrivals} pair of the workspace (every workgroup of a split or one-launch
-// long-segment grid reports once when it is done, the last one advances the generation; the rest of
-// the 8 KiB behind it is reserved); at byte kWsXchgOff the exchange area of the split form: 64-bit
-// words {fp32 bits, tag}, valid when tag == generation + 1.  One generation for the whole
-// workspace: whatever an earlier launch left anywhere in the area, in whatever layout, carries a
-// tag below the current one.
+// uint32 words:  [0] signature | [1] waits that ran out (diagnostic) | ... ; eight states, one for the
+// workgroups of each blockIdx.x of the (8, y, z) grids that use the head: {generation, arrivals,
+// check word}, the first at byte kWsTileOff (the rest of the 8 KiB behind it is reserved), the others
+// 256 bytes apart from kWsStatesOff on; at byte kWsXchgOff the exchange area of the split form: 64-bit
+// words {fp32 bits, tag}, valid when tag == generation + 1.  Every launch takes every generation one step on,
+// so between launches they are the same, and whatever an earlier launch left anywhere in the area, in
+// whatever layout, carries a tag below the current one.
 constexpr uint32_t kWsMagic = 0x4d4c5733u;  // "MLW3"
-// Third word of the {generation, arrivals} pair: generation ^ kWsGenCheck, rewritten with every
-// advance of the generation.  A head is believed only if signature, this word and an arrival count
-// below the grid size all fit: memory that once was a workspace and was handed out again in between
-// can keep the signature while the pair holds something else, and a generation that never advances
-// would make the next launch accept what the last one left.
+// Third word of a state: generation ^ kWsGenCheck, rewritten with every advance of the generation.  A state
+// is believed only if the signature, this word and arrivals that a launch can have come to all fit: memory
+// that once was a workspace and was handed out again in between can keep the signature while the state
+// holds something else, and a generation that never advances would make the next launch accept what
+// the last one left.
 constexpr uint32_t kWsGenCheck = 0x9e3779b9u;
-__device__ __forceinline__ bool ws_state_ok(uint32_t signature, uint32_t generation, uint32_t arrivals, uint32_t check, uint32_t grid) {
-  return signature == kWsMagic && check == (generation ^ kWsGenCheck) && arrivals < grid;
-}
-constexpr int kWsTimeoutsWord = 1;
 constexpr int kWsTileOff = 256;
 constexpr int kWsTiles = 1024;
+constexpr int kWsStatesOff = kWsTileOff + 8 * kWsTiles;
+// How the generation advances.  Every workgroup of a launch reports once that it reads the exchange area no
+// more: it adds one to the arrivals, except the first one of its blockIdx.x (y = z = 0), which adds one to the
+// generation and takes the number of the others off the arrivals, in one 64-bit addition.  So until the last one
+// has reported the arrivals are positive (or 0) before the first one's report and negative behind it, and a
+// workgroup that starts late knows either way which generation its launch began with.  Nobody asks what an
+// addition found, and a counter is shared by an eighth of the grid: a returning count at one word, the last
+// arrival advancing the generation, kept a launch of 160 workgroups 1.9 us longer (11.5 ns each where all XCDs
+// meet), 64 workgroups 0.8.  K = 4096 -> 1024 shared out between four workgroups, 64 tokens of 32 slots, us per call
+// that way / this way: rank 16 5.8 / 4.8, rank 32 6.8 / 6.0, 192 tokens of 48 slots, rank 32, 8.7 / 7.1.
+// (Read as one 128-bit load, and the tests below without branches: sunk into the branches of a test the loads
+// become trips one behind the other.)
+typedef i32x4 WsState;  // generation, arrivals, check word, nothing
+__host__ __device__ inline int ws_state_word(int x) { return (x == 0 ? kWsTileOff : kWsStatesOff + 256 * x) / 4; }
+__device__ __forceinline__ WsState ws_state(const uint32_t* ws, int x) { return *reinterpret_cast<const i32x4*>(ws + ws_state_word(x)); }
+// (a tag, generation + 1, is never 0)
+__device__ __forceinline__ uint32_t ws_next(uint32_t generation) { return generation == 0xfffffffeu ? 0u : generation + 1u; }
+__device__ __forceinline__ uint32_t ws_previous(uint32_t generation) { return generation == 0u ? 0xfffffffeu : generation - 1u; }
+// the generation the launch began with
+__device__ __forceinline__ uint32_t ws_generation(const WsState& s) {
+  const uint32_t g = static_cast<uint32_t>(s[0]);
+  return s[1] >= 0 ? g : ws_previous(g);
+}
+__device__ __forceinline__ int ws_state_ok(uint32_t signature, const WsState& s) {
+  const uint32_t g = ws_generation(s), grid = gridDim.y * gridDim.z, arrivals = static_cast<uint32_t>(s[1] < 0 ? -s[1] : s[1]);
+  const uint32_t c = static_cast<uint32_t>(s[2]) ^ kWsGenCheck;  // (stored beside the addition: one step early or late)
+  return int(signature == kWsMagic) & int(arrivals < grid) & (int(c == g) | int(c == ws_next(g)) | int(c == ws_previous(g)));
+}
+// One thread of every workgroup, once; `generation` is what ws_generation said.
+__device__ __forceinline__ void ws_report(uint32_t* ws, uint32_t generation) {
+  uint32_t* const s = ws + ws_state_word(blockIdx.x);
+  unsigned long long add = 1ull << 32;
+  if (blockIdx.y == 0 && blockIdx.z == 0) {
+    const uint32_t next = ws_next(generation), others = gridDim.y * gridDim.z - 1u;
+    // (the generation's step modulo 2^32, less the carry it makes when it goes back to 0)
+    add = static_cast<unsigned long long>(next - generation) - (static_cast<unsigned long long>(others + (next < generation ? 1u : 0u)) << 32);
+    __hip_atomic_store(s + 2, next ^ kWsGenCheck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  (void)__hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(s), add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+constexpr int kWsTimeoutsWord = 1;
 constexpr int kWsXchgOff = 16384;
 constexpr int kWsXchgBytes = 4 << 20;
 // behind the exchange area: one 64-bit seal per (unit, shrink role) of the one-launch
 // long-segment form: {generation of the unit + 1, XCD of the writer}
 constexpr int kWsSealBytes = 64 << 10;
 constexpr int kWsSealOff = kWsXchgOff + kWsXchgBytes;
-static_assert(kWsTileOff + 8 * kWsTiles <= kWsXchgOff, "tile state overlaps the exchange area");
+static_assert(kWsStatesOff + 256 * 8 <= kWsXchgOff, "tile state overlaps the exchange area");
 static_assert(kWsSealOff + kWsSealBytes == MLORA_WORKSPACE_HEAD_BYTES, "head size");
 
 // The XCD (accelerator die) this wavefront runs on: bits 3:0 of hardware register XCC_ID (id 20).

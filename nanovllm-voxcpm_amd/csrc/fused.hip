@@ -117,11 +117,10 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
   for (int g = 0; g < G; ++g) big[g] = reinterpret_cast<const i32x4*>(plan + big_off)[is_big ? unit * G + g : 0];
   const ExpandSplit sp = splits.split[c];
   const uint32_t signature = ws[0];
-  // {generation, arrivals} of the workspace: one pair for the whole launch, so that every seal any
-  // earlier launch left anywhere (whatever its layout was) carries a tag below this launch's
-  uint32_t* const ustate = ws + kWsTileOff / 4;
-  const uint32_t tag = ustate[0] + 1u;
-  const uint32_t arrivals0 = ustate[1], gen_check = ustate[2];
+  // the workspace's state: every seal any earlier launch left anywhere (whatever its layout was)
+  // carries a tag below this launch's
+  const WsState state = ws_state(ws, blockIdx.x);
+  const uint32_t generation = ws_generation(state), tag = generation + 1u;
   const int n_short = hdr1[MLORA_PLAN_TILES_SHORT - 4];
   int slot[G], start[G], m[G], any = 0;
 #pragma unroll
@@ -148,24 +147,16 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
   const int usable = int(hdr0[MLORA_PLAN_MAGIC] == MLORA_PLAN_MAGIC_VALUE) & int(hdr0[MLORA_PLAN_NUM_TOKENS] == T_) &
                      int(hdr0[MLORA_PLAN_MAX_SLOTS] == num_slots) & int(any > 0);
   // seals and generations can be used: the head is in the state a launch (or the initialisation) left it in
-  const bool xok = trusted | ws_state_ok(signature, tag - 1u, arrivals0, gen_check, gridDim.x * gridDim.y * gridDim.z);
-  // every workgroup of the grid reports exactly once that it is done (also the ones without work);
-  // the last one advances the generation, which makes every seal of this launch stale
-  auto count_done = [&]() {
-    if (xok && tid == 0) {
-      const uint32_t before = __hip_atomic_fetch_add(ustate + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (before + 1u == gridDim.x * gridDim.y * gridDim.z) {
-        const uint32_t next = tag == 0xffffffffu ? 0u : tag;  // generation + 1, the next tag, is never 0
-        __hip_atomic_store(ustate + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ustate + 2, next ^ kWsGenCheck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ustate, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
+  const bool xok = trusted | ws_state_ok(signature, state);
+  // every workgroup of the grid reports exactly once that it is done (also the ones without work),
+  // which advances the generation and so makes every seal of this launch stale
+  auto report = [&]() {
+    if (xok && tid == 0) ws_report(ws, generation);
   };
   if (!usable) {
     count_rejected_plan(plan, hdr0[MLORA_PLAN_MAGIC] == MLORA_PLAN_MAGIC_VALUE && hdr0[MLORA_PLAN_NUM_TOKENS] == T_ &&
                                   hdr0[MLORA_PLAN_MAX_SLOTS] == num_slots);
-    count_done();
+    report();
     return;
   }
   MLORA_STAMP(1);  // records, ranks and generation are here
@@ -256,7 +247,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
   fused_expand<T, R, CPL, TPF, G>(s_h, s_row, s_slot, s_m, s_eff, s_start, plan, hws, yv_, ys, sorted_off, T_, num_slices, ksplit, scaling, sp);
 
   MLORA_STAMP(13);  // expanded (wavefront 0)
-  count_done();
+  report();
 }
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().

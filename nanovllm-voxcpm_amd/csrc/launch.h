@@ -38,6 +38,7 @@ int decode_ranges(const MloraAddArgs* a, int* columns);  // column ranges of tha
 bool slot_supported(const MloraAddArgs* a);
 int slot_k_parts(const MloraAddArgs* a);  // 4 or 8 when the workgroups of a tile would share K out, else 1
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace);
+int small_tiles_about(const MloraAddArgs* a, int active);  // 16-token tiles of a batch (api.hip)
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.
 // trusted_workspace: the head of the workspace is known to be in its initial or a left-behind

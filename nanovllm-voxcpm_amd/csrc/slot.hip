@@ -25,7 +25,7 @@
 // (z beyond the slot layers), which learn their slot from their record like the tile-major
 // kernel: a batch with every token on one adapter spreads over as many workgroups as before.
 //
-// Long K (KP > 1; KP = 8 at K = 8192).  What a compute unit can take in per unit of time is what bounds a decode
+// Long K (KP > 1: four or eight parts of 512 or 1024 columns).  What a compute unit can take in per unit of time is what bounds a decode
 // launch (about 35 bytes per cycle, whether the lines come from HBM or from the L2), and with one
 // workgroup per column range every range pulls ALL of x's tile and of A[slot]: at K = 4096 that is
 // 256 KB per workgroup against 16 KB of B and y.  With KP > 1 the KP workgroups of a tile each take
@@ -33,8 +33,8 @@
 // sums as tagged 64-bit words in the workspace's exchange area, picks up the other parts'
 // words, adds all parts in part order (so every workgroup of the tile holds the same bits) and
 // expands its columns.  The hand-over follows the protocol of split.hip: words are valid when
-// their tag is the workspace's generation + 1, every workgroup of the grid counts itself once,
-// the last one advances the generation, nothing is ever cleared.  Waiting is bounded: a workgroup
+// their tag is the workspace's generation + 1, every workgroup of the grid reports once, which
+// advances the generation, nothing is ever cleared.  Waiting is bounded: a workgroup
 // whose partners' words are not there in time multiplies their parts itself, in their order.
 #include "common.h"
 #include "launch.h"
@@ -43,7 +43,7 @@ namespace mlora {
 
 namespace {
 
-constexpr int kNW = 8;  // wavefronts per workgroup
+constexpr int kNW = 8;  // wavefronts per workgroup (NW: of those that share K out in parts of 512 columns, four)
 
 MLORA_TRACE_DECL
 
@@ -71,7 +71,7 @@ typedef unsigned long long u64;
 // GR (with MASKED): the buffers' rank is `rbuf` < R, a multiple of eight: rows of A[slot] are rbuf * K
 // apart and B rows rbuf elements long; whatever lies beyond rbuf is treated like the ranks beyond
 // an adapter's own (requests clamped into the buffers, values masked).
-template <typename T, int R, int KSPW, int KP, bool MASKED, bool GR, int SA, bool EARLY>
+template <typename T, int NW, int R, int KSPW, int KP, bool MASKED, bool GR, int SA, bool EARLY>
 __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const int slot_early, const int early_ok, const int rbuf_arg, const Range sp,
                                           const int y_col0, const int y_col1, const int y_col2, const int slice, const void* __restrict__ xv,
                                           void* __restrict__ yv_, const int64_t xs, const int64_t ys,
@@ -81,9 +81,9 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   constexpr int RB = (R + 15) / 16;      // 16-rank blocks of the shrink output
   constexpr int KSTEPS = (R + 31) / 32;  // MFMA k-steps of the expand
   constexpr int HSTRIDE = R + 8;         // padded LDS row of the intermediate
-  constexpr int NT = kNW * kWave;
+  constexpr int NT = NW * kWave;
   constexpr int ROUNDS = KSPW / 4;       // groups of four k-steps per wavefront
-  constexpr int KPART = 32 * kNW * KSPW;  // columns of x and A one workgroup multiplies
+  constexpr int KPART = 32 * NW * KSPW;  // columns of x and A one workgroup multiplies
   constexpr int K = KPART * KP;           // row length of A[slot]
   constexpr int WORDS = RB * 256;         // partial sums of one (tile, K part), in the order of the shared sum below
   constexpr int EPT = (WORDS + NT - 1) / NT;  // of which a thread holds this many
@@ -111,14 +111,13 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
 
   const int kp = KP > 1 ? static_cast<int>(blockIdx.y) : 0;  // this workgroup's K part (and column range)
   const int ks0 = kp * (KPART / 32) + wave * KSPW;
-  // the workspace's {generation, arrivals, check word} and signature (KP > 1): requested with the record
-  uint32_t* const tstate = KP > 1 ? xc.ws + kWsTileOff / 4 : nullptr;
-  uint32_t signature = 0, generation = 0, arrivals0 = 0, gen_check = 0;
+  // the workspace's state and signature (KP > 1): requested with the record (requested behind the A rows, or behind
+  // the record, they cost up to 0.7 us more: 64 tokens of 32 slots, K = 2048, rank 64 masked 8.4 / 9.2 / 9.1 us per call)
+  uint32_t signature = 0;
+  WsState state = {0, 0, 0, 0};
   if constexpr (KP > 1) {
     signature = xc.ws[0];
-    generation = tstate[0];
-    arrivals0 = tstate[1];
-    gen_check = tstate[2];
+    state = ws_state(xc.ws, blockIdx.x);
   }
   i32x4 ast[RB][4 * ROUNDS];
   Pack8 bop[SA][4][KSTEPS];
@@ -144,7 +143,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
     const T* B = static_cast<const T*>(sp.b) + static_cast<int64_t>(slot) * sp.n * rbuf;
 #pragma unroll
     for (int s = 0; s < SA; ++s) {
-      const int c0 = sp.n0 + (wave + s * kNW) * 64;
+      const int c0 = sp.n0 + (wave + s * NW) * 64;
       // requested whether the span exists or not (addresses clamped into the range)
       if constexpr (K16) {
         // a span's 64 B rows of 32 bytes are 2 KB of contiguous memory: fetched as such
@@ -193,35 +192,17 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
                      int(__builtin_amdgcn_readfirstlane(rows4[0]) >= 0) & int(rec0[2] >= 0) & int(!EARLY || rec0[0] == slot_early);
   // KP > 1: the exchange area can be used when the head is in the state a launch (or the
   // initialisation) left it in.  Every workgroup of the grid, with or without work, reports once
-  // that it reads the area no more; the last one advances the generation.
-  const uint32_t tag = generation + 1u;
-  const bool xok = KP > 1 && (xc.trusted | ws_state_ok(signature, generation, arrivals0, gen_check, gridDim.x * gridDim.y * gridDim.z));
-  // The count comes back from the memory system long after it was sent: a working workgroup sends
-  // it behind its last barrier (count_sent, by the last wavefront, which has the fewest spans to
-  // expand) and looks at what came back when its stores are out (count_seen).
-  const bool counter = KP > 1 && xok && tid == NT - kWave;
-  uint32_t arrivals_before = 0;
-  auto count_sent = [&]() {
+  // that it reads the area no more.
+  const uint32_t generation = ws_generation(state), tag = generation + 1u;
+  const bool xok = KP > 1 && (xc.trusted | ws_state_ok(signature, state));
+  // (by the last wavefront, which has the fewest spans to expand)
+  auto report = [&]() {
     if constexpr (KP > 1) {
-      if (counter) arrivals_before = __hip_atomic_fetch_add(tstate + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (xok && tid == NT - kWave) ws_report(xc.ws, generation);
     }
-  };
-  auto count_seen = [&]() {
-    if constexpr (KP > 1) {
-      if (counter && arrivals_before + 1u == gridDim.x * gridDim.y * gridDim.z) {
-        const uint32_t next = tag == 0xffffffffu ? 0u : tag;  // so that generation + 1, the next tag, is never 0
-        __hip_atomic_store(tstate + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(tstate + 2, next ^ kWsGenCheck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(tstate, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  };
-  auto count_done = [&]() {
-    count_sent();
-    count_seen();
   };
   if (!usable) {
-    count_done();
+    report();
     // a plan that was built for another batch shape (or never built): count the launch that found
     // it so, once (the first workgroup's record exists in every plan)
     if (!matches && EARLY && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid == 0 && plan_hdr)
@@ -244,7 +225,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
     }
     if (GR && eff > rbuf) eff = rbuf;
     if (eff == 0) {
-      count_done();
+      report();
       if constexpr (EARLY) settle_requests();
       return;
     }
@@ -271,7 +252,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
     for (int i = 0; i < 4; ++i) yy[i] = *reinterpret_cast<const uint2*>(ycols + static_cast<int64_t>(rows4[i]) * ys + c);
   };
 #pragma unroll
-  for (int s = 0; s < SA; ++s) request_y(sp.n0 + (wave + s * kNW) * 64, yq[s]);
+  for (int s = 0; s < SA; ++s) request_y(sp.n0 + (wave + s * NW) * 64, yq[s]);
   MLORA_STAMP(2);  // every load is issued
 
   // ---- shrink: H[token, rank] partial over this wavefront's K range ----------------------------
@@ -330,7 +311,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
       if (WORDS % NT == 0 || e < WORDS) {
         const int rb = e >> 8, ln = (e & 255) >> 2, i = e & 3;
 #pragma unroll
-        for (int w = 0; w < kNW; ++w) sum += s_red[((w * RB + rb) * 64 + ln) * 4 + i];
+        for (int w = 0; w < NW; ++w) sum += s_red[((w * RB + rb) * 64 + ln) * 4 + i];
       }
       out[j] = sum;
     }
@@ -457,10 +438,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   }
   __syncthreads();
   MLORA_STAMP(5);  // the intermediate is in LDS
-  // This workgroup reads the exchange area no more.  Sent behind the last barrier: the compiler
-  // waits for the count on the spot (it is requested inside a branch), and in front of a barrier
-  // the whole workgroup would wait with the wavefront that sent it.
-  count_sent();
+  report();  // this workgroup reads the exchange area no more
 
   // ---- expand: tokens as MFMA rows, lane holds out[token 4 * lg + i][column c0 + 4 * lr + j] ----
   Pack8 hop[KSTEPS], hlo[KSTEPS];
@@ -540,11 +518,10 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   };
 #pragma unroll
   for (int s = 0; s < SA; ++s) {
-    const int c0 = sp.n0 + (wave + s * kNW) * 64;
+    const int c0 = sp.n0 + (wave + s * NW) * 64;
     if (c0 < sp.n1) finish_span(c0, bop[s], yq[s]);
   }
   MLORA_STAMP(6);
-  count_seen();
 #ifdef MLORA_TRACE
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   MLORA_STAMP(7);
@@ -557,8 +534,8 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
 // early requests need.  packed = columns per range / 64 | ranges of slice 0 << 8 | slots << 16.
 // A launch of one slice passes n1 = 0 (blockIdx.y never reaches a second slice).
 // KP > 1: one slice, blockIdx.y is the workgroup's K part and column range alike (ranges of slice 0 = KP).
-template <typename T, int R, int KSPW, int KP, bool MASKED, bool GR, int SA>
-__global__ __launch_bounds__(kNW* kWave) void slot_kernel(const int32_t* __restrict__ recs, const void* __restrict__ a0,
+template <typename T, int NW, int R, int KSPW, int KP, bool MASKED, bool GR, int SA>
+__global__ __launch_bounds__(NW* kWave) void slot_kernel(const int32_t* __restrict__ recs, const void* __restrict__ a0,
                                                           const void* __restrict__ b0, const void* __restrict__ a1,
                                                           const void* __restrict__ b1, int n0, int n1, uint32_t packed, int rbuf,
                                                           const void* __restrict__ xv, void* __restrict__ yv_, int64_t xs, int64_t ys,
@@ -569,10 +546,10 @@ __global__ __launch_bounds__(kNW* kWave) void slot_kernel(const int32_t* __restr
   constexpr int HSTRIDE = R + 8;
   constexpr int kStageRow = 17;
   constexpr int SB = RB < 2 ? RB : 2;
-  __shared__ __attribute__((aligned(16))) float s_red[kNW * RB * 64 * 4];
+  __shared__ __attribute__((aligned(16))) float s_red[NW * RB * 64 * 4];
   __shared__ __attribute__((aligned(16))) T s_hi[16 * HSTRIDE];
   __shared__ __attribute__((aligned(16))) T s_lo[16 * HSTRIDE];
-  __shared__ __attribute__((aligned(16))) i32x4 s_stage[kNW * (1 + SB) * 16 * kStageRow];
+  __shared__ __attribute__((aligned(16))) i32x4 s_stage[NW * (1 + SB) * 16 * kStageRow];
   __shared__ int s_ok;
   MLORA_STAMP(0);
 
@@ -595,11 +572,11 @@ __global__ __launch_bounds__(kNW* kWave) void slot_kernel(const int32_t* __restr
   if (static_cast<int>(blockIdx.z) < zslots) {
     const int s = blockIdx.z * 8 + blockIdx.x;  // its record exists: the list is rounded up to eight
     const int slot = s < num_slots ? s : num_slots - 1;
-    slot_tile<T, R, KSPW, KP, MASKED, GR, SA, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), rbuf, sp, y_col0, y_col1, 0, int(second), xv, yv_,
+    slot_tile<T, NW, R, KSPW, KP, MASKED, GR, SA, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), rbuf, sp, y_col0, y_col1, 0, int(second), xv, yv_,
                                                 xs, ys, num_slots, scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   } else {
     const int q = zslots * 8 + (blockIdx.z - zslots) * 8 + blockIdx.x;
-    slot_tile<T, R, KSPW, KP, MASKED, GR, SA, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, rbuf, sp, y_col0, y_col1, 0, int(second), xv, yv_, xs, ys, num_slots,
+    slot_tile<T, NW, R, KSPW, KP, MASKED, GR, SA, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, rbuf, sp, y_col0, y_col1, 0, int(second), xv, yv_, xs, ys, num_slots,
                                                  scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   }
 }
@@ -649,14 +626,17 @@ __global__ __launch_bounds__(kNW* kWave) void slot_kernel3(const int32_t* __rest
   if (static_cast<int>(blockIdx.z) < zslots) {
     const int s = blockIdx.z * 8 + blockIdx.x;
     const int slot = s < num_slots ? s : num_slots - 1;
-    slot_tile<T, R, 4, 1, MASKED, false, 1, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), R, sp, y_col0, y_col1, y_col2, slice, xv,
+    slot_tile<T, kNW, R, 4, 1, MASKED, false, 1, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), R, sp, y_col0, y_col1, y_col2, slice, xv,
                                                   yv_, xs, ys, num_slots, scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   } else {
     const int q = zslots * 8 + (blockIdx.z - zslots) * 8 + blockIdx.x;
-    slot_tile<T, R, 4, 1, MASKED, false, 1, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, R, sp, y_col0, y_col1, y_col2, slice, xv, yv_, xs, ys,
+    slot_tile<T, kNW, R, 4, 1, MASKED, false, 1, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, R, sp, y_col0, y_col1, y_col2, slice, xv, yv_, xs, ys,
                                                    num_slots, scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   }
 }
+
+// How a tile's K is shared out: between kp workgroups of nw wavefronts.
+struct Parts { int kp, nw; };
 
 struct Launch {
   const MloraAddArgs* a;
@@ -703,67 +683,65 @@ void launch_three(const MloraAddArgs* a, dim3 grid, int nt, int cum1, int cum2) 
                        const_cast<int32_t*>(a->plan));
 }
 
-template <typename T, int R, int KSPW, int KP, bool MASKED, bool GR, int SA>
+template <typename T, int NW, int R, int KSPW, int KP, bool MASKED, bool GR, int SA>
 void launch_spans(const Launch& l) {
   const MloraAddArgs* a = l.a;
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   const MloraSlice& s0 = a->slices[0];
   const MloraSlice s1 = a->num_slices > 1 ? a->slices[1] : MloraSlice{nullptr, nullptr, 0, 0};
-  hipLaunchKernelGGL((slot_kernel<T, R, KSPW, KP, MASKED, GR, SA>), l.grid, dim3(kNW * kWave), 0, static_cast<hipStream_t>(a->stream),
+  hipLaunchKernelGGL((slot_kernel<T, NW, R, KSPW, KP, MASKED, GR, SA>), l.grid, dim3(NW * kWave), 0, static_cast<hipStream_t>(a->stream),
                      a->plan + lay.slotrec_off, s0.a, s0.b, s1.a, s1.b, s0.n, s1.n, l.packed, a->r, a->x, a->y, a->x_stride, a->y_stride,
                      s0.y_col, s1.y_col, static_cast<uint32_t>(MLORA_PLAN_CHECK(a->num_tokens, a->num_slots)), a->scaling,
                      a->effective_rank, const_cast<int32_t*>(a->plan), static_cast<uint32_t*>(a->workspace), l.spin_ticks, l.trusted);
 }
 
-template <typename T, int R, int KSPW, int KP>
+template <typename T, int NW, int R, int KSPW, int KP>
 void launch_one(const Launch& l) {
-  const bool one_span = KP == 8 || l.widest <= kNW * 64;
-  constexpr int kTwo = KP == 8 ? 1 : 2;  // (ranges of two spans are not cut into eight parts)
+  constexpr bool kOne = NW == 8 && KP == 8;  // (eight wavefronts: ranges of two spans are not cut into eight parts)
+  const bool one_span = kOne || l.widest <= NW * 64;
+  constexpr int kTwo = kOne ? 1 : 2;
   if constexpr (R >= 32) {
     if (l.a->r != R) {  // buffers of a rank between the instances': the masked code with the buffers' rank as stride
-      if (one_span) launch_spans<T, R, KSPW, KP, true, true, 1>(l);
-      else launch_spans<T, R, KSPW, KP, true, true, kTwo>(l);
+      if (one_span) launch_spans<T, NW, R, KSPW, KP, true, true, 1>(l);
+      else launch_spans<T, NW, R, KSPW, KP, true, true, kTwo>(l);
       return;
     }
   }
   if (l.a->effective_rank) {
-    if (one_span) launch_spans<T, R, KSPW, KP, true, false, 1>(l);
-    else launch_spans<T, R, KSPW, KP, true, false, kTwo>(l);
+    if (one_span) launch_spans<T, NW, R, KSPW, KP, true, false, 1>(l);
+    else launch_spans<T, NW, R, KSPW, KP, true, false, kTwo>(l);
   } else {
-    if (one_span) launch_spans<T, R, KSPW, KP, false, false, 1>(l);
-    else launch_spans<T, R, KSPW, KP, false, false, kTwo>(l);
+    if (one_span) launch_spans<T, NW, R, KSPW, KP, false, false, 1>(l);
+    else launch_spans<T, NW, R, KSPW, KP, false, false, kTwo>(l);
   }
 }
 
-// kp: K parts (1: every workgroup multiplies the whole of K).
+template <typename T, int NW, int KSPW, int KP>
+bool launch_ranks(const Launch& l, int r) {
+  switch (r) {
+    case 8: launch_one<T, NW, 8, KSPW, KP>(l); return true;
+    case 16: launch_one<T, NW, 16, KSPW, KP>(l); return true;
+    case 32: launch_one<T, NW, 32, KSPW, KP>(l); return true;
+    case 64: launch_one<T, NW, 64, KSPW, KP>(l); return true;
+  }
+  return false;
+}
+
+// parts: of K (one: every workgroup multiplies the whole of it).
 template <typename T>
-bool launch_rank(const Launch& l, int rank, int kspw, int kp) {
-  const int r = compute_rank(rank);
-  if (kspw == 4 && kp == 1) {
+bool launch_rank(const Launch& l, int rank, int k, Parts parts) {
+  const int r = compute_rank(rank), each = k / parts.kp;
+  if (parts.nw == 4 && each == 512) {
+    if (parts.kp == 4) return launch_ranks<T, 4, 4, 4>(l, r);
+    if (parts.kp == 8) return launch_ranks<T, 4, 4, 8>(l, r);
+  } else if (parts.nw == kNW && each == 1024) {
+    if (parts.kp == 1) return launch_ranks<T, kNW, 4, 1>(l, r);
+    if (parts.kp == 4) return launch_ranks<T, kNW, 4, 4>(l, r);
+    if (parts.kp == 8) return launch_ranks<T, kNW, 4, 8>(l, r);
+  } else if (parts.nw == kNW && each == 4096 && parts.kp == 1) {
     switch (r) {
-      case 8: launch_one<T, 8, 4, 1>(l); return true;
-      case 16: launch_one<T, 16, 4, 1>(l); return true;
-      case 32: launch_one<T, 32, 4, 1>(l); return true;
-      case 64: launch_one<T, 64, 4, 1>(l); return true;
-    }
-  } else if (kspw == 4 && kp == 4) {
-    switch (r) {
-      case 8: launch_one<T, 8, 4, 4>(l); return true;
-      case 16: launch_one<T, 16, 4, 4>(l); return true;
-      case 32: launch_one<T, 32, 4, 4>(l); return true;
-      case 64: launch_one<T, 64, 4, 4>(l); return true;
-    }
-  } else if (kspw == 4 && kp == 8) {
-    switch (r) {
-      case 8: launch_one<T, 8, 4, 8>(l); return true;
-      case 16: launch_one<T, 16, 4, 8>(l); return true;
-      case 32: launch_one<T, 32, 4, 8>(l); return true;
-      case 64: launch_one<T, 64, 4, 8>(l); return true;
-    }
-  } else if (kspw == 16 && kp == 1) {
-    switch (r) {
-      case 8: launch_one<T, 8, 16, 1>(l); return true;
-      case 16: launch_one<T, 16, 16, 1>(l); return true;
+      case 8: launch_one<T, kNW, 8, 16, 1>(l); return true;
+      case 16: launch_one<T, kNW, 16, 16, 1>(l); return true;
     }
   }
   return false;
@@ -797,7 +775,7 @@ struct SlotKnobs {
   int generation = -1, kparts, spin_ticks;
   void read() {
     generation = knob_generation();
-    kparts = env_int("MLORA_SLOT_KPARTS", 4);          // 1: never share K out between workgroups
+    kparts = env_int("MLORA_SLOT_KPARTS", 0);          // 1: never share K out between workgroups
     spin_ticks = env_int("MLORA_SLOT_SPIN_TICKS", 20000);  // 200 us; 0: do not wait; < 0: never accept a partner's words
   }
 };
@@ -807,28 +785,39 @@ SlotKnobs& slot_knobs() {
   return k;
 }
 
-// K parts of a launch: of 1024 columns each for K = 4096 and 8192 when the tile's workgroups can hand each
-// other partial sums (one slice of at most 1024 columns per part, a workspace whose exchange area holds every
-// tile's parts), else one.  Eight parts at K = 8192 against the shrink and expand launches (pair.hip): one token,
-// rank 32, 8 slot ids 7.2 -> 5.4 us per call, 16 tokens, rank 16, 16 ids 7.1 -> 5.7.
-int k_parts(const MloraAddArgs* a) {
-  if ((a->k != 4096 && a->k != 8192) || a->num_slices != 1 || slot_knobs().kparts == 1) return 1;
-  const int kp = a->k / 1024;
-  if (a->slices[0].n > kp * 1024 || a->slices[0].n < kp * 64) return 1;
-  if ((kp - 1) * (((a->slices[0].n + kp - 1) / kp + 63) & ~63) >= a->slices[0].n) return 1;  // (a part without columns would leave the tile)
-  if (kp == 8 && a->slices[0].n > kp * 512) return 1;   // (instances of one span per wavefront only)
-  if (a->r > 32 && a->slices[0].n > kp * 512) return 1;  // (two spans per wavefront at rank 64 do not fit the registers beside the parts)
-  if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return 1;
+// Whether a tile's workgroups can hand each other the partial sums of these parts: columns for every part, an
+// instance for their ranges, an exchange area that holds every tile's.
+bool parts_fit(const MloraAddArgs* a, Parts p) {
+  const int n = a->slices[0].n, nt = ((n + p.kp - 1) / p.kp + 63) & ~63;
+  if (n < p.kp * 64 || (p.kp - 1) * nt >= n) return false;  // (a part without columns would leave the tile)
+  const int spans = (nt + 64 * p.nw - 1) / (64 * p.nw);
+  if (spans > 2 || (spans == 2 && p.nw == kNW && (p.kp == 8 || a->r > 32))) return false;  // (instances; registers beside the parts)
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
-  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * kp * ((compute_rank(a->r) + 15) / 16) * 256;
-  if (words * 8 > kWsXchgBytes) return 1;
-  return kp;
+  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * p.kp * ((compute_rank(a->r) + 15) / 16) * 256;
+  return words * 8 <= kWsXchgBytes;
+}
+
+// K parts of a launch (one slice, an initialised workspace), else one.  Of 1024 columns for eight wavefronts or of
+// 512 for four: smaller parts take in less per compute unit, and there are twice as many workgroups that wait
+// for each other, so K = 4096 is cut into eight while parts x tiles (or slot ids) are few (us per call in four parts / in
+// eight: rank 16, 16 slot ids 4.7 / 4.4, 32 4.8 / 4.6, 40 4.9 / 5.0, 64 5.7 / 5.8; rank 32, 16 5.3 / 4.9, 24 5.5 / 5.4, 32 6.0 / 6.0, 40
+// 6.3 / 7.8; rank 64, 16 7.5 / 7.1, 24 8.5 / 8.2, 32 9.2 / 10.5; 250 tokens of 8 slots of 32, rank 32 6.4 / 7.3).
+// K = 2048 in four, 8192 in eight of 1024.
+Parts k_parts(const MloraAddArgs* a) {
+  const Parts one = {1, kNW};
+  if (a->num_slices != 1 || slot_knobs().kparts == 1) return one;
+  if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return one;
+  const Parts small = {a->k / 512, 4}, large = {a->k / 1024, kNW};
+  const int tiles = small_tiles_about(a, 0), most = tiles > a->num_slots ? tiles : a->num_slots;
+  if ((a->k == 2048 || (a->k == 4096 && 8 * most <= (a->r <= 16 ? 256 : 192))) && parts_fit(a, small)) return small;
+  if ((a->k == 4096 || a->k == 8192) && parts_fit(a, large)) return large;
+  return one;
 }
 
 }  // namespace
 
-// K = 1024 at every rank; K = 4096 at every rank with the K parts of a tile shared out between its
-// workgroups, else up to rank 16 (what fits the register file as one batch of loads); one or two
+// K = 1024 at every rank; K = 2048, 4096 and 8192 at every rank with the K parts of a tile shared out between its
+// workgroups, K = 4096 without up to rank 16 (what fits the register file as one batch of loads); one or two
 // slices with their pointers as arguments, three (K = 1024) with the later two's as offsets from
 // the first one's; 16-bit elements.
 bool slot_supported(const MloraAddArgs* a) {
@@ -852,12 +841,10 @@ bool slot_supported(const MloraAddArgs* a) {
     return range_columns(a) <= kNW * 64;
   }
   if (kspw == 4) return true;
-  if (kspw == 16) return a->r <= 16 || k_parts(a) == 4;
-  if (kspw == 32) return k_parts(a) == 8;
-  return false;
+  return k_parts(a).kp > 1 || (kspw == 16 && a->r <= 16);
 }
 
-int slot_k_parts(const MloraAddArgs* a) { return k_parts(a); }
+int slot_k_parts(const MloraAddArgs* a) { return k_parts(a).kp; }
 
 void slot_trace_set(void* buf) {
 #ifdef MLORA_TRACE
@@ -869,7 +856,8 @@ void slot_trace_set(void* buf) {
 
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace) {
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
-  const int kp = k_parts(a);
+  const Parts parts = k_parts(a);
+  const int kp = parts.kp;
   // with K parts the tile's workgroups are its K parts and its column ranges alike
   const int nt = kp > 1 ? ((a->slices[0].n + kp - 1) / kp + 63) & ~63 : range_columns(a);
   const int ranges0 = kp > 1 ? kp : (a->slices[0].n + nt - 1) / nt;
@@ -906,8 +894,7 @@ int launch_slot(const MloraAddArgs* a, bool trusted_workspace) {
     }
     return check_launch("mlora_add_lora(small tiles, one workgroup per slot and column range, three slices)");
   }
-  const int kspw = kspw_of(a) / kp;
-  const bool ok = a->dtype == MLORA_DTYPE_BF16 ? launch_rank<__bf16>(l, a->r, kspw, kp) : launch_rank<_Float16>(l, a->r, kspw, kp);
+  const bool ok = a->dtype == MLORA_DTYPE_BF16 ? launch_rank<__bf16>(l, a->r, a->k, parts) : launch_rank<_Float16>(l, a->r, a->k, parts);
   if (!ok) {
     set_error("mlora_add_lora(slot-major): unsupported rank %d / K %d", a->r, a->k);
     return MLORA_E_UNSUPPORTED;

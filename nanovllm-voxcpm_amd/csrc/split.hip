@@ -60,7 +60,7 @@ struct SplitSlices {
 typedef unsigned long long u64;
 
 // Accesses to words that another workgroup of the same launch writes or reads.  Bits of `wide`
-// select device scope (performed where all XCDs meet) for loads (1), stores (2) and counters (4);
+// select device scope (performed where all XCDs meet) for loads (1) and stores (2);
 // without them they are performed in the L2 of the XCD, which is where all workgroups of a tile run.
 __device__ __forceinline__ u64 xload(const u64* p, int wide) {
   return (wide & 1) ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
@@ -70,15 +70,6 @@ __device__ __forceinline__ void xstore(u64* p, u64 v, int wide) {
   if (wide & 2) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ uint32_t xadd(uint32_t* p, uint32_t v, int wide) {
-  return (wide & 4) ? __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                    : __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void xstore32(uint32_t* p, uint32_t v, int wide) {
-  if (wide & 4) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 // NWP: wavefronts of a producer that take part in the shrink; a K part is NWP * 128 columns.
 template <typename T, int R, int NWP, bool MASKED>
 __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, void* __restrict__ yv_,
@@ -114,12 +105,10 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
   const i32x4 hdr2 = *reinterpret_cast<const i32x4*>(plan + 8);  // long small tiles, ...
   const uint32_t signature = ws[0];
   const RankPrefetch ranks = rank_prefetch(MASKED ? eff_rank : nullptr, num_slots, lane);
-  // {generation, arrivals} of the workspace: one pair for the whole launch, so that every tagged
-  // word any earlier launch left anywhere in the exchange area (whatever its layout was) carries a
-  // tag below this launch's
-  uint32_t* const tstate = ws + kWsTileOff / 4;
-  const uint32_t tag = tstate[0] + 1u;
-  const uint32_t arrivals0 = tstate[1], gen_check = tstate[2];
+  // the workspace's state: every tagged word any earlier launch left anywhere in the exchange area
+  // (whatever its layout was) carries a tag below this launch's
+  const WsState state = ws_state(ws, blockIdx.x);
+  const uint32_t generation = ws_generation(state), tag = generation + 1u;
   const int slot = rec0[0], m = rec0[1];
   const int n_tiles = hdr1[MLORA_PLAN_TILES_SHORT - 4] + hdr2[MLORA_PLAN_TILES_LONG_SMALL - 8] * include_long;
   // One exit test, the same for every workgroup of a tile
@@ -127,26 +116,16 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
                      int(hdr0[MLORA_PLAN_MAX_SLOTS] == num_slots) & int(tile < n_tiles) & int(m > 0) & int(slot >= 0) &
                      int(slot < num_slots);
   // the exchange area can be used: the head is in the state a launch (or the initialisation) left it in
-  const bool xok = trusted | ws_state_ok(signature, tag - 1u, arrivals0, gen_check, gridDim.x * gridDim.y * gridDim.z);
+  const bool xok = trusted | ws_state_ok(signature, state);
   // Every workgroup of the grid reports exactly once that it is done with the exchange area (also
-  // the ones without work); the last one advances the generation.  Counted by the last wavefront,
-  // which has the least other work: the count comes back from the memory system long after it was
-  // sent, and whoever sent it has to wait for it.
-  auto count_done = [&]() {
-    if (xok && tid == kNT - kWave) {
-      const uint32_t before = xadd(tstate + 1, 1u, wide);
-      if (before + 1u == gridDim.x * gridDim.y * gridDim.z) {
-        const uint32_t next = tag == 0xffffffffu ? 0u : tag;  // so that generation + 1, the next tag, is never 0
-        xstore32(tstate + 1, 0u, wide);
-        xstore32(tstate + 2, next ^ kWsGenCheck, wide);
-        xstore32(tstate, next, wide);
-      }
-    }
+  // the ones without work), by the last wavefront, which has the least other work.
+  auto report = [&]() {
+    if (xok && tid == kNT - kWave) ws_report(ws, generation);
   };
   if (!usable) {
     count_rejected_plan(plan, hdr0[MLORA_PLAN_MAGIC] == MLORA_PLAN_MAGIC_VALUE && hdr0[MLORA_PLAN_NUM_TOKENS] == T_ &&
                                   hdr0[MLORA_PLAN_MAX_SLOTS] == num_slots);
-    count_done();
+    report();
     return;
   }
   MLORA_STAMP(1);  // tile record, plan header and generation are here
@@ -156,7 +135,7 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
   // there and every test on it below folds away)
   const int eff = MASKED ? rank_pick(ranks, eff_rank, num_slots, slot, R) : R;
   if (MASKED && eff == 0) {  // nothing resident: the same for every workgroup of the tile
-    count_done();
+    report();
     return;
   }
   const int rb_n = MASKED ? (eff + 15) >> 4 : RB;  // 16-rank blocks of A in use
@@ -317,7 +296,7 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
     MLORA_STAMP(3);  // producer: partial sums handed to the memory system
   }
   if (!consumer || n0 >= n1) {  // nothing to expand here
-    count_done();
+    report();
     MLORA_STAMP(15);  // role marker: pure producers leave slot 15 non-zero
     return;
   }
@@ -398,8 +377,8 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
       if (c0 < n1) load_span(c0, bop[s], yq[s]);
     }
   }
-  count_done();  // this workgroup reads the exchange area no more
-  MLORA_STAMP(6);  // consumer: the intermediate is in LDS, the arrival counted
+  report();  // this workgroup reads the exchange area no more
+  MLORA_STAMP(6);  // consumer: the intermediate is in LDS, the report sent
 
   // ---- expand ---------------------------------------------------------------------------------------
   Pack8 hop[KSTEPS], hlo[KSTEPS];
@@ -494,7 +473,12 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
 __global__ __launch_bounds__(256) void workspace_init_kernel(uint32_t* ws) {
   const int words = MLORA_WORKSPACE_HEAD_BYTES / 4;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
-    ws[i] = i == 0 ? kWsMagic : i == kWsTileOff / 4 + 2 ? kWsGenCheck : 0u;  // generation 0 and its check word
+    {
+    uint32_t v = i == 0 ? kWsMagic : 0u;
+    for (int x = 0; x < 8; ++x)
+      if (i == ws_state_word(x) + 2) v = kWsGenCheck;  // generation 0's check word
+    ws[i] = v;
+  }
 }
 
 struct SplitLaunch {
