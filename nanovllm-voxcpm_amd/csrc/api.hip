@@ -186,6 +186,9 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
     // K = 2048: rank 64 8 slot ids 6.3 / 6.8, 32 8.0 / 10.4 and 8.6 / 11.4, 64 11.1 / 13.5; 8 tokens of 64 8.8 / 7.6.  Rank 32 16 ids
     // 5.2 / 5.3, 48 6.2 / 7.0, 64 7.4 / 8.3; 8 tokens of 32 5.2 / 5.1, 37 of one slot of 8 5.3 / 5.2.  Rank 16 40 ids 4.6 / 4.5, 48 4.7 /
     // 4.8, 64 5.3 / 5.4, 512 tokens of 32 (46 tiles) 5.2 / 5.2, 1000 (76) 6.2 / 7.6; rank 8 alike.
+    // Three slices (rank 64): twelve workgroups a tile, which have to fit the chip together: 8 ids 6.6 / 7.2 and 7.4 / 8.4, 16 8.5 / 9.9 and
+    // 8.9 / 10.4, 256 tokens of 16 (23 tiles) 9.4 / 11.0, 4 tokens of 16 8.0 / 7.6, 24 14.2 / 14.6, 32 16.1 / 13.5 (rank 32, without an instance: 8 ids 5.2 / 5.4, 16 6.0 / 5.8).
+    if (a->num_slices == 3) return slots <= (few ? 8 : 16) && tiles <= 24;
     if (a->k == 2048) return rank <= 16 ? !few && tiles >= 48 : !(few && (rank == 32 || rank * slots >= 2048));
     // K = 4096: 64 slot ids 5.1 / 5.7 at rank 8, 5.7 / 6.1, 8.7 / 10.3, 13.6 / 14.4 at rank 64; 8 tokens of 64 4.8 / 5.3, 5.3 / 5.4, 7.2 /
     // 6.8, 11.7 / 7.9; 64 tokens of 4 slots of 32 4.6 / 4.7, 4.6 / 4.8, 5.6 / 5.7, 9.2 / 8.0.

@@ -64,6 +64,8 @@ struct Exchange {
   uint32_t* ws;    // workspace head
   int spin_ticks;  // bound of the wait for the partners' words, in ticks of the 100 MHz clock (< 0: never accept any)
   int trusted;     // the head is known to be in a launch's or the initial state without carrying the signature
+  int part;        // this workgroup's K part
+  int64_t tile;    // which of the area's (tile, slice) places is theirs
 };
 
 typedef unsigned long long u64;
@@ -109,7 +111,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   const RankPrefetch ranks = rank_prefetch((MASKED && !EARLY) ? eff_rank : nullptr, num_slots, lane);
   if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);  // the record's requests go out first
 
-  const int kp = KP > 1 ? static_cast<int>(blockIdx.y) : 0;  // this workgroup's K part (and column range)
+  const int kp = KP > 1 ? xc.part : 0;  // this workgroup's K part (and column range)
   const int ks0 = kp * (KPART / 32) + wave * KSPW;
   // the workspace's state and signature (KP > 1): requested with the record (requested behind the A rows, or behind
   // the record, they cost up to 0.7 us more: 64 tokens of 32 slots, K = 2048, rank 64 masked 8.4 / 9.2 / 9.1 us per call)
@@ -325,7 +327,7 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   if constexpr (KP > 1) {
     // ---- the other K parts: from the tile's other workgroups, or multiplied here -----------------
     u64* const xchg = reinterpret_cast<u64*>(reinterpret_cast<char*>(xc.ws) + kWsXchgOff) +
-                      static_cast<int64_t>(blockIdx.z * 8 + blockIdx.x) * (KP * WORDS);  // the KP parts of this tile
+                      xc.tile * (KP * WORDS);  // the KP parts of this (tile, slice)
     float part[KP][EPT];
 #pragma unroll
     for (int q = 0; q < KP; ++q)
@@ -568,7 +570,7 @@ __global__ __launch_bounds__(NW* kWave) void slot_kernel(const int32_t* __restri
   // grid (8, column ranges, slot layers + layers of further tiles): blockIdx.x is the XCD, so a
   // slot's column ranges share an L2
   const int zslots = (num_slots + 7) >> 3;
-  const Exchange xc{ws, spin_ticks, trusted};
+  const Exchange xc{ws, spin_ticks, trusted, static_cast<int>(blockIdx.y), static_cast<int64_t>(blockIdx.z * 8 + blockIdx.x)};
   if (static_cast<int>(blockIdx.z) < zslots) {
     const int s = blockIdx.z * 8 + blockIdx.x;  // its record exists: the list is rounded up to eight
     const int slot = s < num_slots ? s : num_slots - 1;
@@ -586,29 +588,31 @@ __global__ __launch_bounds__(NW* kWave) void slot_kernel(const int32_t* __restri
 // 16 bytes (+-8 TiB: the slices of a projection are allocations of their own and may lie far apart;
 // the launcher takes this kernel only when they fit): their low 32 bits as four arguments, their
 // high 8 bits together in a fifth; the widths as 16-bit counts of eight columns.  widths01 = n0 / 8 | n1 / 8 << 16; widths2 = n2 / 8 | ranges of slice 0 << 16 |
-// ranges of slices 0 and 1 << 24; packed = columns per range / 64 | slots << 16.
-template <typename T, int R, bool MASKED>
-__global__ __launch_bounds__(kNW* kWave) void slot_kernel3(const int32_t* __restrict__ recs, const void* __restrict__ a0,
+// ranges of slices 0 and 1 << 24; packed = columns per range / 64 | slots << 16.  KP > 1: KP ranges and K parts of
+// every slice, of a width of its own.
+template <typename T, int NW, int R, int KP, int SA, bool MASKED>
+__global__ __launch_bounds__(NW* kWave) void slot_kernel3(const int32_t* __restrict__ recs, const void* __restrict__ a0,
                                                            const void* __restrict__ b0, uint32_t aoff1, uint32_t aoff2, uint32_t boff1, uint32_t boff2,
                                                            uint32_t off_high, uint32_t widths01, uint32_t widths2, uint32_t packed,
                                                            const void* __restrict__ xv, void* __restrict__ yv_, int64_t xs, int64_t ys,
                                                            int y_col0, int y_col1, int y_col2, uint32_t check, float scaling,
-                                                           const int32_t* __restrict__ eff_rank, int32_t* __restrict__ plan_hdr) {
+                                                           const int32_t* __restrict__ eff_rank, int32_t* __restrict__ plan_hdr,
+                                                           uint32_t* __restrict__ ws, int spin_ticks, int trusted) {
   constexpr int RB = (R + 15) / 16;
   constexpr int HSTRIDE = R + 8;
   constexpr int kStageRow = 17;
   constexpr int SB = RB < 2 ? RB : 2;
-  __shared__ __attribute__((aligned(16))) float s_red[kNW * RB * 64 * 4];
+  __shared__ __attribute__((aligned(16))) float s_red[NW * RB * 64 * 4];
   __shared__ __attribute__((aligned(16))) T s_hi[16 * HSTRIDE];
   __shared__ __attribute__((aligned(16))) T s_lo[16 * HSTRIDE];
-  __shared__ __attribute__((aligned(16))) i32x4 s_stage[kNW * (1 + SB) * 16 * kStageRow];
+  __shared__ __attribute__((aligned(16))) i32x4 s_stage[NW * (1 + SB) * 16 * kStageRow];
   __shared__ int s_ok;
   MLORA_STAMP(0);
 
-  const int nt = static_cast<int>(packed & 255u) * 64, num_slots = static_cast<int>(packed >> 16);
+  const int num_slots = static_cast<int>(packed >> 16);
   const int cum1 = static_cast<int>((widths2 >> 16) & 255u), cum2 = static_cast<int>(widths2 >> 24);
   const int ri = blockIdx.y;
-  const int slice = int(ri >= cum1) + int(ri >= cum2);
+  const int slice = KP > 1 ? ri / KP : int(ri >= cum1) + int(ri >= cum2);
   // (offset i: low word off_i, bits 32..39 in byte i of off_high, sign-extended)
   const uint32_t alo = slice == 1 ? aoff1 : aoff2, blo = slice == 1 ? boff1 : boff2;
   const int32_t ahi = static_cast<int8_t>(off_high >> (slice == 1 ? 0 : 8)), bhi = static_cast<int8_t>(off_high >> (slice == 1 ? 16 : 24));
@@ -618,19 +622,21 @@ __global__ __launch_bounds__(kNW* kWave) void slot_kernel3(const int32_t* __rest
   sp.b = static_cast<const char*>(b0) + bo * 16;
   sp.n = 8 * static_cast<int>(slice == 0 ? widths01 & 0xffffu : slice == 1 ? widths01 >> 16 : widths2 & 0xffffu);
   sp.y_col = 0;  // (selected inside, late)
-  sp.n0 = (ri - (slice == 0 ? 0 : slice == 1 ? cum1 : cum2)) * nt;
+  const int part = KP > 1 ? ri % KP : ri - (slice == 0 ? 0 : slice == 1 ? cum1 : cum2);
+  const int nt = KP > 1 ? ((sp.n + KP - 1) / KP + 63) & ~63 : static_cast<int>(packed & 255u) * 64;
+  sp.n0 = part * nt;
   sp.n1 = sp.n0 + nt < sp.n ? sp.n0 + nt : sp.n;
 
   const int zslots = (num_slots + 7) >> 3;
-  const Exchange xc{nullptr, 0, 0};
+  const Exchange xc{ws, spin_ticks, trusted, part, static_cast<int64_t>(blockIdx.z * 8 + blockIdx.x) * 3 + slice};
   if (static_cast<int>(blockIdx.z) < zslots) {
     const int s = blockIdx.z * 8 + blockIdx.x;
     const int slot = s < num_slots ? s : num_slots - 1;
-    slot_tile<T, kNW, R, 4, 1, MASKED, false, 1, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), R, sp, y_col0, y_col1, y_col2, slice, xv,
+    slot_tile<T, NW, R, 4, KP, MASKED, false, SA, true>(recs + s * MLORA_SMALL_TILE_WORDS, slot, int(s < num_slots), R, sp, y_col0, y_col1, y_col2, slice, xv,
                                                   yv_, xs, ys, num_slots, scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   } else {
     const int q = zslots * 8 + (blockIdx.z - zslots) * 8 + blockIdx.x;
-    slot_tile<T, kNW, R, 4, 1, MASKED, false, 1, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, R, sp, y_col0, y_col1, y_col2, slice, xv, yv_, xs, ys,
+    slot_tile<T, NW, R, 4, KP, MASKED, false, SA, false>(recs + q * MLORA_SMALL_TILE_WORDS, 0, 1, R, sp, y_col0, y_col1, y_col2, slice, xv, yv_, xs, ys,
                                                    num_slots, scaling, eff_rank, check, plan_hdr, xc, s_red, s_hi, s_lo, s_stage, &s_ok);
   }
 }
@@ -658,8 +664,9 @@ bool offsets16(const MloraAddArgs* a, int i, long long* ao, long long* bo) {
   return true;
 }
 
-template <typename T, int R>
-void launch_three(const MloraAddArgs* a, dim3 grid, int nt, int cum1, int cum2) {
+template <typename T, int NW, int R, int KP, int SA>
+void launch_three(const Launch& l, int nt, int cum1, int cum2) {
+  const MloraAddArgs* a = l.a;
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   long long o[4] = {0, 0, 0, 0};  // A of slices 1 and 2, B of slices 1 and 2
   (void)offsets16(a, 1, &o[0], &o[2]);
@@ -671,16 +678,14 @@ void launch_three(const MloraAddArgs* a, dim3 grid, int nt, int cum1, int cum2) 
   const uint32_t w2 = static_cast<uint32_t>(a->slices[2].n / 8) | (static_cast<uint32_t>(cum1) << 16) | (static_cast<uint32_t>(cum2) << 24);
   const uint32_t packed = static_cast<uint32_t>(nt / 64) | (static_cast<uint32_t>(a->num_slots) << 16);
   const uint32_t check = static_cast<uint32_t>(MLORA_PLAN_CHECK(a->num_tokens, a->num_slots));
-  if (a->effective_rank)
-    hipLaunchKernelGGL((slot_kernel3<T, R, true>), grid, dim3(kNW * kWave), 0, static_cast<hipStream_t>(a->stream), a->plan + lay.slotrec_off,
-                       a->slices[0].a, a->slices[0].b, ao1, ao2, bo1, bo2, high, w01, w2, packed, a->x, a->y, a->x_stride, a->y_stride,
-                       a->slices[0].y_col, a->slices[1].y_col, a->slices[2].y_col, check, a->scaling, a->effective_rank,
-                       const_cast<int32_t*>(a->plan));
-  else
-    hipLaunchKernelGGL((slot_kernel3<T, R, false>), grid, dim3(kNW * kWave), 0, static_cast<hipStream_t>(a->stream), a->plan + lay.slotrec_off,
-                       a->slices[0].a, a->slices[0].b, ao1, ao2, bo1, bo2, high, w01, w2, packed, a->x, a->y, a->x_stride, a->y_stride,
-                       a->slices[0].y_col, a->slices[1].y_col, a->slices[2].y_col, check, a->scaling, a->effective_rank,
-                       const_cast<int32_t*>(a->plan));
+  auto launch = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, l.grid, dim3(NW * kWave), 0, static_cast<hipStream_t>(a->stream), a->plan + lay.slotrec_off, a->slices[0].a,
+                       a->slices[0].b, ao1, ao2, bo1, bo2, high, w01, w2, packed, a->x, a->y, a->x_stride, a->y_stride, a->slices[0].y_col,
+                       a->slices[1].y_col, a->slices[2].y_col, check, a->scaling, a->effective_rank, const_cast<int32_t*>(a->plan),
+                       static_cast<uint32_t*>(a->workspace), l.spin_ticks, l.trusted);
+  };
+  if (a->effective_rank) launch(slot_kernel3<T, NW, R, KP, SA, true>);
+  else launch(slot_kernel3<T, NW, R, KP, SA, false>);
 }
 
 template <typename T, int NW, int R, int KSPW, int KP, bool MASKED, bool GR, int SA>
@@ -788,16 +793,18 @@ SlotKnobs& slot_knobs() {
 // Whether a tile's workgroups can hand each other the partial sums of these parts: columns for every part, an
 // instance for their ranges, an exchange area that holds every tile's.
 bool parts_fit(const MloraAddArgs* a, Parts p) {
-  const int n = a->slices[0].n, nt = ((n + p.kp - 1) / p.kp + 63) & ~63;
-  if (n < p.kp * 64 || (p.kp - 1) * nt >= n) return false;  // (a part without columns would leave the tile)
-  const int spans = (nt + 64 * p.nw - 1) / (64 * p.nw);
-  if (spans > 2 || (spans == 2 && p.nw == kNW && (p.kp == 8 || a->r > 32))) return false;  // (instances; registers beside the parts)
+  for (int i = 0; i < a->num_slices; ++i) {
+    const int n = a->slices[i].n, nt = ((n + p.kp - 1) / p.kp + 63) & ~63;
+    if (n < p.kp * 64 || (p.kp - 1) * nt >= n) return false;  // (a part without columns would leave the tile)
+    const int spans = (nt + 64 * p.nw - 1) / (64 * p.nw);
+    if (spans > 2 || (spans == 2 && p.nw == kNW && (p.kp == 8 || a->r > 32))) return false;  // (instances; registers beside the parts)
+  }
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
-  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * p.kp * ((compute_rank(a->r) + 15) / 16) * 256;
+  const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * a->num_slices * p.kp * ((compute_rank(a->r) + 15) / 16) * 256;
   return words * 8 <= kWsXchgBytes;
 }
 
-// K parts of a launch (one slice, an initialised workspace), else one.  Of 1024 columns for eight wavefronts or of
+// K parts of a launch (one slice, or q | k | v at K = 2048 and rank 64; an initialised workspace), else one.  Of 1024 columns for eight wavefronts or of
 // 512 for four: smaller parts take in less per compute unit, and there are twice as many workgroups that wait
 // for each other, so K = 4096 is cut into eight while parts x tiles (or slot ids) are few (us per call in four parts / in
 // eight: rank 16, 16 slot ids 4.7 / 4.4, 32 4.8 / 4.6, 40 4.9 / 5.0, 64 5.7 / 5.8; rank 32, 16 5.3 / 4.9, 24 5.5 / 5.4, 32 6.0 / 6.0, 40
@@ -805,7 +812,8 @@ bool parts_fit(const MloraAddArgs* a, Parts p) {
 // K = 2048 in four, 8192 in eight of 1024.
 Parts k_parts(const MloraAddArgs* a) {
   const Parts one = {1, kNW};
-  if (a->num_slices != 1 || slot_knobs().kparts == 1) return one;
+  const bool three = a->num_slices == 3 && a->k == 2048 && a->r == 64;
+  if (!(a->num_slices == 1 || three) || slot_knobs().kparts == 1) return one;
   if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return one;
   const Parts small = {a->k / 512, 4}, large = {a->k / 1024, kNW};
   const int tiles = small_tiles_about(a, 0), most = tiles > a->num_slots ? tiles : a->num_slots;
@@ -816,7 +824,7 @@ Parts k_parts(const MloraAddArgs* a) {
 
 }  // namespace
 
-// K = 1024 at every rank; K = 2048, 4096 and 8192 at every rank with the K parts of a tile shared out between its
+// K = 1024 at every rank; one slice of K = 2048, 4096 and 8192 at every rank with the K parts of a tile shared out between its
 // workgroups, K = 4096 without up to rank 16 (what fits the register file as one batch of loads); one or two
 // slices with their pointers as arguments, three (K = 1024) with the later two's as offsets from
 // the first one's; 16-bit elements.
@@ -835,9 +843,10 @@ bool slot_supported(const MloraAddArgs* a) {
     // q | k | v: K = 1024, an exact rank, offsets that fit 40 bits, widths that fit 16-bit counts of
     // eight columns, and column ranges of at most 512 columns (one span per wavefront)
     long long ao, bo;
-    if (kspw != 4 || !exact_rank(a->r) || !offsets16(a, 1, &ao, &bo) || !offsets16(a, 2, &ao, &bo)) return false;
+    if (!exact_rank(a->r) || !offsets16(a, 1, &ao, &bo) || !offsets16(a, 2, &ao, &bo)) return false;
     for (int i = 0; i < 3; ++i)
       if (a->slices[i].n % 8 || a->slices[i].n / 8 > 0xffff) return false;
+    if (kspw != 4) return k_parts(a).kp > 1;
     return range_columns(a) <= kNW * 64;
   }
   if (kspw == 4) return true;
@@ -858,11 +867,11 @@ int launch_slot(const MloraAddArgs* a, bool trusted_workspace) {
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   const Parts parts = k_parts(a);
   const int kp = parts.kp;
-  // with K parts the tile's workgroups are its K parts and its column ranges alike
+  // with K parts a (tile, slice)'s workgroups are its K parts and its column ranges alike
   const int nt = kp > 1 ? ((a->slices[0].n + kp - 1) / kp + 63) & ~63 : range_columns(a);
   const int ranges0 = kp > 1 ? kp : (a->slices[0].n + nt - 1) / nt;
   const int ranges1 = a->num_slices > 1 ? (a->slices[1].n + nt - 1) / nt : 0;
-  const int total = ranges0 + ranges1 + (a->num_slices > 2 ? (a->slices[2].n + nt - 1) / nt : 0);
+  const int total = kp > 1 ? a->num_slices * kp : ranges0 + ranges1 + (a->num_slices > 2 ? (a->slices[2].n + nt - 1) / nt : 0);
   if (total > 255) {
     set_error("mlora_add_lora(slot-major): %d column ranges exceed 255", total);
     return MLORA_E_UNSUPPORTED;
@@ -878,12 +887,17 @@ int launch_slot(const MloraAddArgs* a, bool trusted_workspace) {
   l.spin_ticks = slot_knobs().spin_ticks;
   l.trusted = trusted_workspace ? 1 : 0;
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>((lay.cap_slotrec + lay.cap_over) / 8));
+  if (a->num_slices == 3 && kp > 1) {
+    if (a->dtype == MLORA_DTYPE_BF16) launch_three<__bf16, 4, 64, 4, 2>(l, nt, 0, 0);
+    else launch_three<_Float16, 4, 64, 4, 2>(l, nt, 0, 0);
+    return check_launch("mlora_add_lora(small tiles, K parts of three slices)");
+  }
   if (a->num_slices == 3) {
     switch (a->r) {
 #define MLORA_THREE(R)                                                                                      \
   case R:                                                                                                   \
-    if (a->dtype == MLORA_DTYPE_BF16) launch_three<__bf16, R>(a, l.grid, nt, ranges0, ranges0 + ranges1);   \
-    else launch_three<_Float16, R>(a, l.grid, nt, ranges0, ranges0 + ranges1);                              \
+    if (a->dtype == MLORA_DTYPE_BF16) launch_three<__bf16, kNW, R, 1, 1>(l, nt, ranges0, ranges0 + ranges1);   \
+    else launch_three<_Float16, kNW, R, 1, 1>(l, nt, ranges0, ranges0 + ranges1);                              \
     break;
       MLORA_THREE(8)
       MLORA_THREE(16)
