@@ -146,7 +146,7 @@ template <typename F> __device__ __forceinline__ Sums scan_buckets(const Buckets
 }
 
 // Everything that is stored, by the workgroups of a batch together: what belongs to token t (when below T),
-// and of what belongs to no token thread `gid` of `threads` takes its share.  No word is stored to twice,
+// and of what belongs to no token thread `gid` of `threads` (at least four wavefronts) takes its share.  No word is stored to twice,
 // so nothing here waits for a store.
 __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, int T, const Place& me, int gid, int threads, int t) {
   const int L = p.L, NB = k.NB, key = me.key, r = me.r;
@@ -178,12 +178,17 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
         // its record in the list of tiles and the same once more in the list by slot
         int32_t* rec = p.plan + lay.small_off + ((is_short ? k.ts_short[key] : n.small_short + k.ts_long[key]) + tile) * MLORA_SMALL_TILE_WORDS;
         int32_t* rec2 = p.plan + lay.slotrec_off + (tile == 0 ? key - 1 : lay.cap_slotrec + k.ts_over[key] + tile - 1) * MLORA_SMALL_TILE_WORDS;
-        for (int pos = at; pos < MLORA_TILE_SMALL; pos += rows) {
-          rec[MLORA_SMALL_TILE_ROWS + pos] = t;
-          rec2[MLORA_SMALL_TILE_ROWS + pos] = t;
+        i32x4 *w = reinterpret_cast<i32x4*>(rec), *w2 = reinterpret_cast<i32x4*>(rec2);
+        if (rows == 1) {
+#pragma unroll
+          for (int i = MLORA_SMALL_TILE_ROWS / 4; i < kRecordTail; ++i) w[i] = w2[i] = i32x4{t, t, t, t};
+        } else {
+          for (int pos = at; pos < MLORA_TILE_SMALL; pos += rows) {
+            rec[MLORA_SMALL_TILE_ROWS + pos] = t;
+            rec2[MLORA_SMALL_TILE_ROWS + pos] = t;
+          }
         }
         if (at == 0) {
-          i32x4 *w = reinterpret_cast<i32x4*>(rec), *w2 = reinterpret_cast<i32x4*>(rec2);
           w[0] = i32x4{key - 1, rows, first + r, 0};
           w2[0] = i32x4{key - 1, rows, first + r, check};
 #pragma unroll
@@ -209,7 +214,15 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
     for (int i = gid; i < p.padded_len; i += threads) p.padded_tts[i] = i < T ? me.slot : -1;  // (below T: i is t)
   }
 
-  if (gid == 0) {
+  // The rest by other wavefronts than the tokens' while there are any: the header, what is stored per bucket and what no token
+  // stores by one of the last four each (up to 64 tokens of 32 slots 3.3 us per launch, 4.3 with all of it behind
+  // wavefront 0's tokens; in the last workgroup of several, 0.1 to 0.6 us more).
+  auto share_of = [&](int waves) {
+    if (T > kMetaThreads - 4 * kWave) return gid;
+    const int i = threads - 1 - waves * kWave - gid;
+    return i < 0 ? i + threads : i;
+  };
+  if (share_of(1) == 0) {
     if (p.plan) {
       int32_t* h = p.plan;
       h[MLORA_PLAN_MAGIC] = MLORA_PLAN_MAGIC_VALUE;
@@ -238,7 +251,7 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
   }
 
   // Per-bucket outputs.
-  for (int b = gid; b < NB; b += threads) {
+  for (int b = share_of(2); b < NB; b += threads) {
     const int c = b >= 1 ? k.off[b + 1] - k.off[b] : 0;
     if (p.dense_counts) p.dense_counts[b] = c;
     if (p.dense_offsets) p.dense_offsets[b + 1] = k.off[b + 1];
@@ -254,7 +267,7 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
       if (p.compact_offsets) p.compact_offsets[i] = b == 0 ? 0 : n_neg + k.off[b];
     }
   }
-  for (int i = n_compact + gid; i < p.compact_capacity; i += threads) {
+  for (int i = n_compact + share_of(3); i < p.compact_capacity; i += threads) {
     if (p.compact_ids) p.compact_ids[i] = -1;
     if (p.compact_counts) p.compact_counts[i] = 0;
     if (p.compact_offsets) p.compact_offsets[i + 1] = 0;
@@ -266,7 +279,7 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
   if (p.plan) {
     i32x4* big = reinterpret_cast<i32x4*>(p.plan + lay.big_off);
     const int block = lay.cap_big >> 3;
-    for (int q = gid; q < lay.cap_big; q += threads) {
+    for (int q = share_of(3); q < lay.cap_big; q += threads) {
       if (n.big == 0) {
         big[q] = i32x4{-1, 0, 0, 0};
         continue;
@@ -275,7 +288,7 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
       if ((i * 8 + x) * run + (w - i * run) >= n.big) big[q] = i32x4{-1, 0, 0, 0};
     }
     i32x4* byslot = reinterpret_cast<i32x4*>(p.plan + lay.slotrec_off);
-    for (int q = gid; q < lay.cap_slotrec + lay.cap_over; q += threads) {
+    for (int q = share_of(0); q < lay.cap_slotrec + lay.cap_over; q += threads) {
       i32x4 head = i32x4{-1, 0, 0, check};
       if (q < L) {
         if (k.off[q + 2] != k.off[q + 1]) continue;
@@ -298,9 +311,9 @@ __device__ __forceinline__ void put_out(const MetaParams& p, const Buckets& k, i
 // ids and LDS atomics a thread.  A token's place among the equal ids of its 64 is found with ballots, that
 // among the wavefronts with one 64-bit word of byte counts.  Two barriers, none of which waits for memory.
 // Measured in a replayed graph against one workgroup that walked the batch twice (us per launch, plan of random
-// ids / of sorted ids / three domains): 64 tokens and 32 slots 5.8 / 5.9 / 4.1 before, 4.3 / 4.3 / 3.2 now;
+// ids / of sorted ids / three domains): 64 tokens and 32 slots 5.8 / 5.9 / 4.1 before, 3.3 / 3.4 / 3.2 now;
 // 512 and 64 6.0 / 5.9 / 4.5, 4.8 / 4.6 / 3.6; 3001 and 16 11.3 / 13.1 / 7.8, 5.5 / 5.3 / 4.3; 8192 and 128
-// 31.0 / 32.5 / 18.2, 10.1 / 12.7 / 6.7.  A pass of 48 calls on one token takes 181.8 us instead of 185.2, one
+// 31.0 / 32.5 / 18.2, 10.1 / 12.7 / 6.7.  A pass of 48 calls on one token takes 181.2 us instead of 185.3, one
 // of 96 on 9392 tokens 3287 instead of 3323.
 // `s`: slot id of token t, -1 from T on (requested by the caller ahead of everything else)
 template <typename F>
