@@ -173,10 +173,10 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   if (a->num_tokens > 32 * a->num_slots) return false;
   const bool sparse = active > 0 && 2 * active <= a->num_slots;
   const int parts = slot_k_parts(a);
-  // Buffers of a rank between 32 and 64 run rank 64's code masked, whose K parts lose to the pair at almost every
-  // size (rank 48, one token per slot id, slot-major / pair: K = 8192 11.5 / 7.8 at 8 slot ids, 19.8 / 11.9 at 32; K = 4096
-  // 7.4 / 7.5 and 9.8 / 9.7, four tokens per slot id 8.7 / 7.9 and 10.5 / 10.2).
-  if (parts > 1 && a->r > 32 && !exact_rank(a->r)) return false;
+  // Buffers of a rank between 32 and 64 run rank 64's code masked: K = 2048 gains like rank 64's (rank 48, slot-major / pair: 7.0 /
+  // 7.4 at 16 tokens of 8 slot ids, 8.3 / 9.8 at 128 of 32, 10.6 / 12.3 at 256 of 64), eight parts of 1024 columns do not fit
+  // the registers (K = 8192: 11.4 / 7.9 at one token of 8, 20.3 / 13.4 at 128 of 32), and K = 4096 stays with the pair.
+  if (parts > 1 && a->r > 32 && !exact_rank(a->r) && a->k != 2048) return false;
   if (parts > 1) {
     // K shared out: the lines lie where the requests for slots without tokens, and at K = 8192 more workgroups than fit
     // the chip together, cost what the second launch does.  us per call, slot-major / the best other form, at

@@ -23,6 +23,7 @@ CASES = [  # k, tokens, slots, rank, n, dtype, mixed ranks
     (4096, 33, 8, 64, 2048, F16, True),
     (4096, 20, 5, 32, 4096, B16, False),
     (4096, 2, 24, 48, 1000, B16, True),
+    (2048, 35, 12, 48, 1000, F16, True),
 ]
 _STATES = [64] + [(256 + 8192 + 256 * x) // 4 for x in range(1, 8)]  # first words of the states
 
