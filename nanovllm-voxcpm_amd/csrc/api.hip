@@ -338,7 +338,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
   // small tiles with the grid laid over the slots where the shape allows it and slot ids are few.
   // Also where the split form would be taken: at K = 4096 the slot-major kernel shares K out between
   // the workgroups of a tile itself (down, decode batch, us per call, slot-major / split form:
-  // rank 32: 8.1 / 10.6, rank 64: 10.7 / 17.0).
+  // rank 32: 6.3 / 10.6, rank 64: 9.8 / 17.0).
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
       knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, active))
     form = MLORA_FORM_SLOT;
