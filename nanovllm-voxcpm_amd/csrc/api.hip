@@ -206,7 +206,10 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double per_slot = 2.0 * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
   if (a->num_slots * per_slot <= 3.0e6) return true;
-  return a->num_tokens >= 4 * a->num_slots;
+  // Where A[slot] and B[slot] are light the line lies at two tokens per slot id: 64 tokens of 32 ids at random, us per call, slot-major /
+  // tile-major: rank 16 qkv 3.8 / 4.0, gate_up 5.1 / 5.3; rank 32 o 4.3 / 4.5, but gate_up 7.5 / 7.4; rank 64 qkv 7.9 / 7.5, o 6.0 / 5.8.
+  const bool light = a->k == 1024 && (compute_rank(a->r) <= 16 || (compute_rank(a->r) == 32 && a->num_slices == 1 && cols <= 2048));
+  return a->num_tokens >= (light ? 2 : 4) * a->num_slots;
 }
 
 // Where the shrink and the expand as two launches over 16-token tiles (pair.hip) beat the form that
