@@ -700,23 +700,23 @@ void launch_spans(const Launch& l) {
                      a->effective_rank, const_cast<int32_t*>(a->plan), static_cast<uint32_t*>(a->workspace), l.spin_ticks, l.trusted);
 }
 
+// Instances of one span per wavefront alone for eight parts, of two alone for four parts of 512 columns.
 template <typename T, int NW, int R, int KSPW, int KP>
 void launch_one(const Launch& l) {
-  constexpr bool kOne = NW == 8 && KP == 8;  // (eight wavefronts: ranges of two spans are not cut into eight parts)
-  const bool one_span = kOne || l.widest <= NW * 64;
-  constexpr int kTwo = kOne ? 1 : 2;
+  constexpr int kTwo = KP == 8 ? 1 : 2, kOne = NW == 4 && KP == 4 ? 2 : 1;
+  const bool one_span = KP == 8 || l.widest <= NW * 64;
   if constexpr (R >= 32) {
     if (l.a->r != R) {  // buffers of a rank between the instances': the masked code with the buffers' rank as stride
-      if (one_span) launch_spans<T, NW, R, KSPW, KP, true, true, 1>(l);
+      if (one_span) launch_spans<T, NW, R, KSPW, KP, true, true, kOne>(l);
       else launch_spans<T, NW, R, KSPW, KP, true, true, kTwo>(l);
       return;
     }
   }
   if (l.a->effective_rank) {
-    if (one_span) launch_spans<T, NW, R, KSPW, KP, true, false, 1>(l);
+    if (one_span) launch_spans<T, NW, R, KSPW, KP, true, false, kOne>(l);
     else launch_spans<T, NW, R, KSPW, KP, true, false, kTwo>(l);
   } else {
-    if (one_span) launch_spans<T, NW, R, KSPW, KP, false, false, 1>(l);
+    if (one_span) launch_spans<T, NW, R, KSPW, KP, false, false, kOne>(l);
     else launch_spans<T, NW, R, KSPW, KP, false, false, kTwo>(l);
   }
 }
@@ -797,7 +797,7 @@ bool parts_fit(const MloraAddArgs* a, Parts p) {
     const int n = a->slices[i].n, nt = ((n + p.kp - 1) / p.kp + 63) & ~63;
     if (n < p.kp * 64 || (p.kp - 1) * nt >= n) return false;  // (a part without columns would leave the tile)
     const int spans = (nt + 64 * p.nw - 1) / (64 * p.nw);
-    if (spans > 2 || (spans == 2 && p.nw == kNW && (p.kp == 8 || a->r > 32))) return false;  // (instances; registers beside the parts)
+    if (spans > 2 || (spans == 2 && (p.kp == 8 || (p.nw == kNW && a->r > 32)))) return false;  // (instances; registers beside the parts)
   }
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   const long long words = static_cast<long long>(lay.cap_slotrec + lay.cap_over) * a->num_slices * p.kp * ((compute_rank(a->r) + 15) / 16) * 256;
