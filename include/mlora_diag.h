@@ -3,7 +3,7 @@
  * counterpart in the reference and nothing here is needed to use the library: include/mlora.h is
  * the product's C-ABI.
  *
- * mlora_probe_launch and mlora_trace_set are exported by the diagnostic variants only
+ * mlora_probe_launch, mlora_trace_set and mlora_group_layout are exported by the diagnostic variants only
  * (libmlora_gfx950_diag.so from `make diag`, libmlora_gfx950_trace.so from `make trace`).
  * mlora_reload_knobs is exported by every variant: the test-suite changes MLORA_* variables
  * between tests of one process.
@@ -35,6 +35,14 @@ int mlora_probe_launch(void* stream, int32_t kind, void* buf, int64_t bytes, int
  * (uint64 [workgroups][16], device memory the caller zeroes; NULL switches recording off).  The
  * diag variant returns MLORA_E_UNSUPPORTED. */
 int mlora_trace_set(void* buf);
+
+/* How the low-level ops over tiles of a slot are laid over a grid of `parts` workgroups per place (host
+ * arithmetic, nothing is launched; num_tokens and num_slots at least 1, parts at least 1): out[0] 1 if
+ * over the tokens, 0 if over the slots, out[1] places, out[2] slot ids rounded up to eight, out[3]
+ * tiles of a slot with a place of their own, out[4] tokens of a narrow tile; of a slot that has
+ * `count` tokens, out[5] tokens of its tiles, out[6] tiles beyond those with a place of their own.
+ * `extra` is 1 where the tokens without a slot need places (the shrink), else 0. */
+void mlora_group_layout(int32_t num_tokens, int32_t num_slots, int64_t parts, int32_t extra, int32_t count, int32_t* out);
 
 #ifdef __cplusplus
 }

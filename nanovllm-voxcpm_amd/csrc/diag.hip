@@ -1,6 +1,7 @@
 // Entry points of the diagnostic variants of the library (include/mlora_diag.h): none of them has a
 // counterpart in the reference and none is part of the product library.
 #include "common.h"
+#include "group_layout.h"
 #include "launch.h"
 #include "mlora_diag.h"
 
@@ -21,4 +22,13 @@ extern "C" int mlora_trace_set(void* buf) {
   set_error("mlora_trace_set: this library was built without MLORA_TRACE (make trace builds the variant that records timelines)");
   return MLORA_E_UNSUPPORTED;
 #endif
+}
+
+extern "C" void mlora_group_layout(int32_t num_tokens, int32_t num_slots, int64_t parts, int32_t extra, int32_t count, int32_t* out) {
+  GroupPlaces p = {};
+  p.T = num_tokens; p.num_slots = num_slots;
+  out[1] = lay_out(p, &out[0], parts, extra);
+  out[2] = p.slots8; out[3] = p.tiles; out[4] = p.width;
+  out[5] = out[0] == kBySlot ? tile_width(p, count) : p.width;
+  out[6] = out[0] == kBySlot ? tiles_beyond(p, count) : 0;
 }

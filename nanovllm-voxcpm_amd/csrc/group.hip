@@ -10,35 +10,29 @@
 // What bounds it: two trips to memory (ids, then the rows they name) and a compute unit's intake of weights in the second one;
 // hence ranks in blocks of eight or sixteen and tokens in tiles of four to sixteen, as many workgroups as the chip takes.
 #include "common.h"
+#include "group_layout.h"
 #include "launch.h"
 
 namespace mlora {
 
 namespace {
 
-// What the grid is laid over.  By slot: places are (tile of a slot, slot), then the tiles that no slot is expected to have (a
-// popular adapter's), which find out from a histogram whose they are.  By token: a place is a token; the first token of every
-// tile stands for it, the others leave.
-constexpr int kBySlot = 0, kByToken = 1;
-
-struct Places {
+struct Places : GroupPlaces {
   const int32_t* tts;
-  int T, num_slots;
-  int width;        // tokens of a tile: 4, 8 or 16 (tiles beyond the expected ones: 16)
-  int slots8;       // by slot: slot ids (and, in the shrink, one for the tokens without a slot) rounded up to eight
-  int tiles;        // by slot: tiles of a slot that have a place of their own
 };
 
 __device__ __forceinline__ int known_slot(const Places& p, int id) { return id >= 0 && id < p.num_slots ? id : p.num_slots; }
 
-// Lists in s_rows the tokens of `slot` from token `from` on: of those the ones at [first, first + width), in ascending order.  Returns
-// their number, or 0 when the tokens of the slot before `from` do not fill whole tiles.  s_wave: two words per wavefront.
-template <int THREADS>
-__device__ __forceinline__ int list_tile(const Places& p, int first_id, int slot, int from, int first, int width, int* __restrict__ s_rows,
-                                         int* __restrict__ s_wave) {
+// Lists the tokens of a tile in ascending order; returns their number and, through `rows`, where in s_rows they stand.  By token: the
+// tile that starts at token `from` of `slot`; 0 when the tokens of the slot before it do not fill whole tiles.  By slot: the tile-th
+// tile of the slot, whose width follows from the slot's number of tokens; until that is known, both widths are listed.
+// s_rows: MLORA_TILE_SMALL words (by slot: twice as many), s_wave: two words per wavefront.
+template <int THREADS, int GRID>
+__device__ __forceinline__ int list_tile(const Places& p, int first_id, int slot, int from, int tile, int* __restrict__ s_rows,
+                                         int* __restrict__ s_wave, const int*& rows) {
   constexpr int W = THREADS / kWave;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  int late = 0, early = 0, id = first_id, half = 0;
+  int late = 0, early = 0, id = first_id, half = 0, width = p.width;
   for (int base = 0; base < p.T; base += THREADS) {
     const int t = base + tid;
     if (base > 0) id = p.tts[t < p.T ? t : p.T - 1];
@@ -55,16 +49,22 @@ __device__ __forceinline__ int list_tile(const Places& p, int first_id, int slot
       late += n & 0xffff;
       early += n >> 16;
     }
-    pos += __popcll(set & ((1ull << lane) - 1ull)) - first;
-    if (match && t >= from && pos >= 0 && pos < width) s_rows[pos] = t;
+    pos += __popcll(set & ((1ull << lane) - 1ull));
+    if constexpr (GRID == kBySlot) width = tile_width(p, late);
+    const unsigned at = pos - tile * width, wide = pos - tile * MLORA_TILE_SMALL;
+    if (match && t >= from && at < static_cast<unsigned>(width)) s_rows[(width != p.width ? MLORA_TILE_SMALL : 0) + at] = t;
+    if (GRID == kBySlot && base + THREADS < p.T && width == p.width) {  // (ids to come may make the slot's tiles wide ones)
+      if (match && t >= from && wide < static_cast<unsigned>(MLORA_TILE_SMALL)) s_rows[MLORA_TILE_SMALL + wide] = t;
+    }
     half ^= 1;
   }
   __syncthreads();
-  const int n = late - first;
+  rows = s_rows + (width != p.width ? MLORA_TILE_SMALL : 0);
+  const int n = late - tile * width;
   return early % width != 0 || n <= 0 ? 0 : n < width ? n : width;
 }
 
-// By slot, behind the expected tiles: the slot and first token position of the q-th tile beyond them, or slot -1.
+// By slot, behind the tiles with a place of their own: the slot and, of that, the tile that the q-th further place stands for, or slot -1.
 template <int THREADS>
 __device__ __forceinline__ void find_tile(const Places& p, int first_id, int q, int* __restrict__ s_hist, int* __restrict__ s_found) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -85,11 +85,9 @@ __device__ __forceinline__ void find_tile(const Places& p, int first_id, int q, 
   }
   __syncthreads();
   if (tid < kWave) {
-    const int covered = p.tiles * p.width;
     int run = 0;
     for (int base = 0; base < p.num_slots; base += kWave) {
-      const int s = base + lane, c = s < p.num_slots ? s_hist[s] - covered : 0;
-      const int mine = c > 0 ? (c + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL : 0;
+      const int s = base + lane, mine = s < p.num_slots ? tiles_beyond(p, s_hist[s]) : 0;
       int sum = mine;
 #pragma unroll
       for (int d = 1; d < kWave; d *= 2) {
@@ -99,7 +97,7 @@ __device__ __forceinline__ void find_tile(const Places& p, int first_id, int q, 
       const int at = q - (run + sum - mine);
       if (at >= 0 && at < mine) {
         s_found[0] = s;
-        s_found[1] = covered + at * MLORA_TILE_SMALL;
+        s_found[1] = p.tiles + at;
       }
       run += __builtin_amdgcn_readlane(sum, kWave - 1);
     }
@@ -129,15 +127,15 @@ __device__ __forceinline__ void store_as(void* out, int64_t at, float v, int dty
 // out[slice, t, :] = scaling * x[t] . A[s]^T, zero for rows without a slot; grid (8, slices * blocks, places / 8), blockIdx.x the XCD
 // (a slot's workgroups share one).  RW: ranks of a workgroup (8 or 16); CH: rounds whose operands are on their way together.
 template <typename T, int RW, int CH, int GRID>
-__global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width_, int slots8,
+__global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width, int slots8,
                                                                       int tiles, int blocks, int K, int r, const void* __restrict__ x,
                                                                       GroupShrinkParams p) {
-  const Places pl{tts, T_, num_slots, width_, slots8, tiles};
+  const Places pl{{T_, num_slots, width, slots8, tiles}, tts};
   constexpr int kStageRow = 17;  // 16 chunks of 16 bytes + one of padding: operand reads hit every bank once
   constexpr int AI = RW / 4;     // loads of a round's A rows, four rows each
   __shared__ __attribute__((aligned(16))) i32x4 s_stage[kShrinkWaves * 2 * 16 * kStageRow];
   __shared__ __attribute__((aligned(16))) float s_red[kShrinkWaves * 64 * 4];
-  __shared__ int s_rows[MLORA_TILE_SMALL], s_wave[2 * kShrinkWaves], s_found[2];
+  __shared__ int s_rows[(GRID == kBySlot ? 2 : 1) * MLORA_TILE_SMALL], s_wave[2 * kShrinkWaves], s_found[2];
   static_assert(sizeof(s_stage) >= MLORA_MAX_SLOTS * sizeof(int), "the histogram takes the staging area");
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;
@@ -147,7 +145,7 @@ __global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int3
   const int slice = blockIdx.y / blocks, r0 = (blockIdx.y - slice * blocks) * RW;
   const int rounds = K / kRound;
   const int64_t out0 = static_cast<int64_t>(slice) * T_ * r;
-  int slot, from = 0, first = 0, width = width_;
+  int slot, from = 0, tile = 0;
   if constexpr (GRID == kByToken) {
     if (place >= T_) return;
     slot = known_slot(pl, __builtin_amdgcn_readfirstlane(place_id));
@@ -157,15 +155,13 @@ __global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int3
       return;
     }
   } else {
-    const int tile = place / slots8;
+    tile = place / slots8;
     slot = place - tile * slots8;
-    first = tile * width;
     if (tile >= tiles) {
       find_tile<kShrinkThreads>(pl, first_id, place - tiles * slots8, reinterpret_cast<int*>(s_stage), s_found);
       slot = __builtin_amdgcn_readfirstlane(s_found[0]);
       if (slot < 0) return;
-      first = __builtin_amdgcn_readfirstlane(s_found[1]);
-      width = MLORA_TILE_SMALL;
+      tile = __builtin_amdgcn_readfirstlane(s_found[1]);
     } else if (slot >= num_slots) {
       if (slot == num_slots && tile == 0) {  // the tokens without a slot
         for (int e = tid; e < T_ * RW; e += kShrinkThreads) {
@@ -191,7 +187,8 @@ __global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int3
   };
   request_a(0);
   __builtin_amdgcn_sched_barrier(0);
-  const int left = list_tile<kShrinkThreads>(pl, first_id, slot, from, first, width, s_rows, s_wave);
+  const int* rows;
+  const int left = list_tile<kShrinkThreads, GRID>(pl, first_id, slot, from, tile, s_rows, s_wave, rows);
   if (left == 0) {
     // (named as used here too, or the compiler sinks the requests behind the listing of the tokens)
 #pragma unroll
@@ -203,7 +200,7 @@ __global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int3
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int at = 4 * i + lg < left ? 4 * i + lg : left - 1;
-    xrow[i] = static_cast<const T*>(x) + static_cast<int64_t>(s_rows[at]) * p.xs + wave * (rounds * 128) + lr * 8;
+    xrow[i] = static_cast<const T*>(x) + static_cast<int64_t>(rows[at]) * p.xs + wave * (rounds * 128) + lr * 8;
   }
   f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
   for (int now = 0; now < rounds; now += CH) {
@@ -247,7 +244,7 @@ __global__ __launch_bounds__(kShrinkThreads) void group_shrink_kernel(const int3
     float sum = 0.f;
 #pragma unroll
     for (int w = 0; w < kShrinkWaves; ++w) sum += s_red[(w * 64 + (tok >> 2) * 16 + rank) * 4 + (tok & 3)];
-    store_as(p.out, out0 + static_cast<int64_t>(s_rows[tok]) * r + r0 + rank, sum * p.scaling, p.out_dtype);
+    store_as(p.out, out0 + static_cast<int64_t>(rows[tok]) * r + r0 + rank, sum * p.scaling, p.out_dtype);
   }
 }
 
@@ -288,10 +285,11 @@ template <typename T, typename H> __device__ __forceinline__ Pack8 load_h(const 
 
 // y[t, col_i + n] (+)= round_T(h[i, t] . B_i[s]^T); grid (8, column ranges, places / 8).  A wavefront takes SP spans of 64 columns.
 template <typename T, typename H, int KSTEPS, int SP, int GRID>
-__global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width_, int slots8,
+__global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int32_t* __restrict__ tts, int T_, int num_slots, int width, int slots8,
                                                                       int tiles, int r, GroupExpandParams p) {
-  const Places pl{tts, T_, num_slots, width_, slots8, tiles};
-  __shared__ int s_hist[GRID == kBySlot ? MLORA_MAX_SLOTS : 1], s_rows[MLORA_TILE_SMALL], s_wave[2 * kExpandWaves], s_found[2];
+  const Places pl{{T_, num_slots, width, slots8, tiles}, tts};
+  __shared__ int s_hist[GRID == kBySlot ? MLORA_MAX_SLOTS : 1], s_rows[(GRID == kBySlot ? 2 : 1) * MLORA_TILE_SMALL], s_wave[2 * kExpandWaves],
+      s_found[2];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;
   const int place = blockIdx.z * 8 + blockIdx.x;
@@ -300,21 +298,19 @@ __global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int3
   int slice = 0;
   while (slice + 1 < p.num_slices && static_cast<int>(blockIdx.y) >= p.first[slice + 1]) ++slice;
   const int n = p.n[slice], c0 = ((static_cast<int>(blockIdx.y) - p.first[slice]) * kExpandWaves + wave) * (SP * 64);
-  int slot, from = 0, first = 0, width = width_;
+  int slot, from = 0, tile = 0;
   if constexpr (GRID == kByToken) {
     if (place >= T_) return;
     slot = known_slot(pl, __builtin_amdgcn_readfirstlane(place_id));
     from = place;
   } else {
-    const int tile = place / slots8;
+    tile = place / slots8;
     slot = place - tile * slots8;
-    first = tile * width;
     if (tile >= tiles) {
       find_tile<kExpandThreads>(pl, first_id, place - tiles * slots8, s_hist, s_found);
       slot = __builtin_amdgcn_readfirstlane(s_found[0]);
       if (slot < 0) return;
-      first = __builtin_amdgcn_readfirstlane(s_found[1]);
-      width = MLORA_TILE_SMALL;
+      tile = __builtin_amdgcn_readfirstlane(s_found[1]);
     }
   }
   if (slot >= num_slots) return;
@@ -333,7 +329,8 @@ __global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int3
       }
     }
   __builtin_amdgcn_sched_barrier(0);
-  const int left = list_tile<kExpandThreads>(pl, first_id, slot, from, first, width, s_rows, s_wave);
+  const int* rows;
+  const int left = list_tile<kExpandThreads, GRID>(pl, first_id, slot, from, tile, s_rows, s_wave, rows);
   if (left == 0 || c0 >= n) {
     // (named as used here too, or the compiler sinks the requests behind the listing of the tokens)
 #pragma unroll
@@ -351,7 +348,7 @@ __global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int3
   Pack8 hop[KSTEPS];
   {
     const int tok = 4 * (lr & 3) + (lr >> 2);
-    const H* row = hin + static_cast<int64_t>(s_rows[tok < left ? tok : left - 1]) * r;
+    const H* row = hin + static_cast<int64_t>(rows[tok < left ? tok : left - 1]) * r;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       const int piece = lg + 4 * ks;
@@ -360,7 +357,7 @@ __global__ __launch_bounds__(kExpandThreads) void group_expand_kernel(const int3
   }
   int row[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) row[i] = s_rows[4 * i + lg < left ? 4 * i + lg : left - 1];
+  for (int i = 0; i < 4; ++i) row[i] = rows[4 * i + lg < left ? 4 * i + lg : left - 1];
   uint2 yq[SP][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -424,24 +421,6 @@ const GroupKnobs& group_knobs() {
 }
 
 constexpr int kMostTokens = 4096;  // of a call (every workgroup reads the slot vector)
-
-int groups_about(int tokens, int slots) { return tokens < slots ? tokens : slots; }  // slots with tokens, at most
-
-// Fills in how a launch of `parts` workgroups per tile is laid out; returns its places.  extra: places for the tokens without a slot.
-int lay_out(Places& p, int* over, long long parts, int extra) {
-  const int groups = groups_about(p.T, p.num_slots);
-  // tiles of four tokens while that many workgroups find room on the chip, else eight, else sixteen
-  p.width = 4;
-  while (p.width < 16 && parts * groups * (1 + p.T / (groups * p.width)) > 256) p.width *= 2;
-  // over the tokens where slots without any would be most of the places
-  *over = p.T <= p.num_slots ? kByToken : kBySlot;
-  p.slots8 = p.tiles = 0;
-  if (*over == kByToken) return p.T;
-  p.slots8 = (p.num_slots + extra + 7) & ~7;
-  p.tiles = 1 + p.T / (p.num_slots * p.width);
-  const int covered = p.tiles * p.width;
-  return p.slots8 * p.tiles + (p.T > covered ? (p.T - covered + MLORA_TILE_SMALL - 1) / MLORA_TILE_SMALL : 0);
-}
 
 struct ShrinkLaunch {
   const MloraShrinkArgs* a;

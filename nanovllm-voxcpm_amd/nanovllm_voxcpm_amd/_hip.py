@@ -76,7 +76,7 @@ EXPORTS = (
 
 # include/mlora_diag.h: measurement and test aids.  The product library exports the first only; the
 # diag and trace variants export all three.
-DIAG_EXPORTS = ("mlora_reload_knobs", "mlora_probe_launch", "mlora_trace_set")
+DIAG_EXPORTS = ("mlora_reload_knobs", "mlora_probe_launch", "mlora_trace_set", "mlora_group_layout")
 DIAG_LIB_NAME = "libmlora_gfx950_diag.so"
 
 
@@ -268,6 +268,9 @@ def _declare_diag(lib: C.CDLL) -> None:
     if hasattr(lib, "mlora_trace_set"):
         lib.mlora_trace_set.argtypes = [C.c_void_p]
         lib.mlora_trace_set.restype = C.c_int
+    if hasattr(lib, "mlora_group_layout"):
+        lib.mlora_group_layout.argtypes = [C.c_int32, C.c_int32, C.c_int64, C.c_int32, C.c_int32, C.POINTER(C.c_int32)]
+        lib.mlora_group_layout.restype = None
 
 
 _DIAG_LIB: C.CDLL | None = None

@@ -1,6 +1,7 @@
 """The low-level shrink and expand over tiles of a slot (csrc/group.hip) at the sizes where they can go wrong: one token,
-tiles just filled and one over, more tokens of a slot than it has places for, slots without tokens, ids that name no slot, grids over
-the slots and over the tokens, ranks that are no multiple of eight (shrink) or of a block, ragged and tiny slices, every element type."""
+tiles just filled and one over, more tokens of a slot than it has places for, many slots just above that, slots without tokens, ids that
+name no slot, grids over the slots and over the tokens, ranks that are no multiple of eight (shrink) or of a block, ragged and tiny
+slices, every element type; where the tiles are forced and where the library chooses."""
 
 import random
 
@@ -23,6 +24,7 @@ CASES = [
     (512, 3, 16, 1024, [1024, 256, 256], "one", F16, F32),
     (513, 600, 8, 1024, [72], "even", B16, F32),
     (4096, 3, 48, 1024, [8], "popular", B16, B16),
+    (900, 64, 32, 1024, [512], "even", B16, F32),
 ]
 
 
@@ -39,13 +41,35 @@ def _ids(how: str, tokens: int, slots: int, pick: random.Random) -> list[int]:
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", range(len(CASES)))
 def test_ops_over_tiles_against_fp64(case, monkeypatch):
+    tokens, slots, rank, k, widths, how, dtype, h_dtype = CASES[case]
+    print(f"group ops {CASES[case]}", flush=True)
+    # (the tiles wherever they are possible / one workgroup per token)
+    _check(_ids(how, tokens, slots, random.Random(case)), slots, rank, k, widths, dtype, h_dtype, case, ("2", "0"), monkeypatch)
+
+
+# tokens, slot ids, how many of those are in use (0: every token's slot at random over all of them)
+UNEVEN = [(64, 32, 9), (300, 64, 25), (255, 64, 0), (208, 64, 0), (96, 32, 0), (130, 24, 9)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank,widths,dtype", [(32, [1024], B16), (64, [1024], F16), (32, [1024, 256, 256], F16), (64, [2048, 2048], B16)])
+@pytest.mark.parametrize("tokens,slots,used", UNEVEN)
+def test_uneven_batches_where_the_library_chooses(tokens, slots, used, rank, widths, dtype, monkeypatch):
+    """Many slots with a token or two more than their own tiles hold at the narrow width."""
+    print(f"group ops {(tokens, slots, used, rank, widths, dtype)}", flush=True)
+    pick = random.Random(tokens)
+    ids = [(t % used) * (slots // used) if used else pick.randrange(slots) for t in range(tokens)]
+    pick.shuffle(ids)
+    _check(ids, slots, rank, 1024, widths, dtype, F32, tokens, (None,), monkeypatch)
+
+
+def _check(ids, slots, rank, k, widths, dtype, h_dtype, seed, uses, monkeypatch):
+    """Shrink into a buffer of NaN and expand, with MLORA_GROUP as each of `uses` (None: unset), against fp64."""
     from nanovllm_voxcpm_amd import _hip
     from nanovllm_voxcpm_amd.lora_ops import lora_expand, lora_shrink
 
-    tokens, slots, rank, k, widths, how, dtype, h_dtype = CASES[case]
-    print(f"group ops {CASES[case]}", flush=True)
-    pick, g = random.Random(case), torch.Generator().manual_seed(case)
-    ids = torch.tensor(_ids(how, tokens, slots, pick), dtype=torch.int32)
+    tokens, g = len(ids), torch.Generator().manual_seed(seed)
+    ids = torch.tensor(ids, dtype=torch.int32)
     x = torch.randn(tokens, k + 8, generator=g).to(dtype)[:, :k]
     a = [(torch.randn(slots, rank, k, generator=g) * 0.05).to(dtype) for _ in widths]
     b = [(torch.randn(slots, n, rank, generator=g) * 0.1).to(dtype) for n in widths]
@@ -55,8 +79,8 @@ def test_ops_over_tiles_against_fp64(case, monkeypatch):
     slot = torch.where(known, ids, torch.zeros_like(ids)).long()
     got = {}
     try:
-        for use in ("2", "0"):  # the tiles wherever they are possible / one workgroup per token
-            monkeypatch.setenv("MLORA_GROUP", use)
+        for use in uses:
+            monkeypatch.setenv("MLORA_GROUP", use) if use else monkeypatch.delenv("MLORA_GROUP", raising=False)
             _hip.load().mlora_reload_knobs()
             out = torch.full((len(widths), tokens, rank), float("nan"), dtype=h_dtype, device="cuda")
             lora_shrink(x.cuda(), [t.cuda() for t in a], out, ids.cuda(), None, None, None, None, False, 0, 0.5)
