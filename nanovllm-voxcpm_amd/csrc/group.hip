@@ -475,24 +475,38 @@ template <typename T> void expand_type(const ExpandLaunch& l) {
 
 }  // namespace
 
-// Where tiles of a slot beat one workgroup per token.  What a token's workgroup costs grows with the A rows it takes in, so from rank 32
-// on the tiles are the faster ones at every size; below, the listing of the tokens (0.5 us) has to be earned.  Replayed graphs, us per call,
-// per token / tiles: rank 32 and 64, K = 1024, one token: 4.3 / 3.7 and 6.7 / 3.7, 130 tokens over 64 slots, three slices: 7.0 / 5.9 and
-// 11.7 / 9.2, K = 8192, 37 tokens: 15.3 / 7.9 (rank 32) and 41 / 12.5.  Rank 16 by tokens x slices x rank x K in millions: 0.6:
-// 3.4 / 3.8, 4.2: 4.2 / 4.4, 6.4: 4.8 / 4.8, 8.4: 4.75 / 4.75, 12.6 (256 tokens over 32 slots, three slices): 5.4 / 4.4, 25: 7.7 / 4.7; with
-// long K earlier: K = 4096, 2.4: 6.1 / 5.4, K = 8192, 1.2: 8.1 / 7.5; rank 8 alike (0.3 at K = 4096: 4.3 / 5.3).  Beyond 512 tokens every workgroup reads the slot
-// vector in several steps (1000 tokens over 4 slots, rank 64, three slices: 19 / 26).
+// Where tiles of a slot beat one workgroup per token.  What a token's workgroup costs grows with the A rows it takes in; what a tile's
+// costs is finding its tokens (0.5 us), and rounds once places x slices are more workgroups than the chip takes together or, with few
+// slot ids, than their XCDs take (a slot's workgroups share one).  Replayed graphs, slots at random, us per call, per token / tiles:
+//  - above rank 16, over the tokens: rank 32, K = 1024, one slice 64 tokens 5.5 / 4.9, 128 5.7 / 5.4, 256 6.3 / 6.9; three slices 32 tokens
+//    5.6 / 5.1, 64 5.9 / 6.5 (rank 64 10.7 / 9.5);
+//  - over the slots: 131 tokens of 128 ids 5.7 / 4.7, three slices 7.5 / 8.9, 259 of 256 11.0 / 13.9, but 512 of 256 16.4 / 15.5, 384 of 192
+//    13.4 / 12.6; K = 4096 195 of 192 14.7 / 17.6; 403 of 400, one slice 0.73-0.87 of the per-token rate;
+//  - few ids: one 48 tokens 4.52 / 4.51, 64 4.6 / 4.8, three slices 64 4.7 / 10.2 (rank 64, 512 tokens 12 / 39); two 48 tokens of three slices
+//    5.6 / 6.3; four, rank 64, 512 tokens of three slices 12.5 / 14.6; eight 7.8 / 6.7;
+//  - beyond 512 tokens every workgroup reads the slot vector in several steps (1000 tokens over 4 slots, rank 64, three slices: 19 / 26);
+//  - up to rank 16, K = 1024: one slice 512 tokens of 8 ids 4.2 / 4.8, of 16 4.4 / 4.2; three slices 256 of 8 4.55 / 4.9, of 16 4.9 / 4.4, of
+//    128 6.2 / 5.9, 192 of 128 5.75 / 5.96, 256 of 256 6.6 / 9.5 (rank 8 as from twice the tokens);
+//  - K = 4096: 64 tokens of 64 ids 6.3 / 6.6, 192 of 8 6.5 / 5.75, 256 of 8 6.6 / 9.2, 48 of 2 5.3 / 5.6, 64 of one 4.7 / 6.7; K = 8192: 64 of 64
+//    9.1 / 8.8, 128 of 128 12.75 / 11.7.
+// The slots of a batch are not known here: with all tokens on one slot of 16 the tiles lose (rank 32, K = 1024, 384 tokens 5.0 / 6.0; at
+// random 6.0 / 4.9; rank 16, three slices, 256 tokens 4.2 / 5.7 and 4.9 / 4.4).
+static bool shrink_tiles_pay(int T, int L, int S, int r, int k) {
+  if (T > 512) return false;
+  const int spread = S * (T <= L ? T : L);
+  if (r > 16) return T <= L ? spread <= 128 : (spread <= 128 || T >= 2 * L) && (L >= 8 || T * S <= 48 * L);
+  if (static_cast<double>(T) * S * r * k < (k >= 4096 ? 1.2e6 : 9.0e6)) return false;
+  if (T <= L) return k >= 8192 && spread <= 128;
+  return (spread <= 64 || T >= 2 * L) && (L >= 16 || (k >= 4096 && L >= 3 && T <= 24 * L));
+}
+
 bool group_shrink_supported(const MloraShrinkArgs* a) {
   if (group_knobs().use == 0 || a->dtype == MLORA_DTYPE_F32 || a->num_slots < 1 || a->num_slots > MLORA_MAX_SLOTS || a->num_tokens > kMostTokens) return false;
   if (a->r < 1 || a->r > 64 || a->k < kRound || a->k % kRound || a->x_stride % 8 || !aligned(a->x, 16)) return false;
   for (int i = 0; i < a->num_slices; ++i)
     if (!aligned(a->a[i], 16)) return false;
   if (group_knobs().use == 2) return true;
-  if (a->r <= 16) {
-    const double cells = static_cast<double>(a->num_tokens) * a->num_slices * a->r * a->k;
-    if (cells < (a->k >= 4096 ? 1.2e6 : 7.0e6) || a->num_tokens > 64 * a->num_slots) return false;
-  }
-  return a->num_tokens <= 512;
+  return shrink_tiles_pay(a->num_tokens, a->num_slots, a->num_slices, a->r, a->k);
 }
 
 int launch_group_shrink(const MloraShrinkArgs* a) {
@@ -511,12 +525,33 @@ int launch_group_shrink(const MloraShrinkArgs* a) {
   return check_launch("mlora_shrink");
 }
 
-// Measured as above, per token / tiles: rank 16, 1024 columns: one token 3.1 / 2.9, 256 over 32 slots 4.4 / 3.3, 512 over 64 5.6 / 4.4;
-// 8192 columns: 256 over 32 10.8 / 6.4; rank 64: one token 6.0 / 3.2, 130 over 64, 8192 columns 120 / 16, 512 over 64 349 / 20.
-// Not where a grid over the tokens would be mostly workgroups that leave again while B rows are short (rank 16, 8192 columns, 37 tokens of 64
-// slots: 5.4 / 6.1; 16384: 7.3 / 8.7), nor at rank 8 except for many tokens of many slots (512 over 64: 12.6 / 8.3, over 4 slots
-// 9.1 / 9.7), nor, up to rank 16, beyond 64 tokens per slot id or 1024 in all (512 over 4, 1024 columns: 4.0 / 4.6; 1000 over 32 6.2 / 7.0,
-// 8192 columns 29 / 16; 4096 over 32 14.2 / 17.3).  All tokens on one slot of many: 512 tokens, 24 slots, rank 16 3.9 / 5.4, rank 64 17.7 / 6.9.
+// Measured as above, per token / tiles; columns: of all slices.
+//  - rank 8: 8192 columns 256 tokens of 8 ids 6.6 / 5.1, of 128 9.0 / 9.2, 512 of 128 14.6 / 12.8; 1536 columns 512 of 32 4.80 / 4.82; fewer
+//    tokens or columns lose 2 to 15 %;
+//  - rank 16: 256 columns never (256 tokens of 64 3.2 / 3.4).  Over the tokens: 1024 columns 64 tokens 3.65 / 3.42, 128 4.1 / 4.2, 256 4.7 / 5.3; 8192
+//    columns 64 5.9 / 7.5.  One id: 1024 columns 32 tokens 3.4 / 3.3, 64 3.44 / 3.78; 8192 64 4.6 / 7.4; three, 2048 columns 96 0.87 of
+//    the per-token rate.  Four: 1024 columns 128 tokens 3.50 / 3.55, 256 3.6 / 3.7; 8192 512 14.0 / 13.1.  1024 of 128 ids at 1024 columns
+//    0.90 of the per-token rate, 512 of 256 at 8192 24.4 / 25.6, 1024 of 256 39.4 / 33.6;
+//  - above, over the tokens: rank 24 256 of 256 ids 256 columns 3.9 / 3.65, 512 of 512 4.6 / 5.1 (1024 columns 8.1 / 7.8; 1024 tokens 14.5 / 15.6);
+//  - one id, rank 32: 1024 columns 64 tokens 4.2 / 3.9, 192 4.7 / 6.5; rank 24 to 48, of the per-token rate, 1536 columns 32 tokens 1.05-1.14, 48
+//    0.94-1.01, 3072 columns 48 tokens 0.78-0.82, 4096 columns 16 1.03-1.17, 32 0.86; rank 24 8192 columns 4096 tokens 170 / 510.  Rank 56 1.05 to 2.1
+//    from 1536 columns on; rank 64 256 columns 512 tokens 6.3 / 7.6, 1024 18.5 / 10.4, 8192 4096 tokens 990 / 750;
+//  - more ids: rank 32 1024 columns 2048 tokens of 2 19.4 / 20.4, 1024 of 2 11.6 / 9.3; rank 24 256 columns 512 of 2 3.85 / 4.3, 4096 of 16
+//    11.4 / 14.4, of 64 11.8 / 10.5; 8192 columns 4096 of 4 185 / 164; rank 64, 4096 of 64, 1800 / 119.
+// All tokens on one slot of many: rank 24, 1024 columns, 512 tokens of 64 5.2 / 5.9, 8192 columns 21.9 / 13.8.
+static bool expand_tiles_pay(int T, int L, int r, long long cols) {
+  if (r <= 8) return cols >= 4096 && L >= 8 && L <= 128 && T >= 256 && T >= 4 * L && T <= 1024;
+  if (r <= 16) {
+    if (cols < 1024) return false;
+    if (T <= L) return T * cols <= 65536;
+    if (L < 4) return T * cols <= 32768;
+    return T <= 1024 && T <= L * (cols >= 4096 ? 128 : 32) && (L <= 64 || (cols > 1024 && T >= 4 * L));
+  }
+  if (T <= L) return r > 32 || T <= (cols >= 1024 ? 512 : 256);
+  if (L == 1) return r > 48 ? T <= 64 || cols >= 1024 : T <= 64 && T * cols <= 65536;
+  return T <= 64 * L || r > 56 || (T <= 1024 * L && r * cols >= 32768);
+}
+
 bool group_expand_supported(const MloraExpandArgs* a) {
   if (group_knobs().use == 0 || a->dtype == MLORA_DTYPE_F32 || a->num_slots < 1 || a->num_slots > MLORA_MAX_SLOTS || a->num_tokens > kMostTokens) return false;
   if (a->r < 8 || a->r > 64 || a->r % 8 || a->y_stride % 4 || a->offset_start % 4 || !aligned(a->y, 8) || !aligned(a->h, 16)) return false;
@@ -527,10 +562,7 @@ bool group_expand_supported(const MloraExpandArgs* a) {
   }
   if (cols > 1 << 23) return false;  // (column ranges of the grid)
   if (group_knobs().use == 2) return true;
-  if (a->r <= 8 && !(a->num_tokens >= 256 && a->num_slots >= 16)) return false;
-  if (a->r > 16) return true;
-  if (a->num_tokens <= a->num_slots && cols >= 8192) return false;
-  return a->num_tokens <= 1024 && a->num_tokens <= 64 * a->num_slots;
+  return expand_tiles_pay(a->num_tokens, a->num_slots, a->r, cols);
 }
 
 int launch_group_expand(const MloraExpandArgs* a) {
