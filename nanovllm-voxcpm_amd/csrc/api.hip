@@ -206,8 +206,10 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double per_slot = 2.0 * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
   if (a->num_slots * per_slot <= 3.0e6) return true;
-  // Where A[slot] and B[slot] are light the line lies at two tokens per slot id: 64 tokens of 32 ids at random, us per call, slot-major /
-  // tile-major: rank 16 qkv 3.8 / 4.0, gate_up 5.1 / 5.3; rank 32 o 4.3 / 4.5, but gate_up 7.5 / 7.4; rank 64 qkv 7.9 / 7.5, o 6.0 / 5.8.
+  // Where A[slot] and B[slot] are light the line lies at two tokens per slot id: tokens at random, us per call, slot-major / tile-major:
+  // 64 of 32 ids, rank 16 qkv 3.68 / 3.82, gate_up 4.91 / 5.00, rank 8 gate_up 4.51 / 4.74, rank 24 o 4.33 / 4.61, rank 32 o 4.17 / 4.31, but gate_up
+  // 7.5 / 7.4, rank 64 qkv 7.9 / 7.5, o 6.0 / 5.8; 128 of 64, rank 8 gate_up 7.20 / 7.38, rank 16 o 3.61 / 3.86, gate_up 8.03 / 8.24, rank 24 o 4.45 /
+  // 4.70, rank 32 o 4.46 / 4.51.  At two, three and 3.9 tokens of 12 to 64 ids, ranks 8 to 32, 69 of 69 such calls are 0.4 to 7 % faster.
   const bool light = a->k == 1024 && (compute_rank(a->r) <= 16 || (compute_rank(a->r) == 32 && a->num_slices == 1 && cols <= 2048));
   return a->num_tokens >= (light ? 2 : 4) * a->num_slots;
 }
@@ -386,7 +388,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "
-                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or (2048, 4096 and 8192) with one slice of at most 4096 columns and an "
+                    "ranges of at most 512 columns), or K = 4096 with rank <= 16 or (2048, 4096 and 8192; 2048 at rank 64 with three too) with one slice of at most 4096 columns and an "
                     "initialised workspace");
           return MLORA_E_UNSUPPORTED;
         }

@@ -826,8 +826,8 @@ Parts k_parts(const MloraAddArgs* a) {
 
 // K = 1024 at every rank; one slice of K = 2048, 4096 and 8192 at every rank with the K parts of a tile shared out between its
 // workgroups, K = 4096 without up to rank 16 (what fits the register file as one batch of loads); one or two
-// slices with their pointers as arguments, three (K = 1024) with the later two's as offsets from
-// the first one's; 16-bit elements.
+// slices with their pointers as arguments, three (K = 1024 at the exact ranks, K = 2048 in K parts at rank 64) with the later
+// two's as offsets from the first one's; 16-bit elements.
 bool slot_supported(const MloraAddArgs* a) {
   if (a->dtype != MLORA_DTYPE_BF16 && a->dtype != MLORA_DTYPE_F16) return false;
   if (a->num_slices < 1 || a->num_slices > 3 || !a->plan) return false;
@@ -840,8 +840,8 @@ bool slot_supported(const MloraAddArgs* a) {
   if (!padded_rank(a->r)) return false;
   const int kspw = kspw_of(a);
   if (a->num_slices == 3) {
-    // q | k | v: K = 1024, an exact rank, offsets that fit 40 bits, widths that fit 16-bit counts of
-    // eight columns, and column ranges of at most 512 columns (one span per wavefront)
+    // q | k | v: an exact rank, offsets that fit 40 bits, widths that fit 16-bit counts of eight columns; K = 1024
+    // with column ranges of at most 512 columns (one span per wavefront), or K = 2048 at rank 64 in K parts
     long long ao, bo;
     if (!exact_rank(a->r) || !offsets16(a, 1, &ao, &bo) || !offsets16(a, 2, &ao, &bo)) return false;
     for (int i = 0; i < 3; ++i)

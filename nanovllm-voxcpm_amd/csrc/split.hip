@@ -472,8 +472,7 @@ __global__ __launch_bounds__(kNT) void split_kernel(const int32_t* __restrict__ 
 // the signature.
 __global__ __launch_bounds__(256) void workspace_init_kernel(uint32_t* ws) {
   const int words = MLORA_WORKSPACE_HEAD_BYTES / 4;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
-    {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) {
     uint32_t v = i == 0 ? kWsMagic : 0u;
     for (int x = 0; x < 8; ++x)
       if (i == ws_state_word(x) + 2) v = kWsGenCheck;  // generation 0's check word
@@ -524,10 +523,10 @@ struct SplitKnobs {
     generation = knob_generation();
     w = env_int("MLORA_SPLIT_W", 0);
     spin_ticks = env_int("MLORA_SPLIT_SPIN_TICKS", 20000);  // 200 us of the 100 MHz clock; negative: never accept published sums
-    // loads and the arrival counts at device scope, stores in the L2 of the XCD on which every
-    // workgroup of a tile runs: were a tile ever spread over XCDs, its consumers would not see the
-    // stores, give up waiting and compute for themselves, and the generations would still advance
-    wide = env_int("MLORA_SPLIT_WIDE", 5);
+    // loads at device scope, stores in the L2 of the XCD on which every workgroup of a tile runs: were a
+    // tile ever spread over XCDs, its consumers would not see the stores, give up waiting and compute for
+    // themselves, and the generations (reported at device scope always) would still advance
+    wide = env_int("MLORA_SPLIT_WIDE", 1);
     sym = env_int("MLORA_SPLIT_SYM", -1);    // -1: symmetric roles when a tile's shrink has four or more K parts
     kpart = env_int("MLORA_SPLIT_KPART", 0);
   }
