@@ -234,8 +234,9 @@ PyObject* given(PyObject* o, PyObject* name) {
 // The first call of a step: what the Python path looks up for it (HipLoRABackend._plan_for, known_active_slots), where
 // the metadata's own slot vector of exactly these rows carries the plan of the launch that made it
 // (segment_meta.attach_plan) and has not been rewritten since.  The state holds the three objects from then
-// on.  Eager calls only.  In Python this lookup cost 15 us of every step (passes back to back on one host: sixteen calls in
-// fp32 134 us, 119 with this; sixteen linears of 1234 tokens 500, 479).
+// on, until the next step, forget_step or its own end.  Eager calls only.  In Python this lookup cost 15 us of every step on one fast
+// host (passes back to back: sixteen calls in fp32 134 us, 119 with this; sixteen linears of 1234 tokens 500, 479); on another host, paced by its
+// launches, the difference was within two runs' (172.4, 172.9 and 537, 528).
 bool take_step(State* s, const Site& site, PyObject* metadata, PyObject* source_obj, const at::Tensor& source, uint32_t version, void* stream, int64_t rows) {
   static PyObject* const kPlan = PyUnicode_InternFromString("_mlora_plan");
   static PyObject* const kCapacity = PyUnicode_InternFromString("_mlora_capacity");
