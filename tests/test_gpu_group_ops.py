@@ -60,7 +60,7 @@ def test_uneven_batches_where_the_library_chooses(tokens, slots, used, rank, wid
     pick = random.Random(tokens)
     ids = [(t % used) * (slots // used) if used else pick.randrange(slots) for t in range(tokens)]
     pick.shuffle(ids)
-    _check(ids, slots, rank, 1024, widths, dtype, F32, tokens, (None,), monkeypatch)
+    _check(ids, slots, rank, 1024, widths, dtype, F32, tokens, (None, "2"), monkeypatch)  # the library's choice, and the tiles wherever that lies
 
 
 def _check(ids, slots, rank, k, widths, dtype, h_dtype, seed, uses, monkeypatch):
