@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kShrinkWaves* kWave, 2) void sgmv_shrink_kernel(con
 #endif
 }
 
-template <typename T, int R, int CPL, int TPF, int G>
+template <typename T, int R, int CPL, int TPF, int G, bool STREAM>
 __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws,
                                                                              void* __restrict__ yv_, int64_t ys, int big_off, int small_off,
                                                                              int big_units, int bigrows_off, int T_, int num_slots,
@@ -154,10 +154,10 @@ __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(con
 #pragma unroll
   for (int g = 0; g < G; ++g) masked |= m[g] > 0 && eff[g] < R;
   if (masked)
-    expand_body<T, R, CPL, TPF, G, true>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, true, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
                                          m, eff, rowv);
   else
-    expand_body<T, R, CPL, TPF, G, false>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, false, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
                                           m, eff, rowv);
 }
 
@@ -200,29 +200,31 @@ void launch_shrink_rank(const ShrinkLaunch& l, int kr, int xw) {
 
 template <typename T, int R>
 void launch_expand_group(const MloraAddArgs* a, const PlanLayout& lay, int big_units, dim3 grid, int ksplit, int cpl, int group,
-                         const ExpandSplits& sp) {
+                         bool stream, const ExpandSplits& sp) {
   hipStream_t st = static_cast<hipStream_t>(a->stream);
   const float* h = partials_of(a);
-#define MLORA_EXPAND(CPL_, TPF_, G_)                                                                                       \
-  hipLaunchKernelGGL((sgmv_expand_kernel<T, R, CPL_, TPF_, G_>), grid, dim3(kExpandWaves* kWave), 0, st, a->plan, h, a->y, \
+#define MLORA_EXPAND(CPL_, TPF_, G_, S_)                                                                                       \
+  hipLaunchKernelGGL((sgmv_expand_kernel<T, R, CPL_, TPF_, G_, S_>), grid, dim3(kExpandWaves* kWave), 0, st, a->plan, h, a->y, \
                      a->y_stride, lay.big_off, lay.small_off, big_units, lay.bigrows_off, a->num_tokens, a->num_slots,      \
                      a->num_slices, ksplit, a->scaling, a->effective_rank, sp)
   if (cpl == 4) {
-    if (group == 4) MLORA_EXPAND(4, 4, 4); else if (group == 2) MLORA_EXPAND(4, 4, 2); else MLORA_EXPAND(4, 4, 1);
+    if (group == 4) MLORA_EXPAND(4, 4, 4, false); else if (group == 2) MLORA_EXPAND(4, 4, 2, false); else MLORA_EXPAND(4, 4, 1, false);
+  } else if (stream) {
+    if (group == 2) MLORA_EXPAND(8, 2, 2, true); else MLORA_EXPAND(8, 2, 1, true);
   } else {
-    if (group == 4) MLORA_EXPAND(8, 2, 4); else if (group == 2) MLORA_EXPAND(8, 2, 2); else MLORA_EXPAND(8, 2, 1);
+    if (group == 4) MLORA_EXPAND(8, 2, 4, false); else if (group == 2) MLORA_EXPAND(8, 2, 2, false); else MLORA_EXPAND(8, 2, 1, false);
   }
 #undef MLORA_EXPAND
 }
 
 template <typename T>
 void launch_expand_rank(const MloraAddArgs* a, const PlanLayout& lay, int big_units, dim3 grid, int ksplit, int cpl, int group,
-                        const ExpandSplits& sp) {
+                        bool stream, const ExpandSplits& sp) {
   switch (a->r) {
-    case 8: launch_expand_group<T, 8>(a, lay, big_units, grid, ksplit, cpl, group, sp); break;
-    case 16: launch_expand_group<T, 16>(a, lay, big_units, grid, ksplit, cpl, group, sp); break;
-    case 32: launch_expand_group<T, 32>(a, lay, big_units, grid, ksplit, cpl, group, sp); break;
-    default: launch_expand_group<T, 64>(a, lay, big_units, grid, ksplit, cpl, group, sp); break;
+    case 8: launch_expand_group<T, 8>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
+    case 16: launch_expand_group<T, 16>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
+    case 32: launch_expand_group<T, 32>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
+    default: launch_expand_group<T, 64>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
   }
 }
 
@@ -266,8 +268,8 @@ int launch_sgmv(const MloraAddArgs* a) {
   if (rc) return rc;
 
   dim3 grid(8, static_cast<unsigned>(sh.nsplit), static_cast<unsigned>(sh.units / 8));
-  if (a->dtype == MLORA_DTYPE_BF16) launch_expand_rank<__bf16>(a, sh.lay, sh.big_units, grid, sh.ksplit, sh.cpl, sh.group, sh.splits);
-  else launch_expand_rank<_Float16>(a, sh.lay, sh.big_units, grid, sh.ksplit, sh.cpl, sh.group, sh.splits);
+  if (a->dtype == MLORA_DTYPE_BF16) launch_expand_rank<__bf16>(a, sh.lay, sh.big_units, grid, sh.ksplit, sh.cpl, sh.group, sh.stream, sh.splits);
+  else launch_expand_rank<_Float16>(a, sh.lay, sh.big_units, grid, sh.ksplit, sh.cpl, sh.group, sh.stream, sh.splits);
   return check_launch("mlora_add_lora(sgmv expand)");
 }
 

@@ -16,6 +16,13 @@ MLORA_TRACE_DECL
 constexpr int kMaxSplits = 64;
 constexpr int kExpandWaves = 4;
 constexpr int kSlabStages = 4;  // 128-byte pieces of K in a part of slab.hip's at least
+// Bytes of y from which on the expand launch touches it with the non-temporal hint, plain / with it.  The launch by itself,
+// gate_up, us per call: rank 64 9392 tokens (154 MB) 62.9 / 56.4, 6500 (106 MB) 55.2 / 50.7, 5000 (82 MB) 58.3 / 51.5, rank 16 3001
+// tokens x 16384 columns (98 MB) 51.8 / 44.8; mixed batch of 8192 tokens 97.6 / 90.2: a read-modify-write stream at 4.1 -> 4.6
+// TB/s, gate_up's expand at 4.8 -> 5.4.  Between a copy that writes y and one that reads it (all three, us): 131 MB 154.6 / 150.0, 124 MB
+// 143.9 / 136.3, 106 MB 123.2 / 123.8, 82 MB 106.5 / 108.7, and below, where the memory-side cache still holds what the launch
+// before has written, it costs what it gains or more (19 MB: 43.8 / 44.9).  Hint on the loads only 60.9, on the stores only 62.7.
+constexpr long long kStreamBytes = 80ll << 20;
 constexpr int kMaxKSplit = 4;  // most K parts the shrink ever uses (the workspace has room for them)
 
 struct ShrinkSlices {
@@ -432,13 +439,16 @@ template <int N> struct YRaw;
 template <> struct YRaw<4> { typedef u32x2 type; };
 template <> struct YRaw<8> { typedef u32x4 type; };
 
-// y is touched once per launch (a non-temporal hint on its accesses measured no gain).  An item
+// y is touched once per launch.  STREAM: its loads and stores carry the non-temporal hint (kStreamBytes says when
+// and what it gives).  An item
 // stays the raw vectors it was fetched as until it is used: unpacked where it is requested, its
 // arithmetic is scheduled ahead of the barrier that ends the staging of the intermediate, and the
 // wavefront waits for the item in front of work that could have run meanwhile.
-template <typename T, int N>
+template <typename T, int N, bool STREAM>
 __device__ __forceinline__ typename YRaw<N>::type load_y(const T* p) {
-  return *reinterpret_cast<const typename YRaw<N>::type*>(p);
+  const typename YRaw<N>::type* q = reinterpret_cast<const typename YRaw<N>::type*>(p);
+  if constexpr (STREAM) return __builtin_nontemporal_load(q);
+  else return *q;
 }
 template <typename T, int N>
 __device__ __forceinline__ YVec<T, N> unpack_y(const typename YRaw<N>::type& r) {
@@ -446,12 +456,13 @@ __device__ __forceinline__ YVec<T, N> unpack_y(const typename YRaw<N>::type& r) 
   __builtin_memcpy(&v, &r, sizeof(r));
   return v;
 }
-template <typename T, int N>
+template <typename T, int N, bool STREAM>
 __device__ __forceinline__ void store_y(T* p, const YVec<T, N>& v) {
   typedef typename YRaw<N>::type Raw;
   Raw r;
   __builtin_memcpy(&r, &v, sizeof(r));
-  *reinterpret_cast<Raw*>(p) = r;
+  if constexpr (STREAM) __builtin_nontemporal_store(r, reinterpret_cast<Raw*>(p));
+  else *reinterpret_cast<Raw*>(p) = r;
 }
 
 // Body of the expand for the tiles of one workgroup.  MASKED: some tile's slot holds an adapter of
@@ -464,7 +475,7 @@ __device__ __forceinline__ void store_y(T* p, const YVec<T, N>& v) {
 // caches): they were written by other workgroups of the same launch.
 //
 // PRE: the intermediate of the (one) tile is in `s_h` already, put there by this workgroup.
-template <typename T, int R, int CPL, int TPF, int G, bool MASKED, bool SC1 = false, bool PRE = false>
+template <typename T, int R, int CPL, int TPF, int G, bool MASKED, bool SC1 = false, bool PRE = false, bool STREAM = false>
 __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict__ s_row, int* __restrict__ s_slot, int* __restrict__ s_m,
                                             int* __restrict__ s_eff, const int32_t* __restrict__ plan, const float* __restrict__ hws,
                                             void* __restrict__ yv_, int64_t ys, int T_, int num_slices, int ksplit,
@@ -573,7 +584,7 @@ __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict
     for (int u = 0; u < TPF; ++u) {
       const i32x4 rows = *reinterpret_cast<const i32x4*>(&s_row[g * MLORA_TILE_BIG + (tp + u) * 16 + 4 * lg]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) buf[u][i] = load_y<T, CPL>(ybase + static_cast<int64_t>(rows[i]) * ys + cl);
+      for (int i = 0; i < 4; ++i) buf[u][i] = load_y<T, CPL, STREAM>(ybase + static_cast<int64_t>(rows[i]) * ys + cl);
     }
   };
   Pack8 bop[CPL][KSTEPS];
@@ -657,7 +668,7 @@ __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict
           YVec<T, CPL> r;
 #pragma unroll
           for (int j = 0; j < CPL; ++j) r.e[j] = from_f32<T>(to_f32(yv.e[j]) + out[j][i]);
-          store_y<T, CPL>(ybase + static_cast<int64_t>(rows[i]) * ys + c, r);
+          store_y<T, CPL, STREAM>(ybase + static_cast<int64_t>(rows[i]) * ys + c, r);
         }
       }
     }
@@ -790,7 +801,7 @@ size_t partials_room(const MloraAddArgs* a) {
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
 struct SgmvKnobs {
-  int generation = -1, kr, ksplit, all_slices, xdb, group, wgs, nt, cpl, slab;
+  int generation = -1, kr, ksplit, all_slices, xdb, group, wgs, nt, cpl, slab, stream;
   void read() {
     generation = knob_generation();
     kr = env_int("MLORA_SGMV_KR", 0);
@@ -801,6 +812,7 @@ struct SgmvKnobs {
     wgs = env_int("MLORA_SGMV_WGS", 2048);
     nt = env_int("MLORA_SGMV_NT", 0);
     cpl = env_int("MLORA_SGMV_CPL", 8);
+    stream = env_int("MLORA_SGMV_STREAM", -1);
     slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay
   }
 };
@@ -849,6 +861,7 @@ struct SgmvShape {
   bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
   int group;      // expand: consecutive 64-token tiles per workgroup
   int cpl;        // expand: columns per lane
+  bool stream;    // expand: y with the non-temporal hint
   int nsplit;     // expand: column ranges
   int big_units;  // expand: groups of 64-token tiles
   int units;      // expand: those plus the short segments
@@ -971,6 +984,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
   s.group = group;
   s.nsplit = fill_splits(a, nt, s.splits.split);
   s.cpl = sgmv_knobs().cpl == 4 ? 4 : 8;
+  s.stream = s.cpl == 8 && group <= 2 && (sgmv_knobs().stream < 0 ? static_cast<long long>(a->num_tokens) * cols * 2 >= kStreamBytes : sgmv_knobs().stream != 0);
   if (one_launch && a->k % 256 == 0) {
     // the unit's workgroups (one per column range) share out its shrink roles (tile, slice, K part):
     // about one role each
