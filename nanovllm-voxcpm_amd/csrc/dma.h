@@ -28,6 +28,14 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t 
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(base) : "memory");
 }
 
+// The same with the non-temporal hint, for lines that no other workgroup asks for.
+__device__ __forceinline__ void dma16_once(const void* base, uint32_t voff, uint32_t lds) {
+#ifdef MLORA_TRACE
+  base = uniform(static_cast<const char*>(base));
+#endif
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(voff), "s"(base) : "memory");
+}
+
 }  // namespace
 
 }  // namespace mlora
