@@ -377,7 +377,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
                   "in steps the kernels have, 16-byte aligned rows and no empty slice");
         return MLORA_E_UNSUPPORTED;
       }
-      return launch_pair(a);
+      return launch_pair(a, active);
     case MLORA_FORM_SGMV:
     case MLORA_FORM_FUSED:
     case MLORA_FORM_SPLIT:

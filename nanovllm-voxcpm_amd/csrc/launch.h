@@ -72,7 +72,8 @@ int launch_wide(const MloraAddArgs* a);
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
 // direct loads; 16- and 32-bit elements.
 bool pair_supported(const MloraAddArgs* a);
-int launch_pair(const MloraAddArgs* a);
+// Under AUTO fp32 takes one launch where that is the faster one (`active`: slots with tokens where the host counted them, else 0).
+int launch_pair(const MloraAddArgs* a, int active);
 
 // group.hip: the low-level shrink and expand over tiles of a slot; `supported` says where they are the faster ones too.
 bool group_shrink_supported(const MloraShrinkArgs* a);

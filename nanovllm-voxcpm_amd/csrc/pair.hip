@@ -53,10 +53,10 @@ template <int NA8> struct ShrinkShape {
   static constexpr int BYTES = NST * ND * 1024;      // of LDS per wavefront
 };
 
-template <typename T, int NA8>
-__device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
-                                              int c0, int cm, int c1, bool alone, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
-  typedef ShrinkShape<NA8> S;
+// A wavefront's walk over chunks [c0, c1) of the rows.  step(c): before chunk c is multiplied; multiply(rb, ks, a, x).
+template <int NA8, typename S, typename Step, typename Multiply>
+__device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
+                                            int c0, int c1, bool alone, Step step, Multiply multiply) {
   constexpr int RB = S::RB, ND = S::ND, NST = S::NST;
   const int lane = threadIdx.x & (kWave - 1), lr = lane & 15, lg = lane >> 4;
   const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;
@@ -66,8 +66,6 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
     const int row = g * 8 + (lane >> 3);
     aoff[g] = static_cast<uint32_t>(row < rbuf ? row : rbuf - 1) * arow + swz;
   }
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) first[rb] = acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_address(ring));
   auto issue = [&](int c, int stage) {
     const char* a = abase + static_cast<int64_t>(c) * kChunk;
@@ -95,22 +93,11 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
       issue(c0 + c + NST - 1, into);
     }
     const int younger = n - 1 - c < NST - 1 ? n - 1 - c : NST - 1;  // stages requested behind this one
-    if constexpr (NST == 4) {
-      if (younger >= 3) wait_loads<3 * ND>();
-      else if (younger == 2) wait_loads<2 * ND>();
-      else if (younger == 1) wait_loads<ND>();
-      else wait_loads<0>();
-    } else {
-      if (younger >= 1) wait_loads<ND>();
-      else wait_loads<0>();
-    }
-    if (c0 + c == cm) {  // the first of the wavefront's two shares is complete
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        first[rb] = acc[rb];
-        acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
+    if (NST >= 4 && younger >= 3) wait_loads<(NST >= 4 ? 3 : 0) * ND>();
+    else if (NST >= 3 && younger >= 2) wait_loads<(NST >= 3 ? 2 : 0) * ND>();
+    else if (younger >= 1) wait_loads<ND>();
+    else wait_loads<0>();
+    step(c0 + c);
     const char* st = ring + stage * (ND * 1024) + lr * 128 + ((lg ^ (lr & 7)) * 16);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -121,13 +108,33 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
       for (int rb = 0; rb < RB; ++rb) {
         Pack8 aw;
         aw.raw = *reinterpret_cast<const i32x4*>(at + rb * 2048);
-        acc[rb] = Mma<T>::run(aw, xa, acc[rb]);
+        multiply(rb, ks, aw, xa);
       }
     }
     stage = stage + 1 == NST ? 0 : stage + 1;
     into = into + 1 == NST ? 0 : into + 1;
   }
   MLORA_STAMP(3);  // shrink: multiplied
+}
+
+template <typename T, int NA8>
+__device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
+                                              int c0, int cm, int c1, bool alone, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
+  constexpr int RB = ShrinkShape<NA8>::RB;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) first[rb] = acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  walk_chunks<NA8, ShrinkShape<NA8>>(
+      ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
+      [&](int c) {
+        if (c == cm) {  // the first of the wavefront's two shares is complete
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) {
+            first[rb] = acc[rb];
+            acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+      },
+      [&](int rb, int, const Pack8& aw, const Pack8& xa) { acc[rb] = Mma<T>::run(aw, xa, acc[rb]); });
   mfma_settle(acc);  // (the last product and the reads of the sums lie on two sides of the loop's exit)
 }
 
@@ -258,20 +265,112 @@ template <typename T> __device__ __forceinline__ void mask_piece(Pack8& p, int f
   }
 }
 
+// The values of y of a span: four columns of a token.
+template <typename T> using YSpan = typename std::conditional<sizeof(T) == 2, uint2, uint4>::type;
+template <int C> struct ExpandShape {
+  static constexpr int KSTEPS = (C + 3) / 4;     // operand steps of the contraction (four pieces each)
+  static constexpr int HROW = KSTEPS * 64 + 16;  // bytes of an LDS row of the intermediate (one part)
+  static constexpr int SH = C * 4 >= 64 ? 6 : C * 4 >= 32 ? 5 : C * 4 >= 16 ? 4 : 3;  // the swizzle of the B pieces: lanes' rows lie 4 C pieces apart
+};
+
+// A wavefront's B rows [c0, c0 + 64 SP), up to column n1, to its LDS.
+template <typename T, int C, int SP>
+__device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, int n1, int eff, bool alone) {
+  constexpr int E = PieceOf<T>::E, SH = ExpandShape<C>::SH;
+  constexpr int NB = SP * C;  // direct loads of a wavefront's B rows
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t to = __builtin_amdgcn_readfirstlane(lds_address(s_b));
+  const char* src = bbase + static_cast<int64_t>(c0) * (C * 16);
+  const uint32_t last = static_cast<uint32_t>(n1 - c0) * C - 1;  // last piece of the range
+  auto request = [&](auto once) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const uint32_t u = i * 64 + lane;
+      uint32_t s = u ^ ((u >> SH) & 7);
+      const uint32_t kc = s % C;
+      s = s < last ? s : last;
+      if (kc * E < static_cast<uint32_t>(eff)) {  // (piece 0 of a row is always fetched: some lane takes part)
+        if constexpr (decltype(once)::value) dma16_once(src, s * 16, to + i * 1024);
+        else dma16(src, s * 16, to + i * 1024);
+      }
+    }
+  };
+  if (alone) request(std::true_type{});
+  else request(std::false_type{});
+}
+
+template <typename T, int SP>
+__device__ __forceinline__ void request_y(YSpan<T> (&yq)[SP][4], const T* ybase, const int64_t ys, const i32x4 rows, int c0, int n1) {
+  const int lr = threadIdx.x & 15;
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    int c = c0 + s * 64 + 4 * lr;
+    c = c < n1 ? c : n1 - 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) yq[s][i] = *reinterpret_cast<const YSpan<T>*>(ybase + static_cast<int64_t>(rows[i]) * ys + c);
+  }
+}
+
+// Products and stores of a wavefront's spans, once the intermediate is in LDS.
+template <typename T, int C, int SP>
+__device__ __forceinline__ void finish_spans(const char* s_h, const char* s_b, const YSpan<T> (&yq)[SP][4], T* __restrict__ ybase, const int64_t ys,
+                                             const i32x4 rows, int c0, int n1, int m, int eff) {
+  constexpr int E = PieceOf<T>::E, KSTEPS = ExpandShape<C>::KSTEPS, HROW = ExpandShape<C>::HROW, SH = ExpandShape<C>::SH;
+  constexpr bool SPLIT = sizeof(T) == 2;  // 16-bit operands: the intermediate as leading part and remainder
+  const int lane = threadIdx.x & (kWave - 1), lr = lane & 15, lg = lane >> 4;
+  Pack8 hop[KSTEPS], hlo[SPLIT ? KSTEPS : 1];
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    hop[ks].raw = *reinterpret_cast<const i32x4*>(s_h + lr * HROW + (ks * 4 + lg) * 16);
+    if constexpr (SPLIT) hlo[ks].raw = *reinterpret_cast<const i32x4*>(s_h + (16 + lr) * HROW + (ks * 4 + lg) * 16);
+  }
+  wait_loads<0>();
+  MLORA_STAMP(12);  // expand: B rows and y here
+  const bool mask = eff < KSTEPS * 4 * E;
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    const int c = c0 + s * 64 + 4 * lr;
+    f32x4 out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      out[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        int kc = ks * 4 + lg;
+        if (C % 4) kc = kc < C ? kc : C - 1;
+        const uint32_t u = (s * 64 + 4 * lr + j) * C + kc;
+        Pack8 bo;
+        bo.raw = *reinterpret_cast<const i32x4*>(s_b + (u ^ ((u >> SH) & 7)) * 16);
+        if (mask) mask_piece<T>(bo, (ks * 4 + lg) * E, eff);
+        if constexpr (SPLIT) out[j] = Mma<T>::run(hlo[ks], bo, out[j]);
+        out[j] = Mma<T>::run(hop[ks], bo, out[j]);
+      }
+    }
+    if (c < n1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (4 * lg + i < m) {
+          union { YSpan<T> raw; T e[4]; } v;
+          v.raw = yq[s][i];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v.e[j] = from_f32<T>(to_f32(v.e[j]) + out[j][i]);
+          *reinterpret_cast<YSpan<T>*>(ybase + static_cast<int64_t>(rows[i]) * ys + c) = v.raw;
+        }
+      }
+    }
+  }
+}
+
 template <typename T, int C, int SP>
 __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__ hsrc, int64_t part_stride, int kparts, const f32x4 (&hv)[kPartsAhead], const char* bbase,
                                             T* __restrict__ ybase, const int64_t ys, const i32x4 rows, int n0, int n1, int m, int eff,
                                             bool alone, float scaling) {
   constexpr int E = PieceOf<T>::E;          // elements per piece
   constexpr int R = C * E;                  // rank of the buffers
-  constexpr int KSTEPS = (C + 3) / 4;       // operand steps of the contraction (four pieces each)
+  constexpr int KSTEPS = ExpandShape<C>::KSTEPS, HROW = ExpandShape<C>::HROW;
   constexpr int RP = (R + 15) & ~15;
   constexpr bool SPLIT = sizeof(T) == 2;    // 16-bit operands: the intermediate as leading part and remainder
-  constexpr int HROW = KSTEPS * 64 + 16;    // bytes of an LDS row of the intermediate (one part)
-  constexpr int SH = C * 4 >= 64 ? 6 : C * 4 >= 32 ? 5 : C * 4 >= 16 ? 4 : 3;  // the swizzle of the B pieces: lanes' rows lie 4 C pieces apart
-  constexpr int NB = SP * C;                // direct loads of a wavefront's B rows
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int lr = lane & 15, lg = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   char* s_h = lds;                                                   // [2][16] rows
   char* s_b = lds + 2 * 16 * HROW + wave * (SP * 64 * C * 16);  // this wavefront's B rows
 
@@ -279,35 +378,9 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
   const int tok = tid / 16, q4 = tid & 15;  // sixteen threads per token, four ranks (RP = 64: all of them busy) each
   const int c0 = n0 + wave * (SP * 64);
   const bool mine = c0 < n1;
-  if (mine) {
-    const uint32_t to = __builtin_amdgcn_readfirstlane(lds_address(s_b));
-    const char* src = bbase + static_cast<int64_t>(c0) * (C * 16);
-    const uint32_t last = static_cast<uint32_t>(n1 - c0) * C - 1;  // last piece of the range
-    auto request = [&](auto once) {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        const uint32_t u = i * 64 + lane;
-        uint32_t s = u ^ ((u >> SH) & 7);
-        const uint32_t kc = s % C;
-        s = s < last ? s : last;
-        if (kc * E < static_cast<uint32_t>(eff)) {  // (piece 0 of a row is always fetched: some lane takes part)
-          if constexpr (decltype(once)::value) dma16_once(src, s * 16, to + i * 1024);
-          else dma16(src, s * 16, to + i * 1024);
-        }
-      }
-    };
-    if (alone) request(std::true_type{});
-    else request(std::false_type{});
-  }
-  typedef typename std::conditional<sizeof(T) == 2, uint2, uint4>::type Y4;
-  Y4 yq[SP][4];
-#pragma unroll
-  for (int s = 0; s < SP; ++s) {
-    int c = c0 + s * 64 + 4 * lr;
-    c = c < n1 ? c : n1 - 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) yq[s][i] = *reinterpret_cast<const Y4*>(ybase + static_cast<int64_t>(rows[i]) * ys + c);
-  }
+  YSpan<T> yq[SP][4];
+  if (mine) request_b<T, C, SP>(s_b, bbase, c0, n1, eff, alone);
+  request_y<T, SP>(yq, ybase, ys, rows, c0, n1);
   MLORA_STAMP(10);  // expand: B rows and y requested
   // the intermediate: parts summed in order, scaled, split, to LDS in operand rows (its first
   // kPartsAhead parts were requested with the record)
@@ -346,47 +419,7 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
   __syncthreads();
   MLORA_STAMP(11);  // expand: intermediate in LDS
   if (!mine) return;
-  Pack8 hop[KSTEPS], hlo[SPLIT ? KSTEPS : 1];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    hop[ks].raw = *reinterpret_cast<const i32x4*>(s_h + lr * HROW + (ks * 4 + lg) * 16);
-    if constexpr (SPLIT) hlo[ks].raw = *reinterpret_cast<const i32x4*>(s_h + (16 + lr) * HROW + (ks * 4 + lg) * 16);
-  }
-  wait_loads<0>();
-  MLORA_STAMP(12);  // expand: B rows and y here
-  const bool mask = eff < KSTEPS * 4 * E;
-#pragma unroll
-  for (int s = 0; s < SP; ++s) {
-    const int c = c0 + s * 64 + 4 * lr;
-    f32x4 out[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      out[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        int kc = ks * 4 + lg;
-        if (C % 4) kc = kc < C ? kc : C - 1;
-        const uint32_t u = (s * 64 + 4 * lr + j) * C + kc;
-        Pack8 bo;
-        bo.raw = *reinterpret_cast<const i32x4*>(s_b + (u ^ ((u >> SH) & 7)) * 16);
-        if (mask) mask_piece<T>(bo, (ks * 4 + lg) * E, eff);
-        if constexpr (SPLIT) out[j] = Mma<T>::run(hlo[ks], bo, out[j]);
-        out[j] = Mma<T>::run(hop[ks], bo, out[j]);
-      }
-    }
-    if (c < n1) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (4 * lg + i < m) {
-          union { Y4 raw; T e[4]; } v;
-          v.raw = yq[s][i];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v.e[j] = from_f32<T>(to_f32(v.e[j]) + out[j][i]);
-          *reinterpret_cast<Y4*>(ybase + static_cast<int64_t>(rows[i]) * ys + c) = v.raw;
-        }
-      }
-    }
-  }
+  finish_spans<T, C, SP>(s_h, s_b, yq, ybase, ys, rows, c0, n1, m, eff);
 }
 
 #ifdef MLORA_TRACE
@@ -432,6 +465,138 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   MLORA_STAMP_END(13);  // expand: stores issued, acknowledged
 }
 
+// ---- both in one launch, fp32 ------------------------------------------------------------------------
+// A workgroup takes a (tile, column range) and multiplies all of K itself, an eighth per wavefront through the same rings,
+// its B rows and y requested ahead of them; nothing passes between workgroups.  What bounds it is what a compute unit takes
+// in, x and A whole for every range (128 KB at rank 16, K = 1024, in about 3 us); what it saves is the second launch with its
+// record, sums and drain.  Figures: solo_columns.
+constexpr int kSoloWaves = 8;
+constexpr int kSoloThreads = kSoloWaves * kWave;
+template <int NA8> struct SoloShape {
+  static constexpr int RB = (NA8 + 1) / 2;
+  static constexpr int ND = NA8 + 2;
+  static constexpr int NST = ND <= 4 ? 3 : 2;
+  static constexpr int BYTES = NST * ND * 1024;
+};
+
+template <typename T, int NA8, int R>
+__device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_bytes, const char* abase, uint32_t arow, const char* xbase,
+                                            const uint32_t (&xoff)[2], int kchunks, int m, int eff, bool alone, float scaling) {
+  typedef SoloShape<NA8> S;
+  constexpr int RB = S::RB;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int c0 = wave * kchunks / kSoloWaves, c1 = (wave + 1) * kchunks / kSoloWaves;
+  char* ring = rings + wave * S::BYTES;
+  // eight chains per block of ranks: the 16x16x4 products of a chunk do not wait for each other, and sixty-four short
+  // chains added up as a tree come closer to the sum than eight long ones
+  f32x4 acc[RB][2][4];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[rb][ks][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  walk_chunks<NA8, S>(
+      ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
+      [&](int rb, int ks, const Pack8& aw, const Pack8& xa) {
+        f32x4 a, x;
+        __builtin_memcpy(&a, &aw, 16);
+        __builtin_memcpy(&x, &xa, 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[rb][ks][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], x[j], acc[rb][ks][j], 0, 0, 0);
+      });
+  static_assert(RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    mfma_settle(acc[rb][0]);
+    mfma_settle(acc[rb][1]);
+    f32x4 s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      s[i] = ((acc[rb][0][0][i] + acc[rb][0][1][i]) + (acc[rb][0][2][i] + acc[rb][0][3][i])) +
+             ((acc[rb][1][0][i] + acc[rb][1][1][i]) + (acc[rb][1][2][i] + acc[rb][1][3][i]));
+    *reinterpret_cast<f32x4*>(ring + (rb * kWave + lane) * 16) = s;
+  }
+  __syncthreads();
+  MLORA_STAMP(4);  // every wavefront's sums in LDS
+  // the eighths, scaled, to the operand rows of the expand: lane holds ranks 16 rb + 4 (lane / 16) .. + 3 of token lane % 16
+  constexpr int BLOCKS = (R + 15) / 16;
+  if (wave < BLOCKS) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if (wave < RB) {
+      f32x4 v[kSoloWaves];
+#pragma unroll
+      for (int w = 0; w < kSoloWaves; ++w) v[w] = *reinterpret_cast<const f32x4*>(rings + w * S::BYTES + tid * 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] = ((v[0][i] + v[1][i]) + (v[2][i] + v[3][i])) + ((v[4][i] + v[5][i]) + (v[6][i] + v[7][i]));
+    }
+    const int tok = lane & 15, r0 = wave * 16 + 4 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = (tok < m && r0 + i < eff) ? s[i] * scaling : 0.f;
+    *reinterpret_cast<f32x4*>(s_h + tok * hrow_bytes + r0 * 4) = s;
+  }
+}
+
+// grid (8, column ranges, tiles / 8).  C: 16-byte pieces of a B row.
+template <int C>
+__global__ __launch_bounds__(kSoloThreads) void solo_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, void* __restrict__ yv_,
+                                                            int64_t ys, int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, float scaling,
+                                                            int ring_bytes, const int32_t* __restrict__ eff_rank, ShrinkSlices sl, ExpandSplits splits) {
+  typedef float T;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  constexpr int R = C * PieceOf<T>::E, HROW = ExpandShape<C>::HROW;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), lg = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  MLORA_STAMP(0);
+  const ExpandSplit sp = splits.split[blockIdx.y];
+  const int tile = blockIdx.z * 8 + blockIdx.x;
+  const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
+  const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
+  const i32x4 rows = *reinterpret_cast<const i32x4*>(rec + MLORA_SMALL_TILE_ROWS + 4 * lg);  // tokens 4 * lg .. + 3
+  int row[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) row[i] = rec[MLORA_SMALL_TILE_ROWS + i * 8 + (lane >> 3)];
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!t.ok) {
+    count_rejected_plan(plan, t.plan_ok);
+    return;
+  }
+  MLORA_STAMP(1);  // record here
+  const int slot = __builtin_amdgcn_readfirstlane(t.slot), m = __builtin_amdgcn_readfirstlane(t.m);
+  const int eff = rank_pick(ranks, eff_rank, num_slots, slot, R);
+  if (eff == 0) return;
+  const uint32_t arow = static_cast<uint32_t>(kchunks) * kChunk;
+  const char* abase = uniform(static_cast<const char*>(sl.a[sp.slice]) + static_cast<int64_t>(slot) * R * arow);
+  const char* bbase = uniform(static_cast<const char*>(sp.b) + static_cast<int64_t>(slot) * sp.n * (C * 16));
+  uint32_t xoff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) xoff[i] = static_cast<uint32_t>(row[i]) * xrow;
+  char* s_h = lds + ring_bytes;
+  char* s_b = s_h + 16 * HROW + wave * (64 * C * 16);  // (of wavefronts with columns only)
+  T* const ybase = static_cast<T*>(yv_) + sp.y_col;
+  const int c0 = sp.n0 + wave * 64;
+  const bool mine = c0 < sp.n1;
+  YSpan<T> yq[1][4];
+  if (mine) request_b<T, C, 1>(s_b, bbase, c0, sp.n1, eff, false);
+  request_y<T, 1>(yq, ybase, ys, rows, c0, sp.n1);
+  const int groups = (eff + 7) >> 3;
+  if (R <= 8 || groups <= 1) solo_shrink<T, 1, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
+  else if (R <= 16 || groups <= 2) solo_shrink<T, 2, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
+  else solo_shrink<T, 4, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
+  __syncthreads();
+  MLORA_STAMP(5);  // intermediate in LDS
+  if (!mine) return;
+  finish_spans<T, C, 1>(s_h, s_b, yq, ybase, ys, rows, c0, sp.n1, m, eff);
+}
+
+int solo_ring(int r) {
+  int most = SoloShape<1>::BYTES;
+  if (r > 8 && SoloShape<2>::BYTES > most) most = SoloShape<2>::BYTES;
+  if (r > 16 && SoloShape<4>::BYTES > most) most = SoloShape<4>::BYTES;
+  return most * kSoloWaves;
+}
+
 int expand_lds(int c, int sp) {
   const int ksteps = (c + 3) / 4, hrow = ksteps * 64 + 16;
   return 2 * 16 * hrow + kPairWaves * sp * 64 * c * 16;
@@ -439,12 +604,14 @@ int expand_lds(int c, int sp) {
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
 struct PairKnobs {
-  int generation = -1, kparts, sp, wgs;
+  int generation = -1, kparts, sp, wgs, solo, solo_cols;
   void read() {
     generation = knob_generation();
     kparts = env_int("MLORA_PAIR_KPARTS", 0);
     sp = env_int("MLORA_PAIR_SP", 0);
     wgs = env_int("MLORA_PAIR_WGS", 192);
+    solo = env_int("MLORA_SOLO", 1);  // 0: never in one launch, 2: wherever it can be
+    solo_cols = env_int("MLORA_SOLO_COLS", 0) / 64 % 9 * 64;  // at most 512
   }
 };
 const PairKnobs& pair_knobs() {
@@ -539,7 +706,77 @@ bool pair_supported(const MloraAddArgs* a) {
   return total <= kMaxSplits && partials_room(a) >= part_bytes(a, plan_layout(a->num_tokens, a->num_slots));
 }
 
-int launch_pair(const MloraAddArgs* a) {
+namespace {
+int columns_total(const MloraAddArgs* a, int nt) {
+  int total = 0;
+  for (int i = 0; i < a->num_slices; ++i) total += (a->slices[i].n + nt - 1) / nt;
+  return total;
+}
+}  // namespace
+
+// Columns of a range of the one launch where it beats the pair, else 0: fp32, x and A of a tile no more than rank 16's at K = 2048,
+// and every workgroup resident at once (tile t runs on XCD t % 8, which has 32 compute units; a second round repeats the
+// shrink).  us per call, the pair / one launch in ranges of 256 / 512 columns, q|k|v, o and gate_up:
+//   rank 16, K = 1024:  1 token of 4 slots 6.2 / 5.3 / 5.9, 6.1 / 5.2 / 5.9, 7.1 / 5.9 / 6.6; 64 of 4 7.3 / 6.0 / 6.8, 7.2 / 5.8 / 6.5, 8.5 / 7.4 / 8.1; 64 of 32
+//   8.3 / 6.3 / 7.1, 7.6 / 6.1 / 6.7, 10.5 / 18.8 / 13.2 (104 and 52 workgroups an XCD); 256 of 64 10.6 / 10.8 / 8.7 (48 and 32), 8.1 / 7.2 / 7.5.
+//   rank 8, K = 1024:   64 of 4 7.1 / 5.7 / 6.1, 6.9 / 5.7 / 6.1, 8.1 / 6.8 / 7.3; 256 of 8 7.8 / 6.2 / 6.9, 7.3 / 6.0 / 6.6, 11.1 / 15.6 / 12.9.
+//   rank 16, K = 2048:  64 of 4 8.0 / 7.8 / 8.6, 7.6 / 7.4 / 8.2; 64 of 32 10.2 / 12.9 / 8.9 (48 and 24), 8.1 / 8.0 / 8.5; 256 of 64 14.5 / 21.9 / 18.4.
+//   rank 32, K = 1024 (256 columns: B rows of 512 do not fit the LDS):  64 of 4 8.3 / 7.6, 7.8 / 7.0, 9.7 / 9.5; 8 of 8 gate_up 8.6 / 9.0 (32); 64 of
+//   32 9.8 / 8.0, 8.9 / 7.7; 256 of 64 o 10.1 / 9.3 (32), q|k|v 14.2 / 16.6 (48).  At K = 2048 it loses throughout (64 of 4 9.2 / 10.0).
+//   K = 4096 loses at every rank (rank 8, 1 token: 7.1 / 8.9).
+static int solo_columns(const MloraAddArgs* a, int active) {
+  if (a->dtype != MLORA_DTYPE_F32 || a->form != MLORA_FORM_AUTO || !(a->r == 8 || a->r == 16 || a->r == 32)) return 0;
+  if (pair_knobs().solo != 1) {
+    if (pair_knobs().solo != 2) return 0;
+    return pair_knobs().solo_cols > 0 && columns_total(a, pair_knobs().solo_cols) <= kMaxSplits && a->r * pair_knobs().solo_cols <= 8192
+               ? pair_knobs().solo_cols
+               : columns_total(a, 256) <= kMaxSplits ? 256 : 0;
+  }
+  if (a->k > 2048 || static_cast<long long>(a->r) * a->k > 32768) return 0;
+  const int layers = (small_tiles_about(a, active) + 7) / 8;  // tiles of an XCD
+  for (int nt = 256; nt <= (a->r <= 16 ? 512 : 256); nt *= 2) {
+    const int total = columns_total(a, nt);
+    if (total <= kMaxSplits && layers * total <= (a->r <= 16 ? 32 : 24)) return nt;
+  }
+  return 0;
+}
+
+namespace {
+template <int C> void launch_solo_rank(const MloraAddArgs* a, const PlanLayout& lay, int total, int lds, const ShrinkSlices& sl, const ExpandSplits& splits) {
+  allow_lds<solo_kernel<C>>(lds);
+  hipLaunchKernelGGL((solo_kernel<C>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(lay.cap_small / 8)), dim3(kSoloThreads), lds,
+                     static_cast<hipStream_t>(a->stream), a->plan, a->x, a->y, a->y_stride, lay.small_off, a->num_tokens, a->num_slots,
+                     static_cast<int>(a->k * sizeof(float) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(float)), a->scaling, solo_ring(a->r),
+                     a->effective_rank, sl, splits);
+}
+}  // namespace
+
+static int launch_solo(const MloraAddArgs* a, int nt) {
+  const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
+  if (lay.cap_small == 0) return 0;
+  ExpandSplits splits;
+  const int total = columns_total(a, nt);
+  int s = 0;
+  for (int i = 0; i < a->num_slices; ++i)
+    for (int n0 = 0; n0 < a->slices[i].n; n0 += nt) {
+      ExpandSplit& d = splits.split[s++];
+      d.b = a->slices[i].b; d.n = a->slices[i].n; d.y_col = a->slices[i].y_col; d.slice = i; d.pad = 0;
+      d.n0 = n0; d.n1 = n0 + nt < a->slices[i].n ? n0 + nt : a->slices[i].n;
+    }
+  ShrinkSlices sl;
+  for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = i < a->num_slices ? a->slices[i].a : nullptr;
+  const int c = a->r / 4, lds = solo_ring(a->r) + 16 * (((c + 3) / 4) * 64 + 16) + nt * c * 16;
+  switch (a->r) {
+    case 8: launch_solo_rank<2>(a, lay, total, lds, sl, splits); break;
+    case 16: launch_solo_rank<4>(a, lay, total, lds, sl, splits); break;
+    case 32: launch_solo_rank<8>(a, lay, total, lds, sl, splits); break;
+    default: set_error("mlora_add_lora(pair): unsupported rank %d", a->r); return MLORA_E_UNSUPPORTED;
+  }
+  return check_launch("mlora_add_lora(fp32, one launch over small tiles)");
+}
+
+int launch_pair(const MloraAddArgs* a, int active) {
+  if (const int nt = solo_columns(a, active)) return launch_solo(a, nt);
   PairLaunch l;
   l.a = a;
   l.lay = plan_layout(a->num_tokens, a->num_slots);
