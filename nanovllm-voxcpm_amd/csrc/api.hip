@@ -328,7 +328,8 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
     // (fp32 rows and anything else the 128-bit kernels for 16-bit elements do not take: one workgroup per token,
     // which fetches A and B per token and walks K in chained steps, except where the pair of launches has the
     // element type: config 1's batch, 64 tokens over 4 slots, rank 16, fp32, qkv / o / gate_up / down 25 / 25 / 27 /
-    // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches)
+    // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches; rank 24, 36 / 16 / 39 / 104 and 9.5 / 9.2 / 10.7 /
+    // 10.9, rank 56, 81 / 80 / 90 / 243 and 12.6 / 12.1 / 14.3 / 15.5, one token of rank 24 15.3 / 15.4 / 15.8 / 43 and 8.5 / 8.5 / 9.2 / 9.9)
     if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
     else if (one_launch && !(small_tiles && small_batch(a, true))) form = MLORA_FORM_WIDE;
     else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false))) form = MLORA_FORM_SGMV;

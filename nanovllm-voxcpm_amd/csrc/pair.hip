@@ -117,29 +117,79 @@ __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint3
   MLORA_STAMP(3);  // shrink: multiplied
 }
 
-template <typename T, int NA8>
+// fp32 products of a wavefront in eight chains per block of ranks, added up as a tree: the 16x16x4 products of a chunk do not wait for
+// each other, and short chains come closer to the sum than a long one.
+template <int RB> struct Chains {
+  f32x4 v[RB][2][4];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[rb][ks][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ void add(int rb, int ks, const Pack8& aw, const Pack8& xa) {
+    f32x4 a, x;
+    __builtin_memcpy(&a, &aw, 16);
+    __builtin_memcpy(&x, &xa, 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[rb][ks][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], x[j], v[rb][ks][j], 0, 0, 0);
+  }
+  __device__ __forceinline__ void collect(f32x4 (&to)[RB]) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      mfma_settle(v[rb][0]);
+      mfma_settle(v[rb][1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        to[rb][i] = ((v[rb][0][0][i] + v[rb][0][1][i]) + (v[rb][0][2][i] + v[rb][0][3][i])) +
+                    ((v[rb][1][0][i] + v[rb][1][1][i]) + (v[rb][1][2][i] + v[rb][1][3][i]));
+    }
+  }
+};
+
+// CHAINS (fp32): eight chains per block of ranks instead of one, one per element of a piece and half of a chunk, for buffers of the ranks
+// whose calls one workgroup per token used to take, so that their error is no larger than that kernel's (rank 48, K = 1024, 2048
+// tokens: 2.2e-7 of the update, with one chain 2.4e-7); 0.2 us per call.
+template <typename T, int NA8, bool CHAINS>
 __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
                                               int c0, int cm, int c1, bool alone, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
   constexpr int RB = ShrinkShape<NA8>::RB;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) first[rb] = acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  walk_chunks<NA8, ShrinkShape<NA8>>(
-      ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
-      [&](int c) {
-        if (c == cm) {  // the first of the wavefront's two shares is complete
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) {
-            first[rb] = acc[rb];
-            acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (CHAINS) {
+    Chains<RB> chains;
+    chains.clear();
+    walk_chunks<NA8, ShrinkShape<NA8>>(
+        ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
+        [&](int c) {
+          if (c == cm) {  // the first of the wavefront's two shares is complete
+            chains.collect(first);
+            chains.clear();
           }
-        }
-      },
-      [&](int rb, int, const Pack8& aw, const Pack8& xa) { acc[rb] = Mma<T>::run(aw, xa, acc[rb]); });
-  mfma_settle(acc);  // (the last product and the reads of the sums lie on two sides of the loop's exit)
+        },
+        [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
+    chains.collect(acc);
+  } else {
+    walk_chunks<NA8, ShrinkShape<NA8>>(
+        ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
+        [&](int c) {
+          if (c == cm) {  // the first of the wavefront's two shares is complete
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+              first[rb] = acc[rb];
+              acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+          }
+        },
+        [&](int rb, int, const Pack8& aw, const Pack8& xa) { acc[rb] = Mma<T>::run(aw, xa, acc[rb]); });
+    mfma_settle(acc);  // (the last product and the reads of the sums lie on two sides of the loop's exit)
+  }
 }
 
 // dst: this tile's block of partial sums, sixteen rows of rp floats.
-template <typename T, int NA8>
+template <typename T, int NA8, bool CHAINS>
 __device__ __forceinline__ void shrink_tile(char* lds, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2], int c0,
                                             int cm, int c1, bool alone, float* __restrict__ dst, int rp, int m) {
   typedef ShrinkShape<NA8> S;
@@ -147,7 +197,7 @@ __device__ __forceinline__ void shrink_tile(char* lds, const char* abase, uint32
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   char* ring = lds + wave * S::BYTES;
   f32x4 first[RB], acc[RB];
-  shrink_chunks<T, NA8>(ring, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, first, acc);
+  shrink_chunks<T, NA8, CHAINS>(ring, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, first, acc);
   // sum over the eighths of the part, the first one first, through the rings' memory
   static_assert(2 * RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
 #pragma unroll
@@ -188,7 +238,7 @@ __device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __r
 }
 
 // grid (8, slices * K parts, tiles / 8): blockIdx.x is the XCD, so that the workgroups of a tile share an L2.
-template <typename T>
+template <typename T, bool CHAINS>
 __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
                                                                    int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, int rbuf,
                                                                    int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
@@ -227,11 +277,11 @@ __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t
   float* dst = hws + (static_cast<int64_t>(part * num_slices + slice) * (gridDim.z * 8) + tile) * (MLORA_TILE_SMALL * rp);
   const bool alone = __builtin_amdgcn_readfirstlane(t.alone) != 0;
   const int groups = (eff + 7) >> 3;
-  if (groups <= 1) shrink_tile<T, 1>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups == 2) shrink_tile<T, 2>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups <= 4) shrink_tile<T, 4>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups <= 6) shrink_tile<T, 6>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else shrink_tile<T, 8>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  if (groups <= 1) shrink_tile<T, 1, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  else if (groups == 2) shrink_tile<T, 2, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  else if (groups <= 4) shrink_tile<T, 4, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  else if (groups <= 6) shrink_tile<T, 6, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  else shrink_tile<T, 8, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
 #ifdef MLORA_TRACE
   MLORA_STAMP(5);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -487,36 +537,15 @@ __device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_byt
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int c0 = wave * kchunks / kSoloWaves, c1 = (wave + 1) * kchunks / kSoloWaves;
   char* ring = rings + wave * S::BYTES;
-  // eight chains per block of ranks: the 16x16x4 products of a chunk do not wait for each other, and sixty-four short
-  // chains added up as a tree come closer to the sum than eight long ones
-  f32x4 acc[RB][2][4];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[rb][ks][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  walk_chunks<NA8, S>(
-      ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
-      [&](int rb, int ks, const Pack8& aw, const Pack8& xa) {
-        f32x4 a, x;
-        __builtin_memcpy(&a, &aw, 16);
-        __builtin_memcpy(&x, &xa, 16);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[rb][ks][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], x[j], acc[rb][ks][j], 0, 0, 0);
-      });
+  Chains<RB> chains;
+  chains.clear();
+  walk_chunks<NA8, S>(ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
+                      [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
   static_assert(RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
+  f32x4 acc[RB];
+  chains.collect(acc);
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    mfma_settle(acc[rb][0]);
-    mfma_settle(acc[rb][1]);
-    f32x4 s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      s[i] = ((acc[rb][0][0][i] + acc[rb][0][1][i]) + (acc[rb][0][2][i] + acc[rb][0][3][i])) +
-             ((acc[rb][1][0][i] + acc[rb][1][1][i]) + (acc[rb][1][2][i] + acc[rb][1][3][i]));
-    *reinterpret_cast<f32x4*>(ring + (rb * kWave + lane) * 16) = s;
-  }
+  for (int rb = 0; rb < RB; ++rb) *reinterpret_cast<f32x4*>(ring + (rb * kWave + lane) * 16) = acc[rb];
   __syncthreads();
   MLORA_STAMP(4);  // every wavefront's sums in LDS
   // the eighths, scaled, to the operand rows of the expand: lane holds ranks 16 rb + 4 (lane / 16) .. + 3 of token lane % 16
@@ -632,12 +661,12 @@ struct PairLaunch {
   int parts_log2, sp;
 };
 
-template <typename T> void launch_pair_shrink(const PairLaunch& l) {
+template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) {
   const MloraAddArgs* a = l.a;
   ShrinkSlices sl;
   for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = i < a->num_slices ? a->slices[i].a : nullptr;
-  allow_lds<pair_shrink_kernel<T>>(shrink_lds(a->r));
-  hipLaunchKernelGGL((pair_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
+  allow_lds<pair_shrink_kernel<T, CHAINS>>(shrink_lds(a->r));
+  hipLaunchKernelGGL((pair_shrink_kernel<T, CHAINS>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
                      dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
                      a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
                      l.parts_log2, a->num_slices, a->effective_rank, sl);
@@ -658,24 +687,24 @@ template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const 
 }
 
 template <typename T> bool launch_pair_type(const PairLaunch& l, const ExpandSplits& splits, int total) {
-  launch_pair_shrink<T>(l);
-  switch (l.a->r * static_cast<int>(sizeof(T)) / 16) {
-    case 2: return launch_pair_expand<T, 2>(l, splits, total);
-    case 4: return launch_pair_expand<T, 4>(l, splits, total);
-    case 8: return launch_pair_expand<T, 8>(l, splits, total);
-  }
-  if constexpr (sizeof(T) == 2) {
-    switch (l.a->r / 8) {
-      case 1: return launch_pair_expand<T, 1>(l, splits, total);
-      case 3: return launch_pair_expand<T, 3>(l, splits, total);
-      case 5: return launch_pair_expand<T, 5>(l, splits, total);
-      case 6: return launch_pair_expand<T, 6>(l, splits, total);
-      case 7: return launch_pair_expand<T, 7>(l, splits, total);
-    }
-    return false;
+  if constexpr (sizeof(T) == 4) {
+    if (exact_rank(l.a->r)) launch_pair_shrink<T, false>(l);
+    else launch_pair_shrink<T, true>(l);
   } else {
-    return l.a->r == 64 ? launch_pair_expand<T, 16>(l, splits, total) : false;
+    launch_pair_shrink<T, false>(l);
   }
+  constexpr int E8 = sizeof(T) / 2;  // 16-byte pieces of eight ranks
+  switch (l.a->r / 8) {
+    case 1: return launch_pair_expand<T, 1 * E8>(l, splits, total);
+    case 2: return launch_pair_expand<T, 2 * E8>(l, splits, total);
+    case 3: return launch_pair_expand<T, 3 * E8>(l, splits, total);
+    case 4: return launch_pair_expand<T, 4 * E8>(l, splits, total);
+    case 5: return launch_pair_expand<T, 5 * E8>(l, splits, total);
+    case 6: return launch_pair_expand<T, 6 * E8>(l, splits, total);
+    case 7: return launch_pair_expand<T, 7 * E8>(l, splits, total);
+    case 8: return launch_pair_expand<T, 8 * E8>(l, splits, total);
+  }
+  return false;
 }
 
 }  // namespace
@@ -691,7 +720,7 @@ void pair_trace_set(void* buf) {
 bool pair_supported(const MloraAddArgs* a) {
   const int64_t e = element_bytes(a->dtype);
   if (a->k <= 0 || (a->k * e) % kChunk || !a->plan) return false;
-  if (e == 2 ? !padded_rank(a->r) : !exact_rank(a->r)) return false;
+  if (!padded_rank(a->r) || (e == 4 && a->form != MLORA_FORM_AUTO && !exact_rank(a->r))) return false;  // (by name fp32 has the instances' ranks only)
   // 32-bit offsets of the x rows, A rows and B pieces; 16-byte loads of x and B, four columns of y at a time
   if (a->num_tokens * (a->x_stride * e) >= (1ll << 32) || a->r * (a->k * e) >= (1ll << 32)) return false;
   if ((a->x_stride * e) % 16 || a->y_stride % 4 || !a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255)) return false;

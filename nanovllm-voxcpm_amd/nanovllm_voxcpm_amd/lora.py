@@ -96,13 +96,12 @@ class _UnavailableBackend:
 
 
 _VECTOR_RANKS = (8, 16, 24, 32, 40, 48, 56, 64)  # rows of B start on 16-byte boundaries and an instance of the kernels covers them
-_VECTOR_RANKS_F32 = (8, 16, 32, 64)
 
 
 def _vector_shape(dtype: torch.dtype, rank: int, k: int) -> bool:
     """Element type, rank and K for which the library has a form that walks a plan."""
     if dtype == torch.float32:
-        return rank in _VECTOR_RANKS_F32 and k % 32 == 0  # the two-launch form over 16-token tiles
+        return rank in _VECTOR_RANKS and k % 32 == 0  # the two-launch form over 16-token tiles
     return dtype in (torch.float16, torch.bfloat16) and rank in _VECTOR_RANKS and k % 8 == 0
 
 

@@ -111,3 +111,16 @@ def test_auto_takes_one_launch_where_it_pays(tokens, slots, rank, k, widths, one
         _hip.reload_knobs()
     assert torch.equal(chosen, pair) != one_launch  # (the forms add K up in different orders)
     assert torch.allclose(chosen, batch[6], rtol=1e-5, atol=2e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank", [24, 40, 48, 56])
+@pytest.mark.parametrize("tokens, slots, k, widths", [(1, 3, 32, [4]), (17, 2, 1024, [520, 64]), (150, 40, 2080, [256])])
+def test_ranks_between_the_instances_are_two_launches_under_auto(rank, tokens, slots, k, widths):
+    from nanovllm_voxcpm_amd import _hip
+
+    case = (tokens, slots, rank, k, widths, 0, tokens > 1, True)
+    batch = _batch(case, rank)
+    out = _apply(case, batch, _hip.FORM_AUTO)
+    assert torch.equal(out[batch[0] < 0], batch[4][batch[0] < 0])
+    assert torch.allclose(out, batch[6], rtol=1e-5, atol=2e-5)
