@@ -53,8 +53,8 @@ template <int NA8> struct ShrinkShape {
   static constexpr int BYTES = NST * ND * 1024;      // of LDS per wavefront
 };
 
-// A wavefront's walk over chunks [c0, c1) of the rows.  step(c): before chunk c is multiplied; multiply(rb, ks, a, x).
-template <int NA8, typename S, typename Step, typename Multiply>
+// A wavefront's walk over chunks [c0, c1) of the rows.  XG: groups of eight token rows, one where the tile has no more tokens.  step(c): before chunk c is multiplied; multiply(rb, ks, a, x).
+template <int NA8, int XG, typename S, typename Step, typename Multiply>
 __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
                                             int c0, int c1, bool alone, Step step, Multiply multiply) {
   constexpr int RB = S::RB, ND = S::ND, NST = S::NST;
@@ -79,7 +79,7 @@ __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint3
       for (int g = 0; g < NA8; ++g) dma16(a, aoff[g], to + g * 1024);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(x, xoff[i] + swz, to + (NA8 + i) * 1024);
+    for (int i = 0; i < XG; ++i) dma16(x, xoff[i] + swz, to + (NA8 + i) * 1024);
   };
   const int n = c1 - c0;
 #pragma unroll
@@ -103,7 +103,7 @@ __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint3
     for (int ks = 0; ks < 2; ++ks) {
       const char* at = st + (ks == 0 ? 0 : (lg ^ (lr & 7)) & 4 ? -64 : 64);  // chunk lg, then chunk lg + 4, of the swizzled row
       Pack8 xa;
-      xa.raw = *reinterpret_cast<const i32x4*>(at + NA8 * 1024);
+      xa.raw = *reinterpret_cast<const i32x4*>(at + NA8 * 1024 - (XG == 1 ? (lr & 8) * 128 : 0));
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         Pack8 aw;
@@ -161,7 +161,7 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
   if constexpr (CHAINS) {
     Chains<RB> chains;
     chains.clear();
-    walk_chunks<NA8, ShrinkShape<NA8>>(
+    walk_chunks<NA8, 2, ShrinkShape<NA8>>(
         ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
         [&](int c) {
           if (c == cm) {  // the first of the wavefront's two shares is complete
@@ -172,7 +172,7 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
         [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
     chains.collect(acc);
   } else {
-    walk_chunks<NA8, ShrinkShape<NA8>>(
+    walk_chunks<NA8, 2, ShrinkShape<NA8>>(
         ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
         [&](int c) {
           if (c == cm) {  // the first of the wavefront's two shares is complete
@@ -349,7 +349,19 @@ __device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, 
   else request(std::false_type{});
 }
 
-template <typename T, int SP>
+// A tile's tokens spread over the lane groups: row 4 * lg + i of the products is token lg + 4 * i, so that those of a tile of up to four or
+// eight are the rows i = 0 or i < 2 (XI rows).  The one launch has a text per XI and leaves out what the others would request (64 tokens
+// of 32 slots, rank 16, K = 1024, o 6.1 -> 5.8 us; of 4, q|k|v 6.0 -> 5.8); in the pair that gains no more than it loses (two texts of the shrink, three
+// of the expand: -2 to +2 % over 54 shapes).
+__device__ __forceinline__ int row_of_token(int t) { return 4 * (t & 3) + (t >> 2); }
+__device__ __forceinline__ i32x4 spread_rows(const int32_t* __restrict__ rec, int lg) {
+  i32x4 rows;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) rows[i] = rec[MLORA_SMALL_TILE_ROWS + 4 * i + lg];
+  return rows;
+}
+
+template <typename T, int SP, int XI>
 __device__ __forceinline__ void request_y(YSpan<T> (&yq)[SP][4], const T* ybase, const int64_t ys, const i32x4 rows, int c0, int n1) {
   const int lr = threadIdx.x & 15;
 #pragma unroll
@@ -357,12 +369,12 @@ __device__ __forceinline__ void request_y(YSpan<T> (&yq)[SP][4], const T* ybase,
     int c = c0 + s * 64 + 4 * lr;
     c = c < n1 ? c : n1 - 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) yq[s][i] = *reinterpret_cast<const YSpan<T>*>(ybase + static_cast<int64_t>(rows[i]) * ys + c);
+    for (int i = 0; i < XI; ++i) yq[s][i] = *reinterpret_cast<const YSpan<T>*>(ybase + static_cast<int64_t>(rows[i]) * ys + c);
   }
 }
 
 // Products and stores of a wavefront's spans, once the intermediate is in LDS.
-template <typename T, int C, int SP>
+template <typename T, int C, int SP, int XI>
 __device__ __forceinline__ void finish_spans(const char* s_h, const char* s_b, const YSpan<T> (&yq)[SP][4], T* __restrict__ ybase, const int64_t ys,
                                              const i32x4 rows, int c0, int n1, int m, int eff) {
   constexpr int E = PieceOf<T>::E, KSTEPS = ExpandShape<C>::KSTEPS, HROW = ExpandShape<C>::HROW, SH = ExpandShape<C>::SH;
@@ -398,8 +410,8 @@ __device__ __forceinline__ void finish_spans(const char* s_h, const char* s_b, c
     }
     if (c < n1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (4 * lg + i < m) {
+      for (int i = 0; i < XI; ++i) {
+        if (lg + 4 * i < m) {
           union { YSpan<T> raw; T e[4]; } v;
           v.raw = yq[s][i];
 #pragma unroll
@@ -430,7 +442,7 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
   const bool mine = c0 < n1;
   YSpan<T> yq[SP][4];
   if (mine) request_b<T, C, SP>(s_b, bbase, c0, n1, eff, alone);
-  request_y<T, SP>(yq, ybase, ys, rows, c0, n1);
+  request_y<T, SP, 4>(yq, ybase, ys, rows, c0, n1);
   MLORA_STAMP(10);  // expand: B rows and y requested
   // the intermediate: parts summed in order, scaled, split, to LDS in operand rows (its first
   // kPartsAhead parts were requested with the record)
@@ -463,13 +475,13 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
       hi[j] = from_f32<T>(v);
       lo[j] = from_f32<T>(v - to_f32(hi[j]));
     }
-    __builtin_memcpy(__builtin_assume_aligned(s_h + tok * HROW + q4 * 4 * sizeof(T), 8), hi, sizeof(hi));
-    if constexpr (SPLIT) __builtin_memcpy(__builtin_assume_aligned(s_h + (16 + tok) * HROW + q4 * 4 * sizeof(T), 8), lo, sizeof(lo));
+    __builtin_memcpy(__builtin_assume_aligned(s_h + row_of_token(tok) * HROW + q4 * 4 * sizeof(T), 8), hi, sizeof(hi));
+    if constexpr (SPLIT) __builtin_memcpy(__builtin_assume_aligned(s_h + (16 + row_of_token(tok)) * HROW + q4 * 4 * sizeof(T), 8), lo, sizeof(lo));
   }
   __syncthreads();
   MLORA_STAMP(11);  // expand: intermediate in LDS
   if (!mine) return;
-  finish_spans<T, C, SP>(s_h, s_b, yq, ybase, ys, rows, c0, n1, m, eff);
+  finish_spans<T, C, SP, 4>(s_h, s_b, yq, ybase, ys, rows, c0, n1, m, eff);
 }
 
 #ifdef MLORA_TRACE
@@ -490,7 +502,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   const int tile = blockIdx.z * 8 + blockIdx.x;
   const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
   const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
-  const i32x4 rows = *reinterpret_cast<const i32x4*>(rec + MLORA_SMALL_TILE_ROWS + 4 * lg);  // tokens 4 * lg .. + 3
+  const i32x4 rows = spread_rows(rec, lg);
   const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
   const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
   // the intermediate's partial sums lie where the tile's place says: requested with the record
@@ -522,24 +534,24 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
 // record, sums and drain.  Figures: solo_columns.
 constexpr int kSoloWaves = 8;
 constexpr int kSoloThreads = kSoloWaves * kWave;
-template <int NA8> struct SoloShape {
+template <int NA8, int XG = 2> struct SoloShape {
   static constexpr int RB = (NA8 + 1) / 2;
-  static constexpr int ND = NA8 + 2;
+  static constexpr int ND = NA8 + XG;
   static constexpr int NST = ND <= 4 ? 3 : 2;
   static constexpr int BYTES = NST * ND * 1024;
 };
 
-template <typename T, int NA8, int R>
+template <typename T, int NA8, int R, int XG>
 __device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_bytes, const char* abase, uint32_t arow, const char* xbase,
                                             const uint32_t (&xoff)[2], int kchunks, int m, int eff, bool alone, float scaling) {
-  typedef SoloShape<NA8> S;
+  typedef SoloShape<NA8, XG> S;
   constexpr int RB = S::RB;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int c0 = wave * kchunks / kSoloWaves, c1 = (wave + 1) * kchunks / kSoloWaves;
   char* ring = rings + wave * S::BYTES;
   Chains<RB> chains;
   chains.clear();
-  walk_chunks<NA8, S>(ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
+  walk_chunks<NA8, XG, S>(ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
                       [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
   static_assert(RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
   f32x4 acc[RB];
@@ -562,7 +574,7 @@ __device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_byt
     const int tok = lane & 15, r0 = wave * 16 + 4 * (lane >> 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[i] = (tok < m && r0 + i < eff) ? s[i] * scaling : 0.f;
-    *reinterpret_cast<f32x4*>(s_h + tok * hrow_bytes + r0 * 4) = s;
+    *reinterpret_cast<f32x4*>(s_h + row_of_token(tok) * hrow_bytes + r0 * 4) = s;
   }
 }
 
@@ -580,7 +592,7 @@ __global__ __launch_bounds__(kSoloThreads) void solo_kernel(const int32_t* __res
   const int tile = blockIdx.z * 8 + blockIdx.x;
   const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
   const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
-  const i32x4 rows = *reinterpret_cast<const i32x4*>(rec + MLORA_SMALL_TILE_ROWS + 4 * lg);  // tokens 4 * lg .. + 3
+  const i32x4 rows = spread_rows(rec, lg);
   int row[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) row[i] = rec[MLORA_SMALL_TILE_ROWS + i * 8 + (lane >> 3)];
@@ -606,17 +618,23 @@ __global__ __launch_bounds__(kSoloThreads) void solo_kernel(const int32_t* __res
   T* const ybase = static_cast<T*>(yv_) + sp.y_col;
   const int c0 = sp.n0 + wave * 64;
   const bool mine = c0 < sp.n1;
-  YSpan<T> yq[1][4];
-  if (mine) request_b<T, C, 1>(s_b, bbase, c0, sp.n1, eff, false);
-  request_y<T, 1>(yq, ybase, ys, rows, c0, sp.n1);
   const int groups = (eff + 7) >> 3;
-  if (R <= 8 || groups <= 1) solo_shrink<T, 1, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
-  else if (R <= 16 || groups <= 2) solo_shrink<T, 2, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
-  else solo_shrink<T, 4, R>(lds, s_h, HROW, abase, arow, static_cast<const char*>(xv), xoff, kchunks, m, eff, false, scaling);
-  __syncthreads();
-  MLORA_STAMP(5);  // intermediate in LDS
-  if (!mine) return;
-  finish_spans<T, C, 1>(s_h, s_b, yq, ybase, ys, rows, c0, sp.n1, m, eff);
+  auto rest = [&](auto xi, auto xg) __attribute__((always_inline)) {
+    constexpr int XI = decltype(xi)::value, XG = decltype(xg)::value;
+    YSpan<T> yq[1][4];
+    if (mine) request_b<T, C, 1>(s_b, bbase, c0, sp.n1, eff, false);
+    request_y<T, 1, XI>(yq, ybase, ys, rows, c0, sp.n1);
+    const char* xb = static_cast<const char*>(xv);
+    if (R <= 8 || groups <= 1) solo_shrink<T, 1, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
+    else if (R <= 16 || groups <= 2) solo_shrink<T, 2, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
+    else solo_shrink<T, 4, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
+    __syncthreads();
+    MLORA_STAMP(5);  // intermediate in LDS
+    if (mine) finish_spans<T, C, 1, XI>(s_h, s_b, yq, ybase, ys, rows, c0, sp.n1, m, eff);
+  };
+  if (m <= 4) rest(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+  else if (m <= 8) rest(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+  else rest(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
 }
 
 int solo_ring(int r) {
