@@ -20,7 +20,7 @@
 // and counts the younger requests of this file's own.
 //
 // A slot's only tile (its segment has fewer than sixteen tokens) is the only one to ask for the slot's A and B lines, so
-// those carry the non-temporal hint: 201 tokens over 48 slots of mixed rank, K = 2048, us per call without / with: qkv
+// those carry the non-temporal hint where the call's weights are 8 MB or more (kOnceBytes): 201 tokens over 48 slots of mixed rank, K = 2048, us per call without / with: qkv
 // 17.5 / 16.8, gate_up 31.0 / 29.2, down 16.9 / 15.9.  Tiles of one slot do find lines of each other in the caches:
 // hinted as well, 900 tokens of 3 slots, rank 64, take 21.3 instead of 15.4 (qkv) and 18.2 instead of 13.0 (down).
 #include "common.h"
@@ -38,6 +38,10 @@ constexpr int kPairThreads = kPairWaves * kWave;
 constexpr int kChunk = 128;     // bytes of a row that a step of the shrink takes
 constexpr int kMaxParts = 8;    // most K parts of a launch
 constexpr int kPartsAhead = 4;  // of which the expand requests this many together
+// Below, a step's weights (about a hundred such calls) may still lie in the 256 MB of the memory-side cache when the next step comes, and
+// the hint gives that up: 5 tokens of 5 slots, rank 64, K = 1024, weights at hand, q|k|v 7.2 us per call without, 7.7 with, o 6.5 / 7.6; one token, K =
+// 2048, gate_up 8.6 / 9.1.
+constexpr long long kOnceBytes = 8ll << 20;
 
 // ---- shrink -------------------------------------------------------------------------------------
 // A wavefront's own share of a (tile, slice, K part): chunks [c0, c1) of 128 bytes of every row, through
@@ -54,9 +58,9 @@ template <int NA8> struct ShrinkShape {
 };
 
 // A wavefront's walk over chunks [c0, c1) of the rows.  XG: groups of eight token rows, one where the tile has no more tokens.  step(c): before chunk c is multiplied; multiply(rb, ks, a, x).
-template <int NA8, int XG, typename S, typename Step, typename Multiply>
+template <int NA8, int XG, bool ONCE, typename S, typename Step, typename Multiply>
 __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
-                                            int c0, int c1, bool alone, Step step, Multiply multiply) {
+                                            int c0, int c1, Step step, Multiply multiply) {
   constexpr int RB = S::RB, ND = S::ND, NST = S::NST;
   const int lane = threadIdx.x & (kWave - 1), lr = lane & 15, lg = lane >> 4;
   const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;
@@ -71,12 +75,10 @@ __device__ __forceinline__ void walk_chunks(char* ring, const char* abase, uint3
     const char* a = abase + static_cast<int64_t>(c) * kChunk;
     const char* x = xbase + static_cast<int64_t>(c) * kChunk;
     const uint32_t to = lds + stage * (ND * 1024);
-    if (alone) {
 #pragma unroll
-      for (int g = 0; g < NA8; ++g) dma16_once(a, aoff[g], to + g * 1024);
-    } else {
-#pragma unroll
-      for (int g = 0; g < NA8; ++g) dma16(a, aoff[g], to + g * 1024);
+    for (int g = 0; g < NA8; ++g) {
+      if constexpr (ONCE) dma16_once(a, aoff[g], to + g * 1024);
+      else dma16(a, aoff[g], to + g * 1024);
     }
 #pragma unroll
     for (int i = 0; i < XG; ++i) dma16(x, xoff[i] + swz, to + (NA8 + i) * 1024);
@@ -152,17 +154,17 @@ template <int RB> struct Chains {
 // CHAINS (fp32): eight chains per block of ranks instead of one, one per element of a piece and half of a chunk, for buffers of the ranks
 // whose calls one workgroup per token used to take, so that their error is no larger than that kernel's (rank 48, K = 1024, 2048
 // tokens: 2.2e-7 of the update, with one chain 2.4e-7); 0.2 us per call.
-template <typename T, int NA8, bool CHAINS>
+template <typename T, int NA8, bool CHAINS, bool ONCE>
 __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2],
-                                              int c0, int cm, int c1, bool alone, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
+                                              int c0, int cm, int c1, f32x4 (&first)[ShrinkShape<NA8>::RB], f32x4 (&acc)[ShrinkShape<NA8>::RB]) {
   constexpr int RB = ShrinkShape<NA8>::RB;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) first[rb] = acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
   if constexpr (CHAINS) {
     Chains<RB> chains;
     chains.clear();
-    walk_chunks<NA8, 2, ShrinkShape<NA8>>(
-        ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
+    walk_chunks<NA8, 2, ONCE, ShrinkShape<NA8>>(
+        ring, abase, arow, rbuf, xbase, xoff, c0, c1,
         [&](int c) {
           if (c == cm) {  // the first of the wavefront's two shares is complete
             chains.collect(first);
@@ -172,8 +174,8 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
         [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
     chains.collect(acc);
   } else {
-    walk_chunks<NA8, 2, ShrinkShape<NA8>>(
-        ring, abase, arow, rbuf, xbase, xoff, c0, c1, alone,
+    walk_chunks<NA8, 2, ONCE, ShrinkShape<NA8>>(
+        ring, abase, arow, rbuf, xbase, xoff, c0, c1,
         [&](int c) {
           if (c == cm) {  // the first of the wavefront's two shares is complete
 #pragma unroll
@@ -189,15 +191,15 @@ __device__ __forceinline__ void shrink_chunks(char* ring, const char* abase, uin
 }
 
 // dst: this tile's block of partial sums, sixteen rows of rp floats.
-template <typename T, int NA8, bool CHAINS>
+template <typename T, int NA8, bool CHAINS, bool ONCE>
 __device__ __forceinline__ void shrink_tile(char* lds, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2], int c0,
-                                            int cm, int c1, bool alone, float* __restrict__ dst, int rp, int m) {
+                                            int cm, int c1, float* __restrict__ dst, int rp, int m) {
   typedef ShrinkShape<NA8> S;
   constexpr int RB = S::RB;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   char* ring = lds + wave * S::BYTES;
   f32x4 first[RB], acc[RB];
-  shrink_chunks<T, NA8, CHAINS>(ring, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, first, acc);
+  shrink_chunks<T, NA8, CHAINS, ONCE>(ring, abase, arow, rbuf, xbase, xoff, c0, cm, c1, first, acc);
   // sum over the eighths of the part, the first one first, through the rings' memory
   static_assert(2 * RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
 #pragma unroll
@@ -238,7 +240,7 @@ __device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __r
 }
 
 // grid (8, slices * K parts, tiles / 8): blockIdx.x is the XCD, so that the workgroups of a tile share an L2.
-template <typename T, bool CHAINS>
+template <typename T, bool CHAINS, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
                                                                    int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, int rbuf,
                                                                    int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
@@ -275,13 +277,17 @@ __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t
   for (int i = 0; i < 2; ++i) xoff[i] = static_cast<uint32_t>(row[i]) * xrow;
   const int rp = (rbuf + 15) & ~15;
   float* dst = hws + (static_cast<int64_t>(part * num_slices + slice) * (gridDim.z * 8) + tile) * (MLORA_TILE_SMALL * rp);
-  const bool alone = __builtin_amdgcn_readfirstlane(t.alone) != 0;
   const int groups = (eff + 7) >> 3;
-  if (groups <= 1) shrink_tile<T, 1, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups == 2) shrink_tile<T, 2, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups <= 4) shrink_tile<T, 4, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else if (groups <= 6) shrink_tile<T, 6, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
-  else shrink_tile<T, 8, CHAINS>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, alone, dst, rp, m);
+  auto tile_of = [&](auto once) __attribute__((always_inline)) {
+    constexpr bool O = decltype(once)::value;
+    if (groups <= 1) shrink_tile<T, 1, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+    else if (groups == 2) shrink_tile<T, 2, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+    else if (groups <= 4) shrink_tile<T, 4, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+    else if (groups <= 6) shrink_tile<T, 6, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+    else shrink_tile<T, 8, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
+  };
+  if (ONCE && __builtin_amdgcn_readfirstlane(t.alone)) tile_of(std::true_type{});
+  else tile_of(std::false_type{});
 #ifdef MLORA_TRACE
   MLORA_STAMP(5);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -493,7 +499,7 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
 template <typename T, int C, int SP>
 __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws, void* __restrict__ yv_,
                                                                    int64_t ys, int small_off, int T_, int num_slots, int kparts, int num_slices,
-                                                                   float scaling, const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
+                                                                   float scaling, const int32_t* __restrict__ eff_rank, int once, ExpandSplits splits) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int R = C * PieceOf<T>::E, RP = (R + 15) & ~15;
   const int lane = threadIdx.x & (kWave - 1), lg = lane >> 4;
@@ -523,7 +529,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   if (eff == 0) return;
   const char* bbase = uniform(static_cast<const char*>(sp.b) + static_cast<int64_t>(slot) * sp.n * (C * 16));
   expand_tile<T, C, SP>(lds, hsrc, stride, kparts, hv, bbase, static_cast<T*>(yv_) + sp.y_col, ys, rows, sp.n0, sp.n1, m, eff,
-                        __builtin_amdgcn_readfirstlane(t.alone) != 0, scaling);
+                        (once & __builtin_amdgcn_readfirstlane(t.alone)) != 0, scaling);
   MLORA_STAMP_END(13);  // expand: stores issued, acknowledged
 }
 
@@ -543,7 +549,7 @@ template <int NA8, int XG = 2> struct SoloShape {
 
 template <typename T, int NA8, int R, int XG>
 __device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_bytes, const char* abase, uint32_t arow, const char* xbase,
-                                            const uint32_t (&xoff)[2], int kchunks, int m, int eff, bool alone, float scaling) {
+                                            const uint32_t (&xoff)[2], int kchunks, int m, int eff, float scaling) {
   typedef SoloShape<NA8, XG> S;
   constexpr int RB = S::RB;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -551,7 +557,7 @@ __device__ __forceinline__ void solo_shrink(char* rings, char* s_h, int hrow_byt
   char* ring = rings + wave * S::BYTES;
   Chains<RB> chains;
   chains.clear();
-  walk_chunks<NA8, XG, S>(ring, abase, arow, R, xbase, xoff, c0, c1, alone, [](int) {},
+  walk_chunks<NA8, XG, false, S>(ring, abase, arow, R, xbase, xoff, c0, c1, [](int) {},
                       [&](int rb, int ks, const Pack8& aw, const Pack8& xa) { chains.add(rb, ks, aw, xa); });
   static_assert(RB * 1024 <= S::BYTES, "the ring holds the wavefront's sums");
   f32x4 acc[RB];
@@ -625,9 +631,9 @@ __global__ __launch_bounds__(kSoloThreads) void solo_kernel(const int32_t* __res
     if (mine) request_b<T, C, 1>(s_b, bbase, c0, sp.n1, eff, false);
     request_y<T, 1, XI>(yq, ybase, ys, rows, c0, sp.n1);
     const char* xb = static_cast<const char*>(xv);
-    if (R <= 8 || groups <= 1) solo_shrink<T, 1, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
-    else if (R <= 16 || groups <= 2) solo_shrink<T, 2, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
-    else solo_shrink<T, 4, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, false, scaling);
+    if (R <= 8 || groups <= 1) solo_shrink<T, 1, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, scaling);
+    else if (R <= 16 || groups <= 2) solo_shrink<T, 2, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, scaling);
+    else solo_shrink<T, 4, R, XG>(lds, s_h, HROW, abase, arow, xb, xoff, kchunks, m, eff, scaling);
     __syncthreads();
     MLORA_STAMP(5);  // intermediate in LDS
     if (mine) finish_spans<T, C, 1, XI>(s_h, s_b, yq, ybase, ys, rows, c0, sp.n1, m, eff);
@@ -651,12 +657,13 @@ int expand_lds(int c, int sp) {
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
 struct PairKnobs {
-  int generation = -1, kparts, sp, wgs, solo, solo_cols;
+  int generation = -1, kparts, sp, wgs, solo, solo_cols, once;
   void read() {
     generation = knob_generation();
     kparts = env_int("MLORA_PAIR_KPARTS", 0);
     sp = env_int("MLORA_PAIR_SP", 0);
     wgs = env_int("MLORA_PAIR_WGS", 192);
+    once = env_int("MLORA_PAIR_ONCE", -1);
     solo = env_int("MLORA_SOLO", 1);  // 0: never in one launch, 2: wherever it can be
     solo_cols = env_int("MLORA_SOLO_COLS", 0) / 64 % 9 * 64;  // at most 512
   }
@@ -677,17 +684,23 @@ struct PairLaunch {
   const MloraAddArgs* a;
   PlanLayout lay;
   int parts_log2, sp;
+  bool once;  // A and B of a slot's only tile with the non-temporal hint
 };
 
-template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) {
+template <typename T, bool CHAINS, bool ONCE> void launch_pair_shrink_one(const PairLaunch& l) {
   const MloraAddArgs* a = l.a;
   ShrinkSlices sl;
   for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = i < a->num_slices ? a->slices[i].a : nullptr;
-  allow_lds<pair_shrink_kernel<T, CHAINS>>(shrink_lds(a->r));
-  hipLaunchKernelGGL((pair_shrink_kernel<T, CHAINS>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
+  allow_lds<pair_shrink_kernel<T, CHAINS, ONCE>>(shrink_lds(a->r));
+  hipLaunchKernelGGL((pair_shrink_kernel<T, CHAINS, ONCE>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
                      dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
                      a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
                      l.parts_log2, a->num_slices, a->effective_rank, sl);
+}
+
+template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) {
+  if (l.once) launch_pair_shrink_one<T, CHAINS, true>(l);
+  else launch_pair_shrink_one<T, CHAINS, false>(l);
 }
 
 template <typename T, int C, int SP> void launch_pair_expand_one(const PairLaunch& l, const ExpandSplits& splits, int total) {
@@ -695,7 +708,7 @@ template <typename T, int C, int SP> void launch_pair_expand_one(const PairLaunc
   allow_lds<pair_expand_kernel<T, C, SP>>(expand_lds(C, SP));
   hipLaunchKernelGGL((pair_expand_kernel<T, C, SP>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
                      expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
-                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, splits);
+                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, l.once ? 1 : 0, splits);
 }
 
 template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const ExpandSplits& splits, int total) {
@@ -832,6 +845,10 @@ int launch_pair(const MloraAddArgs* a, int active) {
   const int tiles = segs > by_tokens ? segs : by_tokens;  // about the number of tiles in use
   const int kchunks = static_cast<int>(static_cast<int64_t>(a->k) * element_bytes(a->dtype) / kChunk);
   const size_t room = partials_room(a) / part_bytes(a, l.lay);
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  const long long weights = static_cast<long long>(active > 0 ? active : segs) * a->r * (static_cast<long long>(a->num_slices) * a->k + cols) * element_bytes(a->dtype);
+  l.once = pair_knobs().once < 0 ? weights >= kOnceBytes : pair_knobs().once != 0;
   // K parts: workgroups for most compute units, no more (every column range of the second launch
   // takes in every part's sums), and a chunk per wavefront at least
   int want = pair_knobs().kparts;
