@@ -385,7 +385,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
     case MLORA_FORM_SLOT:
     case MLORA_FORM_MFMA: {
       if (!vec || !mfma_supported(a)) { set_error("mlora_add_lora: MFMA forms need 16-bit elements, a plan, a rank that is a multiple of 8 up to 64 and K %% 32 == 0"); return MLORA_E_UNSUPPORTED; }
-      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true);
+      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true, active);
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "

@@ -30,7 +30,7 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 // decode.hip: the same small tiles with both products on the matrix cores, one workgroup per
 // (tile, column range).
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
-int launch_decode(const MloraAddArgs* a, bool include_long);
+int launch_decode(const MloraAddArgs* a, bool include_long, int active);  // active: slots with tokens where the host counted them, else 0
 int decode_ranges(const MloraAddArgs* a, int* columns);  // column ranges of that launch, and columns per range
 
 // slot.hip: the same small tiles, the grid laid over the slots: weights are requested from the
