@@ -111,6 +111,12 @@ __global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SA, SHORT)) void 
   const int split_id = blockIdx.y;
   const int tile = blockIdx.z * 8 + blockIdx.x;
 
+  // URGENT: up to the x and A rows a wavefront goes before those that are at their B rows and y: 64 tokens of 32 slots, rank 32, q|k|v 4.47 -> 4.31 us per call,
+  // o of 100 tokens of 60 4.36 -> 4.19.  Not with two spans each (gate_up of 200 tokens of 30, rank 24, 8.15 -> 8.37) and not with two
+  // workgroups on a compute unit (3001 tokens, K = 2048, rank 16, q|k|v 14.0 -> 16.4); nothing at the other ranks.
+  constexpr bool URGENT = TR && KSPW == 4 && SA == 1 && R == 32;
+  if constexpr (URGENT) __builtin_amdgcn_s_setprio(3);
+
   // ---- round trip 1 ---------------------------------------------------------------------------
   const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;  // tile < capacity: in bounds
   const int row = rec[MLORA_SMALL_TILE_ROWS + lr];
@@ -350,9 +356,9 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
   l.staged = decode_knobs().staged;
   // The texts for short tiles pay where there are some: prompts fill their tiles, and the launch's workgroups then run the last of three texts
   // for the price of the others (155 tokens of 3 slots, us per call without / with them: rank 48 q|k|v 8.4 / 8.6, gate_up 9.7 / 10.0, rank 32 5.5 / 5.6;
-  // 64 tokens of 32 slots, rank 32, 4.8 / 4.5 and 7.5 / 7.1): up to twelve tokens per slot with tokens.
+  // 64 tokens of 32 slots, rank 32, 4.8 / 4.5 and 7.5 / 7.1): up to twelve tokens per slot with tokens.  With two spans per wavefront, whose texts
+  // are longer, up to four (128 tokens of 16 slots, K = 2048, rank 16, gate_up 7.4 / 7.9; 200 of 30, rank 24, 8.2 / 8.2; 100 of 60, rank 32, 12.1 / 11.3).
   const int with_tokens = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  l.short_tiles = a->num_tokens <= 12 * with_tokens;
 
   int nt;
   const int total = decode_ranges(a, &nt);
@@ -368,6 +374,7 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
       if (d.n1 - d.n0 > l.widest) l.widest = d.n1 - d.n0;
     }
   }
+  l.short_tiles = a->num_tokens <= (l.widest <= kNW * 64 ? 12 : 4) * with_tokens;
   for (; s < kMaxSplits; ++s) splits.split[s] = DecodeSplit{nullptr, nullptr, 0, 0, 0, 0};
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(cap / 8));
   const int nks = a->k / 32;

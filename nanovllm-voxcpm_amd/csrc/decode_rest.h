@@ -34,6 +34,11 @@
       }
     }
   }
+  if constexpr (URGENT) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   constexpr int kSpansAhead = SA;
   Pack8 bop[kSpansAhead][4][KSTEPS], yreg[kSpansAhead][2];
   uint2 yq[TR ? kSpansAhead : 1][TR ? 4 : 1];  // TR: four columns of four tokens per lane and span

@@ -101,6 +101,12 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
   const int lr = lane & 15, lg = lane >> 4;
   const int rbuf = GR ? rbuf_arg : R;  // rank of the buffers: row count of A[slot], row length of B
 
+  // URGENT: up to the x rows a wavefront goes before those that are at their B rows and y.  With two spans each those are half of what a compute
+  // unit hands over: 256 tokens of 32 slots, rank 16, gate_up 6.44 -> 6.21 us per call; with one span it costs more than it brings (o of 64 tokens
+  // of 32, rank 32, 3.9 -> 4.1).
+  constexpr bool URGENT = KP == 1 && SA == 2;
+  if constexpr (URGENT) __builtin_amdgcn_s_setprio(3);
+
   // ---- requests that depend on nothing but the workgroup index --------------------------------
   // (the token rows as a vector load, four per lane group: all sixteen through the scalar cache
   // into scalar registers measured slower, 556 -> 598 us per decode step in the tile-major kernel)

@@ -8,6 +8,11 @@
 #pragma unroll
     for (int i = 0; i < XI; ++i) xst[4 * r + i] = load128(static_cast<const T*>(xv) + static_cast<int64_t>(rows4[i]) * xs + koff);
   }
+  if constexpr (URGENT) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // (the B rows behind the x rows: they are not needed before the expand, and in front of the
   // record's wait they would hold the x rows up for as long as it takes to hand them over)
   request_b(slot);
