@@ -496,10 +496,10 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
 #define MLORA_STAMP_END(i) do { } while (0)
 #endif
 // grid (8, column ranges, tiles / 8)
-template <typename T, int C, int SP>
+template <typename T, int C, int SP, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws, void* __restrict__ yv_,
                                                                    int64_t ys, int small_off, int T_, int num_slots, int kparts, int num_slices,
-                                                                   float scaling, const int32_t* __restrict__ eff_rank, int once, ExpandSplits splits) {
+                                                                   float scaling, const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int R = C * PieceOf<T>::E, RP = (R + 15) & ~15;
   const int lane = threadIdx.x & (kWave - 1), lg = lane >> 4;
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   if (eff == 0) return;
   const char* bbase = uniform(static_cast<const char*>(sp.b) + static_cast<int64_t>(slot) * sp.n * (C * 16));
   expand_tile<T, C, SP>(lds, hsrc, stride, kparts, hv, bbase, static_cast<T*>(yv_) + sp.y_col, ys, rows, sp.n0, sp.n1, m, eff,
-                        (once & __builtin_amdgcn_readfirstlane(t.alone)) != 0, scaling);
+                        ONCE && __builtin_amdgcn_readfirstlane(t.alone) != 0, scaling);
   MLORA_STAMP_END(13);  // expand: stores issued, acknowledged
 }
 
@@ -703,17 +703,22 @@ template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) 
   else launch_pair_shrink_one<T, CHAINS, false>(l);
 }
 
-template <typename T, int C, int SP> void launch_pair_expand_one(const PairLaunch& l, const ExpandSplits& splits, int total) {
+template <typename T, int C, int SP, bool ONCE> void launch_pair_expand_one(const PairLaunch& l, const ExpandSplits& splits, int total) {
   const MloraAddArgs* a = l.a;
-  allow_lds<pair_expand_kernel<T, C, SP>>(expand_lds(C, SP));
-  hipLaunchKernelGGL((pair_expand_kernel<T, C, SP>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
+  allow_lds<pair_expand_kernel<T, C, SP, ONCE>>(expand_lds(C, SP));
+  hipLaunchKernelGGL((pair_expand_kernel<T, C, SP, ONCE>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
                      expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
-                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, l.once ? 1 : 0, splits);
+                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, splits);
 }
 
 template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const ExpandSplits& splits, int total) {
-  if (l.sp == 1) launch_pair_expand_one<T, C, 1>(l, splits, total);
-  else launch_pair_expand_one<T, C, 2>(l, splits, total);
+  if (l.sp == 1) {
+    if (l.once) launch_pair_expand_one<T, C, 1, true>(l, splits, total);
+    else launch_pair_expand_one<T, C, 1, false>(l, splits, total);
+  } else {
+    if (l.once) launch_pair_expand_one<T, C, 2, true>(l, splits, total);
+    else launch_pair_expand_one<T, C, 2, false>(l, splits, total);
+  }
   return true;
 }
 

@@ -103,8 +103,8 @@ __device__ __forceinline__ void slot_tile(const int32_t* __restrict__ rec, const
 
   // URGENT: up to the x rows a wavefront goes before those that are at their B rows and y.  With two spans each those are half of what a compute
   // unit hands over: 256 tokens of 32 slots, rank 16, gate_up 6.44 -> 6.21 us per call; with one span it costs more than it brings (o of 64 tokens
-  // of 32, rank 32, 3.9 -> 4.1).
-  constexpr bool URGENT = KP == 1 && SA == 2;
+  // of 32, rank 32, 3.9 -> 4.1), and above rank 16 too (352 of 28, rank 32, gate_up 12.7 -> 13.0).
+  constexpr bool URGENT = KP == 1 && SA == 2 && R <= 16;
   if constexpr (URGENT) __builtin_amdgcn_s_setprio(3);
 
   // ---- requests that depend on nothing but the workgroup index --------------------------------
