@@ -414,6 +414,10 @@ __device__ __forceinline__ void finish_spans(const char* s_h, const char* s_b, c
         out[j] = Mma<T>::run(hop[ks], bo, out[j]);
       }
     }
+    // (Rows that hold no token stay the products' own to the end: handed out again, their registers would be written by the masking between
+    // the products, on whose branches the compiler does not always keep the distance an MFMA's result needs.)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(out[j]));
     if (c < n1) {
 #pragma unroll
       for (int i = 0; i < XI; ++i) {
