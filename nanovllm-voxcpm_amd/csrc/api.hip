@@ -417,7 +417,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
         }
         return launch_fused(a, trusted_workspace);
       }
-      return launch_sgmv(a);
+      return launch_sgmv(a, active);
     }
   }
   set_error("mlora_add_lora: unreachable form %d", form);

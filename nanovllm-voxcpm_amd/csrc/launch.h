@@ -52,12 +52,12 @@ int workspace_init(void* workspace, hipStream_t stream);
 bool sgmv_supported(const MloraAddArgs* a);
 bool sgmv_workspace_ok(const MloraAddArgs* a);
 size_t sgmv_workspace_bytes(int num_tokens, int num_slices, int r, int dtype);
-int launch_sgmv(const MloraAddArgs* a);
+int launch_sgmv(const MloraAddArgs* a, int active);  // active: slots with tokens where the host counted them, else 0
 
 // slab.hip: the shrink launch of that form, operands through LDS by direct loads.
 struct PlanLayout;
 bool slab_supported(const MloraAddArgs* a);
-void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const void* const* slices);
+void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, bool deep, const void* const* slices);
 
 // fused.hip: the same tiles, shrink and expand in one launch (workgroups of a unit exchange the
 // intermediate through the workspace under seals kept in its head).

@@ -255,13 +255,13 @@ bool sgmv_workspace_ok(const MloraAddArgs* a) {
 }
 
 // Every segment of the batch: 64-token tiles of the long ones, one short tile each for the rest.
-int launch_sgmv(const MloraAddArgs* a) {
-  const SgmvShape sh = sgmv_shape(a);
+int launch_sgmv(const MloraAddArgs* a, int active) {
+  const SgmvShape sh = sgmv_shape(a, false, active);
   if (sh.empty) return 0;
   ShrinkLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.tiles8 = sh.tiles8; l.big_cap = sh.big_cap;
   l.ksplit = sh.ksplit; l.krange = sh.krange; l.all_slices = sh.all_slices;
-  if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.sl.a);
+  if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.slab_deep, sh.sl.a);
   else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink_rank<__bf16>(l, sh.kr, sh.xw);
   else launch_shrink_rank<_Float16>(l, sh.kr, sh.xw);
   int rc = check_launch("mlora_add_lora(sgmv shrink)");

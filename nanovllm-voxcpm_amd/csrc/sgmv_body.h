@@ -813,7 +813,7 @@ struct SgmvKnobs {
     nt = env_int("MLORA_SGMV_NT", 0);
     cpl = env_int("MLORA_SGMV_CPL", 8);
     stream = env_int("MLORA_SGMV_STREAM", -1);
-    slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay
+    slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay, 3: rank 64 so with deep rings
   }
 };
 const SgmvKnobs& sgmv_knobs() {
@@ -859,6 +859,7 @@ struct SgmvShape {
   int kr, xw;     // shrink: A slab width, x batch width
   int ksplit, krange, all_slices;
   bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
+  bool slab_deep; // ... with its deep rings
   int group;      // expand: consecutive 64-token tiles per workgroup
   int cpl;        // expand: columns per lane
   bool stream;    // expand: y with the non-temporal hint
@@ -870,7 +871,7 @@ struct SgmvShape {
 
 // one_launch: the cut for the form whose workgroups do both products (256-column slabs and batches,
 // which leave the registers the kernel needs besides; as many shrink roles per unit as it has workgroups).
-inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
+inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int active = 0) {
   SgmvShape s;
   s.empty = true;
   s.lay = plan_layout(a->num_tokens, a->num_slots);
@@ -935,13 +936,44 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false) {
   // 39.0 / 33.0, gate_up 85.4 / 84.7, o 25.0 / 24.6, down (K = 4096) 43.9 / 46.8; rank 64, 8192 mixed
   // tokens: 41.8 / 39.6, 99.0 / 98.3, 24.7 / 23.5, 44.5 / 45.9; rank 64, 4000 tokens, K = 2048: qkv 35.0 / 28.4;
   // rank 32, 5000 tokens: 19.3 / 18.5, 50.3 / 49.6, 13.6 / 13.5, 21.0 / 18.5; rank 32, 2000 tokens: 14.7 / 12.1,
-  // 21.3 / 19.3, 12.0 / 11.0, 14.3 / 13.4.  At rank 64 a workgroup of it holds half a compute unit's LDS,
+  // 21.3 / 19.3, 12.0 / 11.0, 14.3 / 13.4.  At rank 64 a workgroup of it holds 64 KB of LDS,
   // and what is left of the last round of long parts costs about what the operands' path saves.
   // (Whoever asks for the two-launch form by name gets the shrink whose sums the one-launch form repeats bit by bit:
   // slab.hip adds K up in another order.)
   s.slab = !one_launch && slab_supported(a) &&
            (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
-  if (s.slab) {
+  // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
+  // those, per slot): slab.hip with deep rings, while an XCD's workgroups number no more than its 32 compute units (a second
+  // round loses: 5000 tokens of 6 slots in three parts, 33 workgroups on some XCDs, K = 4096 27.6 / 30.7, 3072 36.1 / 41.5).  Parts need
+  // not divide K, so they fill the chip where the other shrink's powers of two halve it.  us per call, the other shrink / this, 2 slots: K = 4096
+  // of 3200 tokens 19.5 / 18.6, 4500 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192, 4500 47.5 / 39.1; K = 2560, 4000 32.7 / 25.5; K = 3072,
+  // 3600 28.5 / 26.4; K = 2048, 6000 29.1 / 26.6; two slices K = 1024, 7000 59.4 / 56.2; K = 2048, 3200 58.5 / 55.7.  The other one
+  // stays where its own parts fit a round and are more (K = 2048, 4000 tokens, four parts of 512 against two 17.9 / 18.8; K = 1024, two
+  // slices, 43.1 / 44.5) or fill it (K = 4096, 20.2 / 20.7), for parts that would be longer than 2800 columns, below half a
+  // round, and for short segments, whose tiles the host can only guess: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens
+  // 23.2 / 25.7.  The guess is off by a tile or two at the edges: 3800 tokens of 12 slots, 64 tiles taken for 66, K = 2048 17.7 / 18.7.
+  // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7, 4096 2.7e-7 / 2.3e-7, 8192 5.3e-7 / 4.4e-7).
+  s.slab_deep = false;
+  const int slots = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+  const bool deep_knob = sgmv_knobs().slab == 3;
+  if (!one_launch && slab_supported(a) && a->r == 64 && a->num_slices <= 2 && slots > 0 && max_parts > 0 &&
+      (deep_knob || (sgmv_knobs().slab == 1 && a->form == MLORA_FORM_AUTO && a->num_tokens / slots >= 4 * MLORA_TILE_BIG))) {
+    const int tiles = static_cast<int>((a->num_tokens + 63ll + 32ll * slots) / MLORA_TILE_BIG);  // a slot's last tile is half full
+    const int per_xcd = (tiles + 7) / 8 * a->num_slices;
+    int parts = 32 / per_xcd;
+    if (parts > (a->num_slices == 1 ? kMaxKSplit : 2)) parts = a->num_slices == 1 ? kMaxKSplit : 2;
+    if (parts > max_parts) parts = max_parts;
+    if (parts > a->k / 1024) parts = a->k / 1024;
+    if (parts < 1 && deep_knob) parts = 1;
+    const bool other_fits = per_xcd * ksplit <= 32, full = a->num_slices == 1 && per_xcd * parts == 32 && a->k <= 1024 * parts;
+    s.slab_deep = deep_knob || (parts > 0 && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128 && !(other_fits && (parts < ksplit || full)));
+    if (s.slab_deep) ksplit = parts;
+    s.slab |= s.slab_deep;
+  }
+  if (s.slab_deep) {
+    s.all_slices = 0;
+    s.ksplit = ksplit;
+  } else if (s.slab) {
     // About 205 workgroups (parts need not be a power of two), a stage of K per wavefront at least.  Measured, us
     // per call with one / two / three / four parts, rank 32: down (K = 4096) of 2000 tokens 20.8 / 15.7 / 14.0 / 13.4,
     // of 4000 22.3 / 17.5 / 16.6 / 18.1, of 5000 23.4 / 18.5 / 20.8 / 19.2, of 6500 29.6 / 22.4 / 25.0 / 23.1; K = 8192,

@@ -1,0 +1,74 @@
+"""The shrink through LDS with deep rings (csrc/slab.hip, rank 64, one or two slices) at the sizes where it can go wrong: K of
+fewer 128-byte pieces per wavefront than the ring has stages, tiles of every number of 16-token blocks, uneven K
+parts, adapters below the buffers' rank with NaN beyond it; and the automatic choice on both sides of its lines."""
+
+import random
+import types
+
+import pytest
+import torch
+
+from test_gpu_parity import _check, _exact
+
+B16, F16 = torch.bfloat16, torch.float16
+
+# segment lengths, K, widths, element type, adapters of lower rank, every fourth segment without adapter, forced
+CASES = [
+    ([64], 128, [8], B16, False, False, True),
+    ([16, 17, 1, 15], 128, [520, 64], F16, False, False, True),
+    ([32, 33, 48, 49, 3], 384, [264], B16, True, True, True),
+    ([130, 20, 64, 31, 5], 2560, [512], F16, True, True, True),
+    ([257, 16, 90], 4096, [72, 200], B16, True, False, True),
+    ([2100, 2400], 2560, [2560], B16, False, False, False),  # two parts of 1280
+    ([1500, 1700, 1300], 4096, [1024], F16, True, False, False),  # three parts
+    ([1600, 1701, 1699], 4096, [1024], B16, False, False, False),  # three parts would be a second round on some XCDs: two
+    ([1000, 2200], 2048, [2048, 2048], B16, False, False, False),
+    ([250] * 14, 2560, [2560], B16, False, False, False),  # short segments: the other shrink
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_deep_rings_against_fp64(case, monkeypatch):
+    from nanovllm_voxcpm_amd import _hip
+    from nanovllm_voxcpm_amd.lora_ops.segment_meta import build_segment_plan
+
+    lengths, k, widths, dtype, mixed, holes, forced = CASES[case]
+    print(f"deep rings {case} {k} {widths}", flush=True)
+    pick, g = random.Random(case), torch.Generator().manual_seed(case)
+    slots, rank = len(lengths), 64
+    ids = [-1 if holes and i % 4 == 3 else i for i, n in enumerate(lengths) for _ in range(n)]
+    pick.shuffle(ids)
+    indices, tokens = torch.tensor(ids, dtype=torch.int32), len(ids)
+    a = [(torch.randn(slots, rank, k, generator=g) * 0.05).to(dtype) for _ in widths]
+    b = [(torch.randn(slots, n, rank, generator=g) * 0.1).to(dtype) for n in widths]
+    x, y = torch.randn(tokens, k, generator=g).to(dtype), torch.randn(tokens, sum(widths), generator=g).to(dtype)
+    ranks = [pick.choice([1, 8, 13, 32, 64]) if mixed else rank for _ in range(slots)]
+    shown_a, shown_b = [t.clone() for t in a], [t.clone() for t in b]  # what the oracle sees: zeros beyond a slot's rank
+    for s, r in enumerate(ranks):
+        for t, z in zip(a, shown_a):
+            t[s, r:], z[s, r:] = float("nan"), 0
+        for t, z in zip(b, shown_b):
+            t[s, :, r:], z[s, :, r:] = float("nan"), 0
+    dev = [t.cuda() for t in a], [t.cuda() for t in b]
+    eff = torch.tensor(ranks, dtype=torch.int32, device="cuda") if mixed else None
+    plan = build_segment_plan(indices.cuda(), slots)
+    scratch = torch.empty(_hip.add_workspace_bytes(tokens, len(widths), rank, dtype), dtype=torch.uint8, device="cuda")
+    _hip.workspace_init(scratch)
+    cols = [sum(widths[:i]) for i in range(len(widths))]
+    runs = []
+    try:
+        if forced:
+            monkeypatch.setenv("MLORA_SLAB", "3")
+            _hip.reload_knobs()
+        for _ in range(2):
+            out = y.cuda()
+            _hip.add_lora(out, x.cuda(), *dev, cols, indices.cuda(), plan.workspace, 0.75, _hip.FORM_SGMV if forced else _hip.FORM_AUTO, scratch,
+                          effective_rank=eff)
+            runs.append(out.cpu())
+    finally:
+        monkeypatch.undo()
+        _hip.reload_knobs()
+    assert torch.equal(runs[0], runs[1])
+    exact, mag = _exact(types.SimpleNamespace(a=shown_a, b=shown_b, widths=widths), x, y, indices, 0.75)
+    _check(runs[0], y, exact, mag, indices, f"deep rings {case}")
