@@ -946,10 +946,11 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   // those, per slot): slab.hip with deep rings, while an XCD's workgroups number no more than its 32 compute units (a second
   // round loses: 5000 tokens of 6 slots in three parts, 33 workgroups on some XCDs, K = 4096 27.6 / 30.7, 3072 36.1 / 41.5).  Parts need
   // not divide K, so they fill the chip where the other shrink's powers of two halve it.  us per call, the other shrink / this, 2 slots: K = 4096
-  // of 3200 tokens 19.5 / 18.6, 4500 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192, 4500 47.5 / 39.1; K = 2560, 4000 32.7 / 25.5; K = 3072,
+  // of 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192, 4500 47.5 / 39.1; K = 2560, 4000 32.7 / 25.5; K = 3072,
   // 3600 28.5 / 26.4; K = 2048, 6000 29.1 / 26.6; two slices K = 1024, 7000 59.4 / 56.2; K = 2048, 3200 58.5 / 55.7.  The other one
   // stays where its own parts fit a round and are more (K = 2048, 4000 tokens, four parts of 512 against two 17.9 / 18.8; K = 1024, two
-  // slices, 43.1 / 44.5) or fill it (K = 4096, 20.2 / 20.7), for parts that would be longer than 2800 columns, below half a
+  // slices, 43.1 / 44.5) or, with one slice, as many (K = 4096, 3200 tokens 19.5 / 18.6, 4000 20.2 / 20.7; its bits are those by name), for
+  // parts that would be longer than 2800 columns, below half a
   // round, and for short segments, whose tiles the host can only guess: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens
   // 23.2 / 25.7.  The guess is off by a tile or two at the edges: 3800 tokens of 12 slots, 64 tiles taken for 66, K = 2048 17.7 / 18.7.
   // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7, 4096 2.7e-7 / 2.3e-7, 8192 5.3e-7 / 4.4e-7).
@@ -965,8 +966,8 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
     if (parts > max_parts) parts = max_parts;
     if (parts > a->k / 1024) parts = a->k / 1024;
     if (parts < 1 && deep_knob) parts = 1;
-    const bool other_fits = per_xcd * ksplit <= 32, full = a->num_slices == 1 && per_xcd * parts == 32 && a->k <= 1024 * parts;
-    s.slab_deep = deep_knob || (parts > 0 && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128 && !(other_fits && (parts < ksplit || full)));
+    const bool other_stays = per_xcd * ksplit <= 32 && parts < ksplit + (a->num_slices == 1);
+    s.slab_deep = deep_knob || (parts > 0 && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128 && !other_stays);
     if (s.slab_deep) ksplit = parts;
     s.slab |= s.slab_deep;
   }
