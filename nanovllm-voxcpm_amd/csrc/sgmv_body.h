@@ -944,30 +944,31 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
            (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
   // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
   // those, per slot): slab.hip with deep rings, while an XCD's workgroups number no more than its 32 compute units (a second
-  // round loses: 5000 tokens of 6 slots in three parts, 33 workgroups on some XCDs, K = 4096 27.6 / 30.7, 3072 36.1 / 41.5).  Parts need
-  // not divide K, so they fill the chip where the other shrink's powers of two halve it.  us per call, the other shrink / this, 2 slots: K = 4096
-  // of 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192, 4500 47.5 / 39.1; K = 2560, 4000 32.7 / 25.5; K = 3072,
-  // 3600 28.5 / 26.4; K = 2048, 6000 29.1 / 26.6; two slices K = 1024, 7000 59.4 / 56.2; K = 2048, 3200 58.5 / 55.7.  The other one
-  // stays where its own parts fit a round and are more (K = 2048, 4000 tokens, four parts of 512 against two 17.9 / 18.8; K = 1024, two
-  // slices, 43.1 / 44.5) or, with one slice, as many (K = 4096, 3200 tokens 19.5 / 18.6, 4000 20.2 / 20.7; its bits are those by name), for
-  // parts that would be longer than 2800 columns, below half a
-  // round, and for short segments, whose tiles the host can only guess: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens
-  // 23.2 / 25.7.  The guess is off by a tile or two at the edges: 3800 tokens of 12 slots, 64 tiles taken for 66, K = 2048 17.7 / 18.7.
-  // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7, 4096 2.7e-7 / 2.3e-7, 8192 5.3e-7 / 4.4e-7).
+  // round loses: 5000 tokens of 6 slots in three parts, 33 workgroups on some XCDs, K = 3072 36.1 / 41.5) and it cuts K into more parts
+  // than the other shrink, whose parts have to divide K (with two slices into as many).  us per call, the other shrink / this, 2 slots: K = 2560,
+  // 4096 tokens 32.4 / 25.8; K = 3072, 3600 27.8 / 25.4; two slices, K = 2560, 6400 52.6 / 52.0; 423 such calls of 2 to 16 slots, K 1536 to 5120, take
+  // 0.67 to 1.00 of the other's time.  With fewer parts it can win too (K = 4096, 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192,
+  // 4500 47.5 / 39.1), but only on as many tiles as the tokens could make: tokens without an adapter make none, how many those are
+  // the host does not say, and with a quarter to three quarters of them two or three parts leave compute units idle
+  // that four would fill (K = 4096, 5200 tokens of 2 slots, half of them adapted, 18.2 / 21.2; K = 2048, 8000 of 12, 19.6 / 23.6; 124 of 171 such
+  // calls slower).  Not for
+  // parts that would be longer than 2800 columns nor below half a
+  // round, and not for short segments: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens 23.2 / 25.7.
+  // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7).
   s.slab_deep = false;
   const int slots = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
   const bool deep_knob = sgmv_knobs().slab == 3;
   if (!one_launch && slab_supported(a) && a->r == 64 && a->num_slices <= 2 && slots > 0 && max_parts > 0 &&
       (deep_knob || (sgmv_knobs().slab == 1 && a->form == MLORA_FORM_AUTO && a->num_tokens / slots >= 4 * MLORA_TILE_BIG))) {
-    const int tiles = static_cast<int>((a->num_tokens + 63ll + 32ll * slots) / MLORA_TILE_BIG);  // a slot's last tile is half full
+    const int tiles = static_cast<int>((a->num_tokens + 63ll * slots) / MLORA_TILE_BIG);  // at most: every slot's last tile has one token
     const int per_xcd = (tiles + 7) / 8 * a->num_slices;
     int parts = 32 / per_xcd;
     if (parts > (a->num_slices == 1 ? kMaxKSplit : 2)) parts = a->num_slices == 1 ? kMaxKSplit : 2;
-    if (parts > max_parts) parts = max_parts;
     if (parts > a->k / 1024) parts = a->k / 1024;
+    if (deep_knob && sgmv_knobs().ksplit > 0) parts = sgmv_knobs().ksplit < kMaxKSplit ? sgmv_knobs().ksplit : kMaxKSplit;
+    if (parts > max_parts) parts = max_parts;
     if (parts < 1 && deep_knob) parts = 1;
-    const bool other_stays = per_xcd * ksplit <= 32 && parts < ksplit + (a->num_slices == 1);
-    s.slab_deep = deep_knob || (parts > 0 && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128 && !other_stays);
+    s.slab_deep = deep_knob || (parts >= ksplit + (a->num_slices == 1) && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128);
     if (s.slab_deep) ksplit = parts;
     s.slab |= s.slab_deep;
   }
