@@ -16,13 +16,19 @@ MLORA_TRACE_DECL
 constexpr int kMaxSplits = 64;
 constexpr int kExpandWaves = 4;
 constexpr int kSlabStages = 4;  // 128-byte pieces of K in a part of slab.hip's at least
-// Bytes of y from which on the expand launch touches it with the non-temporal hint, plain / with it.  The launch by itself,
-// gate_up, us per call: rank 64 9392 tokens (154 MB) 62.9 / 56.4, 6500 (106 MB) 55.2 / 50.7, 5000 (82 MB) 58.3 / 51.5, rank 16 3001
-// tokens x 16384 columns (98 MB) 51.8 / 44.8; mixed batch of 8192 tokens 97.6 / 90.2: a read-modify-write stream at 4.1 -> 4.6
-// TB/s, gate_up's expand at 4.8 -> 5.4.  Between a copy that writes y and one that reads it (all three, us): 131 MB 154.6 / 150.0, 124 MB
-// 143.9 / 136.3, 106 MB 123.2 / 123.8, 82 MB 106.5 / 108.7, and below, where the memory-side cache still holds what the launch
-// before has written, it costs what it gains or more (19 MB: 43.8 / 44.9).  Hint on the loads only 60.9, on the stores only 62.7.
-constexpr long long kStreamBytes = 80ll << 20;
+// Bytes of y from which on the expand launch touches it with the non-temporal hint.  The line is drawn between a launch that has
+// written y and one that reads it, as in a model, for what the hint saves here (y evicts neither A nor B nor the sums) it costs there: what
+// the writer left in the memory-side cache and what the reader would find in it.  gate_up, us, plain and what the hint adds, in a matrix product +
+// apply + SwiGLU / a copy + apply + a copy / the apply by itself (MB = 2^20 bytes; the first within 0.5 to 1, the others within 0.2):
+//   rank 64, K = 1024, 8 slots    78 MB 190 +1.5 / 106 +1.0 / 50 -2.4   102 MB 212 +1.4 / 129 -2.2 / 58 -4.5   125 MB 246 -1.9 / 158 +0.4 / 67 -4.9
+//                                147 MB 317 -1.7 / 194 -1.8 / 82 -7.2
+//   rank 64, K = 2048, 5 slots   100 MB 301 -3.1 / 137 +1.5 / 68 -7.4   138 MB 447 -2.0 / 180 +0.1 / 79 -9.0   188 MB 486 -2.6 / 240 -6.1 / 98 -10
+//   mixed ranks of 128 slots     109 MB 261 +1.8 / 174 -1.5 / 93 -2.5   128 MB 284 +3.3 / 190 -0.9 / 98 -3.1   147 MB 350 +1.5 / 220 -7.3 / 107 -4.6
+//   rank 32, K = 1024            125 MB 239 -1.3 / 147 +0.3 / 60 -4.8   147 MB 313 -1.3 / 181 -0.9 / 74 -8.2   256 MB 475 -9.4 / 316 -9.2 / 123 -13
+//   rank 16, K = 2048             78 MB 247 +1.3 / 98 +2.9 / 42 -2.9     94 MB 247 +0.2 / 115 -0.2 / 49 -3.9   128 MB 325 +3.1 / 154 -0.7 / 65 -5.2
+//                                138 MB 433 +3.2 / 167 +2.6 / 68 -6.0   188 MB 476 -0.1 / 226 -3.2 / 88 -8.6   256 MB 636 -2.9 / 317 -8.6 / 122 -12
+// Up to 138 MB one or the other of the two pays for it somewhere, from 147 MB on they gain or stay within half a percent.
+constexpr long long kStreamBytes = 140ll << 20;
 constexpr int kMaxKSplit = 4;  // most K parts the shrink ever uses (the workspace has room for them)
 
 struct ShrinkSlices {
