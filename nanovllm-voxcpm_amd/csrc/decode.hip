@@ -73,14 +73,16 @@ struct DecodeSplits {
 // 32; 40, 48, 56 in the one for 64): rows of A[slot] are rbuf * K apart, B rows rbuf elements long, and
 // whatever lies beyond rbuf is treated like the ranks beyond an adapter's own (requests clamped
 // into the buffers, values masked).
-// Two workgroups per compute unit (at most 128 registers) where the LDS holds two, up to rank 16; three texts would take more: 3001 tokens of 5
-// slots, K = 2048, rank 16, q|k|v 14.2 us per call, o 10.3; with one, 17.1 and 11.7.  (Rank 32 in 72 KB, its blocks of A staged one by one, and
+// Two workgroups per compute unit (at most 128 registers) where the LDS holds two: up to rank 16 and K = 2048, where the last text alone stays
+// below that by itself and three texts with two spans (rank 8 150 registers, rank 16 146) would not.  us per call with one / two, every tile short, K = 2048,
+// rank 8: gate_up of 64 tokens of 32 slots 8.3 / 6.8, of 256 of 64 16.6 / 13.5, q|k|v of 128 of 64 5.4 / 4.8; rank 16: 9.3 / 7.7, 19.1 / 16.2, 6.6 / 6.4.
+// Nothing at K = 3072, rank 8, where the bound spills (o of 16 tokens of 16 slots 4.27 / 4.39).  (Rank 32 in 72 KB, its blocks of A staged one by one, and
 // 128 registers: q|k|v of 1234 tokens at K = 2048 15.4 -> 14.9, but gate_up of 600 at K = 1024 12.5 -> 13.4, o of 2000 8.2 -> 8.7.)
-constexpr int decode_waves(int r, int kspw, int sa, bool texts) { return texts && ((r <= 16 && kspw <= 8) || (r <= 8 && kspw <= 12 && sa == 1)) ? 4 : 2; }
+constexpr int decode_waves(int r, int kspw, bool texts) { return texts && r <= 16 && kspw <= 8 ? 4 : 2; }
 
 // SHORT (staged form): with a text each for tiles of up to four, up to eight and more tokens (below); without, the last one alone.
 template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR, bool SHORT>
-__global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SA, SHORT)) void decode_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv,
+__global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT)) void decode_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv,
                                                             void* __restrict__ yv_, int64_t xs, int64_t ys, int small_off,
                                                             int include_long, int T_, int K, int num_slots, float scaling,
                                                             const int32_t* __restrict__ eff_rank, int rbuf_arg, DecodeSplits splits) {
