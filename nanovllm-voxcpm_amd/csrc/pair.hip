@@ -40,7 +40,9 @@ constexpr int kMaxParts = 8;    // most K parts of a launch
 constexpr int kPartsAhead = 4;  // of which the expand requests this many together
 // Below, a step's weights (about a hundred such calls) may still lie in the 256 MB of the memory-side cache when the next step comes, and
 // the hint gives that up: 5 tokens of 5 slots, rank 64, K = 1024, weights at hand, q|k|v 7.2 us per call without, 7.7 with, o 6.5 / 7.6; one token, K =
-// 2048, gate_up 8.6 / 9.1.
+// 2048, gate_up 8.6 / 9.1.  The kernels count the weights by the plan's header: a graph over 48 slot ids serves batches of few adapters too (us per
+// call, counted by the ids / by the header: 64 tokens of 8 slots, rank 48, K = 2048, q|k|v 9.3 / 8.5, down 11.3 / 9.8; 32 of 3, rank 64, 9.8 / 8.8 and
+// 10.3 / 9.2; 201 of 48, rank 64, 19.7 / 19.8, gate_up 28.5 / 28.5).
 constexpr long long kOnceBytes = 8ll << 20;
 
 // ---- shrink -------------------------------------------------------------------------------------
@@ -225,14 +227,14 @@ __device__ __forceinline__ void shrink_tile(char* lds, const char* abase, uint32
 // A tile's record, with the plan header's verdict on it.
 struct PairTile {
   int slot, m, ok, plan_ok;
-  int alone;  // the slot has no other tile (short segments come first in the list)
+  int once;  // its A and B lines with the hint: the slot has no other tile (short segments come first in the list), and the batch uses `once_from` slots
 };
-__device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __restrict__ plan, int tile, int T_, int num_slots) {
+__device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __restrict__ plan, int tile, int T_, int num_slots, int once_from) {
   const i32x4 h0 = *reinterpret_cast<const i32x4*>(plan), h1 = *reinterpret_cast<const i32x4*>(plan + 4), h2 = *reinterpret_cast<const i32x4*>(plan + 8);
   PairTile t;
   t.slot = r0[0];
   t.m = r0[1];
-  t.alone = int(tile < h1[MLORA_PLAN_TILES_SHORT - 4]);
+  t.once = int(tile < h1[MLORA_PLAN_TILES_SHORT - 4]) & int(h1[MLORA_PLAN_NUM_ACTIVE - 4] >= once_from);
   t.plan_ok = int(h0[MLORA_PLAN_MAGIC] == MLORA_PLAN_MAGIC_VALUE) & int(h0[MLORA_PLAN_NUM_TOKENS] == T_) & int(h0[MLORA_PLAN_MAX_SLOTS] == num_slots);
   t.ok = t.plan_ok & int(tile < h1[MLORA_PLAN_TILES_SHORT - 4] + h2[MLORA_PLAN_TILES_LONG_SMALL - 8]) & int(t.m > 0) & int(t.slot >= 0) &
          int(t.slot < num_slots);
@@ -243,7 +245,8 @@ __device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __r
 template <typename T, bool CHAINS, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
                                                                    int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, int rbuf,
-                                                                   int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
+                                                                   int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, int once_from,
+                                                                   ShrinkSlices sl) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   // ---- one trip: tile record, plan header, the tile's token rows, the slots' ranks ------------------
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t
   int row[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) row[i] = rec[MLORA_SMALL_TILE_ROWS + i * 8 + (lane >> 3)];
-  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots, once_from);
   const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
   __builtin_amdgcn_sched_barrier(0);
   if (!t.ok) {
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t
     else if (groups <= 6) shrink_tile<T, 6, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
     else shrink_tile<T, 8, CHAINS, O>(lds, abase, arow, rbuf, xbase, xoff, c0, cm, c1, dst, rp, m);
   };
-  if (ONCE && __builtin_amdgcn_readfirstlane(t.alone)) tile_of(std::true_type{});
+  if (ONCE && __builtin_amdgcn_readfirstlane(t.once)) tile_of(std::true_type{});
   else tile_of(std::false_type{});
 #ifdef MLORA_TRACE
   MLORA_STAMP(5);
@@ -331,7 +334,7 @@ template <int C> struct ExpandShape {
 
 // A wavefront's B rows [c0, c0 + 64 SP), up to column n1, to its LDS.
 template <typename T, int C, int SP>
-__device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, int n1, int eff, bool alone) {
+__device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, int n1, int eff, bool once) {
   constexpr int E = PieceOf<T>::E, SH = ExpandShape<C>::SH;
   constexpr int NB = SP * C;  // direct loads of a wavefront's B rows
   const int lane = threadIdx.x & (kWave - 1);
@@ -351,7 +354,7 @@ __device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, 
       }
     }
   };
-  if (alone) request(std::true_type{});
+  if (once) request(std::true_type{});
   else request(std::false_type{});
 }
 
@@ -436,7 +439,7 @@ __device__ __forceinline__ void finish_spans(const char* s_h, const char* s_b, c
 template <typename T, int C, int SP>
 __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__ hsrc, int64_t part_stride, int kparts, const f32x4 (&hv)[kPartsAhead], const char* bbase,
                                             T* __restrict__ ybase, const int64_t ys, const i32x4 rows, int n0, int n1, int m, int eff,
-                                            bool alone, float scaling) {
+                                            bool once, float scaling) {
   constexpr int E = PieceOf<T>::E;          // elements per piece
   constexpr int R = C * E;                  // rank of the buffers
   constexpr int KSTEPS = ExpandShape<C>::KSTEPS, HROW = ExpandShape<C>::HROW;
@@ -451,7 +454,7 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
   const int c0 = n0 + wave * (SP * 64);
   const bool mine = c0 < n1;
   YSpan<T> yq[SP][4];
-  if (mine) request_b<T, C, SP>(s_b, bbase, c0, n1, eff, alone);
+  if (mine) request_b<T, C, SP>(s_b, bbase, c0, n1, eff, once);
   request_y<T, SP, 4>(yq, ybase, ys, rows, c0, n1);
   MLORA_STAMP(10);  // expand: B rows and y requested
   // the intermediate: parts summed in order, scaled, split, to LDS in operand rows (its first
@@ -503,7 +506,7 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
 template <typename T, int C, int SP, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws, void* __restrict__ yv_,
                                                                    int64_t ys, int small_off, int T_, int num_slots, int kparts, int num_slices,
-                                                                   float scaling, const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
+                                                                   float scaling, const int32_t* __restrict__ eff_rank, int once_from, ExpandSplits splits) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int R = C * PieceOf<T>::E, RP = (R + 15) & ~15;
   const int lane = threadIdx.x & (kWave - 1), lg = lane >> 4;
@@ -513,7 +516,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   const int32_t* rec = plan + small_off + tile * MLORA_SMALL_TILE_WORDS;
   const i32x4 r0 = *reinterpret_cast<const i32x4*>(rec);
   const i32x4 rows = spread_rows(rec, lg);
-  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots, once_from);
   const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
   // the intermediate's partial sums lie where the tile's place says: requested with the record
   const int64_t stride = static_cast<int64_t>(num_slices) * (gridDim.z * 8) * (MLORA_TILE_SMALL * RP);  // from K part to K part
@@ -533,7 +536,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t
   if (eff == 0) return;
   const char* bbase = uniform(static_cast<const char*>(sp.b) + static_cast<int64_t>(slot) * sp.n * (C * 16));
   expand_tile<T, C, SP>(lds, hsrc, stride, kparts, hv, bbase, static_cast<T*>(yv_) + sp.y_col, ys, rows, sp.n0, sp.n1, m, eff,
-                        ONCE && __builtin_amdgcn_readfirstlane(t.alone) != 0, scaling);
+                        ONCE && __builtin_amdgcn_readfirstlane(t.once) != 0, scaling);
   MLORA_STAMP_END(13);  // expand: stores issued, acknowledged
 }
 
@@ -606,7 +609,7 @@ __global__ __launch_bounds__(kSoloThreads) void solo_kernel(const int32_t* __res
   int row[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) row[i] = rec[MLORA_SMALL_TILE_ROWS + i * 8 + (lane >> 3)];
-  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots);
+  const PairTile t = pair_tile(r0, plan, tile, T_, num_slots, 0);
   const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
   __builtin_amdgcn_sched_barrier(0);
   if (!t.ok) {
@@ -688,7 +691,8 @@ struct PairLaunch {
   const MloraAddArgs* a;
   PlanLayout lay;
   int parts_log2, sp;
-  bool once;  // A and B of a slot's only tile with the non-temporal hint
+  bool once;      // instances that can request A and B of a slot's only tile with the non-temporal hint
+  int once_from;  // and do so from this many slots with tokens on
 };
 
 template <typename T, bool CHAINS, bool ONCE> void launch_pair_shrink_one(const PairLaunch& l) {
@@ -699,7 +703,7 @@ template <typename T, bool CHAINS, bool ONCE> void launch_pair_shrink_one(const 
   hipLaunchKernelGGL((pair_shrink_kernel<T, CHAINS, ONCE>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
                      dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
                      a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
-                     l.parts_log2, a->num_slices, a->effective_rank, sl);
+                     l.parts_log2, a->num_slices, a->effective_rank, l.once_from, sl);
 }
 
 template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) {
@@ -712,7 +716,7 @@ template <typename T, int C, int SP, bool ONCE> void launch_pair_expand_one(cons
   allow_lds<pair_expand_kernel<T, C, SP, ONCE>>(expand_lds(C, SP));
   hipLaunchKernelGGL((pair_expand_kernel<T, C, SP, ONCE>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
                      expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
-                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, splits);
+                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, l.once_from, splits);
 }
 
 template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const ExpandSplits& splits, int total) {
@@ -856,8 +860,10 @@ int launch_pair(const MloraAddArgs* a, int active) {
   const size_t room = partials_room(a) / part_bytes(a, l.lay);
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  const long long weights = static_cast<long long>(active > 0 ? active : segs) * a->r * (static_cast<long long>(a->num_slices) * a->k + cols) * element_bytes(a->dtype);
-  l.once = pair_knobs().once < 0 ? weights >= kOnceBytes : pair_knobs().once != 0;
+  // (how many slots have tokens is in the plan's header, which the kernels read: behind a capture the host knows only how many may)
+  const long long per_slot = static_cast<long long>(a->r) * (static_cast<long long>(a->num_slices) * a->k + cols) * element_bytes(a->dtype);
+  l.once_from = pair_knobs().once > 0 ? 0 : static_cast<int>((kOnceBytes + per_slot - 1) / per_slot);
+  l.once = pair_knobs().once < 0 ? (active > 0 ? active : segs) >= l.once_from : pair_knobs().once != 0;
   // K parts: workgroups for most compute units, no more (every column range of the second launch
   // takes in every part's sums), and a chunk per wavefront at least
   int want = pair_knobs().kparts;
