@@ -285,11 +285,12 @@ void launch_rank(const Launch& l, int r, int kspw) {
 
 // Diagnostic knobs, read from the environment once per process.
 struct DecodeKnobs {
-  int generation = -1, staged, nt;
+  int generation = -1, staged, nt, short_tiles;
   void read() {
     generation = knob_generation();
     staged = env_int("MLORA_DECODE_STAGED", 1);
     nt = env_int("MLORA_DECODE_NT", 0);
+    short_tiles = env_int("MLORA_DECODE_SHORT", -1);
   }
 };
 const DecodeKnobs& decode_knobs() {
@@ -376,7 +377,7 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
       if (d.n1 - d.n0 > l.widest) l.widest = d.n1 - d.n0;
     }
   }
-  l.short_tiles = a->num_tokens <= (l.widest <= kNW * 64 ? 12 : 4) * with_tokens;
+  l.short_tiles = decode_knobs().short_tiles < 0 ? a->num_tokens <= (l.widest <= kNW * 64 ? 12 : 4) * with_tokens : decode_knobs().short_tiles != 0;
   for (; s < kMaxSplits; ++s) splits.split[s] = DecodeSplit{nullptr, nullptr, 0, 0, 0, 0};
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(cap / 8));
   const int nks = a->k / 32;
