@@ -116,7 +116,7 @@ def test_auto_takes_one_launch_where_it_pays(tokens, slots, rank, k, widths, one
 @pytest.mark.gpu
 @pytest.mark.parametrize("rank", [24, 40, 48, 56])
 @pytest.mark.parametrize("tokens, slots, k, widths", [(1, 3, 32, [4]), (17, 2, 1024, [520, 64]), (150, 40, 2080, [256])])
-def test_ranks_between_the_instances_are_two_launches_under_auto(rank, tokens, slots, k, widths):
+def test_ranks_between_the_instances_are_two_launches_under_auto(rank, tokens, slots, k, widths, monkeypatch):
     from nanovllm_voxcpm_amd import _hip
 
     case = (tokens, slots, rank, k, widths, 0, tokens > 1, True)
@@ -124,3 +124,13 @@ def test_ranks_between_the_instances_are_two_launches_under_auto(rank, tokens, s
     out = _apply(case, batch, _hip.FORM_AUTO)
     assert torch.equal(out[batch[0] < 0], batch[4][batch[0] < 0])
     assert torch.allclose(out, batch[6], rtol=1e-5, atol=2e-5)
+    try:
+        monkeypatch.setenv("MLORA_NO_PAIR", "1")
+        _hip.reload_knobs()
+        one_per_token = _apply(case, batch, _hip.FORM_AUTO)
+    finally:
+        monkeypatch.undo()
+        _hip.reload_knobs()
+    assert torch.allclose(one_per_token, batch[6], rtol=1e-5, atol=2e-5)
+    # (the forms add K up in different orders, which one token of 32 columns need not show)
+    assert tokens == 1 or not torch.equal(out, one_per_token)
