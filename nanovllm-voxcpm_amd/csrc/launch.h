@@ -57,7 +57,7 @@ int launch_sgmv(const MloraAddArgs* a, int active);  // active: slots with token
 // slab.hip: the shrink launch of that form, operands through LDS by direct loads.
 struct PlanLayout;
 bool slab_supported(const MloraAddArgs* a);
-void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, bool deep, const void* const* slices);
+void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const void* const* slices);
 
 // fused.hip: the same tiles, shrink and expand in one launch (workgroups of a unit exchange the
 // intermediate through the workspace under seals kept in its head).

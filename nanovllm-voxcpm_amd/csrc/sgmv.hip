@@ -261,7 +261,7 @@ int launch_sgmv(const MloraAddArgs* a, int active) {
   ShrinkLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.tiles8 = sh.tiles8; l.big_cap = sh.big_cap;
   l.ksplit = sh.ksplit; l.krange = sh.krange; l.all_slices = sh.all_slices;
-  if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.slab_deep, sh.sl.a);
+  if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.sl.a);
   else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink_rank<__bf16>(l, sh.kr, sh.xw);
   else launch_shrink_rank<_Float16>(l, sh.kr, sh.xw);
   int rc = check_launch("mlora_add_lora(sgmv shrink)");

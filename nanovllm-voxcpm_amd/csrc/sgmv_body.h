@@ -819,7 +819,7 @@ struct SgmvKnobs {
     nt = env_int("MLORA_SGMV_NT", 0);
     cpl = env_int("MLORA_SGMV_CPL", 8);
     stream = env_int("MLORA_SGMV_STREAM", -1);
-    slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay, 3: rank 64 so with deep rings
+    slab = env_int("MLORA_SLAB", 1);  // 0: never, 2: also by name and where it does not pay
   }
 };
 const SgmvKnobs& sgmv_knobs() {
@@ -865,7 +865,6 @@ struct SgmvShape {
   int kr, xw;     // shrink: A slab width, x batch width
   int ksplit, krange, all_slices;
   bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
-  bool slab_deep; // ... with its deep rings
   int group;      // expand: consecutive 64-token tiles per workgroup
   int cpl;        // expand: columns per lane
   bool stream;    // expand: y with the non-temporal hint
@@ -949,11 +948,11 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   s.slab = !one_launch && slab_supported(a) &&
            (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
   // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
-  // those, per slot): slab.hip with deep rings, while an XCD's workgroups number no more than its 32 compute units (a second
-  // round loses: 5000 tokens of 6 slots in three parts, 33 workgroups on some XCDs, K = 3072 36.1 / 41.5) and it cuts K into more parts
+  // those, per slot): while an XCD's workgroups number no more than its 32 compute units (a second
+  // round loses: 5200 tokens of 2 slots, K = 2560, two parts 29.8 us, three, 33 workgroups on some XCDs, 33.2) and it cuts K into more parts
   // than the other shrink, whose parts have to divide K (with two slices into as many).  us per call, the other shrink / this, 2 slots: K = 2560,
-  // 4096 tokens 32.4 / 25.8; K = 3072, 3600 27.8 / 25.4; two slices, K = 2560, 6400 52.6 / 52.0; 423 such calls of 2 to 16 slots, K 1536 to 5120, take
-  // 0.67 to 1.00 of the other's time.  With fewer parts it can win too (K = 4096, 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192,
+  // 4096 tokens 32.9 / 25.6; K = 3072, 3600 27.9 / 25.9; K = 5120, 4096 28.1 / 23.2; two slices, K = 2560, 6400 52.7 / 51.9; 498 such
+  // calls of 2 to 16 slots, K 1536 to 5120, take 0.65 to 0.99 of the other's time.  With fewer parts it can win too (rings of 48 KB: K = 4096, 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192,
   // 4500 47.5 / 39.1), but only on as many tiles as the tokens could make: tokens without an adapter make none, how many those are
   // the host does not say, and with a quarter to three quarters of them two or three parts leave compute units idle
   // that four would fill (K = 4096, 5200 tokens of 2 slots, half of them adapted, 18.2 / 21.2; K = 2048, 8000 of 12, 19.6 / 23.6; 124 of 171 such
@@ -961,27 +960,22 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   // parts that would be longer than 2800 columns nor below half a
   // round, and not for short segments: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens 23.2 / 25.7.
   // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7).
-  s.slab_deep = false;
+  int round_parts = 0;
   const int slots = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  const bool deep_knob = sgmv_knobs().slab == 3;
-  if (!one_launch && slab_supported(a) && a->r == 64 && a->num_slices <= 2 && slots > 0 && max_parts > 0 &&
-      (deep_knob || (sgmv_knobs().slab == 1 && a->form == MLORA_FORM_AUTO && a->num_tokens / slots >= 4 * MLORA_TILE_BIG))) {
+  if (!one_launch && !s.slab && sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 && slots > 0 &&
+      a->num_tokens / slots >= 4 * MLORA_TILE_BIG) {
     const int tiles = static_cast<int>((a->num_tokens + 63ll * slots) / MLORA_TILE_BIG);  // at most: every slot's last tile has one token
-    const int per_xcd = (tiles + 7) / 8 * a->num_slices;
-    int parts = 32 / per_xcd;
-    if (parts > (a->num_slices == 1 ? kMaxKSplit : 2)) parts = a->num_slices == 1 ? kMaxKSplit : 2;
+    const int most = a->num_slices == 1 ? kMaxKSplit : 2;
+    int parts = 32 / ((tiles + 7) / 8 * a->num_slices);
+    if (parts > most) parts = most;
     if (parts > a->k / 1024) parts = a->k / 1024;
-    if (deep_knob && sgmv_knobs().ksplit > 0) parts = sgmv_knobs().ksplit < kMaxKSplit ? sgmv_knobs().ksplit : kMaxKSplit;
     if (parts > max_parts) parts = max_parts;
-    if (parts < 1 && deep_knob) parts = 1;
-    s.slab_deep = deep_knob || (parts >= ksplit + (a->num_slices == 1) && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128);
-    if (s.slab_deep) ksplit = parts;
-    s.slab |= s.slab_deep;
+    if (parts >= ksplit + (a->num_slices == 1) && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128) {
+      round_parts = parts;
+      s.slab = true;
+    }
   }
-  if (s.slab_deep) {
-    s.all_slices = 0;
-    s.ksplit = ksplit;
-  } else if (s.slab) {
+  if (s.slab) {
     // About 205 workgroups (parts need not be a power of two), a stage of K per wavefront at least.  Measured, us
     // per call with one / two / three / four parts, rank 32: down (K = 4096) of 2000 tokens 20.8 / 15.7 / 14.0 / 13.4,
     // of 4000 22.3 / 17.5 / 16.6 / 18.1, of 5000 23.4 / 18.5 / 20.8 / 19.2, of 6500 29.6 / 22.4 / 25.0 / 23.1; K = 8192,
@@ -994,7 +988,9 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
     // taken from K = 4096 on, and from K = 8192 on throughout.
     s.all_slices = 0;
     ksplit = sgmv_knobs().ksplit;
-    if (ksplit <= 0) {
+    if (ksplit <= 0 && round_parts > 0) {
+      ksplit = round_parts;
+    } else if (ksplit <= 0) {
       const int units = est_tiles * a->num_slices;
       ksplit = (205 + 2 * units / 5) / units;
       if (a->k >= 8192 || (a->k >= 4096 && ksplit <= 1)) ksplit = kMaxKSplit;

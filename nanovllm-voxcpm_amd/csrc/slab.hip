@@ -12,7 +12,8 @@
 // the sums at the end passes between them and no barrier stands between request and product.
 // Two wavefronts, not four: their rings (64 KB at rank 64) keep a compute unit's 64 KB of requests on their way, and two
 // workgroups fit a compute unit, so that one starts while the other sums up (rank 64, 9392 tokens, a quarter without
-// adapter, with the expand: qkv 28.3 -> 26.4 us per call, 8192 mixed tokens: gate_up 99.3 -> 98.3).
+// adapter, with the expand: qkv 28.3 -> 26.4 us per call, 8192 mixed tokens: gate_up 99.3 -> 98.3).  Rings of 48 KB, three
+// stages at rank 64 with one workgroup per compute unit, are 1 % slower (494 calls of one or two slices, in the same K parts).
 // Shrink and expand at rank 32, 5000 tokens, K = 4096: 21.0 -> 18.5 us per call, 3.1 -> 3.5 TB/s.
 #include "common.h"
 #include "dma.h"
@@ -29,27 +30,18 @@ constexpr int kSlabThreads = kSlabWaves * kWave;
 constexpr int kPiece = 128;  // bytes of a row per stage
 
 // NA8: groups of eight ranks, TB: blocks of sixteen tokens; both operands in groups of eight rows, 1 KB each.
-// DEEP: rings of 48 KB, one workgroup per compute unit (rank 64: three stages instead of two; sgmv_shape() says when).
-template <int NA8, int TB, bool DEEP> struct SlabShape {
+template <int NA8, int TB> struct SlabShape {
   static constexpr int RB = (NA8 + 1) / 2;
   static constexpr int ND = NA8 + 2 * TB;                          // direct loads per stage
-  static constexpr int NST = DEEP ? 48 / ND : ND > 6 ? 2 : ND > 4 ? 3 : 4;  // stages of a wavefront's ring
+  static constexpr int NST = ND > 6 ? 2 : ND > 4 ? 3 : 4;  // stages of a wavefront's ring
   static constexpr int BYTES = NST * ND * 1024;
   static_assert(RB * TB <= NST * ND, "the ring holds the wavefront's sums");
-  static_assert((NST - 1) * ND <= 63, "a wait counts 63 loads at most");
 };
 
-// Waits until only the stages requested behind the current one, `younger` of them and N at most, are on their way.
-template <int ND, int N> __device__ __forceinline__ void wait_younger(int younger) {
-  if constexpr (N == 0) wait_loads<0>();
-  else if (younger >= N) wait_loads<N * ND>();
-  else wait_younger<ND, N - 1>(younger);
-}
-
-template <typename T, int NA8, int TB, bool DEEP>
+template <typename T, int NA8, int TB>
 __device__ __forceinline__ void slab_tile(char* lds, const char* abase, uint32_t arow, int rbuf, const char* xbase, const uint32_t (&xoff)[2 * TB], int c0,
                                           int c1, float* __restrict__ dst, int64_t hrow, int m) {
-  typedef SlabShape<NA8, TB, DEEP> S;
+  typedef SlabShape<NA8, TB> S;
   constexpr int RB = S::RB, ND = S::ND, NST = S::NST;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;
@@ -88,7 +80,10 @@ __device__ __forceinline__ void slab_tile(char* lds, const char* abase, uint32_t
       issue(c0 + c + NST - 1, into);
     }
     const int younger = n - 1 - c < NST - 1 ? n - 1 - c : NST - 1;  // stages requested behind this one
-    wait_younger<ND, NST - 1>(younger);
+    if (NST >= 4 && younger == 3) wait_loads<(NST >= 4 ? 3 : 0) * ND>();
+    else if (NST >= 3 && younger == 2) wait_loads<(NST >= 3 ? 2 : 0) * ND>();
+    else if (younger == 1) wait_loads<ND>();
+    else wait_loads<0>();
     const char* st = ring + stage * (ND * 1024) + lr * 128 + ((lg ^ (lr & 7)) * 16);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -132,20 +127,20 @@ __device__ __forceinline__ void slab_tile(char* lds, const char* abase, uint32_t
   }
 }
 
-template <typename T, int TB, bool DEEP>
+template <typename T, int TB>
 __device__ __forceinline__ void slab_ranks(int groups, char* lds, const char* abase, uint32_t arow, int rbuf, const char* xbase,
                                            const uint32_t (&xrows)[8], int c0, int c1, float* __restrict__ dst, int64_t hrow, int m) {
   uint32_t xoff[2 * TB];
 #pragma unroll
   for (int g = 0; g < 2 * TB; ++g) xoff[g] = xrows[g];
-  if (groups <= 1) slab_tile<T, 1, TB, DEEP>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
-  else if (groups == 2) slab_tile<T, 2, TB, DEEP>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
-  else if (groups <= 4) slab_tile<T, 4, TB, DEEP>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
-  else slab_tile<T, 8, TB, DEEP>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  if (groups <= 1) slab_tile<T, 1, TB>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  else if (groups == 2) slab_tile<T, 2, TB>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  else if (groups <= 4) slab_tile<T, 4, TB>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  else slab_tile<T, 8, TB>(lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
 }
 
 // grid (8, slices * K parts, tiles / 8): blockIdx.x is the XCD
-template <typename T, bool DEEP>
+template <typename T>
 __global__ __launch_bounds__(kSlabThreads) void slab_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
                                                                    int big_off, int small_off, int big_cap, int bigrows_off, int T_, int num_slots,
                                                                    int kchunks, uint32_t xrow, int rbuf, int parts, int num_slices,
@@ -178,30 +173,30 @@ __global__ __launch_bounds__(kSlabThreads) void slab_shrink_kernel(const int32_t
   const int64_t hrow = static_cast<int64_t>(num_slices) * rbuf;
   float* dst = hws + static_cast<int64_t>(part) * T_ * hrow + static_cast<int64_t>(start) * hrow + slice * rbuf;
   const int groups = (eff + 7) >> 3;
-  if (m <= 16) slab_ranks<T, 1, DEEP>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
-  else if (m <= 32) slab_ranks<T, 2, DEEP>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
-  else slab_ranks<T, 4, DEEP>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  if (m <= 16) slab_ranks<T, 1>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  else if (m <= 32) slab_ranks<T, 2>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
+  else slab_ranks<T, 4>(groups, lds, abase, arow, rbuf, xbase, xoff, c0, c1, dst, hrow, m);
 }
 
 // The most LDS any adapter and tile of buffers of this rank may need.
-template <int NA8, bool DEEP> int slab_bytes_of() {
-  int most = SlabShape<NA8, 1, DEEP>::BYTES;
-  most = SlabShape<NA8, 2, DEEP>::BYTES > most ? SlabShape<NA8, 2, DEEP>::BYTES : most;
-  return SlabShape<NA8, 4, DEEP>::BYTES > most ? SlabShape<NA8, 4, DEEP>::BYTES : most;
+template <int NA8> int slab_bytes_of() {
+  int most = SlabShape<NA8, 1>::BYTES;
+  most = SlabShape<NA8, 2>::BYTES > most ? SlabShape<NA8, 2>::BYTES : most;
+  return SlabShape<NA8, 4>::BYTES > most ? SlabShape<NA8, 4>::BYTES : most;
 }
-template <bool DEEP> int slab_lds(int r) {
-  int most = slab_bytes_of<1, DEEP>();
+int slab_lds(int r) {
+  int most = slab_bytes_of<1>();
   auto with = [&](int b) { most = b > most ? b : most; };
-  if (r > 8) with(slab_bytes_of<2, DEEP>());
-  if (r > 16) with(slab_bytes_of<4, DEEP>());
-  if (r > 32) with(slab_bytes_of<8, DEEP>());
+  if (r > 8) with(slab_bytes_of<2>());
+  if (r > 16) with(slab_bytes_of<4>());
+  if (r > 32) with(slab_bytes_of<8>());
   return most * kSlabWaves;
 }
 
-template <typename T, bool DEEP> void launch_slab_type(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const ShrinkSlices& sl) {
-  allow_lds<slab_shrink_kernel<T, DEEP>>(slab_lds<DEEP>(a->r));
-  hipLaunchKernelGGL((slab_shrink_kernel<T, DEEP>), dim3(8, static_cast<unsigned>(a->num_slices * parts), static_cast<unsigned>(tiles8)), dim3(kSlabThreads),
-                     slab_lds<DEEP>(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), lay.big_off, lay.small_off, big_cap,
+template <typename T> void launch_slab_type(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const ShrinkSlices& sl) {
+  allow_lds<slab_shrink_kernel<T>>(slab_lds(a->r));
+  hipLaunchKernelGGL((slab_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices * parts), static_cast<unsigned>(tiles8)), dim3(kSlabThreads),
+                     slab_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), lay.big_off, lay.small_off, big_cap,
                      lay.bigrows_off, a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kPiece),
                      static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r, parts, a->num_slices, a->effective_rank, sl);
 }
@@ -213,11 +208,11 @@ bool slab_supported(const MloraAddArgs* a) {
   return a->k % 64 == 0 && a->num_tokens * (a->x_stride * 2) < (1ll << 32) && static_cast<int64_t>(a->r) * a->k * 2 < (1ll << 32);
 }
 
-void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, bool deep, const void* const* slices) {
+void launch_slab_shrink(const MloraAddArgs* a, const PlanLayout& lay, int big_cap, int tiles8, int parts, const void* const* slices) {
   ShrinkSlices sl;
   for (int i = 0; i < MLORA_MAX_SLICES; ++i) sl.a[i] = slices[i];
-  if (a->dtype == MLORA_DTYPE_BF16) deep ? launch_slab_type<__bf16, true>(a, lay, big_cap, tiles8, parts, sl) : launch_slab_type<__bf16, false>(a, lay, big_cap, tiles8, parts, sl);
-  else deep ? launch_slab_type<_Float16, true>(a, lay, big_cap, tiles8, parts, sl) : launch_slab_type<_Float16, false>(a, lay, big_cap, tiles8, parts, sl);
+  if (a->dtype == MLORA_DTYPE_BF16) launch_slab_type<__bf16>(a, lay, big_cap, tiles8, parts, sl);
+  else launch_slab_type<_Float16>(a, lay, big_cap, tiles8, parts, sl);
 }
 
 }  // namespace mlora

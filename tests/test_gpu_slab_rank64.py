@@ -1,4 +1,4 @@
-"""The shrink through LDS with deep rings (csrc/slab.hip, rank 64, one or two slices) at the sizes where it can go wrong: K of
+"""The shrink through LDS (csrc/slab.hip) at rank 64, one or two slices, at the sizes where it can go wrong: K of
 fewer 128-byte pieces per wavefront than the ring has stages, tiles of every number of 16-token blocks, uneven K
 parts, adapters below the buffers' rank with NaN beyond it; and which shrink, in how many K parts, the automatic choice takes on both
 sides of its lines."""
@@ -13,7 +13,7 @@ from test_gpu_parity import _check, _exact
 
 B16, F16 = torch.bfloat16, torch.float16
 
-# segment lengths, K, widths, element type, adapters of lower rank, every fourth segment without adapter, K parts of the deep rings (None: forced, 0: the
+# segment lengths, K, widths, element type, adapters of lower rank, every fourth segment without adapter, K parts of this shrink (None: forced, 0: the
 # automatic choice is the other shrink)
 CASES = [
     ([64], 128, [8], B16, False, False, None),
@@ -36,12 +36,12 @@ CASES = [
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", range(len(CASES)))
-def test_deep_rings_against_fp64(case, monkeypatch):
+def test_rank_64_through_lds_against_fp64(case, monkeypatch):
     from nanovllm_voxcpm_amd import _hip
     from nanovllm_voxcpm_amd.lora_ops.segment_meta import build_segment_plan
 
     lengths, k, widths, dtype, mixed, holes, parts = CASES[case]
-    print(f"deep rings {case} {k} {widths}", flush=True)
+    print(f"slab, rank 64 {case} {k} {widths}", flush=True)
     pick, g = random.Random(case), torch.Generator().manual_seed(case)
     slots, rank = len(lengths), 64
     ids = [-1 if holes and i % 4 == 3 else i for i, n in enumerate(lengths) for _ in range(n)]
@@ -76,15 +76,15 @@ def test_deep_rings_against_fp64(case, monkeypatch):
 
     try:
         if parts is None:
-            runs = [run(_hip.FORM_SGMV, 3) for _ in range(2)]
+            runs = [run(_hip.FORM_SGMV, 2) for _ in range(2)]
         else:
             runs = [run(_hip.FORM_AUTO) for _ in range(2)]
             # which shrink that was, by the order in which it adds K up
-            others = {n: run(_hip.FORM_AUTO, 3, n) for n in (2, 3, 4)} | {0: run(_hip.FORM_AUTO, 0)}  # (one part may be two of the other's)
+            others = {n: run(_hip.FORM_AUTO, 2, n) for n in (2, 3, 4)} | {0: run(_hip.FORM_AUTO, 0)}  # (one part may be two of the other's)
             assert [n for n in sorted(others) if torch.equal(runs[0], others[n])] == [parts]
     finally:
         monkeypatch.undo()
         _hip.reload_knobs()
     assert torch.equal(runs[0], runs[1])
     exact, mag = _exact(types.SimpleNamespace(a=shown_a, b=shown_b, widths=widths), x, y, indices, 0.75)
-    _check(runs[0], y, exact, mag, indices, f"deep rings {case}")
+    _check(runs[0], y, exact, mag, indices, f"slab, rank 64 {case}")
