@@ -361,6 +361,9 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
   // for the price of the others (155 tokens of 3 slots, us per call without / with them: rank 48 q|k|v 8.4 / 8.6, gate_up 9.7 / 10.0, rank 32 5.5 / 5.6;
   // 64 tokens of 32 slots, rank 32, 4.8 / 4.5 and 7.5 / 7.1): up to twelve tokens per slot with tokens.  With two spans per wavefront, whose texts
   // are longer, up to four (128 tokens of 16 slots, K = 2048, rank 16, gate_up 7.4 / 7.9; 200 of 30, rank 24, 8.2 / 8.2; 100 of 60, rank 32, 12.1 / 11.3).
+  // Behind a capture the slots of the buffers count for those with tokens: a graph is captured for batches of about one token per slot, and one that
+  // then brings full tiles loses up to 3 % of a call (64 tokens of 3 of 48 slots, without / with the texts: rank 16, K = 2048, q|k|v 5.1 / 5.2, o 4.9 / 4.8; rank 32, K =
+  // 1024, 4.4 / 4.5 and 4.2 / 4.3; rank 48 6.9 / 6.9, gate_up 9.3 / 9.5), less than short tiles would lose without.
   const int with_tokens = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
 
   int nt;

@@ -360,8 +360,10 @@ __device__ __forceinline__ void request_b(char* s_b, const char* bbase, int c0, 
 
 // A tile's tokens spread over the lane groups: row 4 * lg + i of the products is token lg + 4 * i, so that those of a tile of up to four or
 // eight are the rows i = 0 or i < 2 (XI rows).  The one launch has a text per XI and leaves out what the others would request (64 tokens
-// of 32 slots, rank 16, K = 1024, o 6.1 -> 5.8 us; of 4, q|k|v 6.0 -> 5.8); in the pair that gains no more than it loses (two texts of the shrink, three
-// of the expand: -2 to +2 % over 54 shapes).
+// of 32 slots, rank 16, K = 1024, o 6.1 -> 5.8 us; of 4, q|k|v 6.0 -> 5.8); in the pair those texts gain no more than they lose (two of the shrink, three
+// of the expand: -2 to +2 % over 54 shapes), but the order by itself stays: a tile of up to four tokens stores one row per lane group
+// instead of four of one group (row 4 * lg + i for token 4 * lg + i / this order, us per call: 16 tokens of 4 slots, rank 64, K = 2048, q|k|v 8.17 / 7.85, o
+// 7.85 / 7.51; 201 of 48 gate_up 30.2 / 28.5, rank 48 26.2 / 24.2; full tiles alike: 591 of 12, rank 24, 13.2 / 13.2 and 10.6 / 10.6).
 __device__ __forceinline__ int row_of_token(int t) { return 4 * (t & 3) + (t >> 2); }
 __device__ __forceinline__ i32x4 spread_rows(const int32_t* __restrict__ rec, int lg) {
   i32x4 rows;
