@@ -41,8 +41,8 @@ constexpr int kPartsAhead = 4;  // of which the expand requests this many togeth
 // Below, a step's weights (about a hundred such calls) may still lie in the 256 MB of the memory-side cache when the next step comes, and
 // the hint gives that up: 5 tokens of 5 slots, rank 64, K = 1024, weights at hand, q|k|v 7.2 us per call without, 7.7 with, o 6.5 / 7.6; one token, K =
 // 2048, gate_up 8.6 / 9.1.  The kernels count the weights by the plan's header: a graph over 48 slot ids serves batches of few adapters too (us per
-// call, counted by the ids / by the header: 64 tokens of 8 slots, rank 48, K = 2048, q|k|v 9.3 / 8.5, down 11.3 / 9.8; 32 of 3, rank 64, 9.8 / 8.8 and
-// 10.3 / 9.2; 201 of 48, rank 64, 19.7 / 19.8, gate_up 28.5 / 28.5).
+// call, counted by the ids / by the header: 64 tokens of 8 slots, rank 48, K = 2048, q|k|v 9.3 / 8.5, down 11.4 / 9.6; 32 of 3, rank 64, 9.8 / 8.8 and
+// 10.2 / 9.1; 201 of 48, rank 64, 19.6 / 19.7, gate_up 28.5 / 28.6).
 constexpr long long kOnceBytes = 8ll << 20;
 
 // ---- shrink -------------------------------------------------------------------------------------
@@ -245,10 +245,10 @@ __device__ __forceinline__ PairTile pair_tile(const i32x4 r0, const int32_t* __r
 template <typename T, bool CHAINS, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
                                                                    int small_off, int T_, int num_slots, int kchunks, uint32_t xrow, int rbuf,
-                                                                   int parts_log2, int num_slices, const int32_t* __restrict__ eff_rank, int once_from,
-                                                                   ShrinkSlices sl) {
+                                                                   int parts_log2, int slices_once, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int num_slices = ONCE ? slices_once & 255 : slices_once, once_from = slices_once >> 8;
   // ---- one trip: tile record, plan header, the tile's token rows, the slots' ranks ------------------
   MLORA_STAMP(0);  // shrink: first instruction
   const int tile = blockIdx.z * 8 + blockIdx.x;
@@ -507,11 +507,12 @@ __device__ __forceinline__ void expand_tile(char* lds, const float* __restrict__
 // grid (8, column ranges, tiles / 8)
 template <typename T, int C, int SP, bool ONCE>
 __global__ __launch_bounds__(kPairThreads) void pair_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws, void* __restrict__ yv_,
-                                                                   int64_t ys, int small_off, int T_, int num_slots, int kparts, int num_slices,
-                                                                   float scaling, const int32_t* __restrict__ eff_rank, int once_from, ExpandSplits splits) {
+                                                                   int64_t ys, int small_off, int T_, int num_slots, int kparts, int slices_once,
+                                                                   float scaling, const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int R = C * PieceOf<T>::E, RP = (R + 15) & ~15;
   const int lane = threadIdx.x & (kWave - 1), lg = lane >> 4;
+  const int num_slices = ONCE ? slices_once & 255 : slices_once, once_from = slices_once >> 8;
   MLORA_STAMP(8);  // expand: first instruction
   const ExpandSplit sp = splits.split[blockIdx.y];
   const int tile = blockIdx.z * 8 + blockIdx.x;
@@ -694,7 +695,8 @@ struct PairLaunch {
   PlanLayout lay;
   int parts_log2, sp;
   bool once;      // instances that can request A and B of a slot's only tile with the non-temporal hint
-  int once_from;  // and do so from this many slots with tokens on
+  int slices_once;  // number of slices, and for those instances above its eight bits from how many slots with tokens on they do (a word of its own
+                    // would lie behind the sixteen that arrive preloaded: 201 streams, 1760 us a step instead of 1754)
 };
 
 template <typename T, bool CHAINS, bool ONCE> void launch_pair_shrink_one(const PairLaunch& l) {
@@ -705,7 +707,7 @@ template <typename T, bool CHAINS, bool ONCE> void launch_pair_shrink_one(const 
   hipLaunchKernelGGL((pair_shrink_kernel<T, CHAINS, ONCE>), dim3(8, static_cast<unsigned>(a->num_slices << l.parts_log2), static_cast<unsigned>(l.lay.cap_small / 8)),
                      dim3(kPairThreads), shrink_lds(a->r), static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), l.lay.small_off,
                      a->num_tokens, a->num_slots, static_cast<int>(a->k * sizeof(T) / kChunk), static_cast<uint32_t>(a->x_stride * sizeof(T)), a->r,
-                     l.parts_log2, a->num_slices, a->effective_rank, l.once_from, sl);
+                     l.parts_log2, l.slices_once, a->effective_rank, sl);
 }
 
 template <typename T, bool CHAINS> void launch_pair_shrink(const PairLaunch& l) {
@@ -718,7 +720,7 @@ template <typename T, int C, int SP, bool ONCE> void launch_pair_expand_one(cons
   allow_lds<pair_expand_kernel<T, C, SP, ONCE>>(expand_lds(C, SP));
   hipLaunchKernelGGL((pair_expand_kernel<T, C, SP, ONCE>), dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(l.lay.cap_small / 8)), dim3(kPairThreads),
                      expand_lds(C, SP), static_cast<hipStream_t>(a->stream), a->plan, partials_of(a), a->y, a->y_stride, l.lay.small_off, a->num_tokens,
-                     a->num_slots, 1 << l.parts_log2, a->num_slices, a->scaling, a->effective_rank, l.once_from, splits);
+                     a->num_slots, 1 << l.parts_log2, l.slices_once, a->scaling, a->effective_rank, splits);
 }
 
 template <typename T, int C> bool launch_pair_expand(const PairLaunch& l, const ExpandSplits& splits, int total) {
@@ -864,8 +866,11 @@ int launch_pair(const MloraAddArgs* a, int active) {
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   // (how many slots have tokens is in the plan's header, which the kernels read: behind a capture the host knows only how many may)
   const long long per_slot = static_cast<long long>(a->r) * (static_cast<long long>(a->num_slices) * a->k + cols) * element_bytes(a->dtype);
-  l.once_from = pair_knobs().once > 0 ? 0 : static_cast<int>((kOnceBytes + per_slot - 1) / per_slot);
-  l.once = pair_knobs().once < 0 ? (active > 0 ? active : segs) >= l.once_from : pair_knobs().once != 0;
+  const long long need = (kOnceBytes + per_slot - 1) / per_slot;  // slots whose weights are that much
+  const int once_from = pair_knobs().once > 0 ? 0 : need <= MLORA_MAX_SLOTS ? static_cast<int>(need) : MLORA_MAX_SLOTS + 1;
+  l.once = pair_knobs().once < 0 ? (active > 0 ? active : segs) >= once_from : pair_knobs().once != 0;
+  static_assert(MLORA_MAX_SLICES < 256 && MLORA_MAX_SLOTS + 1 < 1 << 23, "one word");
+  l.slices_once = l.once ? a->num_slices | once_from << 8 : a->num_slices;
   // K parts: workgroups for most compute units, no more (every column range of the second launch
   // takes in every part's sums), and a chunk per wavefront at least
   int want = pair_knobs().kparts;
