@@ -40,6 +40,24 @@ union Pack8 {
 __device__ __forceinline__ i32x4 load128(const void* p) { return *reinterpret_cast<const i32x4*>(p); }
 __device__ __forceinline__ void store128(void* p, i32x4 v) { *reinterpret_cast<i32x4*>(p) = v; }
 
+// Stores of y that leave for memory at once (agent scope) instead of staying in the L2 until the kernel ends, where what is dirty is written back
+// with nothing else going on.  The memory-side cache keeps such lines as it keeps others, so a launch that reads y next pays nothing
+// (a copy, the apply and a copy of y, less the copies, us, plain stores / these: 9392 tokens, rank 64, down 30.1 / 28.9; 3001 tokens, rank 16, K = 2048, gate_up
+// 35.0 / 34.1, down 17.9 / 17.4; 1234 tokens, rank 32, gate_up 13.8 / 13.1).  By themselves, us per call: 64-token tiles, 9392 tokens, rank 64, K = 1024, o 15.8 /
+// 14.8, q|k|v 24.0 / 23.0, down 29.1 / 28.3, 3001 tokens, rank 16, K = 2048, gate_up 52.0 / 49.9; 16-token tiles, 3001 tokens q|k|v 14.6 / 14.1, o 10.6 / 10.3.
+// Launches that write less lose the wait for every store, so 16-token tiles take them from kThroughBytes of y on: 1000 tokens, K = 1024, o (2.0 MB) 5.0 / 4.85, gate_up
+// of 120 tokens at K = 2048 (3.9 MB) 6.9 / 6.5; 400 tokens q|k|v (1.2 MB) 4.82 / 4.87, o (0.8 MB) 4.67 / 4.74; one stream's step of 48 calls 158 / 161; 256 streams'
+// and the pair's outputs the same or 1 % slower a step.
+constexpr long long kThroughBytes = 2000000;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store_through(void* p, u32x4 v) {
+  __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)(p), v, "agent");
+}
+__device__ __forceinline__ void store_through(void* p, u32x2 v) {
+  __hip_atomic_store(static_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Dot product of eight 16-bit pairs accumulated in fp32 with the packed dot2 instructions.
 template <typename T> __device__ __forceinline__ float dot8(const Pack8& a, const Pack8& b, float acc);
 template <> __device__ __forceinline__ float dot8<__bf16>(const Pack8& a, const Pack8& b, float acc) {

@@ -36,6 +36,7 @@ namespace {
 
 constexpr int kMaxSplits = 32;
 constexpr int kNW = 8;          // wavefronts per workgroup
+constexpr int kThrough = 2;     // bit of include_long: y leaves at once (store_through)
 constexpr int kSpansAheadMax = 2;  // output spans per wavefront whose loads are issued up front (SA: 1 or 2)
 
 MLORA_TRACE_DECL
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT)) void deco
   // compiler requests this launch's column range only after the header has arrived)
   __builtin_amdgcn_sched_barrier(0);
   const int slot = rec0[0], m = rec0[1];
-  const int n_tiles = hdr[MLORA_PLAN_TILES_SHORT] + hdr[MLORA_PLAN_TILES_LONG_SMALL] * include_long;
+  const int n_tiles = hdr[MLORA_PLAN_TILES_SHORT] + hdr[MLORA_PLAN_TILES_LONG_SMALL] * (include_long & 1);
   // One exit test, evaluated without short-circuit, that consumes everything fetched above
   // (the token index through its first lane), so that all of it is requested here, together,
   // instead of piece by piece behind a chain of branches.
@@ -285,12 +286,13 @@ void launch_rank(const Launch& l, int r, int kspw) {
 
 // Diagnostic knobs, read from the environment once per process.
 struct DecodeKnobs {
-  int generation = -1, staged, nt, short_tiles;
+  int generation = -1, staged, nt, short_tiles, through;
   void read() {
     generation = knob_generation();
     staged = env_int("MLORA_DECODE_STAGED", 1);
     nt = env_int("MLORA_DECODE_NT", 0);
     short_tiles = env_int("MLORA_DECODE_SHORT", -1);
+    through = env_int("MLORA_DECODE_THROUGH", -1);
   }
 };
 const DecodeKnobs& decode_knobs() {
@@ -381,6 +383,9 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
     }
   }
   l.short_tiles = decode_knobs().short_tiles < 0 ? a->num_tokens <= (l.widest <= kNW * 64 ? 12 : 4) * with_tokens : decode_knobs().short_tiles != 0;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  if (decode_knobs().through < 0 ? a->num_tokens * cols * 2 >= kThroughBytes : decode_knobs().through != 0) l.include_long |= kThrough;
   for (; s < kMaxSplits; ++s) splits.split[s] = DecodeSplit{nullptr, nullptr, 0, 0, 0, 0};
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(cap / 8));
   const int nks = a->k / 32;

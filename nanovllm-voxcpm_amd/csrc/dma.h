@@ -36,6 +36,24 @@ __device__ __forceinline__ void dma16_once(const void* base, uint32_t voff, uint
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(voff), "s"(base) : "memory");
 }
 
+// From a lane's own 64-bit address (rows of x and y lie anywhere).
+__device__ __forceinline__ void dma16v(const char* p, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
+}
+
+// Waits until no more than `younger` (at most MOST) stages of PER loads each are on their way.
+template <int PER, int MOST> __device__ __forceinline__ void wait_stages(int younger) {
+  if (younger >= MOST) wait_loads<MOST * PER>();
+  else if (MOST > 1 && younger == MOST - 1) wait_loads<(MOST > 1 ? MOST - 1 : 0) * PER>();
+  else if (MOST > 2 && younger == MOST - 2) wait_loads<(MOST > 2 ? MOST - 2 : 0) * PER>();
+  else if (MOST > 3 && younger == MOST - 3) wait_loads<(MOST > 3 ? MOST - 3 : 0) * PER>();
+  else if (MOST > 4 && younger == MOST - 4) wait_loads<(MOST > 4 ? MOST - 4 : 0) * PER>();
+  else wait_loads<0>();
+}
+
+// A barrier that waits for no load.
+__device__ __forceinline__ void stage_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
 }  // namespace
 
 }  // namespace mlora

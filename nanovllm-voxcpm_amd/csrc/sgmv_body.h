@@ -28,6 +28,8 @@ constexpr int kSlabStages = 4;  // 128-byte pieces of K in a part of slab.hip's 
 //   rank 16, K = 2048             78 MB 247 +1.3 / 98 +2.9 / 42 -2.9     94 MB 247 +0.2 / 115 -0.2 / 49 -3.9   128 MB 325 +3.1 / 154 -0.7 / 65 -5.2
 //                                138 MB 433 +3.2 / 167 +2.6 / 68 -6.0   188 MB 476 -0.1 / 226 -3.2 / 88 -8.6   256 MB 636 -2.9 / 317 -8.6 / 122 -12
 // Up to 138 MB one or the other of the two pays for it somewhere, from 147 MB on they gain or stay within half a percent.
+// (The figures are of plain stores without the hint.  With store_through instead, copies' way, hint / without: rank 64, K = 2048, 140 MB 49.2 / 51.4, K = 1024, 147 MB
+// 55.7 / 55.3, rank 16, 147 MB 47.7 / 48.3, and 125 MB of 64 slots 39.9 / 39.8 without by the line.)
 constexpr long long kStreamBytes = 140ll << 20;
 constexpr int kMaxKSplit = 4;  // most K parts the shrink ever uses (the workspace has room for them)
 
@@ -439,14 +441,13 @@ template <typename T, int N> union alignas(N * sizeof(T)) YVec {
   uint32_t u[N / 2];
 };
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <int N> struct YRaw;
 template <> struct YRaw<4> { typedef u32x2 type; };
 template <> struct YRaw<8> { typedef u32x4 type; };
 
 // y is touched once per launch.  STREAM: its loads and stores carry the non-temporal hint (kStreamBytes says when
-// and what it gives).  An item
+// and what it gives); without, the stores leave at once (store_through; hinted loads with such stores are slower than either: 9392 tokens, rank
+// 64, gate_up 57.5 -> 60.6).  An item
 // stays the raw vectors it was fetched as until it is used: unpacked where it is requested, its
 // arithmetic is scheduled ahead of the barrier that ends the staging of the intermediate, and the
 // wavefront waits for the item in front of work that could have run meanwhile.
@@ -468,7 +469,7 @@ __device__ __forceinline__ void store_y(T* p, const YVec<T, N>& v) {
   Raw r;
   __builtin_memcpy(&r, &v, sizeof(r));
   if constexpr (STREAM) __builtin_nontemporal_store(r, reinterpret_cast<Raw*>(p));
-  else *reinterpret_cast<Raw*>(p) = r;
+  else store_through(p, r);
 }
 
 // Body of the expand for the tiles of one workgroup.  MASKED: some tile's slot holds an adapter of
