@@ -907,7 +907,8 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   if (kr != 128 && kr != 256 && kr != 512) kr = xw;
   if (kr > xw) kr = xw;
   if (kr == 128) xw = 128;  // 128-column slabs come with 128-column batches only
-  const int max_parts = static_cast<int>(partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r));
+  int max_parts = static_cast<int>(partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r));
+  if (max_parts < 1) max_parts = 1;  // (wide.hip's cut needs no workspace; the others' launches have made sure of one)
   int ksplit = sgmv_knobs().ksplit;
   if (ksplit <= 0) {
     ksplit = 1;
