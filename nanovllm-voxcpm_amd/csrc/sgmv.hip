@@ -154,10 +154,10 @@ __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(con
 #pragma unroll
   for (int g = 0; g < G; ++g) masked |= m[g] > 0 && eff[g] < R;
   if (masked)
-    expand_body<T, R, CPL, TPF, G, true, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, true, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
                                          m, eff, rowv);
   else
-    expand_body<T, R, CPL, TPF, G, false, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
                                           m, eff, rowv);
 }
 
