@@ -37,26 +37,26 @@ static_assert(kFusedThreads == kShrinkWaves * kWave && kFusedThreads == kExpandW
 // The two products as functions of their own (not inlined into the kernel): each gets the register
 // file to itself, as in the two-launch form, instead of one allocation that has to carry the
 // kernel's state through both.
-template <typename T, int R, int KR, int XW, bool DB>
+template <typename T, int R, int KR>
 __device__ __forceinline__ void fused_shrink_role(T* __restrict__ s_a, const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws, int64_t xs, int sorted_off,
-                                                            int T_, int K, int num_slices, int krange, int all_slices, const ShrinkSlices& sl,
+                                                            int T_, int K, int num_slices, int krange, const ShrinkSlices& sl,
                                                             int slice0, int kpart, int slot, int start, int m, int eff) {
   // token row of this lane (positions past the end of the tile repeat its last token)
   const int ti = (threadIdx.x / kWave) * 16 + (threadIdx.x & 15);
   const int row = plan[sorted_off + start + (ti < m ? ti : m - 1)];
   if (R > 16 && ((eff + 15) >> 4) < (R + 15) / 16)
-    shrink_body<T, R, KR, XW, DB, true, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, slot, start, m, eff, row);
+    shrink_body<T, R, KR, true, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
   else
-    shrink_body<T, R, KR, XW, DB, false, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, slot, start, m, eff, row);
+    shrink_body<T, R, KR, false, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
 }
 
 // The same for the roles a workgroup computes because their seals did not arrive: the exception, so
 // a function of its own (called in a loop) rather than a second inlined copy.
-template <typename T, int R, int KR, int XW, bool DB>
+template <typename T, int R, int KR>
 __device__ __attribute__((noinline)) void fused_shrink_role_late(T* s_a, const int32_t* plan, const void* xv, float* hws, int64_t xs, int sorted_off,
-                                                                 int T_, int K, int num_slices, int krange, int all_slices, const ShrinkSlices& sl,
+                                                                 int T_, int K, int num_slices, int krange, const ShrinkSlices& sl,
                                                                  int slice0, int kpart, int slot, int start, int m, int eff) {
-  fused_shrink_role<T, R, KR, XW, DB>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, slot, start, m, eff);
+  fused_shrink_role<T, R, KR>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff);
 }
 
 template <typename T, int R, int CPL, int TPF, int G>
@@ -82,11 +82,11 @@ __device__ __forceinline__ void fused_expand(T* s_h, int* s_row, int* s_slot, in
                                                 m, eff, rowv);
 }
 
-template <typename T, int R, int KR, int XW, bool DB, int CPL, int TPF, int G>
+template <typename T, int R, int KR, int CPL, int TPF, int G>
 __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
     const int32_t* __restrict__ plan, const void* __restrict__ xv, void* __restrict__ yv_, uint32_t* __restrict__ ws,
     float* __restrict__ hws, int64_t xs, int64_t ys, int big_off, int small_off, int big_units, int sorted_off, int T_, int K,
-    int num_slots, int num_slices, int ksplit, int krange, int all_slices, float scaling, int spin_ticks, int trusted,
+    int num_slots, int num_slices, int ksplit, int krange, float scaling, int spin_ticks, int trusted,
     const int32_t* __restrict__ eff_rank, ShrinkSlices sl, ExpandSplits splits) {
   constexpr int HSTRIDE = 2 * R + 8;
   constexpr int kShrinkLds = R * (KR + 8) * static_cast<int>(sizeof(T));
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
 
   // ---- the unit's shrink roles ------------------------------------------------------------------------
   // role s = (tile g of the group, q): q is a K part when a workgroup walks all slices, else (slice, K part)
-  const int rpt = all_slices ? ksplit : num_slices * ksplit;
+  const int rpt = num_slices * ksplit;
   const int YS = G * rpt;  // <= 64 (host)
   // a seal: {tag, XCD the sealing workgroup ran on}.  The partial sums are ordinary stores, which
   // come to rest in the L2 of the writer's XCD; only a reader on the same XCD finds them there, so
@@ -184,17 +184,17 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
   for (int s = 0; s < YS; ++s) {
     const int g = s / rpt, q = s - g * rpt;
     if (__builtin_amdgcn_readfirstlane(s_m[g]) <= 0) continue;
-    if (all_slices || q / ksplit == sp.slice) need |= 1ull << s;
+    if (q / ksplit == sp.slice) need |= 1ull << s;
   }
   const uint64_t mine = have_role ? 1ull << c : 0;
 
   if (have_role) {
     const int q = c - my_g * rpt;
-    const int slice0 = all_slices ? 0 : q / ksplit, kpart = all_slices ? q : q % ksplit;
+    const int slice0 = q / ksplit, kpart = q % ksplit;
     // (the same for every lane: kept in scalar registers, and with them every address derived from them)
     const int gs = __builtin_amdgcn_readfirstlane(s_slot[my_g]), gm = __builtin_amdgcn_readfirstlane(s_m[my_g]);
     const int ge = __builtin_amdgcn_readfirstlane(s_eff[my_g]), gstart = __builtin_amdgcn_readfirstlane(s_start[my_g]);
-    fused_shrink_role<T, R, KR, XW, DB>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, gs, gstart,
+    fused_shrink_role<T, R, KR>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, sl, slice0, kpart, gs, gstart,
                                         gm, ge);
   }
   MLORA_STAMP(10);  // own role multiplied, its stores issued
@@ -233,9 +233,9 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
     for (int s = 0; s < YS; ++s) {
       if (!((todo >> s) & 1)) continue;
       const int g = s / rpt, q = s - g * rpt;
-      const int slice0 = all_slices ? 0 : q / ksplit, kpart = all_slices ? q : q % ksplit;
+      const int slice0 = q / ksplit, kpart = q % ksplit;
       __syncthreads();  // every wavefront is done with the previous role's last slab
-      fused_shrink_role_late<T, R, KR, XW, DB>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, all_slices, sl, slice0, kpart,
+      fused_shrink_role_late<T, R, KR>(s_a, plan, xv, hws, xs, sorted_off, T_, K, num_slices, krange, sl, slice0, kpart,
                                                s_slot[g], s_start[g], s_m[g], s_eff[g]);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -270,21 +270,21 @@ struct FusedLaunch {
   int trusted;
 };
 
-template <typename T, int R, int KR, int XW, bool DB, int G>
+template <typename T, int R, int KR, int G>
 void launch_fused_one(const FusedLaunch& l) {
   const MloraAddArgs* a = l.a;
   const SgmvShape& sh = *l.sh;
   dim3 grid(8, static_cast<unsigned>(sh.nsplit), static_cast<unsigned>(sh.units / 8));
-  hipLaunchKernelGGL((sgmv_fused_kernel<T, R, KR, XW, DB, 8, 2, G>), grid, dim3(kFusedThreads), 0, static_cast<hipStream_t>(a->stream), a->plan,
+  hipLaunchKernelGGL((sgmv_fused_kernel<T, R, KR, 8, 2, G>), grid, dim3(kFusedThreads), 0, static_cast<hipStream_t>(a->stream), a->plan,
                      a->x, a->y, static_cast<uint32_t*>(a->workspace), partials_of(a), a->x_stride, a->y_stride, sh.lay.big_off,
                      sh.lay.small_off, sh.big_units, sh.lay.sorted_off, a->num_tokens, a->k, a->num_slots, a->num_slices, sh.ksplit,
-                     sh.krange, sh.all_slices, a->scaling, fused_knobs().spin_ticks, l.trusted, a->effective_rank,
+                     sh.krange, a->scaling, fused_knobs().spin_ticks, l.trusted, a->effective_rank,
                      sh.sl, sh.splits);
 }
 
 template <typename T, int R, int G>
 void launch_fused_slab(const FusedLaunch& l) {
-  launch_fused_one<T, R, 256, 256, true, G>(l);
+  launch_fused_one<T, R, 256, G>(l);
 }
 
 template <typename T, int R>
@@ -307,9 +307,8 @@ void launch_fused_rank(const FusedLaunch& l) {
 // one tile or four per unit.  And what the head of the workspace has room for.
 bool shape_fits(const MloraAddArgs* a, const SgmvShape& sh) {
   if (sh.empty) return true;
-  const bool slab = sh.kr == 256 && sh.xw == 256 && !sh.all_slices;
-  if (!slab || sh.cpl != 8 || (sh.group != 1 && sh.group != 4)) return false;
-  const int roles = sh.group * (sh.all_slices ? sh.ksplit : a->num_slices * sh.ksplit);
+  if (a->k % 256 != 0 || sh.cpl != 8 || (sh.group != 1 && sh.group != 4)) return false;
+  const int roles = sh.group * a->num_slices * sh.ksplit;
   if (roles > 64 || roles > sh.nsplit || sh.units > kWsTiles) return false;  // one shrink role per workgroup of a unit
   return static_cast<int64_t>(sh.units) * roles * 8 <= kWsSealBytes;
 }

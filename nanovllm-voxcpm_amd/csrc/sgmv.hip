@@ -9,16 +9,15 @@
 // short segments (one small-tile record each).
 //
 //   shrink — H^T[rank x tokens] = A[slot] . X_tile^T for a (tile, slice, K part).  What bounds
-//            this product is the number of bytes a compute unit takes in (cache hits cost about
-//            as much as misses: the limit is requests in flight), so each operand element is
-//            fetched once per workgroup: the A[slot] slab of the workgroup's K part is copied to
-//            LDS with row-contiguous 128-bit loads and shared by the four wavefronts, each of
-//            which owns sixteen tokens of the tile and streams their x rows straight from global
-//            memory into the MFMA operand layout, a whole batch of k-steps in flight at a time.
-//            No wavefront shares a sum with another, so the accumulators go straight to the
+//            this product is what a compute unit takes in (down of the prefill batch: 117 MB of x and A, 13.4 us as loads
+//            alone), so each operand element is fetched once per workgroup, in whole row pieces straight to LDS, through a
+//            ring of up to eight stages that the four wavefronts fill and read together.  No wavefront shares a sum with
+//            another, so the accumulators go straight to the
 //            workspace as fp32; when K is split across workgroups each part writes its own
-//            partial.  For three or more slices one workgroup walks all of them with the x rows
-//            it holds.
+//            partial.  (Before, the wavefronts streamed their x rows into registers in the matrix cores' operand layout, at a third of the
+//            rate out of the L2, and A slab by slab through LDS: us per call, before / now, in the parts that were cut then: 7000 tokens, rank 64, K = 4096
+//            30.4 / 29.4, gate_up 66.2 / 65.4; with parts that need not divide K 9000 tokens 43.4 / 39.4 and 76.8 / 72.1, K = 8192, 4500
+//            47.5 / 38.0; 5000 mixed tokens down 34.1 / 32.4, gate_up 78.5 / 75.7.)
 //   expand — OUT[tokens x cols] = H . B[slot]^T for a (group of tiles, column range).  The H
 //            tiles are staged in LDS once (K partials summed, scaled, and split into a hi + lo
 //            pair of operand-precision values, about 16 significant bits: the expand loses
@@ -31,45 +30,173 @@
 //            in fully coalesced accesses with no transposition pass.
 // Splitting the two products means no column range repeats the shrink of its tile, and each
 // kernel keeps only its own operands in registers.
+#include "dma.h"
+#include "lds.h"
 #include "sgmv_body.h"
 
 namespace mlora {
 
 namespace {
 
-template <typename T, int R, int KR, int XW, bool DB>
-__global__ __launch_bounds__(kShrinkWaves* kWave, 2) void sgmv_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv,
-                                                                             float* __restrict__ hws, int64_t xs, int big_off,
-                                                                             int small_off, int big_cap, int bigrows_off, int T_, int K,
-                                                                             int num_slots, int num_slices, int ksplit, int krange,
-                                                                             int all_slices, const int32_t* __restrict__ eff_rank, ShrinkSlices sl) {
-  constexpr int ASTRIDE = KR + 8;  // padded LDS row: 16 rows x 16 bytes cover all banks once
-  __shared__ __attribute__((aligned(16))) T s_a[R * ASTRIDE];
-  // all_slices: the workgroup walks every slice of the projection with the x rows it holds in
-  // registers (its K part is a single batch then), instead of one workgroup per slice
-  const int slice0 = all_slices ? 0 : blockIdx.y / ksplit, kpart = all_slices ? blockIdx.y : blockIdx.y % ksplit;
-  const int tile = tile_position(big_cap);  // blockIdx.x is the XCD
+// ---- shrink -------------------------------------------------------------------------------------
+constexpr int kRingWaves = 4;
+constexpr int kRingThreads = kRingWaves * kWave;
+constexpr int kRing = kMostLds / 2;  // of LDS, so that two workgroups fit a compute unit
+constexpr int kRingStage = 24;       // KB of a stage at most
+
+// NA8: groups of eight ranks, TB: blocks of sixteen tokens; both operands in groups of eight rows, 1 KB (128 bytes of K) each.
+template <int NA8, int TB> struct RingShape {
+  static constexpr int RB = (NA8 + 1) / 2;
+  static constexpr int PIECE = NA8 + 2 * TB;                                                   // direct loads of 128 bytes of K
+  static constexpr int P = PIECE * 4 <= kRingStage ? 4 : PIECE * 2 <= kRingStage ? 2 : 1;      // such pieces of a stage
+  static constexpr int BYTES = P * PIECE * 1024;
+  static constexpr int NST = kRing / BYTES > 8 ? 8 : kRing / BYTES;                            // stages of the ring
+  static constexpr int LO = PIECE / kRingWaves, HI = (PIECE + kRingWaves - 1) / kRingWaves;    // a wavefront's loads of a piece
+  static constexpr int WT = RB > 1 ? (TB < 2 ? TB : 2) : TB;                                   // wavefronts across the tokens
+  static constexpr int WR = RB < kRingWaves / WT ? RB : kRingWaves / WT;                       // and across the ranks
+  static constexpr int BR = RB / WR, BT = TB / WT;
+  static_assert(NST >= 3 && (NST - 2) * HI * P <= 63, "the wait for a stage counts what is younger");
+};
+
+// The sums of a tile over pieces [c0, c1) of K.  The wavefronts share out the loads of a stage and the blocks of sixteen tokens by sixteen ranks; every
+// block adds K up in one chain, as the one-launch form (fused.hip) does.
+template <typename T, int NA8, int TB>
+__device__ __forceinline__ void ring_tile(char* lds, const char* abase, uint32_t arow, const char* const (&xrow)[2], int c0, int c1, float* __restrict__ dst,
+                                          int64_t hrow, int r_all, int m) {
+  typedef RingShape<NA8, TB> S;
+  constexpr int NST = S::NST, BR = S::BR, BT = S::BT, P = S::P;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lr = lane & 15, lg = lane >> 4;
+  // which groups of eight rows a wavefront asks for: of tokens `wave` and `wave + 4`, of ranks the same, where there are fewer from the last wavefront down
+  constexpr int NX = TB == 4 ? 2 : 1, NA = NA8 == 8 ? 2 : 1;
+  const bool has_x = TB > 1 || wave < 2, has_a = NA8 >= 4 || wave >= 4 - NA8;
+  const int a0 = NA8 >= 4 ? wave : has_a ? wave - (4 - NA8) : 0;
+  const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;  // chunk p of a row goes to place p ^ (row & 7)
+  uint32_t aoff[NA];
+#pragma unroll
+  for (int g = 0; g < NA; ++g) aoff[g] = static_cast<uint32_t>((a0 + 4 * g) * 8 + (lane >> 3)) * arow + swz;
+  const uint32_t to0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
+  auto issue = [&](int s, int stage) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      int c = c0 + s * P + p;
+      if (P > 1) c = c < c1 ? c : c1 - 1;  // (a repeated piece is not multiplied)
+      const uint32_t to = to0 + stage * S::BYTES + p * (S::PIECE * 1024);
+      if (has_x) {
+#pragma unroll
+        for (int g = 0; g < NX; ++g) dma16v(xrow[g] + static_cast<int64_t>(c) * 128 + swz, to + (NA8 + wave + 4 * g) * 1024);
+      }
+      if (has_a) {
+#pragma unroll
+        for (int g = 0; g < NA; ++g) dma16(abase + static_cast<int64_t>(c) * 128, aoff[g], to + (a0 + 4 * g) * 1024);
+      }
+    }
+  };
+  const bool hi = S::HI == S::LO || (has_x ? NX : 0) + (has_a ? NA : 0) == S::HI;
+  const int wt = wave % S::WT, wr = wave / S::WT;
+  const bool works = wr < S::WR;
+  f32x4 acc[BR][BT];
+#pragma unroll
+  for (int rb = 0; rb < BR; ++rb)
+#pragma unroll
+    for (int tb = 0; tb < BT; ++tb) acc[rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int n = (c1 - c0 + P - 1) / P;
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < n) issue(s, s);
+  MLORA_STAMP(2);  // shrink: first stages requested
+  const uint32_t read = lr * 128 + ((lg ^ (lr & 7)) * 16);
+  int stage = 0, into = NST - 1;
+  for (int s = 0; s < n; ++s) {
+    const int younger = n - 1 - s < NST - 2 ? n - 1 - s : NST - 2;
+    wait_lds();  // this wavefront's operand reads of the stage before are through
+    if (hi) wait_stages<S::HI * P, NST - 2>(younger);
+    else wait_stages<S::LO * P, NST - 2>(younger);
+    stage_barrier();  // the stage is whole, and the one before has been read by all
+    if (s + NST - 1 < n) issue(s + NST - 1, into);
+    if (works) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        if (P > 1 && c0 + s * P + p >= c1) break;
+        Pack8 xa[2][BT], aw[2][BR];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const char* at = lds + stage * S::BYTES + p * (S::PIECE * 1024) + (read ^ (ks * 64));  // chunk lg, then chunk lg + 4, of the swizzled row
+#pragma unroll
+          for (int tb = 0; tb < BT; ++tb) xa[ks][tb].raw = *reinterpret_cast<const i32x4*>(at + (NA8 + 2 * (wt * BT + tb)) * 1024);
+#pragma unroll
+          for (int rb = 0; rb < BR; ++rb) aw[ks][rb].raw = *reinterpret_cast<const i32x4*>(at + (wr * BR + rb) * 2048 - (NA8 == 1 ? (lr & 8) * 128 : 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int rb = 0; rb < BR; ++rb)
+#pragma unroll
+            for (int tb = 0; tb < BT; ++tb) acc[rb][tb] = Mma<T>::run(aw[ks][rb], xa[ks][tb], acc[rb][tb]);
+      }
+    }
+    stage = stage + 1 == NST ? 0 : stage + 1;
+    into = into + 1 == NST ? 0 : into + 1;
+  }
+#pragma unroll
+  for (int rb = 0; rb < BR; ++rb) mfma_settle(acc[rb]);  // (the last products and the reads of the sums lie on two sides of branches)
+  MLORA_STAMP(5);  // shrink: multiplied
+  if (!works) return;
+  // acc[rb][tb]: lane holds ranks 16 rb + 4 lg .. + 3 of token lr of the block
+#pragma unroll
+  for (int rb = 0; rb < BR; ++rb)
+#pragma unroll
+    for (int tb = 0; tb < BT; ++tb) {
+      const int tok = (wt * BT + tb) * 16 + lr, r = (wr * BR + rb) * 16 + 4 * lg;
+      if (tok < m && r < r_all) *reinterpret_cast<f32x4*>(dst + tok * hrow + r) = acc[rb][tb];
+    }
+}
+
+// grid (8, slices * K parts, tiles / 8): blockIdx.x is the XCD
+template <typename T>
+__global__ __launch_bounds__(kRingThreads, 2) void sgmv_shrink_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, float* __restrict__ hws,
+                                                                      int64_t xs, int big_off, int small_off, int big_cap, int bigrows_off, int T_, int K,
+                                                                      int num_slots, int num_slices, int parts, int R, const int32_t* __restrict__ eff_rank,
+                                                                      ShrinkSlices sl) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int tile = tile_position(big_cap);
   MLORA_STAMP(0);  // first instruction
-  const int row = tile_row(plan, bigrows_off, small_off, big_cap, tile, (threadIdx.x / kWave) * 16 + (threadIdx.x & 15));
+  int row[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) row[g] = tile_row(plan, bigrows_off, small_off, big_cap, tile, (wave + 4 * g) * 8 + (lane >> 3));
   const TileRef tr = fetch_tile(plan, big_off, small_off, big_cap, tile, T_, num_slots);
+  const RankPrefetch ranks = rank_prefetch(eff_rank, num_slots, lane);
+  __builtin_amdgcn_sched_barrier(0);
   if (!tr.ok) {
     count_rejected_plan(plan, tr.plan_ok);
     return;
   }
   MLORA_STAMP(1);  // tile record here
-  // rank of the adapter in this slot (a second, dependent fetch, only with the vector given)
-  int eff = R;
-  if (R > 16 && eff_rank) {
-    eff = eff_rank[tr.slot];
-    eff = eff < 0 ? 0 : eff > R ? R : eff;
-    if (eff == 0) return;
-  }
-  if (R > 16 && ((eff + 15) >> 4) < (R + 15) / 16)
-    shrink_body<T, R, KR, XW, DB, true>(s_a, xv, hws, xs, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, tr.slot, tr.start, tr.m,
-                                        eff, row);
-  else
-    shrink_body<T, R, KR, XW, DB, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, all_slices, sl, slice0, kpart, tr.slot, tr.start, tr.m,
-                                         eff, row);
+  const int slot = __builtin_amdgcn_readfirstlane(tr.slot), m = __builtin_amdgcn_readfirstlane(tr.m), start = __builtin_amdgcn_readfirstlane(tr.start);
+  const int eff = __builtin_amdgcn_readfirstlane(rank_pick(ranks, eff_rank, num_slots, slot, R));
+  if (eff == 0) return;
+  const int slice = blockIdx.y / parts, part = blockIdx.y - slice * parts;
+  const int chunks = K / 64, c0 = part * chunks / parts, c1 = (part + 1) * chunks / parts;
+  const uint32_t arow = static_cast<uint32_t>(K) * sizeof(T);
+  const char* abase = uniform(static_cast<const char*>(sl.a[slice]) + static_cast<int64_t>(slot) * R * arow);
+  const char* xrow[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) xrow[g] = reinterpret_cast<const char*>(static_cast<const T*>(xv) + static_cast<int64_t>(row[g]) * xs);
+  const int64_t hrow = static_cast<int64_t>(num_slices) * R;
+  float* dst = hws + (static_cast<int64_t>(part) * T_ + start) * hrow + slice * R;
+  const int groups = (eff + 7) >> 3;  // (ranks beyond the adapter's in its last block: the expand does not use them)
+  auto by_groups = [&](auto tb) __attribute__((always_inline)) {
+    constexpr int TB = decltype(tb)::value;
+    if (groups <= 1) ring_tile<T, 1, TB>(lds, abase, arow, xrow, c0, c1, dst, hrow, R, m);
+    else if (groups == 2) ring_tile<T, 2, TB>(lds, abase, arow, xrow, c0, c1, dst, hrow, R, m);
+    else if (groups <= 4) ring_tile<T, 4, TB>(lds, abase, arow, xrow, c0, c1, dst, hrow, R, m);
+    else ring_tile<T, 8, TB>(lds, abase, arow, xrow, c0, c1, dst, hrow, R, m);
+  };
+  if (m <= 16) by_groups(std::integral_constant<int, 1>{});
+  else if (m <= 32) by_groups(std::integral_constant<int, 2>{});
+  else by_groups(std::integral_constant<int, 4>{});
 #ifdef MLORA_TRACE
   MLORA_STAMP(6);  // partial sums issued
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -77,6 +204,7 @@ __global__ __launch_bounds__(kShrinkWaves* kWave, 2) void sgmv_shrink_kernel(con
 #endif
 }
 
+// ---- expand -------------------------------------------------------------------------------------
 template <typename T, int R, int CPL, int TPF, int G, bool STREAM>
 __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws,
                                                                              void* __restrict__ yv_, int64_t ys, int big_off, int small_off,
@@ -161,41 +289,11 @@ __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(con
                                           m, eff, rowv);
 }
 
-struct ShrinkLaunch {
-  const MloraAddArgs* a;
-  PlanLayout lay;
-  ShrinkSlices sl;
-  int tiles8;   // grid extent over tiles / 8
-  int big_cap;  // workgroups below this index take 64-token tiles, the rest short segments
-  int ksplit, krange, all_slices;
-};
-
-template <typename T, int R, int KR, int XW, bool DB>
-void launch_shrink_one(const ShrinkLaunch& l) {
-  const MloraAddArgs* a = l.a;
-  dim3 grid(8, static_cast<unsigned>(l.all_slices ? l.ksplit : a->num_slices * l.ksplit), static_cast<unsigned>(l.tiles8));
-  hipLaunchKernelGGL((sgmv_shrink_kernel<T, R, KR, XW, DB>), grid, dim3(kShrinkWaves * kWave), 0, static_cast<hipStream_t>(a->stream),
-                     a->plan, a->x, partials_of(a), a->x_stride, l.lay.big_off, l.lay.small_off, l.big_cap,
-                     l.lay.bigrows_off, a->num_tokens, a->k, a->num_slots, a->num_slices, l.ksplit, l.krange, l.all_slices, a->effective_rank, l.sl);
-}
-
-// (slab width, x batch width): 128/128 and 256/256 with two x buffers, 256/512 and 512/512 with one
-template <typename T, int R>
-void launch_shrink_slab(const ShrinkLaunch& l, int kr, int xw) {
-  if (kr == 128) launch_shrink_one<T, R, 128, 128, true>(l);
-  else if (kr == 256 && xw == 256) launch_shrink_one<T, R, 256, 256, true>(l);
-  else if (kr == 256) launch_shrink_one<T, R, 256, 512, false>(l);
-  else launch_shrink_one<T, R, 512, 512, false>(l);
-}
-
-template <typename T>
-void launch_shrink_rank(const ShrinkLaunch& l, int kr, int xw) {
-  switch (l.a->r) {
-    case 8: launch_shrink_slab<T, 8>(l, kr, xw); break;
-    case 16: launch_shrink_slab<T, 16>(l, kr, xw); break;
-    case 32: launch_shrink_slab<T, 32>(l, kr, xw); break;
-    default: launch_shrink_slab<T, 64>(l, kr, xw); break;
-  }
+template <typename T> void launch_shrink(const MloraAddArgs* a, const SgmvShape& sh) {
+  allow_lds<sgmv_shrink_kernel<T>>(kRing);
+  hipLaunchKernelGGL((sgmv_shrink_kernel<T>), dim3(8, static_cast<unsigned>(a->num_slices * sh.ksplit), static_cast<unsigned>(sh.tiles8)), dim3(kRingThreads), kRing,
+                     static_cast<hipStream_t>(a->stream), a->plan, a->x, partials_of(a), a->x_stride, sh.lay.big_off, sh.lay.small_off, sh.big_cap,
+                     sh.lay.bigrows_off, a->num_tokens, a->k, a->num_slots, a->num_slices, sh.ksplit, a->r, a->effective_rank, sh.sl);
 }
 
 template <typename T, int R>
@@ -258,12 +356,9 @@ bool sgmv_workspace_ok(const MloraAddArgs* a) {
 int launch_sgmv(const MloraAddArgs* a, int active) {
   const SgmvShape sh = sgmv_shape(a, false, active);
   if (sh.empty) return 0;
-  ShrinkLaunch l;
-  l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.tiles8 = sh.tiles8; l.big_cap = sh.big_cap;
-  l.ksplit = sh.ksplit; l.krange = sh.krange; l.all_slices = sh.all_slices;
   if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.sl.a);
-  else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink_rank<__bf16>(l, sh.kr, sh.xw);
-  else launch_shrink_rank<_Float16>(l, sh.kr, sh.xw);
+  else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink<__bf16>(a, sh);
+  else launch_shrink<_Float16>(a, sh);
   int rc = check_launch("mlora_add_lora(sgmv shrink)");
   if (rc) return rc;
 

@@ -100,14 +100,10 @@ __device__ __forceinline__ int tile_row(const int32_t* __restrict__ plan, int bi
 }
 
 // ---- shrink -------------------------------------------------------------------------------------
-// grid (8, slices * K parts, tiles / 8), four wavefronts of sixteen tokens each.  The workgroup's
-// K part is walked in x batches of XW columns (a wavefront holds the batch of its sixteen token
-// rows in registers) and, inside a batch, in A slabs of KR columns that pass through LDS.  Both
+// Of the one-launch form (fused.hip): four wavefronts of sixteen tokens each walk a K part in batches of KR columns (a wavefront holds the batch of its
+// sixteen token rows in registers) and A slabs of as many columns that pass through LDS.  Both
 // streams run one step ahead of the MFMAs: the next slab sits in registers and the next x batch
-// is in flight while the current slab is multiplied, so that a compute unit keeps requesting
-// data for the whole life of the workgroup instead of in bursts between barriers.  DB: a second
-// register buffer for the x batches (without it a K part of several batches fetches each batch
-// after the previous one has been consumed; the launcher gives such parts the DB form).
+// is in flight while the current slab is multiplied.  (The two launches' shrink is a kernel of its own, in sgmv.hip.)
 constexpr int kShrinkWaves = 4;
 
 // Body of the shrink for one tile.  MASKED: the adapter in the tile's slot has fewer ranks than
@@ -117,10 +113,10 @@ constexpr int kShrinkWaves = 4;
 //
 // SC1: the partial sums leave with agent-scope stores (they pass the compute unit's and the XCD's
 // caches on their way), for readers in other workgroups of the same launch.
-template <typename T, int R, int KR, int XW, bool DB, bool MASKED, bool SC1 = false>
+template <typename T, int R, int KR, bool MASKED, bool SC1 = false>
 __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __restrict__ xv, float* __restrict__ hws, int64_t xs, int T_, int K,
-                                            int num_slices, int krange, int all_slices, const ShrinkSlices& sl, int slice0, int kpart, int slot,
-                                            int start, int m, int eff, int row) {
+                                            int num_slices, int krange, const ShrinkSlices& sl, int slice, int kpart, int slot, int start, int m,
+                                            int eff, int row) {
   constexpr int RB = (R + 15) / 16;      // 16-rank blocks
   constexpr int NT = kShrinkWaves * kWave;
   constexpr int ASTRIDE = KR + 8;        // padded LDS row: 16 rows x 16 bytes cover all banks once
@@ -128,18 +124,14 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
   constexpr int TOTAL = R * CPR;         // chunks per slab
   constexpr int CHUNKS = (TOTAL + NT - 1) / NT;  // chunks each thread copies per slab
   constexpr int KS = KR / 32;            // k-steps per slab
-  constexpr int XK = XW / 32;            // k-steps per x batch
-  constexpr int SPB = XW / KR;           // slabs per x batch
-  static_assert(XW % KR == 0 && XK <= 16, "batch shape");
 
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int lr = lane & 15, lg = lane >> 4;
-  const int nsl = all_slices ? num_slices : 1;
   const int rb_n = MASKED ? (eff + 15) >> 4 : RB;          // 16-rank blocks of A[slot] in use
   const int rows_used = MASKED ? (rb_n * 16 < R ? rb_n * 16 : R) : R;
 
   const int k0 = kpart * krange;
-  const int nbatch = krange / XW;
+  const int nbatch = krange / KR;
   const bool active = wave * 16 < m;  // this wavefront's token block exists
   // `row`: token row of this lane, position wave * 16 + lane % 16 of the tile (positions past the
   // end of the tile name valid rows too: they feed the MFMA harmlessly and are never
@@ -170,15 +162,15 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
       if (TOTAL % NT == 0 || c < TOTAL) *reinterpret_cast<i32x4*>(&s_a[(c / CPR) * ASTRIDE + (c % CPR) * 8]) = v[i];
     }
   };
-  auto request_x = [&](Pack8(&buf)[XK], int kc) {
+  auto request_x = [&](Pack8(&buf)[KS], int kc) {
 #pragma unroll
-    for (int i = 0; i < XK; ++i) buf[i].raw = load128(xptr + kc + i * 32);
+    for (int i = 0; i < KS; ++i) buf[i].raw = load128(xptr + kc + i * 32);
   };
 
   // D layout: lane holds H[rank 16*rb + 4*(lane/16) + i][token lane%16]: four consecutive ranks
-  auto write_partials = [&](const f32x4(&part)[RB], int si) {
+  auto write_partials = [&](const f32x4(&part)[RB]) {
     if (active && ti < m) {
-      float* dst = hws + ((static_cast<int64_t>(kpart) * T_ + start + ti) * num_slices + slice0 + si) * R;
+      float* dst = hws + ((static_cast<int64_t>(kpart) * T_ + start + ti) * num_slices + slice) * R;
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int r0 = rb * 16 + 4 * lg;
@@ -197,201 +189,64 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
     }
   };
 
-  if constexpr (!DB && KR == XW && KR >= 256) {
-    // A batch that is one slab: slab and batch are requested in NS column pieces, piece after
-    // piece (A piece, then the x columns it meets), all of them up front; a piece is copied to LDS
-    // and multiplied as soon as it is there, while the later ones are still on their way.  A piece
-    // of the slab has its own place in LDS and NS - 1 barriers lie between two uses of a place, so
-    // one barrier per piece is enough; a piece's registers take the next slab's piece (next batch
-    // or next slice) as soon as they are stored.
-    constexpr int NS = MASKED ? 2 : 4, SW = KR / NS, SCPR = SW / 8, STOTAL = R * SCPR, SCH = (STOTAL + NT - 1) / NT, KSS = KS / NS;
-    static_assert(KS % NS == 0, "pieces of whole k-steps");
-    i32x4 v[NS][SCH];
-    Pack8 xa[XK];
-    f32x4 acc[RB];
-    auto request_piece = [&](const T* Aslab, int s, i32x4(&buf)[SCH]) {
-#pragma unroll
-      for (int i = 0; i < SCH; ++i) {
-        const int c = i * NT + tid;
-        if constexpr (MASKED) {
-          if (i * (NT / SCPR) >= rows_used) continue;  // rows beyond the adapter's rank (the same for every thread)
-        }
-        if (STOTAL % NT == 0 || c < STOTAL) buf[i] = load128(Aslab + static_cast<int64_t>(c / SCPR) * K + s * SW + (c % SCPR) * 8);
-      }
-    };
-    auto store_piece = [&](int s, const i32x4(&buf)[SCH]) {
-#pragma unroll
-      for (int i = 0; i < SCH; ++i) {
-        const int c = i * NT + tid;
-        if constexpr (MASKED) {
-          if (i * (NT / SCPR) >= rows_used) continue;
-        }
-        if (STOTAL % NT == 0 || c < STOTAL) *reinterpret_cast<i32x4*>(&s_a[(c / SCPR) * ASTRIDE + s * SW + (c % SCPR) * 8]) = buf[i];
-      }
-    };
-    auto request_x_piece = [&](int kc, int s) {
-#pragma unroll
-      for (int i = 0; i < KSS; ++i) xa[s * KSS + i].raw = load128(xptr + kc + (s * KSS + i) * 32);
-    };
-    {
-      const T* A0 = static_cast<const T*>(sl.a[slice0]) + aoff;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        // (piece by piece: with every A piece ahead of the x columns the prefill step takes 3816
-        // against 3753 us)
-        request_piece(A0, s, v[s]);
-        if (active) request_x_piece(0, s);
-      }
-    }
-    MLORA_STAMP(3);  // shrink: first slab and first x batch requested (the token rows are here)
-    for (int si = 0; si < nsl; ++si) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int b = 0; b < nbatch; ++b) {
-        // the slab after this one: next batch, or the first of the next slice
-        const T* An = nullptr;
-        if (b + 1 < nbatch) An = static_cast<const T*>(sl.a[slice0 + si]) + aoff + (b + 1) * XW;
-        else if (si + 1 < nsl) An = static_cast<const T*>(sl.a[slice0 + si + 1]) + aoff;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          store_piece(s, v[s]);
-          if (b == 0 && s == 0 && si == 0) MLORA_STAMP(4);  // shrink: first piece arrived and is on its way to LDS
-          if (An) request_piece(An, s, v[s]);
-          __syncthreads();
-          if (active) {
-#pragma unroll
-            for (int i = s * KSS; i < (s + 1) * KSS; ++i) {
-#pragma unroll
-              for (int rb = 0; rb < RB; ++rb) {
-                if constexpr (MASKED) {
-                  if (rb >= rb_n) continue;
-                }
-                const int rr = rb * 16 + lr;
-                Pack8 aw;
-                aw.raw = *reinterpret_cast<const i32x4*>(&s_a[(rr < R ? rr : R - 1) * ASTRIDE + i * 32 + lg * 8]);
-                acc[rb] = Mma<T>::run(aw, xa[i], acc[rb]);
-              }
-            }
-            if constexpr (MASKED) {
-              if (s == NS - 1) mfma_settle(acc);  // rank blocks were skipped by branches
-            }
-          }
-        }
-        if (active && b + 1 < nbatch) {
-#pragma unroll
-          for (int s = 0; s < NS; ++s) request_x_piece((b + 1) * XW, s);
-        }
-      }
-      if (si == 0) MLORA_STAMP(5);  // shrink: first slice multiplied
-      write_partials(acc, si);
-    }
-    return;
-  }
-
   // (Written once for wavefronts whose token block exists and once for those without one, which
   // only help with the slabs: a branch on `active` around the x requests keeps the compiler from
   // counting the loads in flight, and the wait for a slab then is a wait for the x batch requested
   // after it as well.)
   auto batches = [&](auto act_tag) {
   constexpr bool ACT = decltype(act_tag)::value;
-  Pack8 xa[XK], xb[DB ? XK : 1];
+  Pack8 xa[KS], xb[KS];
   f32x4 acc[RB];
-  bool first = true;
-  // One x batch: `cur` holds it (or is about to), `nxt` receives the following one meanwhile.
-  auto run_batch = [&](Pack8(&cur)[XK], Pack8(&nxt)[XK], int si, int b) {
-    const T* A = static_cast<const T*>(sl.a[slice0 + si]) + aoff;
-    if (DB && ACT && b + 1 < nbatch) request_x(nxt, (b + 1) * XW);
-#pragma unroll
-    for (int s = 0; s < SPB; ++s) {
-      if (!first) __syncthreads();  // everyone is done reading the previous slab
-      first = false;
-      store_slab();
-      if (b == 0 && s == 0 && si == 0) MLORA_STAMP(4);  // shrink: first slab arrived and is on its way to LDS
-      __syncthreads();
-      // the slab after this one: same batch, next batch, or the first of the next slice
-      if (s + 1 < SPB) request_slab(A + b * XW + (s + 1) * KR);
-      else if (b + 1 < nbatch) request_slab(A + (b + 1) * XW);
-      else if (si + 1 < nsl) request_slab(static_cast<const T*>(sl.a[slice0 + si + 1]) + aoff);
-      if (ACT) {
-#pragma unroll
-        for (int i = 0; i < KS; ++i) {
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) {
-            if constexpr (MASKED) {
-              if (rb >= rb_n) continue;
-            }
-            const int rr = rb * 16 + lr;
-            Pack8 aw;
-            aw.raw = *reinterpret_cast<const i32x4*>(&s_a[(rr < R ? rr : R - 1) * ASTRIDE + i * 32 + lg * 8]);
-            acc[rb] = Mma<T>::run(aw, cur[s * KS + i], acc[rb]);
-          }
-        }
-        if constexpr (MASKED) {
-          if (s == SPB - 1) mfma_settle(acc);  // rank blocks were skipped by branches
-        }
-      }
-    }
-    if (!DB && ACT && b + 1 < nbatch) request_x(cur, (b + 1) * XW);
-  };
-
-  request_slab(static_cast<const T*>(sl.a[slice0]) + aoff);
+  const T* A = static_cast<const T*>(sl.a[slice]) + aoff;
+  request_slab(A);
   if (ACT) request_x(xa, 0);
   MLORA_STAMP(3);  // shrink: first slab and first x batch requested (the token rows are here)
-  for (int si = 0; si < nsl; ++si) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (DB) {
-      // Two x buffers, one slab per batch.  A batch that has a successor (MORE) requests the
-      // successor's x batch, waits for its own slab alone, and requests the successor's slab
-      // after the barrier; the last batch of the K part is a copy of its own without those
-      // requests.  Written that way (instead of tests on b inside one body) every wait counts
-      // the requests younger than what it waits for: the x batch that was just requested stays
-      // in flight while the current one is multiplied.
-      auto batch = [&](auto more_tag, Pack8(&cur)[XK], Pack8(&nxt)[XK], int b) __attribute__((always_inline)) {
-        constexpr bool MORE = decltype(more_tag)::value;
-        static_assert(SPB == 1, "one slab per batch");
-        const T* A = static_cast<const T*>(sl.a[slice0 + si]) + aoff;
-        if (MORE && ACT) request_x(nxt, (b + 1) * XW);
-        __syncthreads();  // everyone is done reading the previous slab
-        store_slab();
-        if (b == 0 && si == 0) MLORA_STAMP(4);  // shrink: first slab arrived and is on its way to LDS
-        __syncthreads();
-        if constexpr (MORE) request_slab(A + (b + 1) * XW);
-        else if (si + 1 < nsl) request_slab(static_cast<const T*>(sl.a[slice0 + si + 1]) + aoff);
-        if (ACT) {
+  for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Two x buffers, one slab per batch.  A batch that has a successor (MORE) requests the
+  // successor's x batch, waits for its own slab alone, and requests the successor's slab
+  // after the barrier; the last batch of the K part is a copy of its own without those
+  // requests.  Written that way (instead of tests on b inside one body) every wait counts
+  // the requests younger than what it waits for: the x batch that was just requested stays
+  // in flight while the current one is multiplied.
+  auto batch = [&](auto more_tag, Pack8(&cur)[KS], Pack8(&nxt)[KS], int b) __attribute__((always_inline)) {
+    constexpr bool MORE = decltype(more_tag)::value;
+    if (MORE && ACT) request_x(nxt, (b + 1) * KR);
+    __syncthreads();  // everyone is done reading the previous slab
+    store_slab();
+    if (b == 0) MLORA_STAMP(4);  // shrink: first slab arrived and is on its way to LDS
+    __syncthreads();
+    if constexpr (MORE) request_slab(A + (b + 1) * KR);
+    if (ACT) {
 #pragma unroll
-          for (int i = 0; i < KS; ++i) {
+      for (int i = 0; i < KS; ++i) {
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-              if constexpr (MASKED) {
-                if (rb >= rb_n) continue;
-              }
-              const int rr = rb * 16 + lr;
-              Pack8 aw;
-              aw.raw = *reinterpret_cast<const i32x4*>(&s_a[(rr < R ? rr : R - 1) * ASTRIDE + i * 32 + lg * 8]);
-              acc[rb] = Mma<T>::run(aw, cur[i], acc[rb]);
-            }
+        for (int rb = 0; rb < RB; ++rb) {
+          if constexpr (MASKED) {
+            if (rb >= rb_n) continue;
           }
-          if constexpr (MASKED && !MORE) mfma_settle(acc);  // rank blocks were skipped by branches
+          const int rr = rb * 16 + lr;
+          Pack8 aw;
+          aw.raw = *reinterpret_cast<const i32x4*>(&s_a[(rr < R ? rr : R - 1) * ASTRIDE + i * 32 + lg * 8]);
+          acc[rb] = Mma<T>::run(aw, cur[i], acc[rb]);
         }
-      };
-      int b = 0;
-      for (; b + 2 < nbatch; b += 2) {
-        batch(std::true_type{}, xa, xb, b);
-        batch(std::true_type{}, xb, xa, b + 1);
       }
-      if (b + 1 < nbatch) {
-        batch(std::true_type{}, xa, xb, b);
-        batch(std::false_type{}, xb, xa, b + 1);
-      } else {
-        batch(std::false_type{}, xa, xb, b);
-      }
-    } else {
-      for (int b = 0; b < nbatch; ++b) run_batch(xa, xa, si, b);
+      if constexpr (MASKED && !MORE) mfma_settle(acc);  // rank blocks were skipped by branches
     }
-    if (si == 0) MLORA_STAMP(5);  // shrink: first slice multiplied
-    if (ACT) write_partials(acc, si);
+  };
+  int b = 0;
+  for (; b + 2 < nbatch; b += 2) {
+    batch(std::true_type{}, xa, xb, b);
+    batch(std::true_type{}, xb, xa, b + 1);
   }
+  if (b + 1 < nbatch) {
+    batch(std::true_type{}, xa, xb, b);
+    batch(std::false_type{}, xb, xa, b + 1);
+  } else {
+    batch(std::false_type{}, xa, xb, b);
+  }
+  MLORA_STAMP(5);  // shrink: multiplied
+  if (ACT) write_partials(acc);
   };
   if (active) batches(std::true_type{});
   else batches(std::false_type{});
@@ -773,13 +628,10 @@ size_t partials_room(const MloraAddArgs* a) {
 
 // Diagnostic knobs, read from the environment once and again after mlora_reload_knobs().
 struct SgmvKnobs {
-  int generation = -1, kr, ksplit, all_slices, xdb, group, wgs, nt, cpl, slab, stream;
+  int generation = -1, ksplit, group, wgs, nt, cpl, slab, stream;
   void read() {
     generation = knob_generation();
-    kr = env_int("MLORA_SGMV_KR", 0);
     ksplit = env_int("MLORA_SGMV_KSPLIT", 0);
-    all_slices = env_int("MLORA_SGMV_ALL_SLICES", 3);
-    xdb = env_int("MLORA_SGMV_XDB", 1);
     group = env_int("MLORA_SGMV_GROUP", 0);
     wgs = env_int("MLORA_SGMV_WGS", 2048);
     nt = env_int("MLORA_SGMV_NT", 0);
@@ -821,6 +673,14 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
   return static_cast<size_t>(num_tokens) * static_cast<size_t>(num_slices) * static_cast<size_t>(r) * sizeof(float);
 }
 
+// About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile (active: slots with tokens where the
+// host counted them, else 0).
+inline int big_tiles_about(const MloraAddArgs* a, int active) {
+  const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+  const int tiles = static_cast<int>((a->num_tokens + 31ll * segs) / MLORA_TILE_BIG);
+  return tiles > segs ? tiles : segs;
+}
+
 // How a call is cut into work, shared by the two-launch and the one-launch form.
 struct SgmvShape {
   bool empty;
@@ -828,8 +688,8 @@ struct SgmvShape {
   ShrinkSlices sl;
   int tiles8;     // tiles / 8: 64-token tiles of the long segments, then the short segments
   int big_cap;    // tiles below this index are 64-token tiles
-  int kr, xw;     // shrink: A slab width, x batch width
-  int ksplit, krange, all_slices;
+  int ksplit;     // shrink: K parts
+  int krange;     // of the one-launch form: columns of a part
   bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
   int group;      // expand: consecutive 64-token tiles per workgroup
   int cpl;        // expand: columns per lane
@@ -862,58 +722,33 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   s.empty = false;
   const int est_tiles = a->num_tokens / MLORA_TILE_BIG + 1;
 
-  // shrink: x batch width (what a wavefront holds in registers: 512 columns when K allows), A
-  // slab width (a whole batch: on the prefill and the mixed batch 128-, 256- and 512-column
-  // slabs measured within 2 % of each other), then K parts so that the grid has a few
-  // workgroups per compute unit
-  int xw = 512;
-  while (xw > 128 && a->k % xw != 0) xw /= 2;
-  int kr = sgmv_knobs().kr;
-  if (kr != 128 && kr != 256 && kr != 512) kr = xw;
-  if (kr > xw) kr = xw;
-  if (kr == 128) xw = 128;  // 128-column slabs come with 128-column batches only
+  // shrink: K parts so that the grid has a workgroup per compute unit and parts of at most 1024 columns, as far as multiples of 512 columns (256, 128 where K
+  // is no multiple) divide K; (gate_up of the prefill batch with one part 72.2 us per call against 73.3 with two, o with two 19.6
+  // against 22.4 with one, down with four 33.6 against 35.7 with two and 50.5 with one)
+  int unit = 512;
+  while (unit > 128 && a->k % unit != 0) unit /= 2;
   int max_parts = static_cast<int>(partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r));
   if (max_parts < 1) max_parts = 1;  // (wide.hip's cut needs no workspace; the others' launches have made sure of one)
   int ksplit = sgmv_knobs().ksplit;
   if (ksplit <= 0) {
     ksplit = 1;
-    // (a workgroup per compute unit, and K parts of at most 1024 columns: on the prefill batch
-    // gate_up with one part takes 72.2 us per call against 73.3 with two, o with two 19.6
-    // against 22.4 with one, down with four 33.6 against 35.7 with two and 50.5 with one)
-    while (ksplit < kMaxKSplit && a->k % (xw * ksplit * 2) == 0 &&
+    while (ksplit < kMaxKSplit && a->k % (unit * ksplit * 2) == 0 &&
            (static_cast<long long>(est_tiles) * a->num_slices * ksplit < 256 || a->k / ksplit > 1024))
       ksplit *= 2;
   }
   if (ksplit > max_parts) ksplit = max_parts;
   if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
-  while (ksplit > 1 && a->k % (xw * ksplit) != 0) --ksplit;
-  // three or more slices: one workgroup walks them all with the x rows it already holds, when
-  // its K part is a single batch (measured on the prefill batch: qkv 31.9 -> 29.6 us per call;
-  // with two slices the shorter chain of separate workgroups wins, gate_up 76.6 vs 77.8)
-  s.all_slices = 0;
-  if (a->num_slices >= sgmv_knobs().all_slices) {
-    const int parts = a->k / xw;
-    if (parts <= kMaxKSplit && parts <= max_parts) {
-      ksplit = parts;
-      s.all_slices = 1;
-    }
-  }
+  while (ksplit > 1 && a->k % (unit * ksplit) != 0) --ksplit;
   s.ksplit = ksplit;
   s.krange = a->k / ksplit;
-  // a K part of several batches: the form with two x buffers (256-column batches)
-  if (xw == 512 && s.krange > xw && sgmv_knobs().xdb) { xw = 256; kr = 256; }
-  s.kr = kr;
-  s.xw = xw;
-  // Which shrink.  Measured, us per call, this file's kernel / slab.hip's: rank 64, 9392 tokens (K = 1024): qkv
-  // 39.0 / 33.0, gate_up 85.4 / 84.7, o 25.0 / 24.6, down (K = 4096) 43.9 / 46.8; rank 64, 8192 mixed
-  // tokens: 41.8 / 39.6, 99.0 / 98.3, 24.7 / 23.5, 44.5 / 45.9; rank 64, 4000 tokens, K = 2048: qkv 35.0 / 28.4;
-  // rank 32, 5000 tokens: 19.3 / 18.5, 50.3 / 49.6, 13.6 / 13.5, 21.0 / 18.5; rank 32, 2000 tokens: 14.7 / 12.1,
-  // 21.3 / 19.3, 12.0 / 11.0, 14.3 / 13.4.  At rank 64 a workgroup of it holds 64 KB of LDS,
-  // and what is left of the last round of long parts costs about what the operands' path saves.
+  // Which shrink.  Up to rank 32 the one whose wavefronts have rings of their own (slab.hip): down, us per call, that / the shared ring of
+  // sgmv.hip, each in its best parts: rank 16, K = 8192, 3500 tokens 24.5 / 25.4, 7500 47.4 / 48.4, rank 32 25.8 / 27.3 and 51.6 / 52.2; K = 4096, rank 8, 6500 23.9 /
+  // 24.0, rank 32, 3500 17.9 / 17.0.  At rank 64 its stages are 16 KB a wavefront, of which one is on its way: 7000 tokens 30.2 / 29.4, K = 8192
+  // 54.6 / 52.1, gate_up 63.5 / 62.7, K = 2048 3500 tokens 72 / 67, three slices 2500 23.6 / 21.9.
   // (Whoever asks for the two-launch form by name gets the shrink whose sums the one-launch form repeats bit by bit:
   // slab.hip adds K up in another order.)
   s.slab = !one_launch && slab_supported(a) &&
-           (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && (a->r <= 32 || a->num_slices > 2)));
+           (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && a->r <= 32));
   // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
   // those, per slot): while an XCD's workgroups number no more than its 32 compute units (a second
   // round loses: 5200 tokens of 2 slots, K = 2560, two parts 29.8 us, three, 33 workgroups on some XCDs, 33.2) and it cuts K into more parts
@@ -953,7 +788,6 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
     // 37.4 / 35.0, of 12000 38.1 / 44.7 / 40.1 / 41.6 / 39.2; K = 8192, 5500 tokens 41.5 / 51.5 / 42.9 / 43.0 / 39.4, 7000 45.6 /
     // 55.4 / 49.7 / 47.2 / 45.2, 9392 61.4 / 67.5 / 70.2 / 58.8 / 60.5; rank 32 alike): four parts where one would be
     // taken from K = 4096 on, and from K = 8192 on throughout.
-    s.all_slices = 0;
     ksplit = sgmv_knobs().ksplit;
     if (ksplit <= 0 && round_parts > 0) {
       ksplit = round_parts;
@@ -964,10 +798,38 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
       if (ksplit < 1) ksplit = 1;
       if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
       while (ksplit > 1 && a->k / 64 < ksplit * kSlabStages) --ksplit;
+      // Unless other parts leave fewer columns to the compute unit with the most workgroups (below): rank 16, K = 8192, 4500 tokens 35.7 us in four
+      // parts (three rounds of a quarter where the last is nearly empty), 31.6 in three; 9000 59.8 / 56.5; K = 4096, 9000 34.0 / 33.1, 4000 18.0 / 17.4 in four.
+      if (a->num_slices == 1) {
+        const int tiles = big_tiles_about(a, active);
+        auto columns = [&](int p) { return (static_cast<long long>(tiles) * p + 255) / 256 * (a->k / p); };
+        for (int p = 1; p <= kMaxKSplit && a->k / 64 >= p * kSlabStages; ++p)
+          if (10 * columns(p) < 9 * columns(ksplit)) ksplit = p;
+      }
     }
     if (ksplit > max_parts) ksplit = max_parts;
     if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
     s.ksplit = ksplit;
+  }
+
+  if (!one_launch && !s.slab && sgmv_knobs().ksplit <= 0) {
+    // The ring's parts need not divide K evenly, and what counts is how many of its workgroups come to a compute unit: one, or two that
+    // run side by side for the price of both.  The cheapest of one to as many parts as above by workgroups per unit x columns of a
+    // part; a part also costs its sums, which every column range reads (`extra`, in columns; at equal cost the more parts up to K = 4096, the fewer beyond).
+    // us per call with one / two / three / four parts, rank 64: K = 4096, 4000 tokens of 3 slots 31.0 / 24.1 / 21.9 / 20.4, 5500 33.5 / 27.4 / 30.3 / 27.5, 7000
+    // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
+    // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
+    // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
+    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(a, active);
+    long long least = 0;
+    for (int p = 1; p <= ksplit; ++p) {
+      const long long wgs = static_cast<long long>(tiles) * a->num_slices * p;
+      const long long cost = (wgs + 255) / 256 * (a->k / p) + extra * p;
+      if (p == 1 || cost < least + (extra == 0)) {
+        least = cost;
+        s.ksplit = p;
+      }
+    }
   }
 
   // expand: consecutive tiles per workgroup (they share their B rows when they share their
@@ -991,8 +853,6 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   if (one_launch && a->k % 256 == 0) {
     // the unit's workgroups (one per column range) share out its shrink roles (tile, slice, K part):
     // about one role each
-    s.kr = s.xw = 256;
-    s.all_slices = 0;
     if (group * a->num_slices > s.nsplit) s.group = group = 1;  // every slice has a column range: one role each at least
     int parts = sgmv_knobs().ksplit;
     if (parts <= 0) {
