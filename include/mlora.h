@@ -129,6 +129,8 @@ int mlora_add_lora(const MloraAddArgs* args);
 /* The same with the number of slots that have tokens in this batch, where the host knows it (0: it does not);
  * only MLORA_FORM_AUTO's choice depends on it. */
 int mlora_add_lora_active(const MloraAddArgs* args, int32_t active_slots);
+/* The same with the number of tokens that have a slot as well (0: unknown): it moves AUTO's lines and how a launch is cut. */
+int mlora_add_lora_counts(const MloraAddArgs* args, int32_t active_slots, int32_t active_tokens);
 
 /* The same fused apply for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the

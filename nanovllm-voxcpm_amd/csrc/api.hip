@@ -273,16 +273,19 @@ static bool wide_instead(const MloraAddArgs* a, int active) {
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active);
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int active_tokens);
 
 }  // namespace
 
-extern "C" int mlora_add_lora(const MloraAddArgs* a) { return add_lora_impl(a, false, 0); }
-extern "C" int mlora_add_lora_active(const MloraAddArgs* a, int32_t active_slots) { return add_lora_impl(a, false, active_slots); }
+extern "C" int mlora_add_lora(const MloraAddArgs* a) { return add_lora_impl(a, false, 0, 0); }
+extern "C" int mlora_add_lora_active(const MloraAddArgs* a, int32_t active_slots) { return add_lora_impl(a, false, active_slots, 0); }
+extern "C" int mlora_add_lora_counts(const MloraAddArgs* a, int32_t active_slots, int32_t active_tokens) {
+  return add_lora_impl(a, false, active_slots, active_tokens);
+}
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int active_tokens) {
   if (!a) { set_error("mlora_add_lora: NULL args"); return MLORA_E_INVALID; }
   if (a->num_tokens < 0 || a->k < 0 || a->r < 0 || a->num_slots < 0 || a->num_slices < 0) {
     set_error("mlora_add_lora: negative size"); return MLORA_E_INVALID;
@@ -371,7 +374,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
                   "and no empty slice");
         return MLORA_E_UNSUPPORTED;
       }
-      return launch_wide(a);
+      return launch_wide(a, active, active_tokens);
     case MLORA_FORM_PAIR:
       if (!pair_supported(a)) {
         set_error("mlora_add_lora: the pair form needs a plan, a workspace, rows of x of a multiple of 128 bytes, B rows of 16 to 128 (fp32: 256) bytes "
@@ -417,7 +420,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active) {
         }
         return launch_fused(a, trusted_workspace);
       }
-      return launch_sgmv(a, active);
+      return launch_sgmv(a, active, active_tokens);
     }
   }
   set_error("mlora_add_lora: unreachable form %d", form);
@@ -485,7 +488,7 @@ extern "C" int mlora_add_lora_static(const MloraAddArgs* a) {
   b.workspace_bytes = MLORA_STATIC_SCRATCH_BYTES;
   // The array starts out zeroed (it is part of the loaded image) and only this library's kernels
   // ever write it, so its head is always either in the initial state or as a launch left it.
-  return add_lora_impl(&b, /*trusted_workspace=*/true, 0);
+  return add_lora_impl(&b, /*trusted_workspace=*/true, 0, 0);
 }
 
 extern "C" size_t mlora_add_workspace_bytes(int32_t num_tokens, int32_t num_slices, int32_t r, int32_t dtype) {

@@ -7,7 +7,7 @@
 // same reads and checks on the tensors' C++ objects.  It decides nothing by itself: it handles a
 // call only when everything the Python path would look up for it is what the Python path looked up
 // last time (the argument block of these weight buffers, the plan of this step's slot vector, the
-// scratch buffer of this stream), fills the per-step fields of the block and calls mlora_add_lora_active.
+// scratch buffer of this stream), fills the per-step fields of the block and calls mlora_add_lora_counts.
 // One lookup it makes itself: the first call of a step whose slot vector carries a plan (take_step below).
 // Everything else - a first call of these buffers, a step without a plan, a capture in progress, anything
 // that has to raise - is answered with "not handled", and the Python path runs as if this module did not
@@ -46,7 +46,7 @@ struct Site {
 };
 
 struct State {
-  int (*add_lora)(const MloraAddArgs*, int32_t) = nullptr;  // mlora_add_lora_active
+  int (*add_lora)(const MloraAddArgs*, int32_t, int32_t) = nullptr;  // mlora_add_lora_counts
   size_t (*workspace_bytes)(int32_t, int32_t, int32_t, int32_t) = nullptr;
   std::unordered_map<std::string, Site> sites;
   // what the last call of the Python path looked up for its step
@@ -54,7 +54,7 @@ struct State {
   const PyObject* source = nullptr;
   uint32_t version = 0;
   void* stream = nullptr;
-  int num_slots = 0, active_slots = 0;
+  int num_slots = 0, active_slots = 0, active_tokens = 0;
   int64_t rows = -1;
   const void* plan = nullptr;
   PyObject* held[3] = {};  // metadata, slot vector and plan of a step that was taken here (set_step's are its caller's to hold)
@@ -120,7 +120,7 @@ PyObject* py_create(PyObject*, PyObject* args) {
   unsigned long long add = 0, ws = 0;
   if (!PyArg_ParseTuple(args, "KK", &add, &ws)) return nullptr;
   State* s = new State();
-  s->add_lora = reinterpret_cast<int (*)(const MloraAddArgs*, int32_t)>(static_cast<uintptr_t>(add));
+  s->add_lora = reinterpret_cast<int (*)(const MloraAddArgs*, int32_t, int32_t)>(static_cast<uintptr_t>(add));
   s->workspace_bytes = reinterpret_cast<size_t (*)(int32_t, int32_t, int32_t, int32_t)>(static_cast<uintptr_t>(ws));
   return PyCapsule_New(s, kCapsule, destroy);
 }
@@ -181,22 +181,23 @@ PyObject* py_clear_sites(PyObject*, PyObject* cap) {
   Py_RETURN_NONE;
 }
 
-// set_step(state, metadata, source, version, stream, num_slots, rows, plan address, active slots): what a call
+// set_step(state, metadata, source, version, stream, num_slots, rows, plan address, tokens with a slot, active slots): what a call
 // outside any capture looked up; the caller keeps metadata, source and the plan alive for as long
 // as this stands.  forget_step(state) withdraws it.
 PyObject* py_set_step(PyObject*, PyObject* args) {
   PyObject *cap, *metadata, *source;
   unsigned long version = 0;
   unsigned long long stream = 0, plan = 0;
-  int num_slots = 0, active_slots = 0;
+  int num_slots = 0, active_tokens = 0, active_slots = 0;
   long long rows = 0;
-  if (!PyArg_ParseTuple(args, "OOOkKiLKi", &cap, &metadata, &source, &version, &stream, &num_slots, &rows, &plan, &active_slots)) return nullptr;
+  if (!PyArg_ParseTuple(args, "OOOkKiLKii", &cap, &metadata, &source, &version, &stream, &num_slots, &rows, &plan, &active_tokens, &active_slots)) return nullptr;
   State* s = state_of(cap);
   if (!s) return nullptr;
   const Released before(s);
   s->metadata = metadata; s->source = source; s->version = static_cast<uint32_t>(version);
   s->stream = reinterpret_cast<void*>(static_cast<uintptr_t>(stream));
   s->num_slots = num_slots; s->rows = rows; s->active_slots = active_slots < 0 ? 0 : active_slots;
+  s->active_tokens = active_tokens < 0 ? 0 : active_tokens;
   s->plan = reinterpret_cast<const void*>(static_cast<uintptr_t>(plan));
   Py_RETURN_NONE;
 }
@@ -242,6 +243,7 @@ bool take_step(State* s, const Site& site, PyObject* metadata, PyObject* source_
   static PyObject* const kCapacity = PyUnicode_InternFromString("_mlora_capacity");
   static PyObject* const kActiveIds = PyUnicode_InternFromString("active_slot_ids");
   static PyObject* const kActive = PyUnicode_InternFromString("num_active_loras");
+  static PyObject* const kSorted = PyUnicode_InternFromString("token_indices_sorted_by_slot");
   if (source.numel() != rows) return false;
   PyObject* made = given(source_obj, kPlan);  // (workspace, max_slots, version)
   if (!made || !PyTuple_Check(made) || PyTuple_GET_SIZE(made) != 3 || !THPVariable_Check(PyTuple_GET_ITEM(made, 0))) return false;
@@ -251,7 +253,7 @@ bool take_step(State* s, const Site& site, PyObject* metadata, PyObject* source_
   if (PyErr_Occurred() || slots != site.num_slots || at != version || !on_device(plan, site.device)) return false;
   const Ref plan_held{(Py_INCREF(made), made)};  // (the attribute reads below can run Python code)
   long active = 0;
-  const Ref ids{PyObject_GetAttr(metadata, kActiveIds)}, number{PyObject_GetAttr(metadata, kActive)};
+  const Ref ids{PyObject_GetAttr(metadata, kActiveIds)}, number{PyObject_GetAttr(metadata, kActive)}, sorted{PyObject_GetAttr(metadata, kSorted)};
   PyErr_Clear();
   PyObject* capacity = ids.p ? given(ids.p, kCapacity) : nullptr;
   if (number.p && !(capacity && PyObject_IsTrue(capacity) == 1)) active = PyLong_AsLong(number.p);
@@ -262,6 +264,8 @@ bool take_step(State* s, const Site& site, PyObject* metadata, PyObject* source_
   s->metadata = metadata; s->source = source_obj; s->version = version; s->stream = stream;
   s->num_slots = site.num_slots; s->rows = rows; s->plan = plan.data_ptr();
   s->active_slots = active > 0 && active <= site.num_slots ? static_cast<int>(active) : 0;
+  const int64_t tokens = s->active_slots && sorted.p && THPVariable_Check(sorted.p) ? THPVariable_Unpack(sorted.p).numel() : 0;
+  s->active_tokens = tokens <= rows ? static_cast<int>(tokens) : 0;
   return true;
 }
 
@@ -349,7 +353,7 @@ long call_at(State* s, const Site& site, PyObject* x_obj, PyObject* target_obj, 
   a->workspace = ws;
   a->workspace_bytes = ws_bytes;
   a->effective_rank = static_cast<const int32_t*>(eff_ptr);
-  return s->add_lora(a, plan ? s->active_slots : 0);
+  return s->add_lora(a, plan ? s->active_slots : 0, plan ? s->active_tokens : 0);
 }
 
 // A call with lists of slices.
@@ -798,10 +802,10 @@ PyMethodDef kMethods[] = {
     {"install_batch", py_install_batch, METH_NOARGS, "install_batch() -> an empty batch of slot installs"},
     {"install_add", method(py_install_add), METH_FASTCALL, "install_add(batch, A, Bs, lora_a, lora_b, slot, rank, scaling, packed, staged, ranks, scalings, base scalings) -> bool"},
     {"install_flush", py_install_flush, METH_VARARGS, "install_flush(batch, address of mlora_install_slots) -> 0 or a library error code"},
-    {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora_active, address of mlora_add_workspace_bytes) -> state"},
+    {"create", py_create, METH_VARARGS, "create(address of mlora_add_lora_counts, address of mlora_add_workspace_bytes) -> state"},
     {"register_site", py_register_site, METH_VARARGS, "register_site(state, a_list, b_list, widths, block address, block owner, vectorisable) -> bool"},
     {"clear_sites", py_clear_sites, METH_O, "clear_sites(state)"},
-    {"set_step", py_set_step, METH_VARARGS, "set_step(state, metadata, source, version, stream, num_slots, rows, plan address, active slots)"},
+    {"set_step", py_set_step, METH_VARARGS, "set_step(state, metadata, source, version, stream, num_slots, rows, plan address, tokens with a slot, active slots)"},
     {"forget_step", py_forget_step, METH_O, "forget_step(state)"},
     {"set_scratch", py_set_scratch, METH_VARARGS, "set_scratch(state, device index, stream, address, bytes)"},
     {"counters", py_counters, METH_O, "counters(state) -> (calls enqueued here, calls left to the Python path)"},

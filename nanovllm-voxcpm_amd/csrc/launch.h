@@ -52,7 +52,7 @@ int workspace_init(void* workspace, hipStream_t stream);
 bool sgmv_supported(const MloraAddArgs* a);
 bool sgmv_workspace_ok(const MloraAddArgs* a);
 size_t sgmv_workspace_bytes(int num_tokens, int num_slices, int r, int dtype);
-int launch_sgmv(const MloraAddArgs* a, int active);  // active: slots with tokens where the host counted them, else 0
+int launch_sgmv(const MloraAddArgs* a, int active, int active_tokens);  // slots with tokens and tokens with a slot where the host counted them, else 0
 
 // slab.hip: the shrink launch of that form, operands through LDS by direct loads.
 struct PlanLayout;
@@ -67,7 +67,7 @@ int launch_fused(const MloraAddArgs* a, bool trusted_workspace);
 // wide.hip: the same tiles, one launch, one workgroup per (tile, column range) doing both products.
 bool wide_supported(const MloraAddArgs* a);
 bool wide_pays(const MloraAddArgs* a);
-int launch_wide(const MloraAddArgs* a);
+int launch_wide(const MloraAddArgs* a, int active, int active_tokens);
 
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
 // direct loads; 16- and 32-bit elements.

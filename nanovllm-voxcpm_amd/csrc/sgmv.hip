@@ -353,8 +353,8 @@ bool sgmv_workspace_ok(const MloraAddArgs* a) {
 }
 
 // Every segment of the batch: 64-token tiles of the long ones, one short tile each for the rest.
-int launch_sgmv(const MloraAddArgs* a, int active) {
-  const SgmvShape sh = sgmv_shape(a, false, active);
+int launch_sgmv(const MloraAddArgs* a, int active, int active_tokens) {
+  const SgmvShape sh = sgmv_shape(a, false, active, active_tokens);
   if (sh.empty) return 0;
   if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.sl.a);
   else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink<__bf16>(a, sh);

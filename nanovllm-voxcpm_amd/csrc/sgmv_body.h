@@ -673,11 +673,13 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
   return static_cast<size_t>(num_tokens) * static_cast<size_t>(num_slices) * static_cast<size_t>(r) * sizeof(float);
 }
 
-// About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile (active: slots with tokens where the
-// host counted them, else 0).
-inline int big_tiles_about(const MloraAddArgs* a, int active) {
-  const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  const int tiles = static_cast<int>((a->num_tokens + 31ll * segs) / MLORA_TILE_BIG);
+// Tokens with a slot and slots with tokens: what the host counted (else 0), or at most.
+inline int tokens_with_slot(const MloraAddArgs* a, int active_tokens) { return active_tokens > 0 && active_tokens < a->num_tokens ? active_tokens : a->num_tokens; }
+inline int slots_with_tokens(const MloraAddArgs* a, int active) { return active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens; }
+// About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile.
+inline int big_tiles_about(const MloraAddArgs* a, int active, int active_tokens) {
+  const int segs = slots_with_tokens(a, active);
+  const int tiles = static_cast<int>((tokens_with_slot(a, active_tokens) + 31ll * segs) / MLORA_TILE_BIG);
   return tiles > segs ? tiles : segs;
 }
 
@@ -702,7 +704,7 @@ struct SgmvShape {
 
 // one_launch: the cut for the form whose workgroups do both products (256-column slabs and batches,
 // which leave the registers the kernel needs besides; as many shrink roles per unit as it has workgroups).
-inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int active = 0) {
+inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int active = 0, int active_tokens = 0) {
   SgmvShape s;
   s.empty = true;
   s.lay = plan_layout(a->num_tokens, a->num_slots);
@@ -801,7 +803,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
       // Unless other parts leave fewer columns to the compute unit with the most workgroups (below): rank 16, K = 8192, 4500 tokens 35.7 us in four
       // parts (three rounds of a quarter where the last is nearly empty), 31.6 in three; 9000 59.8 / 56.5; K = 4096, 9000 34.0 / 33.1, 4000 18.0 / 17.4 in four.
       if (a->num_slices == 1) {
-        const int tiles = big_tiles_about(a, active);
+        const int tiles = big_tiles_about(a, active, active_tokens);
         auto columns = [&](int p) { return (static_cast<long long>(tiles) * p + 255) / 256 * (a->k / p); };
         for (int p = 1; p <= kMaxKSplit && a->k / 64 >= p * kSlabStages; ++p)
           if (10 * columns(p) < 9 * columns(ksplit)) ksplit = p;
@@ -820,7 +822,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
     // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
     // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
     // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
-    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(a, active);
+    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(a, active, active_tokens);
     long long least = 0;
     for (int p = 1; p <= ksplit; ++p) {
       const long long wgs = static_cast<long long>(tiles) * a->num_slices * p;

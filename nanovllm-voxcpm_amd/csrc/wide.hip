@@ -435,7 +435,7 @@ struct WideKnobs {
   int generation = -1, nt;
   void read() {
     generation = knob_generation();
-    nt = env_int("MLORA_WIDE_NT", 0);  // columns per range (0: 512)
+    nt = env_int("MLORA_WIDE_NT", 0);  // columns per range (0: wide_columns)
   }
 };
 const WideKnobs& wide_knobs() {
@@ -452,6 +452,36 @@ void wide_trace_set(void* buf) {
 #else
   (void)buf;
 #endif
+}
+
+// Columns of a range.  Wider ranges repeat less of a tile's shrink, narrower ones are more workgroups.  Segments of 128 tokens and more are whole
+// tiles: the width (512, 1024, 2048) whose fullest compute unit has the fewest columns of K and of ranges to stream, two workgroups side by
+// side counted as one after the other.  us per call with 512 / 1024 columns, rank 64, K = 1024, 3 slots: q|k|v 6000 tokens 22.3 / 24.9, 9000
+// 34.8 / 26.7, o 13.6 / 17.3 and 22.9 / 18.9; rank 32, 9000 29.7 / 23.0 and 20.0 / 16.5; rank 64, K = 2048, q|k|v 2500 23.9 / 23.1, 4000 30.9 /
+// 25.0, 6000 48.5 / 41.4, o 4000 20.0 / 22.9, 6000 31.9 / 24.2.  Shorter ones are mostly single tiles of a few blocks, which end at
+// different times and fill in behind each other: 1024 once the narrow ranges fill the chip twice over (rank 64, K = 1024, 128 slots, 8192
+// tokens: q|k|v 34.5 / 29.8 with 756 workgroups of 512 columns, 5000 tokens 28.7 / 24.3 with 552, o 19.5 / 24.4 with 378).
+static int wide_columns(const MloraAddArgs* a, int active, int active_tokens) {
+  const long long segs = slots_with_tokens(a, active), n = tokens_with_slot(a, active_tokens);
+  const bool short_segments = n < 128 * segs;
+  const long long tiles = short_segments ? (n + 31 * segs) / MLORA_TILE_BIG : n / MLORA_TILE_BIG + segs / 2;
+  int best = 512;
+  long long least = 0;
+  for (int nt = 512; nt <= 2048; nt *= 2) {
+    long long ranges = 0, widest = 0;
+    for (int i = 0; i < a->num_slices; ++i) {
+      const int n_i = a->slices[i].n;
+      ranges += (n_i + nt - 1) / nt;
+      if ((n_i < nt ? n_i : nt) > widest) widest = n_i < nt ? n_i : nt;
+    }
+    if (short_segments) return tiles * ranges > 512 ? 1024 : 512;
+    const long long cost = (tiles * ranges + 255) / 256 * (a->k + widest);
+    if (nt == 512 || cost < least) {
+      least = cost;
+      best = nt;
+    }
+  }
+  return best;
 }
 
 // Whether this form beats the two-launch one.  What it saves is a launch with its latency from
@@ -474,17 +504,13 @@ bool wide_supported(const MloraAddArgs* a) {
   return true;
 }
 
-int launch_wide(const MloraAddArgs* a) {
+int launch_wide(const MloraAddArgs* a, int active, int active_tokens) {
   const SgmvShape sh = sgmv_shape(a);
   if (sh.empty) return 0;
   WideLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.big_cap = sh.big_cap;
-  // Column ranges of 512 columns (a span of 128 per wavefront).  Measured on the prefill batch (7608
-  // tokens with adapter, rank 64; us per call at 512 / 1024 / 4096 columns): qkv 24.8 / 27.6 / 27.9,
-  // o 17.2 / 21.2 / 21.4 (wider ranges leave compute units without a workgroup), gate_up 92.0 / 75.7 /
-  // 68.2, down 38.8 / 43.5 / 43.6 (where the two-launch form is taken instead, wide_pays()).
   int nt = wide_knobs().nt;
-  if (nt <= 0) nt = 512;
+  if (nt <= 0) nt = wide_columns(a, active, active_tokens);
   const int nsplit = fill_splits(a, nt, l.splits.split);
   l.grid = dim3(8, static_cast<unsigned>(nsplit), static_cast<unsigned>(sh.tiles8));
   if (a->dtype == MLORA_DTYPE_BF16) launch_wide_rank<__bf16>(l);

@@ -56,6 +56,7 @@ _DTYPES = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: D
 EXPORTS = (
     "mlora_add_lora",
     "mlora_add_lora_active",
+    "mlora_add_lora_counts",
     "mlora_add_lora_static",
     "mlora_add_workspace_bytes",
     "mlora_workspace_init",
@@ -234,6 +235,8 @@ def load() -> C.CDLL:
         fn.restype = C.c_int
     lib.mlora_add_lora_active.argtypes = [C.POINTER(MloraAddArgs), C.c_int32]
     lib.mlora_add_lora_active.restype = C.c_int
+    lib.mlora_add_lora_counts.argtypes = [C.POINTER(MloraAddArgs), C.c_int32, C.c_int32]
+    lib.mlora_add_lora_counts.restype = C.c_int
     lib.mlora_meta_build_many.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32]
     lib.mlora_meta_build_many.restype = C.c_int
     lib.mlora_meta_build_runs.argtypes = [C.POINTER(MloraMetaArgs), C.c_int32, C.c_void_p, C.c_void_p, C.c_int32]
@@ -329,12 +332,12 @@ def load_fastcall():
 
 
 def entry_point_addresses() -> tuple[int, int] | None:
-    """Addresses of mlora_add_lora_active and mlora_add_workspace_bytes in the loaded library, None without it."""
+    """Addresses of mlora_add_lora_counts and mlora_add_workspace_bytes in the loaded library, None without it."""
     try:
         load()
     except RuntimeError:
         return None
-    return entry_point("mlora_add_lora_active"), entry_point("mlora_add_workspace_bytes")
+    return entry_point("mlora_add_lora_counts"), entry_point("mlora_add_workspace_bytes")
 
 
 _ADDRESSES: dict[str, int] = {}
@@ -452,6 +455,7 @@ def add_lora(
     static_scratch: bool = False,
     effective_rank: torch.Tensor | None = None,
     active_slots: int = 0,
+    active_tokens: int = 0,
 ) -> None:
     """y[:, col_i : col_i + n_i] += scaling * (x . A_i[slot]^T) . B_i[slot]^T for every slice.
     ``stream``: handle of the stream to launch on, torch's current one when omitted.
@@ -459,7 +463,8 @@ def add_lora(
     library's own device image (``workspace`` is ignored then).
     ``effective_rank``: int32 [slots] on the device, rank of the adapter resident in each slot of
     these buffers; rows / columns at or above it are then neither read nor multiplied.
-    ``active_slots``: how many slots have tokens in this batch, where known."""
+    ``active_slots``, ``active_tokens``: how many slots have tokens in this batch and how many
+    tokens a slot, where known."""
     lib = load()
     if len(a_slices) > MAX_SLICES:
         raise ValueError(f"at most {MAX_SLICES} slices per call, got {len(a_slices)}")
@@ -523,12 +528,13 @@ def add_lora(
         if static_scratch:
             _check(lib.mlora_add_lora_static(C.byref(args)), "mlora_add_lora_static")
         else:
-            _check(lib.mlora_add_lora_active(C.byref(args), active_slots), "mlora_add_lora")
+            _check(lib.mlora_add_lora_counts(C.byref(args), active_slots, active_tokens), "mlora_add_lora")
 
 
 def call_add_lora(args: MloraAddArgs, active_slots: int) -> None:
-    """Enqueue the fused apply described by an argument block the caller filled and checked."""
-    rc = load().mlora_add_lora_active(C.byref(args), active_slots)
+    """Enqueue the fused apply described by an argument block the caller filled and checked, and whose
+    ``active_tokens`` (no field of the C struct) it set where it knows them."""
+    rc = load().mlora_add_lora_counts(C.byref(args), active_slots, getattr(args, "active_tokens", 0))
     if rc != 0:
         _check(rc, "mlora_add_lora")
 

@@ -23,7 +23,7 @@ from typing import Protocol
 import torch
 
 from nanovllm_voxcpm_amd import _hip
-from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, attached_plan, build_segment_plan, known_active_slots
+from nanovllm_voxcpm_amd.lora_ops.segment_meta import SegmentPlan, as_slot_vector, attached_plan, build_segment_plan, known_active_slots, known_active_tokens
 
 
 @dataclass(frozen=True)
@@ -429,6 +429,7 @@ class HipLoRABackend:
                         self._fastcall.forget_step(fast)
                     else:  # (the tuple above keeps metadata, slot vector and plan alive for as long as this stands)
                         self._fastcall.set_step(fast, metadata, source, version, stream or 0, site.num_slots, rows, plan_ptr,
+                                                known_active_tokens(metadata, site.num_slots, rows, capture),
                                                 known_active_slots(metadata, site.num_slots, capture))
             scratch = self._scratch_for(x, site.num_slices, site.rank, stream, capture)
             ws_ptr, ws_bytes = scratch.data_ptr(), scratch.numel()
@@ -441,6 +442,7 @@ class HipLoRABackend:
         _STEP_HEAD.pack_into(site.view, 0, stream or 0, x_ptr, y_ptr, xs, ys, source.data_ptr(), plan_ptr, rows)
         _STEP_SCALE.pack_into(site.view, _OFF_SCALING, scaling)
         _STEP_TAIL.pack_into(site.view, _OFF_WORKSPACE, ws_ptr, ws_bytes, eff_ptr)
+        args.active_tokens = known_active_tokens(metadata, site.num_slots, rows, capture)
         _hip.call_add_lora(args, known_active_slots(metadata, site.num_slots, capture))
         return True
 
@@ -556,7 +558,8 @@ class HipLoRABackend:
                     plan = self._plan_for(metadata, tts, a_list[0].size(0), capture).workspace
                     scratch = self._scratch_for(x2, len(chunk), a_list[0].size(-2), stream, capture)
                 _hip.add_lora(target, x2, a_list, b_list, c_list, tts, plan, float(scaling), form, scratch, stream,
-                              effective_rank=effective_rank, active_slots=known_active_slots(metadata, a_list[0].size(0), capture))
+                              effective_rank=effective_rank, active_slots=known_active_slots(metadata, a_list[0].size(0), capture),
+                              active_tokens=known_active_tokens(metadata, a_list[0].size(0), x2.size(0), capture))
         if staged is not None:
             staged.copy_(target)
         return outputs

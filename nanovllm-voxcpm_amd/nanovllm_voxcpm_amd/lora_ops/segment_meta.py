@@ -98,6 +98,15 @@ def known_active_slots(metadata, num_slots: int, capture: int | None) -> int:
     return active if 0 < active <= num_slots else 0
 
 
+def known_active_tokens(metadata, num_slots: int, rows: int, capture: int | None) -> int:
+    """How many tokens of a batch of ``rows`` have a slot, 0 where nobody knows: as many as a context lists by slot,
+    where its counts are the batch's own (`known_active_slots`)."""
+    listed = getattr(metadata, "token_indices_sorted_by_slot", None)
+    if not isinstance(listed, torch.Tensor) or not known_active_slots(metadata, num_slots, capture):
+        return 0
+    return listed.numel() if listed.numel() <= rows else 0
+
+
 @dataclass
 class LoRAKernelMeta:
     """Preallocated index buffers in the layout of the reference's grouped kernels.
