@@ -224,7 +224,7 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
 //  - one workgroup per (tile, column range): from rank x K = 131072 on (1234 tokens, rank 32, K = 4096: 19.1 /
 //    13.9; it loses below: rank 16, K = 4096, 2000 tokens 11.5 / 12.5, and ties at rank 32, K = 2048), and for
 //    buffers of a rank between the instances', whose code is the general one away from K = 1024 (64 tokens, rank 48, K = 2048:
-//    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9) and which have no form over 64-token tiles (6000
+//    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9) and which had no form over 64-token tiles (6000
 //    tokens, rank 48: 40.5 / 32.7, 24.3 / 22.6, 115 / 74, 50 / 35; at 1500 tokens and rank 24 qkv and o are
 //    still the faster ones in one launch: 12.7 / 13.3, 8.1 / 11.2);
 //  - 64-token tiles, where A is as large and the outputs are not wide (rank 64, K = 2048 -> 16384: 32.2 / 33.2 at 1000
@@ -236,11 +236,17 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
 //    23.7 / 28.5; rank 32, K = 4096 16.0 / 15.3, 16.7 / 18.8.  Two slices, rank 32, K = 4096, 900 and 1300 tokens of 4
 //    slots (58 and 83 tiles): 12.6 / 11.6, 13.0 / 15.5; three, rank 64, K = 2048, 500 and 700 (33 and 46): 14.6 / 12.5,
 //    14.7 / 16.7.  (Below the line batches of 16 to 32 slots and more than about 40 tokens in each lose up to a quarter: rank
-//    64, K = 4096, 32 slots: 14.6 / 16.2 at 700 tokens, 19.2 / 20.1 at 1600.)
+//    64, K = 4096, 32 slots: 14.6 / 16.2 at 700 tokens, 19.2 / 20.1 at 1600.)  Between the
+//    instances' ranks, which had no 64-token tiles before, from rank x K = 98304 on: rank 24, K = 4096, 1564 tokens of 3 slots 12.8 / 10.8, 1500 of 16 13.1 / 14.2, and with up to 26 tokens to a slot
+//    (rank 24 and up to 2000 tokens: 34) and 20 MB of weights: half of the tokens in two prompts and the others over 128 slots, two launches over 64-token tiles / pair, gate_up and down of 2500
+//    tokens, rank 24 40.4 / 35.1, 18.0 / 15.1, rank 48 50.5 / 45.8, 20.8 / 17.9, of 3600, rank 24 47.7 / 46.3, 20.3 / 18.7, rank 48 58.0 / 59.9, 22.9 / 21.6.
 static bool pair_pays(const MloraAddArgs* a, int form, int active) {
   const long long rk = static_cast<long long>(a->r) * a->k;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_tokens < (a->r <= 24 || a->num_tokens <= 2000 ? 34ll : 26ll) * slots_with_tokens(a, active) &&
+      2.0 * slots_with_tokens(a, active) * a->r * (static_cast<double>(a->num_slices) * a->k + cols) >= 2.0e7)
+    return true;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
     case MLORA_FORM_MFMA: {
@@ -252,7 +258,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active) {
     }
     case MLORA_FORM_SGMV:
     case MLORA_FORM_WIDE:
-      return rk >= 131072 && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active)) * a->num_slices <= 128;
+      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active)) * a->num_slices <= 128;
     default: return false;
   }
 }
@@ -262,13 +268,14 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active) {
 // units of an XCD, they run in two rounds, each of which shrinks its tile anew.  16-token / 64-token tiles, us per call, q|k|v
 // at workgroups per XCD: K = 1024, rank 64: 11.7 / 13.7 at 32, 16.6 / 13.8 at 36, 17.5 / 12.8 at 44, 17.7 / 13.6 at 48; rank
 // 32: 7.5 / 9.3 at 32, 10.4 / 10.9 at 36, 10.9 / 9.1 at 44; K = 768, rank 64: 10.7 / 12.6 at 32, 17.3 / 12.5 at 36; rank 32: 7.0 /
-// 8.7 and 10.9 / 9.9; K = 512, rank 64: 7.7 / 9.7 and 11.8 / 10.8.  With a smaller A the rounds are too short to matter (K = 512,
+// 8.7 and 10.9 / 9.9; K = 512, rank 64: 7.7 / 9.7 and 11.8 / 10.8; between these ranks the 16-token tiles fit two to a compute unit: K = 1024, rank 24 8.1 / 10.8 at
+// 36, 12.5 / 10.8 at 48, rank 48 11.4 / 14.6 and 18.0 / 14.6.  With a smaller A the rounds are too short to matter (K = 512,
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
 // of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
 static bool wide_instead(const MloraAddArgs* a, int active) {
   if (a->num_slices < 3 || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a)) return false;
   int columns;
-  return (small_tiles_about(a, active) + 7) / 8 * decode_ranges(a, &columns) > 32;
+  return (small_tiles_about(a, active) + 7) / 8 * decode_ranges(a, &columns) > (exact_rank(a->r) ? 32 : 40);
 }
 
 namespace {

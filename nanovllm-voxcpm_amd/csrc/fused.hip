@@ -75,10 +75,10 @@ __device__ __forceinline__ void fused_expand(T* s_h, int* s_row, int* s_slot, in
   }
   __syncthreads();  // expand_body rewrites the arrays read above
   if (masked)
-    expand_body<T, R, CPL, TPF, G, true, true>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, true, true>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, R, num_slices, ksplit, scaling, sp, slot, start,
                                                m, eff, rowv);
   else
-    expand_body<T, R, CPL, TPF, G, false, true>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, false, true>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, R, num_slices, ksplit, scaling, sp, slot, start,
                                                 m, eff, rowv);
 }
 
@@ -324,7 +324,7 @@ void fused_trace_set(void* buf) {
 }
 
 bool fused_supported(const MloraAddArgs* a) {
-  if (!sgmv_supported(a) || !sgmv_workspace_ok(a) || a->k % 256 != 0) return false;
+  if (!exact_rank(a->r) || !sgmv_supported(a) || !sgmv_workspace_ok(a) || a->k % 256 != 0) return false;
   if (a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return false;
   return shape_fits(a, sgmv_shape(a, true));
 }

@@ -15,6 +15,11 @@ int env_int(const char* name, int fallback);
 // rank; the other forms take exact ranks only.
 inline bool exact_rank(int r) { return r == 8 || r == 16 || r == 32 || r == 64; }
 inline bool padded_rank(int r) { return r >= 8 && r <= 64 && r % 8 == 0; }
+// Tokens with a slot and slots with tokens: what the host counted (else 0), or at most.
+inline int tokens_with_slot(const MloraAddArgs* a, int active_tokens) { return active_tokens > 0 && active_tokens < a->num_tokens ? active_tokens : a->num_tokens; }
+inline int slots_with_tokens(const MloraAddArgs* a, int active) { return active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens; }
+// The 64-token tiles serve buffers of every padded rank; by name only those of the instances' own, as ever.
+inline bool tiles64_rank(const MloraAddArgs* a) { return a->form == MLORA_FORM_AUTO ? padded_rank(a->r) : exact_rank(a->r); }
 inline int compute_rank(int r) { return r <= 8 ? 8 : r <= 16 ? 16 : r <= 32 ? 32 : 64; }
 // Diagnostic knobs are read from the environment once and kept; mlora_reload_knobs() advances
 // this number, and a holder whose copy is older reads its variables again.

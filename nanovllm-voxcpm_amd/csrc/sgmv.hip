@@ -74,7 +74,10 @@ __device__ __forceinline__ void ring_tile(char* lds, const char* abase, uint32_t
   const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;  // chunk p of a row goes to place p ^ (row & 7)
   uint32_t aoff[NA];
 #pragma unroll
-  for (int g = 0; g < NA; ++g) aoff[g] = static_cast<uint32_t>((a0 + 4 * g) * 8 + (lane >> 3)) * arow + swz;
+  for (int g = 0; g < NA; ++g) {
+    const int rank = (a0 + 4 * g) * 8 + (lane >> 3);  // (buffers of a rank in between: the last row again, whose sums are not stored)
+    aoff[g] = static_cast<uint32_t>(rank < r_all ? rank : r_all - 1) * arow + swz;
+  }
   const uint32_t to0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
   auto issue = [&](int s, int stage) {
 #pragma unroll
@@ -208,7 +211,7 @@ __global__ __launch_bounds__(kRingThreads, 2) void sgmv_shrink_kernel(const int3
 template <typename T, int R, int CPL, int TPF, int G, bool STREAM>
 __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(const int32_t* __restrict__ plan, const float* __restrict__ hws,
                                                                              void* __restrict__ yv_, int64_t ys, int big_off, int small_off,
-                                                                             int big_units, int bigrows_off, int T_, int num_slots,
+                                                                             int big_units, int bigrows_off, int T_, int num_slots, int r,
                                                                              int num_slices, int ksplit, float scaling,
                                                                              const int32_t* __restrict__ eff_rank, ExpandSplits splits) {
   constexpr int HSTRIDE = 2 * R + 8;     // padded LDS row: R leading parts, R remainders
@@ -261,10 +264,10 @@ __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(con
   int eff[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    eff[g] = R;
+    eff[g] = r;
     if (eff_rank && m[g] > 0) {
       const int e = eff_rank[slot[g]];
-      eff[g] = e < 0 ? 0 : e > R ? R : e;
+      eff[g] = e < 0 ? 0 : e > r ? r : e;
       if (eff[g] == 0) m[g] = 0;  // nothing resident: the tile is skipped
     }
     any |= m[g];
@@ -282,10 +285,10 @@ __global__ __launch_bounds__(kExpandWaves* kWave, 2) void sgmv_expand_kernel(con
 #pragma unroll
   for (int g = 0; g < G; ++g) masked |= m[g] > 0 && eff[g] < R;
   if (masked)
-    expand_body<T, R, CPL, TPF, G, true, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, true, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, r, num_slices, ksplit, scaling, sp, slot, start,
                                          m, eff, rowv);
   else
-    expand_body<T, R, CPL, TPF, G, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, num_slices, ksplit, scaling, sp, slot, start,
+    expand_body<T, R, CPL, TPF, G, false, false, STREAM>(s_h, s_row, s_slot, s_m, s_eff, plan, hws, yv_, ys, T_, r, num_slices, ksplit, scaling, sp, slot, start,
                                           m, eff, rowv);
 }
 
@@ -303,7 +306,7 @@ void launch_expand_group(const MloraAddArgs* a, const PlanLayout& lay, int big_u
   const float* h = partials_of(a);
 #define MLORA_EXPAND(CPL_, TPF_, G_, S_)                                                                                       \
   hipLaunchKernelGGL((sgmv_expand_kernel<T, R, CPL_, TPF_, G_, S_>), grid, dim3(kExpandWaves* kWave), 0, st, a->plan, h, a->y, \
-                     a->y_stride, lay.big_off, lay.small_off, big_units, lay.bigrows_off, a->num_tokens, a->num_slots,      \
+                     a->y_stride, lay.big_off, lay.small_off, big_units, lay.bigrows_off, a->num_tokens, a->num_slots, a->r, \
                      a->num_slices, ksplit, a->scaling, a->effective_rank, sp)
   if (cpl == 4) {
     if (group == 4) MLORA_EXPAND(4, 4, 4, false); else if (group == 2) MLORA_EXPAND(4, 4, 2, false); else MLORA_EXPAND(4, 4, 1, false);
@@ -318,7 +321,7 @@ void launch_expand_group(const MloraAddArgs* a, const PlanLayout& lay, int big_u
 template <typename T>
 void launch_expand_rank(const MloraAddArgs* a, const PlanLayout& lay, int big_units, dim3 grid, int ksplit, int cpl, int group,
                         bool stream, const ExpandSplits& sp) {
-  switch (a->r) {
+  switch (compute_rank(a->r)) {
     case 8: launch_expand_group<T, 8>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
     case 16: launch_expand_group<T, 16>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
     case 32: launch_expand_group<T, 32>(a, lay, big_units, grid, ksplit, cpl, group, stream, sp); break;
@@ -342,7 +345,7 @@ void sgmv_trace_set(void* buf) {
 #endif
 }
 
-bool sgmv_supported(const MloraAddArgs* a) { return a->k % 128 == 0 && a->k >= 128 && exact_rank(a->r); }
+bool sgmv_supported(const MloraAddArgs* a) { return a->k % 128 == 0 && a->k >= 128 && tiles64_rank(a); }
 
 // A workspace that holds at least one partial can be used (fewer K parts are taken then).
 bool sgmv_workspace_ok(const MloraAddArgs* a) {

@@ -298,7 +298,7 @@ __device__ __forceinline__ void store_y(T* p, const YVec<T, N>& v) {
 }
 
 // Body of the expand for the tiles of one workgroup.  MASKED: some tile's slot holds an adapter of
-// fewer ranks than the buffers: chunks of the intermediate the shrink did not write are not read,
+// fewer ranks than the kernel's R, which the buffers' `rank` may be too: chunks of the intermediate the shrink did not write are not read,
 // ranks at or above the adapter's are zero in the intermediate, B columns from that rank on are
 // not fetched (zeros take their place in the operand).  The unmasked instance is the code without
 // any of those tests.
@@ -308,7 +308,7 @@ __device__ __forceinline__ void store_y(T* p, const YVec<T, N>& v) {
 template <typename T, int R, int CPL, int TPF, int G, bool MASKED, bool SC1 = false, bool STREAM = false>
 __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict__ s_row, int* __restrict__ s_slot, int* __restrict__ s_m,
                                             int* __restrict__ s_eff, const int32_t* __restrict__ plan, const float* __restrict__ hws,
-                                            void* __restrict__ yv_, int64_t ys, int T_, int num_slices, int ksplit,
+                                            void* __restrict__ yv_, int64_t ys, int T_, int rank, int num_slices, int ksplit,
                                             float scaling, const ExpandSplit& sp, const int (&slot)[G], const int (&start)[G],
                                             const int (&m)[G], const int (&eff)[G], const int (&rowv)[G]) {
   constexpr int TB = MLORA_TILE_BIG / 16;
@@ -327,18 +327,19 @@ __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict
   // The partial sums of a tile's intermediate: requested (every K part together), then summed,
   // scaled, split and written to LDS.  The first tile's are requested before anything else: they
   // depend on the tile record alone, and are on their way while the token rows make theirs.
-  const int64_t hrow = static_cast<int64_t>(num_slices) * R;
+  const int r = MASKED ? rank : R;  // of the buffers
+  const int64_t hrow = static_cast<int64_t>(num_slices) * r;
   const int64_t part = static_cast<int64_t>(T_) * hrow;
   f32x4 t[HC][kMaxKSplit][2];
   auto request_h = [&](int g) {
-    const float* src = hws + static_cast<int64_t>(start[g]) * hrow + sp.slice * R;
+    const float* src = hws + static_cast<int64_t>(start[g]) * hrow + sp.slice * r;
 #pragma unroll
     for (int h = 0; h < HC; ++h) {
       const int c = h * NT + tid;
       int tok = c / CPR;
       tok = tok < m[g] ? tok : m[g] - 1;
       const float* q = src + tok * hrow + (c % CPR) * 8;
-      const bool used = !MASKED || (c % CPR) * 8 < ((eff[g] + 15) & ~15);  // the shrink wrote this chunk
+      const bool used = !MASKED || (c % CPR) * 8 < eff[g];  // the shrink wrote this chunk
 #pragma unroll
       for (int kp = 0; kp < kMaxKSplit; ++kp) {
         if (kp < ksplit) {
@@ -422,7 +423,7 @@ __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict
   auto load_b = [&](int c0, int sg, int eg) {
     // the B rows of the span (lanes whose chunk lies beyond the rank fetch a valid chunk anyway,
     // their H operand is zero; columns past the range repeat the last one and are never stored)
-    const T* B = static_cast<const T*>(sp.b) + static_cast<int64_t>(sg) * sp.n * R;
+    const T* B = static_cast<const T*>(sp.b) + static_cast<int64_t>(sg) * sp.n * r;
     if (!MASKED || eg >= R) {
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
@@ -446,7 +447,7 @@ __device__ __forceinline__ void expand_body(T* __restrict__ s_h, int* __restrict
         for (int ks = 0; ks < KSTEPS; ++ks) {
           const int kc = lg + 4 * ks;
           if (kc < eg8) {
-            bop[j][ks].raw = load128(B + static_cast<int64_t>(n) * R + kc * 8);
+            bop[j][ks].raw = load128(B + static_cast<int64_t>(n) * r + kc * 8);
             if (eg & 7) mask_ranks(bop[j][ks], kc * 8, eg);
           } else {
             bop[j][ks].raw = i32x4{0, 0, 0, 0};
@@ -673,9 +674,6 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
   return static_cast<size_t>(num_tokens) * static_cast<size_t>(num_slices) * static_cast<size_t>(r) * sizeof(float);
 }
 
-// Tokens with a slot and slots with tokens: what the host counted (else 0), or at most.
-inline int tokens_with_slot(const MloraAddArgs* a, int active_tokens) { return active_tokens > 0 && active_tokens < a->num_tokens ? active_tokens : a->num_tokens; }
-inline int slots_with_tokens(const MloraAddArgs* a, int active) { return active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens; }
 // About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile.
 inline int big_tiles_about(const MloraAddArgs* a, int active, int active_tokens) {
   const int segs = slots_with_tokens(a, active);
@@ -749,7 +747,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   // 54.6 / 52.1, gate_up 63.5 / 62.7, K = 2048 3500 tokens 72 / 67, three slices 2500 23.6 / 21.9.
   // (Whoever asks for the two-launch form by name gets the shrink whose sums the one-launch form repeats bit by bit:
   // slab.hip adds K up in another order.)
-  s.slab = !one_launch && slab_supported(a) &&
+  s.slab = !one_launch && exact_rank(a->r) && slab_supported(a) &&
            (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && a->r <= 32));
   // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
   // those, per slot): while an XCD's workgroups number no more than its 32 compute units (a second

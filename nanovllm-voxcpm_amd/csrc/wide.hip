@@ -44,7 +44,7 @@ constexpr int kRing = kMostLds / 2;
 // 32 q|k|v of 1234 tokens 12.9 -> 16.3, mixed 34.7 -> 36.7.
 constexpr int kStage = 24;
 
-// C: 16-byte pieces of a B row (buffers' rank / 8); NA8: groups of eight ranks of the adapter; TB: blocks of sixteen tokens
+// C: 16-byte pieces of a B row in LDS (the buffers' rank / 8, or the next power of two); NA8: groups of eight ranks of the adapter, likewise; TB: blocks of sixteen tokens
 template <int C, int NA8, int TB> struct WideShape {
   static constexpr int RB = (NA8 + 1) / 2;
   static constexpr int PIECE = NA8 + 2 * TB;                  // direct loads of 128 bytes of K
@@ -67,23 +67,28 @@ template <int C, int NA8, int TB> struct WideShape {
 
 template <int C, int NA8, int TB>
 __device__ __forceinline__ void wide_ask(char* lds, const char* abase, uint32_t arow, const char* const (&xrow)[8], int chunks, const char* bbase,
-                                         const char* const (&yrow)[8], int ncols, int spans, int eff) {
+                                         const char* const (&yrow)[8], int ncols, int spans, int eff, int R) {
   typedef WideShape<C, NA8, TB> F;
   constexpr int NST = F::NST;
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t swz = static_cast<uint32_t>((lane & 7) ^ (lane >> 3)) * 16;
   uint32_t aoff[NA8];
 #pragma unroll
-  for (int g = 0; g < NA8; ++g) aoff[g] = static_cast<uint32_t>(g * 8 + (lane >> 3)) * arow + swz;
-  uint32_t bpiece[C];
+  for (int g = 0; g < NA8; ++g) {
+    const int rank = g * 8 + (lane >> 3);  // (buffers of a rank in between: the last row again, whose products are not used)
+    aoff[g] = static_cast<uint32_t>(rank < R ? rank : R - 1) * arow + swz;
+  }
+  const uint32_t brow = static_cast<uint32_t>(R) * 2;
+  uint32_t boff[C], bwant = 0;  // where a lane's pieces of a span come from, and which of them the adapter has
 #pragma unroll
   for (int i = 0; i < C; ++i) {
-    const uint32_t u = i * 64 + lane;
-    bpiece[i] = u ^ ((u >> F::SH) & 7);
+    const uint32_t u = i * 64 + lane, piece = u ^ ((u >> F::SH) & 7), c = piece % C;
+    boff[i] = piece / C * brow + (c * 16 < brow ? c * 16 : brow - 16);  // (beyond the rank: the last piece again, and masked)
+    bwant |= static_cast<uint32_t>(static_cast<int>(c) * 8 < eff) << i;
   }
   const uint32_t to0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
-  const uint32_t lasty = static_cast<uint32_t>(ncols) * 2 - 16, lastb = static_cast<uint32_t>(ncols) * C - 1;
-  const int eff8 = (eff + 7) >> 3, n = (chunks + F::P - 1) / F::P;
+  const uint32_t lasty = static_cast<uint32_t>(ncols) * 2 - 16, lastb = static_cast<uint32_t>(ncols) * brow - 16;
+  const int n = (chunks + F::P - 1) / F::P;
   // Stages are asked for in order; the pointers walk along (an address computed from a stage's number would be kept in registers of its own).
   const char *xp[2 * TB], *yp[2 * TB], *ap = abase, *bp = bbase;
 #pragma unroll
@@ -115,7 +120,7 @@ __device__ __forceinline__ void wide_ask(char* lds, const char* abase, uint32_t 
 #pragma unroll
         for (int i = 0; i < C; ++i) {
           // (piece 0 of a row is always fetched, so every one of these requests is made by some lane and counts)
-          if (NA8 >= C || static_cast<int>(bpiece[i] % C) < eff8) dma16(bp, (bpiece[i] < left ? bpiece[i] : left) * 16, at + (2 * TB + i) * 1024);
+          if (NA8 >= C || (bwant >> i & 1)) dma16(bp, boff[i] < left ? boff[i] : left, at + (2 * TB + i) * 1024);
         }
         const bool more = ++span < spans;
         uint32_t next = static_cast<uint32_t>(span) * 128 + swz;
@@ -127,8 +132,8 @@ __device__ __forceinline__ void wide_ask(char* lds, const char* abase, uint32_t 
           yp[g] += next - yoff;
         }
         yoff = next;
-        bp += more ? 64 * C * 16 : 0;
-        left -= more ? 64 * C : 0;
+        bp += more ? 64 * brow : 0;
+        left -= more ? 64 * brow : 0;
       }
     }
   };
@@ -334,10 +339,9 @@ __device__ __forceinline__ void wide_work(char* lds, int wave, int chunks, int s
 template <typename T, int C>
 __global__ __launch_bounds__(kWideThreads, 4) void wide_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv, void* __restrict__ yv_,
                                                                int64_t xs, int64_t ys, int big_off, int small_off, int big_cap, int bigrows_off,
-                                                               int T_, int K, int num_slots, float scaling, const int32_t* __restrict__ eff_rank,
+                                                               int T_, int K, int R, int num_slots, float scaling, const int32_t* __restrict__ eff_rank,
                                                                ShrinkSlices sl, ExpandSplits splits) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  constexpr int R = C * 8;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const bool asks = wave == kWorkers;
   const int tile = tile_position(big_cap);
@@ -388,7 +392,7 @@ __global__ __launch_bounds__(kWideThreads, 4) void wide_kernel(const int32_t* __
     const char* abase = uniform(static_cast<const char*>(sl.a[sp.slice]) + static_cast<int64_t>(slot) * R * arow);
     const char* bbase = uniform(static_cast<const char*>(sp.b) + (static_cast<int64_t>(slot) * sp.n + sp.n0) * (R * sizeof(T)));
     by_tile([&](auto na8, auto tb) __attribute__((always_inline)) {
-      wide_ask<C, decltype(na8)::value, decltype(tb)::value>(lds, abase, arow, xrow, chunks, bbase, yrow, ncols, spans, eff);
+      wide_ask<C, decltype(na8)::value, decltype(tb)::value>(lds, abase, arow, xrow, chunks, bbase, yrow, ncols, spans, eff, R);
     });
   } else {
     // (the rows of the tokens it stores: a wavefront's block of tokens follows from the tile's count, and they are wanted at the end only)
@@ -416,13 +420,13 @@ void launch_wide_one(const WideLaunch& l) {
   const MloraAddArgs* a = l.a;
   allow_lds<wide_kernel<T, C>>(kRing);
   hipLaunchKernelGGL((wide_kernel<T, C>), l.grid, dim3(kWideThreads), kRing, static_cast<hipStream_t>(a->stream), a->plan, a->x, a->y, a->x_stride,
-                     a->y_stride, l.lay.big_off, l.lay.small_off, l.big_cap, l.lay.bigrows_off, a->num_tokens, a->k, a->num_slots, a->scaling,
+                     a->y_stride, l.lay.big_off, l.lay.small_off, l.big_cap, l.lay.bigrows_off, a->num_tokens, a->k, a->r, a->num_slots, a->scaling,
                      a->effective_rank, l.sl, l.splits);
 }
 
 template <typename T>
 void launch_wide_rank(const WideLaunch& l) {
-  switch (l.a->r) {
+  switch (compute_rank(l.a->r)) {
     case 8: launch_wide_one<T, 1>(l); break;
     case 16: launch_wide_one<T, 2>(l); break;
     case 32: launch_wide_one<T, 4>(l); break;
@@ -498,7 +502,7 @@ bool wide_pays(const MloraAddArgs* a) {
 }
 
 bool wide_supported(const MloraAddArgs* a) {
-  if (!(a->k % 128 == 0 && a->k >= 128 && exact_rank(a->r))) return false;
+  if (!(a->k % 128 == 0 && a->k >= 128 && tiles64_rank(a))) return false;
   for (int i = 0; i < a->num_slices; ++i)
     if (a->slices[i].n <= 0) return false;
   return true;
