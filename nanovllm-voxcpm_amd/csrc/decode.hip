@@ -309,7 +309,10 @@ const DecodeKnobs& decode_knobs() {
 // columns for narrow projections and stay at 1024 (two 64-column spans per wavefront, all loads still
 // in registers) for wide ones.  Measured per launch at 32 tiles: o 6.2 us at 1024 columns, 5.1 at 512,
 // 4.7 at 256; gate_up 8.2 / 8.9 / 11.1.
-int decode_ranges(const MloraAddArgs* a, int* columns) {
+// Above rank 16 a workgroup has its compute unit to itself, 32 on an XCD, and what does not fit runs in a second round that shrinks its tile
+// anew: one slice whose ranges spill takes as many fewer as fit (o, K = 1024, 2000 / 2400 / 2800 tokens of 32 slots, in ranges of 832, 960 and 1024 columns: rank 64 11.5 / 18.3 /
+// 13.2, rank 24 8.3 / 12.2 / 8.8; 2400 tokens in one range 12.2 and 8.3).
+int decode_ranges(const MloraAddArgs* a, int active, int* columns) {
   int nt = decode_knobs().nt;
   if (nt <= 0) {
     long long cols = 0;
@@ -320,6 +323,10 @@ int decode_ranges(const MloraAddArgs* a, int* columns) {
     nt = static_cast<int>(cols * tiles / 160);
     if (nt > 1024) nt = 1024;
     if (nt < 128) nt = 128;
+    if (a->num_slices == 1 && a->r > 16) {
+      const int n = a->slices[0].n, fit = 32 / ((small_tiles_about(a, active) + 7) / 8);
+      if ((n + nt - 1) / nt > fit && fit > 0 && (n + fit - 1) / fit <= 1024) nt = (n + fit - 1) / fit;
+    }
   }
   if (nt < 64) nt = 64;
   nt = (nt + 63) & ~63;
@@ -369,7 +376,7 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active) {
   const int with_tokens = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
 
   int nt;
-  const int total = decode_ranges(a, &nt);
+  const int total = decode_ranges(a, active, &nt);
   if (total == 0) return 0;
   int s = 0;
   l.widest = 0;

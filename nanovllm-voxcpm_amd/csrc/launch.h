@@ -36,7 +36,7 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 // (tile, column range).
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
 int launch_decode(const MloraAddArgs* a, bool include_long, int active);  // active: slots with tokens where the host counted them, else 0
-int decode_ranges(const MloraAddArgs* a, int* columns);  // column ranges of that launch, and columns per range
+int decode_ranges(const MloraAddArgs* a, int active, int* columns);  // column ranges of that launch, and columns per range
 
 // slot.hip: the same small tiles, the grid laid over the slots: weights are requested from the
 // workgroup index alone, before the slot's record has arrived.
@@ -71,7 +71,7 @@ int launch_fused(const MloraAddArgs* a, bool trusted_workspace);
 
 // wide.hip: the same tiles, one launch, one workgroup per (tile, column range) doing both products.
 bool wide_supported(const MloraAddArgs* a);
-bool wide_pays(const MloraAddArgs* a);
+bool wide_pays(const MloraAddArgs* a, int active, int active_tokens);
 int launch_wide(const MloraAddArgs* a, int active, int active_tokens);
 
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by

@@ -439,7 +439,7 @@ struct WideKnobs {
   int generation = -1, nt;
   void read() {
     generation = knob_generation();
-    nt = env_int("MLORA_WIDE_NT", 0);  // columns per range (0: wide_columns)
+    nt = env_int("MLORA_WIDE_NT", 0);  // columns per range (0: wide_cut)
   }
 };
 const WideKnobs& wide_knobs() {
@@ -465,40 +465,59 @@ void wide_trace_set(void* buf) {
 // 25.0, 6000 48.5 / 41.4, o 4000 20.0 / 22.9, 6000 31.9 / 24.2.  Shorter ones are mostly single tiles of a few blocks, which end at
 // different times and fill in behind each other: 1024 once the narrow ranges fill the chip twice over (rank 64, K = 1024, 128 slots, 8192
 // tokens: q|k|v 34.5 / 29.8 with 756 workgroups of 512 columns, 5000 tokens 28.7 / 24.3 with 552, o 19.5 / 24.4 with 378).
-static int wide_columns(const MloraAddArgs* a, int active, int active_tokens) {
+struct WideCut {
+  int columns;
+  long long workgroups;
+  bool short_segments;
+};
+static WideCut wide_cut(const MloraAddArgs* a, int active, int active_tokens) {
   const long long segs = slots_with_tokens(a, active), n = tokens_with_slot(a, active_tokens);
   const bool short_segments = n < 128 * segs;
   const long long tiles = short_segments ? (n + 31 * segs) / MLORA_TILE_BIG : n / MLORA_TILE_BIG + segs / 2;
+  auto ranges = [&](int columns) {
+    long long all = 0;
+    for (int i = 0; i < a->num_slices; ++i) all += (a->slices[i].n + columns - 1) / columns;
+    return all;
+  };
   int best = 512;
-  long long least = 0;
-  for (int nt = 512; nt <= 2048; nt *= 2) {
-    long long ranges = 0, widest = 0;
-    for (int i = 0; i < a->num_slices; ++i) {
-      const int n_i = a->slices[i].n;
-      ranges += (n_i + nt - 1) / nt;
-      if ((n_i < nt ? n_i : nt) > widest) widest = n_i < nt ? n_i : nt;
-    }
-    if (short_segments) return tiles * ranges > 512 ? 1024 : 512;
-    const long long cost = (tiles * ranges + 255) / 256 * (a->k + widest);
-    if (nt == 512 || cost < least) {
-      least = cost;
-      best = nt;
+  if (short_segments) {
+    if (tiles * ranges(512) > 512) best = 1024;
+  } else {
+    long long least = 0;
+    for (int columns = 512; columns <= 2048; columns *= 2) {
+      long long widest = 0;
+      for (int i = 0; i < a->num_slices; ++i) {
+        const int n_i = a->slices[i].n < columns ? a->slices[i].n : columns;
+        if (n_i > widest) widest = n_i;
+      }
+      const long long cost = (tiles * ranges(columns) + 255) / 256 * (a->k + widest);
+      if (columns == 512 || cost < least) {
+        least = cost;
+        best = columns;
+      }
     }
   }
-  return best;
+  return {best, tiles * ranges(best), short_segments};
 }
 
 // Whether this form beats the two-launch one.  What it saves is a launch with its latency from
 // launch to first byte, and the partial sums' trip through the workspace; what it adds is the
-// intake of x and A rows by every column range of a tile beyond the first of its slice.  Measured
-// on the prefill and the mixed batch (us per call, this form / two launches): qkv (K = 1024, ranges
-// beyond the slices' first: 1) 24.8 / 28.6 and 35.9 / 41.6; o (K = 1024, 1) 17.2 / 18.0 and 19.9 /
-// 23.0; gate_up (K = 1024, 14) 92.0 / 67.6; down (K = 4096, 1) 38.8 / 31.1: taken while the repeats
-// are at most 1024 columns of K per tile.
-bool wide_pays(const MloraAddArgs* a) {
+// intake of x and A rows by every column range of a tile beyond the first of its slice.  us per call, this form / two launches, K = 1024
+// (ranges of 512 columns beyond the slices' first: 1), rank 64: q|k|v of 2500, 5000, 7500 tokens of 3 slots 13.8 / 15.7, 18.6 / 21.4, 23.6 / 29.1, of 16 slots 13.6 /
+// 15.9, 20.7 / 21.1, 24.8 / 29.4, o 13.5 / 14.0, 13.6 / 14.4, 13.9 / 15.7; gate_up of the prefill (14) 69.7 / 54.0 at rank 48: taken while the repeats
+// are at most 1024 columns of K per tile.  K = 2048 (3 repeats), above rank 16, segments of 128 tokens and more: only where the workgroups
+// fill their rounds of 256, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 / 38.9);
+// q|k|v of 252 25.2 / 30.3 (r 24 22.1 / 25.5), of 436 to 500 37.4 / 39.0, 42.6 / 47.5, 44.6 / 49.8, but of 210 33.9 / 30.9, of 344 42.0 / 33.1, of 404 43.9 / 42.6.
+// K = 4096: never by more than 5 %, and 31.5 / 30.5 at 7500 tokens.
+bool wide_pays(const MloraAddArgs* a, int active, int active_tokens) {
   long long repeats = 0;
   for (int i = 0; i < a->num_slices; ++i) repeats += (a->slices[i].n + 511) / 512 - 1;
-  return repeats * a->k <= 1024;
+  if (repeats * a->k <= 1024) return true;
+  if (a->k != 2048 || repeats > 3 || a->r <= 16) return false;
+  const WideCut cut = wide_cut(a, active, active_tokens);
+  if (cut.short_segments) return false;
+  const long long w = cut.workgroups;
+  return (cut.columns == 1024 && w <= 256 && w >= (a->num_slices == 1 ? 156 : 244)) || (a->num_slices > 1 && w > 420 && w <= 512);
 }
 
 bool wide_supported(const MloraAddArgs* a) {
@@ -514,7 +533,7 @@ int launch_wide(const MloraAddArgs* a, int active, int active_tokens) {
   WideLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.big_cap = sh.big_cap;
   int nt = wide_knobs().nt;
-  if (nt <= 0) nt = wide_columns(a, active, active_tokens);
+  if (nt <= 0) nt = wide_cut(a, active, active_tokens).columns;
   const int nsplit = fill_splits(a, nt, l.splits.split);
   l.grid = dim3(8, static_cast<unsigned>(nsplit), static_cast<unsigned>(sh.tiles8));
   if (a->dtype == MLORA_DTYPE_BF16) launch_wide_rank<__bf16>(l);
