@@ -143,10 +143,10 @@ static bool short_segments(const MloraAddArgs* a, int active) {
 // 11.1 / 10.5, 6500 17.4 / 13.2; rank 24 12.4 / 11.0 at 6500): 0.36 times.  And at K = 2048, where the two launches' shrink has become faster, above
 // rank 16: us per call over small tiles (one or two launches) / in two over 64-token tiles, o of 1500, 2500 tokens of 3 slots, rank 24 11.8 / 11.5, 14.4 / 12.2, rank 32 8.7 /
 // 11.8, 14.8 / 12.3, of 16 slots 13.5 / 11.8, 16.0 / 12.3 and 10.2 / 11.9, 16.5 / 12.3; rank 48, 1000 and 1500 of 16 13.0 / 14.2, 16.4 / 14.3, rank 64, 1500
-// 18.6 / 14.3; q|k|v, 1000 and 1500 of 16, rank 24 14.8 / 12.6, 19.0 / 13.3, rank 32, 1500 18.2 / 13.4.  Segments of fewer than 16 tokens are what
+// 18.6 / 14.3; q|k|v, 1000 and 1500 of 16, rank 24 14.8 / 12.6, 19.0 / 13.3, rank 32, 740 (of 986, the others without an adapter: tokens with a slot are what counts) 8.1 / 11.3, 1500 18.2 / 13.4.  Segments of fewer than 16 tokens are what
 // the small tiles are for (1000 tokens of 64 slots, rank 32, q|k|v 13.3 / 19.2): these lines are not drawn for them.
 // MLORA_SMALL_BATCH_TOKENS, when set, replaces the rule by a plain token count.
-static bool small_batch(const MloraAddArgs* a, bool one_launch, int active) {
+static bool small_batch(const MloraAddArgs* a, bool one_launch, int active, int active_tokens) {
   const int fixed = knobs().small_batch_tokens;
   if (fixed > 0) return a->num_tokens <= fixed;
   double cols = 0;
@@ -155,15 +155,15 @@ static bool small_batch(const MloraAddArgs* a, bool one_launch, int active) {
   double limit = (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) * (one_launch ? 0.65 : 1.0);
   if (a->r > 16 && !short_segments(a, active)) {
     if (one_launch && a->r <= 32) limit = 0.36 * 2.6e7;
-    else if (!one_launch && a->k == 2048 && cols <= 2.0 * a->k && (a->r <= 32 || a->num_slices == 1)) limit = a->r <= 32 ? 1.3e7 : 7.7e6;
+    else if (!one_launch && a->k == 2048 && cols <= 2.0 * a->k && (a->r <= 32 || a->num_slices == 1)) limit = a->r > 32 ? 7.7e6 : a->num_slices > 1 && exact_rank(a->r) ? 1.7e7 : 1.3e7;
   }
-  return a->num_tokens * width <= limit;
+  return tokens_with_slot(a, active_tokens) * width <= limit;
 }
 
 // About how many 16-token tiles a batch has: its segments end anywhere inside their last tile.
-int mlora::small_tiles_about(const MloraAddArgs* a, int active) {
+int mlora::small_tiles_about(const MloraAddArgs* a, int active, int active_tokens) {
   const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  const int tiles = static_cast<int>((a->num_tokens + 7ll * segs) / MLORA_TILE_SMALL);
+  const int tiles = static_cast<int>((tokens_with_slot(a, active_tokens) + 7ll * segs) / MLORA_TILE_SMALL);
   return tiles > segs ? tiles : segs;
 }
 
@@ -253,25 +253,30 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
 //    14.7 / 16.7.  (Below the line batches of 16 to 32 slots and more than about 40 tokens in each lose up to a quarter: rank
 //    64, K = 4096, 32 slots: 14.6 / 16.2 at 700 tokens, 19.2 / 20.1 at 1600; so one slice above rank 16 and segments counted at 16 to 127 tokens stop at 96 tiles: 1500 tokens of 16 and 64 slots, 100
 //    and 121 tiles, 64-token tiles / pair: rank 64, K = 4096 16.1 / 20.1, 19.5 / 25.3, rank 32 13.3 / 15.1, 13.1 / 17.9; K = 2048, rank 64
-//    14.3 / 18.6, 16.4 / 22.9; 1000 of 16, 69 tiles, rank 48, K = 4096 16.1 / 13.4, but rank 16, K = 8192, 1500 of 8 15.3 / 13.6.  Between the
+//    14.3 / 18.6, 16.4 / 22.9; but 1602 of 16 slots, half of them in one, rank 24 12.5 / 10.9, rank 16, K = 8192, 1500 of 8 15.3 / 13.6.  Between the
 //    instances' ranks, which had no 64-token tiles before, from rank x K = 98304 on: rank 24, K = 4096, 1564  of 3 12.8 / 10.8, 1500 of 16 13.1 / 14.2, and with up to 26 tokens to a slot
 //    (rank 24 and up to 2000 tokens: 34) and 20 MB of weights: half of the tokens in two prompts and the others over 128 slots, two launches over 64-token tiles / pair, gate_up and down of 2500
-//    tokens, rank 24 40.4 / 35.1, 18.0 / 15.1, rank 48 50.5 / 45.8, 20.8 / 17.9, of 3600, rank 24 47.7 / 46.3, 20.3 / 18.7, rank 48 58.0 / 59.9, 22.9 / 21.6);
+//    tokens, rank 24 40.4 / 35.1, 18.0 / 15.1, rank 48 50.5 / 45.8, 20.8 / 17.9, of 3600, rank 24 47.7 / 46.3, 20.3 / 18.7, rank 48 58.0 / 59.9, 22.9 / 21.6;
+//    two slices of K = 2048, up to 1100 tokens in segments of 64 and more: gate_up, rank 24, 520 tokens of 8 of 64 slots 21.5 / 17.4, 820 of 9 21.4 / 18.3, 1000 of 3 27.3 / 24.0, rank 48
+//    32.5 / 30.7, 600 17.2 / 18.3; beyond, 1500 32.3 / 33.5 and 37.3 / 41.4, shorter, 1000 of 16 25.3 / 27.0 and 29.0 / 35.4);
 //  - segments of fewer than 16 tokens with many weights (the slots' A and B in all), each of which passes once through either
 //    form: 64-token tiles where they are 40 MB, one launch over small tiles where they are 60 MB and the outputs wide.  us per call without / with,
 //    128 slots: gate_up, K = 1024, rank 64, 600, 1000, 1500 tokens 43.9 / 36.5, 47.2 / 38.1, 50.8 / 40.6, rank 32 27.7 / 23.6, 29.3 / 24.6, 36.2 / 26.6, rank 16 (42 MB) 16.8 /
 //    17.5, 18.6 / 18.7, 21.5 / 20.9; K = 2048, rank 64 84.6 / 65.9, 94.2 / 83.0, rank 16 32.7 / 28.2, 51.2 / 39.6; down of 1500, K = 4096, rank 64 27.9 / 22.9, rank 32 20.7 / 16.2, K =
 //    8192, rank 64 54.5 / 40.1; q|k|v, K = 2048, rank 64, 1000 42.1 / 36.6, but rank 32 22.5 / 23.5.  64 slots: gate_up, 600, K = 1024, rank 64 26.2 / 24.2, rank 32 (42
 //    MB) 16.6 / 16.9, rank 48 23.8 / 21.0, rank 24 (31 MB) 15.0 / 15.5; K = 2048, rank 64 49.8 / 39.4, rank 32 33.4 / 25.7.
-static bool pair_pays(const MloraAddArgs* a, int form, int active) {
+static bool pair_pays(const MloraAddArgs* a, int form, int active, int active_tokens) {
   const long long rk = static_cast<long long>(a->r) * a->k;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  const bool few_tokens = short_segments(a, active), middling = !few_tokens && active > 0 && a->r > 16 && a->num_tokens < 128ll * active;
+  const bool few_tokens = short_segments(a, active), middling = !few_tokens && active > 0 && a->r > 16 && exact_rank(a->r) && a->num_tokens < 128ll * active;
   const double weights = 2.0 * slots_with_tokens(a, active) * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
   if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_tokens < (a->r <= 24 || a->num_tokens <= 2000 ? 34ll : 26ll) * slots_with_tokens(a, active) && weights >= 2.0e7) return true;
   if (few_tokens && ((form == MLORA_FORM_SGMV && weights >= 4.0e7) ||
                      (form == MLORA_FORM_MFMA && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k)))
+    return true;
+  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_slices == 2 && a->k == 2048 && a->num_tokens <= 1100 &&
+      a->num_tokens >= 64ll * slots_with_tokens(a, active))
     return true;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
@@ -284,7 +289,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active) {
     }
     case MLORA_FORM_SGMV:
     case MLORA_FORM_WIDE:
-      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
+      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active, active_tokens)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
     default: return false;
   }
 }
@@ -300,10 +305,10 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active) {
 // / 12.2, 15.1 / 14.1, 23.3 / 16.2.  With a smaller A the rounds are too short to matter (K = 512,
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
 // of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
-static bool wide_instead(const MloraAddArgs* a, int active) {
-  if (a->num_slices == 2 || (a->num_slices == 1 && a->r <= 16) || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, active, 0)) return false;
+static bool wide_instead(const MloraAddArgs* a, int active, int active_tokens) {
+  if (a->num_slices == 2 || (a->num_slices == 1 && a->r <= 16) || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, active, active_tokens)) return false;
   int columns;
-  return (small_tiles_about(a, active) + 7) / 8 * decode_ranges(a, active, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
+  return (small_tiles_about(a, active, active_tokens) + 7) / 8 * decode_ranges(a, active, active_tokens, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
 }
 
 namespace {
@@ -369,8 +374,8 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
     // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches; rank 24, 36 / 16 / 39 / 104 and 9.5 / 9.2 / 10.7 /
     // 10.9, rank 56, 81 / 80 / 90 / 243 and 12.6 / 12.1 / 14.3 / 15.5, one token of rank 24 15.3 / 15.4 / 15.8 / 43 and 8.5 / 8.5 / 9.2 / 9.9)
     if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
-    else if (one_launch && !(small_tiles && small_batch(a, true, active))) form = MLORA_FORM_WIDE;
-    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, active))) form = MLORA_FORM_SGMV;
+    else if (one_launch && !(small_tiles && small_batch(a, true, active, active_tokens))) form = MLORA_FORM_WIDE;
+    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, active, active_tokens))) form = MLORA_FORM_SGMV;
     else if (small_tiles) form = MLORA_FORM_SPLIT;
     else form = MLORA_FORM_BGMV;
   }
@@ -386,10 +391,10 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
       knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, active))
     form = MLORA_FORM_SLOT;
-  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, active))
+  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, active, active_tokens))
     form = MLORA_FORM_PAIR;
   if (form == MLORA_FORM_MFMA && a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_wide && knobs().small_batch_tokens <= 0 &&
-      wide_instead(a, active))
+      wide_instead(a, active, active_tokens))
     form = MLORA_FORM_WIDE;
   // long-segment batches in one launch, on request
   if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_SGMV && knobs().auto_fused && fused_supported(a))
@@ -423,7 +428,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
     case MLORA_FORM_SLOT:
     case MLORA_FORM_MFMA: {
       if (!vec || !mfma_supported(a)) { set_error("mlora_add_lora: MFMA forms need 16-bit elements, a plan, a rank that is a multiple of 8 up to 64 and K %% 32 == 0"); return MLORA_E_UNSUPPORTED; }
-      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true, active);
+      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true, active, active_tokens);
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "

@@ -47,7 +47,7 @@ __device__ __forceinline__ void store128(void* p, i32x4 v) { *reinterpret_cast<i
 // 14.8, q|k|v 24.0 / 23.0, down 29.1 / 28.3, 3001 tokens, rank 16, K = 2048, gate_up 52.0 / 49.9; 16-token tiles, 3001 tokens q|k|v 14.6 / 14.1, o 10.6 / 10.3.
 // Launches that write less lose the wait for every store, so 16-token tiles take them from kThroughBytes of y on: 1000 tokens, K = 1024, o (2.0 MB) 5.0 / 4.85, gate_up
 // of 120 tokens at K = 2048 (3.9 MB) 6.9 / 6.5; 400 tokens q|k|v (1.2 MB) 4.82 / 4.87, o (0.8 MB) 4.67 / 4.74; one stream's step of 48 calls 158 / 161; 256 streams'
-// and the pair's outputs the same or 1 % slower a step.
+// and the pair's outputs the same or 1 % slower a step; with K = 4096 over 16-token tiles 2365 tokens of 45 slots, rank 8, 14.2 / 14.8, 1939 of 38, rank 16, 13.0 / 13.8: up to K = 2048.
 constexpr long long kThroughBytes = 2000000;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -35,15 +35,15 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 // decode.hip: the same small tiles with both products on the matrix cores, one workgroup per
 // (tile, column range).
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
-int launch_decode(const MloraAddArgs* a, bool include_long, int active);  // active: slots with tokens where the host counted them, else 0
-int decode_ranges(const MloraAddArgs* a, int active, int* columns);  // column ranges of that launch, and columns per range
+int launch_decode(const MloraAddArgs* a, bool include_long, int active, int active_tokens);  // slots with tokens, tokens with a slot where the host counted them, else 0
+int decode_ranges(const MloraAddArgs* a, int active, int active_tokens, int* columns);  // column ranges of that launch, and columns per range
 
 // slot.hip: the same small tiles, the grid laid over the slots: weights are requested from the
 // workgroup index alone, before the slot's record has arrived.
 bool slot_supported(const MloraAddArgs* a);
 int slot_k_parts(const MloraAddArgs* a);  // 4 or 8 when the workgroups of a tile would share K out, else 1
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace);
-int small_tiles_about(const MloraAddArgs* a, int active);  // 16-token tiles of a batch (api.hip)
+int small_tiles_about(const MloraAddArgs* a, int active, int active_tokens = 0);  // 16-token tiles of a batch (api.hip)
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.
 // trusted_workspace: the head of the workspace is known to be in its initial or a left-behind
