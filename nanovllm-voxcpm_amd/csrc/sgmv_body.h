@@ -754,11 +754,9 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   // round loses: 5200 tokens of 2 slots, K = 2560, two parts 29.8 us, three, 33 workgroups on some XCDs, 33.2) and it cuts K into more parts
   // than the other shrink, whose parts have to divide K (with two slices into as many).  us per call, the other shrink / this, 2 slots: K = 2560,
   // 4096 tokens 32.9 / 25.6; K = 3072, 3600 27.9 / 25.9; K = 5120, 4096 28.1 / 23.2; two slices, K = 2560, 6400 52.7 / 51.9; 498 such
-  // calls of 2 to 16 slots, K 1536 to 5120, take 0.65 to 0.99 of the other's time.  With fewer parts it can win too (rings of 48 KB: K = 4096, 4500 tokens 26.2 / 21.4, 6000 29.3 / 27.3; K = 8192,
-  // 4500 47.5 / 39.1), but only on as many tiles as the tokens could make: tokens without an adapter make none, how many those are
-  // the host does not say, and with a quarter to three quarters of them two or three parts leave compute units idle
-  // that four would fill (K = 4096, 5200 tokens of 2 slots, half of them adapted, 18.2 / 21.2; K = 2048, 8000 of 12, 19.6 / 23.6; 124 of 171 such
-  // calls slower).  Not for
+  // calls of 2 to 16 slots, K 1536 to 5120, take 0.65 to 0.99 of the other's time.  With fewer parts the other, which cuts K by rounds below, is the
+  // faster one (K = 4096, 4500 tokens 22.4, K = 8192 38.0, against 21.4 and 39.1 in these rings on full batches, and where a quarter to three quarters of the tokens
+  // have no adapter 124 of 171 such calls were slower in these).  Not for
   // parts that would be longer than 2800 columns nor below half a
   // round, and not for short segments: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens 23.2 / 25.7.
   // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7).
