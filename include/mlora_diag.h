@@ -3,7 +3,7 @@
  * counterpart in the reference and nothing here is needed to use the library: include/mlora.h is
  * the product's C-ABI.
  *
- * mlora_probe_launch, mlora_trace_set and mlora_group_layout are exported by the diagnostic variants only
+ * mlora_probe_launch, mlora_trace_set, mlora_group_layout and mlora_choice are exported by the diagnostic variants only
  * (libmlora_gfx950_diag.so from `make diag`, libmlora_gfx950_trace.so from `make trace`).
  * mlora_reload_knobs is exported by every variant: the test-suite changes MLORA_* variables
  * between tests of one process.
@@ -12,6 +12,8 @@
 #define MLORA_DIAG_H_
 
 #include <stdint.h>
+
+#include "mlora.h"
 
 #ifdef __cplusplus
 extern "C" {
@@ -43,6 +45,11 @@ int mlora_trace_set(void* buf);
  * `count` tokens, out[5] tokens of its tiles, out[6] tiles beyond those with a place of their own.
  * `extra` is 1 where the tokens without a slot need places (the shrink), else 0. */
 void mlora_group_layout(int32_t num_tokens, int32_t num_slots, int64_t parts, int32_t extra, int32_t count, int32_t* out);
+
+/* What mlora_add_lora_counts would take for a call (host arithmetic, nothing is launched; the same error codes): out[0] the form,
+ * 0 where there is nothing to do, out[1] the K parts of MLORA_FORM_SGMV, out[2] the columns per range of MLORA_FORM_WIDE and
+ * MLORA_FORM_MFMA. */
+int mlora_choice(const MloraAddArgs* args, int32_t active_slots, int32_t active_tokens, int32_t* out);
 
 #ifdef __cplusplus
 }

@@ -118,9 +118,7 @@ const ApiKnobs& knobs() {
 }  // namespace
 
 // Fewer than sixteen tokens to a slot that has any: one small tile each.
-static bool short_segments(const MloraAddArgs* a, int active) {
-  return a->num_tokens < 16ll * slots_with_tokens(a, active);
-}
+static bool short_segments(const Batch& batch) { return batch.tokens < 16ll * batch.slots; }
 
 // Where the one-launch form over 16-token tiles stops paying.  Its cost per token grows with the
 // rank (every tile fetches A[slot] and B[slot] again, every column range repeats its tile's shrink)
@@ -146,25 +144,24 @@ static bool short_segments(const MloraAddArgs* a, int active) {
 // 18.6 / 14.3; q|k|v, 1000 and 1500 of 16, rank 24 14.8 / 12.6, 19.0 / 13.3, rank 32, 740 (of 986, the others without an adapter: tokens with a slot are what counts) 8.1 / 11.3, 1500 18.2 / 13.4.  Segments of fewer than 16 tokens are what
 // the small tiles are for (1000 tokens of 64 slots, rank 32, q|k|v 13.3 / 19.2): these lines are not drawn for them.
 // MLORA_SMALL_BATCH_TOKENS, when set, replaces the rule by a plain token count.
-static bool small_batch(const MloraAddArgs* a, bool one_launch, int active, int active_tokens) {
+static bool small_batch(const MloraAddArgs* a, bool one_launch, const Batch& batch) {
   const int fixed = knobs().small_batch_tokens;
   if (fixed > 0) return a->num_tokens <= fixed;
   double cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double width = static_cast<double>(a->num_slices) * a->k * (a->k > 1024 ? a->k / 1024.0 : 1.0) + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
   double limit = (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) * (one_launch ? 0.65 : 1.0);
-  if (a->r > 16 && !short_segments(a, active)) {
+  if (a->r > 16 && !short_segments(batch)) {
     if (one_launch && a->r <= 32) limit = 0.36 * 2.6e7;
     else if (!one_launch && a->k == 2048 && cols <= 2.0 * a->k && (a->r <= 32 || a->num_slices == 1)) limit = a->r > 32 ? 7.7e6 : a->num_slices > 1 && exact_rank(a->r) ? 1.7e7 : 1.3e7;
   }
-  return tokens_with_slot(a, active_tokens) * width <= limit;
+  return batch.tokens * width <= limit;
 }
 
 // About how many 16-token tiles a batch has: its segments end anywhere inside their last tile.
-int mlora::small_tiles_about(const MloraAddArgs* a, int active, int active_tokens) {
-  const int segs = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  const int tiles = static_cast<int>((tokens_with_slot(a, active_tokens) + 7ll * segs) / MLORA_TILE_SMALL);
-  return tiles > segs ? tiles : segs;
+int mlora::small_tiles_about(const Batch& batch) {
+  const int tiles = static_cast<int>((batch.tokens + 7ll * batch.slots) / MLORA_TILE_SMALL);
+  return tiles > batch.slots ? tiles : batch.slots;
 }
 
 // Where the slot-major grid pays.  Its workgroups request the weights of EVERY slot id, with or
@@ -178,15 +175,15 @@ int mlora::small_tiles_about(const MloraAddArgs* a, int active, int active_token
 // All of this was measured on decode batches; on batches of many tiles per slot (a prefill of
 // 2098 tokens over 8 slot ids, o: 15.4 us per call against 10.1 tile-major) the grid over the slots
 // is the slower one: it is taken up to 32 tokens per slot id.
-// `active` (when the caller knows it, else 0) is the number of slots with tokens.  Prompts are few long
+// (Where the number of slots with tokens was counted.)  Prompts are few long
 // segments: most of the grid is then workgroups without a tile, and the tiles behind a slot's first one learn
 // their slot from a record after all (rank 32, 37 tokens of one slot of 8: gate_up 7.4 / 4.9; 100 tokens
 // of 4 slots: gate_up 7.7 / 5.0; rank 64, 200 tokens of 3 slots of 32: qkv 9.0 / 6.5, gate_up 12.9 / 10.0,
 // down 10.2 / 9.1; rank 16, 250 tokens of 4 slots of 8: 4.05 / 4.11, 3.86 / 3.97, 5.67 / 5.58).
-static bool slot_major_pays(const MloraAddArgs* a, int active) {
+static bool slot_major_pays(const MloraAddArgs* a, const Batch& batch) {
   if (a->num_slots > knobs().slot_max_slots) return false;
-  if (a->num_tokens > 32 * a->num_slots) return false;
-  const bool sparse = active > 0 && 2 * active <= a->num_slots;
+  if (batch.tokens > 32 * a->num_slots) return false;
+  const bool sparse = batch.slots_counted && 2 * batch.slots <= a->num_slots;
   const int parts = slot_k_parts(a);
   // Buffers of a rank between 32 and 64 run rank 64's code masked: K = 2048 gains like rank 64's (rank 48, slot-major / pair: 7.0 /
   // 7.4 at 16 tokens of 8 slot ids, 8.3 / 9.8 at 128 of 32, 10.6 / 12.3 at 256 of 64), eight parts of 1024 columns do not fit
@@ -196,8 +193,8 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
     // K shared out: the lines lie where the requests for slots without tokens, and at K = 8192 more workgroups than fit
     // the chip together, cost what the second launch does.  us per call, slot-major / the best other form, at
     // one and four tokens per slot id unless said:
-    const int tiles = small_tiles_about(a, active), slots = a->num_slots, rank = compute_rank(a->r);
-    const bool few = sparse || 2 * a->num_tokens <= slots;
+    const int tiles = small_tiles_about(batch), slots = a->num_slots, rank = compute_rank(a->r);
+    const bool few = sparse || 2 * batch.tokens <= slots;
     // K = 2048: rank 64 8 slot ids 6.3 / 6.8, 32 8.0 / 10.4 and 8.6 / 11.4, 64 11.1 / 13.5; 8 tokens of 64 8.8 / 7.6.  Rank 32 16 ids
     // 5.2 / 5.3, 48 6.2 / 7.0, 64 7.4 / 8.3; 8 tokens of 32 5.2 / 5.1, 37 of one slot of 8 5.3 / 5.2.  Rank 16 40 ids 4.6 / 4.5, 48 4.7 /
     // 4.8, 64 5.3 / 5.4, 512 tokens of 32 (46 tiles) 5.2 / 5.2, 1000 (76) 6.2 / 7.6; rank 8 alike.
@@ -213,10 +210,10 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
     // 512 tokens of 32 (46 tiles) 11.3 / 13.1, 1000 (76) 17.5 / 16.9, 8 of 32 7.6 / 7.4.  Rank 64 32 ids 13.7 / 15.0, 40 20.2 / 20.0, 512
     // tokens of 32 16.5 / 17.8, 2 of 16 9.3 / 9.2 (rank 32 6.0 / 7.2), 37 of one slot of 8 8.0 / 8.3.
     if (few) return slots <= 8 || rank <= 8 || (rank <= 32 && slots <= 16) || (rank <= 16 && slots <= 32 && tiles <= 16);
-    if (rank <= 8) return slots <= 48 || a->num_tokens >= 2 * slots;
+    if (rank <= 8) return slots <= 48 || batch.tokens >= 2 * slots;
     return rank <= 16 || (tiles <= 48 && slots <= (rank <= 32 ? 40 : 32));
   }
-  if (sparse || (active > 0 && a->num_tokens > MLORA_TILE_SMALL * active)) return false;
+  if (sparse || (batch.slots_counted && batch.tokens > MLORA_TILE_SMALL * batch.slots)) return false;
   double cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double per_slot = 2.0 * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
@@ -226,7 +223,7 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
   // 7.5 / 7.4, rank 64 qkv 7.9 / 7.5, o 6.0 / 5.8; 128 of 64, rank 8 gate_up 7.20 / 7.38, rank 16 o 3.61 / 3.86, gate_up 8.03 / 8.24, rank 24 o 4.45 /
   // 4.70, rank 32 o 4.46 / 4.51.  At two, three and 3.9 tokens of 12 to 64 ids, ranks 8 to 32, 69 of 69 such calls are 0.4 to 7 % faster.
   const bool light = a->k == 1024 && (compute_rank(a->r) <= 16 || (compute_rank(a->r) == 32 && a->num_slices == 1 && cols <= 2048));
-  return a->num_tokens >= (light ? 2 : 4) * a->num_slots;
+  return batch.tokens >= (light ? 2 : 4) * a->num_slots;
 }
 
 // Where the shrink and the expand as two launches over 16-token tiles (pair.hip) beat the form that
@@ -265,31 +262,31 @@ static bool slot_major_pays(const MloraAddArgs* a, int active) {
 //    17.5, 18.6 / 18.7, 21.5 / 20.9; K = 2048, rank 64 84.6 / 65.9, 94.2 / 83.0, rank 16 32.7 / 28.2, 51.2 / 39.6; down of 1500, K = 4096, rank 64 27.9 / 22.9, rank 32 20.7 / 16.2, K =
 //    8192, rank 64 54.5 / 40.1; q|k|v, K = 2048, rank 64, 1000 42.1 / 36.6, but rank 32 22.5 / 23.5.  64 slots: gate_up, 600, K = 1024, rank 64 26.2 / 24.2, rank 32 (42
 //    MB) 16.6 / 16.9, rank 48 23.8 / 21.0, rank 24 (31 MB) 15.0 / 15.5; K = 2048, rank 64 49.8 / 39.4, rank 32 33.4 / 25.7.
-static bool pair_pays(const MloraAddArgs* a, int form, int active, int active_tokens) {
+static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
   const long long rk = static_cast<long long>(a->r) * a->k;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  const bool few_tokens = short_segments(a, active), middling = !few_tokens && active > 0 && a->r > 16 && exact_rank(a->r) && a->num_tokens < 128ll * active;
-  const double weights = 2.0 * slots_with_tokens(a, active) * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
-  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_tokens < (a->r <= 24 || a->num_tokens <= 2000 ? 34ll : 26ll) * slots_with_tokens(a, active) && weights >= 2.0e7) return true;
+  const bool few_tokens = short_segments(batch), middling = !few_tokens && batch.slots_counted && a->r > 16 && exact_rank(a->r) && batch.tokens < 128ll * batch.slots;
+  const double weights = 2.0 * batch.slots * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
+  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && batch.tokens < (a->r <= 24 || batch.tokens <= 2000 ? 34ll : 26ll) * batch.slots && weights >= 2.0e7) return true;
   if (few_tokens && ((form == MLORA_FORM_SGMV && weights >= 4.0e7) ||
                      (form == MLORA_FORM_MFMA && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k)))
     return true;
-  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_slices == 2 && a->k == 2048 && a->num_tokens <= 1100 &&
-      a->num_tokens >= 64ll * slots_with_tokens(a, active))
+  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_slices == 2 && a->k == 2048 && batch.tokens <= 1100 &&
+      batch.tokens >= 64ll * batch.slots)
     return true;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
     case MLORA_FORM_MFMA: {
       if (!exact_rank(a->r)) {
         const double width = static_cast<double>(a->num_slices) * a->k + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
-        return a->k != 1024 || a->num_tokens * width > (a->r > 32 ? 1.0e7 : 2.0e7);
+        return a->k != 1024 || batch.tokens * width > (a->r > 32 ? 1.0e7 : 2.0e7);
       }
       return rk >= 131072;
     }
     case MLORA_FORM_SGMV:
     case MLORA_FORM_WIDE:
-      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(a, active, active_tokens)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
+      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(batch)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
     default: return false;
   }
 }
@@ -305,15 +302,15 @@ static bool pair_pays(const MloraAddArgs* a, int form, int active, int active_to
 // / 12.2, 15.1 / 14.1, 23.3 / 16.2.  With a smaller A the rounds are too short to matter (K = 512,
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
 // of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
-static bool wide_instead(const MloraAddArgs* a, int active, int active_tokens) {
-  if (a->num_slices == 2 || (a->num_slices == 1 && a->r <= 16) || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, active, active_tokens)) return false;
+static bool wide_instead(const MloraAddArgs* a, const Batch& batch) {
+  if (a->num_slices == 2 || (a->num_slices == 1 && a->r <= 16) || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, batch)) return false;
   int columns;
-  return (small_tiles_about(a, active, active_tokens) + 7) / 8 * decode_ranges(a, active, active_tokens, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
+  return (small_tiles_about(batch) + 7) / 8 * decode_ranges(a, batch, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
 }
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int active_tokens);
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active_slots, int active_tokens);
 
 }  // namespace
 
@@ -325,7 +322,9 @@ extern "C" int mlora_add_lora_counts(const MloraAddArgs* a, int32_t active_slots
 
 namespace {
 
-int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int active_tokens) {
+}  // namespace
+
+int mlora::check_args(const MloraAddArgs* a) {
   if (!a) { set_error("mlora_add_lora: NULL args"); return MLORA_E_INVALID; }
   if (a->num_tokens < 0 || a->k < 0 || a->r < 0 || a->num_slots < 0 || a->num_slices < 0) {
     set_error("mlora_add_lora: negative size"); return MLORA_E_INVALID;
@@ -337,7 +336,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
   if (a->num_slices > MLORA_MAX_SLICES) { set_error("mlora_add_lora: %d slices exceed %d", a->num_slices, MLORA_MAX_SLICES); return MLORA_E_TOO_LARGE; }
   if (a->r > MLORA_MAX_RANK) { set_error("mlora_add_lora: rank %d exceeds %d", a->r, MLORA_MAX_RANK); return MLORA_E_TOO_LARGE; }
   if (a->num_slots > MLORA_MAX_SLOTS) { set_error("mlora_add_lora: %d slots exceed %d", a->num_slots, MLORA_MAX_SLOTS); return MLORA_E_TOO_LARGE; }
-  if (a->num_tokens == 0 || a->num_slices == 0 || a->num_slots == 0 || a->r == 0) return 0;
+  if (a->num_tokens == 0 || a->num_slices == 0 || a->num_slots == 0 || a->r == 0) return kNothingToDo;
   if (!a->x || !a->y || !a->token_to_slot) { set_error("mlora_add_lora: NULL tensor pointer"); return MLORA_E_INVALID; }
   bool any = false;
   for (int i = 0; i < a->num_slices; ++i) {
@@ -352,9 +351,12 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
     any |= s.n > 0;
   }
   if (a->x_stride < a->k) { set_error("mlora_add_lora: x row stride %lld is below K = %d", static_cast<long long>(a->x_stride), a->k); return MLORA_E_INVALID; }
-  if (!any) return 0;
+  if (!any) return kNothingToDo;
   if (reinterpret_cast<uintptr_t>(a->plan) & 15) { set_error("mlora_add_lora: plan must be 16-byte aligned"); return MLORA_E_INVALID; }
+  return 0;
+}
 
+int mlora::chosen_form(const MloraAddArgs* a, const Batch& batch) {
   int form = a->form;
   const bool vec = vector_ok(a);
   if (form == MLORA_FORM_AUTO) {
@@ -367,38 +369,49 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
     // both products where a tile's column ranges repeat little of its shrink, else two launches.
     const bool small_tiles = mfma_supported(a) && decode_supported(a);
     const bool two_launches = mfma_supported(a) && sgmv_supported(a) && sgmv_workspace_ok(a);
-    const bool one_launch = mfma_supported(a) && wide_supported(a) && wide_pays(a, active, active_tokens) && !knobs().no_wide;
+    const bool one_launch = mfma_supported(a) && wide_supported(a) && wide_pays(a, batch) && !knobs().no_wide;
     // (fp32 rows and anything else the 128-bit kernels for 16-bit elements do not take: one workgroup per token,
     // which fetches A and B per token and walks K in chained steps, except where the pair of launches has the
     // element type: config 1's batch, 64 tokens over 4 slots, rank 16, fp32, qkv / o / gate_up / down 25 / 25 / 27 /
     // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches; rank 24, 36 / 16 / 39 / 104 and 9.5 / 9.2 / 10.7 /
     // 10.9, rank 56, 81 / 80 / 90 / 243 and 12.6 / 12.1 / 14.3 / 15.5, one token of rank 24 15.3 / 15.4 / 15.8 / 43 and 8.5 / 8.5 / 9.2 / 9.9)
     if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
-    else if (one_launch && !(small_tiles && small_batch(a, true, active, active_tokens))) form = MLORA_FORM_WIDE;
-    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, active, active_tokens))) form = MLORA_FORM_SGMV;
+    else if (one_launch && !(small_tiles && small_batch(a, true, batch))) form = MLORA_FORM_WIDE;
+    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, batch))) form = MLORA_FORM_SGMV;
     else if (small_tiles) form = MLORA_FORM_SPLIT;
     else form = MLORA_FORM_BGMV;
   }
   // the split form where it pays (a large A[slot]) and shape and workspace allow it, else one
   // workgroup per (tile, column range)
   if (form == MLORA_FORM_SPLIT && a->form != MLORA_FORM_SPLIT &&
-      (knobs().no_split || !split_supported(a) || ((static_cast<long long>(a->r) * a->k < knobs().split_min_rk || a->num_tokens > knobs().split_max_tokens) && knobs().force_form != MLORA_FORM_SPLIT)))
+      (knobs().no_split || !split_supported(a) || ((static_cast<long long>(a->r) * a->k < knobs().split_min_rk || batch.tokens > knobs().split_max_tokens) && knobs().force_form != MLORA_FORM_SPLIT)))
     form = MLORA_FORM_MFMA;
   // small tiles with the grid laid over the slots where the shape allows it and slot ids are few.
   // Also where the split form would be taken: at K = 4096 the slot-major kernel shares K out between
   // the workgroups of a tile itself (down, decode batch, us per call, slot-major / split form:
   // rank 32: 6.3 / 10.6, rank 64: 9.8 / 17.0).
   if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
-      knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, active))
+      knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, batch))
     form = MLORA_FORM_SLOT;
-  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, active, active_tokens))
+  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, batch))
     form = MLORA_FORM_PAIR;
   if (form == MLORA_FORM_MFMA && a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_wide && knobs().small_batch_tokens <= 0 &&
-      wide_instead(a, active, active_tokens))
+      wide_instead(a, batch))
     form = MLORA_FORM_WIDE;
   // long-segment batches in one launch, on request
   if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_SGMV && knobs().auto_fused && fused_supported(a))
     form = MLORA_FORM_FUSED;
+  return form;
+}
+
+namespace {
+
+int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active_slots, int active_tokens) {
+  const int rc = check_args(a);
+  if (rc) return rc == kNothingToDo ? 0 : rc;
+  const Batch batch = batch_of(a, active_slots, active_tokens);
+  const bool vec = vector_ok(a);
+  const int form = chosen_form(a, batch);
   switch (form) {
     case MLORA_FORM_TOKEN:
       return launch_token_add(a);
@@ -414,21 +427,21 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
                   "and no empty slice");
         return MLORA_E_UNSUPPORTED;
       }
-      return launch_wide(a, active, active_tokens);
+      return launch_wide(a, batch);
     case MLORA_FORM_PAIR:
       if (!pair_supported(a)) {
         set_error("mlora_add_lora: the pair form needs a plan, a workspace, rows of x of a multiple of 128 bytes, B rows of 16 to 128 (fp32: 256) bytes "
                   "in steps the kernels have, 16-byte aligned rows and no empty slice");
         return MLORA_E_UNSUPPORTED;
       }
-      return launch_pair(a, active);
+      return launch_pair(a, batch);
     case MLORA_FORM_SGMV:
     case MLORA_FORM_FUSED:
     case MLORA_FORM_SPLIT:
     case MLORA_FORM_SLOT:
     case MLORA_FORM_MFMA: {
       if (!vec || !mfma_supported(a)) { set_error("mlora_add_lora: MFMA forms need 16-bit elements, a plan, a rank that is a multiple of 8 up to 64 and K %% 32 == 0"); return MLORA_E_UNSUPPORTED; }
-      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true, active, active_tokens);
+      if (form == MLORA_FORM_MFMA) return launch_decode(a, /*include_long=*/true, batch);
       if (form == MLORA_FORM_SLOT) {
         if (!slot_supported(a)) {
           set_error("mlora_add_lora: the slot-major form needs one or two non-empty slices and K = 1024 (three at an exact rank with column "
@@ -460,7 +473,7 @@ int add_lora_impl(const MloraAddArgs* a, bool trusted_workspace, int active, int
         }
         return launch_fused(a, trusted_workspace);
       }
-      return launch_sgmv(a, active, active_tokens);
+      return launch_sgmv(a, batch);
     }
   }
   set_error("mlora_add_lora: unreachable form %d", form);

@@ -312,7 +312,7 @@ const DecodeKnobs& decode_knobs() {
 // Above rank 16 a workgroup has its compute unit to itself, 32 on an XCD, and what does not fit runs in a second round that shrinks its tile
 // anew: one slice whose ranges spill takes as many fewer as fit (o, K = 1024, 2000 / 2400 / 2800 tokens of 32 slots, in ranges of 832, 960 and 1024 columns: rank 64 11.5 / 18.3 /
 // 13.2, rank 24 8.3 / 12.2 / 8.8; 2400 tokens in one range 12.2 and 8.3).
-int decode_ranges(const MloraAddArgs* a, int active, int active_tokens, int* columns) {
+int decode_ranges(const MloraAddArgs* a, const Batch& batch, int* columns) {
   int nt = decode_knobs().nt;
   if (nt <= 0) {
     long long cols = 0;
@@ -324,7 +324,7 @@ int decode_ranges(const MloraAddArgs* a, int active, int active_tokens, int* col
     if (nt > 1024) nt = 1024;
     if (nt < 128) nt = 128;
     if (a->num_slices == 1 && a->r > 16) {
-      const int n = a->slices[0].n, fit = 32 / ((small_tiles_about(a, active, active_tokens) + 7) / 8);
+      const int n = a->slices[0].n, fit = 32 / ((small_tiles_about(batch) + 7) / 8);
       if ((n + nt - 1) / nt > fit && fit > 0 && (n + fit - 1) / fit <= 1024) nt = (n + fit - 1) / fit;
     }
   }
@@ -352,7 +352,7 @@ void decode_trace_set(void* buf) {
 #endif
 }
 
-int launch_decode(const MloraAddArgs* a, bool include_long, int active, int active_tokens) {
+int launch_decode(const MloraAddArgs* a, bool include_long, const Batch& batch) {
   DecodeSplits splits;
   const PlanLayout lay = plan_layout(a->num_tokens, a->num_slots);
   int cap = lay.cap_small;
@@ -373,10 +373,9 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active, int acti
   // Behind a capture the slots of the buffers count for those with tokens: a graph is captured for batches of about one token per slot, and one that
   // then brings full tiles loses up to 3 % of a call (64 tokens of 3 of 48 slots, without / with the texts: rank 16, K = 2048, q|k|v 5.1 / 5.2, o 4.9 / 4.8; rank 32, K =
   // 1024, 4.4 / 4.5 and 4.2 / 4.3; rank 48 6.9 / 6.9, gate_up 9.3 / 9.5), less than short tiles would lose without.
-  const int with_tokens = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
 
   int nt;
-  const int total = decode_ranges(a, active, active_tokens, &nt);
+  const int total = decode_ranges(a, batch, &nt);
   if (total == 0) return 0;
   int s = 0;
   l.widest = 0;
@@ -389,10 +388,10 @@ int launch_decode(const MloraAddArgs* a, bool include_long, int active, int acti
       if (d.n1 - d.n0 > l.widest) l.widest = d.n1 - d.n0;
     }
   }
-  l.short_tiles = decode_knobs().short_tiles < 0 ? a->num_tokens <= (l.widest <= kNW * 64 ? 12 : 4) * with_tokens : decode_knobs().short_tiles != 0;
+  l.short_tiles = decode_knobs().short_tiles < 0 ? batch.tokens <= (l.widest <= kNW * 64 ? 12 : 4) * batch.slots : decode_knobs().short_tiles != 0;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  if (decode_knobs().through < 0 ? a->k <= 2048 && a->num_tokens * cols * 2 >= kThroughBytes : decode_knobs().through != 0) l.include_long |= kThrough;
+  if (decode_knobs().through < 0 ? a->k <= 2048 && batch.tokens * cols * 2 >= kThroughBytes : decode_knobs().through != 0) l.include_long |= kThrough;
   for (; s < kMaxSplits; ++s) splits.split[s] = DecodeSplit{nullptr, nullptr, 0, 0, 0, 0};
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(cap / 8));
   const int nks = a->k / 32;

@@ -24,6 +24,18 @@ extern "C" int mlora_trace_set(void* buf) {
 #endif
 }
 
+extern "C" int mlora_choice(const MloraAddArgs* a, int32_t active_slots, int32_t active_tokens, int32_t* out) {
+  out[0] = out[1] = out[2] = 0;
+  const int rc = check_args(a);
+  if (rc) return rc == kNothingToDo ? 0 : rc;
+  const Batch batch = batch_of(a, active_slots, active_tokens);
+  out[0] = chosen_form(a, batch);
+  if (out[0] == MLORA_FORM_SGMV) out[1] = sgmv_parts(a, batch);
+  if (out[0] == MLORA_FORM_WIDE) out[2] = wide_columns(a, batch);
+  if (out[0] == MLORA_FORM_MFMA) decode_ranges(a, batch, &out[2]);
+  return 0;
+}
+
 extern "C" void mlora_group_layout(int32_t num_tokens, int32_t num_slots, int64_t parts, int32_t extra, int32_t count, int32_t* out) {
   GroupPlaces p = {};
   p.T = num_tokens; p.num_slots = num_slots;

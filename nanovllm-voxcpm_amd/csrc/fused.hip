@@ -326,11 +326,11 @@ void fused_trace_set(void* buf) {
 bool fused_supported(const MloraAddArgs* a) {
   if (!exact_rank(a->r) || !sgmv_supported(a) || !sgmv_workspace_ok(a) || a->k % 256 != 0) return false;
   if (a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return false;
-  return shape_fits(a, sgmv_shape(a, true));
+  return shape_fits(a, sgmv_shape(a, batch_of(a, 0, 0), true));
 }
 
 int launch_fused(const MloraAddArgs* a, bool trusted_workspace) {
-  const SgmvShape sh = sgmv_shape(a, true);
+  const SgmvShape sh = sgmv_shape(a, batch_of(a, 0, 0), true);
   if (sh.empty) return 0;
   FusedLaunch l{a, &sh, trusted_workspace ? 1 : 0};
   if (a->dtype == MLORA_DTYPE_BF16) launch_fused_rank<__bf16>(l);

@@ -15,15 +15,32 @@ int env_int(const char* name, int fallback);
 // rank; the other forms take exact ranks only.
 inline bool exact_rank(int r) { return r == 8 || r == 16 || r == 32 || r == 64; }
 inline bool padded_rank(int r) { return r >= 8 && r <= 64 && r % 8 == 0; }
-// Tokens with a slot and slots with tokens: what the host counted (else 0), or at most.
-inline int tokens_with_slot(const MloraAddArgs* a, int active_tokens) { return active_tokens > 0 && active_tokens < a->num_tokens ? active_tokens : a->num_tokens; }
-inline int slots_with_tokens(const MloraAddArgs* a, int active) { return active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens; }
+// What the host knows of a batch beyond its size: how many slots have tokens and how many tokens a slot, each as counted, else (a captured call, a
+// caller who does not say) the most there can be.
+struct Batch {
+  int slots, tokens;
+  bool slots_counted, tokens_counted;
+};
+inline Batch batch_of(const MloraAddArgs* a, int active_slots, int active_tokens) {
+  Batch b;
+  b.slots_counted = active_slots > 0;
+  b.tokens_counted = active_tokens > 0;
+  b.slots = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
+  if (b.slots_counted && active_slots < b.slots) b.slots = active_slots;
+  b.tokens = b.tokens_counted && active_tokens < a->num_tokens ? active_tokens : a->num_tokens;
+  return b;
+}
 // The 64-token tiles serve buffers of every padded rank; by name only those of the instances' own, as ever.
 inline bool tiles64_rank(const MloraAddArgs* a) { return a->form == MLORA_FORM_AUTO ? padded_rank(a->r) : exact_rank(a->r); }
 inline int compute_rank(int r) { return r <= 8 ? 8 : r <= 16 ? 16 : r <= 32 ? 32 : 64; }
 // Diagnostic knobs are read from the environment once and kept; mlora_reload_knobs() advances
 // this number, and a holder whose copy is older reads its variables again.
 int knob_generation();
+
+// api.hip: the checks on a call's arguments (0, kNothingToDo or an error code), and the form that serves it.
+constexpr int kNothingToDo = INT32_MIN;
+int check_args(const MloraAddArgs* a);
+int chosen_form(const MloraAddArgs* a, const Batch& batch);
 
 // token.hip: one workgroup per token; needs only token_to_slot.
 int launch_token_add(const MloraAddArgs* a);
@@ -35,15 +52,15 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 // decode.hip: the same small tiles with both products on the matrix cores, one workgroup per
 // (tile, column range).
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
-int launch_decode(const MloraAddArgs* a, bool include_long, int active, int active_tokens);  // slots with tokens, tokens with a slot where the host counted them, else 0
-int decode_ranges(const MloraAddArgs* a, int active, int active_tokens, int* columns);  // column ranges of that launch, and columns per range
+int launch_decode(const MloraAddArgs* a, bool include_long, const Batch& batch);
+int decode_ranges(const MloraAddArgs* a, const Batch& batch, int* columns);  // column ranges of that launch, and columns per range
 
 // slot.hip: the same small tiles, the grid laid over the slots: weights are requested from the
 // workgroup index alone, before the slot's record has arrived.
 bool slot_supported(const MloraAddArgs* a);
 int slot_k_parts(const MloraAddArgs* a);  // 4 or 8 when the workgroups of a tile would share K out, else 1
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace);
-int small_tiles_about(const MloraAddArgs* a, int active, int active_tokens = 0);  // 16-token tiles of a batch (api.hip)
+int small_tiles_about(const Batch& batch);  // 16-token tiles of a batch (api.hip)
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.
 // trusted_workspace: the head of the workspace is known to be in its initial or a left-behind
@@ -57,7 +74,8 @@ int workspace_init(void* workspace, hipStream_t stream);
 bool sgmv_supported(const MloraAddArgs* a);
 bool sgmv_workspace_ok(const MloraAddArgs* a);
 size_t sgmv_workspace_bytes(int num_tokens, int num_slices, int r, int dtype);
-int launch_sgmv(const MloraAddArgs* a, int active, int active_tokens);  // slots with tokens and tokens with a slot where the host counted them, else 0
+int launch_sgmv(const MloraAddArgs* a, const Batch& batch);
+int sgmv_parts(const MloraAddArgs* a, const Batch& batch);  // K parts of that launch
 
 // slab.hip: the shrink launch of that form, operands through LDS by direct loads.
 struct PlanLayout;
@@ -71,14 +89,15 @@ int launch_fused(const MloraAddArgs* a, bool trusted_workspace);
 
 // wide.hip: the same tiles, one launch, one workgroup per (tile, column range) doing both products.
 bool wide_supported(const MloraAddArgs* a);
-bool wide_pays(const MloraAddArgs* a, int active, int active_tokens);
-int launch_wide(const MloraAddArgs* a, int active, int active_tokens);
+bool wide_pays(const MloraAddArgs* a, const Batch& batch);
+int launch_wide(const MloraAddArgs* a, const Batch& batch);
+int wide_columns(const MloraAddArgs* a, const Batch& batch);  // columns per range of that launch
 
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
 // direct loads; 16- and 32-bit elements.
 bool pair_supported(const MloraAddArgs* a);
-// Under AUTO fp32 takes one launch where that is the faster one (`active`: slots with tokens where the host counted them, else 0).
-int launch_pair(const MloraAddArgs* a, int active);
+// Under AUTO fp32 takes one launch where that is the faster one .
+int launch_pair(const MloraAddArgs* a, const Batch& batch);
 
 // group.hip: the low-level shrink and expand over tiles of a slot; `supported` says where they are the faster ones too.
 bool group_shrink_supported(const MloraShrinkArgs* a);

@@ -801,7 +801,7 @@ int columns_total(const MloraAddArgs* a, int nt) {
 //   rank 32, K = 1024 (256 columns: B rows of 512 do not fit the LDS):  64 of 4 8.3 / 7.6, 7.8 / 7.0, 9.7 / 9.5; 8 of 8 gate_up 8.6 / 9.0 (32); 64 of
 //   32 9.8 / 8.0, 8.9 / 7.7; 256 of 64 o 10.1 / 9.3 (32), q|k|v 14.2 / 16.6 (48).  At K = 2048 it loses throughout (64 of 4 9.2 / 10.0).
 //   K = 4096 loses at every rank (rank 8, 1 token: 7.1 / 8.9).
-static int solo_columns(const MloraAddArgs* a, int active) {
+static int solo_columns(const MloraAddArgs* a, const Batch& batch) {
   if (a->dtype != MLORA_DTYPE_F32 || a->form != MLORA_FORM_AUTO || !(a->r == 8 || a->r == 16 || a->r == 32)) return 0;
   if (pair_knobs().solo != 1) {
     if (pair_knobs().solo != 2) return 0;
@@ -810,7 +810,7 @@ static int solo_columns(const MloraAddArgs* a, int active) {
                : columns_total(a, 256) <= kMaxSplits ? 256 : 0;
   }
   if (a->k > 2048 || static_cast<long long>(a->r) * a->k > 32768) return 0;
-  const int layers = (small_tiles_about(a, active) + 7) / 8;  // tiles of an XCD
+  const int layers = (small_tiles_about(batch) + 7) / 8;  // tiles of an XCD
   for (int nt = 256; nt <= (a->r <= 16 ? 512 : 256); nt *= 2) {
     const int total = columns_total(a, nt);
     if (total <= kMaxSplits && layers * total <= (a->r <= 16 ? 32 : 24)) return nt;
@@ -852,8 +852,8 @@ static int launch_solo(const MloraAddArgs* a, int nt) {
   return check_launch("mlora_add_lora(fp32, one launch over small tiles)");
 }
 
-int launch_pair(const MloraAddArgs* a, int active) {
-  if (const int nt = solo_columns(a, active)) return launch_solo(a, nt);
+int launch_pair(const MloraAddArgs* a, const Batch& batch) {
+  if (const int nt = solo_columns(a, batch)) return launch_solo(a, nt);
   PairLaunch l;
   l.a = a;
   l.lay = plan_layout(a->num_tokens, a->num_slots);
@@ -868,7 +868,7 @@ int launch_pair(const MloraAddArgs* a, int active) {
   const long long per_slot = static_cast<long long>(a->r) * (static_cast<long long>(a->num_slices) * a->k + cols) * element_bytes(a->dtype);
   const long long need = (kOnceBytes + per_slot - 1) / per_slot;  // slots whose weights are that much
   const int once_from = pair_knobs().once > 0 ? 0 : need <= MLORA_MAX_SLOTS ? static_cast<int>(need) : MLORA_MAX_SLOTS + 1;
-  l.once = pair_knobs().once < 0 ? (active > 0 ? active : segs) >= once_from : pair_knobs().once != 0;
+  l.once = pair_knobs().once < 0 ? batch.slots >= once_from : pair_knobs().once != 0;
   static_assert(MLORA_MAX_SLICES < 256 && MLORA_MAX_SLOTS + 1 < 1 << 23, "one word");
   l.slices_once = l.once ? a->num_slices | once_from << 8 : a->num_slices;
   // K parts: workgroups for most compute units, no more (every column range of the second launch

@@ -355,9 +355,11 @@ bool sgmv_workspace_ok(const MloraAddArgs* a) {
   return partials_room(a) >= partial_bytes(a->num_tokens, a->num_slices, a->r);
 }
 
+int sgmv_parts(const MloraAddArgs* a, const Batch& batch) { return sgmv_shape(a, batch).ksplit; }
+
 // Every segment of the batch: 64-token tiles of the long ones, one short tile each for the rest.
-int launch_sgmv(const MloraAddArgs* a, int active, int active_tokens) {
-  const SgmvShape sh = sgmv_shape(a, false, active, active_tokens);
+int launch_sgmv(const MloraAddArgs* a, const Batch& batch) {
+  const SgmvShape sh = sgmv_shape(a, batch);
   if (sh.empty) return 0;
   if (sh.slab) launch_slab_shrink(a, sh.lay, sh.big_cap, sh.tiles8, sh.ksplit, sh.sl.a);
   else if (a->dtype == MLORA_DTYPE_BF16) launch_shrink<__bf16>(a, sh);

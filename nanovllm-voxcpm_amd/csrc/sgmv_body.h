@@ -675,10 +675,9 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
 }
 
 // About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile.
-inline int big_tiles_about(const MloraAddArgs* a, int active, int active_tokens) {
-  const int segs = slots_with_tokens(a, active);
-  const int tiles = static_cast<int>((tokens_with_slot(a, active_tokens) + 31ll * segs) / MLORA_TILE_BIG);
-  return tiles > segs ? tiles : segs;
+inline int big_tiles_about(const Batch& batch) {
+  const int tiles = static_cast<int>((batch.tokens + 31ll * batch.slots) / MLORA_TILE_BIG);
+  return tiles > batch.slots ? tiles : batch.slots;
 }
 
 // How a call is cut into work, shared by the two-launch and the one-launch form.
@@ -702,7 +701,7 @@ struct SgmvShape {
 
 // one_launch: the cut for the form whose workgroups do both products (256-column slabs and batches,
 // which leave the registers the kernel needs besides; as many shrink roles per unit as it has workgroups).
-inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int active = 0, int active_tokens = 0) {
+inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_launch = false) {
   SgmvShape s;
   s.empty = true;
   s.lay = plan_layout(a->num_tokens, a->num_slots);
@@ -720,7 +719,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   for (int i = a->num_slices; i < MLORA_MAX_SLICES; ++i) s.sl.a[i] = nullptr;
   if (cols == 0) return s;
   s.empty = false;
-  const int est_tiles = a->num_tokens / MLORA_TILE_BIG + 1;
+  const int est_tiles = batch.tokens / MLORA_TILE_BIG + 1;
 
   // shrink: K parts so that the grid has a workgroup per compute unit and parts of at most 1024 columns, as far as multiples of 512 columns (256, 128 where K
   // is no multiple) divide K; (gate_up of the prefill batch with one part 72.2 us per call against 73.3 with two, o with two 19.6
@@ -761,10 +760,9 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
   // round, and not for short segments: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens 23.2 / 25.7.
   // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7).
   int round_parts = 0;
-  const int slots = active > 0 ? active : a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;
-  if (!one_launch && !s.slab && sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 && slots > 0 &&
-      a->num_tokens / slots >= 4 * MLORA_TILE_BIG) {
-    const int tiles = static_cast<int>((a->num_tokens + 63ll * slots) / MLORA_TILE_BIG);  // at most: every slot's last tile has one token
+  if (!one_launch && !s.slab && sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 &&
+      batch.tokens / batch.slots >= 4 * MLORA_TILE_BIG) {
+    const int tiles = static_cast<int>((batch.tokens + 63ll * batch.slots) / MLORA_TILE_BIG);  // at most: every slot's last tile has one token
     const int most = a->num_slices == 1 ? kMaxKSplit : 2;
     int parts = 32 / ((tiles + 7) / 8 * a->num_slices);
     if (parts > most) parts = most;
@@ -799,7 +797,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
       // Unless other parts leave fewer columns to the compute unit with the most workgroups (below): rank 16, K = 8192, 4500 tokens 35.7 us in four
       // parts (three rounds of a quarter where the last is nearly empty), 31.6 in three; 9000 59.8 / 56.5; K = 4096, 9000 34.0 / 33.1, 4000 18.0 / 17.4 in four.
       if (a->num_slices == 1) {
-        const int tiles = big_tiles_about(a, active, active_tokens);
+        const int tiles = big_tiles_about(batch);
         auto columns = [&](int p) { return (static_cast<long long>(tiles) * p + 255) / 256 * (a->k / p); };
         for (int p = 1; p <= kMaxKSplit && a->k / 64 >= p * kSlabStages; ++p)
           if (10 * columns(p) < 9 * columns(ksplit)) ksplit = p;
@@ -818,7 +816,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, bool one_launch = false, int 
     // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
     // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
     // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
-    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(a, active, active_tokens);
+    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(batch);
     long long least = 0;
     for (int p = 1; p <= ksplit; ++p) {
       const long long wgs = static_cast<long long>(tiles) * a->num_slices * p;

@@ -559,7 +559,7 @@ Parts k_parts(const MloraAddArgs* a) {
   if (!(a->num_slices == 1 || three) || slot_knobs().kparts == 1) return one;
   if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < MLORA_WORKSPACE_HEAD_BYTES) return one;
   const Parts small = {a->k / 512, 4}, large = {a->k / 1024, kNW};
-  const int tiles = small_tiles_about(a, 0), most = tiles > a->num_slots ? tiles : a->num_slots;
+  const int tiles = small_tiles_about(batch_of(a, 0, 0)), most = tiles > a->num_slots ? tiles : a->num_slots;
   if ((a->k == 2048 || (a->k == 4096 && 8 * most <= (a->r <= 16 ? 256 : 192))) && parts_fit(a, small)) return small;
   if ((a->k == 4096 || a->k == 8192) && parts_fit(a, large)) return large;
   return one;

@@ -473,8 +473,8 @@ struct WideCut {
   long long workgroups;
   bool short_segments;
 };
-static WideCut wide_cut(const MloraAddArgs* a, int active, int active_tokens) {
-  const long long segs = slots_with_tokens(a, active), n = tokens_with_slot(a, active_tokens);
+static WideCut wide_cut(const MloraAddArgs* a, const Batch& batch) {
+  const long long segs = batch.slots, n = batch.tokens;
   const bool short_segments = n < 128 * segs;
   const long long tiles = short_segments ? (n + 31 * segs) / MLORA_TILE_BIG : n / MLORA_TILE_BIG + segs / 2;
   auto ranges = [&](int columns) {
@@ -512,12 +512,12 @@ static WideCut wide_cut(const MloraAddArgs* a, int active, int active_tokens) {
 // fill their rounds of 256, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 / 38.9);
 // q|k|v of 252 25.2 / 30.3 (r 24 22.1 / 25.5), of 436 to 500 37.4 / 39.0, 42.6 / 47.5, 44.6 / 49.8, but of 210 33.9 / 30.9, of 344 42.0 / 33.1, of 404 43.9 / 42.6.
 // K = 4096: never by more than 5 %, and 31.5 / 30.5 at 7500 tokens.
-bool wide_pays(const MloraAddArgs* a, int active, int active_tokens) {
+bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
   long long repeats = 0;
   for (int i = 0; i < a->num_slices; ++i) repeats += (a->slices[i].n + 511) / 512 - 1;
   if (repeats * a->k <= 1024) return true;
   if (a->k != 2048 || repeats > 3 || a->r <= 16) return false;
-  const WideCut cut = wide_cut(a, active, active_tokens);
+  const WideCut cut = wide_cut(a, batch);
   if (cut.short_segments) return false;
   const long long w = cut.workgroups;
   return (cut.columns == 1024 && w <= 256 && w >= (a->num_slices == 1 ? 156 : 244)) || (a->num_slices > 1 && w > 420 && w <= 512);
@@ -530,14 +530,14 @@ bool wide_supported(const MloraAddArgs* a) {
   return true;
 }
 
-int launch_wide(const MloraAddArgs* a, int active, int active_tokens) {
-  const SgmvShape sh = sgmv_shape(a);
+int wide_columns(const MloraAddArgs* a, const Batch& batch) { return wide_knobs().nt > 0 ? wide_knobs().nt : wide_cut(a, batch).columns; }
+
+int launch_wide(const MloraAddArgs* a, const Batch& batch) {
+  const SgmvShape sh = sgmv_shape(a, batch);
   if (sh.empty) return 0;
   WideLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.big_cap = sh.big_cap;
-  int nt = wide_knobs().nt;
-  if (nt <= 0) nt = wide_cut(a, active, active_tokens).columns;
-  const int nsplit = fill_splits(a, nt, l.splits.split);
+  const int nsplit = fill_splits(a, wide_columns(a, batch), l.splits.split);
   l.grid = dim3(8, static_cast<unsigned>(nsplit), static_cast<unsigned>(sh.tiles8));
   if (a->dtype == MLORA_DTYPE_BF16) launch_wide_rank<__bf16>(l);
   else launch_wide_rank<_Float16>(l);

@@ -76,8 +76,8 @@ EXPORTS = (
 
 
 # include/mlora_diag.h: measurement and test aids.  The product library exports the first only; the
-# diag and trace variants export all three.
-DIAG_EXPORTS = ("mlora_reload_knobs", "mlora_probe_launch", "mlora_trace_set", "mlora_group_layout")
+# diag and trace variants export all of them.
+DIAG_EXPORTS = ("mlora_reload_knobs", "mlora_probe_launch", "mlora_trace_set", "mlora_group_layout", "mlora_choice")
 DIAG_LIB_NAME = "libmlora_gfx950_diag.so"
 
 
@@ -274,6 +274,9 @@ def _declare_diag(lib: C.CDLL) -> None:
     if hasattr(lib, "mlora_group_layout"):
         lib.mlora_group_layout.argtypes = [C.c_int32, C.c_int32, C.c_int64, C.c_int32, C.c_int32, C.POINTER(C.c_int32)]
         lib.mlora_group_layout.restype = None
+    if hasattr(lib, "mlora_choice"):
+        lib.mlora_choice.argtypes = [C.POINTER(MloraAddArgs), C.c_int32, C.c_int32, C.POINTER(C.c_int32)]
+        lib.mlora_choice.restype = C.c_int
 
 
 _DIAG_LIB: C.CDLL | None = None

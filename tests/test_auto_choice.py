@@ -1,0 +1,43 @@
+"""What AUTO takes for a call and how it cuts it (mlora_choice of the diagnostic library: host arithmetic, nothing is launched)."""
+
+import ctypes
+
+import pytest
+import torch
+
+from nanovllm_voxcpm_amd import _hip
+
+NAMES = {code: name for name, code in _hip.FORMS.items()}
+
+
+def choice(rows, k, widths, rank, slots, active_slots=0, active_tokens=0, room=8 << 20):
+    """(form, K parts, columns per range) of a 16-bit call with `room` bytes of workspace beyond what is asked for."""
+    args = _hip.MloraAddArgs()
+    args.x = args.y = 1 << 28
+    args.x_stride, args.y_stride = k, sum(widths)
+    args.token_to_slot, args.plan = 1 << 29, 1 << 30
+    args.num_tokens, args.k, args.r, args.num_slots, args.num_slices = rows, k, rank, slots, len(widths)
+    args.dtype, args.scaling = _hip.dtype_code(torch.bfloat16), 1.0
+    for i, n in enumerate(widths):
+        args.slices[i].a, args.slices[i].b, args.slices[i].n, args.slices[i].y_col = 1 << 31, 1 << 32, n, sum(widths[:i])
+    args.workspace = 1 << 33
+    args.workspace_bytes = _hip.add_workspace_bytes(rows, len(widths), rank, torch.bfloat16) + room
+    out = (ctypes.c_int32 * 3)()
+    assert _hip.load_diag().mlora_choice(ctypes.byref(args), active_slots, active_tokens, out) == 0
+    return NAMES[out[0]], out[1], out[2]
+
+
+@pytest.mark.parametrize("rows,tokens,k,widths,rank,slots", [
+    (1331, 665, 1536, [6144, 6144], 24, 32), (2496, 1872, 4096, [4096, 1024, 1024], 24, 64), (5915, 2070, 1024, [1024], 48, 2),
+    (451, 225, 2048, [2048], 64, 8), (973, 340, 1024, [256], 24, 32), (4269, 2134, 1024, [4096, 4096], 48, 100), (1821, 637, 2048, [8192, 8192], 64, 100),
+    (1536, 768, 1024, [1024], 64, 64), (329, 164, 1024, [256], 64, 64),
+])
+def test_rows_known_to_have_no_slot_do_not_count(rows, tokens, k, widths, rank, slots):
+    assert choice(rows, k, widths, rank, slots, slots, tokens)[0] == choice(tokens, k, widths, rank, slots, slots, tokens)[0]
+
+
+def test_nothing_to_do_has_no_form():
+    args, out = _hip.MloraAddArgs(), (ctypes.c_int32 * 3)(9, 9, 9)
+    assert _hip.load_diag().mlora_choice(ctypes.byref(args), 0, 0, out) == 0 and list(out) == [0, 0, 0]
+    args.form = 99
+    assert _hip.load_diag().mlora_choice(ctypes.byref(args), 0, 0, out) != 0
