@@ -60,6 +60,13 @@ int decode_ranges(const MloraAddArgs* a, const Batch& batch, int* columns);  // 
 bool slot_supported(const MloraAddArgs* a);
 int slot_k_parts(const MloraAddArgs* a);  // 4 or 8 when the workgroups of a tile would share K out, else 1
 int launch_slot(const MloraAddArgs* a, bool trusted_workspace);
+// How often the fullest of 256 compute units has the time of a workgroup, of which two fit side by side and take the price of both: between the whole
+// rounds and the share of one that the workgroups come to, since tiles that end early let others in and the number of tiles is an estimate.
+inline double rounds_of(long long workgroups) {
+  const double share = workgroups / 256.0;
+  return 0.5 * (static_cast<double>((workgroups + 255) / 256) + (share > 1 ? share : 1));
+}
+
 int small_tiles_about(const Batch& batch);  // 16-token tiles of a batch (api.hip)
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.

@@ -721,9 +721,8 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
   s.empty = false;
   const int est_tiles = batch.tokens / MLORA_TILE_BIG + 1;
 
-  // shrink: K parts so that the grid has a workgroup per compute unit and parts of at most 1024 columns, as far as multiples of 512 columns (256, 128 where K
-  // is no multiple) divide K; (gate_up of the prefill batch with one part 72.2 us per call against 73.3 with two, o with two 19.6
-  // against 22.4 with one, down with four 33.6 against 35.7 with two and 50.5 with one)
+  // Parts that divide K, as many as powers of two until the grid has a workgroup per compute unit and parts of at most 1024 columns: of the one-launch
+  // form, and what the line of slab.hip at rank 64 compares with.  (The ring's are further down.)
   int unit = 512;
   while (unit > 128 && a->k % unit != 0) unit /= 2;
   int max_parts = static_cast<int>(partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r));
@@ -808,22 +807,29 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
     s.ksplit = ksplit;
   }
 
-  if (!one_launch && !s.slab && sgmv_knobs().ksplit <= 0) {
-    // The ring's parts need not divide K evenly, and what counts is how many of its workgroups come to a compute unit: one, or two that
-    // run side by side for the price of both.  The cheapest of one to as many parts as above by workgroups per unit x columns of a
-    // part; a part also costs its sums, which every column range reads (`extra`, in columns; at equal cost the more parts up to K = 4096, the fewer beyond).
+  if (!one_launch && !s.slab) {
+    // The ring's parts need not divide K.  What counts is how many of its workgroups come to a compute unit (rounds_of), times the columns of a part; a
+    // part also costs its sums, which every column range reads: as much as 40 columns a slice.  Against the best of one to four parts, each
+    // measured, on 5400 calls of K = 384 to 16384, every rank, 200 to 9392 tokens of 1 to 128 slots, this takes 1.008 of the time for one
+    // slice, 1.009 for two, 1.020 for three; parts that divide K, as many as powers of two, took 1.122, 1.054 and 1.079 (one
+    // slice, rank 48, K = 2560, 2384 tokens of a slot, one part / four 20.7 / 13.8 us; K = 2048, rank 40, 1436 of 3 13.4 / 9.6).
     // us per call with one / two / three / four parts, rank 64: K = 4096, 4000 tokens of 3 slots 31.0 / 24.1 / 21.9 / 20.4, 5500 33.5 / 27.4 / 30.3 / 27.5, 7000
     // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
     // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
     // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
-    const int extra = a->num_slices > 1 ? 100 : a->k < 8192 ? 0 : 30, tiles = big_tiles_about(batch);
-    long long least = 0;
-    for (int p = 1; p <= ksplit; ++p) {
-      const long long wgs = static_cast<long long>(tiles) * a->num_slices * p;
-      const long long cost = (wgs + 255) / 256 * (a->k / p) + extra * p;
-      if (p == 1 || cost < least + (extra == 0)) {
-        least = cost;
-        s.ksplit = p;
+    int most = a->k / 64 < kMaxKSplit ? a->k / 64 : kMaxKSplit;
+    if (most > max_parts) most = max_parts;
+    if (sgmv_knobs().ksplit > 0) {
+      s.ksplit = sgmv_knobs().ksplit < most ? sgmv_knobs().ksplit : most;
+    } else {
+      const long long wgs = static_cast<long long>(big_tiles_about(batch)) * a->num_slices;
+      double least = 0;
+      for (int p = 1; p <= most; ++p) {
+        const double cost = rounds_of(wgs * p) * a->k / p + 40.0 * a->num_slices * p;
+        if (p == 1 || cost < least) {
+          least = cost;
+          s.ksplit = p;
+        }
       }
     }
   }

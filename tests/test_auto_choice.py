@@ -41,3 +41,18 @@ def test_nothing_to_do_has_no_form():
     assert _hip.load_diag().mlora_choice(ctypes.byref(args), 0, 0, out) == 0 and list(out) == [0, 0, 0]
     args.form = 99
     assert _hip.load_diag().mlora_choice(ctypes.byref(args), 0, 0, out) != 0
+
+
+@pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
+    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (7000, 1536, [1536], 64, 100, 3), (3000, 4096, [16384, 16384], 64, 16, 2),
+    (9000, 4096, [1024], 64, 3, 3), (2200, 1920, [7680, 7680], 24, 3, 3),
+])
+def test_k_parts_need_not_divide_k(rows, k, widths, rank, slots, parts):
+    form, got, _ = choice(rows, k, widths, rank, slots, slots, rows)
+    assert (form, got) == ("sgmv", parts)
+
+
+def test_as_many_k_parts_as_the_workspace_holds():
+    for held in (1, 2, 3):
+        room = (held - 4) * 4 * 2200 * 2 * 24  # of four parts
+        assert choice(2200, 1920, [7680, 7680], 24, 3, 3, 2200, room)[:2] == ("sgmv", held)
