@@ -59,7 +59,9 @@ template <int NA8, int TB> struct RingShape {
 };
 
 // The sums of a tile over pieces [c0, c1) of K.  The wavefronts share out the loads of a stage and the blocks of sixteen tokens by sixteen ranks; every
-// block adds K up in one chain, as the one-launch form (fused.hip) does.
+// block adds K up in two chains, the even and the odd 32 columns, as the one-launch form (fused.hip) does.  In one chain the sums' error against 64
+// bits was larger than what slab.hip leaves (rms, one part / slab.hip's or this: K = 1024 1.84e-7 / 1.27e-7; three parts, K = 4096 2.2e-7 / 1.5e-7, 8192
+// 3.2e-7 / 2.2e-7), and 0.4 % faster (4346 calls; K = 10240 at rank 24 and 600 tokens 16.4 / 16.7 us).
 template <typename T, int NA8, int TB>
 __device__ __forceinline__ void ring_tile(char* lds, const char* abase, uint32_t arow, const char* const (&xrow)[2], int c0, int c1, float* __restrict__ dst,
                                           int64_t hrow, int r_all, int m) {
@@ -98,11 +100,13 @@ __device__ __forceinline__ void ring_tile(char* lds, const char* abase, uint32_t
   const bool hi = S::HI == S::LO || (has_x ? NX : 0) + (has_a ? NA : 0) == S::HI;
   const int wt = wave % S::WT, wr = wave / S::WT;
   const bool works = wr < S::WR;
-  f32x4 acc[BR][BT];
+  f32x4 acc[2][BR][BT];
 #pragma unroll
-  for (int rb = 0; rb < BR; ++rb)
+  for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-    for (int tb = 0; tb < BT; ++tb) acc[rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rb = 0; rb < BR; ++rb)
+#pragma unroll
+      for (int tb = 0; tb < BT; ++tb) acc[ks][rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int n = (c1 - c0 + P - 1) / P;
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s)
@@ -136,23 +140,25 @@ __device__ __forceinline__ void ring_tile(char* lds, const char* abase, uint32_t
 #pragma unroll
           for (int rb = 0; rb < BR; ++rb)
 #pragma unroll
-            for (int tb = 0; tb < BT; ++tb) acc[rb][tb] = Mma<T>::run(aw[ks][rb], xa[ks][tb], acc[rb][tb]);
+            for (int tb = 0; tb < BT; ++tb) acc[ks][rb][tb] = Mma<T>::run(aw[ks][rb], xa[ks][tb], acc[ks][rb][tb]);
       }
     }
     stage = stage + 1 == NST ? 0 : stage + 1;
     into = into + 1 == NST ? 0 : into + 1;
   }
 #pragma unroll
-  for (int rb = 0; rb < BR; ++rb) mfma_settle(acc[rb]);  // (the last products and the reads of the sums lie on two sides of branches)
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int rb = 0; rb < BR; ++rb) mfma_settle(acc[ks][rb]);  // (the last products and the reads of the sums lie on two sides of branches)
   MLORA_STAMP(5);  // shrink: multiplied
   if (!works) return;
-  // acc[rb][tb]: lane holds ranks 16 rb + 4 lg .. + 3 of token lr of the block
+  // acc[.][rb][tb]: lane holds ranks 16 rb + 4 lg .. + 3 of token lr of the block
 #pragma unroll
   for (int rb = 0; rb < BR; ++rb)
 #pragma unroll
     for (int tb = 0; tb < BT; ++tb) {
       const int tok = (wt * BT + tb) * 16 + lr, r = (wr * BR + rb) * 16 + 4 * lg;
-      if (tok < m && r < r_all) *reinterpret_cast<f32x4*>(dst + tok * hrow + r) = acc[rb][tb];
+      if (tok < m && r < r_all) *reinterpret_cast<f32x4*>(dst + tok * hrow + r) = acc[0][rb][tb] + acc[1][rb][tb];
     }
 }
 

@@ -196,13 +196,13 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
   auto batches = [&](auto act_tag) {
   constexpr bool ACT = decltype(act_tag)::value;
   Pack8 xa[KS], xb[KS];
-  f32x4 acc[RB];
+  f32x4 acc[2][RB];
   const T* A = static_cast<const T*>(sl.a[slice]) + aoff;
   request_slab(A);
   if (ACT) request_x(xa, 0);
   MLORA_STAMP(3);  // shrink: first slab and first x batch requested (the token rows are here)
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int rb = 0; rb < RB; ++rb) acc[0][rb] = acc[1][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Two x buffers, one slab per batch.  A batch that has a successor (MORE) requests the
   // successor's x batch, waits for its own slab alone, and requests the successor's slab
   // after the barrier; the last batch of the K part is a copy of its own without those
@@ -228,10 +228,13 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
           const int rr = rb * 16 + lr;
           Pack8 aw;
           aw.raw = *reinterpret_cast<const i32x4*>(&s_a[(rr < R ? rr : R - 1) * ASTRIDE + i * 32 + lg * 8]);
-          acc[rb] = Mma<T>::run(aw, cur[i], acc[rb]);
+          acc[i & 1][rb] = Mma<T>::run(aw, cur[i], acc[i & 1][rb]);
         }
       }
-      if constexpr (MASKED && !MORE) mfma_settle(acc);  // rank blocks were skipped by branches
+      if constexpr (MASKED && !MORE) {  // rank blocks were skipped by branches
+        mfma_settle(acc[0]);
+        mfma_settle(acc[1]);
+      }
     }
   };
   int b = 0;
@@ -246,7 +249,9 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
     batch(std::false_type{}, xa, xb, b);
   }
   MLORA_STAMP(5);  // shrink: multiplied
-  if (ACT) write_partials(acc);
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) acc[0][rb] += acc[1][rb];
+  if (ACT) write_partials(acc[0]);
   };
   if (active) batches(std::true_type{});
   else batches(std::false_type{});
