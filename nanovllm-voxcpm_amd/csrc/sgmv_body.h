@@ -15,7 +15,6 @@ MLORA_TRACE_DECL
 
 constexpr int kMaxSplits = 64;
 constexpr int kExpandWaves = 4;
-constexpr int kSlabStages = 4;  // 128-byte pieces of K in a part of slab.hip's at least
 // Bytes of y from which on the expand launch touches it with the non-temporal hint.  The line is drawn between a launch that has
 // written y and one that reads it, as in a model, for what the hint saves here (y evicts neither A nor B nor the sums) it costs there: what
 // the writer left in the memory-side cache and what the reader would find in it.  gate_up, us, plain and what the hint adds, in a matrix product +
@@ -744,25 +743,17 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
   while (ksplit > 1 && a->k % (unit * ksplit) != 0) --ksplit;
   s.ksplit = ksplit;
   s.krange = a->k / ksplit;
-  // Which shrink.  Up to rank 32 the one whose wavefronts have rings of their own (slab.hip): down, us per call, that / the shared ring of
-  // sgmv.hip, each in its best parts: rank 16, K = 8192, 3500 tokens 24.5 / 25.4, 7500 47.4 / 48.4, rank 32 25.8 / 27.3 and 51.6 / 52.2; K = 4096, rank 8, 6500 23.9 /
-  // 24.0, rank 32, 3500 17.9 / 17.0.  At rank 64 its stages are 16 KB a wavefront, of which one is on its way: 7000 tokens 30.2 / 29.4, K = 8192
-  // 54.6 / 52.1, gate_up 63.5 / 62.7, K = 2048 3500 tokens 72 / 67, three slices 2500 23.6 / 21.9.
-  // (Whoever asks for the two-launch form by name gets the shrink whose sums the one-launch form repeats bit by bit:
-  // slab.hip adds K up in another order.)
-  s.slab = !one_launch && exact_rank(a->r) && slab_supported(a) &&
-           (sgmv_knobs().slab == 2 || (sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && a->r <= 32));
-  // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens; where the host did not count
-  // those, per slot): while an XCD's workgroups number no more than its 32 compute units (a second
-  // round loses: 5200 tokens of 2 slots, K = 2560, two parts 29.8 us, three, 33 workgroups on some XCDs, 33.2) and it cuts K into more parts
-  // than the other shrink, whose parts have to divide K (with two slices into as many).  us per call, the other shrink / this, 2 slots: K = 2560,
-  // 4096 tokens 32.9 / 25.6; K = 3072, 3600 27.9 / 25.9; K = 5120, 4096 28.1 / 23.2; two slices, K = 2560, 6400 52.7 / 51.9; 498 such
-  // calls of 2 to 16 slots, K 1536 to 5120, take 0.65 to 0.99 of the other's time.  With fewer parts the other, which cuts K by rounds below, is the
-  // faster one (K = 4096, 4500 tokens 22.4, K = 8192 38.0, against 21.4 and 39.1 in these rings on full batches, and where a quarter to three quarters of the tokens
-  // have no adapter 124 of 171 such calls were slower in these).  Not for
-  // parts that would be longer than 2800 columns nor below half a
-  // round, and not for short segments: 100 slots of ranks 8 to 64, K = 4096, 2000 tokens 23.2 / 25.7.
-  // Its error against 64 bits is the smaller one (rms of the intermediate, K = 2560 3.3e-7 / 1.7e-7).
+  // Which shrink.  The one of sgmv.hip, whose wavefronts share a ring, except as below: where slab.hip, whose wavefronts have rings of their own, was
+  // taken (up to rank 32, and by parts of its own), it takes 1.020 of that time (876 random calls; K = 8192, rank 32, 5051 tokens 42.0 / 39.4).  The best
+  // of one to four parts of each, the shared ring's time over the other's, K below 1100 / 2100 / 4200 / beyond, rank 8 0.996 / 0.996 / 0.984 / 0.956, rank 16
+  // 0.992 / 0.993 / 0.981 / 0.958, rank 32 0.976 / 0.980 / 0.977 / 0.972, rank 64 0.958 / 0.965 / 0.965 / 0.962 (3980 calls).
+  // (MLORA_SLAB=2 takes slab.hip also by name.)
+  s.slab = !one_launch && exact_rank(a->r) && slab_supported(a) && sgmv_knobs().slab == 2;
+  // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens) while an XCD's workgroups number no more than its 32
+  // compute units and slab.hip then cuts K into more parts than divide it (with two slices into as many), none longer than 2800 columns.  The line is from when the
+  // other shrink's parts had to divide K (2 slots, K = 2560, 4096 tokens 32.9 / 25.6 us, K = 3072, 3600 27.9 / 25.9, K = 5120, 4096 28.1 / 23.2).
+  // In its parts of today that shrink takes 0.967 of the time on such calls (42, K 1536 to 5632, 0.87 to 1.14); tests/test_gpu_slab_rank64.py
+  // holds AUTO to the line.
   int round_parts = 0;
   if (!one_launch && !s.slab && sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 &&
       batch.tokens / batch.slots >= 4 * MLORA_TILE_BIG) {
@@ -777,42 +768,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
       s.slab = true;
     }
   }
-  if (s.slab) {
-    // About 205 workgroups (parts need not be a power of two), a stage of K per wavefront at least.  Measured, us
-    // per call with one / two / three / four parts, rank 32: down (K = 4096) of 2000 tokens 20.8 / 15.7 / 14.0 / 13.4,
-    // of 4000 22.3 / 17.5 / 16.6 / 18.1, of 5000 23.4 / 18.5 / 20.8 / 19.2, of 6500 29.6 / 22.4 / 25.0 / 23.1; K = 8192,
-    // 4000 tokens 48.8 / 37.5 / 32.0 / 36.1; o of 2000 tokens 12.7 / 11.6 / 11.3 / 11.1; gate_up of 6500 56.5 / 57.0 / 58.3.
-    // Long K is cut further: a workgroup's two wavefronts walk 2048 columns in about the time the rest of a tile takes, and
-    // uncut parts lose to the other shrink (sgmv.hip's / one / two / three / four parts, rank 16: K = 4096, 8200 tokens of 6
-    // slots 31.4 / 34.0 / 31.4 / 29.1 / 29.8, of 9392 33.8 / 37.9 / 35.8 / 33.1 / 34.0, of 9392 of 32 slots 34.3 / 38.5 / 36.6 /
-    // 37.4 / 35.0, of 12000 38.1 / 44.7 / 40.1 / 41.6 / 39.2; K = 8192, 5500 tokens 41.5 / 51.5 / 42.9 / 43.0 / 39.4, 7000 45.6 /
-    // 55.4 / 49.7 / 47.2 / 45.2, 9392 61.4 / 67.5 / 70.2 / 58.8 / 60.5; rank 32 alike): four parts where one would be
-    // taken from K = 4096 on, and from K = 8192 on throughout.
-    ksplit = sgmv_knobs().ksplit;
-    if (ksplit <= 0 && round_parts > 0) {
-      ksplit = round_parts;
-    } else if (ksplit <= 0) {
-      const int units = est_tiles * a->num_slices;
-      ksplit = (205 + 2 * units / 5) / units;
-      if (a->k >= 8192 || (a->k >= 4096 && ksplit <= 1)) ksplit = kMaxKSplit;
-      if (ksplit < 1) ksplit = 1;
-      if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
-      while (ksplit > 1 && a->k / 64 < ksplit * kSlabStages) --ksplit;
-      // Unless other parts leave fewer columns to the compute unit with the most workgroups (below): rank 16, K = 8192, 4500 tokens 35.7 us in four
-      // parts (three rounds of a quarter where the last is nearly empty), 31.6 in three; 9000 59.8 / 56.5; K = 4096, 9000 34.0 / 33.1, 4000 18.0 / 17.4 in four.
-      if (a->num_slices == 1) {
-        const int tiles = big_tiles_about(batch);
-        auto columns = [&](int p) { return (static_cast<long long>(tiles) * p + 255) / 256 * (a->k / p); };
-        for (int p = 1; p <= kMaxKSplit && a->k / 64 >= p * kSlabStages; ++p)
-          if (10 * columns(p) < 9 * columns(ksplit)) ksplit = p;
-      }
-    }
-    if (ksplit > max_parts) ksplit = max_parts;
-    if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
-    s.ksplit = ksplit;
-  }
-
-  if (!one_launch && !s.slab) {
+  if (!one_launch) {
     // The ring's parts need not divide K.  What counts is how many of its workgroups come to a compute unit (rounds_of), times the columns of a part; a
     // part also costs its sums, which every column range reads: as much as 40 columns a slice.  Against the best of one to four parts, each
     // measured, on 5400 calls of K = 384 to 16384, every rank, 200 to 9392 tokens of 1 to 128 slots, this takes 1.008 of the time for one
@@ -826,6 +782,8 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
     if (most > max_parts) most = max_parts;
     if (sgmv_knobs().ksplit > 0) {
       s.ksplit = sgmv_knobs().ksplit < most ? sgmv_knobs().ksplit : most;
+    } else if (round_parts > 0) {
+      s.ksplit = round_parts;
     } else {
       const long long wgs = static_cast<long long>(big_tiles_about(batch)) * a->num_slices;
       double least = 0;

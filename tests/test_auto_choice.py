@@ -56,3 +56,10 @@ def test_as_many_k_parts_as_the_workspace_holds():
     for held in (1, 2, 3):
         room = (held - 4) * 4 * 2200 * 2 * 24  # of four parts
         assert choice(2200, 1920, [7680, 7680], 24, 3, 3, 2200, room)[:2] == ("sgmv", held)
+
+
+@pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
+    (5051, 8192, [2048], 32, 3, 3), (5500, 2048, [8192, 8192], 32, 8, 4), (4000, 1536, [6144, 6144], 32, 40, 3), (6000, 6144, [1536], 32, 8, 4),
+])
+def test_parts_up_to_rank_32_by_the_same_cost(rows, k, widths, rank, slots, parts):
+    assert choice(rows, k, widths, rank, slots, slots, rows)[:2] == ("sgmv", parts) == choice(rows, k, widths, 48, slots, slots, rows)[:2]
