@@ -303,7 +303,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
 // of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
 static bool wide_instead(const MloraAddArgs* a, const Batch& batch) {
-  if (a->num_slices == 2 || (a->num_slices == 1 && a->r <= 16) || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, batch)) return false;
+  if (a->num_slices == 2 || a->r <= 16 || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, batch)) return false;
   int columns;
   return (small_tiles_about(batch) + 7) / 8 * decode_ranges(a, batch, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
 }

@@ -31,7 +31,7 @@ extern "C" int mlora_choice(const MloraAddArgs* a, int32_t active_slots, int32_t
   const Batch batch = batch_of(a, active_slots, active_tokens);
   out[0] = chosen_form(a, batch);
   if (out[0] == MLORA_FORM_SGMV) out[1] = sgmv_parts(a, batch);
-  if (out[0] == MLORA_FORM_WIDE) out[2] = wide_columns(a, batch);
+  if (out[0] == MLORA_FORM_WIDE) out[2] = wide_cut(a, batch).count;
   if (out[0] == MLORA_FORM_MFMA) decode_ranges(a, batch, &out[2]);
   return 0;
 }

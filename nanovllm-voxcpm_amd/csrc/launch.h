@@ -67,6 +67,17 @@ inline double rounds_of(long long workgroups) {
   return 0.5 * (static_cast<double>((workgroups + 255) / 256) + (share > 1 ? share : 1));
 }
 
+// How a launch over 64-token tiles is cut, into `count` K parts or into ranges of `count` columns, and how many columns (of K, of a range) the fullest compute
+// unit then streams.
+struct Cut {
+  int count;
+  double columns;
+};
+int big_tiles_about(const Batch& batch, int tokens);  // 64-token tiles and short segments of a batch with that many tokens with a slot (sgmv.hip)
+Cut ring_cut(const MloraAddArgs* a, const Batch& batch, int most_parts);  // the shrink of two launches (sgmv.hip)
+Cut wide_cut(const MloraAddArgs* a, const Batch& batch);  // both products in one (wide.hip)
+int sgmv_parts(const MloraAddArgs* a, const Batch& batch);  // K parts of launch_sgmv
+
 int small_tiles_about(const Batch& batch);  // 16-token tiles of a batch (api.hip)
 
 // split.hip: the same small tiles, producers and consumers of the intermediate in one launch.
@@ -82,7 +93,6 @@ bool sgmv_supported(const MloraAddArgs* a);
 bool sgmv_workspace_ok(const MloraAddArgs* a);
 size_t sgmv_workspace_bytes(int num_tokens, int num_slices, int r, int dtype);
 int launch_sgmv(const MloraAddArgs* a, const Batch& batch);
-int sgmv_parts(const MloraAddArgs* a, const Batch& batch);  // K parts of that launch
 
 // slab.hip: the shrink launch of that form, operands through LDS by direct loads.
 struct PlanLayout;
@@ -96,9 +106,8 @@ int launch_fused(const MloraAddArgs* a, bool trusted_workspace);
 
 // wide.hip: the same tiles, one launch, one workgroup per (tile, column range) doing both products.
 bool wide_supported(const MloraAddArgs* a);
-bool wide_pays(const MloraAddArgs* a, const Batch& batch);
+bool wide_pays(const MloraAddArgs* a, const Batch& batch);  // against the two launches
 int launch_wide(const MloraAddArgs* a, const Batch& batch);
-int wide_columns(const MloraAddArgs* a, const Batch& batch);  // columns per range of that launch
 
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
 // direct loads; 16- and 32-bit elements.

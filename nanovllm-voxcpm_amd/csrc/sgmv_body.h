@@ -678,11 +678,13 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
   return static_cast<size_t>(num_tokens) * static_cast<size_t>(num_slices) * static_cast<size_t>(r) * sizeof(float);
 }
 
-// About how many 64-token tiles and short segments a batch has: its segments end anywhere inside their last tile.
-inline int big_tiles_about(const Batch& batch) {
-  const int tiles = static_cast<int>((batch.tokens + 31ll * batch.slots) / MLORA_TILE_BIG);
-  return tiles > batch.slots ? tiles : batch.slots;
+// K parts whose sums the workspace holds (one where there is none: wide.hip needs none, the others' launches have made sure of it).
+inline int parts_held(const MloraAddArgs* a) {
+  const size_t held = partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r);
+  return held < 1 ? 1 : held < kMaxKSplit ? static_cast<int>(held) : kMaxKSplit;
 }
+// Of those, and of pieces of 64 columns, the ring's most.
+inline int most_parts(const MloraAddArgs* a) { return a->k / 64 < parts_held(a) ? a->k / 64 : parts_held(a); }
 
 // How a call is cut into work, shared by the two-launch and the one-launch form.
 struct SgmvShape {
@@ -729,8 +731,7 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
   // form, and what the line of slab.hip at rank 64 compares with.  (The ring's are further down.)
   int unit = 512;
   while (unit > 128 && a->k % unit != 0) unit /= 2;
-  int max_parts = static_cast<int>(partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r));
-  if (max_parts < 1) max_parts = 1;  // (wide.hip's cut needs no workspace; the others' launches have made sure of one)
+  const int max_parts = parts_held(a);
   int ksplit = sgmv_knobs().ksplit;
   if (ksplit <= 0) {
     ksplit = 1;
@@ -769,32 +770,8 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
     }
   }
   if (!one_launch) {
-    // The ring's parts need not divide K.  What counts is how many of its workgroups come to a compute unit (rounds_of), times the columns of a part; a
-    // part also costs its sums, which every column range reads: as much as 40 columns a slice.  Against the best of one to four parts, each
-    // measured, on 5400 calls of K = 384 to 16384, every rank, 200 to 9392 tokens of 1 to 128 slots, this takes 1.008 of the time for one
-    // slice, 1.009 for two, 1.020 for three; parts that divide K, as many as powers of two, took 1.122, 1.054 and 1.079 (one
-    // slice, rank 48, K = 2560, 2384 tokens of a slot, one part / four 20.7 / 13.8 us; K = 2048, rank 40, 1436 of 3 13.4 / 9.6).
-    // us per call with one / two / three / four parts, rank 64: K = 4096, 4000 tokens of 3 slots 31.0 / 24.1 / 21.9 / 20.4, 5500 33.5 / 27.4 / 30.3 / 27.5, 7000
-    // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
-    // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
-    // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
-    int most = a->k / 64 < kMaxKSplit ? a->k / 64 : kMaxKSplit;
-    if (most > max_parts) most = max_parts;
-    if (sgmv_knobs().ksplit > 0) {
-      s.ksplit = sgmv_knobs().ksplit < most ? sgmv_knobs().ksplit : most;
-    } else if (round_parts > 0) {
-      s.ksplit = round_parts;
-    } else {
-      const long long wgs = static_cast<long long>(big_tiles_about(batch)) * a->num_slices;
-      double least = 0;
-      for (int p = 1; p <= most; ++p) {
-        const double cost = rounds_of(wgs * p) * a->k / p + 40.0 * a->num_slices * p;
-        if (p == 1 || cost < least) {
-          least = cost;
-          s.ksplit = p;
-        }
-      }
-    }
+    if (sgmv_knobs().ksplit > 0) s.ksplit = sgmv_knobs().ksplit < most_parts(a) ? sgmv_knobs().ksplit : most_parts(a);
+    else s.ksplit = round_parts > 0 ? round_parts : ring_cut(a, batch, most_parts(a)).count;
   }
 
   // expand: consecutive tiles per workgroup (they share their B rows when they share their

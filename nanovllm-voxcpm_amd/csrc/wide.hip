@@ -461,66 +461,48 @@ void wide_trace_set(void* buf) {
 #endif
 }
 
-// Columns of a range.  Wider ranges repeat less of a tile's shrink, narrower ones are more workgroups.  Segments of 128 tokens and more are whole
-// tiles: the width (512, 1024, 2048) whose fullest compute unit has the fewest columns of K and of ranges to stream, two workgroups side by
-// side counted as one after the other.  us per call with 512 / 1024 columns, rank 64, K = 1024, 3 slots: q|k|v 6000 tokens 22.3 / 24.9, 9000
+// Columns of a range.  Wider ranges repeat less of a tile's shrink, narrower ones are more workgroups: the width (512, 1024, 2048) whose fullest compute
+// unit has the fewest columns of K and of ranges to stream, by the tiles the two launches count.  Against the best of the three, each measured, on
+// 4400 calls where this form is a fast one 1.024 of the time, 512 columns throughout 1.10; where nobody counted the tokens with a slot, the mean
+// of all of them and half of them 1.033 (all of them alone 1.046: o of 9392 tokens, a quarter without adapter, rank 64, K = 1024, then takes one range of 1024 columns,
+// 17.0 us for 16.3).  us per call with 512 / 1024 columns, rank 64, K = 1024, 3 slots: q|k|v 6000 tokens 22.3 / 24.9, 9000
 // 34.8 / 26.7, o 13.6 / 17.3 and 22.9 / 18.9; rank 32, 9000 29.7 / 23.0 and 20.0 / 16.5; rank 64, K = 2048, q|k|v 2500 23.9 / 23.1, 4000 30.9 /
-// 25.0, 6000 48.5 / 41.4, o 4000 20.0 / 22.9, 6000 31.9 / 24.2.  Shorter ones are mostly single tiles of a few blocks, which end at
-// different times and fill in behind each other: 1024 once the narrow ranges fill the chip twice over (rank 64, K = 1024, 128 slots, 8192
-// tokens: q|k|v 34.5 / 29.8 with 756 workgroups of 512 columns, 5000 tokens 28.7 / 24.3 with 552, o 19.5 / 24.4 with 378).
-struct WideCut {
-  int columns;
-  long long workgroups;
-  bool short_segments;
-};
-static WideCut wide_cut(const MloraAddArgs* a, const Batch& batch) {
-  const long long segs = batch.slots, n = batch.tokens;
-  const bool short_segments = n < 128 * segs;
-  const long long tiles = short_segments ? (n + 31 * segs) / MLORA_TILE_BIG : n / MLORA_TILE_BIG + segs / 2;
-  auto ranges = [&](int columns) {
-    long long all = 0;
-    for (int i = 0; i < a->num_slices; ++i) all += (a->slices[i].n + columns - 1) / columns;
-    return all;
-  };
-  int best = 512;
-  if (short_segments) {
-    if (tiles * ranges(512) > 512) best = 1024;
-  } else {
-    long long least = 0;
-    for (int columns = 512; columns <= 2048; columns *= 2) {
-      long long widest = 0;
-      for (int i = 0; i < a->num_slices; ++i) {
-        const int n_i = a->slices[i].n < columns ? a->slices[i].n : columns;
-        if (n_i > widest) widest = n_i;
-      }
-      const long long cost = (tiles * ranges(columns) + 255) / 256 * (a->k + widest);
-      if (columns == 512 || cost < least) {
-        least = cost;
-        best = columns;
-      }
+// 25.0, 6000 48.5 / 41.4, o 4000 20.0 / 22.9, 6000 31.9 / 24.2; rank 64, K = 1024, 128 slots, 8192
+// tokens: q|k|v 34.5 / 29.8, 5000 tokens 28.7 / 24.3, o 19.5 / 24.4.
+Cut wide_cut(const MloraAddArgs* a, const Batch& batch) {
+  const long long tiles = big_tiles_about(batch, batch.tokens), fewer = batch.tokens_counted ? tiles : big_tiles_about(batch, batch.tokens / 2);
+  Cut best = {512, 0};
+  for (int columns = 512; columns <= 2048; columns *= 2) {
+    long long ranges = 0;
+    int widest = 0;
+    for (int i = 0; i < a->num_slices; ++i) {
+      ranges += (a->slices[i].n + columns - 1) / columns;
+      const int n = a->slices[i].n < columns ? a->slices[i].n : columns;
+      if (n > widest) widest = n;
     }
+    const double streamed = 0.5 * (rounds_of(tiles * ranges) + rounds_of(fewer * ranges)) * (a->k + widest);
+    if (columns == 512 || streamed < best.columns) best = {columns, streamed};
   }
-  return {best, tiles * ranges(best), short_segments};
+  return best;
 }
 
-// Whether this form beats the two-launch one.  What it saves is a launch with its latency from
-// launch to first byte, and the partial sums' trip through the workspace; what it adds is the
-// intake of x and A rows by every column range of a tile beyond the first of its slice.  us per call, this form / two launches, K = 1024
-// (ranges of 512 columns beyond the slices' first: 1), rank 64: q|k|v of 2500, 5000, 7500 tokens of 3 slots 13.8 / 15.7, 18.6 / 21.4, 23.6 / 29.1, of 16 slots 13.6 /
-// 15.9, 20.7 / 21.1, 24.8 / 29.4, o 13.5 / 14.0, 13.6 / 14.4, 13.9 / 15.7; gate_up of the prefill (14) 69.7 / 54.0 at rank 48: taken while the repeats
-// are at most 1024 columns of K per tile.  K = 2048 (3 repeats), above rank 16, segments of 128 tokens and more: only where the workgroups
-// fill their rounds of 256, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 / 38.9);
-// q|k|v of 252 25.2 / 30.3 (r 24 22.1 / 25.5), of 436 to 500 37.4 / 39.0, 42.6 / 47.5, 44.6 / 49.8, but of 210 33.9 / 30.9, of 344 42.0 / 33.1, of 404 43.9 / 42.6.
-// K = 4096: never by more than 5 %, and 31.5 / 30.5 at 7500 tokens.
+// Whether this form beats the two-launch one.  What it saves is a launch with its latency from launch to first byte and the partial sums' trip
+// through the workspace, as much as streaming 1100 columns, and the second launch's own stream of y and B; what it adds is the intake of x and A rows by every column
+// range of a tile beyond the first of its slice.  So by what the fullest compute unit streams in either, where the outputs are not wide; these (gate_up) stay with
+// two launches (rank 64, K = 1024, 1100 tokens of 16 slots), and where nobody counted the tokens only repeats of at most 1024 columns of K a tile count.  Against the
+// best cut of either form, outputs not wide, 5100 calls of K 512 to 8192, every rank, 100 to 9392 tokens: 1.030 up to rank 16, 1.022 up to 32,
+// 1.026 up to 64; by the repeats alone 1.037, 1.034, 1.028.  us per call, this form / two launches, rank 64: K = 1024, q|k|v of 2500, 5000, 7500 tokens of 3 slots 13.8 / 15.7, 18.6 / 21.4,
+// 23.6 / 29.1, o 13.5 / 14.0, 13.6 / 14.4, 13.9 / 15.7; K = 2048, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 /
+// 38.9); q|k|v of 252 25.2 / 30.3, of 210 33.9 / 30.9, of 344 42.0 / 33.1.
 bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
-  long long repeats = 0;
-  for (int i = 0; i < a->num_slices; ++i) repeats += (a->slices[i].n + 511) / 512 - 1;
+  long long cols = 0, repeats = 0;
+  for (int i = 0; i < a->num_slices; ++i) {
+    cols += a->slices[i].n;
+    repeats += (a->slices[i].n + 511) / 512 - 1;
+  }
   if (repeats * a->k <= 1024) return true;
-  if (a->k != 2048 || repeats > 3 || a->r <= 16) return false;
-  const WideCut cut = wide_cut(a, batch);
-  if (cut.short_segments) return false;
-  const long long w = cut.workgroups;
-  return (cut.columns == 1024 && w <= 256 && w >= (a->num_slices == 1 ? 156 : 244)) || (a->num_slices > 1 && w > 420 && w <= 512);
+  if (!batch.tokens_counted || cols > 2ll * a->k) return false;
+  return wide_cut(a, batch).columns <= ring_cut(a, batch, most_parts(a)).columns + 1100.0 + 1.2 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
 }
 
 bool wide_supported(const MloraAddArgs* a) {
@@ -530,14 +512,12 @@ bool wide_supported(const MloraAddArgs* a) {
   return true;
 }
 
-int wide_columns(const MloraAddArgs* a, const Batch& batch) { return wide_knobs().nt > 0 ? wide_knobs().nt : wide_cut(a, batch).columns; }
-
 int launch_wide(const MloraAddArgs* a, const Batch& batch) {
   const SgmvShape sh = sgmv_shape(a, batch);
   if (sh.empty) return 0;
   WideLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.big_cap = sh.big_cap;
-  const int nsplit = fill_splits(a, wide_columns(a, batch), l.splits.split);
+  const int nsplit = fill_splits(a, wide_knobs().nt > 0 ? wide_knobs().nt : wide_cut(a, batch).count, l.splits.split);
   l.grid = dim3(8, static_cast<unsigned>(nsplit), static_cast<unsigned>(sh.tiles8));
   if (a->dtype == MLORA_DTYPE_BF16) launch_wide_rank<__bf16>(l);
   else launch_wide_rank<_Float16>(l);

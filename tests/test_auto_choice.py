@@ -44,7 +44,7 @@ def test_nothing_to_do_has_no_form():
 
 
 @pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
-    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (7000, 1536, [1536], 64, 100, 3), (3000, 4096, [16384, 16384], 64, 16, 2),
+    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (3000, 4096, [16384, 16384], 64, 16, 2),
     (9000, 4096, [1024], 64, 3, 3), (2200, 1920, [7680, 7680], 24, 3, 3),
 ])
 def test_k_parts_need_not_divide_k(rows, k, widths, rank, slots, parts):
@@ -63,3 +63,20 @@ def test_as_many_k_parts_as_the_workspace_holds():
 ])
 def test_parts_up_to_rank_32_by_the_same_cost(rows, k, widths, rank, slots, parts):
     assert choice(rows, k, widths, rank, slots, slots, rows)[:2] == ("sgmv", parts) == choice(rows, k, widths, 48, slots, slots, rows)[:2]
+
+
+@pytest.mark.parametrize("rows,k,widths,rank,slots,tokens,columns", [
+    (9392, 1024, [1024], 64, 8, 0, 512),  # nobody counted: half of the tokens may be without adapter, and all the slot ids but one
+    (9392, 1024, [1024], 64, 8, 9392, 1024), (9392, 1024, [1024], 64, 8, 7044, 512),
+    (1000, 1024, [1024, 256, 256], 64, 128, 1000, 512),  # a tile for every slot at least: 512 and 384 workgroups, not 308 and 231
+])
+def test_columns_of_a_range_by_what_is_known(rows, k, widths, rank, slots, tokens, columns):
+    form, _, got = choice(rows, k, widths, rank, slots, slots if tokens else 0, tokens)
+    assert (form, got) == ("wide", columns)
+
+
+@pytest.mark.parametrize("k", [1536, 1792, 2048, 2304, 2560, 3072])
+def test_one_launch_or_two_by_the_same_cost_at_every_k(k):
+    """Over 64-token tiles from one launch to two as the workgroups of 1024 columns spill, wherever K lies."""
+    forms = [choice(rows, k, [k], 64, 3, 3, rows)[0] for rows in range(3000, 9400, 200)]
+    assert "sgmv" in forms and ("wide" in forms) == (k <= 2048), forms
