@@ -368,20 +368,26 @@ int big_tiles_about(const Batch& batch, int tokens) {
   return tiles > batch.slots ? tiles : batch.slots;
 }
 
-// The ring's parts need not divide K.  What counts is how many of its workgroups come to a compute unit (rounds_of), times the columns of a part; a
-// part also costs its sums, which every column range reads: as much as 40 columns a slice.  Against the best of one to four parts, each
-// measured, on 5400 calls of K = 384 to 16384, every rank, 200 to 9392 tokens of 1 to 128 slots, this takes 1.008 of the time for one
-// slice, 1.009 for two, 1.020 for three; parts that divide K, as many as powers of two, took 1.122, 1.054 and 1.079 (one
+// The ring's parts need not divide K.  What counts is how many of its workgroups come to a compute unit of the fullest XCD, whose block of the tile list
+// is whole runs (big_tile_run: 81 tiles of three slots are runs of 11, and three parts of them 33 workgroups on 32 compute units: K = 8192, rank 32, 5051
+// tokens 43.7 us, in four parts 40.8), times the columns of a part.  A part also costs its sums, which every column range of the second launch
+// reads: as much as 40 columns a slice and, by tiles x columns of the outputs, 0.3 r / (r + 64) a range (gate_up of 9392 tokens, a quarter without adapter, rank 64, one / three parts 62.9 / 67.6).
+// Against the best of one to four parts, each measured, on 5800 calls of K = 384 to 16384, every rank, 200 to 9392 tokens of 1 to 128 slots, this takes 1.010 of
+// the time for one slice, 1.004 for two, 1.012 for three; parts that divide K, as many as powers of two, took 1.122, 1.054 and 1.079 (one
 // slice, rank 48, K = 2560, 2384 tokens of a slot, one part / four 20.7 / 13.8 us; K = 2048, rank 40, 1436 of 3 13.4 / 9.6).
 // us per call with one / two / three / four parts, rank 64: K = 4096, 4000 tokens of 3 slots 31.0 / 24.1 / 21.9 / 20.4, 5500 33.5 / 27.4 / 30.3 / 27.5, 7000
 // 35.1 / 29.7 / 31.9 / 29.4, 9000 42.7 / 45.6 / 39.1 / 41.3; K = 8192, 5500 58.9 / 45.5 / 51.3 / 47.2, 7000 63.8 / 52.1 / 57.3 / 54.1, 9000 72.4 / 77.4 / 64.9 / 69.4; gate_up, K = 1024,
 // 2500 34.6 / 33.1 / 34.9 / 34.0, 4000 43.4 / 41.9 / 44.0 / 44.8, 5500 52.6 / 54.4, 7000 62.7 / 65.4; K = 2048, 1500 42.2 / 38.5 / 37.5 / 37.0, 2500 56.6 / 52.3
 // / 54.9 / 54.9, 4000 77.0 / 73.9 / 76.9 / 77.1.
 Cut ring_cut(const MloraAddArgs* a, const Batch& batch, int most_parts) {
-  const long long wgs = static_cast<long long>(big_tiles_about(batch, batch.tokens)) * a->num_slices;
+  const int tiles = big_tiles_about(batch, batch.tokens), run = big_tile_run(tiles, batch.slots < tiles ? batch.slots : tiles);
+  const long long wgs = static_cast<long long>((tiles + 8 * run - 1) / (8 * run)) * 8 * run * a->num_slices;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  const double sums = 40.0 * a->num_slices + 0.3 * a->r / (a->r + 64) * tiles * cols / 512;
   Cut best = {1, 0};
   for (int p = 1; p <= most_parts; ++p) {
-    const double columns = rounds_of(wgs * p) * a->k / p + 40.0 * a->num_slices * p;
+    const double columns = rounds_of(wgs * p) * a->k / p + sums * p;
     if (p == 1 || columns < best.columns) best = {p, columns};
   }
   return best;

@@ -502,7 +502,7 @@ bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
   }
   if (repeats * a->k <= 1024) return true;
   if (!batch.tokens_counted || cols > 2ll * a->k) return false;
-  return wide_cut(a, batch).columns <= ring_cut(a, batch, most_parts(a)).columns + 1100.0 + 1.2 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
+  return wide_cut(a, batch).columns <= ring_cut(a, batch, most_parts(a)).columns + 1100.0 + 1.0 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
 }
 
 bool wide_supported(const MloraAddArgs* a) {

@@ -44,7 +44,7 @@ def test_nothing_to_do_has_no_form():
 
 
 @pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
-    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (3000, 4096, [16384, 16384], 64, 16, 2),
+    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (3000, 4096, [16384, 16384], 64, 16, 3),
     (9000, 4096, [1024], 64, 3, 3), (2200, 1920, [7680, 7680], 24, 3, 3),
 ])
 def test_k_parts_need_not_divide_k(rows, k, widths, rank, slots, parts):
@@ -59,7 +59,7 @@ def test_as_many_k_parts_as_the_workspace_holds():
 
 
 @pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
-    (5051, 8192, [2048], 32, 3, 3), (5500, 2048, [8192, 8192], 32, 8, 4), (4000, 1536, [6144, 6144], 32, 40, 3), (6000, 6144, [1536], 32, 8, 4),
+    (5051, 8192, [2048], 32, 3, 3), (4000, 1536, [6144, 6144], 32, 40, 1), (6000, 6144, [1536], 32, 8, 4),
 ])
 def test_parts_up_to_rank_32_by_the_same_cost(rows, k, widths, rank, slots, parts):
     assert choice(rows, k, widths, rank, slots, slots, rows)[:2] == ("sgmv", parts) == choice(rows, k, widths, 48, slots, slots, rows)[:2]
@@ -80,3 +80,20 @@ def test_one_launch_or_two_by_the_same_cost_at_every_k(k):
     """Over 64-token tiles from one launch to two as the workgroups of 1024 columns spill, wherever K lies."""
     forms = [choice(rows, k, [k], 64, 3, 3, rows)[0] for rows in range(3000, 9400, 200)]
     assert "sgmv" in forms and ("wide" in forms) == (k <= 2048), forms
+
+
+def test_sums_that_many_ranges_read_have_their_price():
+    assert choice(9392, 1024, [4096, 4096], 64, 8)[:2] == ("sgmv", 1) == choice(9392, 1024, [4096, 4096], 64, 8, 8, 7044)[:2]
+    assert choice(9392, 4096, [1024], 64, 8, 8, 7044)[:2] == ("sgmv", 2)
+
+
+def test_parts_fit_the_fullest_xcd():
+    # 82 tiles of three slots: runs of 11 a block, 33 workgroups in three parts on 32 compute units
+    assert choice(5160, 8192, [2048], 32, 3, 3, 5160)[:2] == ("sgmv", 4)
+    assert choice(5000, 8192, [2048], 32, 3, 3, 5000)[:2] == ("sgmv", 3)
+
+
+@pytest.mark.parametrize("slots", [1, 5, 100, 1000])
+def test_more_slot_ids_than_tiles(slots):
+    for rows in (1, 40, 700, 3000):
+        choice(rows, 2048, [2048, 2048], 64, slots)
