@@ -117,45 +117,44 @@ const ApiKnobs& knobs() {
 
 }  // namespace
 
+static bool slot_major_pays(const MloraAddArgs* a, const Batch& batch);
+
 // Fewer than sixteen tokens to a slot that has any: one small tile each.
 static bool short_segments(const Batch& batch) { return batch.tokens < 16ll * batch.slots; }
 
-// Where the one-launch form over 16-token tiles stops paying.  Its cost per token grows with the
+// Where 16-token tiles stop paying.  Their cost per token grows with the
 // rank (every tile fetches A[slot] and B[slot] again, every column range repeats its tile's shrink)
-// while a two-launch call pays about 10 us before it moves any data (3.5 us for one launch over
-// small tiles).  Measured per projection shape on prefill batches of 1011..9392 tokens (1..16
-// sequences, up to 8 adapters), the two forms meet where tokens x width reaches about 1.5e7-1.7e7
-// at rank 64, 2.6e7 at rank 32 and 8.3e7 at rank 16, with width = slices x K x max(1, K / 1024) +
-// columns x max(1, columns / 4096): long K and wide outputs cost the small tiles more than their
-// share (tokens at the crossing, rank 64 / 32 / 16: qkv 4000 / 6000 / 19000, o 8300 / 12700 / -,
-// gate_up 900 / 1400 / 4500, down 1000 / 1500 / 4800).
-// The rank-64 limit is 1.5e7: with many adapters in the batch the small tiles lose earlier (the
-// mixed batch, 8192 tokens and 128 adapters: o 28.8 us per call on small tiles, 23.0 in two launches).
-// Where the other form would be the one-launch form over 64-token tiles (`one_launch`), which
-// pays about half as much before it moves data, the small tiles lose earlier: measured on the same
-// batches, us per call over small tiles / in one launch over 64-token tiles, by tokens of the batch:
-// rank 64, qkv: 14.8 / 14.3 at 1620, 15.4 / 14.6 at 2098, 18.0 / 15.0 at 3250, 21.2 / 15.5 at 4511;
-// o: 10.5 / 14.8 at 4511, 18.1 / 15.2 at 6648; rank 32, qkv: 11.5 / 12.3 at 3250, 14.4 / 12.8 at 4511;
-// o: 12.4 / 12.6 at 6648, 13.9 / 14.8 at 9392: the limits are 0.65 times the above there.
-// Ranks 24 and 32 lose from 4500 tokens on there (o, K = 1024, 4000 / 5000 / 6000 tokens of 3 slots 7.7 / 10.2, 12.4 / 10.2, 12.3 / 10.2; of 64 slots 4000
-// 11.1 / 10.5, 6500 17.4 / 13.2; rank 24 12.4 / 11.0 at 6500): 0.36 times.  And at K = 2048, where the two launches' shrink has become faster, above
-// rank 16: us per call over small tiles (one or two launches) / in two over 64-token tiles, o of 1500, 2500 tokens of 3 slots, rank 24 11.8 / 11.5, 14.4 / 12.2, rank 32 8.7 /
-// 11.8, 14.8 / 12.3, of 16 slots 13.5 / 11.8, 16.0 / 12.3 and 10.2 / 11.9, 16.5 / 12.3; rank 48, 1000 and 1500 of 16 13.0 / 14.2, 16.4 / 14.3, rank 64, 1500
-// 18.6 / 14.3; q|k|v, 1000 and 1500 of 16, rank 24 14.8 / 12.6, 19.0 / 13.3, rank 32, 740 (of 986, the others without an adapter: tokens with a slot are what counts) 8.1 / 11.3, 1500 18.2 / 13.4.  Segments of fewer than 16 tokens are what
-// the small tiles are for (1000 tokens of 64 slots, rank 32, q|k|v 13.3 / 19.2): these lines are not drawn for them.
+// while 64-token tiles pay more before they move any data (one launch over small tiles 3.5 us, two
+// about 10).  The forms meet where tokens (with a slot) x width does not depend on the shape: width = slices x K x max(1, K / 1024) +
+// columns x max(1, columns / 4096), for long K and wide outputs cost the small tiles more than their share.  What it does depend on: whether the
+// small tiles' kernel asks for all of K at once (decode_one_batch) or walks K batch by batch (above rank 16 the pair stands in for it then), and whether the other form
+// is one launch (`one_launch`), which pays about half as much before it moves data.  The lines lie where 22166 random calls (K 512 to
+// 16384, every rank, 100 to 9392 tokens of 1 to 128 slots, even and uneven, up to half of the tokens without adapter) take the least time together, and they are flat there: time of the forms on the lines' sides over the
+// fastest form's, on gate_ups by two launches, at 7e6, 1e7, 1.4e7, 1.8e7, 2.2e7, 2.6e7: rank 24 all of K at once 1.033, 1.019, 1.017, 1.017, 1.019, 1.017, batch by batch 1.039, 1.047, 1.061, 1.078, 1.102,
+// 1.120; rank 32 1.029, 1.023, 1.024, 1.027, 1.034, 1.036 and 1.025, 1.037, 1.059, 1.081, 1.107, 1.129; rank 64 1.023, 1.033, 1.057, 1.079, 1.102, 1.126 and 1.037, 1.070, 1.107, 1.151, 1.170, 1.208; one slice with outputs
+// that are not wide at 5.5e6, 7.7e6, 1e7, 1.3e7: ranks 24 and 32, K 1100 to 1700 1.034, 1.047, 1.053, 1.061, 1700 to 1950 1.066, 1.065, 1.072, 1.088, 2100 to 3000 1.083, 1.082, 1.089, 1.101, above rank 32 1.079, 1.093,
+// 1.113, 1.141, 1.099, 1.098, 1.108, 1.119 and 1.014, 1.013, 1.013, 1.011; K = 2048 and rank 32, all of K at once, at 1e7, 1.3e7, 1.7e7, 2.1e7 1.027, 1.019, 1.029, 1.031.  Against one launch, us per call over
+// small tiles / 64-token tiles, K = 1024: rank 64, q|k|v 14.8 / 14.3 at 1620 tokens, 18.0 / 15.0 at 3250; o 10.5 / 14.8 at 4511, 18.1 / 15.2 at 6648; rank 32, o of 3 slots 7.7 / 10.2 at
+// 4000, 12.4 / 10.2 at 5000; up to rank 16 they meet at 19000 tokens for q|k|v, 4500 for gate_up, 4800 for down of K = 4096.
 // MLORA_SMALL_BATCH_TOKENS, when set, replaces the rule by a plain token count.
+static double small_work(const MloraAddArgs* a, const Batch& batch) {
+  double cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  return batch.tokens * (static_cast<double>(a->num_slices) * a->k * (a->k > 1024 ? a->k / 1024.0 : 1.0) + cols * (cols > 4096 ? cols / 4096.0 : 1.0));
+}
 static bool small_batch(const MloraAddArgs* a, bool one_launch, const Batch& batch) {
   const int fixed = knobs().small_batch_tokens;
   if (fixed > 0) return a->num_tokens <= fixed;
-  double cols = 0;
-  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  const double width = static_cast<double>(a->num_slices) * a->k * (a->k > 1024 ? a->k / 1024.0 : 1.0) + cols * (cols > 4096 ? cols / 4096.0 : 1.0);
-  double limit = (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) * (one_launch ? 0.65 : 1.0);
-  if (a->r > 16 && !short_segments(batch)) {
-    if (one_launch && a->r <= 32) limit = 0.36 * 2.6e7;
-    else if (!one_launch && a->k == 2048 && cols <= 2.0 * a->k && (a->r <= 32 || a->num_slices == 1)) limit = a->r > 32 ? 7.7e6 : a->num_slices > 1 && exact_rank(a->r) ? 1.7e7 : 1.3e7;
-  }
-  return batch.tokens * width <= limit;
+  const bool whole = decode_one_batch(a);
+  double limit;
+  if (a->r <= 16) limit = (whole ? 8.3e7 : 3.5e7) * (one_launch ? 0.65 : 1.0);
+  else limit = one_launch ? 9.4e6 : !whole ? 8.5e6 : a->r <= 32 ? 2.1e7 : 1.1e7;
+  return small_work(a, batch) <= limit;
+}
+// Over the slots with K shared out (slot.hip) small tiles pay for longer (25 such calls between the lines: 0.872 of the time; K = 4096, rank 32, 558 tokens of 25 slots 7.1 / 11.2).
+static bool small_batch_in_parts(const MloraAddArgs* a, const Batch& batch) {
+  return knobs().small_batch_tokens <= 0 && slot_supported(a) && slot_k_parts(a) > 1 && small_work(a, batch) <= (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) &&
+         slot_major_pays(a, batch);
 }
 
 // About how many 16-token tiles a batch has: its segments end anywhere inside their last tile.
@@ -236,45 +235,33 @@ static bool slot_major_pays(const MloraAddArgs* a, const Batch& batch) {
 //  - one workgroup per (tile, column range): from rank x K = 131072 on (1234 tokens, rank 32, K = 4096: 19.1 /
 //    13.9; it loses below: rank 16, K = 4096, 2000 tokens 11.5 / 12.5, and ties at rank 32, K = 2048), and for
 //    buffers of a rank between the instances', whose code is the general one away from K = 1024 (64 tokens, rank 48, K = 2048:
-//    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9) and which had no form over 64-token tiles (6000
-//    tokens, rank 48: 40.5 / 32.7, 24.3 / 22.6, 115 / 74, 50 / 35; at 1500 tokens and rank 24 qkv and o are
+//    14.5 / 12.1, 12.5 / 9.4, 29.4 / 19.3, 35.7 / 12.9; at 1500 tokens and rank 24 qkv and o are
 //    still the faster ones in one launch: 12.7 / 13.3, 8.1 / 11.2);
-//  - 64-token tiles, where A is as large and the outputs are not wide (rank 64, K = 2048 -> 16384: 32.2 / 33.2 at 1000
-//    tokens): while two K parts of every (tile, slice) find a compute unit, tiles x slices <= 128.  The shrink is
+//  - 64-token tiles, where A is as large (between the instances' ranks from rank x K = 49152 on: K = 3072, rank 24, 1565 tokens 11.9 / 8.3) and the outputs are not
+//    wide: while two K parts of every (tile, slice) find a compute unit, tiles x slices <= 128.  The shrink is
 //    one workgroup per compute unit, and a second round of them costs what the first one does.  64-token tiles /
 //    pair, at 1900 and 2200 tokens of 4 slots (123 and 141 tiles): rank 64, K = 4096 16.8 / 13.1, 17.1 / 19.0, K = 2048
 //    14.9 / 12.8, 15.2 / 17.7, K = 8192 23.4 / 20.0, 24.4 / 29.9; rank 32, K = 4096 12.8 / 11.2, 13.2 / 15.2; rank 16, K =
 //    8192 15.7 / 13.8, 16.5 / 17.2.  At 1300 and 1600 tokens of 100 slots (125 and 144 tiles): rank 64, K = 4096 23.4 / 22.3,
-//    23.7 / 28.5; rank 32, K = 4096 16.0 / 15.3, 16.7 / 18.8.  Two slices, rank 32, K = 4096, 900 and 1300 tokens of 4
-//    slots (58 and 83 tiles): 12.6 / 11.6, 13.0 / 15.5; three, rank 64, K = 2048, 500 and 700 (33 and 46): 14.6 / 12.5,
-//    14.7 / 16.7.  (Below the line batches of 16 to 32 slots and more than about 40 tokens in each lose up to a quarter: rank
-//    64, K = 4096, 32 slots: 14.6 / 16.2 at 700 tokens, 19.2 / 20.1 at 1600; so one slice above rank 16 and segments counted at 16 to 127 tokens stop at 96 tiles: 1500 tokens of 16 and 64 slots, 100
-//    and 121 tiles, 64-token tiles / pair: rank 64, K = 4096 16.1 / 20.1, 19.5 / 25.3, rank 32 13.3 / 15.1, 13.1 / 17.9; K = 2048, rank 64
-//    14.3 / 18.6, 16.4 / 22.9; but 1602 of 16 slots, half of them in one, rank 24 12.5 / 10.9, rank 16, K = 8192, 1500 of 8 15.3 / 13.6.  Between the
-//    instances' ranks, which had no 64-token tiles before, from rank x K = 98304 on: rank 24, K = 4096, 1564  of 3 12.8 / 10.8, 1500 of 16 13.1 / 14.2, and with up to 26 tokens to a slot
-//    (rank 24 and up to 2000 tokens: 34) and 20 MB of weights: half of the tokens in two prompts and the others over 128 slots, two launches over 64-token tiles / pair, gate_up and down of 2500
-//    tokens, rank 24 40.4 / 35.1, 18.0 / 15.1, rank 48 50.5 / 45.8, 20.8 / 17.9, of 3600, rank 24 47.7 / 46.3, 20.3 / 18.7, rank 48 58.0 / 59.9, 22.9 / 21.6;
-//    two slices of K = 2048, up to 1100 tokens in segments of 64 and more: gate_up, rank 24, 520 tokens of 8 of 64 slots 21.5 / 17.4, 820 of 9 21.4 / 18.3, 1000 of 3 27.3 / 24.0, rank 48
-//    32.5 / 30.7, 600 17.2 / 18.3; beyond, 1500 32.3 / 33.5 and 37.3 / 41.4, shorter, 1000 of 16 25.3 / 27.0 and 29.0 / 35.4);
-//  - segments of fewer than 16 tokens with many weights (the slots' A and B in all), each of which passes once through either
-//    form: 64-token tiles where they are 40 MB, one launch over small tiles where they are 60 MB and the outputs wide.  us per call without / with,
-//    128 slots: gate_up, K = 1024, rank 64, 600, 1000, 1500 tokens 43.9 / 36.5, 47.2 / 38.1, 50.8 / 40.6, rank 32 27.7 / 23.6, 29.3 / 24.6, 36.2 / 26.6, rank 16 (42 MB) 16.8 /
-//    17.5, 18.6 / 18.7, 21.5 / 20.9; K = 2048, rank 64 84.6 / 65.9, 94.2 / 83.0, rank 16 32.7 / 28.2, 51.2 / 39.6; down of 1500, K = 4096, rank 64 27.9 / 22.9, rank 32 20.7 / 16.2, K =
-//    8192, rank 64 54.5 / 40.1; q|k|v, K = 2048, rank 64, 1000 42.1 / 36.6, but rank 32 22.5 / 23.5.  64 slots: gate_up, 600, K = 1024, rank 64 26.2 / 24.2, rank 32 (42
-//    MB) 16.6 / 16.9, rank 48 23.8 / 21.0, rank 24 (31 MB) 15.0 / 15.5; K = 2048, rank 64 49.8 / 39.4, rank 32 33.4 / 25.7.
+//    23.7 / 28.5; rank 32, K = 4096 16.0 / 15.3, 16.7 / 18.8.  (One slice above rank 16 and segments counted at 16 to 127 tokens stop at 96 tiles: 1500 tokens of 16 and 64 slots, 100
+//    and 121 tiles, 64-token tiles / pair: rank 64, K = 4096 16.1 / 20.1, 19.5 / 25.3, rank 32 13.3 / 15.1, 13.1 / 17.9);
+//  - wide outputs above rank 16: while tiles x slices x rank <= 2048, since the tiles' B rows are what the second launch takes in.  Pair's time over
+//    64-token tiles' on random gate_ups of K 1100 to 1950 by tiles x slices (16 to 32, to 48, to 64, to 96): rank 24 0.91, -, -, 0.96, rank 32 0.95, 0.97, -, 1.06,
+//    rank 40 to 56 0.86, 0.95, 0.98, 0.96, rank 64 0.93, 1.07, 1.08, 1.06; beyond K = 2100 rank 40 to 56 0.92, 0.99, 1.12, rank 64 1.08, 1.14;
+//  - segments of few tokens, whose 64-token tiles are mostly copies of their last row: two launches over 64-token tiles up to 22 tokens to a slot that has any (pair's time over theirs
+//    by tokens per slot, below 8, to 16, to 20, to 26, to 34: rank 24 and 32 0.82, 0.86, 0.98, 1.04, 1.08; rank 40 to 56 0.78, 0.82, 1.01, 1.05, 1.06; rank 64 0.86, 0.88, 1.08, 1.12,
+//    1.14; 540 calls); one launch over small tiles below 16, where A and B of the slots are 60 MB and the outputs wide (128 slots, gate_up, K = 1024, rank 64, 600, 1000, 1500 tokens
+//    43.9 / 36.5, 47.2 / 38.1, 50.8 / 40.6; K = 2048, rank 16 32.7 / 28.2, 51.2 / 39.6).  Where nobody counted the slots in use, below 8 tokens to a slot id: with all,
+//    half and a quarter of the ids in use 0.78, 0.78 and 0.93 of 64-token tiles' time, and beyond, up to 16, 0.79, 0.90 and 1.02 (up to rank 16 0.68, 0.70 and 0.80).
 static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
   const long long rk = static_cast<long long>(a->r) * a->k;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const bool few_tokens = short_segments(batch), middling = !few_tokens && batch.slots_counted && a->r > 16 && exact_rank(a->r) && batch.tokens < 128ll * batch.slots;
   const double weights = 2.0 * batch.slots * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
-  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && batch.tokens < (a->r <= 24 || batch.tokens <= 2000 ? 34ll : 26ll) * batch.slots && weights >= 2.0e7) return true;
-  if (few_tokens && ((form == MLORA_FORM_SGMV && weights >= 4.0e7) ||
-                     (form == MLORA_FORM_MFMA && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k)))
-    return true;
-  if (!exact_rank(a->r) && form == MLORA_FORM_SGMV && a->num_slices == 2 && a->k == 2048 && batch.tokens <= 1100 &&
-      batch.tokens >= 64ll * batch.slots)
-    return true;
+  if (form == MLORA_FORM_SGMV && batch.tokens < (batch.slots_counted ? 22ll : a->r <= 16 ? 16ll : 8ll) * batch.slots) return true;
+  if (form == MLORA_FORM_MFMA && batch.tokens < (batch.slots_counted ? 16ll : 8ll) * batch.slots && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k) return true;
+  if (form == MLORA_FORM_SGMV && a->r > 16 && cols > 2ll * a->k && static_cast<long long>(small_tiles_about(batch)) * a->num_slices * a->r <= 2048) return true;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
     case MLORA_FORM_MFMA: {
@@ -286,7 +273,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
     }
     case MLORA_FORM_SGMV:
     case MLORA_FORM_WIDE:
-      return rk >= (exact_rank(a->r) ? 131072 : 98304) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(batch)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
+      return rk >= (exact_rank(a->r) ? 131072 : 49152) && (a->k >= 4096 || cols <= 2ll * a->k) && static_cast<long long>(small_tiles_about(batch)) * a->num_slices <= (a->num_slices == 1 && middling ? 96 : 128);
     default: return false;
   }
 }
@@ -296,8 +283,8 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
 // units of an XCD, they run in two rounds, each of which shrinks its tile anew.  16-token / 64-token tiles, us per call, q|k|v
 // at workgroups per XCD: K = 1024, rank 64: 11.7 / 13.7 at 32, 16.6 / 13.8 at 36, 17.5 / 12.8 at 44, 17.7 / 13.6 at 48; rank
 // 32: 7.5 / 9.3 at 32, 10.4 / 10.9 at 36, 10.9 / 9.1 at 44; K = 768, rank 64: 10.7 / 12.6 at 32, 17.3 / 12.5 at 36; rank 32: 7.0 /
-// 8.7 and 10.9 / 9.9; K = 512, rank 64: 7.7 / 9.7 and 11.8 / 10.8; between the instances' ranks K = 1024, rank 24 8.1 / 10.8 at
-// 36, 12.5 / 10.8 at 48, rank 48 11.4 / 14.6 and 18.0 / 14.6.  One slice, o, K = 1024, in one range of 1024 columns (decode_ranges has made the most of the
+// 8.7 and 10.9 / 9.9; K = 512, rank 64: 7.7 / 9.7 and 11.8 / 10.8; between the instances' ranks the gain begins further on (K = 1024, rank 24 8.1 / 10.8 at
+// 36, 12.5 / 10.8 at 48, rank 48 11.4 / 14.6 and 18.0 / 14.6), but the tiles' number is an estimate: 32 for them too takes no more time than 40, counted or not.  One slice, o, K = 1024, in one range of 1024 columns (decode_ranges has made the most of the
 // ranges): 2800 / 4000 / 4700 tokens of 48 slots rank 64 13.0 / 13.6, 22.8 / 13.6, 23.4 / 14.1, rank 24 8.7 / 10.9, 14.2 / 10.7, 14.7 / 11.0, of 128 slots rank 48 14.2
 // / 12.2, 15.1 / 14.1, 23.3 / 16.2.  With a smaller A the rounds are too short to matter (K = 512,
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
@@ -305,7 +292,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
 static bool wide_instead(const MloraAddArgs* a, const Batch& batch) {
   if (a->num_slices == 2 || a->r <= 16 || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, batch)) return false;
   int columns;
-  return (small_tiles_about(batch) + 7) / 8 * decode_ranges(a, batch, &columns) > (a->num_slices == 1 || exact_rank(a->r) ? 32 : 40);
+  return (small_tiles_about(batch) + 7) / 8 * decode_ranges(a, batch, &columns) > 32;
 }
 
 namespace {
@@ -376,6 +363,7 @@ int mlora::chosen_form(const MloraAddArgs* a, const Batch& batch) {
     // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches; rank 24, 36 / 16 / 39 / 104 and 9.5 / 9.2 / 10.7 /
     // 10.9, rank 56, 81 / 80 / 90 / 243 and 12.6 / 12.1 / 14.3 / 15.5, one token of rank 24 15.3 / 15.4 / 15.8 / 43 and 8.5 / 8.5 / 9.2 / 9.9)
     if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
+    else if (small_tiles && small_batch_in_parts(a, batch)) form = MLORA_FORM_SPLIT;
     else if (one_launch && !(small_tiles && small_batch(a, true, batch))) form = MLORA_FORM_WIDE;
     else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, batch))) form = MLORA_FORM_SGMV;
     else if (small_tiles) form = MLORA_FORM_SPLIT;

@@ -341,6 +341,12 @@ int decode_ranges(const MloraAddArgs* a, const Batch& batch, int* columns) {
   return total;
 }
 
+// Whether there is an instance that asks for all of this K at once (launch_kspw); the general text walks K batch by batch.
+bool decode_one_batch(const MloraAddArgs* a) {
+  if (a->k == 1024) return true;
+  return exact_rank(a->r) && (a->k == 256 || a->k == 512 || (a->k == 2048 && a->r <= 32) || ((a->k == 3072 || a->k == 4096) && a->r <= 16));
+}
+
 // Nothing in the kernel limits the size of x or y.
 bool decode_supported(const MloraAddArgs*) { return true; }
 

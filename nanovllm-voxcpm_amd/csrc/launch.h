@@ -51,6 +51,7 @@ int launch_bgmv(const MloraAddArgs* a, bool include_long);
 
 // decode.hip: the same small tiles with both products on the matrix cores, one workgroup per
 // (tile, column range).
+bool decode_one_batch(const MloraAddArgs* a);  // its wavefronts ask for all of their K at once
 bool decode_supported(const MloraAddArgs* a);  // x and y below 2 GiB each
 int launch_decode(const MloraAddArgs* a, bool include_long, const Batch& batch);
 int decode_ranges(const MloraAddArgs* a, const Batch& batch, int* columns);  // column ranges of that launch, and columns per range
@@ -75,7 +76,7 @@ struct Cut {
 };
 int big_tiles_about(const Batch& batch, int tokens);  // 64-token tiles and short segments of a batch with that many tokens with a slot (sgmv.hip)
 Cut ring_cut(const MloraAddArgs* a, const Batch& batch, int most_parts);  // the shrink of two launches (sgmv.hip)
-Cut wide_cut(const MloraAddArgs* a, const Batch& batch);  // both products in one (wide.hip)
+Cut wide_cut(const MloraAddArgs* a, const Batch& batch, int widest_range = 2048);  // both products in one (wide.hip)
 int sgmv_parts(const MloraAddArgs* a, const Batch& batch);  // K parts of launch_sgmv
 
 int small_tiles_about(const Batch& batch);  // 16-token tiles of a batch (api.hip)

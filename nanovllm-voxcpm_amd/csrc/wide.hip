@@ -463,16 +463,27 @@ void wide_trace_set(void* buf) {
 
 // Columns of a range.  Wider ranges repeat less of a tile's shrink, narrower ones are more workgroups: the width (512, 1024, 2048) whose fullest compute
 // unit has the fewest columns of K and of ranges to stream, by the tiles the two launches count.  Against the best of the three, each measured, on
-// 4400 calls where this form is a fast one 1.024 of the time, 512 columns throughout 1.10; where nobody counted the tokens with a slot, the mean
+// 6900 calls where this form is a fast one 1.020 of the time, 512 columns throughout 1.10; where nobody counted the tokens with a slot, the mean
 // of all of them and half of them 1.033 (all of them alone 1.046: o of 9392 tokens, a quarter without adapter, rank 64, K = 1024, then takes one range of 1024 columns,
 // 17.0 us for 16.3).  us per call with 512 / 1024 columns, rank 64, K = 1024, 3 slots: q|k|v 6000 tokens 22.3 / 24.9, 9000
 // 34.8 / 26.7, o 13.6 / 17.3 and 22.9 / 18.9; rank 32, 9000 29.7 / 23.0 and 20.0 / 16.5; rank 64, K = 2048, q|k|v 2500 23.9 / 23.1, 4000 30.9 /
 // 25.0, 6000 48.5 / 41.4, o 4000 20.0 / 22.9, 6000 31.9 / 24.2; rank 64, K = 1024, 128 slots, 8192
 // tokens: q|k|v 34.5 / 29.8, 5000 tokens 28.7 / 24.3, o 19.5 / 24.4.
-Cut wide_cut(const MloraAddArgs* a, const Batch& batch) {
-  const long long tiles = big_tiles_about(batch, batch.tokens), fewer = batch.tokens_counted ? tiles : big_tiles_about(batch, batch.tokens / 2);
+Cut wide_cut(const MloraAddArgs* a, const Batch& batch, int widest_range) {
+  // of `ranges` ranges over the tiles of so many tokens with a slot
+  auto rounds = [&](int tokens, long long ranges) {
+    const int tiles = big_tiles_about(batch, tokens);
+    if (tokens >= 128ll * batch.slots) return rounds_of(tiles * ranges);
+    // Short segments are tiles of any number of tokens, which end at different times and let the next ones in: no whole rounds, and a workgroup of `fill` of a
+    // full one's rows counts for two thirds of those and a third of a full one.
+    const double fill = (a->r + static_cast<double>(tokens) / tiles) / (a->r + MLORA_TILE_BIG), share = tiles * ranges / 256.0 * (1 + 2 * (fill < 1 ? fill : 1)) / 3;
+    return share > 1 ? share : 1.0;
+  };
+  int longest = 0;
+  for (int i = 0; i < a->num_slices; ++i)
+    if (a->slices[i].n > longest) longest = a->slices[i].n;
   Cut best = {512, 0};
-  for (int columns = 512; columns <= 2048; columns *= 2) {
+  for (int columns = 512; columns <= widest_range && (columns == 512 || columns < 2 * longest); columns *= 2) {
     long long ranges = 0;
     int widest = 0;
     for (int i = 0; i < a->num_slices; ++i) {
@@ -480,20 +491,24 @@ Cut wide_cut(const MloraAddArgs* a, const Batch& batch) {
       const int n = a->slices[i].n < columns ? a->slices[i].n : columns;
       if (n > widest) widest = n;
     }
-    const double streamed = 0.5 * (rounds_of(tiles * ranges) + rounds_of(fewer * ranges)) * (a->k + widest);
-    if (columns == 512 || streamed < best.columns) best = {columns, streamed};
+    double streamed = rounds(batch.tokens, ranges);
+    if (!batch.tokens_counted) streamed = 0.5 * (streamed + rounds(batch.tokens / 2, ranges));
+    streamed *= a->k + widest;
+    if (columns == 512 || streamed <= best.columns * (1 + 1e-9)) best = {columns, streamed};  // (of equals the fewer workgroups)
   }
   return best;
 }
 
 // Whether this form beats the two-launch one.  What it saves is a launch with its latency from launch to first byte and the partial sums' trip
-// through the workspace, as much as streaming 1100 columns, and the second launch's own stream of y and B; what it adds is the intake of x and A rows by every column
-// range of a tile beyond the first of its slice.  So by what the fullest compute unit streams in either, where the outputs are not wide; these (gate_up) stay with
+// through the workspace, as much as streaming 1200 columns, and the second launch's own stream of y and B, 1.6 columns for each of its; what it adds is the intake of x and A
+// rows by every column range of a tile beyond the first of its slice, and a stage costs 1.2 of the ring's, which two launches' workgroups fill in fours.  So by what the fullest compute unit
+// streams in either, where the outputs are not wide; these (gate_up) stay with
 // two launches (rank 64, K = 1024, 1100 tokens of 16 slots), and where nobody counted the tokens only repeats of at most 1024 columns of K a tile count.  Against the
-// best cut of either form, outputs not wide, 5100 calls of K 512 to 8192, every rank, 100 to 9392 tokens: 1.030 up to rank 16, 1.022 up to 32,
-// 1.026 up to 64; by the repeats alone 1.037, 1.034, 1.028.  us per call, this form / two launches, rank 64: K = 1024, q|k|v of 2500, 5000, 7500 tokens of 3 slots 13.8 / 15.7, 18.6 / 21.4,
+// best cut of either form this takes 1.018 of the time (8700 calls of K 512 to 16384, every rank, 100 to 9392 tokens, even and uneven, outputs not wide; the repeats alone
+// 1.036).  us per call, this form / two launches, rank 64: K = 1024, q|k|v of 2500, 5000, 7500 tokens of 3 slots 13.8 / 15.7, 18.6 / 21.4,
 // 23.6 / 29.1, o 13.5 / 14.0, 13.6 / 14.4, 13.9 / 15.7; K = 2048, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 /
-// 38.9); q|k|v of 252 25.2 / 30.3, of 210 33.9 / 30.9, of 344 42.0 / 33.1.
+// 38.9); q|k|v of 252 25.2 / 30.3, of 210 33.9 / 30.9, of 344 42.0 / 33.1; 8192 tokens of 126 slots, K = 4096, 55.2 / 40.9.  Ranges of 2048 columns stay out of the comparison: of three slices only the widest fills
+// them (q|k|v that one launch in such ranges would win by its cost took 1.10 of two launches' time).
 bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
   long long cols = 0, repeats = 0;
   for (int i = 0; i < a->num_slices; ++i) {
@@ -502,7 +517,7 @@ bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
   }
   if (repeats * a->k <= 1024) return true;
   if (!batch.tokens_counted || cols > 2ll * a->k) return false;
-  return wide_cut(a, batch).columns <= ring_cut(a, batch, most_parts(a)).columns + 1100.0 + 1.0 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
+  return 1.2 * wide_cut(a, batch, 1024).columns <= ring_cut(a, batch, most_parts(a)).columns + 1200.0 + 1.6 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
 }
 
 bool wide_supported(const MloraAddArgs* a) {

@@ -44,7 +44,7 @@ def test_nothing_to_do_has_no_form():
 
 
 @pytest.mark.parametrize("rows,k,widths,rank,slots,parts", [
-    (2384, 2560, [2560], 48, 1, 4), (1436, 2048, [2048], 40, 3, 4), (3000, 4096, [16384, 16384], 64, 16, 3),
+    (2384, 2560, [2560], 48, 1, 4), (2436, 2048, [2048], 40, 3, 4), (3000, 4096, [16384, 16384], 64, 16, 3),
     (9000, 4096, [1024], 64, 3, 3), (2200, 1920, [7680, 7680], 24, 3, 3),
 ])
 def test_k_parts_need_not_divide_k(rows, k, widths, rank, slots, parts):
@@ -68,7 +68,7 @@ def test_parts_up_to_rank_32_by_the_same_cost(rows, k, widths, rank, slots, part
 @pytest.mark.parametrize("rows,k,widths,rank,slots,tokens,columns", [
     (9392, 1024, [1024], 64, 8, 0, 512),  # nobody counted: half of the tokens may be without adapter, and all the slot ids but one
     (9392, 1024, [1024], 64, 8, 9392, 1024), (9392, 1024, [1024], 64, 8, 7044, 512),
-    (1000, 1024, [1024, 256, 256], 64, 128, 1000, 512),  # a tile for every slot at least: 512 and 384 workgroups, not 308 and 231
+    (1000, 1024, [1024, 256, 256], 64, 128, 1000, 1024),  # a tile for every slot at least: 512 and 384 workgroups, not 308 and 231
 ])
 def test_columns_of_a_range_by_what_is_known(rows, k, widths, rank, slots, tokens, columns):
     form, _, got = choice(rows, k, widths, rank, slots, slots if tokens else 0, tokens)
@@ -97,3 +97,18 @@ def test_parts_fit_the_fullest_xcd():
 def test_more_slot_ids_than_tiles(slots):
     for rows in (1, 40, 700, 3000):
         choice(rows, 2048, [2048, 2048], 64, slots)
+
+
+@pytest.mark.parametrize("k", [1536, 1792, 2048, 2304, 2560, 3072])
+def test_lines_do_not_depend_on_one_k(k):
+    """Small tiles, the pair and 64-token tiles meet at tokens x width and at tokens per slot, whatever K is."""
+    width = k * k / 1024 + k
+    big = ("sgmv", "wide")
+    for rank, limit in ((24, 8.5e6), (48, 8.5e6), (64, 8.5e6), (32, 2.1e7 if k == 2048 else 8.5e6)):
+        more = int(limit / width) + 40
+        assert choice(more, k, [k], rank, 16, 16, more)[0] in big + (("pair",) if more < 1950 else ())  # (128 tiles)
+        assert choice(more - 80, k, [k], rank, 4, 4, more - 80)[0] not in big
+    for rank in (24, 32, 48, 64):
+        assert choice(2400, k, [4 * k, 4 * k], rank, 128, 128, 2400)[0] == "pair"  # 18.75 tokens to a slot
+        assert choice(3000, k, [4 * k, 4 * k], rank, 128, 128, 3000)[0] == "sgmv"
+        assert choice(1000, k, [4 * k, 4 * k], rank, 128, 0, 0)[0] == "pair" and choice(1200, k, [4 * k, 4 * k], rank, 128, 0, 0)[0] != "pair"
