@@ -250,7 +250,8 @@ static bool slot_major_pays(const MloraAddArgs* a, const Batch& batch) {
 //    rank 40 to 56 0.86, 0.95, 0.98, 0.96, rank 64 0.93, 1.07, 1.08, 1.06; beyond K = 2100 rank 40 to 56 0.92, 0.99, 1.12, rank 64 1.08, 1.14;
 //  - segments of few tokens, whose 64-token tiles are mostly copies of their last row: two launches over 64-token tiles up to 22 tokens to a slot that has any (pair's time over theirs
 //    by tokens per slot, below 8, to 16, to 20, to 26, to 34: rank 24 and 32 0.82, 0.86, 0.98, 1.04, 1.08; rank 40 to 56 0.78, 0.82, 1.01, 1.05, 1.06; rank 64 0.86, 0.88, 1.08, 1.12,
-//    1.14; 540 calls); one launch over small tiles below 16, where A and B of the slots are 60 MB and the outputs wide (128 slots, gate_up, K = 1024, rank 64, 600, 1000, 1500 tokens
+//    1.14; 540 calls); one launch over them below 16, unless its ranges repeat little of the shrink (K > 1100, below 8, to 12, to 16, to 22: rank 24 and 32 0.88, 0.88, 1.02, 1.09; rank 40 to 56
+//    0.89, -, 0.78, 1.00; rank 64 0.94, 0.97, 0.94, 0.98; at K = 1024 1.10 and more); one launch over small tiles below 16, where A and B of the slots are 60 MB and the outputs wide (128 slots, gate_up, K = 1024, rank 64, 600, 1000, 1500 tokens
 //    43.9 / 36.5, 47.2 / 38.1, 50.8 / 40.6; K = 2048, rank 16 32.7 / 28.2, 51.2 / 39.6).  Where nobody counted the slots in use, below 8 tokens to a slot id: with all,
 //    half and a quarter of the ids in use 0.78, 0.78 and 0.93 of 64-token tiles' time, and beyond, up to 16, 0.79, 0.90 and 1.02 (up to rank 16 0.68, 0.70 and 0.80).
 static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
@@ -260,6 +261,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
   const bool few_tokens = short_segments(batch), middling = !few_tokens && batch.slots_counted && a->r > 16 && exact_rank(a->r) && batch.tokens < 128ll * batch.slots;
   const double weights = 2.0 * batch.slots * a->r * (static_cast<double>(a->num_slices) * a->k + cols);
   if (form == MLORA_FORM_SGMV && batch.tokens < (batch.slots_counted ? 22ll : a->r <= 16 ? 16ll : 8ll) * batch.slots) return true;
+  if (form == MLORA_FORM_WIDE && few_tokens && batch.slots_counted && !wide_repeats_little(a)) return true;
   if (form == MLORA_FORM_MFMA && batch.tokens < (batch.slots_counted ? 16ll : 8ll) * batch.slots && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k) return true;
   if (form == MLORA_FORM_SGMV && a->r > 16 && cols > 2ll * a->k && static_cast<long long>(small_tiles_about(batch)) * a->num_slices * a->r <= 2048) return true;
   switch (form) {

@@ -107,6 +107,7 @@ int launch_fused(const MloraAddArgs* a, bool trusted_workspace);
 
 // wide.hip: the same tiles, one launch, one workgroup per (tile, column range) doing both products.
 bool wide_supported(const MloraAddArgs* a);
+bool wide_repeats_little(const MloraAddArgs* a);  // of a tile's shrink: at most 1024 columns of K over all its ranges of 512
 bool wide_pays(const MloraAddArgs* a, const Batch& batch);  // against the two launches
 int launch_wide(const MloraAddArgs* a, const Batch& batch);
 

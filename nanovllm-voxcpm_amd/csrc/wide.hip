@@ -509,13 +509,15 @@ Cut wide_cut(const MloraAddArgs* a, const Batch& batch, int widest_range) {
 // 23.6 / 29.1, o 13.5 / 14.0, 13.6 / 14.4, 13.9 / 15.7; K = 2048, o of 158 to 250 workgroups of 1024 columns 24.2 / 26.6, 24.6 / 28.1, 26.7 / 31.3 (with 126 19.3 / 16.9, with 284 37.2 /
 // 38.9); q|k|v of 252 25.2 / 30.3, of 210 33.9 / 30.9, of 344 42.0 / 33.1; 8192 tokens of 126 slots, K = 4096, 55.2 / 40.9.  Ranges of 2048 columns stay out of the comparison: of three slices only the widest fills
 // them (q|k|v that one launch in such ranges would win by its cost took 1.10 of two launches' time).
+bool wide_repeats_little(const MloraAddArgs* a) {
+  long long repeats = 0;
+  for (int i = 0; i < a->num_slices; ++i) repeats += (a->slices[i].n + 511) / 512 - 1;
+  return repeats * a->k <= 1024;
+}
 bool wide_pays(const MloraAddArgs* a, const Batch& batch) {
-  long long cols = 0, repeats = 0;
-  for (int i = 0; i < a->num_slices; ++i) {
-    cols += a->slices[i].n;
-    repeats += (a->slices[i].n + 511) / 512 - 1;
-  }
-  if (repeats * a->k <= 1024) return true;
+  long long cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
+  if (wide_repeats_little(a)) return true;
   if (!batch.tokens_counted || cols > 2ll * a->k) return false;
   return 1.2 * wide_cut(a, batch, 1024).columns <= ring_cut(a, batch, most_parts(a)).columns + 1200.0 + 1.6 * big_tiles_about(batch, batch.tokens) * cols / 256.0;
 }

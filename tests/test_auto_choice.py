@@ -112,3 +112,8 @@ def test_lines_do_not_depend_on_one_k(k):
         assert choice(2400, k, [4 * k, 4 * k], rank, 128, 128, 2400)[0] == "pair"  # 18.75 tokens to a slot
         assert choice(3000, k, [4 * k, 4 * k], rank, 128, 128, 3000)[0] == "sgmv"
         assert choice(1000, k, [4 * k, 4 * k], rank, 128, 0, 0)[0] == "pair" and choice(1200, k, [4 * k, 4 * k], rank, 128, 0, 0)[0] != "pair"
+
+
+def test_few_tokens_a_slot_take_the_pair_unless_one_launch_repeats_little():
+    assert choice(851, 2048, [2048, 512, 512], 48, 117, 88, 851)[0] == "pair"
+    assert choice(1100, 1024, [1024, 256, 256], 64, 128, 128, 1100)[0] == "wide"
