@@ -245,9 +245,10 @@ static bool slot_major_pays(const MloraAddArgs* a, const Batch& batch) {
 //    8192 15.7 / 13.8, 16.5 / 17.2.  At 1300 and 1600 tokens of 100 slots (125 and 144 tiles): rank 64, K = 4096 23.4 / 22.3,
 //    23.7 / 28.5; rank 32, K = 4096 16.0 / 15.3, 16.7 / 18.8.  (One slice above rank 16 and segments counted at 16 to 127 tokens stop at 96 tiles: 1500 tokens of 16 and 64 slots, 100
 //    and 121 tiles, 64-token tiles / pair: rank 64, K = 4096 16.1 / 20.1, 19.5 / 25.3, rank 32 13.3 / 15.1, 13.1 / 17.9);
-//  - wide outputs above rank 16: while tiles x slices x rank <= 2048, since the tiles' B rows are what the second launch takes in.  Pair's time over
-//    64-token tiles' on random gate_ups of K 1100 to 1950 by tiles x slices (16 to 32, to 48, to 64, to 96): rank 24 0.91, -, -, 0.96, rank 32 0.95, 0.97, -, 1.06,
-//    rank 40 to 56 0.86, 0.95, 0.98, 0.96, rank 64 0.93, 1.07, 1.08, 1.06; beyond K = 2100 rank 40 to 56 0.92, 0.99, 1.12, rank 64 1.08, 1.14;
+//  - wide outputs above rank 16: while tiles x slices x rank <= 2048, since the tiles' B rows are what the second launch takes in, and 3600 between the
+//    instances' ranks, whose 64-token tiles take in as many as the next instance's.  Pair's time over 64-token tiles' on random gate_ups by that product (to 1024, 2048, 3000, 4500),
+//    even segments: rank 24 0.87, 0.98, 1.02, 1.03, rank 32 0.92, 1.00, 1.03, 1.09, rank 40 to 56 0.78, 0.90, 0.98, 1.05, rank 64 0.82, 0.97, 1.05, 1.11; a few popular slots: -, 0.94, 0.92, 0.97, -, 0.91,
+//    0.95, 1.03, -, 0.89, 0.89, 0.93, -, -, -, 1.04;
 //  - segments of few tokens, whose 64-token tiles are mostly copies of their last row: two launches over 64-token tiles up to 22 tokens to a slot that has any (pair's time over theirs
 //    by tokens per slot, below 8, to 16, to 20, to 26, to 34: rank 24 and 32 0.82, 0.86, 0.98, 1.04, 1.08; rank 40 to 56 0.78, 0.82, 1.01, 1.05, 1.06; rank 64 0.86, 0.88, 1.08, 1.12,
 //    1.14; 540 calls); one launch over them below 16, unless its ranges repeat little of the shrink (K > 1100, below 8, to 12, to 16, to 22: rank 24 and 32 0.88, 0.88, 1.02, 1.09; rank 40 to 56
@@ -263,7 +264,7 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
   if (form == MLORA_FORM_SGMV && batch.tokens < (batch.slots_counted ? 22ll : a->r <= 16 ? 16ll : 8ll) * batch.slots) return true;
   if (form == MLORA_FORM_WIDE && few_tokens && batch.slots_counted && !wide_repeats_little(a)) return true;
   if (form == MLORA_FORM_MFMA && batch.tokens < (batch.slots_counted ? 16ll : 8ll) * batch.slots && weights >= 6.0e7 && cols >= 2ll * a->num_slices * a->k) return true;
-  if (form == MLORA_FORM_SGMV && a->r > 16 && cols > 2ll * a->k && static_cast<long long>(small_tiles_about(batch)) * a->num_slices * a->r <= 2048) return true;
+  if (form == MLORA_FORM_SGMV && a->r > 16 && cols > 2ll * a->k && static_cast<long long>(small_tiles_about(batch)) * a->num_slices * a->r <= (exact_rank(a->r) ? 2048 : 3600)) return true;
   switch (form) {
     case MLORA_FORM_SPLIT: return true;  // (AUTO keeps the split form for workspaces without room for the pair's partial sums)
     case MLORA_FORM_MFMA: {
