@@ -45,9 +45,12 @@ __device__ __forceinline__ void store128(void* p, i32x4 v) { *reinterpret_cast<i
 // (a copy, the apply and a copy of y, less the copies, us, plain stores / these: 9392 tokens, rank 64, down 30.1 / 28.9; 3001 tokens, rank 16, K = 2048, gate_up
 // 35.0 / 34.1, down 17.9 / 17.4; 1234 tokens, rank 32, gate_up 13.8 / 13.1).  By themselves, us per call: 64-token tiles, 9392 tokens, rank 64, K = 1024, o 15.8 /
 // 14.8, q|k|v 24.0 / 23.0, down 29.1 / 28.3, 3001 tokens, rank 16, K = 2048, gate_up 52.0 / 49.9; 16-token tiles, 3001 tokens q|k|v 14.6 / 14.1, o 10.6 / 10.3.
-// Launches that write less lose the wait for every store, so 16-token tiles take them from kThroughBytes of y on: 1000 tokens, K = 1024, o (2.0 MB) 5.0 / 4.85, gate_up
-// of 120 tokens at K = 2048 (3.9 MB) 6.9 / 6.5; 400 tokens q|k|v (1.2 MB) 4.82 / 4.87, o (0.8 MB) 4.67 / 4.74; one stream's step of 48 calls 158 / 161; 256 streams'
-// and the pair's outputs the same or 1 % slower a step; with K = 4096 over 16-token tiles 2365 tokens of 45 slots, rank 8, 14.2 / 14.8, 1939 of 38, rank 16, 13.0 / 13.8: up to K = 2048.
+// Launches that write less lose the wait for every store, so 16-token tiles take them from kThroughBytes of y on, in instances of their own, up to K = 2048.  Their time over that
+// of plain stores, by themselves, at 0.2 to 0.5, to 1, to 2, to 8 and more MB of y, one slice: up to rank 16 1.010, 0.985, 0.979, 0.974, 0.965, ranks 24 and 32 1.000, 0.992, 0.988, 0.980, 0.985, above 1.002, 0.996, 0.992,
+// 0.983, 0.990; two 0.93, 0.92, 0.943, 0.952, 0.956, 0.985, 0.983, 0.989, 0.966, 0.974, 0.984, 0.982, 0.983, 0.977, 0.987; three up to rank 16 1.002, 0.984, 0.977, 0.980, 0.971, above 0.998, 0.994, 0.992, 1.010, 1.016; between a
+// copy to y and one of y a call of ranks 24 to 64 gains 0.2 to 1.0 us from 2 MB on (three slices lose 0.1 to 0.7), up to rank 16 0.1 to 0.2 us, and from 8 MB on loses 0.1 to 0.3
+// (4200 calls); one stream's step of 48 calls 158 / 161; 256 streams' and the pair's outputs the same or 1 % slower a step; with K = 4096 over 16-token tiles 2365 tokens of 45 slots, rank 8,
+// 14.2 / 14.8, 1939 of 38, rank 16, 13.0 / 13.8.
 constexpr long long kThroughBytes = 2000000;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

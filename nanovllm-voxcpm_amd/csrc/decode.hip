@@ -36,7 +36,6 @@ namespace {
 
 constexpr int kMaxSplits = 32;
 constexpr int kNW = 8;          // wavefronts per workgroup
-constexpr int kThrough = 2;     // bit of include_long: y leaves at once (store_through)
 constexpr int kSpansAheadMax = 2;  // output spans per wavefront whose loads are issued up front (SA: 1 or 2)
 
 MLORA_TRACE_DECL
@@ -75,15 +74,18 @@ struct DecodeSplits {
 // whatever lies beyond rbuf is treated like the ranks beyond an adapter's own (requests clamped
 // into the buffers, values masked).
 // Two workgroups per compute unit (at most 128 registers) where the LDS holds two: up to rank 16 and K = 2048, where the last text alone stays
-// below that by itself and three texts with two spans (rank 8 150 registers, rank 16 146) would not.  us per call with one / two, every tile short, K = 2048,
+// below that by itself and three texts with two spans (rank 8 150 registers, rank 16 146) would not, nor the last with y leaving at once (masked, rank 16, two spans: 129
+// registers, q|k|v of 3001 tokens at K = 2048 17.7 -> 19.5 us).  us per call with one / two, every tile short, K = 2048,
 // rank 8: gate_up of 64 tokens of 32 slots 8.3 / 6.8, of 256 of 64 16.6 / 13.5, q|k|v of 128 of 64 5.4 / 4.8; rank 16: 9.3 / 7.7, 19.1 / 16.2, 6.6 / 6.4.
 // Nothing at K = 3072, rank 8, where the bound spills (o of 16 tokens of 16 slots 4.27 / 4.39).  (Rank 32 in 72 KB, its blocks of A staged one by one, and
 // 128 registers: q|k|v of 1234 tokens at K = 2048 15.4 -> 14.9, but gate_up of 600 at K = 1024 12.5 -> 13.4, o of 2000 8.2 -> 8.7.)
-constexpr int decode_waves(int r, int kspw, bool texts) { return texts && r <= 16 && kspw <= 8 ? 4 : 2; }
+constexpr int decode_waves(int r, int kspw, bool bound) { return bound && r <= 16 && kspw <= 8 ? 4 : 2; }
 
 // SHORT (staged form): with a text each for tiles of up to four, up to eight and more tokens (below); without, the last one alone.
-template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR, bool SHORT>
-__global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT)) void decode_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv,
+// THROUGH (staged form): y leaves at once (store_through), in instances of its own: a branch on it around every store costs calls with plain stores
+// 1 to 3 % (0.1 us; a prompt of 37 tokens, 96 calls, 500 -> 507 us), one around a span's 0.3 to 1 %.
+template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR, bool SHORT, bool THROUGH>
+__global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT || THROUGH)) void decode_kernel(const int32_t* __restrict__ plan, const void* __restrict__ xv,
                                                             void* __restrict__ yv_, int64_t xs, int64_t ys, int small_off,
                                                             int include_long, int T_, int K, int num_slots, float scaling,
                                                             const int32_t* __restrict__ eff_rank, int rbuf_arg, DecodeSplits splits) {
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT)) void deco
   // compiler requests this launch's column range only after the header has arrived)
   __builtin_amdgcn_sched_barrier(0);
   const int slot = rec0[0], m = rec0[1];
-  const int n_tiles = hdr[MLORA_PLAN_TILES_SHORT] + hdr[MLORA_PLAN_TILES_LONG_SMALL] * (include_long & 1);
+  const int n_tiles = hdr[MLORA_PLAN_TILES_SHORT] + hdr[MLORA_PLAN_TILES_LONG_SMALL] * include_long;
   // One exit test, evaluated without short-circuit, that consumes everything fetched above
   // (the token index through its first lane), so that all of it is requested here, together,
   // instead of piece by piece behind a chain of branches.
@@ -198,16 +200,16 @@ __global__ __launch_bounds__(kNW* kWave, decode_waves(R, KSPW, SHORT)) void deco
 
 struct Launch {
   const MloraAddArgs* a;
-  int small_off, include_long, staged, short_tiles;
+  int small_off, include_long, staged, short_tiles, through;
   int widest;  // columns of the widest column range
   dim3 grid;
   const DecodeSplits* splits;
 };
 
-template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR, bool SHORT>
+template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR, bool SHORT, bool THROUGH>
 void launch_texts(const Launch& l) {
   const MloraAddArgs* a = l.a;
-  hipLaunchKernelGGL((decode_kernel<T, R, KSPW, TR, MASKED, SA, GR, SHORT>), l.grid, dim3(kNW * kWave), 0, static_cast<hipStream_t>(a->stream),
+  hipLaunchKernelGGL((decode_kernel<T, R, KSPW, TR, MASKED, SA, GR, SHORT, THROUGH>), l.grid, dim3(kNW * kWave), 0, static_cast<hipStream_t>(a->stream),
                      a->plan, a->x, a->y, a->x_stride, a->y_stride, l.small_off, l.include_long, a->num_tokens, a->k,
                      a->num_slots, a->scaling, a->effective_rank, a->r, *l.splits);
 }
@@ -215,9 +217,12 @@ void launch_texts(const Launch& l) {
 template <typename T, int R, int KSPW, bool TR, bool MASKED, int SA, bool GR = false>
 void launch_spans(const Launch& l) {
   if constexpr (TR) {
-    if (l.short_tiles) return launch_texts<T, R, KSPW, TR, MASKED, SA, GR, true>(l);
+    if (l.short_tiles) return launch_texts<T, R, KSPW, TR, MASKED, SA, GR, true, false>(l);
+    if constexpr (KSPW <= 8) {
+      if (l.through) return launch_texts<T, R, KSPW, TR, MASKED, SA, GR, false, true>(l);
+    }
   }
-  launch_texts<T, R, KSPW, TR, MASKED, SA, GR, false>(l);
+  launch_texts<T, R, KSPW, TR, MASKED, SA, GR, false, false>(l);
 }
 
 // One span per wavefront up front when no column range holds more (staged form; the other form
@@ -397,7 +402,8 @@ int launch_decode(const MloraAddArgs* a, bool include_long, const Batch& batch) 
   l.short_tiles = decode_knobs().short_tiles < 0 ? batch.tokens <= (l.widest <= kNW * 64 ? 12 : 4) * batch.slots : decode_knobs().short_tiles != 0;
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
-  if (decode_knobs().through < 0 ? a->k <= 2048 && batch.tokens * cols * 2 >= kThroughBytes : decode_knobs().through != 0) l.include_long |= kThrough;
+  // (three slices above rank 16 lose by it, q|k|v of 2 to 8 MB 1 %, of more 1.5 %; the line itself stands at store_through)
+  l.through = decode_knobs().through < 0 ? batch.tokens * cols * 2 >= kThroughBytes && (a->num_slices < 3 || a->r <= 16) : decode_knobs().through != 0;
   for (; s < kMaxSplits; ++s) splits.split[s] = DecodeSplit{nullptr, nullptr, 0, 0, 0, 0};
   l.grid = dim3(8, static_cast<unsigned>(total), static_cast<unsigned>(cap / 8));
   const int nks = a->k / 32;

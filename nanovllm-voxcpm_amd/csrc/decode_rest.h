@@ -305,7 +305,7 @@
 #pragma unroll
           for (int j = 0; j < 4; ++j) v.e[j] = from_f32<T>(to_f32(v.e[j]) + out[j][i]);
           T* const to = ycols + static_cast<int64_t>(rows4[i]) * ys + c;
-          if (!SHORT && (include_long & kThrough)) store_through(to, __builtin_bit_cast(u32x2, v.raw));
+          if constexpr (THROUGH) store_through(to, __builtin_bit_cast(u32x2, v.raw));
           else *reinterpret_cast<uint2*>(to) = v.raw;
         }
       }

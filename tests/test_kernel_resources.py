@@ -1,6 +1,7 @@
 """What the built library's own metadata says of its kernels' registers: the small-tile kernel (csrc/decode.hip), whose instances are
 held to a number of registers by their launch bounds, keeps none of them in memory."""
 
+import re
 import struct
 
 import msgpack
@@ -45,3 +46,16 @@ def test_small_tile_kernel_keeps_its_registers():
     decode = {k[".name"]: k for k in _kernels() if "decode_kernel" in k[".name"]}
     assert len(decode) > 100
     assert [n for n, k in decode.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]] == []
+
+
+def test_two_small_tile_workgroups_fit_a_compute_unit():
+    """Up to rank 16 and K = 2048 (four, eight steps of K a wavefront) eight wavefronts hold at most 128 registers each, whatever the instance."""
+    staged = re.compile(r"decode_kernelI\w+?Li(8|16)ELi(4|8)ELb1E")
+    some = {k[".name"]: k[".vgpr_count"] for k in _kernels() if staged.search(k[".name"])}
+    assert len(some) >= 48 and [n for n, v in some.items() if v > 128] == []
+
+
+def test_kernels_over_64_token_tiles_keep_their_registers():
+    some = {k[".name"]: k for k in _kernels() if re.search("wide_kernel|sgmv_shrink_kernel", k[".name"])}
+    assert len(some) == 10
+    assert [n for n, k in some.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"] or k[".vgpr_count"] > 128] == []
