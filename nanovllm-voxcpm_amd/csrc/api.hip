@@ -142,18 +142,18 @@ static double small_work(const MloraAddArgs* a, const Batch& batch) {
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   return batch.tokens * (static_cast<double>(a->num_slices) * a->k * (a->k > 1024 ? a->k / 1024.0 : 1.0) + cols * (cols > 4096 ? cols / 4096.0 : 1.0));
 }
-static bool small_batch(const MloraAddArgs* a, bool one_launch, const Batch& batch) {
+static bool small_batch(const MloraAddArgs* a, bool one_launch, double work) {
   const int fixed = knobs().small_batch_tokens;
   if (fixed > 0) return a->num_tokens <= fixed;
   const bool whole = decode_one_batch(a);
   double limit;
   if (a->r <= 16) limit = (whole ? 8.3e7 : 3.5e7) * (one_launch ? 0.65 : 1.0);
   else limit = one_launch ? 9.4e6 : !whole ? 8.5e6 : a->r <= 32 ? 2.1e7 : 1.1e7;
-  return small_work(a, batch) <= limit;
+  return work <= limit;
 }
 // Over the slots with K shared out (slot.hip) small tiles pay for longer (25 such calls between the lines: 0.872 of the time; K = 4096, rank 32, 558 tokens of 25 slots 7.1 / 11.2).
-static bool small_batch_in_parts(const MloraAddArgs* a, const Batch& batch) {
-  return knobs().small_batch_tokens <= 0 && slot_supported(a) && slot_k_parts(a) > 1 && small_work(a, batch) <= (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) &&
+static bool small_batch_in_parts(const MloraAddArgs* a, const Batch& batch, double work) {
+  return knobs().small_batch_tokens <= 0 && work <= (a->r <= 16 ? 8.3e7 : a->r <= 32 ? 2.6e7 : 1.5e7) && slot_supported(a) && slot_k_parts(a) > 1 &&
          slot_major_pays(a, batch);
 }
 
@@ -293,9 +293,12 @@ static bool pair_pays(const MloraAddArgs* a, int form, const Batch& batch) {
 // rank 32: 7.2 / 8.8 at 36).  The two-launch pair lies above both nearly throughout (K = 1024, rank 32 / 64, 1500 tokens
 // of 8 slots: 11.0 / 13.3 / 11.0 and 17.7 / 17.3 / 13.8 over 16-token tiles, as a pair, over 64-token tiles).
 static bool wide_instead(const MloraAddArgs* a, const Batch& batch) {
-  if (a->num_slices == 2 || a->r <= 16 || a->r * static_cast<long long>(a->k) < 24576 || !wide_supported(a) || !wide_pays(a, batch)) return false;
-  int columns;
-  return (small_tiles_about(batch) + 7) / 8 * decode_ranges(a, batch, &columns) > 32;
+  if (a->num_slices == 2 || a->r <= 16 || a->r * static_cast<long long>(a->k) < 24576) return false;
+  const int layers = (small_tiles_about(batch) + 7) / 8;
+  int columns = 0;
+  for (int i = 0; i < a->num_slices; ++i) columns += a->slices[i].n;
+  if (layers * (columns / 64ll + a->num_slices) <= 32) return false;  // (a range has 64 columns at least)
+  return layers * decode_ranges(a, batch, &columns) > 32 && wide_supported(a) && wide_pays(a, batch);
 }
 
 namespace {
@@ -349,48 +352,52 @@ int mlora::check_args(const MloraAddArgs* a) {
 int mlora::chosen_form(const MloraAddArgs* a, const Batch& batch) {
   int form = a->form;
   const bool vec = vector_ok(a);
+  const ApiKnobs& kn = knobs();
   if (form == MLORA_FORM_AUTO) {
-    const int forced = knobs().force_form;
+    const int forced = kn.force_form;
     if (forced >= MLORA_FORM_TOKEN && forced <= MLORA_FORM_PAIR && (forced == MLORA_FORM_TOKEN || vec)) form = forced;
   }
   if (form == MLORA_FORM_AUTO) {
     // Small batches (decode) are one launch over 16-token tiles; large ones split into 64-token
     // tiles for the long segments and 16-token tiles for the rest: one launch whose workgroups do
     // both products where a tile's column ranges repeat little of its shrink, else two launches.
-    const bool small_tiles = mfma_supported(a) && decode_supported(a);
-    const bool two_launches = mfma_supported(a) && sgmv_supported(a) && sgmv_workspace_ok(a);
-    const bool one_launch = mfma_supported(a) && wide_supported(a) && wide_pays(a, batch) && !knobs().no_wide;
+    // (What the two kinds of large ones cost is looked at only where small tiles do not win over both.)
+    const bool mfma = mfma_supported(a), small_tiles = mfma && decode_supported(a);
+    const double work = small_work(a, batch);
+    const bool small = small_tiles && small_batch(a, true, work) && small_batch(a, false, work);
+    const bool two_launches = !small && mfma && sgmv_supported(a) && sgmv_workspace_ok(a);
+    const bool one_launch = !small && mfma && !kn.no_wide && wide_supported(a) && wide_pays(a, batch);
     // (fp32 rows and anything else the 128-bit kernels for 16-bit elements do not take: one workgroup per token,
     // which fetches A and B per token and walks K in chained steps, except where the pair of launches has the
     // element type: config 1's batch, 64 tokens over 4 slots, rank 16, fp32, qkv / o / gate_up / down 25 / 25 / 27 /
     // 70 us per call in one workgroup per token, 7.0 / 6.7 / 8.0 / 7.6 in two launches; rank 24, 36 / 16 / 39 / 104 and 9.5 / 9.2 / 10.7 /
     // 10.9, rank 56, 81 / 80 / 90 / 243 and 12.6 / 12.1 / 14.3 / 15.5, one token of rank 24 15.3 / 15.4 / 15.8 / 43 and 8.5 / 8.5 / 9.2 / 9.9)
-    if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !knobs().no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
-    else if (small_tiles && small_batch_in_parts(a, batch)) form = MLORA_FORM_SPLIT;
-    else if (one_launch && !(small_tiles && small_batch(a, true, batch))) form = MLORA_FORM_WIDE;
-    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, batch))) form = MLORA_FORM_SGMV;
+    if (!vec) form = a->dtype == MLORA_DTYPE_F32 && !kn.no_pair && pair_supported(a) ? MLORA_FORM_PAIR : MLORA_FORM_TOKEN;
+    else if (small_tiles && !small && small_batch_in_parts(a, batch, work)) form = MLORA_FORM_SPLIT;
+    else if (one_launch && !(small_tiles && small_batch(a, true, work))) form = MLORA_FORM_WIDE;
+    else if (!one_launch && two_launches && !(small_tiles && small_batch(a, false, work))) form = MLORA_FORM_SGMV;
     else if (small_tiles) form = MLORA_FORM_SPLIT;
     else form = MLORA_FORM_BGMV;
   }
   // the split form where it pays (a large A[slot]) and shape and workspace allow it, else one
   // workgroup per (tile, column range)
   if (form == MLORA_FORM_SPLIT && a->form != MLORA_FORM_SPLIT &&
-      (knobs().no_split || !split_supported(a) || ((static_cast<long long>(a->r) * a->k < knobs().split_min_rk || batch.tokens > knobs().split_max_tokens) && knobs().force_form != MLORA_FORM_SPLIT)))
+      (kn.no_split || ((static_cast<long long>(a->r) * a->k < kn.split_min_rk || batch.tokens > kn.split_max_tokens) && kn.force_form != MLORA_FORM_SPLIT) || !split_supported(a)))
     form = MLORA_FORM_MFMA;
   // small tiles with the grid laid over the slots where the shape allows it and slot ids are few.
   // Also where the split form would be taken: at K = 4096 the slot-major kernel shares K out between
   // the workgroups of a tile itself (down, decode batch, us per call, slot-major / split form:
   // rank 32: 6.3 / 10.6, rank 64: 9.8 / 17.0).
-  if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_MFMA &&
-      knobs().force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, batch))
+  if ((form == MLORA_FORM_MFMA || form == MLORA_FORM_SPLIT) && a->form == MLORA_FORM_AUTO && kn.force_form != MLORA_FORM_MFMA &&
+      kn.force_form != MLORA_FORM_SPLIT && slot_supported(a) && slot_major_pays(a, batch))
     form = MLORA_FORM_SLOT;
-  if (a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_pair && !knobs().auto_fused && vec && pair_supported(a) && pair_pays(a, form, batch))
+  if (a->form == MLORA_FORM_AUTO && kn.force_form == 0 && !kn.no_pair && !kn.auto_fused && vec && pair_pays(a, form, batch) && pair_supported(a))
     form = MLORA_FORM_PAIR;
-  if (form == MLORA_FORM_MFMA && a->form == MLORA_FORM_AUTO && knobs().force_form == 0 && !knobs().no_wide && knobs().small_batch_tokens <= 0 &&
+  if (form == MLORA_FORM_MFMA && a->form == MLORA_FORM_AUTO && kn.force_form == 0 && !kn.no_wide && kn.small_batch_tokens <= 0 &&
       wide_instead(a, batch))
     form = MLORA_FORM_WIDE;
   // long-segment batches in one launch, on request
-  if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && knobs().force_form != MLORA_FORM_SGMV && knobs().auto_fused && fused_supported(a))
+  if (form == MLORA_FORM_SGMV && a->form == MLORA_FORM_AUTO && kn.force_form != MLORA_FORM_SGMV && kn.auto_fused && fused_supported(a))
     form = MLORA_FORM_FUSED;
   return form;
 }

@@ -385,9 +385,11 @@ Cut ring_cut(const MloraAddArgs* a, const Batch& batch, int most_parts) {
   long long cols = 0;
   for (int i = 0; i < a->num_slices; ++i) cols += a->slices[i].n;
   const double sums = 40.0 * a->num_slices + 0.3 * a->r / (a->r + 64) * tiles * cols / 512;
+  constexpr double share[] = {1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4};
+  static_assert(kMaxKSplit == 4, "a share of K for every number of parts");
   Cut best = {1, 0};
   for (int p = 1; p <= most_parts; ++p) {
-    const double columns = rounds_of(wgs * p) * a->k / p + sums * p;
+    const double columns = rounds_of(wgs * p) * a->k * share[p - 1] + sums * p;
     if (p == 1 || columns < best.columns) best = {p, columns};
   }
   return best;

@@ -680,19 +680,47 @@ inline size_t partial_bytes(int num_tokens, int num_slices, int r) {
 
 // K parts whose sums the workspace holds (one where there is none: wide.hip needs none, the others' launches have made sure of it).
 inline int parts_held(const MloraAddArgs* a) {
-  const size_t held = partials_room(a) / partial_bytes(a->num_tokens, a->num_slices, a->r);
-  return held < 1 ? 1 : held < kMaxKSplit ? static_cast<int>(held) : kMaxKSplit;
+  const size_t room = partials_room(a), bytes = partial_bytes(a->num_tokens, a->num_slices, a->r);
+  int held = 1;
+  while (held < kMaxKSplit && (held + 1) * bytes <= room) ++held;
+  return held;
 }
 // Of those, and of pieces of 64 columns, the ring's most.
-inline int most_parts(const MloraAddArgs* a) { return a->k / 64 < parts_held(a) ? a->k / 64 : parts_held(a); }
+inline int most_parts(const MloraAddArgs* a) {
+  const int held = parts_held(a);
+  return a->k / 64 < held ? a->k / 64 : held;
+}
 
-// How a call is cut into work, shared by the two-launch and the one-launch form.
-struct SgmvShape {
+// The tiles of a call, as every launch over 64-token tiles walks them.
+struct TileShape {
   bool empty;
   PlanLayout lay;
   ShrinkSlices sl;
   int tiles8;     // tiles / 8: 64-token tiles of the long segments, then the short segments
   int big_cap;    // tiles below this index are 64-token tiles
+  int cols;       // columns of the outputs
+};
+inline TileShape tile_shape(const MloraAddArgs* a) {
+  TileShape s;
+  s.empty = true;
+  s.lay = plan_layout(a->num_tokens, a->num_slots);
+  s.big_cap = (s.lay.cap_big + 7) & ~7;
+  int short_cap = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;  // a short segment is one small tile
+  if (short_cap > s.lay.cap_small) short_cap = s.lay.cap_small;
+  const int cap = s.big_cap + ((short_cap + 7) & ~7);
+  s.tiles8 = cap / 8;
+  s.cols = 0;
+  for (int i = 0; i < a->num_slices; ++i) {
+    s.cols += a->slices[i].n;
+    s.sl.a[i] = a->slices[i].a;
+  }
+  for (int i = a->num_slices; i < MLORA_MAX_SLICES; ++i) s.sl.a[i] = nullptr;
+  s.empty = cap == 0 || s.cols == 0;
+  return s;
+}
+
+// How a call is cut into work, shared by the two-launch form and the one with an exchange.
+struct SgmvShape : TileShape {
   int ksplit;     // shrink: K parts
   int krange;     // of the one-launch form: columns of a part
   bool slab;      // shrink: the kernel of slab.hip, whose K parts need no common length
@@ -708,55 +736,44 @@ struct SgmvShape {
 // one_launch: the cut for the form whose workgroups do both products (256-column slabs and batches,
 // which leave the registers the kernel needs besides; as many shrink roles per unit as it has workgroups).
 inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_launch = false) {
+  const SgmvKnobs& kn = sgmv_knobs();
   SgmvShape s;
-  s.empty = true;
-  s.lay = plan_layout(a->num_tokens, a->num_slots);
-  s.big_cap = (s.lay.cap_big + 7) & ~7;
-  int short_cap = a->num_slots < a->num_tokens ? a->num_slots : a->num_tokens;  // a short segment is one small tile
-  if (short_cap > s.lay.cap_small) short_cap = s.lay.cap_small;
-  const int cap = s.big_cap + ((short_cap + 7) & ~7);
-  if (cap == 0) return s;
-  s.tiles8 = cap / 8;
-  int cols = 0;
-  for (int i = 0; i < a->num_slices; ++i) {
-    cols += a->slices[i].n;
-    s.sl.a[i] = a->slices[i].a;
-  }
-  for (int i = a->num_slices; i < MLORA_MAX_SLICES; ++i) s.sl.a[i] = nullptr;
-  if (cols == 0) return s;
-  s.empty = false;
+  static_cast<TileShape&>(s) = tile_shape(a);
+  if (s.empty) return s;
+  const int cols = s.cols;
   const int est_tiles = batch.tokens / MLORA_TILE_BIG + 1;
 
   // Parts that divide K, as many as powers of two until the grid has a workgroup per compute unit and parts of at most 1024 columns: of the one-launch
   // form, and what the line of slab.hip at rank 64 compares with.  (The ring's are further down.)
-  int unit = 512;
-  while (unit > 128 && a->k % unit != 0) unit /= 2;
   const int max_parts = parts_held(a);
-  int ksplit = sgmv_knobs().ksplit;
-  if (ksplit <= 0) {
-    ksplit = 1;
-    while (ksplit < kMaxKSplit && a->k % (unit * ksplit * 2) == 0 &&
-           (static_cast<long long>(est_tiles) * a->num_slices * ksplit < 256 || a->k / ksplit > 1024))
-      ksplit *= 2;
-  }
-  if (ksplit > max_parts) ksplit = max_parts;
-  if (ksplit > kMaxKSplit) ksplit = kMaxKSplit;
-  while (ksplit > 1 && a->k % (unit * ksplit) != 0) --ksplit;
-  s.ksplit = ksplit;
-  s.krange = a->k / ksplit;
+  auto dividing_parts = [&] {
+    int unit = 512;
+    while (unit > 128 && a->k % unit != 0) unit /= 2;
+    int parts = kn.ksplit;
+    if (parts <= 0) {
+      parts = 1;
+      while (parts < kMaxKSplit && a->k % (unit * parts * 2) == 0 &&
+             (static_cast<long long>(est_tiles) * a->num_slices * parts < 256 || a->k / parts > 1024))
+        parts *= 2;
+    }
+    if (parts > max_parts) parts = max_parts;
+    if (parts > kMaxKSplit) parts = kMaxKSplit;
+    while (parts > 1 && a->k % (unit * parts) != 0) --parts;
+    return parts;
+  };
   // Which shrink.  The one of sgmv.hip, whose wavefronts share a ring, except as below: where slab.hip, whose wavefronts have rings of their own, was
   // taken (up to rank 32, and by parts of its own), it takes 1.020 of that time (876 random calls; K = 8192, rank 32, 5051 tokens 42.0 / 39.4).  The best
   // of one to four parts of each, the shared ring's time over the other's, K below 1100 / 2100 / 4200 / beyond, rank 8 0.996 / 0.996 / 0.984 / 0.956, rank 16
   // 0.992 / 0.993 / 0.981 / 0.958, rank 32 0.976 / 0.980 / 0.977 / 0.972, rank 64 0.958 / 0.965 / 0.965 / 0.962 (3980 calls).
   // (MLORA_SLAB=2 takes slab.hip also by name.)
-  s.slab = !one_launch && exact_rank(a->r) && slab_supported(a) && sgmv_knobs().slab == 2;
+  s.slab = !one_launch && exact_rank(a->r) && slab_supported(a) && kn.slab == 2;
   // Rank 64 with one or two slices and long segments (256 tokens or more per slot with tokens) while an XCD's workgroups number no more than its 32
   // compute units and slab.hip then cuts K into more parts than divide it (with two slices into as many), none longer than 2800 columns.  The line is from when the
   // other shrink's parts had to divide K (2 slots, K = 2560, 4096 tokens 32.9 / 25.6 us, K = 3072, 3600 27.9 / 25.9, K = 5120, 4096 28.1 / 23.2).
   // In its parts of today that shrink takes 0.967 of the time on such calls (42, K 1536 to 5632, 0.87 to 1.14); tests/test_gpu_slab_rank64.py
   // holds AUTO to the line.
   int round_parts = 0;
-  if (!one_launch && !s.slab && sgmv_knobs().slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 &&
+  if (!one_launch && !s.slab && kn.slab && a->form == MLORA_FORM_AUTO && slab_supported(a) && a->r == 64 && a->num_slices <= 2 &&
       batch.tokens / batch.slots >= 4 * MLORA_TILE_BIG) {
     const int tiles = static_cast<int>((batch.tokens + 63ll * batch.slots) / MLORA_TILE_BIG);  // at most: every slot's last tile has one token
     const int most = a->num_slices == 1 ? kMaxKSplit : 2;
@@ -764,39 +781,42 @@ inline SgmvShape sgmv_shape(const MloraAddArgs* a, const Batch& batch, bool one_
     if (parts > most) parts = most;
     if (parts > a->k / 1024) parts = a->k / 1024;
     if (parts > max_parts) parts = max_parts;
-    if (parts >= ksplit + (a->num_slices == 1) && a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128) {
+    if (a->k <= 2800 * parts && tiles * a->num_slices * parts >= 128 && parts >= dividing_parts() + (a->num_slices == 1)) {
       round_parts = parts;
       s.slab = true;
     }
   }
-  if (!one_launch) {
-    if (sgmv_knobs().ksplit > 0) s.ksplit = sgmv_knobs().ksplit < most_parts(a) ? sgmv_knobs().ksplit : most_parts(a);
+  if (one_launch) {
+    s.ksplit = dividing_parts();
+    s.krange = a->k / s.ksplit;
+  } else {
+    if (kn.ksplit > 0) s.ksplit = kn.ksplit < most_parts(a) ? kn.ksplit : most_parts(a);
     else s.ksplit = round_parts > 0 ? round_parts : ring_cut(a, batch, most_parts(a)).count;
   }
 
   // expand: consecutive tiles per workgroup (they share their B rows when they share their
   // slot), then column ranges so that the grid has about 2048 workgroups
-  int group = sgmv_knobs().group;
+  int group = kn.group;
   // wide projections only: narrow ones need the workgroups.  Two tiles per workgroup, not four: on
   // the prefill batch (8 adapters) gate_up takes 72.2 against 73.2 us per call, on the mixed batch
   // (126 adapters, many of them with fewer than four tiles) 105.8 against 110.4
   if (group != 1 && group != 2 && group != 4) group = (cols >= 4096 && est_tiles >= 64) ? 2 : 1;
   if (one_launch && group == 2) group = 4;  // the one-launch kernel exists for one tile and for four
-  const int target = sgmv_knobs().wgs;
-  int nt = sgmv_knobs().nt;
+  const int target = kn.wgs;
+  int nt = kn.nt;
   if (nt <= 0) {
     const long long want = static_cast<long long>(cols) * (est_tiles / group + 1) / (target > 0 ? target : 1);
     nt = want > 8192 ? 8192 : static_cast<int>(want);
   }
   s.group = group;
   s.nsplit = fill_splits(a, nt, s.splits.split);
-  s.cpl = sgmv_knobs().cpl == 4 ? 4 : 8;
-  s.stream = s.cpl == 8 && group <= 2 && (sgmv_knobs().stream < 0 ? static_cast<long long>(a->num_tokens) * cols * 2 >= kStreamBytes : sgmv_knobs().stream != 0);
+  s.cpl = kn.cpl == 4 ? 4 : 8;
+  s.stream = s.cpl == 8 && group <= 2 && (kn.stream < 0 ? static_cast<long long>(a->num_tokens) * cols * 2 >= kStreamBytes : kn.stream != 0);
   if (one_launch && a->k % 256 == 0) {
     // the unit's workgroups (one per column range) share out its shrink roles (tile, slice, K part):
     // about one role each
     if (group * a->num_slices > s.nsplit) s.group = group = 1;  // every slice has a column range: one role each at least
-    int parts = sgmv_knobs().ksplit;
+    int parts = kn.ksplit;
     if (parts <= 0) {
       parts = 1;
       while (parts < kMaxKSplit && group * a->num_slices * parts * 2 <= s.nsplit && a->k % (256 * parts * 2) == 0) parts *= 2;

@@ -483,11 +483,11 @@ Cut wide_cut(const MloraAddArgs* a, const Batch& batch, int widest_range) {
   for (int i = 0; i < a->num_slices; ++i)
     if (a->slices[i].n > longest) longest = a->slices[i].n;
   Cut best = {512, 0};
-  for (int columns = 512; columns <= widest_range && (columns == 512 || columns < 2 * longest); columns *= 2) {
+  for (int log2 = 9, columns = 512; columns <= widest_range && (columns == 512 || columns < 2 * longest); columns = 1 << ++log2) {
     long long ranges = 0;
     int widest = 0;
     for (int i = 0; i < a->num_slices; ++i) {
-      ranges += (a->slices[i].n + columns - 1) / columns;
+      ranges += (a->slices[i].n + columns - 1) >> log2;
       const int n = a->slices[i].n < columns ? a->slices[i].n : columns;
       if (n > widest) widest = n;
     }
@@ -530,7 +530,7 @@ bool wide_supported(const MloraAddArgs* a) {
 }
 
 int launch_wide(const MloraAddArgs* a, const Batch& batch) {
-  const SgmvShape sh = sgmv_shape(a, batch);
+  const TileShape sh = tile_shape(a);
   if (sh.empty) return 0;
   WideLaunch l;
   l.a = a; l.lay = sh.lay; l.sl = sh.sl; l.big_cap = sh.big_cap;
