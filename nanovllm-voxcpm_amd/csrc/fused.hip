@@ -45,9 +45,9 @@ __device__ __forceinline__ void fused_shrink_role(T* __restrict__ s_a, const int
   const int ti = (threadIdx.x / kWave) * 16 + (threadIdx.x & 15);
   const int row = plan[sorted_off + start + (ti < m ? ti : m - 1)];
   if (R > 16 && ((eff + 15) >> 4) < (R + 15) / 16)
-    shrink_body<T, R, KR, true, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
+    shrink_body<T, R, KR, true>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
   else
-    shrink_body<T, R, KR, false, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
+    shrink_body<T, R, KR, false>(s_a, xv, hws, xs, T_, K, num_slices, krange, sl, slice0, kpart, slot, start, m, eff, row);
 }
 
 // The same for the roles a workgroup computes because their seals did not arrive: the exception, so
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void sgmv_fused_kernel(
   __syncthreads();
 
   // ---- the unit's shrink roles ------------------------------------------------------------------------
-  // role s = (tile g of the group, q): q is a K part when a workgroup walks all slices, else (slice, K part)
+  // role s = (tile g of the group, slice, K part)
   const int rpt = num_slices * ksplit;
   const int YS = G * rpt;  // <= 64 (host)
   // a seal: {tag, XCD the sealing workgroup ran on}.  The partial sums are ordinary stores, which
@@ -282,15 +282,10 @@ void launch_fused_one(const FusedLaunch& l) {
                      sh.sl, sh.splits);
 }
 
-template <typename T, int R, int G>
-void launch_fused_slab(const FusedLaunch& l) {
-  launch_fused_one<T, R, 256, G>(l);
-}
-
 template <typename T, int R>
 void launch_fused_group(const FusedLaunch& l) {
-  if (l.sh->group == 4) launch_fused_slab<T, R, 4>(l);
-  else launch_fused_slab<T, R, 1>(l);
+  if (l.sh->group == 4) launch_fused_one<T, R, 256, 4>(l);
+  else launch_fused_one<T, R, 256, 1>(l);
 }
 
 template <typename T>

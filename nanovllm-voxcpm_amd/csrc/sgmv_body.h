@@ -109,10 +109,7 @@ constexpr int kShrinkWaves = 4;
 // the buffers (eff < R): 16-rank blocks of A[slot] at or above its rank are neither copied to LDS
 // nor multiplied, and their partial sums are not written (the expand does not read them).  The
 // unmasked instance is the code without any of those tests.
-//
-// SC1: the partial sums leave with agent-scope stores (they pass the compute unit's and the XCD's
-// caches on their way), for readers in other workgroups of the same launch.
-template <typename T, int R, int KR, bool MASKED, bool SC1 = false>
+template <typename T, int R, int KR, bool MASKED>
 __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __restrict__ xv, float* __restrict__ hws, int64_t xs, int T_, int K,
                                             int num_slices, int krange, const ShrinkSlices& sl, int slice, int kpart, int slot, int start, int m,
                                             int eff, int row) {
@@ -173,17 +170,7 @@ __device__ __forceinline__ void shrink_body(T* __restrict__ s_a, const void* __r
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int r0 = rb * 16 + 4 * lg;
-        if (r0 < R && (!MASKED || rb < rb_n)) {
-          if constexpr (SC1) {
-            uint64_t* q = reinterpret_cast<uint64_t*>(dst + r0);
-            __hip_atomic_store(q, (static_cast<uint64_t>(__float_as_uint(part[rb][1])) << 32) | __float_as_uint(part[rb][0]), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(q + 1, (static_cast<uint64_t>(__float_as_uint(part[rb][3])) << 32) | __float_as_uint(part[rb][2]), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-          } else {
-            *reinterpret_cast<f32x4*>(dst + r0) = part[rb];
-          }
-        }
+        if (r0 < R && (!MASKED || rb < rb_n)) *reinterpret_cast<f32x4*>(dst + r0) = part[rb];
       }
     }
   };
