@@ -310,8 +310,8 @@ def run_backbone(args) -> None:
 
 KERNELS = {
     "decode": "slot_kernel3<bf16,16> (qkv) + slot_kernel<bf16,16> (o, gate_up, down)",
-    "prefill": "wide_kernel<bf16,64> (qkv, o) + sgmv_shrink_kernel<bf16,64> + sgmv_expand_kernel<bf16,64> (gate_up, down)",
-    "mixed": "wide_kernel<bf16,64> (qkv, o) + sgmv_shrink_kernel<bf16,64> + sgmv_expand_kernel<bf16,64> (gate_up, down)",
+    "prefill": "wide_kernel<bf16,8> (qkv, o) + sgmv_shrink_kernel<bf16> + sgmv_expand_kernel<bf16,64> (gate_up, down)",
+    "mixed": "wide_kernel<bf16,8> (qkv, o) + sgmv_shrink_kernel<bf16> + sgmv_expand_kernel<bf16,64> (gate_up, down)",
 }
 
 

@@ -127,7 +127,7 @@ typedef struct MloraAddArgs {
 
 int mlora_add_lora(const MloraAddArgs* args);
 /* The same with the number of slots that have tokens in this batch, where the host knows it (0: it does not);
- * only MLORA_FORM_AUTO's choice depends on it. */
+ * MLORA_FORM_AUTO's choice depends on it, and how launches are cut, also those of a form by name. */
 int mlora_add_lora_active(const MloraAddArgs* args, int32_t active_slots);
 /* The same with the number of tokens that have a slot as well (0: unknown): it moves AUTO's lines and how a launch is cut. */
 int mlora_add_lora_counts(const MloraAddArgs* args, int32_t active_slots, int32_t active_tokens);

@@ -114,7 +114,7 @@ int launch_wide(const MloraAddArgs* a, const Batch& batch);
 // pair.hip: a shrink launch and an expand launch over the 16-token tiles, operands through LDS by
 // direct loads; 16- and 32-bit elements.
 bool pair_supported(const MloraAddArgs* a);
-// Under AUTO fp32 takes one launch where that is the faster one .
+// Under AUTO fp32 takes one launch where that is the faster one.
 int launch_pair(const MloraAddArgs* a, const Batch& batch);
 
 // group.hip: the low-level shrink and expand over tiles of a slot; `supported` says where they are the faster ones too.

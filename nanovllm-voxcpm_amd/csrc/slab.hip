@@ -11,10 +11,10 @@
 // cut K between them, each multiplies all tokens and ranks of the tile over its share, so nothing but
 // the sums at the end passes between them and no barrier stands between request and product.
 // Two wavefronts, not four: their rings (64 KB at rank 64) keep a compute unit's 64 KB of requests on their way, and two
-// workgroups fit a compute unit, so that one starts while the other sums up (rank 64, 9392 tokens, a quarter without
-// adapter, with the expand: qkv 28.3 -> 26.4 us per call, 8192 mixed tokens: gate_up 99.3 -> 98.3).  Rings of 48 KB, three
+// workgroups fit a compute unit, so that one starts while the other sums up.  Rings of 48 KB, three
 // stages at rank 64 with one workgroup per compute unit, are 1 % slower (494 calls of one or two slices, in the same K parts).
-// Shrink and expand at rank 32, 5000 tokens, K = 4096: 21.0 -> 18.5 us per call, 3.1 -> 3.5 TB/s.
+// Against x through registers it gained (rank 32, 5000 tokens, K = 4096, with the expand 21.0 -> 18.5 us per call); the ring that the wavefronts of
+// sgmv.hip share takes 0.96 to 0.99 of its time (sgmv_shape), so AUTO takes this kernel for some calls of rank 64 only.
 #include "common.h"
 #include "dma.h"
 #include "launch.h"

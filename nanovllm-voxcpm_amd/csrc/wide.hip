@@ -12,7 +12,7 @@
 // repeats the tile's shrink: its x rows and the slot's A rows come from the XCD's L2 after the
 // first range has fetched them (a tile's ranges are dispatched together on one XCD), so the
 // repeats cost compute-unit intake, not HBM traffic.  The library takes this form where the
-// repeats are few or its workgroups fill their rounds (wide_pays): projections of few, narrow slices over a short K.
+// repeats are few or it streams less than two launches would (wide_pays): projections of few, narrow slices over a short K.
 // Buffers of a rank between the instances' (24, 40, 48, 56) take the next instance up: their B rows lie in LDS at its pitch, and what their rank does
 // not have is fetched from their last row or piece and masked.  Steps of 24 layers, K = 1024, over 16-token tiles / this and sgmv.hip: rank 48, 9392 tokens
 // 4320 / 2941 us, 8192 mixed 5144 / 4288, rank 24 3359 / 2692 and 4171 / 3860.
